@@ -148,7 +148,9 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_mfma_kernel(GemmArgs a) {
         }
     }
 
-    gemm_epilogue<T, MT, NTL, F32>(a, acc, m0 + wm * TM, n0 + wn * TN, l31, hi);
+    static_assert(NW * epilogue_wave_bytes<NTL>() <= 2 * BUF_BYTES, "row images must fit the buffers");
+    __syncthreads();                                        // every wave has left the operand buffers
+    gemm_epilogue<T, MT, NTL, F32>(a, acc, m0 + wm * TM, n0 + wn * TN, lane, smem + wave * epilogue_wave_bytes<NTL>());
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -325,7 +327,10 @@ __global__ __launch_bounds__(WM * WN * 64 * KS) void gemm_pipe_kernel(GemmArgs a
                     for (int r = 0; r < 16; ++r) acc[i][j][r] += src[((i * MT + j) * 16 + r) * 64 + lane];
         }
     }
-    gemm_epilogue<T, MT, NTL>(a, acc, m0 + wm * TM, n0 + wn * TN, l31, hi);
+    constexpr int XCH_BYTES = (KS - 1) * NW * NTL * MT * 16 * 64 * 4;     // K groups: the accumulators handed over may still be read by other waves
+    static_assert(XCH_BYTES + NW * epilogue_wave_bytes<NTL>() <= KS * NSTAGE * BUF_BYTES, "row images must fit the rings");
+    if constexpr (KS == 1) __syncthreads();                 // every wave has left the ring
+    gemm_epilogue<T, MT, NTL>(a, acc, m0 + wm * TM, n0 + wn * TN, lane, smem + XCH_BYTES + wave * epilogue_wave_bytes<NTL>());
 }
 
 // ---------------------------------------------------------------------------------------------

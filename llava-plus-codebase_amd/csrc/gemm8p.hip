@@ -13,12 +13,15 @@
 //     so each phase needs at most one new operand half: 12 / 4 / 8 / 0 ds_read_b128 per wave (W half 0 stays in registers).
 //   * Operand staging is a ring of 8 HALF-tiles (128 rows x 64 k = 16 KiB: X half = rows {0..63} (+64*half) of both wave rows,
 //     W half = rows {0..31} (+32*half) of all four wave columns), filled by LDS-DMA (buffer_load_dwordx4 ... lds, 2 per wave per
-//     half-tile) SIX phases ahead of their first use: one half-tile is issued per phase, two stay in flight across the
-//     once-per-K-step `s_waitcnt vmcnt(4)`; nothing in the main loop ever waits for vmcnt(0).
+//     half-tile) five or six phases ahead of their first use: one half-tile is issued per phase, and the phase before the first
+//     read of a half-tile waits for that one alone (`s_waitcnt vmcnt(8)`: the four issued after it stay in flight), so every
+//     half-tile has a whole K-step to land; nothing in the main loop ever waits for vmcnt(0).  (One wait per K-step for all four
+//     halves gave the last one half a K-step: 575.8 -> 556.9 us at 6528 x 11008 x 4096, 106.6 -> 101.7 at 2048 x 11264 x 2048.)
 //   * Hazards (MI355X_MICROARCH.md "Two waves per SIMD" item 7, guide §5 "Read a staged buffer one phase AFTER the wait"):
 //       RAW  a half-tile is read only after every wave's counted vmcnt that covers it AND a barrier both groups have passed:
-//            the wait sits in phase 3 of K-step kt (before that phase's first barrier) and covers all four half-tiles of
-//            K-step kt+1, whose first read is in phase 0 of kt+1 — two barrier instances later for either group.
+//            the wait sits in the load segment of the phase before (in front of that phase's first barrier).  With group 1 one
+//            barrier behind, group 0's load segment of phase p + 1 begins behind the instance that is group 1's first barrier of
+//            phase p, i.e. behind group 1's wait; group 1's begins one instance later still.
 //       WAR  half-tile h goes into the ring slot of half-tile h-8, whose last ds_read is in phase h-8 (or h-9); h is issued in
 //            phase h-6, i.e. two phases (four barrier instances) after those reads were retired by lgkmcnt(0) in both groups.
 //   * LDS image per half-tile: 128 rows x 128 B, 16-byte chunk c of row r stored at chunk c ^ ((r >> 1) & 7): the 16-lane
@@ -297,7 +300,7 @@ __global__ __launch_bounds__(512) void gemm8p_kernel(GemmArgs a) {
 #pragma unroll
     for (int h = 0; h < 6; ++h)
         if (h < n_half && ((h & 3) != 3 || a.M - m0 > 64)) stage(kt_begin + (h >> 2), h & 3, ((h >> 2) & 1) * 4 + (h & 3));
-    wait_halves(nk >= 2 ? 2 : 0);
+    wait_halves((nk >= 2 ? 3 : 1) + (a.M - m0 > 64 ? 1 : 0));      // X and W half 0 of K-step 0 have landed
     __builtin_amdgcn_s_barrier();
     if (group1) __builtin_amdgcn_s_barrier();          // stagger: group 1 runs one barrier behind group 0
 
@@ -331,6 +334,8 @@ __global__ __launch_bounds__(512) void gemm8p_kernel(GemmArgs a) {
             }
             __builtin_amdgcn_s_setprio(0);
         };
+        // half-tiles in flight behind the one a wait is for: the four that were issued after it (three where X half 1 is left out)
+        constexpr int AHEAD = SKIPX1 ? 3 : 4;
         // one K-step = 4 phases; PAR = ring half (kt & 1), known at compile time so every LDS offset is an immediate.
         // Half-tile issued in phase p of K-step kt: sequence index 4 kt + p + 6 -> K-step kt+1 (j = p+2) for p < 2, K-step kt+2 (j = p-2) else.
         auto kstep = [&](auto par_c, int kt) {
@@ -342,13 +347,17 @@ __global__ __launch_bounds__(512) void gemm8p_kernel(GemmArgs a) {
             read_x(SX0);
             __builtin_amdgcn_sched_barrier(0);
             if (kt + 1 < nk) stage(kt_begin + kt + 1, 2, (1 - PAR) * 4 + 2);
+            wait_halves(kt + 1 < nk ? AHEAD : AHEAD - 3);             // W half 1 of this K-step (read in phase 1)
             __builtin_amdgcn_s_barrier();
             mma(wb0, 0, 0);
             __builtin_amdgcn_s_barrier();
             // phase 1 -----------------------------------------------------------------------------------------------------------
             read_w(SW1, wb1);
             __builtin_amdgcn_sched_barrier(0);
-            if constexpr (!SKIPX1) { if (kt + 1 < nk) stage(kt_begin + kt + 1, 3, (1 - PAR) * 4 + 3); }
+            if constexpr (!SKIPX1) {
+                if (kt + 1 < nk) stage(kt_begin + kt + 1, 3, (1 - PAR) * 4 + 3);
+                wait_halves(kt + 1 < nk ? 4 : 0);                     // X half 1 of this K-step (read in phase 2)
+            }
             __builtin_amdgcn_s_barrier();
             mma(wb1, 1, 0);
             __builtin_amdgcn_s_barrier();
@@ -361,8 +370,7 @@ __global__ __launch_bounds__(512) void gemm8p_kernel(GemmArgs a) {
             __builtin_amdgcn_s_barrier();
             // phase 3 -----------------------------------------------------------------------------------------------------------
             if (kt + 2 < nk) stage(kt_begin + kt + 2, 1, PAR * 4 + 1);
-            // every half-tile of K-step kt+1 must have landed; the two of kt+2 issued in this K-step may stay in flight
-            wait_halves(kt + 2 < nk ? 2 : 0);
+            wait_halves(kt + 2 < nk ? AHEAD : AHEAD - 2);             // X and W half 0 of K-step kt + 1 (read in its phase 0)
             __builtin_amdgcn_s_barrier();
             if constexpr (!SKIPX1) mma(wb0, 0, 1);
             __builtin_amdgcn_s_barrier();
@@ -383,7 +391,8 @@ __global__ __launch_bounds__(512) void gemm8p_kernel(GemmArgs a) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     if constexpr (SPLIT == 1) {
         if (a.qf_kc) { qkv_rope_epilogue<T>(a, acc, smem, m0, n0, wm, wn, l31, hi, tid); return; }
-        gemm_epilogue<T, 4, 2>(a, acc, m_base, n_base, l31, hi);
+        // (the operand ring is dead: every half-tile has landed and been read before the balancing barrier)
+        gemm_epilogue<T, 4, 2>(a, acc, m_base, n_base, lane, smem + wave * epilogue_wave_bytes<2>());
     } else {
         // ---- split-K: store the partial tile and exit; the kernel boundary publishes it (plain stores) ---------------------------------------
         // accumulator order: float4 number (i*4 + j)*4 + q of lane `tid` lives at byte ((idx * 512) + tid) * 16 of the slab, so every wave-instruction
@@ -452,7 +461,8 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(GemmArgs a) {
                 t += f32x4{__uint_as_float(w[i][sl][q].x), __uint_as_float(w[i][sl][q].y), __uint_as_float(w[i][sl][q].z), __uint_as_float(w[i][sl][q].w)};
             acc[i][0][4 * q] = t.x; acc[i][0][4 * q + 1] = t.y; acc[i][0][4 * q + 2] = t.z; acc[i][0][4 * q + 3] = t.w;
         }
-    gemm_epilogue<T, 1, 2>(a, acc, m_base, n_base, l31, hi);
+    __shared__ __attribute__((aligned(16))) char img[4 * epilogue_wave_bytes<2>()];
+    gemm_epilogue<T, 1, 2>(a, acc, m_base, n_base, lane, img + wn * epilogue_wave_bytes<2>());
 }
 
 // splitk_reduce_rows_kernel: the same sums, with the output side turned into ROW order through LDS.  In accumulator order a lane owns 4 consecutive n of one row
@@ -524,8 +534,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_rows_kernel(GemmArgs a) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) v[e] += b[e];
         }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = apply_act(v[e], act);
+        apply_act_n<4>(v, act);
         if (R) {
             v[0] += unpack_lo<T>(rr[k].x); v[1] += unpack_hi<T>(rr[k].x); v[2] += unpack_lo<T>(rr[k].y); v[3] += unpack_hi<T>(rr[k].y);
         }

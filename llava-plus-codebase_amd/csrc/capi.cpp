@@ -472,7 +472,18 @@ int lmx_op_gemm(int32_t dtype, const void* x, const void* w, void* c, const void
         skinny_op(dtype, GemmArgs{x, w, c, bias, residual, M, N, K, ldx, ldw, ldc, ldr, act}, variant, S(stream));
         return 0;
     }
-    launch_gemm(dtype, GemmArgs{x, w, c, bias, residual, M, N, K, ldx, ldw, ldc, ldr, act}, variant, S(stream));
+    GemmArgs g{x, w, c, bias, residual, M, N, K, ldx, ldw, ldc, ldr, act};
+    if (variant >= 1000 && variant % 100 > 1) {          // K slices of gemm_rows: this entry's own slab, one stream at a time
+        static std::mutex mu;
+        static DevBuf slab;
+        std::lock_guard<std::mutex> lk(mu);
+        const size_t need = gemm_rows_slab_bytes(M, N, variant % 100);
+        if (slab.bytes < need) { LMX_CHECK_HIP(hipDeviceSynchronize()); slab.ensure(need); }
+        g.skw = slab.p;
+        launch_gemm(dtype, g, variant, S(stream));
+        return 0;
+    }
+    launch_gemm(dtype, g, variant, S(stream));
     LMX_API_END
 }
 int lmx_op_gemv(int32_t dtype, const void* x, const void* w, void* c, const void* bias, const void* residual, const void* norm_w, float eps,

@@ -681,6 +681,10 @@ static void launch_gemm16(const GemmArgs& a, int variant, hipStream_t st) {
     // variant: 0 = auto, 2 = 128x128 reg-staged (kept as an independent cross-check of the LDS-DMA path), 4 = 64x128 glds, 5 = 64x64 glds,
     //          7 / 9 = LDS-ring kernels with counted vmcnt (128x256x64 3-slot, 256x256x64 2-slot; 8 waves), 15 = 64x64 4-slot ring (4 waves),
     //          18 = 128x128x64 2-slot 4 waves.  (Round 5 removed the arms auto never picks: 1, 12, 14 and the deeper rings 23 - 26 of round 4, EXPERIMENTS.md r4-C.)
+    if (variant == 0) {
+        const RowsForm f = gemm_rows_form(TypeInfo<T>::id, a);
+        if (f.mtiles) { launch_gemm_rows(TypeInfo<T>::id, a, f.mtiles, f.bn, f.slices, st); return; }
+    }
     if (a.c_f32) { launch_gemm_cfg<T, 64, 128, 2, 2, true, true>(a, st); return; }      // fp32 logits of a few wanted rows: one tile form
     if (variant == 0) {
         // Large problems: the ping-pong 256x256x64 kernel (gemm8p.hip), K-sliced when N = hidden leaves CUs idle and the caller brought
@@ -753,6 +757,7 @@ void launch_gemm(int dtype, const GemmArgs& a, int variant, hipStream_t st) {
         launch_gemm8p(dtype, b, st);
         return;
     }
+    if (variant >= 1000) { launch_gemm_rows(dtype, a, variant / 1000, variant / 100 % 10 * 64, variant % 100, st); return; }
     LMX_REQUIRE(a.N % 8 == 0, "gemm: N must be a multiple of 8");
     LMX_REQUIRE(!a.c_f32 || (!a.skw && !a.pk_kc && !a.qf_kc && !a.R && !act_gated(a.act)), "gemm: fp32 output is for plain un-split linears");
     if (act_gated(a.act)) LMX_REQUIRE(a.N % 64 == 0, "gemm: SiLU·mul needs N (fused gate|up rows) % 64 == 0");

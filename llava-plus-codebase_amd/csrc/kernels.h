@@ -46,6 +46,14 @@ bool gemm8p_enabled();
 void launch_gemm8p(int dtype, const GemmArgs& a, hipStream_t st);
 size_t gemm8p_splitk_ws_bytes(int M, int N, int split_k);
 int gemm8p_pick_split(int M, int N, int K);
+// linears of up to a few hundred rows (gemm_rows.hip): mtiles row tiles of <= 256 rows, BN = 64 / 128 weight rows a workgroup, S slices of K (S > 1: fp32 slabs in a.skw,
+// gemm_rows_slab_bytes, and a second launch that adds them); variant 1000 mtiles + 100 (BN / 64) + S of launch_gemm
+bool gemm_rows_applies(int dtype, const GemmArgs& a);
+struct RowsForm { int mtiles, bn, slices; };
+RowsForm gemm_rows_form(int dtype, const GemmArgs& a);                // the form variant 0 takes (mtiles 0: another kernel)
+constexpr size_t ROWS_SLAB_MAX = (size_t)64 << 20;                    // what a caller's a.skw holds
+size_t gemm_rows_slab_bytes(int M, int N, int S);
+void launch_gemm_rows(int dtype, const GemmArgs& a, int mtiles, int BN, int S, hipStream_t st);
 // decode-batch linear (skinny.hip): M <= 32 rows, 16-bit, weights streamed once straight into MFMA operands; variant 20 of launch_gemm
 void launch_skinny_gemm(int dtype, const GemmArgs& a, hipStream_t st);
 int skinny_kslices(int M, int N, int K);          // K slices the narrow-layer form takes when a.skw / a.sk_cnt are given (1 = the 16-rows-per-workgroup form)

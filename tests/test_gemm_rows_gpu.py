@@ -1,0 +1,58 @@
+"""Linears of a few dozen to a few hundred rows (csrc/gemm_rows.hip): every form at the edges of its tiles — rows around 32 and 256, weight rows that fill no tile, fewer slabs of K
+than the ring holds, slices of unequal length — against the float64 product rounded once (one unit in the last place, as tests/test_gemm8p_gpu.py derives it), and the rule
+that sends a product here."""
+import pytest
+import torch
+
+from test_gemm8p_gpu import DT, _mk, assert_one_ulp
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("variant", [1101, 1103, 1201, 1202, 2101, 2202, 3203])
+@pytest.mark.parametrize("M,N,K", [(1, 64, 64), (31, 72, 192), (33, 136, 320), (128, 200, 448), (200, 776, 1024), (256, 128, 640), (257, 384, 1152), (500, 520, 704), (600, 264, 2048)])
+def test_forms(cuda, dt, variant, M, N, K):
+    from llava_mi355x import ops
+    if -(-M // (variant // 1000)) > 256 or variant % 100 > K // 64:
+        pytest.skip("not a form of this shape")
+    x, w = _mk(M, N, K, dt, cuda, M + N + K + variant)
+    ref = x.double() @ w.double().t()
+    got = ops.gemm(x, w, variant=variant)
+    assert_one_ulp(got, ref, dt, 2e-5 * float(ref.abs().max()), f"variant {variant} {M}x{N}x{K}")
+    assert torch.equal(got, ops.gemm(x, w, variant=variant))
+
+
+@pytest.mark.parametrize("variant", [1101, 1102, 1201, 1204, 2202])
+@pytest.mark.parametrize("act", [0, 1, 2, 3, 4])
+def test_epilogues(cuda, variant, act):
+    from llava_mi355x import ops
+    M, N, K = 139, 448, 832
+    x, w = _mk(M, N, K, "bf16", cuda, act + variant)
+    b = torch.randn(N, device=cuda).bfloat16()
+    y = x.double() @ w.double().t() + b.double()
+    if act >= 3:
+        y = y.view(M, N // 64, 2, 32)
+        ref = ((torch.nn.functional.silu(y[:, :, 0]) if act == 3 else torch.relu(y[:, :, 0])) * y[:, :, 1]).reshape(M, N // 2)
+        got = ops.gemm(x, w, bias=b, act=act, variant=variant, out=torch.empty(M, N // 2, device=cuda, dtype=DT["bf16"]))
+        assert_one_ulp(got, ref, "bf16", 6e-5 * float(ref.abs().max()), f"variant {variant} act {act}")
+        return
+    y = y * torch.sigmoid(1.702 * y) if act == 1 else torch.nn.functional.gelu(y) if act == 2 else y
+    r = torch.randn(M, N, device=cuda).bfloat16()
+    got = ops.gemm(x, w, bias=b, residual=r, act=act, variant=variant)
+    assert_one_ulp(got, y + r.double(), "bf16", 3e-5 * float((y + r.double()).abs().max()), f"variant {variant} act {act}")
+    ops.gemm(x, w, bias=b, residual=r, act=act, variant=variant, out=r)              # in place
+    assert torch.equal(r, got)
+
+
+@pytest.mark.parametrize("M", [2, 32, 128, 129, 256, 257, 384, 385, 512, 513])
+@pytest.mark.parametrize("N,K,ldc", [(12288, 1024, 12288), (22016, 1024, 22016), (12288, 1024, 12292)])
+def test_rule(cuda, M, N, K, ldc):
+    """What variant 0 takes, on both sides of every line of the rule and with rows that are not 16-byte aligned (another kernel's)."""
+    from llava_mi355x import ops
+    x, w = _mk(M, N, K, "bf16", cuda, M)
+    out = torch.zeros(M, ldc, device=cuda, dtype=DT["bf16"])
+    got = ops.gemm(x, w, out=out[:, :N])
+    ref = x.double() @ w.double().t()
+    assert_one_ulp(got, ref, "bf16", 2e-5 * float(ref.abs().max()), f"{M}x{N}x{K}")
+    assert ldc == N or not bool(out[:, N:].any())

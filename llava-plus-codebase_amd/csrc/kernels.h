@@ -217,6 +217,7 @@ struct WinDecodeArgs {
     float scale = 1.f, eps = 0.f;
 };
 void launch_decode_win(int dtype, int D, const WinDecodeArgs& a, hipStream_t st);
+bool decode_win_grouped(int dtype, int D, int n_heads, int n_kv_heads, int n_seq);      // one workgroup per kv head and split instead of one per query head and split
 
 // ---- gated delta rule (delta.hip): per head a state S [key channel][value channel] in fp32, S <- g S;  u = beta (v - S^T k);  S <- S + k u^T;  o = S^T q -----------------
 // Projection rows of a layer: q [G][DK] | k [G][DK] | v [H][DV] | beta [H] | ...; DK in {64, 128, 256} and DV (a multiple of 64) are padded head widths, the padding is

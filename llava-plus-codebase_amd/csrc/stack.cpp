@@ -531,7 +531,7 @@ void Model::stack_prefill(Seq* const* seqs, const void* const* embeds, const int
 // ---------------------------------------------------------------------------------------------------------------
 // decode
 // ---------------------------------------------------------------------------------------------------------------
-static WinDecodeArgs decode_args(const Stack& S, const StackLayer& l, const void* qkv, void* out, int n_seq, int max_len, int s_max) {
+static WinDecodeArgs decode_args(const Stack& S, const StackLayer& l, int dtype, const void* qkv, void* out, int n_seq, int max_len, int s_max) {
     const lmx_layer_config& d = l.c;
     WinDecodeArgs a;
     a.qkv = qkv; a.out = out; a.q_norm = l.qn; a.k_norm = l.kn; a.cos_sin = d.rope_dims ? S.rope[(size_t)d.rope_table] : nullptr;
@@ -541,7 +541,9 @@ static WinDecodeArgs decode_args(const Stack& S, const StackLayer& l, const void
     int span = max_len + 1;
     if (d.window > 0 && d.window + 127 < span) span = d.window + 127;
     const int chunks = std::max(1, std::min((span + 127) / 128, 32));
-    const int fill = (1024 + d.n_heads * n_seq - 1) / (d.n_heads * n_seq);
+    const bool grouped = decode_win_grouped(dtype, l.D, d.n_heads, d.n_kv_heads, n_seq);
+    const int wgs = (grouped ? d.n_kv_heads : d.n_heads) * n_seq, want = grouped ? 256 : 1024;       // workgroups of one split
+    const int fill = (want + wgs - 1) / wgs;
     a.n_split = std::max(1, std::min(chunks, fill));
     return a;
 }
@@ -620,7 +622,7 @@ void Model::stack_decode_step(Seq* s, hipStream_t st, int64_t* id_out) {
         top = 0;
         if (l.c.mixer == LMX_MIXER_ATTENTION) {
             LMX_PROF_K("decode.attn");
-            WinDecodeArgs a = decode_args(S, l, s->d_qkv, s->d_attn, 1, s->len, s_max);
+            WinDecodeArgs a = decode_args(S, l, dt, s->d_qkv, s->d_attn, 1, s->len, s_max);
             a.one = stack_seq_ref(r, s);
             a.pos = s->len;
             launch_decode_win(dt, l.D, a, st);
@@ -689,7 +691,7 @@ void Model::stack_decode_batch_step(Batch* b, Seq* const* seqs, int n, int64_t* 
         const DecodeFusedSeq* tab = b->d_attn_tab + (size_t)r * b->cap;
         if (l.c.mixer == LMX_MIXER_ATTENTION) {
             LMX_PROF("decode_batch.attn");
-            WinDecodeArgs a = decode_args(S, l, b->qkv, b->attn, n, max_len, s_max);
+            WinDecodeArgs a = decode_args(S, l, dt, b->qkv, b->attn, n, max_len, s_max);
             a.tab = tab;
             launch_decode_win(dt, l.D, a, st);
         } else stack_mix_decode(r, tab, DecodeFusedSeq{}, n, max_len, b->qkv, b->attn, b->sw, b, st);

@@ -638,12 +638,255 @@ __global__ __launch_bounds__(256) void decode_win_kernel(WinDecodeArgs a) {
     if (tid == 0) __hip_atomic_store(e.counters + head, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);    // re-arm for the next launch
 }
 
+// The same launch for 16-bit models with head widths up to 128: one workgroup per (kv head, split, sequence) serves ALL query heads of the kv head on MFMA tiles, so a cached
+// key and value leaves memory once instead of once per query head.  A wave takes 32 of a 128-key chunk (no barrier inside the walk): scores = K tile (16 keys, straight from the
+// cache rows into the MFMA operand) x query heads (16 columns), the softmax over the lane's 8 keys and 4 lanes, then V^T rows x probabilities.  The C layout of the scores
+// (lane = head, 4 rows a tile) is the B layout of the probabilities when row 4 q + r of tile t is key 8 q + 4 t + r, so no value changes lanes.  Probabilities
+// stay exact to 24 bits: three 16-bit terms, three MFMAs.  Bound: the cache stream (32 sequences x 1024 keys, 8 kv heads of 128: 134 MB a launch); figures: decode_win_grouped.
+template <typename T> struct WinMfma;
+template <> struct WinMfma<bf16_t> {
+    static __device__ __forceinline__ f32x4 run(const uint4& a, const uint4& b, f32x4 c) {
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_v, a), __builtin_bit_cast(bf16x8_v, b), c, 0, 0, 0);
+    }
+};
+template <> struct WinMfma<f16_t> {
+    static __device__ __forceinline__ f32x4 run(const uint4& a, const uint4& b, f32x4 c) {
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_v, a), __builtin_bit_cast(f16x8_v, b), c, 0, 0, 0);
+    }
+};
+constexpr int WIN_GROUP_MAX = 16;                              // query heads of a kv head: the columns of a tile
+static int win_group_smem(int group, int D) { return (group * D + 5 * D + 4 * group * D + 2 * 4 * 16 + 8) * (int)sizeof(float); }
+
+template <typename T, int D>
+__global__ __launch_bounds__(256) void decode_win_group_kernel(WinDecodeArgs a) {
+    extern __shared__ __attribute__((aligned(16))) float wsm[];
+    const int group = a.n_heads / a.n_kv_heads;
+    float *qs = wsm, *ks = qs + group * D, *tmp = ks + D, *wo = tmp + 4 * D, *wm = wo + 4 * group * D, *wl = wm + 64, *flag = wl + 64;      // wo: [wave][head][D]
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int i16 = lane & 15, q4 = lane >> 4;
+    const int kvh = blockIdx.x, split = blockIdx.y, z = blockIdx.z;
+    const DecodeFusedSeq e = a.tab ? a.tab[z] : a.one;
+    int pos = a.pos >= 0 ? a.pos : *e.pos_ptr;
+    pos = pos < a.s_max ? pos : a.s_max - 1;
+    const int lo = a.window > 0 && pos - a.window + 1 > 0 ? pos - a.window + 1 : 0;
+    const int c0 = lo / DF_CHUNK, c1 = pos / DF_CHUNK;
+    const T* row = reinterpret_cast<const T*>(a.qkv) + (size_t)z * a.qkv_stride;
+    T* Kc = reinterpret_cast<T*>(e.K) + (size_t)kvh * a.s_max * D;
+    T* Vt = reinterpret_cast<T*>(e.VT) + (size_t)kvh * D * a.s_max;
+    const T* vnew = row + (a.n_heads + a.n_kv_heads + kvh) * D;
+    const float* cs = a.cos_sin + (size_t)pos * a.rot_dims;
+    const bool owner = (c1 - c0) % a.n_split == split;         // this workgroup takes the new key
+    constexpr int NT = D / 32, ND = D / 16;                    // 32-deep steps of a score, 16-row tiles of V^T
+    const float scl = a.scale * 1.4426950408889634f;
+
+    // contraction step t of a score: lane group q4 holds dimensions q4 D / 4 + 8 t .. + 7, so a key row leaves in 16-byte pieces of one contiguous quarter per lane
+    // the next chunk's keys are requested when this one's are in the scores, its values when this one's are in the sums (past the last chunk of the split: the last one again,
+    // no branch around the loads).  Two whole chunks in registers are slower: the walk's code doubles, and a launch this short waits for its instructions
+    uint4 kf[2][NT], vf[ND];
+    auto load_k = [&](int c) {
+        const int base = c * DF_CHUNK + wave * 32;
+#pragma unroll
+        for (int t2 = 0; t2 < 2; ++t2) {
+            int key = base + 8 * (i16 >> 2) + 4 * t2 + (i16 & 3);
+            key = key < pos ? key : (pos > 0 ? pos - 1 : 0);   // rows past the cached keys re-read the last one; their scores are dropped
+#pragma unroll
+            for (int t = 0; t < NT; ++t) kf[t2][t] = *reinterpret_cast<const uint4*>(Kc + (size_t)key * D + q4 * (D / 4) + 8 * t);
+        }
+    };
+    auto load_v = [&](int c) {
+        const T* p = Vt + (size_t)i16 * a.s_max + c * DF_CHUNK + wave * 32 + 8 * q4;
+#pragma unroll
+        for (int d = 0; d < ND; ++d) vf[d] = *reinterpret_cast<const uint4*>(p + (size_t)d * 16 * a.s_max);
+    };
+    // this split's chunks, from a place of its own on: in step, all workgroups would read the same columns of their V^T rows, which lie a power of two apart
+    const int mine = c1 - c0 < split ? 0 : (c1 - c0 - split) / a.n_split + 1, rot = mine ? (int)((kvh * 5u + z * 3u) % (unsigned)mine) : 0;
+    auto chunk = [&](int i) { i += rot; i = i < mine ? i : i - mine; return c0 + split + i * a.n_split; };
+    if (mine) { load_k(chunk(0)); load_v(chunk(0)); }
+    for (int h = wave; h < group + (owner ? 1 : 0); h += 4) {  // the query heads, then the new key
+        const bool isk = h == group;
+        norm_rope_vec<T, D>(row + (isk ? a.n_heads + kvh : kvh * group + h) * D, reinterpret_cast<const T*>(isk ? a.k_norm : a.q_norm), a.eps, a.qk_dim, cs, a.rot_dims, tmp + wave * D,
+                            qs + h * D, lane);
+    }
+    __syncthreads();
+    if (owner) {
+        for (int d = tid; d < D; d += 256) {
+            Kc[(size_t)pos * D + d] = from_f32<T>(ks[d]);
+            Vt[(size_t)d * a.s_max + pos] = vnew[d];
+        }
+    }
+    auto frag = [&](const float* v) -> uint4 {                 // 8 consecutive fp32 values that are 16-bit ones already
+        float x[8]; load8<float>(v, x);
+        return uint4{pack2<T>(x[0], x[1]), pack2<T>(x[2], x[3]), pack2<T>(x[4], x[5]), pack2<T>(x[6], x[7])};
+    };
+    uint4 qf[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) qf[t] = i16 < group ? frag(qs + i16 * D + q4 * (D / 4) + 8 * t) : uint4{0u, 0u, 0u, 0u};
+
+    float m = -INFINITY, l = 0.f;                              // of head i16; l: this lane's keys
+    f32x4 acc[ND];                                             // [16 d + 4 q4 + r][head i16]
+#pragma unroll
+    for (int d = 0; d < ND; ++d) acc[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < mine; ++i) {
+        const int c = chunk(i), base = c * DF_CHUNK + wave * 32;
+        f32x4 s[2];
+#pragma unroll
+        for (int t2 = 0; t2 < 2; ++t2) {
+            s[t2] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int t = 0; t < NT; ++t) s[t2] = WinMfma<T>::run(kf[t2][t], qf[t], s[t2]);
+        }
+        if (i + 1 < mine) load_k(chunk(i + 1));
+        const bool edge = base < lo || base + 32 > pos;        // some of the wave's keys are outside: their scores are dropped and their values, whatever they hold, cleared
+        float mx = -INFINITY;
+#pragma unroll
+        for (int t2 = 0; t2 < 2; ++t2)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int key = base + 8 * q4 + 4 * t2 + r;
+                s[t2][r] = !edge || (key >= lo && key < pos) ? s[t2][r] * scl : -INFINITY;
+                mx = fmaxf(mx, s[t2][r]);
+            }
+        if (edge) {
+            uint32_t keep[4];
+#pragma unroll
+            for (int h = 0; h < 4; ++h) {
+                const int key = base + 8 * q4 + 2 * h;
+                keep[h] = (key >= lo && key < pos ? 0x0000ffffu : 0u) | (key + 1 >= lo && key + 1 < pos ? 0xffff0000u : 0u);
+            }
+#pragma unroll
+            for (int d = 0; d < ND; ++d) { vf[d].x &= keep[0]; vf[d].y &= keep[1]; vf[d].z &= keep[2]; vf[d].w &= keep[3]; }
+        }
+        mx = fmaxf(mx, __shfl_xor(mx, 16, 64)); mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        const float m_new = fmaxf(m, mx), ms = m_new == -INFINITY ? 0.f : m_new;
+        const float alpha = __builtin_amdgcn_exp2f(m - ms);
+        m = m_new;
+        float p[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) p[k] = __builtin_amdgcn_exp2f(s[k >> 2][k & 3] - ms);
+        l = l * alpha + (((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7])));
+        uint4 pf[3];
+#pragma unroll
+        for (int n = 0; n < 3; ++n) {
+            pf[n] = uint4{pack2<T>(p[0], p[1]), pack2<T>(p[2], p[3]), pack2<T>(p[4], p[5]), pack2<T>(p[6], p[7])};
+            p[0] -= unpack_lo<T>(pf[n].x); p[1] -= unpack_hi<T>(pf[n].x); p[2] -= unpack_lo<T>(pf[n].y); p[3] -= unpack_hi<T>(pf[n].y);
+            p[4] -= unpack_lo<T>(pf[n].z); p[5] -= unpack_hi<T>(pf[n].z); p[6] -= unpack_lo<T>(pf[n].w); p[7] -= unpack_hi<T>(pf[n].w);
+        }
+#pragma unroll
+        for (int d = 0; d < ND; ++d) {
+            acc[d] *= alpha;
+#pragma unroll
+            for (int n = 2; n >= 0; --n) acc[d] = WinMfma<T>::run(vf[d], pf[n], acc[d]);
+        }
+        if (i + 1 < mine) load_v(chunk(i + 1));
+    }
+    if (owner && wave == 0) {                                  // the new key: its score from the MFMA (every row of the tile is the key), its value from the row
+        f32x4 s = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int t = 0; t < NT; ++t) s = WinMfma<T>::run(frag(ks + q4 * (D / 4) + 8 * t), qf[t], s);
+        const float sn = s[0] * scl, m_new = fmaxf(m, sn);
+        const float alpha = __builtin_amdgcn_exp2f(m - m_new), pn = __builtin_amdgcn_exp2f(sn - m_new);
+        m = m_new;
+        l = l * alpha + (q4 == 0 ? pn : 0.f);
+#pragma unroll
+        for (int d = 0; d < ND; ++d) {
+            const uint2 v = *reinterpret_cast<const uint2*>(vnew + d * 16 + 4 * q4);
+            const f32x4 vv = {unpack_lo<T>(v.x), unpack_hi<T>(v.x), unpack_lo<T>(v.y), unpack_hi<T>(v.y)};
+            acc[d] = acc[d] * alpha + vv * pn;
+        }
+    }
+    // ---- the four waves, then the splits ----
+    l += __shfl_xor(l, 16, 64); l += __shfl_xor(l, 32, 64);
+    if (q4 == 0) { wm[wave * 16 + i16] = m; wl[wave * 16 + i16] = l; }
+    if (i16 < group) {
+#pragma unroll
+        for (int d = 0; d < ND; ++d) *reinterpret_cast<f32x4*>(wo + (wave * group + i16) * D + d * 16 + 4 * q4) = acc[d];
+    }
+    __syncthreads();
+    constexpr int WS = D + 4;
+    T* out = reinterpret_cast<T*>(a.out) + (size_t)z * a.out_stride + kvh * group * D;
+    auto gate = [&](int h) { return a.gate_off >= 0 ? sigmoid_f32(to_f32(row[a.gate_off + kvh * group + h])) : 1.f; };
+    for (int i = tid; i < group * D; i += 256) {
+        const int h = i / D, d = i % D;
+        float M = -INFINITY, lt = 0.f, o = 0.f;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) M = fmaxf(M, wm[w * 16 + h]);
+        const float Ms = M == -INFINITY ? 0.f : M;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            const float f = __builtin_amdgcn_exp2f(wm[w * 16 + h] - Ms);
+            lt += f * wl[w * 16 + h]; o += f * wo[(w * group + h) * D + d];
+        }
+        if (a.n_split == 1) out[i] = from_f32<T>(o * softmax_scale(lt, M, a.sink != 0) * gate(h));
+        else {
+            float* ws = e.ws + ((size_t)(kvh * group + h) * a.n_split + split) * WS;
+            __hip_atomic_store(ws + d, o, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (d == 0) {
+                __hip_atomic_store(ws + D, M, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_store(ws + D + 1, lt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        }
+    }
+    if (a.n_split == 1) return;
+    // merge by the last workgroup to arrive for this kv head (decode_win_kernel's protocol; the ticket is the group's first head's)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    int* ticket = e.counters + kvh * group;
+    if (tid == 0) flag[0] = __hip_atomic_fetch_add(ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == a.n_split - 1 ? 1.f : 0.f;
+    __syncthreads();
+    if (flag[0] == 0.f) return;
+    for (int i = tid; i < group * D; i += 256) {
+        const int h = i / D, d = i % D;
+        const float* wsh = e.ws + (size_t)(kvh * group + h) * a.n_split * WS;
+        float M = -INFINITY, lt = 0.f, o = 0.f;
+        for (int s0 = 0; s0 < a.n_split; s0 += 8) {            // eight splits' words are on their way together
+            float mi[8], li[8], oi[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const float* w = wsh + (s0 + k) * WS;
+                const bool in = s0 + k < a.n_split;
+                mi[k] = in ? __hip_atomic_load(w + D, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : -INFINITY;
+                li[k] = in ? __hip_atomic_load(w + D + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0.f;
+                oi[k] = in ? __hip_atomic_load(w + d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0.f;
+            }
+            float Mn = M;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) Mn = fmaxf(Mn, mi[k]);
+            const float Ms = Mn == -INFINITY ? 0.f : Mn, f = __builtin_amdgcn_exp2f(M - Ms);      // a split without a key of its own: (-inf, 0, 0)
+            lt *= f; o *= f;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const float fk = __builtin_amdgcn_exp2f(mi[k] - Ms);
+                lt += li[k] * fk; o += oi[k] * fk;
+            }
+            M = Mn;
+        }
+        out[i] = from_f32<T>(o * softmax_scale(lt, M, a.sink != 0) * gate(h));
+    }
+    if (tid == 0) __hip_atomic_store(ticket, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);          // re-arm for the next launch
+}
+
+// 16-bit caches of heads up to 128 wide, up to 16 query heads a kv head, more than one sequence.  32 sequences of 568 - 1300 keys, window 1024, 32 heads on 8 kv heads of 128:
+// 86.7 -> 35.9 us (3.7 TB/s) with one split (2 splits 36.4, 4 43.3: the merge and a shorter walk cost more than a fuller chip gives).  One sequence of 601 keys, 16 heads on 4:
+// 11.1 us either way, all of it latency, so the form with more workgroups stays.
+bool decode_win_grouped(int dtype, int D, int n_heads, int n_kv_heads, int n_seq) {
+    return dtype != kF32 && D <= 128 && n_heads / n_kv_heads <= WIN_GROUP_MAX && n_seq > 1;
+}
+
 void launch_decode_win(int dtype, int D, const WinDecodeArgs& a, hipStream_t st) {
     LMX_REQUIRE(D == 64 || D == 128 || D == 256, "decode_win: padded head width must be 64, 128 or 256");
     LMX_REQUIRE(a.s_max % DF_CHUNK == 0 && a.n_split >= 1 && a.n_split <= DF_MAX_SPLIT && a.n_seq >= 1, "decode_win: cache in whole 128-key chunks, 1..32 splits");
     LMX_REQUIRE(a.n_heads >= 1 && a.n_kv_heads >= 1 && a.n_heads % a.n_kv_heads == 0 && a.qkv && a.out, "decode_win: bad arguments");
     LMX_REQUIRE(a.rot_dims % 2 == 0 && a.rot_dims <= a.qk_dim && a.qk_dim <= D && (a.rot_dims == 0 || a.cos_sin), "decode_win: bad rotation");
     LMX_REQUIRE(a.tab || (a.n_seq == 1 && a.one.K && a.one.VT && a.one.ws && a.one.counters && (a.pos >= 0 || a.one.pos_ptr)), "decode_win: bad sequence");
+    if (decode_win_grouped(dtype, D, a.n_heads, a.n_kv_heads, a.n_seq) && a.qkv_stride % 4 == 0 && reinterpret_cast<uintptr_t>(a.qkv) % 8 == 0) {
+        const dim3 grid(a.n_kv_heads, a.n_split, a.n_seq);
+        const int smem = win_group_smem(a.n_heads / a.n_kv_heads, D);
+#define L(TT, DD) LMX_LAUNCH((decode_win_group_kernel<TT, DD>), grid, dim3(256), smem, st, a)
+        if (dtype == kBF16) { if (D == 128) L(bf16_t, 128); else L(bf16_t, 64); } else { if (D == 128) L(f16_t, 128); else L(f16_t, 64); }
+#undef L
+        LMX_CHECK_HIP(hipGetLastError());
+        return;
+    }
     const dim3 grid(a.n_heads, a.n_split, a.n_seq);
 #define L(TT, DD) LMX_LAUNCH((decode_win_kernel<TT, DD>), grid, dim3(256), 0, st, a)
 #define LD(TT) do { if (D == 256) L(TT, 256); else if (D == 128) L(TT, 128); else L(TT, 64); } while (0)

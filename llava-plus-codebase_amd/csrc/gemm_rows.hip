@@ -226,11 +226,29 @@ __global__ __launch_bounds__(512) void gemm_rows_kernel(GemmArgs a, int mtiles, 
         }
         return;
     }
+    const int pk_q = a.pk_kc ? a.pk_heads * a.pk_D : 0x3fffffff;        // CLIP q|k|v: the k columns leave as K rows, the v columns as V^T (GemmArgs::pk_kc)
     for (int i = tid; i < rows * (BN / 8); i += NW * 64) {
         const int m = i / (BN / 8), c = (i % (BN / 8)) * 8;
-        if (n0 + c >= a.N) continue;
+        if (n0 + c >= a.N || n0 + c >= 2 * pk_q) continue;
         float v[8]; load8<float>(tile + m * PITCH + c, v);
-        rows_store<T>(a, m0 + m, n0 + c, v);
+        if (n0 + c < pk_q) { rows_store<T>(a, m0 + m, n0 + c, v); continue; }
+        if (a.bias) {
+            float b[8]; load8<T>(static_cast<const T*>(a.bias) + n0 + c, b);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] += b[e];
+        }
+        apply_act_n<8>(v, a.act);
+        const int im = (m0 + m) / a.pk_rows, pos = m0 + m - im * a.pk_rows, kc = n0 + c - pk_q, head = kc / a.pk_D, d = kc - head * a.pk_D;
+        store8<T>(static_cast<T*>(a.pk_kc) + im * a.pk_img_stride + ((size_t)head * a.pk_spad + pos) * a.pk_D + d, v);
+    }
+    const int v0 = 2 * pk_q > n0 ? 2 * pk_q - n0 : 0, v1 = a.N - n0 < BN ? a.N - n0 : BN;
+    if (v0 >= v1) return;
+    for (int i = tid; i < rows * (v1 - v0); i += NW * 64) {               // lanes along the rows: consecutive positions of one V^T row
+        const int c = v0 + i / rows, m = i % rows;
+        float v[1] = {tile[m * PITCH + c] + (a.bias ? to_f32(static_cast<const T*>(a.bias)[n0 + c]) : 0.f)};
+        apply_act_n<1>(v, a.act);
+        const int im = (m0 + m) / a.pk_rows, pos = m0 + m - im * a.pk_rows;
+        static_cast<T*>(a.pk_vt)[im * a.pk_img_stride + (size_t)(n0 + c - 2 * pk_q) * a.pk_spad + pos] = from_f32<T>(v[0]);
     }
 }
 
@@ -308,7 +326,7 @@ static void launch_rows_n(const GemmArgs& a, int mtiles, int S, hipStream_t st) 
 bool gemm_rows_applies(int dtype, const GemmArgs& a) {
     auto al = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
     return (dtype == kBF16 || dtype == kF16) && a.K % GEMM_BK == 0 && a.N % 8 == 0 && a.ldc % 8 == 0 && al(a.C) && (!a.bias || al(a.bias)) && (!a.R || (al(a.R) && a.ldr % 8 == 0)) &&
-           (!act_gated(a.act) || a.N % 64 == 0) && !a.qf_kc && !a.pk_kc && (size_t)a.M * a.ldx * 2 < ((size_t)1 << 32) && (size_t)a.N * a.ldw * 2 < ((size_t)1 << 32);
+           (!act_gated(a.act) || a.N % 64 == 0) && !a.qf_kc && (!a.pk_kc || (a.pk_D % 8 == 0 && al(a.pk_kc) && a.pk_img_stride % 8 == 0 && !a.c_f32)) && (size_t)a.M * a.ldx * 2 < ((size_t)1 << 32) && (size_t)a.N * a.ldw * 2 < ((size_t)1 << 32);
 }
 
 size_t gemm_rows_slab_bytes(int M, int N, int S) { return S > 1 ? (size_t)S * M * N * sizeof(float) : 0; }
@@ -324,23 +342,40 @@ size_t gemm_rows_slab_bytes(int M, int N, int S) { return S > 1 ? (size_t)S * M 
 //    512   74.1 -> 64.3  34.0 (36.1)   94.3 (128.7)  91.3 -> 69.7
 // so: 64 weight rows up to 128 rows, where the weights are the time; 128 above, where the rows' re-reads are; no more than one workgroup per CU; slices of at least 10 slabs,
 // and above 128 rows no slicing of a short K (the slabs of o cost what its weights cost).  Short products (K < 1024, under 4 M weights) are launch time on any form.
+//
+// More rows (or what the slices above do not take): tiles of 32 .. 256 rows x 128 weight rows, as many as make ONE round of workgroups, where 256 x 256 tiles would be too few and
+// small tiles several rounds (us, best other form -> here; 16-bit, weights cold):
+//   2048 x 2048 x 2048  33.6 -> 23.9   1400 x 2048 x 2048  30.9 -> 20.0   2679 x 1280 x 2048  30.9 -> 22.9   600 x 4096 x 4096  40.5 -> 32.8   1087 x 4096 x 4096  51.9 -> 47.1
+//   2048 x 2048 x 5632  58.8 -> 56.6   2308 x 1024 x 4096  61.2 -> 37.0   4616 x 1024 x 4096  59.1 -> 56.9   577 x 4096 x 1024   17.3 -> 13.8   2308 x 1024 x 1024   17.9 -> 14.9
+// Not: long K under tiles of 160 rows and more (1087 x 4096 x 11008: 100.7 (116.4): three slices of 256 x 256 tiles read less), 160 and more tiles of 256 x 256, and the few small
+// tiles of 577 x 1024 and its like (7.4, 16.9 us on 64 x 64), whose time is their chain of K steps.
 RowsForm gemm_rows_form(int dtype, const GemmArgs& a) {
-    RowsForm f{0, 0, 1};
-    if (a.M > 512 || a.K < 1024 || (size_t)a.N * a.K < ((size_t)4 << 20) || !gemm_rows_applies(dtype, a)) return f;
-    const int mt = cdiv(a.M, 256), nk = a.K / GEMM_BK;
-    const bool few = a.M <= 128 && cdiv(a.N, 64) <= 256;
-    const int bn = few ? 64 : 128, tiles = mt * cdiv(a.N, bn);
-    if (tiles > 256) return f;
-    int s = std::min(256 / tiles, few ? 4 : mt == 2 ? 4 : 6);
-    while (s > 1 && (nk / s < 10 || !a.skw || gemm_rows_slab_bytes(a.M, a.N, s) > ROWS_SLAB_MAX)) --s;
-    if (tiles * s < 128 || (!few && s > 2 && nk < 128 && !(mt == 2 && a.M <= 384))) return f;
-    return RowsForm{mt, bn, s};
+    const RowsForm none{0, 0, 1};
+    if (a.K < 1024 || (size_t)a.N * a.K < ((size_t)1 << 20) || !gemm_rows_applies(dtype, a)) return none;
+    const int nk = a.K / GEMM_BK;
+    if (a.M <= 512 && (size_t)a.N * a.K >= ((size_t)4 << 20)) {
+        const int mt = cdiv(a.M, 256);
+        const bool few = a.M <= 128 && cdiv(a.N, 64) <= 256;
+        const int bn = few ? 64 : 128, tiles = mt * cdiv(a.N, bn);
+        if (tiles <= 256) {
+            int s = std::min(256 / tiles, few ? 4 : mt == 2 ? 4 : 6);
+            while (s > 1 && (nk / s < 10 || !a.skw || a.pk_kc || gemm_rows_slab_bytes(a.M, a.N, s) > ROWS_SLAB_MAX)) --s;
+            if (tiles * s >= 128 && (few || s <= 2 || nk >= 128 || (mt == 2 && a.M <= 384))) return RowsForm{mt, bn, s};
+        }
+    }
+    const int64_t t64 = (int64_t)cdiv(a.M, 64) * cdiv(a.N, 64);
+    if (a.M <= 384 || cdiv(a.M, 256) * cdiv(a.N, 256) >= 160 || t64 <= (a.K >= 2048 ? 320 : 512)) return none;
+    const int nt = cdiv(a.N, 128), fit = 256 / nt;
+    if (fit < 1 || cdiv(a.M, fit) > 256) return none;
+    const int mt = cdiv(a.M, cdiv(cdiv(a.M, fit), 32) * 32), rows32 = cdiv(cdiv(a.M, mt), 32);
+    if (mt * nt < 144 || (rows32 > 4 && nk > 64)) return none;
+    return RowsForm{mt, 128, 1};
 }
 
 
 void launch_gemm_rows(int dtype, const GemmArgs& a, int mtiles, int BN, int S, hipStream_t st) {
     LMX_REQUIRE(gemm_rows_applies(dtype, a) && mtiles >= 1 && cdiv(a.M, mtiles) <= 256 && (BN == 64 || BN == 128), "gemm_rows: shape or alignment");
-    LMX_REQUIRE(S >= 1 && S <= a.K / GEMM_BK && (S == 1 || a.skw), "gemm_rows: K slices");
+    LMX_REQUIRE(S >= 1 && S <= a.K / GEMM_BK && (S == 1 || (a.skw && !a.pk_kc)), "gemm_rows: K slices");
     // every M tile covers cdiv(rows per tile, 32) * 32 rows: the tiles that start past M are left out
     mtiles = cdiv(a.M, cdiv(cdiv(a.M, mtiles), 32) * 32);
     if (dtype == kBF16) { if (BN == 64) launch_rows_n<bf16_t, 64>(a, mtiles, S, st); else launch_rows_n<bf16_t, 128>(a, mtiles, S, st); }

@@ -45,6 +45,17 @@ def test_epilogues(cuda, variant, act):
     assert torch.equal(r, got)
 
 
+@pytest.mark.parametrize("M,N,K,res", [(385, 2048, 2048, False), (577, 4096, 1024, False), (640, 2112, 4096, True), (1087, 4096, 4096, True), (1087, 4096, 4160, True), (2308, 1024, 1024, True),
+                                       (2679, 1280, 2048, False), (4616, 1024, 1024, False), (1153, 1024, 2048, True)])
+def test_one_round_of_tiles(cuda, M, N, K, res):
+    """The other part of the rule: row tiles of a height that makes one round of workgroups."""
+    from llava_mi355x import ops
+    x, w = _mk(M, N, K, "bf16", cuda, M + N)
+    r = torch.randn(M, N, device=cuda).bfloat16() if res else None
+    ref = x.double() @ w.double().t() + (r.double() if res else 0)
+    assert_one_ulp(ops.gemm(x, w, residual=r), ref, "bf16", 2e-5 * float(ref.abs().max()), f"{M}x{N}x{K}")
+
+
 @pytest.mark.parametrize("M", [2, 32, 128, 129, 256, 257, 384, 385, 512, 513])
 @pytest.mark.parametrize("N,K,ldc", [(12288, 1024, 12288), (22016, 1024, 22016), (12288, 1024, 12292)])
 def test_rule(cuda, M, N, K, ldc):

@@ -63,6 +63,7 @@ Model::Model(const lmx_config& c) : cfg(c) {
     // a TP=1 token, 40 % of a TP=8 token if replicated); replicated when the vocabulary does not split into 8-row-aligned shards
     if (c.tp_world > 1 && V % (8 * c.tp_world) == 0) { V_l = V / c.tp_world; v_off = c.tp_rank * V_l; } else { V_l = V; v_off = 0; }
     s_max = round_up(c.max_position > 0 ? c.max_position : 2048, 128);   // decode attention works in 128-key chunks
+    kv_pitch = s_max + (c.dtype != kF32 && s_max % 256 == 0 ? 128 : 0);
     dec.resize(L);
 
     if (c.v_layers > 0) {
@@ -299,7 +300,9 @@ void Model::finalize() {
 void Model::set_rope(const float* host, int n_pos) {
     LMX_REQUIRE(host != nullptr && n_pos >= s_max, "rope table must cover max_position (rounded up to 64)");
     if (rope) { (void)hipFree(rope); rope = nullptr; }
-    LMX_CHECK_HIP(hipMalloc(reinterpret_cast<void**>(&rope), (size_t)n_pos * D * sizeof(float)));
+    const size_t rows = (size_t)std::max(n_pos, kv_pitch);               // the decode kernels clamp a position word to the cache row
+    LMX_CHECK_HIP(hipMalloc(reinterpret_cast<void**>(&rope), rows * D * sizeof(float)));
+    LMX_CHECK_HIP(hipMemset(rope, 0, rows * D * sizeof(float)));
     LMX_CHECK_HIP(hipMemcpy(rope, host, (size_t)n_pos * D * sizeof(float), hipMemcpyHostToDevice));
     rope_npos = n_pos;
 }
@@ -524,7 +527,7 @@ uint64_t next_seq_uid() { return g_seq_uid.fetch_add(1); }
 
 Seq::Seq(Model* mm) : m(mm) {
     uid = g_seq_uid.fetch_add(1);
-    layer_stride = (size_t)m->nkv_l * m->s_max * m->D * m->es;
+    layer_stride = (size_t)m->nkv_l * m->kv_pitch * m->D * m->es;
     if (m->stk) { if (m->stk->k_bytes) kc.ensure(m->stk->k_bytes, true); if (m->stk->v_bytes) vt.ensure(m->stk->v_bytes, true); if (m->stk->s_bytes) rs.ensure(m->stk->s_bytes, true); }
     else { kc.ensure(layer_stride * m->L, true); vt.ensure(layer_stride * m->L, true); }
     log_cap = m->s_max + 8;
@@ -628,22 +631,22 @@ void Model::prefill(Seq* s, const void* embeds, int T, int chunk, void* logits, 
             void *hr = rows(h, r0, H), *xr = rows(x, r0, H), *qr = rows(qkv, r0, qkv_n), *ar = rows(attn, r0, (size_t)nh_l * D);
             { LMX_PROF("prefill.rmsnorm"); launch_rmsnorm(dt, hr, w.ln1, xr, n, H, H, H, cfg.rms_eps, st); }
             // RoPE + KV-cache append ride in the q|k|v GEMM's epilogue where that launch is the un-split ping-pong kernel over head-aligned tiles
-            const bool qf = gv == 0 && opt_fuse_rope && gemm_fuses_qkv(dt, n, H, D, nh_l, nkv_l, pos0 + r0, s_max, false);
+            const bool qf = gv == 0 && opt_fuse_rope && gemm_fuses_qkv(dt, n, H, D, nh_l, nkv_l, pos0 + r0, kv_pitch, false);
             {
                 LMX_PROF_K("prefill.gemm.qkv");
                 GemmArgs g = with_scratch(GemmArgs{xr, w.wqkv, qr, nullptr, nullptr, n, qkv_n, H, H, H, qkv_n, 0, kActNone});
-                if (qf) { g.qf_rope = rope; g.qf_kc = kc; g.qf_vt = vt; g.qf_pos0 = pos0 + r0; g.qf_nh = nh_l; g.qf_nkv = nkv_l; g.qf_smax = s_max; g.qf_D = D; }
+                if (qf) { g.qf_rope = rope; g.qf_kc = kc; g.qf_vt = vt; g.qf_pos0 = pos0 + r0; g.qf_nh = nh_l; g.qf_nkv = nkv_l; g.qf_smax = kv_pitch; g.qf_D = D; }
                 launch_gemm(dt, g, gv, st);
             }
-            if (!qf) { LMX_PROF("prefill.rope_kv"); launch_rope_kv(dt, D, RopeKvArgs{qr, kc, vt, rope, nullptr, pos0 + r0, n, qkv_n, nh_l, nkv_l, s_max}, st); }
+            if (!qf) { LMX_PROF("prefill.rope_kv"); launch_rope_kv(dt, D, RopeKvArgs{qr, kc, vt, rope, nullptr, pos0 + r0, n, qkv_n, nh_l, nkv_l, kv_pitch}, st); }
             if (attn_probs) {
                 void* pl = static_cast<char*>(attn_probs) + (size_t)l * nh_l * T * kv_after * es;
-                launch_attn_probs(dt, D, AttnProbsArgs{qr, kc, pl, n, c0 + r0, T, pos0 + r0, kv_after, qkv_n, nh_l, nkv_l, s_max, scale}, st);
+                launch_attn_probs(dt, D, AttnProbsArgs{qr, kc, pl, n, c0 + r0, T, pos0 + r0, kv_after, qkv_n, nh_l, nkv_l, kv_pitch, scale}, st);
             }
             if (dt == kF32) {
-                { LMX_PROF("prefill.attn"); launch_decode_attn(dt, D, DecodeAttnArgs{qr, ar, kc, vt, nullptr, pos0 + r0, n, 0, 1, qkv_n, nh_l * D, nh_l, nkv_l, s_max, 1, scale, aws}, st); }
+                { LMX_PROF("prefill.attn"); launch_decode_attn(dt, D, DecodeAttnArgs{qr, ar, kc, vt, nullptr, pos0 + r0, n, 0, 1, qkv_n, nh_l * D, nh_l, nkv_l, kv_pitch, 1, scale, aws}, st); }
             } else {
-                { LMX_PROF("prefill.attn"); launch_flash_prefill(dt, D, FlashArgs{qr, ar, kc, vt, n, pos0 + r0 + n, pos0 + r0, qkv_n, nh_l * D, nh_l, nkv_l, s_max, scale, 1}, st); }
+                { LMX_PROF("prefill.attn"); launch_flash_prefill(dt, D, FlashArgs{qr, ar, kc, vt, n, pos0 + r0 + n, pos0 + r0, qkv_n, nh_l * D, nh_l, nkv_l, kv_pitch, scale, 1}, st); }
             }
             { LMX_PROF_K("prefill.gemm.o"); launch_gemm(dt, with_scratch(GemmArgs{ar, w.wo, hr, nullptr, lead ? hr : nullptr, n, H, nh_l * D, nh_l * D, nh_l * D, H, H, kActNone}), gv, st); }
         };
@@ -789,10 +792,10 @@ void Model::prefill_multi(Seq* const* seqs, const void* const* embeds, const int
                 void* kc = s->kc.as<char>() + (size_t)l * s->layer_stride;
                 void* vt = s->vt.as<char>() + (size_t)l * s->layer_stride;
                 void *qr = rows(qkv, g.dst0, qkv_n), *ar = rows(attn, g.dst0, (size_t)nh_l * D);
-                { LMX_PROF("prefill.rope_kv"); launch_rope_kv(dt, D, RopeKvArgs{qr, kc, vt, rope, nullptr, g.pos0, g.n, qkv_n, nh_l, nkv_l, s_max}, st); }
+                { LMX_PROF("prefill.rope_kv"); launch_rope_kv(dt, D, RopeKvArgs{qr, kc, vt, rope, nullptr, g.pos0, g.n, qkv_n, nh_l, nkv_l, kv_pitch}, st); }
                 LMX_PROF("prefill.attn");
-                if (dt == kF32) launch_decode_attn(dt, D, DecodeAttnArgs{qr, ar, kc, vt, nullptr, g.pos0, g.n, 0, 1, qkv_n, nh_l * D, nh_l, nkv_l, s_max, 1, scale, aws}, st);
-                else launch_flash_prefill(dt, D, FlashArgs{qr, ar, kc, vt, g.n, g.pos0 + g.n, g.pos0, qkv_n, nh_l * D, nh_l, nkv_l, s_max, scale, 1}, st);
+                if (dt == kF32) launch_decode_attn(dt, D, DecodeAttnArgs{qr, ar, kc, vt, nullptr, g.pos0, g.n, 0, 1, qkv_n, nh_l * D, nh_l, nkv_l, kv_pitch, 1, scale, aws}, st);
+                else launch_flash_prefill(dt, D, FlashArgs{qr, ar, kc, vt, g.n, g.pos0 + g.n, g.pos0, qkv_n, nh_l * D, nh_l, nkv_l, kv_pitch, scale, 1}, st);
             }
             { LMX_PROF_K("prefill.gemm.o"); launch_gemm(dt, with_scratch(GemmArgs{attn, w.wo, h, nullptr, lead ? h : nullptr, fill, H, nh_l * D, nh_l * D, nh_l * D, H, H, kActNone}), gv, st); }
             allreduce(h, (size_t)fill * H, st);
@@ -856,7 +859,7 @@ void Model::decode_step_launch(Seq* s, hipStream_t st, int64_t* id_out) {
         DecAttnArgs a{};
         a.qkv = s->d_qkv; a.attn = s->d_attn; a.kc = kc; a.vt = vt; a.rope = rope; a.aws = s->d_aws; a.cnt = s->d_cnt;
         // only the 128-key chunks that exist are launched: the host mirrors the position (s->len == *d_len while this step is queued)
-        a.pos = s->len; a.n_split = s->len / 128 + 1; a.nh = nh_l; a.nkv = nkv_l; a.s_max = s_max; a.scale = scale;
+        a.pos = s->len; a.n_split = s->len / 128 + 1; a.nh = nh_l; a.nkv = nkv_l; a.s_max = kv_pitch; a.scale = scale;
         a.status = s->d_status;                      // both forms: the merger's wait for the other chunks is bounded in either
         // rows [q_n, q_n + kv_n) of the fused q|k|v weight: the k | v projection of the split-q form
         const GemvArgs gkv{s->d_h, static_cast<const char*>(w.wqkv) + (size_t)q_n * H * es, nullptr, nullptr, nullptr, w.ln1, cfg.rms_eps, kv_n, H, H, H, kv_n, 0, kActNone};
@@ -871,7 +874,7 @@ void Model::decode_step_launch(Seq* s, hipStream_t st, int64_t* id_out) {
             LMX_PROF("decode.attn");
             if (attn16) launch_decode_attn_step(dt, D, a, st);
             else {
-                DecodeFusedArgs fa{s->d_qkv, kc, vt, rope, s->d_len, nh_l, nkv_l, s_max, s->len / 128 + 1, scale, s->d_aws, s->d_cnt, s->d_attn};
+                DecodeFusedArgs fa{s->d_qkv, kc, vt, rope, s->d_len, nh_l, nkv_l, kv_pitch, s->len / 128 + 1, scale, s->d_aws, s->d_cnt, s->d_attn};
                 launch_decode_fused(dt, D, fa, st);
             }
         }
@@ -897,9 +900,9 @@ void Model::seq_copy(Seq* dst, const Seq* src, hipStream_t st) {
     const size_t n = (size_t)src->len;
     if (stk) stack_seq_copy(dst, src, st);
     else {
-    // K rows [L][kv_head][s_max][D]: n * D contiguous elements per (layer, head);  V^T [L][kv_head][D][s_max]: n contiguous elements per (layer, head, d)
-    LMX_CHECK_HIP(hipMemcpy2DAsync(dst->kc.p, (size_t)s_max * D * es, src->kc.p, (size_t)s_max * D * es, n * D * es, (size_t)L * nkv_l, hipMemcpyDeviceToDevice, st));
-    LMX_CHECK_HIP(hipMemcpy2DAsync(dst->vt.p, (size_t)s_max * es, src->vt.p, (size_t)s_max * es, n * es, (size_t)L * nkv_l * D, hipMemcpyDeviceToDevice, st));
+    // K rows [L][kv_head][kv_pitch][D]: n * D contiguous elements per (layer, head);  V^T [L][kv_head][D][kv_pitch]: n contiguous elements per (layer, head, d)
+    LMX_CHECK_HIP(hipMemcpy2DAsync(dst->kc.p, (size_t)kv_pitch * D * es, src->kc.p, (size_t)kv_pitch * D * es, n * D * es, (size_t)L * nkv_l, hipMemcpyDeviceToDevice, st));
+    LMX_CHECK_HIP(hipMemcpy2DAsync(dst->vt.p, (size_t)kv_pitch * es, src->vt.p, (size_t)kv_pitch * es, n * es, (size_t)L * nkv_l * D, hipMemcpyDeviceToDevice, st));
     }
     dst->len = src->len;
     launch_set_state(dst->d_len, dst->len, dst->d_tok, 0, 0, dst->d_nout, 0, st);
@@ -1067,7 +1070,7 @@ void Model::decode_batch(Batch* b, Seq* const* seqs, int n, const int64_t* token
                 int max_len = 0;
                 for (int i = 0; i < n; ++i) max_len = std::max(max_len, seqs[i]->len);
                 // live 128-key chunks of the longest member (the host mirrors every position); shorter members' surplus workgroups only take their ticket
-                DecodeFusedArgs a{b->qkv, nullptr, nullptr, rope, nullptr, nh_l, nkv_l, s_max, max_len / 128 + 1, scale, nullptr, nullptr, b->attn};
+                DecodeFusedArgs a{b->qkv, nullptr, nullptr, rope, nullptr, nh_l, nkv_l, kv_pitch, max_len / 128 + 1, scale, nullptr, nullptr, b->attn};
                 a.tab = b->d_attn_tab + (size_t)l * b->cap; a.n_seq = n; a.qkv_stride = qkv_n; a.o_stride = nh_l * D;
                 launch_decode_fused(dt, D, a, st);
             }

@@ -105,6 +105,9 @@ struct Model {
     std::unique_ptr<Stack> stk; // set: a layer-stack decoder instead of the LLaMA decoder
     // decoder geometry (TP-local)
     int H = 0, I_l = 0, I_sh = 0, nh_l = 0, nkv_l = 0, D = 0, V = 0, L = 0, qkv_n = 0, s_max = 0;
+    // keys a cache row has room for, >= s_max.  The rows of V^T are this far apart: an odd multiple of 256 bytes for 16-bit caches, because rows a power of two apart share memory
+    // channels (a batched decode's cache stream, 16 sequences of ~800 keys: 4.9 TB/s at 2048 keys a row, 5.6 at 2176)
+    int kv_pitch = 0;
     int V_l = 0, v_off = 0;     // lm_head rows held by this rank (vocabulary-parallel head under TP) and the id of its first row
     int Vr = 0;                 // ids a pick may return (real vocabulary, lmx_set_vocab_limit); V is the padded row pitch of logits / embeddings
     // vision geometry
@@ -241,7 +244,7 @@ struct Seq {
     hipStream_t last_stream = nullptr; bool used = false;   // stream of the most recent work on this sequence (pool reuse waits for it)
     hipEvent_t ev_idle = nullptr;
     SampleParams samp;          // temperature <= 0: greedy; set by lmx_seq_set_sampling (bumps uid so a Batch re-reads it)
-    DevBuf kc, vt;              // [L][nkv_l][s_max][D] and [L][nkv_l][D][s_max]
+    DevBuf kc, vt;              // [L][nkv_l][kv_pitch][D] and [L][nkv_l][D][kv_pitch]
     DevBuf rs;                  // recurrent state of a layer-stack decoder (per run: delta states and convolution rings); nothing of it is read at position 0
     size_t pool_bytes() const { return kc.bytes + vt.bytes + rs.bytes + dws.bytes + pws.bytes; }
     size_t layer_stride = 0;    // bytes per layer in each cache

@@ -37,6 +37,7 @@ Model::Model(const lmx_stack_config& c, const lmx_layer_config* layers) {
     V = round_up(c.vocab_size, 8); Vr = c.vocab_size; V_l = V; v_off = 0;
     les = 4;
     s_max = round_up(c.max_position > 0 ? c.max_position : 2048, 128);
+    kv_pitch = s_max + (c.dtype != kF32 && s_max % 256 == 0 ? 128 : 0);
     S.layers.resize((size_t)c.n_layers);
     for (int i = 0; i < c.n_layers; ++i) {
         StackLayer& l = S.layers[(size_t)i];
@@ -84,7 +85,7 @@ Model::Model(const lmx_stack_config& c, const lmx_layer_config* layers) {
         auto up = [](size_t b) { return (b + 255) / 256 * 256; };
         StackRun r{layer, begins && !c.loop_mix && pass > 0, begins && c.loop_mix != 0, S.k_bytes, S.v_bytes, S.s_bytes, 0};
         if (l.c.mixer == LMX_MIXER_ATTENTION) {
-            const size_t bytes = up((size_t)l.c.n_kv_heads * s_max * l.D * es);
+            const size_t bytes = up((size_t)l.c.n_kv_heads * kv_pitch * l.D * es);
             S.k_bytes += bytes; S.v_bytes += bytes;
         } else if (l.c.mixer == LMX_MIXER_LATENT) S.k_bytes += up((size_t)s_max * l.R * es);
         else {
@@ -107,7 +108,9 @@ void Model::stack_set_rope(int table, int dims, const float* host, int n_pos) {
     LMX_REQUIRE(table >= 0 && table < (int)stk->rope.size() && dims > 0 && host && n_pos >= s_max, "rope table: bad index or too few positions");
     float*& p = stk->rope[(size_t)table];
     if (p) { (void)hipFree(p); p = nullptr; }
-    LMX_CHECK_HIP(hipMalloc(reinterpret_cast<void**>(&p), (size_t)n_pos * dims * sizeof(float)));
+    const size_t rows = (size_t)std::max(n_pos, kv_pitch);               // the decode kernels clamp a position word to the cache row
+    LMX_CHECK_HIP(hipMalloc(reinterpret_cast<void**>(&p), rows * dims * sizeof(float)));
+    LMX_CHECK_HIP(hipMemset(p, 0, rows * dims * sizeof(float)));
     LMX_CHECK_HIP(hipMemcpy(p, host, (size_t)n_pos * dims * sizeof(float), hipMemcpyHostToDevice));
     stk->rope_dims[(size_t)table] = dims;
 }
@@ -458,9 +461,9 @@ void Model::stack_prefill(Seq* const* seqs, const void* const* embeds, const int
                 Seq* s = seqs[g.seq];
                 void *kc = s->kc.as<char>() + S.runs[(size_t)r].k_off, *vt = s->vt.as<char>() + S.runs[(size_t)r].v_off;
                 void *qr = rows(qkv, g.dst0, l.qkv_n), *ar = rows(attn, g.dst0, l.out_k);
-                { LMX_PROF("prefill.norm_rope_kv"); launch_qkv_norm_rope_kv(dt, l.D, rope_args(S, l, qr, kc, vt, g.n, g.pos0, s_max), st); }
+                { LMX_PROF("prefill.norm_rope_kv"); launch_qkv_norm_rope_kv(dt, l.D, rope_args(S, l, qr, kc, vt, g.n, g.pos0, kv_pitch), st); }
                 LMX_PROF("prefill.attn");
-                FlashArgs fa{qr, ar, kc, vt, g.n, g.pos0 + g.n, g.pos0, l.qkv_n, l.out_k, d.n_heads, d.n_kv_heads, s_max, d.attn_scale, 1};
+                FlashArgs fa{qr, ar, kc, vt, g.n, g.pos0 + g.n, g.pos0, l.qkv_n, l.out_k, d.n_heads, d.n_kv_heads, kv_pitch, d.attn_scale, 1};
                 fa.win = 1; fa.window = d.window; fa.sink = d.softmax_sink; fa.gate = l.gate_off >= 0 ? static_cast<char*>(qr) + (size_t)l.gate_off * es : nullptr;
                 if (dt == kF32 || l.D > 128) launch_rows_attn(dt, l.D, fa, st); else launch_flash_prefill(dt, l.D, fa, st);
             }
@@ -622,7 +625,7 @@ void Model::stack_decode_step(Seq* s, hipStream_t st, int64_t* id_out) {
         top = 0;
         if (l.c.mixer == LMX_MIXER_ATTENTION) {
             LMX_PROF_K("decode.attn");
-            WinDecodeArgs a = decode_args(S, l, dt, s->d_qkv, s->d_attn, 1, s->len, s_max);
+            WinDecodeArgs a = decode_args(S, l, dt, s->d_qkv, s->d_attn, 1, s->len, kv_pitch);
             a.one = stack_seq_ref(r, s);
             a.pos = s->len;
             launch_decode_win(dt, l.D, a, st);
@@ -691,7 +694,7 @@ void Model::stack_decode_batch_step(Batch* b, Seq* const* seqs, int n, int64_t* 
         const DecodeFusedSeq* tab = b->d_attn_tab + (size_t)r * b->cap;
         if (l.c.mixer == LMX_MIXER_ATTENTION) {
             LMX_PROF("decode_batch.attn");
-            WinDecodeArgs a = decode_args(S, l, dt, b->qkv, b->attn, n, max_len, s_max);
+            WinDecodeArgs a = decode_args(S, l, dt, b->qkv, b->attn, n, max_len, kv_pitch);
             a.tab = tab;
             launch_decode_win(dt, l.D, a, st);
         } else stack_mix_decode(r, tab, DecodeFusedSeq{}, n, max_len, b->qkv, b->attn, b->sw, b, st);
@@ -730,8 +733,8 @@ void Model::stack_seq_copy(Seq* dst, const Seq* src, hipStream_t st) {
         const size_t nk = (size_t)l.c.n_kv_heads;
         if (l.c.mixer == LMX_MIXER_LATENT) LMX_CHECK_HIP(hipMemcpyAsync(dst->kc.as<char>() + r.k_off, src->kc.as<char>() + r.k_off, n * l.R * es, hipMemcpyDeviceToDevice, st));
         if (l.c.mixer != LMX_MIXER_ATTENTION) continue;
-        LMX_CHECK_HIP(hipMemcpy2DAsync(dst->kc.as<char>() + r.k_off, (size_t)s_max * l.D * es, src->kc.as<char>() + r.k_off, (size_t)s_max * l.D * es, n * l.D * es, nk, hipMemcpyDeviceToDevice, st));
-        LMX_CHECK_HIP(hipMemcpy2DAsync(dst->vt.as<char>() + r.v_off, (size_t)s_max * es, src->vt.as<char>() + r.v_off, (size_t)s_max * es, n * es, nk * l.D, hipMemcpyDeviceToDevice, st));
+        LMX_CHECK_HIP(hipMemcpy2DAsync(dst->kc.as<char>() + r.k_off, (size_t)kv_pitch * l.D * es, src->kc.as<char>() + r.k_off, (size_t)kv_pitch * l.D * es, n * l.D * es, nk, hipMemcpyDeviceToDevice, st));
+        LMX_CHECK_HIP(hipMemcpy2DAsync(dst->vt.as<char>() + r.v_off, (size_t)kv_pitch * es, src->vt.as<char>() + r.v_off, (size_t)kv_pitch * es, n * es, nk * l.D, hipMemcpyDeviceToDevice, st));
     }
     if (stk->s_bytes) LMX_CHECK_HIP(hipMemcpyAsync(dst->rs.p, src->rs.p, stk->s_bytes, hipMemcpyDeviceToDevice, st));
     if (stk->ids_in()) launch_set_prev(dst->d_prev, nullptr, src->d_prev, st);

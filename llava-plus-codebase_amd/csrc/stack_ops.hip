@@ -698,8 +698,9 @@ __global__ __launch_bounds__(256) void decode_win_group_kernel(WinDecodeArgs a) 
 #pragma unroll
         for (int d = 0; d < ND; ++d) vf[d] = *reinterpret_cast<const uint4*>(p + (size_t)d * 16 * a.s_max);
     };
-    // this split's chunks, from a place of its own on: in step, all workgroups would read the same columns of their V^T rows, which lie a power of two apart
-    const int mine = c1 - c0 < split ? 0 : (c1 - c0 - split) / a.n_split + 1, rot = mine ? (int)((kvh * 5u + z * 3u) % (unsigned)mine) : 0;
+    // this split's chunks, from a place of the head's own on: in step, all workgroups would read the same columns of their V^T rows, which lie a power of two apart (not of the
+    // sequence's own: a request's result must not depend on its place in the batch)
+    const int mine = c1 - c0 < split ? 0 : (c1 - c0 - split) / a.n_split + 1, rot = mine ? (int)((kvh * 5u) % (unsigned)mine) : 0;
     auto chunk = [&](int i) { i += rot; i = i < mine ? i : i - mine; return c0 + split + i * a.n_split; };
     if (mine) { load_k(chunk(0)); load_v(chunk(0)); }
     for (int h = wave; h < group + (owner ? 1 : 0); h += 4) {  // the query heads, then the new key

@@ -431,12 +431,12 @@ int lmx_profile_read(lmx_model* m, char* names_buf, int32_t names_cap, double* m
 // decode-batch kernel on the fragment-order copy of w (tests: variant 21 = copy made on every call; microbenchmarks: 22 = copy cached per
 // (pointer, N, K) — only valid while that weight tensor is alive and unchanged); 20 = the [N][K] layout as it is
 static void skinny_op(int32_t dtype, GemmArgs g, int32_t variant, hipStream_t st) {
-    // 23 / 24 = 22 / 21 with the K-slices-across-workgroups form's scratch (narrow layers, more than 8 rows: skinny_kslices)
+    // 23 / 24 = 22 / 21 with the K-slices-across-workgroups form's scratch (narrow layers)
     if (variant == 23 || variant == 24) {
         static std::mutex mu2;
         static DevBuf sk_scratch, sk_cnt;
         std::lock_guard<std::mutex> lk(mu2);
-        const size_t need = skinny_scratch_bytes(g.N), ncnt = (size_t)(g.N / 64 + 1) * sizeof(int);
+        const size_t need = skinny_scratch_bytes(g.N), ncnt = (size_t)(g.N / 16 + 1) * sizeof(int);
         if (sk_scratch.bytes < need || sk_cnt.bytes < ncnt) { LMX_CHECK_HIP(hipDeviceSynchronize()); sk_scratch.ensure(need); sk_cnt.ensure(ncnt, true); }
         g.skw = sk_scratch.p; g.sk_cnt = sk_cnt.as<int>();
         variant = variant == 23 ? 22 : 21;

@@ -973,9 +973,8 @@ Batch::Batch(Model* mm, int capacity) : m(mm), cap(capacity) {
     if (m->stk) { y = W + o_y; xr = reinterpret_cast<float*>(W + o_xr); sw = m->stk->ws(W + o_sw, cap, m->H, es, true); }
     const size_t attn_bytes = sizeof(DecodeFusedSeq) * (size_t)m->L * cap, state_bytes = sizeof(SeqStateRef) * (size_t)cap;
     tab.ensure(attn_bytes + state_bytes, true);
-    if (m->cfg.dtype != kF32) {                     // K-sliced linears of a decode batch: o_proj / down_proj (N = H) and q|k|v
-        const int nmax = std::max(std::max(m->H, m->qkv_n), m->stk ? m->stk->q_n : 0);
-        sk_scratch.ensure(skinny_scratch_bytes(nmax)); sk_cnt.ensure((size_t)(nmax / 64 + 1) * sizeof(int), true);
+    if (m->cfg.dtype != kF32) {                     // K-sliced linears of a decode batch: any narrower than SKINNY_SLICED_N
+        sk_scratch.ensure(skinny_scratch_bytes(SKINNY_SLICED_N)); sk_cnt.ensure((size_t)(SKINNY_SLICED_N / 16 + 1) * sizeof(int), true);
     }
     d_attn_tab = tab.as<DecodeFusedSeq>();
     d_state_tab = reinterpret_cast<SeqStateRef*>(tab.as<char>() + attn_bytes);

@@ -9,8 +9,10 @@
 //   * A operand = weights: lane (i = lane & 15, q = lane >> 4) owns row n0+i and, per "super-step" of 128 k, the 64
 //     contiguous bytes k0 + 32q .. +32  (four 16-byte loads = the A fragments of four MFMA steps).  A wave
 //     therefore touches 16 rows × 256 contiguous bytes per super-step: whole 128-byte lines, no LDS staging, no swizzle.
-//   * B operand = activations: lane (t = lane & 15, q) owns token t and the SAME k bytes of x — the MFMA's k order is
-//     arbitrary as long as A and B agree, so the permuted k order costs nothing.  x is M·K·2 B ≤ 0.7 MB: L2-resident.
+//   * B operand = activations: lane (t = lane & 15, q) owns token t and the SAME k bytes of x.  x is M·K·2 B ≤ 0.7 MB: L2-resident, read again by every workgroup, and 16 B out of
+//     64 different places per load instruction cost more than its bytes: with the fragment-order copy a wave loads x in whole 256-byte pieces of four rows and turns
+//     them round in wave-private LDS (XOR-swizzled 16-byte chunks, no barrier).  Plain lane-owned loads: 22016 x 4096 gated at 16 / 32 rows 36.6 / 45.0 -> 32.2 / 36.8 us,
+//     12288 x 4096 24.2 / 29.7 -> 22.6 / 26.1, 4096 x 11008 23.0 / 25.9 -> 20.0 / 23.3, 4096 x 4096 13.3 / 16.2 -> 11.4 / 13.0.
 //   * the NW waves of a workgroup split K (wave w takes super-steps w, w+NW, ...: concurrent loads of a row are adjacent)
 //     and reduce their partial C tiles through LDS in fixed wave order — deterministic, no atomics.
 //   * from the [N][K] layout every 16-lane group of such a load touches 16 different rows; the engine therefore keeps a second copy of
@@ -66,7 +68,8 @@ __device__ __forceinline__ void ba_store16_wt(__amdgpu_buffer_rsrc_t rs, uint32_
 template <typename T, int NW, int RT, int CT, bool SWZ = false, bool STREAM = false>
 __global__ __launch_bounds__(NW * 64) void skinny_gemm_kernel(GemmArgs a) {
     static_assert(!STREAM || SWZ, "the hand-counted stream reads the fragment-order copy");
-    __shared__ float red[NW][RT * CT][256];
+    // a wave's partial tiles; with STREAM before that the wave's 128-k piece of x on its way from row order to the operand's order (wave-private: no barrier)
+    __shared__ __attribute__((aligned(16))) float red[NW][STREAM && RT < 4 ? 4 * CT : RT * CT][256];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int i = lane & 15, q = lane >> 4;
@@ -150,14 +153,19 @@ __global__ __launch_bounds__(NW * 64) void skinny_gemm_kernel(GemmArgs a) {
         static_assert(LPS <= 63, "vmcnt is a 6-bit field");
         const int wave_u = __builtin_amdgcn_readfirstlane(wave);
         const ws_v4i rsW = ws_make_rsrc(a.Wsw, 0x7fffffffu), rsX = ws_make_rsrc(a.X, 0x7fffffffu);
-        uint32_t wvo[RT], xvo[CT];
+        uint32_t wvo[RT], xvo[CT][4];
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) wvo[rt] = (uint32_t)(rowbase[rt] >> 4) * (uint32_t)nsuper * 4096u + (uint32_t)lane * 16u;
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct) {
-            int m = ct * 16 + i; m = m < a.M ? m : a.M - 1;                    // rows past M: a real row's bytes — their output columns are never stored
-            xvo[ct] = (uint32_t)m * (uint32_t)a.ldx * (uint32_t)sizeof(T) + (uint32_t)q * 64u;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int t = 4 * j + q;
+                int m = ct * 16 + t; m = m < a.M ? m : a.M - 1;                // rows past M: a real row's bytes — their output columns are never stored
+                xvo[ct][j] = (uint32_t)m * (uint32_t)a.ldx * (uint32_t)sizeof(T) + (uint32_t)(i ^ t) * 16u;
+            }
         }
+        char* xl = reinterpret_cast<char*>(&red[wave][0][0]);
         auto issue = [&](Stage& s, int r) {                  // round r of this wave = super-step s_lo + wave + r NW
             const int sup = s_lo + wave_u + r * NW;
             const uint32_t wo = (uint32_t)sup * 4096u, xo = (uint32_t)sup * (uint32_t)(SK_SUPER * sizeof(T));
@@ -168,7 +176,7 @@ __global__ __launch_bounds__(NW * 64) void skinny_gemm_kernel(GemmArgs a) {
 #pragma unroll
             for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) ws_load_plain(s.x[ct][j], xvo[ct], rsX, xo + (uint32_t)j * 16u);
+                for (int j = 0; j < 4; ++j) ws_load_plain(s.x[ct][j], xvo[ct][j], rsX, xo);
         };
         auto landed = [&](Stage& s, bool younger) {          // younger: the other stage's LPS loads may stay on the wire; the stage's registers pass through: no use above
             if (younger) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LPS) : "memory"); else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -181,17 +189,30 @@ __global__ __launch_bounds__(NW * 64) void skinny_gemm_kernel(GemmArgs a) {
 #pragma unroll
                 for (int j = 0; j < 4; ++j) asm volatile("" : "+v"(s.x[ct][j]));
         };
+        auto consume_x = [&](Stage& s) {                     // row order -> lane (i, q) holds 16-byte chunks 4 q + j of row i
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) *reinterpret_cast<u32x4_s*>(xl + ct * 4096 + j * 1024 + lane * 16) = s.x[ct][j];
+            asm volatile("" ::: "memory");                   // the wave's LDS operations retire in order; the compiler must not turn them round either
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) s.x[ct][j] = *reinterpret_cast<const u32x4_s*>(xl + ct * 4096 + i * 256 + ((4 * q + j) ^ i) * 16);
+            asm volatile("" ::: "memory");
+            consume(s);
+        };
         // this wave's share: rounds 0 .. nr - 1 (wave-uniform); no load is issued past it, so every count below is exact without dummy loads
         const int nr = s_lo + wave_u < s_hi ? (s_hi - s_lo - wave_u + NW - 1) / NW : 0;
         if (nr > 0) issue(sa, 0);
         if (nr > 1) issue(sb, 1);
         for (int r = 0; r < nr; r += 2) {
             landed(sa, r + 1 < nr);
-            consume(sa);
+            consume_x(sa);
             if (r + 2 < nr) issue(sa, r + 2);
             if (r + 1 < nr) {
                 landed(sb, r + 2 < nr);
-                consume(sb);
+                consume_x(sb);
                 if (r + 3 < nr) issue(sb, r + 3);
             }
         }
@@ -292,52 +313,49 @@ __global__ __launch_bounds__(NW * 64) void skinny_gemm_kernel(GemmArgs a) {
     }
 }
 
-// K slices across workgroups for the 64-rows-per-workgroup form of a narrow layer: enough workgroups for every CU and a LONG K (each of a slice's 8 waves keeps at
-// least two super-steps).  Measured at 32 rows, 7B (profiles/r06_skinny_kslices.jsonl): down_proj (K = 11008) 31.4 -> 23.0 us with 4 slices (3: 24.7, 2: 30.6, 8: 26.8),
-// 16 rows 23.8 -> 20.7; o_proj (K = 4096) 13.7 -> 13.3 (4 slices) / 12.8 (2 slices of 32 rows): a slice of 8 super-steps is one per wave — not worth a hand-over.
-int skinny_kslices(int M, int N, int K) {
-    if (M <= 8 || N % 64 != 0) return 1;
-    const int tiles = N / 64, nsuper = cdiv(K, SK_SUPER);
-    int ks = cdiv(256, tiles);
-    if (ks > 4) ks = 4;
-    while (ks > 1 && nsuper / ks < 16) --ks;
-    return tiles * ks >= 192 ? ks : 1;              // fewer slices than fill the chip: the 16-rows-per-workgroup form (256 workgroups) is the better one
+size_t skinny_scratch_bytes(int N) { return (size_t)cdiv(N, 64) * 8 * (4 * 2 * 256) * sizeof(float); }      // at most N / 16 row tiles x 4 slices x 2 token tiles of 256 sums
+
+// Row tiles per workgroup and K slices of a linear.  What a form costs is its weight stream, made longer by the x rows that every workgroup reads again (CT / RT of the weights, a
+// quarter of the price of as many weight bytes: they come from L2), by workgroups that do not divide evenly over the 256 CUs (less than in proportion: the CUs that are
+// done leave their bandwidth to the others), and by the hand-over between slices (about 2.5 us for two, 5 for four).  us at 16 / 32 rows, RT x slices, events' 2 us included:
+//   22016 x 4096 gated  2: 32.3 / 36.8   4: 36.8 / 42.8      4096 x 11008  1: 20.0 / 25.3   2 x 2: 20.5 / 23.3   4 x 4: 21.5 / 24.2
+//   27648 x 5120 gated  2: 52.7 / 61.2   4: 49.8 / 58.1      4096 x  4096  1: 11.4 / 13.0   2 x 2: 12.7 / 13.8
+//   12288 x 4096  1: 23.6 / 29.9   2: 25.0 / 28.3   4: 22.8 / 26.1       6208 x 4096  1: 16.9 / 19.3   2: 15.1 / 18.8   4 x 2: 16.4 / 18.1
+struct SkinnyForm { int rt, ks; };
+static SkinnyForm skinny_form(const GemmArgs& a) {
+    const bool gated = act_gated(a.act), slices = !gated && a.skw && a.sk_cnt && a.N % 64 == 0 && a.N < SKINNY_SLICED_N;
+    const int ct = a.M > 16 ? 2 : 1, nsuper = cdiv(a.K, SK_SUPER);
+    const double weights = (double)a.N * a.K / (4096.0 * 11008.0);
+    SkinnyForm best{gated ? 2 : 1, 1};
+    double least = 1e30;
+    for (int rt = 4; rt >= (gated ? 2 : 1); rt /= 2) {
+        if (a.N % (16 * rt) != 0 && rt > 1) continue;                   // the fragment-order copy ends with the last 16 rows
+        const int tiles = cdiv(a.N, 16 * rt);
+        for (int ks = 1; ks <= (slices ? 4 : 1); ks *= 2) {
+            if (ks > 1 && nsuper / ks < 8) break;                       // two super-steps for each of a slice's waves
+            const double even = (double)tiles * ks / (256.0 * cdiv(tiles * ks, 256));
+            const double cost = (1 + 0.25 * ct / rt) * (1 + 0.42 * (1 / even - 1)) * (1 + (ks == 1 ? 0.0 : ks == 2 ? 0.15 : 0.30) / weights);
+            if (cost < least) { least = cost; best = SkinnyForm{rt, ks}; }
+        }
+    }
+    return best;
 }
-size_t skinny_scratch_bytes(int N) { return (size_t)cdiv(N, 64) * 8 * (4 * 2 * 256) * sizeof(float); }      // tiles x max slices x (RT 4 x CT 2) accumulator blocks
 
 template <typename T, bool SWZ>
 static void launch_skinny_s(const GemmArgs& a, hipStream_t st) {
-    constexpr int NW = 8;
-    const bool silu = act_gated(a.act);
-    const int ct = a.M > 16 ? 2 : 1;
+    const SkinnyForm f = skinny_form(a);
+    const dim3 grid(cdiv(a.N, 16 * f.rt), f.ks);
+    constexpr int NW = 4;                                               // eight waves: 2 - 10 % slower above 16 rows, equal below
     // the fragment-order copy with whole 128-k super-steps takes the hand-counted load stream; same tile forms, same bits
     const bool stream = SWZ && a.K % SK_SUPER == 0;
-    auto go = [&](auto rt_c, auto ct_c, int grid, int ks = 1) {
+    auto go = [&](auto rt_c, auto ct_c) {
         constexpr int RTV = decltype(rt_c)::value, CTV = decltype(ct_c)::value;
-        if constexpr (SWZ) { if (stream) { hipLaunchKernelGGL((skinny_gemm_kernel<T, NW, RTV, CTV, true, true>), dim3(grid, ks), dim3(NW * 64), 0, st, a); return; } }
-        hipLaunchKernelGGL((skinny_gemm_kernel<T, NW, RTV, CTV, SWZ, false>), dim3(grid, ks), dim3(NW * 64), 0, st, a);
+        if constexpr (SWZ) { if (stream) { hipLaunchKernelGGL((skinny_gemm_kernel<T, NW, RTV, CTV, true, true>), grid, dim3(NW * 64), 0, st, a); return; } }
+        hipLaunchKernelGGL((skinny_gemm_kernel<T, NW, RTV, CTV, SWZ, false>), grid, dim3(NW * 64), 0, st, a);
     };
     using I1 = std::integral_constant<int, 1>; using I2 = std::integral_constant<int, 2>; using I4 = std::integral_constant<int, 4>;
-    if (silu) {
-        // more than 16 token rows: x re-reads from L2 rival the weight stream, so a workgroup takes a whole 64-row fused block
-        if (ct == 2 && a.N >= 16384) go(I4{}, I2{}, a.N / 64);
-        else if (ct == 1) go(I2{}, I1{}, a.N / 2 / 16);
-        else go(I2{}, I2{}, a.N / 2 / 16);
-    } else if (a.N % 64 == 0 && a.N >= 8192 && ct == 2) {
-        // (two K slices for q|k|v's 192 tiles — 384 workgroups of 384 KB instead of 192 of 768 KB — measured SLOWER: 25.2 -> 29.1 us at 32 rows, r6-G)
-        go(I4{}, I2{}, a.N / 64);
-    } else if (a.N % 32 == 0 && a.N >= 8192) {
-        // wide layers: two row tiles per workgroup halve the x re-reads; narrow ones keep one tile for more workgroups
-        if (ct == 1) go(I2{}, I1{}, a.N / 32); else go(I2{}, I2{}, a.N / 32);
-    } else if (a.skw && a.sk_cnt && a.N % 64 == 0 && skinny_kslices(a.M, a.N, a.K) > 1) {
-        // narrow layers with scratch: 64 rows per workgroup (a quarter of the x re-reads) and K slices across workgroups to fill the chip
-        const int ks = skinny_kslices(a.M, a.N, a.K);
-        if (ct == 1) go(I4{}, I1{}, a.N / 64, ks); else go(I4{}, I2{}, a.N / 64, ks);
-    } else {
-        // narrow layers (N = hidden): 16 rows per workgroup — with only N/16 = 256 workgroups parallelism matters more than x re-reads
-        // (32 / 64 rows per workgroup measured 21.5 / 29.6 us vs 16.7 us on o_proj at M = 32)
-        if (ct == 1) go(I1{}, I1{}, cdiv(a.N, 16)); else go(I1{}, I2{}, cdiv(a.N, 16));
-    }
+    auto rows = [&](auto rt_c) { if (a.M > 16) go(rt_c, I2{}); else go(rt_c, I1{}); };
+    if (f.rt == 4) rows(I4{}); else if (f.rt == 2) rows(I2{}); else rows(I1{});
     LMX_CHECK_HIP(hipGetLastError());
 }
 

@@ -11,6 +11,7 @@
 // norm divides by the true width.
 #include "common.h"
 #include "kernels.h"
+#include "attention_batch.h"
 #include "attention_decode.h"
 
 namespace lmx {
@@ -639,10 +640,11 @@ __global__ __launch_bounds__(256) void decode_win_kernel(WinDecodeArgs a) {
 }
 
 // The same launch for 16-bit models with head widths up to 128: one workgroup per (kv head, split, sequence) serves ALL query heads of the kv head on MFMA tiles, so a cached
-// key and value leaves memory once instead of once per query head.  A wave takes 32 of a 128-key chunk (no barrier inside the walk): scores = K tile (16 keys, straight from the
-// cache rows into the MFMA operand) x query heads (16 columns), the softmax over the lane's 8 keys and 4 lanes, then V^T rows x probabilities.  The C layout of the scores
-// (lane = head, 4 rows a tile) is the B layout of the probabilities when row 4 q + r of tile t is key 8 q + 4 t + r, so no value changes lanes.  Probabilities
-// stay exact to 24 bits: three 16-bit terms, three MFMAs.  Bound: the cache stream (32 sequences x 1024 keys, 8 kv heads of 128: 134 MB a launch); figures: decode_win_grouped.
+// key and value leaves memory once instead of once per query head.  A wave walks 64-key pieces (no barrier inside the walk): keys and V^T rows come in whole lines (16 loads of
+// 1 KiB each, marked streaming) and reach the operands' order through 16 KiB of wave-private LDS, chunks XOR-swizzled; the next piece is requested as soon as this one is in LDS.
+// Scores = K tile (16 keys) x query heads (16 columns), the softmax over the lane's 16 keys and 4 lanes, then V^T rows x probabilities.  The C layout of the scores (lane = head,
+// 4 rows a tile) is the B layout of the probabilities when row 4 q + r of tile t is key 8 q + 4 t + r of 32, so no probability changes lanes.  Probabilities stay exact to 24
+// bits: three 16-bit terms, three MFMAs.  Bound: the cache stream (32 sequences x 1024 keys, 8 kv heads of 128: 134 MB a launch); figures: decode_win_grouped.
 template <typename T> struct WinMfma;
 template <> struct WinMfma<bf16_t> {
     static __device__ __forceinline__ f32x4 run(const uint4& a, const uint4& b, f32x4 c) {
@@ -655,66 +657,71 @@ template <> struct WinMfma<f16_t> {
     }
 };
 constexpr int WIN_GROUP_MAX = 16;                              // query heads of a kv head: the columns of a tile
-static int win_group_smem(int group, int D) { return (group * D + 5 * D + 4 * group * D + 2 * 4 * 16 + 8) * (int)sizeof(float); }
+// q heads, new key, one row of scratch per wave | the waves' partial rows [wave][head][D], statistics | the waves' tiles (the partial rows take their place after the walk)
+static int win_group_smem(int group, int D) { return ((group + 5) * D + 2 * 4 * 16 + 8 + std::max(4 * 64 * D / 2, 4 * group * D)) * (int)sizeof(float); }
 
 template <typename T, int D>
 __global__ __launch_bounds__(256) void decode_win_group_kernel(WinDecodeArgs a) {
     extern __shared__ __attribute__((aligned(16))) float wsm[];
     const int group = a.n_heads / a.n_kv_heads;
-    float *qs = wsm, *ks = qs + group * D, *tmp = ks + D, *wo = tmp + 4 * D, *wm = wo + 4 * group * D, *wl = wm + 64, *flag = wl + 64;      // wo: [wave][head][D]
+    float *qs = wsm, *ks = qs + group * D, *tmp = ks + D, *wm = tmp + 4 * D, *wl = wm + 64, *flag = wl + 64, *wo = flag + 8;      // wo: [wave][head][D] after the walk, [wave] tiles of 64 keys before
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int i16 = lane & 15, q4 = lane >> 4;
     const int kvh = blockIdx.x, split = blockIdx.y, z = blockIdx.z;
     const DecodeFusedSeq e = a.tab ? a.tab[z] : a.one;
     int pos = a.pos >= 0 ? a.pos : *e.pos_ptr;
-    pos = pos < a.s_max ? pos : a.s_max - 1;
+    pos = __builtin_amdgcn_readfirstlane(pos < a.s_max ? pos : a.s_max - 1);
     const int lo = a.window > 0 && pos - a.window + 1 > 0 ? pos - a.window + 1 : 0;
-    const int c0 = lo / DF_CHUNK, c1 = pos / DF_CHUNK;
+    const int p0 = lo / 64, np = (pos + 63) / 64 - p0;         // 64-key pieces with a cached key that is seen (np <= 0: none); split's wave w takes 4 split + w, + 4 n_split, ...
     const T* row = reinterpret_cast<const T*>(a.qkv) + (size_t)z * a.qkv_stride;
     T* Kc = reinterpret_cast<T*>(e.K) + (size_t)kvh * a.s_max * D;
     T* Vt = reinterpret_cast<T*>(e.VT) + (size_t)kvh * D * a.s_max;
     const T* vnew = row + (a.n_heads + a.n_kv_heads + kvh) * D;
     const float* cs = a.cos_sin + (size_t)pos * a.rot_dims;
-    const bool owner = (c1 - c0) % a.n_split == split;         // this workgroup takes the new key
+    const bool owner = split == a.n_split - 1;                 // this workgroup takes the new key
     constexpr int NT = D / 32, ND = D / 16;                    // 32-deep steps of a score, 16-row tiles of V^T
     const float scl = a.scale * 1.4426950408889634f;
 
-    // contraction step t of a score: lane group q4 holds dimensions q4 D / 4 + 8 t .. + 7, so a key row leaves in 16-byte pieces of one contiguous quarter per lane
-    // the next chunk's keys are requested when this one's are in the scores, its values when this one's are in the sums (past the last chunk of the split: the last one again,
-    // no branch around the loads).  Two whole chunks in registers are slower: the walk's code doubles, and a launch this short waits for its instructions
-    uint4 kf[2][NT], vf[ND];
-    auto load_k = [&](int c) {
-        const int base = c * DF_CHUNK + wave * 32;
+    // piece loads: instruction u brings 1 KiB = whole key rows (K) or 8 V^T rows of 64 keys; lane l's 16 bytes land at l 16 of the tile's KiB u, so the chunk it fetches is the swizzled one
+    constexpr int NL = D / 8, CPR = D / 8;                     // loads a tile; 16-byte chunks of a key row
+    char* tile = reinterpret_cast<char*>(wo) + wave * 64 * D * 2;
+    const int krow = lane / CPR, kch = lane % CPR, vrow = lane >> 3, vch = lane & 7;
+    auto kswz = [](int row) { return ((row & 3) | (row >> 1 & 12)) & (CPR - 1); };      // the 16 rows a fragment read takes are 8 a + 4 t + b: distinct
+    uint32_t k_lane[NL];                                       // u-dependent only through the swizzle; the row offsets are whole KiB
 #pragma unroll
-        for (int t2 = 0; t2 < 2; ++t2) {
-            int key = base + 8 * (i16 >> 2) + 4 * t2 + (i16 & 3);
-            key = key < pos ? key : (pos > 0 ? pos - 1 : 0);   // rows past the cached keys re-read the last one; their scores are dropped
-#pragma unroll
-            for (int t = 0; t < NT; ++t) kf[t2][t] = *reinterpret_cast<const uint4*>(Kc + (size_t)key * D + q4 * (D / 4) + 8 * t);
-        }
+    for (int u = 0; u < NL; ++u) { const int row = u * (64 / CPR) + krow; k_lane[u] = (uint32_t)((krow * CPR + (kch ^ kswz(row))) * 16); }
+    const uint32_t v_lane = ((uint32_t)vrow * (uint32_t)a.s_max) * 2u + (uint32_t)((vch ^ (vrow >> 1)) * 16);      // rows 8 u + vrow: (row >> 1) & 7 = 4 (u & 1) + (vrow >> 1)
+    uint4 kr[NL], vr[NL];
+    auto view = [](const T* p, bool on) {                      // the table's words come by vector loads: as they are, every buffer load would loop over the lanes' views
+        const uint64_t v = reinterpret_cast<uint64_t>(p);
+        return ba_rsrc(reinterpret_cast<const void*>((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)v) | (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32), on);
     };
-    auto load_v = [&](int c) {
-        const T* p = Vt + (size_t)i16 * a.s_max + c * DF_CHUNK + wave * 32 + 8 * q4;
+    auto load_k = [&](int p, bool on) {                        // a piece that is not there: an empty view, no traffic and no branch around the loads
+        const __amdgpu_buffer_rsrc_t rs = view(Kc, on);
 #pragma unroll
-        for (int d = 0; d < ND; ++d) vf[d] = *reinterpret_cast<const uint4*>(p + (size_t)d * 16 * a.s_max);
+        for (int u = 0; u < NL; ++u) kr[u] = __builtin_bit_cast(uint4, ba_ld16<true>(rs, k_lane[u], (uint32_t)((p * 64) * D * 2 + u * 1024)));
     };
-    // this split's chunks, from a place of the head's own on: in step, all workgroups would read the same columns of their V^T rows, which lie a power of two apart (not of the
-    // sequence's own: a request's result must not depend on its place in the batch)
-    const int mine = c1 - c0 < split ? 0 : (c1 - c0 - split) / a.n_split + 1, rot = mine ? (int)((kvh * 5u) % (unsigned)mine) : 0;
-    auto chunk = [&](int i) { i += rot; i = i < mine ? i : i - mine; return c0 + split + i * a.n_split; };
-    if (mine) { load_k(chunk(0)); load_v(chunk(0)); }
+    auto load_v = [&](int p, bool on) {
+        const __amdgpu_buffer_rsrc_t rs = view(Vt, on);
+#pragma unroll
+        for (int u = 0; u < NL; ++u) vr[u] = __builtin_bit_cast(uint4, ba_ld16<true>(rs, v_lane ^ (u & 1 ? 64u : 0u), (uint32_t)(8 * u) * (uint32_t)a.s_max * 2u + (uint32_t)p * 128u));
+    };
+    auto to_lds = [&](const uint4 (&r)[NL]) {
+#pragma unroll
+        for (int u = 0; u < NL; ++u) *reinterpret_cast<uint4*>(tile + u * 1024 + lane * 16) = r[u];
+        asm volatile("" ::: "memory");                         // the wave's LDS operations retire in order; the compiler must not turn them round either
+    };
+    const int first = 4 * split + wave, step = 4 * a.n_split;
+    load_k(p0 + first, first < np);
+    asm volatile("" ::: "memory");                             // keys before values: the order of the walk
+    load_v(p0 + first, first < np);
+    asm volatile("" ::: "memory");
     for (int h = wave; h < group + (owner ? 1 : 0); h += 4) {  // the query heads, then the new key
         const bool isk = h == group;
         norm_rope_vec<T, D>(row + (isk ? a.n_heads + kvh : kvh * group + h) * D, reinterpret_cast<const T*>(isk ? a.k_norm : a.q_norm), a.eps, a.qk_dim, cs, a.rot_dims, tmp + wave * D,
                             qs + h * D, lane);
     }
     __syncthreads();
-    if (owner) {
-        for (int d = tid; d < D; d += 256) {
-            Kc[(size_t)pos * D + d] = from_f32<T>(ks[d]);
-            Vt[(size_t)d * a.s_max + pos] = vnew[d];
-        }
-    }
     auto frag = [&](const float* v) -> uint4 {                 // 8 consecutive fp32 values that are 16-bit ones already
         float x[8]; load8<float>(v, x);
         return uint4{pack2<T>(x[0], x[1]), pack2<T>(x[2], x[3]), pack2<T>(x[4], x[5]), pack2<T>(x[6], x[7])};
@@ -727,58 +734,78 @@ __global__ __launch_bounds__(256) void decode_win_group_kernel(WinDecodeArgs a) 
     f32x4 acc[ND];                                             // [16 d + 4 q4 + r][head i16]
 #pragma unroll
     for (int d = 0; d < ND; ++d) acc[d] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int i = 0; i < mine; ++i) {
-        const int c = chunk(i), base = c * DF_CHUNK + wave * 32;
-        f32x4 s[2];
+    for (int i = first; i < np; i += step) {
+        const int base = (p0 + i) * 64;
+        to_lds(kr);
+        load_k(p0 + i + step, i + step < np);
+        f32x4 s[4];                                            // [2 h + t]: keys 32 h + 8 q4 + 4 t + r
 #pragma unroll
-        for (int t2 = 0; t2 < 2; ++t2) {
-            s[t2] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int g = 0; g < 4; ++g) {
+            s[g] = f32x4{0.f, 0.f, 0.f, 0.f};
+            const int row = 32 * (g >> 1) + 8 * (i16 >> 2) + 4 * (g & 1) + (i16 & 3);
 #pragma unroll
-            for (int t = 0; t < NT; ++t) s[t2] = WinMfma<T>::run(kf[t2][t], qf[t], s[t2]);
+            for (int t = 0; t < NT; ++t)
+                s[g] = WinMfma<T>::run(*reinterpret_cast<const uint4*>(tile + row * D * 2 + (((q4 * NT + t) ^ kswz(row)) * 16)), qf[t], s[g]);
         }
-        if (i + 1 < mine) load_k(chunk(i + 1));
-        const bool edge = base < lo || base + 32 > pos;        // some of the wave's keys are outside: their scores are dropped and their values, whatever they hold, cleared
+        const bool edge = base < lo || base + 64 > pos;        // some of the piece's keys are outside: their scores are dropped and their values, whatever they hold, cleared
         float mx = -INFINITY;
 #pragma unroll
-        for (int t2 = 0; t2 < 2; ++t2)
+        for (int g = 0; g < 4; ++g)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int key = base + 8 * q4 + 4 * t2 + r;
-                s[t2][r] = !edge || (key >= lo && key < pos) ? s[t2][r] * scl : -INFINITY;
-                mx = fmaxf(mx, s[t2][r]);
+                const int key = base + 32 * (g >> 1) + 8 * q4 + 4 * (g & 1) + r;
+                s[g][r] = !edge || (key >= lo && key < pos) ? s[g][r] * scl : -INFINITY;
+                mx = fmaxf(mx, s[g][r]);
             }
-        if (edge) {
-            uint32_t keep[4];
-#pragma unroll
-            for (int h = 0; h < 4; ++h) {
-                const int key = base + 8 * q4 + 2 * h;
-                keep[h] = (key >= lo && key < pos ? 0x0000ffffu : 0u) | (key + 1 >= lo && key + 1 < pos ? 0xffff0000u : 0u);
-            }
-#pragma unroll
-            for (int d = 0; d < ND; ++d) { vf[d].x &= keep[0]; vf[d].y &= keep[1]; vf[d].z &= keep[2]; vf[d].w &= keep[3]; }
-        }
         mx = fmaxf(mx, __shfl_xor(mx, 16, 64)); mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
         const float m_new = fmaxf(m, mx), ms = m_new == -INFINITY ? 0.f : m_new;
         const float alpha = __builtin_amdgcn_exp2f(m - ms);
         m = m_new;
-        float p[8];
+        float ps = 0.f;
+        uint4 pf[2][3];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) p[k] = __builtin_amdgcn_exp2f(s[k >> 2][k & 3] - ms);
-        l = l * alpha + (((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7])));
-        uint4 pf[3];
+        for (int h = 0; h < 2; ++h) {
+            float p[8];
 #pragma unroll
-        for (int n = 0; n < 3; ++n) {
-            pf[n] = uint4{pack2<T>(p[0], p[1]), pack2<T>(p[2], p[3]), pack2<T>(p[4], p[5]), pack2<T>(p[6], p[7])};
-            p[0] -= unpack_lo<T>(pf[n].x); p[1] -= unpack_hi<T>(pf[n].x); p[2] -= unpack_lo<T>(pf[n].y); p[3] -= unpack_hi<T>(pf[n].y);
-            p[4] -= unpack_lo<T>(pf[n].z); p[5] -= unpack_hi<T>(pf[n].z); p[6] -= unpack_lo<T>(pf[n].w); p[7] -= unpack_hi<T>(pf[n].w);
+            for (int k = 0; k < 8; ++k) p[k] = __builtin_amdgcn_exp2f(s[2 * h + (k >> 2)][k & 3] - ms);
+            ps += ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
+#pragma unroll
+            for (int n = 0; n < 3; ++n) {
+                pf[h][n] = uint4{pack2<T>(p[0], p[1]), pack2<T>(p[2], p[3]), pack2<T>(p[4], p[5]), pack2<T>(p[6], p[7])};
+                p[0] -= unpack_lo<T>(pf[h][n].x); p[1] -= unpack_hi<T>(pf[h][n].x); p[2] -= unpack_lo<T>(pf[h][n].y); p[3] -= unpack_hi<T>(pf[h][n].y);
+                p[4] -= unpack_lo<T>(pf[h][n].z); p[5] -= unpack_hi<T>(pf[h][n].z); p[6] -= unpack_lo<T>(pf[h][n].w); p[7] -= unpack_hi<T>(pf[h][n].w);
+            }
         }
+        l = l * alpha + ps;
+        asm volatile("" ::: "memory");                         // the keys have been read out of the tile
+        to_lds(vr);
+        load_v(p0 + i + step, i + step < np);
 #pragma unroll
-        for (int d = 0; d < ND; ++d) {
-            acc[d] *= alpha;
+        for (int d = 0; d < ND; ++d) acc[d] *= alpha;
 #pragma unroll
-            for (int n = 2; n >= 0; --n) acc[d] = WinMfma<T>::run(vf[d], pf[n], acc[d]);
+        for (int h = 0; h < 2; ++h) {
+            uint32_t keep[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const int key = base + 32 * h + 8 * q4 + 2 * c;
+                keep[c] = !edge ? 0xffffffffu : (key >= lo && key < pos ? 0x0000ffffu : 0u) | (key + 1 >= lo && key + 1 < pos ? 0xffff0000u : 0u);
+            }
+#pragma unroll
+            for (int d = 0; d < ND; ++d) {
+                uint4 vf = *reinterpret_cast<const uint4*>(tile + (d * 16 + i16) * 128 + (((4 * h + q4) ^ (i16 >> 1)) * 16));
+                vf.x &= keep[0]; vf.y &= keep[1]; vf.z &= keep[2]; vf.w &= keep[3];
+#pragma unroll
+                for (int n = 2; n >= 0; --n) acc[d] = WinMfma<T>::run(vf, pf[h][n], acc[d]);
+            }
         }
-        if (i + 1 < mine) load_v(chunk(i + 1));
+        asm volatile("" ::: "memory");                         // the next piece's keys go into the tile after every read of this one's values
+    }
+    // into the caches after the walk: a store in flight (to a pointer out of the table) makes every wait of the walk one for everything
+    if (owner) {
+        for (int d = tid; d < D; d += 256) {
+            Kc[(size_t)pos * D + d] = from_f32<T>(ks[d]);
+            Vt[(size_t)d * a.s_max + pos] = vnew[d];
+        }
     }
     if (owner && wave == 0) {                                  // the new key: its score from the MFMA (every row of the tile is the key), its value from the row
         f32x4 s = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -798,6 +825,7 @@ __global__ __launch_bounds__(256) void decode_win_group_kernel(WinDecodeArgs a) 
     // ---- the four waves, then the splits ----
     l += __shfl_xor(l, 16, 64); l += __shfl_xor(l, 32, 64);
     if (q4 == 0) { wm[wave * 16 + i16] = m; wl[wave * 16 + i16] = l; }
+    __syncthreads();                                           // every wave is done with its tile: the partial rows take their place
     if (i16 < group) {
 #pragma unroll
         for (int d = 0; d < ND; ++d) *reinterpret_cast<f32x4*>(wo + (wave * group + i16) * D + d * 16 + 4 * q4) = acc[d];
@@ -867,7 +895,8 @@ __global__ __launch_bounds__(256) void decode_win_group_kernel(WinDecodeArgs a) 
 }
 
 // 16-bit caches of heads up to 128 wide, up to 16 query heads a kv head, more than one sequence.  32 sequences of 568 - 1300 keys, window 1024, 32 heads on 8 kv heads of 128:
-// 86.7 -> 35.9 us (3.7 TB/s) with one split (2 splits 36.4, 4 43.3: the merge and a shorter walk cost more than a fuller chip gives).  One sequence of 601 keys, 16 heads on 4:
+// one head a workgroup 86.7 us; keys and values straight into the operands 36.9; whole lines through LDS, the next piece on the wire 32.0 (4.2 TB/s) — one split (straight: 2 splits
+// 36.4, 4 43.3: the merge and a shorter walk cost more than a fuller chip gives).  One sequence of 601 keys, 16 heads on 4:
 // 11.1 us either way, all of it latency, so the form with more workgroups stays.
 bool decode_win_grouped(int dtype, int D, int n_heads, int n_kv_heads, int n_seq) {
     return dtype != kF32 && D <= 128 && n_heads / n_kv_heads <= WIN_GROUP_MAX && n_seq > 1;
@@ -882,7 +911,15 @@ void launch_decode_win(int dtype, int D, const WinDecodeArgs& a, hipStream_t st)
     if (decode_win_grouped(dtype, D, a.n_heads, a.n_kv_heads, a.n_seq) && a.qkv_stride % 4 == 0 && reinterpret_cast<uintptr_t>(a.qkv) % 8 == 0) {
         const dim3 grid(a.n_kv_heads, a.n_split, a.n_seq);
         const int smem = win_group_smem(a.n_heads / a.n_kv_heads, D);
-#define L(TT, DD) LMX_LAUNCH((decode_win_group_kernel<TT, DD>), grid, dim3(256), smem, st, a)
+#define L(TT, DD)                                                                                                                                          \
+    do {                                                                                                                                                   \
+        static bool attr_set = false;                                                                                                                      \
+        if (!attr_set) {                                                                                                                                   \
+            LMX_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&decode_win_group_kernel<TT, DD>), hipFuncAttributeMaxDynamicSharedMemorySize, win_group_smem(WIN_GROUP_MAX, DD))); \
+            attr_set = true;                                                                                                                               \
+        }                                                                                                                                                  \
+        LMX_LAUNCH((decode_win_group_kernel<TT, DD>), grid, dim3(256), smem, st, a);                                                                       \
+    } while (0)
         if (dtype == kBF16) { if (D == 128) L(bf16_t, 128); else L(bf16_t, 64); } else { if (D == 128) L(f16_t, 128); else L(f16_t, 64); }
 #undef L
         LMX_CHECK_HIP(hipGetLastError());

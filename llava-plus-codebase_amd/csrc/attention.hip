@@ -61,9 +61,10 @@ __global__ __launch_bounds__(512) void flash_prefill2_kernel(FlashArgs a) {
     const int qrow = q0 + l31;                           // this lane's query row (column of both products)
     const int krow_pi = fa_key_perm(l31);                // key row this lane feeds to QKᵀ as tile row l31
 
-    const T* __restrict__ Q = reinterpret_cast<const T*>(a.Q);
-    const T* __restrict__ Kc = reinterpret_cast<const T*>(a.K) + (size_t)kvh * a.s_max * D;
-    const T* __restrict__ Vt = reinterpret_cast<const T*>(a.VT) + (size_t)kvh * D * a.s_max;
+    const size_t bz = blockIdx.y;                        // problem of the batch
+    const T* __restrict__ Q = reinterpret_cast<const T*>(a.Q) + bz * a.q_batch;
+    const T* __restrict__ Kc = reinterpret_cast<const T*>(a.K) + bz * a.kv_batch + (size_t)kvh * a.s_max * D;
+    const T* __restrict__ Vt = reinterpret_cast<const T*>(a.VT) + bz * a.kv_batch + (size_t)kvh * D * a.s_max;
 
     // ---- Q fragments: B operand, lane holds Q[qrow][s*16 + hi*8 .. +8) ----------------------------------------
     uint4 qf[KSTEPS];
@@ -292,7 +293,7 @@ __global__ __launch_bounds__(512) void flash_prefill2_kernel(FlashArgs a) {
     }
     if (a.lse && hi == 0 && qrow < a.q_len) a.lse[(size_t)head * a.lse_stride + qrow] = m_run + __builtin_amdgcn_logf(l_tot);      // v_log_f32 = log2
     if (qrow < a.q_len) {
-        T* op = reinterpret_cast<T*>(a.O) + (size_t)qrow * a.o_stride + head * D;
+        T* op = reinterpret_cast<T*>(a.O) + bz * a.o_batch + (size_t)qrow * a.o_stride + head * D;
 #pragma unroll
         for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -312,7 +313,8 @@ void launch_flash_prefill(int dtype, int D, const FlashArgs& a, hipStream_t st) 
     LMX_REQUIRE(a.s_max % 64 == 0, "KV cache length must be a multiple of 64");
     LMX_REQUIRE(a.kv_len <= a.s_max && a.q_len > 0, "bad lengths");
     LMX_REQUIRE(a.q_stride % 8 == 0 && a.o_stride % 4 == 0, "q/o strides must keep 16-byte alignment");
-    const dim3 grid(cdiv(a.q_len, FA_QB) * a.n_heads, 1, 1);
+    LMX_REQUIRE(a.n_batch >= 1 && (a.n_batch == 1 || (!a.win && !a.lse && a.q_batch % 8 == 0 && a.o_batch % 4 == 0 && a.kv_batch % 8 == 0)), "flash prefill: a batch is of plain problems, 16 bytes apart");
+    const dim3 grid(cdiv(a.q_len, FA_QB) * a.n_heads, a.n_batch, 1);
     {
         // two key groups per query block (flash_prefill2_kernel): 8 waves, ring of 2 (D = 128) / 3 (D = 64) rounds of two tiles
         const int smem2 = (D == 128 ? 2 : 3) * 2 * (FA_KT * D * 2 + D * FA_KT * 2);

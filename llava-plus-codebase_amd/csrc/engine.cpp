@@ -468,21 +468,23 @@ void Model::encode_images(const void* pixels, int n, void* feats, hipStream_t st
             if (pack_fused) { g.pk_kc = vkc.p; g.pk_vt = vvt.p; g.pk_heads = vh; g.pk_D = vD; g.pk_rows = Tv; g.pk_spad = spad; g.pk_img_stride = kv_bytes / es; }
             launch_gemm(dt, g, gv, st);
         }
-        for (int i = 0; i < n; ++i) {
+        for (int i = 0; i < n && (!pack_fused || dt == kF32); ++i) {
             char* qkv_i = static_cast<char*>(qkv) + (size_t)i * Tv * 3 * Dv * es;
             char* attn_i = static_cast<char*>(attn) + (size_t)i * Tv * Dv * es;
             void* kc = vkc.as<char>() + (size_t)i * kv_bytes;
             void* vt = vvt.as<char>() + (size_t)i * kv_bytes;
             RopeKvArgs ra{qkv_i, kc, vt, nullptr, nullptr, 0, Tv, 3 * Dv, vh, vh, spad};
-            if (!pack_fused) { LMX_PROF("vis.kv_pack"); launch_rope_kv(dt, vD, ra, st); }
+            { LMX_PROF("vis.kv_pack"); launch_rope_kv(dt, vD, ra, st); }
             if (dt == kF32) {
                 DecodeAttnArgs da{qkv_i, attn_i, kc, vt, nullptr, 0, Tv, Tv, 0, 3 * Dv, Dv, vh, vh, spad, 1, scale,
                                   reinterpret_cast<float*>(W + o_aws)};
                 { LMX_PROF("vis.attn"); launch_decode_attn(dt, vD, da, st); }
-            } else {
-                FlashArgs fa{qkv_i, attn_i, kc, vt, Tv, Tv, 0, 3 * Dv, Dv, vh, vh, spad, scale, 0};
-                { LMX_PROF("vis.attn"); launch_flash_prefill(dt, vD, fa, st); }
             }
+        }
+        if (dt != kF32) {        // all images in one launch (577 rows, 16 heads: 80 workgroups an image)
+            FlashArgs fa{qkv, attn, vkc.p, vvt.p, Tv, Tv, 0, 3 * Dv, Dv, vh, vh, spad, scale, 0};
+            fa.n_batch = n; fa.q_batch = (size_t)Tv * 3 * Dv; fa.o_batch = (size_t)Tv * Dv; fa.kv_batch = kv_bytes / es;
+            { LMX_PROF("vis.attn"); launch_flash_prefill(dt, vD, fa, st); }
         }
         { LMX_PROF("vis.gemm.out"); launch_gemm(dt, GemmArgs{attn, w.wo, h, w.bo, h, rows, Dv, Dv, Dv, Dv, Dv, Dv, kActNone}, gv, st); }
         { LMX_PROF("vis.layernorm"); launch_layernorm(dt, h, w.ln2w, w.ln2b, x, rows, Dv, Dv, Dv, cfg.v_ln_eps, st); }

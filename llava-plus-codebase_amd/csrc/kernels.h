@@ -100,6 +100,9 @@ struct FlashArgs {
     // gate: head h's output row is multiplied by sigmoid(gate[row][h]) (model dtype, row pitch q_stride; null = off).  `win` switches the form on.
     int win = 0, window = 0, sink = 0;
     const void* gate = nullptr;
+    // n_batch alike problems in one launch, these strides apart (elements): rows of Q and O, caches
+    int n_batch = 1;
+    size_t q_batch = 0, o_batch = 0, kv_batch = 0;
 };
 void launch_flash_prefill(int dtype, int D, const FlashArgs& a, hipStream_t st);
 

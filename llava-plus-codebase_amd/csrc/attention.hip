@@ -31,19 +31,21 @@ namespace lmx {
 // free) ring and group 0 merges the two online-softmax states per lane: m = max(m0, m1), O = O0 2^(m0 - m) + O1 2^(m1 - m), l likewise.
 // WIN (FlashArgs::win): sliding window, softmax sink and output gate of the windowed decoders.  Only the key tiles a query block can see are walked: the tile
 // range starts at the tile of the first row's oldest visible key, so the work per block is bounded by the window.
-template <typename T, int D, bool CAUSAL, bool WIN = false>
-__global__ __launch_bounds__(512) void flash_prefill2_kernel(FlashArgs a) {
+// Without a causal limit every row's position lies behind the last key (launch_flash_prefill): the same code, and fewer registers than a form of its own took (D = 64: 125, 177).
+// D = 64: two workgroups a CU (a ring of two rounds, 128 registers); four images of 577 rows, 16 heads: 24.2 us with one workgroup a CU and a ring of three -> 19.5.
+constexpr int FA_SLICES_MAX = 8;
+template <typename T, int D, bool WIN = false>
+__global__ __launch_bounds__(512, D == 64 && !WIN ? 4 : 2) void flash_prefill2_kernel(FlashArgs a) {
     constexpr int KSTEPS = D / 16;        // MFMA k-steps over the head dim (QKᵀ)
     constexpr int DB = D / 32;            // 32-row blocks of Oᵀ
     constexpr int K_BYTES = FA_KT * D * 2;
     constexpr int V_BYTES = D * FA_KT * 2;
     constexpr int BUF_BYTES = K_BYTES + V_BYTES;
-    constexpr int NRND = D == 128 ? 2 : 3;        // rounds in the ring: 2 x 2 x 32 KiB (D = 128) / 3 x 2 x 16 KiB (D = 64)
+    constexpr int NRND = 2;                       // rounds in the ring: 2 x 2 x 32 KiB (D = 128) / 2 x 2 x 16 KiB (D = 64)
     constexpr int KROWS_PP = 1024 / (D * 2);      // K rows per 1-KiB DMA piece (4 for D=128, 8 for D=64)
     constexpr int KCPR = D / 8;                   // 16-byte chunks per K row
     constexpr int KPPW = K_BYTES / 1024 / 4;      // K pieces per wave per tile
     constexpr int VPPW = V_BYTES / 1024 / 4;      // Vᵀ pieces per wave per tile (8 rows each)
-    constexpr int PPW = KPPW + VPPW;
 
     extern __shared__ __attribute__((aligned(16))) char smem[];
 
@@ -83,7 +85,7 @@ __global__ __launch_bounds__(512) void flash_prefill2_kernel(FlashArgs a) {
 
     // number of key tiles this workgroup needs
     int kv_end = a.kv_len;
-    if (CAUSAL) {
+    {
         const int last_q = qb * FA_QB + FA_QB - 1;
         const int lim = a.q_pos0 + (last_q < a.q_len ? last_q : a.q_len - 1) + 1;
         kv_end = lim < kv_end ? lim : kv_end;
@@ -94,7 +96,12 @@ __global__ __launch_bounds__(512) void flash_prefill2_kernel(FlashArgs a) {
         const int oldest = a.window > 0 ? a.q_pos0 + qb * FA_QB - a.window + 1 : 0;
         tile0 = oldest > 0 ? oldest / FA_KT : 0;
     }
-    const int ntiles = (kv_end + FA_KT - 1) / FA_KT - tile0;
+    int ntiles = (kv_end + FA_KT - 1) / FA_KT - tile0;
+    if (a.part) {                                        // this workgroup's slice of the keys (blockIdx.z); 0 tiles: a partial row of weight 0
+        const int lo = ntiles * (int)blockIdx.z / (int)gridDim.z;
+        ntiles = ntiles * ((int)blockIdx.z + 1) / (int)gridDim.z - lo;
+        tile0 += lo;
+    }
 
     f32x16 oacc[DB];
 #pragma unroll
@@ -105,7 +112,7 @@ __global__ __launch_bounds__(512) void flash_prefill2_kernel(FlashArgs a) {
     const float sc = a.scale * 1.4426950408889634f;      // work in the log2 domain
     const int my_pos = a.q_pos0 + qrow;                   // causal limit of this lane's row
 
-    // ---- K / Vᵀ tiles by LDS-DMA into a 3-slot ring (inline asm: see gemm_pipe_kernel for why) -----------------------
+    // ---- K / Vᵀ tiles by LDS-DMA into a ring of two rounds (inline asm: see gemm_pipe_kernel for why) -----------------------
     // per-lane source offsets (elements) inside a tile; the swizzle lives in the SOURCE address, the LDS image is lane-linear
     int ksrc[KPPW], vsrc[VPPW];
 #pragma unroll
@@ -147,9 +154,7 @@ __global__ __launch_bounds__(512) void flash_prefill2_kernel(FlashArgs a) {
         if (r < nrounds) stage_round(r);
     for (int r = 0; r < nrounds; ++r) {
         const int t = 2 * r + grp;
-        // everything this wave staged for round r has landed; with a 3-round ring round r + 1 may still be on the wire
-        if (NRND == 3 && r + 1 < nrounds && 2 * (r + 1) + grp < ntiles) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PPW) : "memory");
-        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // everything this wave staged for round r has landed
         __builtin_amdgcn_s_barrier();          // round r visible to every wave; everyone is done with round r - 1 (its slots are free)
         if (r + NRND - 1 < nrounds) stage_round(r + NRND - 1);
         if (t >= ntiles) continue;             // odd tile count: group 1 sits out the last round (it still takes the barriers)
@@ -177,7 +182,7 @@ __global__ __launch_bounds__(512) void flash_prefill2_kernel(FlashArgs a) {
         float p[2][16];
         float tmax = -INFINITY;
         const int tile_first = (tile0 + t) * FA_KT, tile_last = tile_first + FA_KT - 1;
-        bool need_mask = tile_last >= a.kv_len || (CAUSAL && tile_last > a.q_pos0 + q0);
+        bool need_mask = tile_last >= a.kv_len || tile_last > a.q_pos0 + q0;
         if constexpr (WIN) need_mask = need_mask || (a.window > 0 && tile_first <= a.q_pos0 + q0 + 31 - a.window);
         if (need_mask) {
 #pragma unroll
@@ -186,7 +191,7 @@ __global__ __launch_bounds__(512) void flash_prefill2_kernel(FlashArgs a) {
                 for (int r = 0; r < 16; ++r) {
                     const int key = tile_first + kb * 32 + (r & 3) + 4 * ((r >> 2) & 1) + 8 * hi + 16 * (r >> 3);
                     bool ok = key < a.kv_len;
-                    if (CAUSAL) ok = ok && (key <= my_pos);
+                    ok = ok && key <= my_pos;
                     if constexpr (WIN) ok = ok && (a.window <= 0 || my_pos - key < a.window);
                     const float v = ok ? sacc[kb][r] * sc : -INFINITY;
                     p[kb][r] = v;
@@ -280,6 +285,17 @@ __global__ __launch_bounds__(512) void flash_prefill2_kernel(FlashArgs a) {
             for (int r = 0; r < 16; ++r) oacc[i][r] = oacc[i][r] * a0 + mg[(i * 16 + r) * 64 + lane] * a1;
     }
     const float l_tot = l_run + __shfl_xor(l_run, 32, 64);
+    if (a.part) {                                        // sums as they are, with their maximum: flash_merge_kernel
+        if (qrow >= a.q_len) return;
+        float* pp = a.part + (((size_t)blockIdx.z * a.q_len + qrow) * a.n_heads + head) * (D + 4);
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+#pragma unroll
+            for (int q4 = 0; q4 < 4; ++q4)
+                *reinterpret_cast<float4*>(pp + db * 32 + 8 * q4 + 4 * hi) = float4{oacc[db][4 * q4], oacc[db][4 * q4 + 1], oacc[db][4 * q4 + 2], oacc[db][4 * q4 + 3]};
+        if (hi == 0) { pp[D] = m_run; pp[D + 1] = l_tot; }
+        return;
+    }
     float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
     if constexpr (WIN) {
         if (a.sink) {                          // the running maximum may lie below the sink's score 0: bring both sums to max(m, 0)
@@ -307,6 +323,44 @@ __global__ __launch_bounds__(512) void flash_prefill2_kernel(FlashArgs a) {
     }
 }
 
+// the slices' partial rows of one (query row, head), in slice order: four dims a thread
+template <typename T, int D>
+__global__ __launch_bounds__(256) void flash_merge_kernel(FlashArgs a, int slices) {
+    const int i = blockIdx.x * 256 + threadIdx.x, pair = i / (D / 4), d = i % (D / 4) * 4;
+    if (pair >= a.q_len * a.n_heads) return;
+    const size_t step = (size_t)a.q_len * a.n_heads * (D + 4);
+    const float* p = a.part + (size_t)pair * (D + 4);
+    float m[FA_SLICES_MAX], l[FA_SLICES_MAX];
+    float4 o[FA_SLICES_MAX];
+#pragma unroll
+    for (int s = 0; s < FA_SLICES_MAX; ++s) {
+        const float* ps = p + (s < slices ? s : 0) * step;
+        m[s] = s < slices ? ps[D] : -INFINITY; l[s] = ps[D + 1]; o[s] = *reinterpret_cast<const float4*>(ps + d);
+    }
+    float M = m[0];
+#pragma unroll
+    for (int s = 1; s < FA_SLICES_MAX; ++s) M = fmaxf(M, m[s]);
+    float lt = 0.f, t[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < FA_SLICES_MAX; ++s) {
+        const float w = __builtin_amdgcn_exp2f(m[s] - M);
+        lt = fmaf(w, l[s], lt); t[0] = fmaf(w, o[s].x, t[0]); t[1] = fmaf(w, o[s].y, t[1]); t[2] = fmaf(w, o[s].z, t[2]); t[3] = fmaf(w, o[s].w, t[3]);
+    }
+    const float inv = lt > 0.f ? 1.f / lt : 0.f;
+    uint2 u;
+    u.x = pack2<T>(t[0] * inv, t[1] * inv); u.y = pack2<T>(t[2] * inv, t[3] * inv);
+    *reinterpret_cast<uint2*>(reinterpret_cast<T*>(a.O) + (size_t)(pair / a.n_heads) * a.o_stride + (pair % a.n_heads) * D + d) = u;
+}
+
+// Key slices of a launch: where its workgroups leave half of the CUs idle or more, as many as fill them, of at least four 64-key tiles (two rounds) each.
+// 139 rows on 1347 keys, 32 heads of 128 (64 workgroups of 11 rounds): 30.5 us -> 17.5 with four slices and 5.0 for the merge.
+static int flash_slices(int D, const FlashArgs& a, int workgroups) {
+    if (!a.part || a.win || a.lse || a.n_batch != 1) return 1;
+    int s = std::min(std::min(256 / workgroups, cdiv(a.kv_len, FA_KT) / 4), FA_SLICES_MAX);
+    while (s > 1 && (size_t)s * a.q_len * a.n_heads * (D + 4) * sizeof(float) > a.part_bytes) --s;
+    return std::max(s, 1);
+}
+
 void launch_flash_prefill(int dtype, int D, const FlashArgs& a, hipStream_t st) {
     LMX_REQUIRE(dtype == kBF16 || dtype == kF16, "flash prefill is the 16-bit path (fp32 verification uses decode_attn)");
     LMX_REQUIRE(D == 64 || D == 128, "head_dim must be 64 or 128");
@@ -314,34 +368,38 @@ void launch_flash_prefill(int dtype, int D, const FlashArgs& a, hipStream_t st) 
     LMX_REQUIRE(a.kv_len <= a.s_max && a.q_len > 0, "bad lengths");
     LMX_REQUIRE(a.q_stride % 8 == 0 && a.o_stride % 4 == 0, "q/o strides must keep 16-byte alignment");
     LMX_REQUIRE(a.n_batch >= 1 && (a.n_batch == 1 || (!a.win && !a.lse && a.q_batch % 8 == 0 && a.o_batch % 4 == 0 && a.kv_batch % 8 == 0)), "flash prefill: a batch is of plain problems, 16 bytes apart");
-    const dim3 grid(cdiv(a.q_len, FA_QB) * a.n_heads, a.n_batch, 1);
+    const int slices = flash_slices(D, a, cdiv(a.q_len, FA_QB) * a.n_heads);
+    const dim3 grid(cdiv(a.q_len, FA_QB) * a.n_heads, a.n_batch, slices);
     {
-        // two key groups per query block (flash_prefill2_kernel): 8 waves, ring of 2 (D = 128) / 3 (D = 64) rounds of two tiles
-        const int smem2 = (D == 128 ? 2 : 3) * 2 * (FA_KT * D * 2 + D * FA_KT * 2);
-#define LMX_FA2_LAUNCH(TT, DD, CC) LMX_FA2_LAUNCH_W(TT, DD, CC, false)
-#define LMX_FA2_LAUNCH_W(TT, DD, CC, WW)                                                                            \
+        // two key groups per query block (flash_prefill2_kernel): 8 waves, ring of 2 rounds of two tiles
+        const int smem2 = 2 * 2 * (FA_KT * D * 2 + D * FA_KT * 2);
+#define LMX_FA2_LAUNCH(TT, DD, WW)                                                                                  \
     do {                                                                                                            \
-        auto kern = flash_prefill2_kernel<TT, DD, CC, WW>;                                                            \
+        auto kern = flash_prefill2_kernel<TT, DD, WW>;                                                                \
         static bool attr_set = false;                                                                               \
         if (!attr_set) {                                                                                            \
             LMX_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, smem2)); \
             attr_set = true;                                                                                        \
         }                                                                                                           \
-        hipLaunchKernelGGL(kern, grid, dim3(512), smem2, st, a);                                                    \
+        hipLaunchKernelGGL(kern, grid, dim3(512), smem2, st, b);                                                    \
     } while (0)
+#define LMX_FA2_D(TT, WW) do { if (D == 128) LMX_FA2_LAUNCH(TT, 128, WW); else LMX_FA2_LAUNCH(TT, 64, WW); } while (0)
+        FlashArgs b = a;
+        if (!a.causal) b.q_pos0 = a.kv_len;                  // every row sees every key
+        if (slices == 1) b.part = nullptr;
         if (a.win) {
             LMX_REQUIRE(a.causal && !a.lse, "flash prefill: the windowed form is causal and keeps no log-sum-exp");
-            if (dtype == kBF16) { if (D == 128) LMX_FA2_LAUNCH_W(bf16_t, 128, true, true); else LMX_FA2_LAUNCH_W(bf16_t, 64, true, true); }
-            else { if (D == 128) LMX_FA2_LAUNCH_W(f16_t, 128, true, true); else LMX_FA2_LAUNCH_W(f16_t, 64, true, true); }
-        } else if (dtype == kBF16) {
-            if (D == 128) { if (a.causal) LMX_FA2_LAUNCH(bf16_t, 128, true); else LMX_FA2_LAUNCH(bf16_t, 128, false); }
-            else          { if (a.causal) LMX_FA2_LAUNCH(bf16_t, 64, true);  else LMX_FA2_LAUNCH(bf16_t, 64, false); }
-        } else {
-            if (D == 128) { if (a.causal) LMX_FA2_LAUNCH(f16_t, 128, true); else LMX_FA2_LAUNCH(f16_t, 128, false); }
-            else          { if (a.causal) LMX_FA2_LAUNCH(f16_t, 64, true);  else LMX_FA2_LAUNCH(f16_t, 64, false); }
-        }
+            if (dtype == kBF16) LMX_FA2_D(bf16_t, true); else LMX_FA2_D(f16_t, true);
+        } else if (dtype == kBF16) LMX_FA2_D(bf16_t, false);
+        else LMX_FA2_D(f16_t, false);
+#undef LMX_FA2_D
 #undef LMX_FA2_LAUNCH
-#undef LMX_FA2_LAUNCH_W
+        if (slices > 1) {
+            const dim3 mgrid(cdiv(a.q_len * a.n_heads * (D / 4), 256));
+#define LM(TT, DD) hipLaunchKernelGGL((flash_merge_kernel<TT, DD>), mgrid, dim3(256), 0, st, b, slices)
+            if (dtype == kBF16) { if (D == 128) LM(bf16_t, 128); else LM(bf16_t, 64); } else { if (D == 128) LM(f16_t, 128); else LM(f16_t, 64); }
+#undef LM
+        }
         LMX_CHECK_HIP(hipGetLastError());
         return;
     }

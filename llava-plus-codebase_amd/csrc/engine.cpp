@@ -648,7 +648,9 @@ void Model::prefill(Seq* s, const void* embeds, int T, int chunk, void* logits, 
             if (dt == kF32) {
                 { LMX_PROF("prefill.attn"); launch_decode_attn(dt, D, DecodeAttnArgs{qr, ar, kc, vt, nullptr, pos0 + r0, n, 0, 1, qkv_n, nh_l * D, nh_l, nkv_l, kv_pitch, 1, scale, aws}, st); }
             } else {
-                { LMX_PROF("prefill.attn"); launch_flash_prefill(dt, D, FlashArgs{qr, ar, kc, vt, n, pos0 + r0 + n, pos0 + r0, qkv_n, nh_l * D, nh_l, nkv_l, kv_pitch, scale, 1}, st); }
+                FlashArgs fa{qr, ar, kc, vt, n, pos0 + r0 + n, pos0 + r0, qkv_n, nh_l * D, nh_l, nkv_l, kv_pitch, scale, 1};
+                fa.part = s->skw.as<float>(); fa.part_bytes = s->skw.bytes;
+                { LMX_PROF("prefill.attn"); launch_flash_prefill(dt, D, fa, st); }
             }
             { LMX_PROF_K("prefill.gemm.o"); launch_gemm(dt, with_scratch(GemmArgs{ar, w.wo, hr, nullptr, lead ? hr : nullptr, n, H, nh_l * D, nh_l * D, nh_l * D, H, H, kActNone}), gv, st); }
         };

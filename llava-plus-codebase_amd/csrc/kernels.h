@@ -103,6 +103,9 @@ struct FlashArgs {
     // n_batch alike problems in one launch, these strides apart (elements): rows of Q and O, caches
     int n_batch = 1;
     size_t q_batch = 0, o_batch = 0, kv_batch = 0;
+    // scratch (optional): a launch of few workgroups over many keys cuts the keys into slices, fp32 partial rows here, and merges them in a second launch
+    float* part = nullptr;
+    size_t part_bytes = 0;
 };
 void launch_flash_prefill(int dtype, int D, const FlashArgs& a, hipStream_t st);
 

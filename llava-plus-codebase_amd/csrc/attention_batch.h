@@ -1,11 +1,10 @@
 // Decode attention of the decode BATCH (continuous batching), 16-bit models with head_dim 128: one workgroup per (sequence, head) whose waves STREAM the head's
-// keys (attention.hip includes this; launch_decode_fused takes it for the batch form).  Written at the end of round 4, first run in round 5 (parity green,
-// profiles/r05_batch_attn_wave.jsonl: 44.8 -> 38.9 us per layer at 8 sequences, 143 -> 134 at 32; the same body as the SINGLE request's launch lost, 16.8 -> 20.4 us:
-// 32 workgroups cannot pull 19 MB fast enough — that wiring is gone, EXPERIMENTS.md r5-A).
+// keys (attention.hip includes this; launch_decode_fused takes it for the batch form).  As the SINGLE request's launch the same body loses, 16.8 -> 20.4 us a layer: 32
+// workgroups cannot pull 19 MB fast enough.
 //
-// Why (profiles/EXPERIMENTS.md r4-N): the batch launch of decode_fused_kernel — one workgroup per (sequence, head, 128-key chunk), the whole chunk
-// in registers, partials through memory, ticket, merge by the last arriver — moves a batch-8 layer's 142 MB of K / V^T at 3.2 TB/s (4.0 at 32 sequences): its
-// resident workgroups start together, request everything at once, then compute and merge together with the HBM idle.  Contract reproduced: the single-token branch of
+// Why: the batch launch of decode_fused_kernel — one workgroup per (sequence, head, 128-key chunk), the whole chunk in registers, partials through memory, ticket, merge by
+// the last arriver — moves a batch-8 layer's 142 MB of K / V^T at 3.2 TB/s (4.0 at 32 sequences): its resident workgroups start together, request everything at once, then
+// compute and merge together with the HBM idle.  Contract reproduced: the single-token branch of
 // llava/model/llava_arch.py:103-112 -> HF5:models/llama/modeling_llama.py:191-214, 243-281 (RoPE on q and the new key, KV append, softmax in fp32, probabilities x V),
 // same inputs and outputs as decode_fused_kernel's batch form (DecodeFusedArgs with `tab`); NOT the same summation order (online softmax over 64-key pieces instead
 // of 128-key partials merged in chunk order), so parity is by tolerance against the reference arithmetic, not bit-identity with the chunked launch.
@@ -210,7 +209,7 @@ __global__ __launch_bounds__(BA_NW * 64) void decode_attn_wave_kernel(DecodeFuse
     (reinterpret_cast<T*>(a.O) + (size_t)zseq * a.o_stride)[head * D + tid] = from_f32<T>(l > 0.f ? o / l : 0.f);
 }
 
-// The batch form of launch_decode_fused through the kernel above.  Workgroup forms measured at equal contexts (profiles/r06_batch_attn_forms.jsonl; ms per batched step at
+// The batch form of launch_decode_fused through the kernel above.  Workgroup forms measured at equal contexts, with a piece's loads requested together (ms per batched step at
 // 8 / 16 / 24 / 32 sequences): 8 waves x 1 head 3.75 / 5.19 / 6.51 / 7.76, 8 x 2 3.95 / 5.16 / 6.71 / 7.76, 4 x 2 4.01 / 5.10 / 6.59 / 7.62, **4 x 1 3.77 / 5.10 / 6.38 /
 // 7.62**, 4 or 8 waves x 4 heads 25 - 30 % slower: two independent 4-wave workgroups per CU, one head each, drift apart, so one's merge tail and start-up run under the
 // other's stream; walking several heads per workgroup only lengthens the tail.

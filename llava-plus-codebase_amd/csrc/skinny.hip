@@ -20,15 +20,13 @@
 //     the lane-linear A fragments of MFMA step j) and the SWZ instantiation reads 1 KiB of contiguous memory per load instruction.
 //   * a workgroup owns 16·RT weight rows (RT = 2: for SiLU·mul the two tiles are the gate rows and the matching up rows of
 //     the [32 gate | 32 up] interleaved weight, so silu(g)·u happens in the epilogue like in the GEMM / GEMV).
-//   * K SLICES ACROSS WORKGROUPS (round 6, narrow layers: N = hidden).  The x rows are re-read from L2 by every workgroup, and a CU's load path does not tell an L2
+//   * K SLICES ACROSS WORKGROUPS (narrow layers: N = hidden).  The x rows are re-read from L2 by every workgroup, and a CU's load path does not tell an L2
 //     hit from an HBM line: at 32 rows o_proj moved 33.5 MB of weights + 256 workgroups x 256 KB of x = 67 MB and down_proj 90 + 180 MB (13.1 / 30.5 us: 2.6 / 3.0 TB/s of
 //     weights).  Four row tiles per workgroup cut the x traffic by four but leave N / 64 = 64 workgroups; so gridDim.y = KS workgroups share a 64-row tile, each takes a
-//     contiguous K range (its 8 waves split that range as before), stores its fp32 partial tile write-through, and the LAST to arrive (one agent-scope ticket per
+//     contiguous K range (its waves split that range as before), stores its fp32 partial tile write-through, and the LAST to arrive (one agent-scope ticket per
 //     tile) adds the KS partials in slice order — deterministic — and runs the epilogue (guide §6 Guideline 16, R1: sc1 payload, drain, ticket; one acquire).
 //     The same form fills the chip on tensor-parallel shards, whose linears are 48 - 96 workgroups otherwise.
 // Epilogue order (bias -> activation -> residual -> round) is the GEMV's, so the batched step rounds like the single step.
-// (Round 4's opt-in arm with the input rows' RMSNorm inside the launch — bit-identical, slower at full width, equal on small shards — was removed in round 5:
-// profiles/EXPERIMENTS.md r4-L.)
 #include <cstdlib>
 #include <type_traits>
 #include "common.h"

@@ -9,6 +9,8 @@
 //
 // Head vectors are stored padded to D in {64, 128, 256} lanes: the padding weights are zero, so padded lanes of q, k and v are zero and add nothing; the query / key
 // norm divides by the true width.
+#include <type_traits>
+
 #include "common.h"
 #include "kernels.h"
 #include "attention_batch.h"
@@ -643,8 +645,9 @@ __global__ __launch_bounds__(256) void decode_win_kernel(WinDecodeArgs a) {
 // key and value leaves memory once instead of once per query head.  A wave walks 64-key pieces (no barrier inside the walk): keys and V^T rows come in whole lines (16 loads of
 // 1 KiB each, marked streaming) and reach the operands' order through 16 KiB of wave-private LDS, chunks XOR-swizzled; the next piece is requested as soon as this one is in LDS.
 // Scores = K tile (16 keys) x query heads (16 columns), the softmax over the lane's 16 keys and 4 lanes, then V^T rows x probabilities.  The C layout of the scores (lane = head,
-// 4 rows a tile) is the B layout of the probabilities when row 4 q + r of tile t is key 8 q + 4 t + r of 32, so no probability changes lanes.  Probabilities stay exact to 24
-// bits: three 16-bit terms, three MFMAs.  Bound: the cache stream (32 sequences x 1024 keys, 8 kv heads of 128: 134 MB a launch); figures: decode_win_grouped.
+// 4 rows a tile) is the B layout of the probabilities when row 4 q + r of tile t is key 8 q + 4 t + r of 32, so no probability changes lanes.  Probabilities keep fp32's 24
+// bits: three 16-bit terms, three MFMAs; f16 terms of a probability times 2^15, because f16 ends at 2^-24: without the factor a probability of 2^-12 kept 12 bits and one below 2^-25
+// none, with it the sums are off by 2^-40 a key.  Bound: the cache stream (32 sequences x 1024 keys, 8 kv heads of 128: 134 MB a launch); figures: decode_win_grouped.
 template <typename T> struct WinMfma;
 template <> struct WinMfma<bf16_t> {
     static __device__ __forceinline__ f32x4 run(const uint4& a, const uint4& b, f32x4 c) {
@@ -680,6 +683,7 @@ __global__ __launch_bounds__(256) void decode_win_group_kernel(WinDecodeArgs a) 
     const float* cs = a.cos_sin + (size_t)pos * a.rot_dims;
     const bool owner = split == a.n_split - 1;                 // this workgroup takes the new key
     constexpr int NT = D / 32, ND = D / 16;                    // 32-deep steps of a score, 16-row tiles of V^T
+    constexpr float UP = std::is_same_v<T, f16_t> ? 32768.f : 1.f;      // the accumulators hold UP times the sums (probabilities are <= 1); the normaliser l does not
     const float scl = a.scale * 1.4426950408889634f;
 
     // piece loads: instruction u brings 1 KiB = whole key rows (K) or 8 V^T rows of 64 keys; lane l's 16 bytes land at l 16 of the tile's KiB u, so the chunk it fetches is the swizzled one
@@ -770,6 +774,8 @@ __global__ __launch_bounds__(256) void decode_win_group_kernel(WinDecodeArgs a) 
             for (int k = 0; k < 8; ++k) p[k] = __builtin_amdgcn_exp2f(s[2 * h + (k >> 2)][k & 3] - ms);
             ps += ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
 #pragma unroll
+            for (int k = 0; k < 8; ++k) p[k] *= UP;
+#pragma unroll
             for (int n = 0; n < 3; ++n) {
                 pf[h][n] = uint4{pack2<T>(p[0], p[1]), pack2<T>(p[2], p[3]), pack2<T>(p[4], p[5]), pack2<T>(p[6], p[7])};
                 p[0] -= unpack_lo<T>(pf[h][n].x); p[1] -= unpack_hi<T>(pf[h][n].x); p[2] -= unpack_lo<T>(pf[h][n].y); p[3] -= unpack_hi<T>(pf[h][n].y);
@@ -819,7 +825,7 @@ __global__ __launch_bounds__(256) void decode_win_group_kernel(WinDecodeArgs a) 
         for (int d = 0; d < ND; ++d) {
             const uint2 v = *reinterpret_cast<const uint2*>(vnew + d * 16 + 4 * q4);
             const f32x4 vv = {unpack_lo<T>(v.x), unpack_hi<T>(v.x), unpack_lo<T>(v.y), unpack_hi<T>(v.y)};
-            acc[d] = acc[d] * alpha + vv * pn;
+            acc[d] = acc[d] * alpha + vv * (pn * UP);
         }
     }
     // ---- the four waves, then the splits ----
@@ -828,7 +834,7 @@ __global__ __launch_bounds__(256) void decode_win_group_kernel(WinDecodeArgs a) 
     __syncthreads();                                           // every wave is done with its tile: the partial rows take their place
     if (i16 < group) {
 #pragma unroll
-        for (int d = 0; d < ND; ++d) *reinterpret_cast<f32x4*>(wo + (wave * group + i16) * D + d * 16 + 4 * q4) = acc[d];
+        for (int d = 0; d < ND; ++d) *reinterpret_cast<f32x4*>(wo + (wave * group + i16) * D + d * 16 + 4 * q4) = acc[d] * (1.f / UP);
     }
     __syncthreads();
     constexpr int WS = D + 4;

@@ -1,6 +1,8 @@
 """One new token of several sequences, all query heads of a kv head in one workgroup (csrc/stack_ops.hip: decode_win_group_kernel): group sizes up to the tile's 16 columns and
 one past it, positions at the borders of a wave's 32 and a chunk's 128 keys, windows that start inside either, splits without a chunk; against float64 and against the
 same sequence on its own (the one-head-per-workgroup kernel)."""
+import math
+
 import pytest
 import torch
 
@@ -49,3 +51,27 @@ def test_groups(cuda, dt, H, G, D, dim, window, n_split):
         assert _err(got[i:i + 1, :, :dim], want) < TOL[dt], p
         alone = ops.decode_win(row[i:i + 1].to(cuda), k1[i:i + 1], v1[i:i + 1], words[i:i + 1], *args).reshape(H, D)
         assert _err(got[i], alone.double().cpu()) < TOL[dt] and torch.equal(ks[i][:, p], k1[i][:, p]) and torch.equal(vs[i][:, :, p], v1[i][:, :, p])
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("n_split", [1, 3])
+def test_small_probabilities(cuda, dt, n_split):
+    """One key of weight 1 whose value is 0 and a tail of 1000 keys of weights 2^-22 .. 2^-27: the output is the tail's alone, to the bits of fp32 weights.  Bound: the output's
+    rounding, the fp32 sum's 1000 terms, a score's rounding (27 x 2^-23 in the exponent)."""
+    from llava_mi355x import ops
+    H, G, D, n, tail = 4, 1, 64, 2, 1000
+    T = DT[dt]
+    g = torch.Generator().manual_seed(4)
+    row = torch.zeros(n, (H + 2 * G) * D)
+    row[:, [h * D for h in range(H)]] = 1
+    row[:, H * D] = -100                                                         # the new key: out of sight
+    k, v = torch.zeros(n, 1, tail + 128 - tail % 128, D), torch.zeros(n, 1, D, tail + 128 - tail % 128)
+    k[:, 0, 1:tail + 1, 0] = -(22 + 5 * torch.rand(n, tail, generator=g))
+    v[:, 0, :, 1:tail + 1] = 1024 * (0.5 + 0.5 * torch.rand(n, D, tail, generator=g))
+    k, v = k.to(T), v.to(T)
+    words = [torch.tensor([tail + 1], dtype=torch.int32, device=cuda) for _ in range(n)]
+    got = ops.decode_win(row.to(T).to(cuda), [c.to(cuda) for c in k], [c.to(cuda) for c in v], words, None, H, G, D, 0, math.log(2.0), 1e-5, sink=False, n_split=n_split)
+    p = torch.exp2(k[:, 0, :tail + 1, 0].double())
+    want = (v[:, 0, :, :tail + 1].double() @ p.unsqueeze(2)).squeeze(2) / p.sum(1, keepdim=True)
+    bound = (2.0 ** -8 if dt == "bf16" else 2.0 ** -11) + tail * 2.0 ** -24 + 27 * 2.0 ** -23
+    assert ((got.double().cpu().view(n, H, D) - want[:, None]).abs() <= bound * want[:, None]).all()

@@ -299,6 +299,12 @@ int lmx_model_set_option(lmx_model* m, const char* key, int32_t value);
 /* ---- single-op entry points (unit parity tests + microbenchmarks; same kernels the engine launches) --------------- */
 int lmx_op_gemm(int32_t dtype, const void* x, const void* w, void* c, const void* bias, const void* residual,
                 int32_t M, int32_t N, int32_t K, int32_t ldx, int32_t ldw, int32_t ldc, int32_t ldr, int32_t act, int32_t variant, void* stream);
+/* variant LMX_GEMM_SCRATCH: the choice a prefill makes, which brings scratch for K slices (this entry's own 64 MiB: one stream at a time); variant 0 chooses without.
+ * lmx_op_gemm_form: that choice for contiguous 16-byte aligned operands and `scratch_bytes` of scratch, on the host alone.  form[4]: batch = 0: {1, row tiles, weight
+ * rows of a workgroup, K slices} of the kernel for few row tiles, {0, 0, 0, K slices} of the others; batch = 1 (linears of a decode batch, M <= 32): {0, 16-row weight tiles of
+ * a workgroup, 16-row token tiles, K slices}. */
+#define LMX_GEMM_SCRATCH 40
+int lmx_op_gemm_form(int32_t dtype, int32_t M, int32_t N, int32_t K, int32_t act, int64_t scratch_bytes, int32_t batch, int32_t* form);
 int lmx_op_gemv(int32_t dtype, const void* x, const void* w, void* c, const void* bias, const void* residual, const void* norm_w, float eps,
                 int32_t MB, int32_t N, int32_t K, int32_t ldx, int32_t ldw, int32_t ldc, int32_t ldr, int32_t act, void* stream);
 int lmx_op_rmsnorm(int32_t dtype, const void* x, const void* w, void* y, int32_t rows, int32_t H, float eps, void* stream);

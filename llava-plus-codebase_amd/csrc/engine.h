@@ -208,7 +208,7 @@ struct Model {
     void stack_seq_copy(Seq* dst, const Seq* src, hipStream_t st);
     struct Segment { int seq, src0, dst0, n, pos0; };    // rows [src0, src0 + n) of sequence `seq` sit at rows [dst0, ...) of the piece; first position pos0
     // a mixer over the normed rows x of a piece -> rows [an] of pitch out_k; qkv: its projection rows
-    void stack_mix_prefill(int r, Seq* const* seqs, const std::vector<Segment>& seg, int fill, const void* x, void* qkv, void* mix, void* scratch, void* skw, hipStream_t st);
+    void stack_mix_prefill(int r, Seq* const* seqs, const std::vector<Segment>& seg, int fill, const void* x, void* qkv, void* mix, void* scratch, const DevBuf& skw, hipStream_t st);
     size_t stack_mix_scratch(int rows, int keys) const;
     // the same over one new token of every sequence (tab: batch; else `one`), projection rows already there
     void stack_mix_decode(int r, const DecodeFusedSeq* tab, const DecodeFusedSeq& one, int n, int max_len, void* qkv, void* mix, const StackWs& w, Batch* b, hipStream_t st);

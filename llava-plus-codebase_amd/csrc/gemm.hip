@@ -676,6 +676,12 @@ static void launch_gemm_pipe(const GemmArgs& a, hipStream_t st) {
     LMX_CHECK_HIP(hipGetLastError());
 }
 
+int gemm_slices(const GemmArgs& a) {
+    int s = a.skw ? gemm8p_pick_split(a.M, a.N, a.K) : 1;
+    while (s > 1 && gemm8p_splitk_ws_bytes(a.M, a.N, s) > a.skw_bytes) --s;
+    return s;
+}
+
 template <typename T>
 static void launch_gemm16(const GemmArgs& a, int variant, hipStream_t st) {
     // variant: 0 = auto, 2 = 128x128 reg-staged (kept as an independent cross-check of the LDS-DMA path), 4 = 64x128 glds, 5 = 64x64 glds,
@@ -691,7 +697,7 @@ static void launch_gemm16(const GemmArgs& a, int variant, hipStream_t st) {
         // the partial-tile scratch (the engine does, per sequence; LMX_GEMM8P=0 switches the kernel off: the ring kernels below as an A/B and cross-check).
         if (gemm8p_enabled()) {
             const int tiles = cdiv(a.M, 256) * cdiv(a.N, 256);
-            const int S = a.skw ? gemm8p_pick_split(a.M, a.N, a.K) : 1;
+            const int S = gemm_slices(a);
             if (tiles * S >= 160) { GemmArgs b = a; b.split_k = S; launch_gemm8p(TypeInfo<T>::id, b, st); return; }
         }
         // Tile choice from the round-1 microbenchmarks (profiles/r01_microbench.jsonl).  The pipelined ring kernels are

@@ -18,10 +18,11 @@ struct GemmArgs {
     int ldx, ldw, ldc, ldr;
     int act;            // lmx::Act
     const void* Wsw = nullptr;   // skinny kernel only: W re-laid in MFMA-fragment order (skinny_swizzle), else null
-    // ping-pong kernel (gemm8p.hip) only: K slices per 256x256 tile (0 = let the launcher pick) and the fp32 partial-tile scratch
-    // (gemm8p_splitk_ws_bytes; null = the launcher's own, one stream at a time)
-    int split_k = 0;
+    int split_k = 0;             // ping-pong kernel (gemm8p.hip): K slices per 256x256 tile (0 = let the launcher pick)
+    // fp32 scratch of the K slices and what it holds: every rule takes only as many slices as fit, every launcher refuses more.  Null: the ping-pong kernel takes the
+    // launcher's own (one stream at a time), the others do not slice
     void* skw = nullptr;
+    size_t skw_bytes = 0;
     int* sk_cnt = nullptr;       // skinny kernel's K slices across workgroups: one arrival ticket per workgroup of rows (N / 16 at most), zero before the first launch (the last arriver re-arms)
     // q|k|v projection of a prefill with RoPE and the KV-cache append in the EPILOGUE (gemm8p.hip: qkv_rope_epilogue; where gemm_fuses_qkv()
     // says so): the tile is rounded to T into LDS and leaves the workgroup as  q rows -> rotated, into C (the q columns; k | v columns of C are not
@@ -51,13 +52,15 @@ int gemm8p_pick_split(int M, int N, int K);
 bool gemm_rows_applies(int dtype, const GemmArgs& a);
 struct RowsForm { int mtiles, bn, slices; };
 RowsForm gemm_rows_form(int dtype, const GemmArgs& a);                // the form variant 0 takes (mtiles 0: another kernel)
-constexpr size_t ROWS_SLAB_MAX = (size_t)64 << 20;                    // what a caller's a.skw holds
 size_t gemm_rows_slab_bytes(int M, int N, int S);
 void launch_gemm_rows(int dtype, const GemmArgs& a, int mtiles, int BN, int S, hipStream_t st);
 // decode-batch linear (skinny.hip): M <= 32 rows, 16-bit, weights streamed once straight into MFMA operands; variant 20 of launch_gemm
 void launch_skinny_gemm(int dtype, const GemmArgs& a, hipStream_t st);
 constexpr int SKINNY_SLICED_N = 8192;              // linears this wide and wider fill the CUs without K slices
 size_t skinny_scratch_bytes(int N);               // fp32 partial tiles of one launch (a.skw); tickets: N / 16 ints (a.sk_cnt)
+struct SkinnyForm { int rt, ks; };                // 16-row weight tiles of a workgroup, K slices
+SkinnyForm skinny_form(const GemmArgs& a);
+int gemm_slices(const GemmArgs& a);               // K slices of the ping-pong kernel under launch_gemm's own choice: what its rule says and a.skw holds
 // fragment-order copy of a [N, K] weight for the skinny kernel: per (16-row tile, 128-k super-step) four 1-KiB pieces, piece j =
 // lane-linear 16-byte A fragments of MFMA step j (lane = 16 q + i holds row i, k = 32 q + 8 j ...), K zero-padded to 128
 size_t skinny_swizzled_bytes(int N, int K, int es);

@@ -319,8 +319,7 @@ size_t skinny_scratch_bytes(int N) { return (size_t)cdiv(N, 64) * 8 * (4 * 2 * 2
 //   22016 x 4096 gated  2: 32.3 / 36.8   4: 36.8 / 42.8      4096 x 11008  1: 20.0 / 25.3   2 x 2: 20.5 / 23.3   4 x 4: 21.5 / 24.2
 //   27648 x 5120 gated  2: 52.7 / 61.2   4: 49.8 / 58.1      4096 x  4096  1: 11.4 / 13.0   2 x 2: 12.7 / 13.8
 //   12288 x 4096  1: 23.6 / 29.9   2: 25.0 / 28.3   4: 22.8 / 26.1       6208 x 4096  1: 16.9 / 19.3   2: 15.1 / 18.8   4 x 2: 16.4 / 18.1
-struct SkinnyForm { int rt, ks; };
-static SkinnyForm skinny_form(const GemmArgs& a) {
+SkinnyForm skinny_form(const GemmArgs& a) {
     const bool gated = act_gated(a.act), slices = !gated && a.skw && a.sk_cnt && a.N % 64 == 0 && a.N < SKINNY_SLICED_N;
     const int ct = a.M > 16 ? 2 : 1, nsuper = cdiv(a.K, SK_SUPER);
     const double weights = (double)a.N * a.K / (4096.0 * 11008.0);
@@ -331,6 +330,7 @@ static SkinnyForm skinny_form(const GemmArgs& a) {
         const int tiles = cdiv(a.N, 16 * rt);
         for (int ks = 1; ks <= (slices ? 4 : 1); ks *= 2) {
             if (ks > 1 && nsuper / ks < 8) break;                       // two super-steps for each of a slice's waves
+            if (ks > 1 && (size_t)tiles * ks * rt * ct * 1024 > a.skw_bytes) break;
             const double even = (double)tiles * ks / (256.0 * cdiv(tiles * ks, 256));
             const double cost = (1 + 0.25 * ct / rt) * (1 + 0.42 * (1 / even - 1)) * (1 + (ks == 1 ? 0.0 : ks == 2 ? 0.15 : 0.30) / weights);
             if (cost < least) { least = cost; best = SkinnyForm{rt, ks}; }

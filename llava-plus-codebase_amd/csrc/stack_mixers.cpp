@@ -53,7 +53,7 @@ size_t Model::stack_mix_scratch(int rows, int keys) const {
     return most;
 }
 
-void Model::stack_mix_prefill(int r, Seq* const* seqs, const std::vector<Segment>& seg, int fill, const void* x, void* qkv, void* mix, void* scratch, void* skw, hipStream_t st) {
+void Model::stack_mix_prefill(int r, Seq* const* seqs, const std::vector<Segment>& seg, int fill, const void* x, void* qkv, void* mix, void* scratch, const DevBuf& skw, hipStream_t st) {
     Stack& S = *stk;
     const StackRun& run = S.runs[(size_t)r];
     const StackLayer& l = S.layers[(size_t)run.layer];
@@ -64,7 +64,7 @@ void Model::stack_mix_prefill(int r, Seq* const* seqs, const std::vector<Segment
     auto gemm = [&](const char* name, GemmArgs g) { LMX_PROF_K(name);
         // inner sizes of a few K-steps: the time is the launch's fixed part and the output; the smaller tiles write it sooner than the large ones
         const int v = gv == 0 && dt != kF32 && g.K <= 512 ? (g.K <= 256 ? 5 : 18) : gv;
-        g.skw = g.K >= 1024 ? skw : nullptr;
+        if (g.K >= 1024) { g.skw = skw.p; g.skw_bytes = skw.bytes; }
         launch_gemm(dt, g, v, st); };
     if (d.mixer == LMX_MIXER_DELTA) {
         DeltaPrefillArgs a{};

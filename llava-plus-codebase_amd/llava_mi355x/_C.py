@@ -15,6 +15,7 @@ LIB_PATH = os.path.join(_HERE, "libllava_mi355x.so")
 LMX_ABI_VERSION = 2
 DTYPE_F32, DTYPE_BF16, DTYPE_F16 = 0, 1, 2
 ACT_NONE, ACT_QUICK_GELU, ACT_GELU_ERF, ACT_SILU_MUL, ACT_RELU_MUL = 0, 1, 2, 3, 4
+GEMM_SCRATCH = 40                # variant of lmx_op_gemm: LMX_GEMM_SCRATCH
 MIXER_ATTENTION, MIXER_LATENT, MIXER_DELTA = 0, 1, 2
 PROJ_LINEAR, PROJ_MLP_GELU, PROJ_IDENTITY = 0, 1, 2
 FEATURE_PATCH, FEATURE_CLS_PATCH = 0, 1
@@ -124,6 +125,7 @@ _SIGS = {
     "lmx_profile_read": (c_int32, [c_void_p, c_void_p, c_int32, c_void_p, c_void_p, c_int32, _i32p]),
     "lmx_model_set_option": (c_int32, [c_void_p, ctypes.c_char_p, c_int32]),
     "lmx_op_gemm": (c_int32, [c_int32, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p] + [c_int32] * 9 + [c_void_p]),
+    "lmx_op_gemm_form": (c_int32, [c_int32] * 5 + [c_int64, c_int32, POINTER(c_int32)]),
     "lmx_op_gemv": (c_int32, [c_int32, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_float] + [c_int32] * 8 + [c_void_p]),
     "lmx_op_rmsnorm": (c_int32, [c_int32, c_void_p, c_void_p, c_void_p, c_int32, c_int32, c_float, c_void_p]),
     "lmx_op_layernorm": (c_int32, [c_int32, c_void_p, c_void_p, c_void_p, c_void_p, c_int32, c_int32, c_float, c_void_p]),

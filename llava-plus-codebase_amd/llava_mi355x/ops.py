@@ -2,6 +2,7 @@
 tests and microbenchmarks.  torch tensors are containers only (pointers + current stream)."""
 from __future__ import annotations
 
+import ctypes
 import math
 
 import torch
@@ -39,6 +40,13 @@ def gemm(x, w, bias=None, residual=None, act=_C.ACT_NONE, variant=0, out=None):
                           x.stride(0), w.stride(0), out.stride(0), residual.stride(0) if residual is not None else 0,
                           act, variant, stream_handle()), "gemm")
     return out
+
+
+def gemm_form(dtype, M, N, K, act=_C.ACT_NONE, scratch_bytes=64 << 20, batch=False):
+    """What launch_gemm (batch: the decode batch's linears) takes for such a product and scratch, as lmx_op_gemm_form describes it.  No GPU needed."""
+    form = (ctypes.c_int32 * 4)()
+    check(lib.lmx_op_gemm_form(torch_dtype_code(dtype), M, N, K, act, scratch_bytes, int(batch), form), "gemm_form")
+    return tuple(form)
 
 
 def gemv(x, w, bias=None, residual=None, norm_w=None, eps=1e-5, act=_C.ACT_NONE, out=None):

@@ -1,0 +1,34 @@
+"""Which form of a linear a call takes (csrc/gemm_rows.hip: gemm_rows_form, csrc/skinny.hip: skinny_form), asked of the library on the host: K slices never need more scratch than
+the caller brings."""
+import pytest
+import torch
+
+ROWS = [(20, 4096, 11008), (139, 12288, 4096), (139, 4096, 11008), (250, 4096, 11008), (300, 4096, 4096), (512, 4096, 11008), (1087, 4096, 11008)]
+BATCH = [(2, 1088, 11008), (16, 640, 13824), (32, 2048, 13824), (32, 4032, 13824), (32, 4096, 11008), (32, 5120, 13824)]
+
+
+@pytest.mark.parametrize("M,N,K", ROWS)
+def test_slices_fit_the_scratch(M, N, K):
+    from llava_mi355x import ops
+    full = ops.gemm_form(torch.bfloat16, M, N, K)
+    assert full[3] > 1
+    for s in range(1, full[3] + 1):
+        for short in (0, 1):                            # room for s slices, and one byte less
+            room = s * (M if full[0] else -(-M // 256) * 256) * (N if full[0] else -(-N // 256) * 256) * 4
+            form = ops.gemm_form(torch.bfloat16, M, N, K, scratch_bytes=room - short)
+            if form[0] == full[0]:
+                assert form[3] <= max(1, s - short)
+            assert form[3] == 1 or form[3] * M * N * 4 <= room
+    assert ops.gemm_form(torch.bfloat16, M, N, K, scratch_bytes=0)[3] == 1
+
+
+@pytest.mark.parametrize("M,N,K", BATCH)
+def test_slices_of_a_decode_batch_fit_the_scratch(M, N, K):
+    from llava_mi355x import ops
+    _, rt, ct, ks = ops.gemm_form(torch.bfloat16, M, N, K, batch=True)
+    need = -(-N // (16 * rt)) * ks * rt * ct * 1024
+    assert need <= 64 << 20
+    if ks > 1:
+        assert ops.gemm_form(torch.bfloat16, M, N, K, batch=True, scratch_bytes=need) == (0, rt, ct, ks)
+        assert ops.gemm_form(torch.bfloat16, M, N, K, batch=True, scratch_bytes=need - 1) != (0, rt, ct, ks)
+    assert ops.gemm_form(torch.bfloat16, M, N, K, batch=True, scratch_bytes=0)[3] == 1

@@ -67,3 +67,19 @@ def test_rule(cuda, M, N, K, ldc):
     ref = x.double() @ w.double().t()
     assert_one_ulp(got, ref, "bf16", 2e-5 * float(ref.abs().max()), f"{M}x{N}x{K}")
     assert ldc == N or not bool(out[:, N:].any())
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("form,M,N,K", [((1, 64, 2), 64, 6144, 2048), ((1, 64, 3), 33, 3072, 2048), ((1, 64, 4), 2, 2048, 4096), ((1, 128, 2), 129, 12288, 2048), ((1, 128, 4), 129, 8192, 8192),
+                                        ((1, 128, 5), 200, 6144, 8192), ((1, 128, 6), 139, 3072, 8192), ((2, 128, 2), 257, 6144, 2048), ((2, 128, 3), 290, 3072, 2048), ((2, 128, 4), 257, 2048, 4096)])
+def test_slices_of_the_rule(cuda, dt, form, M, N, K):
+    """The slice counts that the rule itself picks with a prefill's scratch; three launches on the same slabs, another input between."""
+    from llava_mi355x import _C, ops
+    assert ops.gemm_form(DT[dt], M, N, K) == (1,) + form
+    x, w = _mk(M, N, K, dt, cuda, M + N)
+    r = torch.randn(M, N, device=cuda).to(DT[dt])
+    ref = x.double() @ w.double().t() + r.double()
+    got = ops.gemm(x, w, residual=r, variant=_C.GEMM_SCRATCH)
+    assert_one_ulp(got, ref, dt, 2e-5 * float(ref.abs().max()), f"{M}x{N}x{K}")
+    ops.gemm(-x, w, residual=r, variant=_C.GEMM_SCRATCH)
+    assert torch.equal(got, ops.gemm(x, w, residual=r, variant=_C.GEMM_SCRATCH))

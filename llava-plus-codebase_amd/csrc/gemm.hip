@@ -763,11 +763,11 @@ void launch_gemm(int dtype, const GemmArgs& a, int variant, hipStream_t st) {
         launch_gemm8p(dtype, b, st);
         return;
     }
-    if (variant >= 1000) { launch_gemm_rows(dtype, a, variant / 1000, variant / 100 % 10 * 64, variant % 100, st); return; }
     LMX_REQUIRE(a.N % 8 == 0, "gemm: N must be a multiple of 8");
     LMX_REQUIRE(!a.c_f32 || (!a.skw && !a.pk_kc && !a.qf_kc && !a.R && !act_gated(a.act)), "gemm: fp32 output is for plain un-split linears");
     if (act_gated(a.act)) LMX_REQUIRE(a.N % 64 == 0, "gemm: SiLU·mul needs N (fused gate|up rows) % 64 == 0");
     if (dtype == kF32) {
+        LMX_REQUIRE(variant < 1000, "gemm: the row-tile forms are for 16-bit dtypes");
         LMX_REQUIRE(a.K % 16 == 0, "gemm f32: K must be a multiple of 16");
         const int mtiles = cdiv(a.M, 64), ntiles = cdiv(a.N, 64);
         LMX_LAUNCH(gemm_f32_kernel, dim3(mtiles * ntiles), dim3(256), 0, st, a);
@@ -776,6 +776,7 @@ void launch_gemm(int dtype, const GemmArgs& a, int variant, hipStream_t st) {
     }
     LMX_REQUIRE(a.K % GEMM_BK == 0, "gemm: K must be a multiple of 64 (pad the operand)");
     LMX_REQUIRE(a.ldx % 8 == 0 && a.ldw % 8 == 0 && a.ldc % 4 == 0, "gemm: leading dims must keep 16-byte row alignment");
+    if (variant >= 1000) { launch_gemm_rows(dtype, a, variant / 1000, variant / 100 % 10 * 64, variant % 100, st); return; }
     if (dtype == kBF16) launch_gemm16<bf16_t>(a, variant, st);
     else if (dtype == kF16) launch_gemm16<f16_t>(a, variant, st);
     else throw Error{"gemm: bad dtype"};

@@ -32,3 +32,15 @@ def test_slices_of_a_decode_batch_fit_the_scratch(M, N, K):
         assert ops.gemm_form(torch.bfloat16, M, N, K, batch=True, scratch_bytes=need) == (0, rt, ct, ks)
         assert ops.gemm_form(torch.bfloat16, M, N, K, batch=True, scratch_bytes=need - 1) != (0, rt, ct, ks)
     assert ops.gemm_form(torch.bfloat16, M, N, K, batch=True, scratch_bytes=0)[3] == 1
+
+
+@pytest.mark.parametrize("dt,N,K,ldx,ldw,words", [(torch.bfloat16, 256, 128, 132, 128, "16-byte row alignment"), (torch.float16, 256, 128, 128, 129, "16-byte row alignment"),
+                                                  (torch.bfloat16, 250, 128, 128, 128, "multiple of 8"), (torch.bfloat16, 256, 96, 96, 96, "multiple of 64"), (torch.float32, 256, 128, 128, 128, "16-bit dtypes")])
+@pytest.mark.parametrize("variant", [1101, 2201])
+def test_a_form_by_number_checks_what_the_choice_checks(dt, N, K, ldx, ldw, words, variant):
+    """Refused on the host, before anything is allocated or launched (the pointers are not memory)."""
+    import ctypes
+    from llava_mi355x import _C
+    any_ = ctypes.c_void_p(4096)
+    assert _C.lib.lmx_op_gemm(_C.torch_dtype_code(dt), any_, any_, any_, None, None, 64, N, K, ldx, ldw, N, 0, 0, variant, None) != 0
+    assert words in _C.last_error()

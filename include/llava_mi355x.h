@@ -119,6 +119,8 @@ int lmx_stack_set_rope(lmx_model* m, int32_t table, int32_t dims, const float* h
 /* widths of the rows this model exchanges: embedding / residual rows (elements), logit rows (elements), dtype of logits, layer runs (cache slots; rows of a residual trace) */
 int lmx_row_pitch(const lmx_model* m);
 int lmx_input_pitch(const lmx_model* m);      /* elements of an input row of lmx_prefill* (lmx_gather_embeds writes such rows): the embedding row, or the id (see bigram_buckets) */
+/* keys that a cache row of a model of this dtype and max_position takes memory for: max_position in whole 128s, and at most 1/16 more (16-bit caches of 2048 keys and more) */
+int32_t lmx_kv_row_pitch(int32_t dtype, int32_t max_position);
 int lmx_recurrent(const lmx_model* m);        /* 1: a sequence carries state that cannot be cut back to an earlier position (lmx_seq_truncate keeps all of it or nothing) */
 int lmx_vocab_pitch(const lmx_model* m);
 int lmx_logit_dtype(const lmx_model* m);

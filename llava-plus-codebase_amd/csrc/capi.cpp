@@ -54,6 +54,7 @@ int lmx_stack_set_rope(lmx_model* m, int32_t table, int32_t dims, const float* h
 }
 int lmx_row_pitch(const lmx_model* m) { return m ? m->impl.H : -1; }
 int lmx_input_pitch(const lmx_model* m) { return m ? m->impl.input_pitch() : -1; }
+int32_t lmx_kv_row_pitch(int32_t dtype, int32_t max_position) { return kv_row_pitch(dtype, (max_position > 0 ? max_position + 127 : 2048) / 128 * 128); }
 int lmx_recurrent(const lmx_model* m) { return m ? (m->impl.fixed_context() ? 1 : 0) : -1; }
 int lmx_vocab_pitch(const lmx_model* m) { return m ? m->impl.V : -1; }
 int lmx_logit_dtype(const lmx_model* m) { return m ? m->impl.logit_dtype() : -1; }

@@ -63,7 +63,7 @@ Model::Model(const lmx_config& c) : cfg(c) {
     // a TP=1 token, 40 % of a TP=8 token if replicated); replicated when the vocabulary does not split into 8-row-aligned shards
     if (c.tp_world > 1 && V % (8 * c.tp_world) == 0) { V_l = V / c.tp_world; v_off = c.tp_rank * V_l; } else { V_l = V; v_off = 0; }
     s_max = round_up(c.max_position > 0 ? c.max_position : 2048, 128);   // decode attention works in 128-key chunks
-    kv_pitch = s_max + (c.dtype != kF32 && s_max % 256 == 0 ? 128 : 0);
+    kv_pitch = kv_row_pitch(c.dtype, s_max);
     dec.resize(L);
 
     if (c.v_layers > 0) {

@@ -98,6 +98,11 @@ struct StackOutputs {
 struct Seq;
 struct Batch;
 
+// Keys a row of the K / V^T caches has room for, >= s_max.  The rows of V^T are this far apart: an odd multiple of 256 bytes for 16-bit caches of 2048 keys and more, because rows a
+// power of two apart share memory channels (a batched decode's cache stream, 16 sequences of ~800 keys: 4.9 TB/s at 2048 keys a row, 5.6 at 2176).  It costs 128 keys of
+// memory a row, K rows too: 1/16 at 2048 keys and less above.  Shorter caches pay nothing: at 256 keys it would be half of their size again.
+inline int kv_row_pitch(int dtype, int s_max) { return s_max + (dtype != kF32 && s_max >= 2048 && s_max % 256 == 0 ? 128 : 0); }
+
 struct Model {
     lmx_config cfg{};
     int es = 2;                 // element size
@@ -105,9 +110,7 @@ struct Model {
     std::unique_ptr<Stack> stk; // set: a layer-stack decoder instead of the LLaMA decoder
     // decoder geometry (TP-local)
     int H = 0, I_l = 0, I_sh = 0, nh_l = 0, nkv_l = 0, D = 0, V = 0, L = 0, qkv_n = 0, s_max = 0;
-    // keys a cache row has room for, >= s_max.  The rows of V^T are this far apart: an odd multiple of 256 bytes for 16-bit caches, because rows a power of two apart share memory
-    // channels (a batched decode's cache stream, 16 sequences of ~800 keys: 4.9 TB/s at 2048 keys a row, 5.6 at 2176)
-    int kv_pitch = 0;
+    int kv_pitch = 0;           // keys a cache row has room for: kv_row_pitch(dtype, s_max)
     int V_l = 0, v_off = 0;     // lm_head rows held by this rank (vocabulary-parallel head under TP) and the id of its first row
     int Vr = 0;                 // ids a pick may return (real vocabulary, lmx_set_vocab_limit); V is the padded row pitch of logits / embeddings
     // vision geometry

@@ -37,7 +37,7 @@ Model::Model(const lmx_stack_config& c, const lmx_layer_config* layers) {
     V = round_up(c.vocab_size, 8); Vr = c.vocab_size; V_l = V; v_off = 0;
     les = 4;
     s_max = round_up(c.max_position > 0 ? c.max_position : 2048, 128);
-    kv_pitch = s_max + (c.dtype != kF32 && s_max % 256 == 0 ? 128 : 0);
+    kv_pitch = kv_row_pitch(c.dtype, s_max);
     S.layers.resize((size_t)c.n_layers);
     for (int i = 0; i < c.n_layers; ++i) {
         StackLayer& l = S.layers[(size_t)i];

@@ -80,6 +80,7 @@ _SIGS = {
     "lmx_row_pitch": (c_int32, [c_void_p]),
     "lmx_input_pitch": (c_int32, [c_void_p]),
     "lmx_recurrent": (c_int32, [c_void_p]),
+    "lmx_kv_row_pitch": (c_int32, [c_int32, c_int32]),
     "lmx_vocab_pitch": (c_int32, [c_void_p]),
     "lmx_logit_dtype": (c_int32, [c_void_p]),
     "lmx_layer_runs": (c_int32, [c_void_p]),

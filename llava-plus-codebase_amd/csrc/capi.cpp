@@ -63,8 +63,10 @@ int lmx_destroy(lmx_model* m) {
     LMX_API_BEGIN
     if (m) {
         (void)hipDeviceSynchronize();
+        std::lock_guard<std::mutex> lk(m->impl.pool_mu);
         for (lmx_seq* s : m->impl.seq_pool) delete s;
         m->impl.seq_pool.clear();
+        for (lmx_seq* s : m->impl.seq_out) s->impl.m = nullptr;
     }
     delete m;
     LMX_API_END
@@ -228,6 +230,10 @@ int lmx_seq_create(lmx_model* m, lmx_seq** out) {
         s = new lmx_seq(&m->impl);
     }
     m->impl.live_seqs.fetch_add(1, std::memory_order_relaxed);
+    {
+        std::lock_guard<std::mutex> lk(m->impl.pool_mu);
+        m->impl.seq_out.insert(s);
+    }
     *out = s;
     LMX_API_END
 }
@@ -235,7 +241,11 @@ int lmx_seq_destroy(lmx_seq* s) {
     LMX_API_BEGIN
     if (!s) return 0;
     Model* m = s->impl.m;
-    if (m) m->live_seqs.fetch_sub(1, std::memory_order_relaxed);
+    if (m) {
+        m->live_seqs.fetch_sub(1, std::memory_order_relaxed);
+        std::lock_guard<std::mutex> lk(m->pool_mu);
+        m->seq_out.erase(s);
+    }
     bool pooled = false;
     bool idle_known = true;
     if (m && s->impl.used) {
@@ -830,13 +840,13 @@ int lmx_prefill_batch_logits(lmx_model* m, lmx_seq* const* seqs, int32_t n, cons
 }
 int lmx_seq_copy(lmx_seq* dst, const lmx_seq* src, void* stream) {
     LMX_API_BEGIN
-    LMX_REQUIRE(dst && src, "null argument");
+    LMX_REQUIRE(dst && src && dst->impl.m, "null argument");
     dst->impl.m->seq_copy(&dst->impl, &src->impl, S(stream));
     LMX_API_END
 }
 int lmx_seq_truncate(lmx_seq* s, int32_t n_rows, void* stream) {
     LMX_API_BEGIN
-    LMX_REQUIRE(s, "null sequence");
+    LMX_REQUIRE(s && s->impl.m, "null sequence");
     LMX_REQUIRE(n_rows >= 0 && n_rows <= s->impl.len, "seq_truncate: 0 <= n_rows <= current length");
     LMX_REQUIRE(n_rows == 0 || n_rows == s->impl.len || !s->impl.m->fixed_context(), "seq_truncate: this model's sequences carry state that cannot be cut back");
     // a finished request's sequence starts another request that shares its first n_rows positions (prefix reuse): keep K / V^T rows [0, n_rows), forget the

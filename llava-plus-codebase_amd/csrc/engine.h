@@ -131,6 +131,7 @@ struct Model {
     // Sequence pool: a finished request's KV caches / workspaces (≈ 1 GB at 7B, s_max 2048) are handed to the next request instead of
     // hipFree + hipMalloc — hipFree synchronises the whole device, which stalls every other request of a busy worker.
     std::mutex pool_mu; std::vector<struct lmx_seq*> seq_pool; size_t seq_pool_max = 64;
+    std::set<struct lmx_seq*> seq_out;   // handed out, not yet destroyed: lmx_destroy cuts them loose, so that they may outlive the model (a collector's order is arbitrary)
     size_t seq_pool_bytes = 0, seq_pool_bytes_max = (size_t)96 << 30;
     DevBuf vws;                 // vision workspace
     int vws_images = 0;

@@ -449,7 +449,7 @@ static void skinny_op(int32_t dtype, GemmArgs g, int32_t variant, hipStream_t st
         std::lock_guard<std::mutex> lk(mu2);
         const size_t need = skinny_scratch_bytes(g.N), ncnt = (size_t)(g.N / 16 + 1) * sizeof(int);
         if (sk_scratch.bytes < need || sk_cnt.bytes < ncnt) { LMX_CHECK_HIP(hipDeviceSynchronize()); sk_scratch.ensure(need); sk_cnt.ensure(ncnt, true); }
-        g.skw = sk_scratch.p; g.skw_bytes = sk_scratch.bytes; g.sk_cnt = sk_cnt.as<int>();
+        g.scratch(sk_scratch.p, sk_scratch.bytes); g.sk_cnt = sk_cnt.as<int>();
         variant = variant == 23 ? 22 : 21;
     }
     if (variant == 21 || variant == 22) {
@@ -488,9 +488,9 @@ int lmx_op_gemm(int32_t dtype, const void* x, const void* w, void* c, const void
         static std::mutex mu;
         static DevBuf slab;
         std::lock_guard<std::mutex> lk(mu);
-        const size_t need = variant >= 1000 ? gemm_rows_slab_bytes(M, N, variant % 100) : (size_t)64 << 20;
+        const size_t need = variant >= 1000 ? (gemm_rows_slab_bytes(M, N, variant % 100) + 1023) / 1024 * 1024 : (size_t)64 << 20;
         if (slab.bytes < need) { LMX_CHECK_HIP(hipDeviceSynchronize()); slab.ensure(need); }
-        g.skw = slab.p; g.skw_bytes = variant >= 1000 ? slab.bytes : need;
+        g.scratch(slab.p, variant >= 1000 ? slab.bytes : need);
         launch_gemm(dtype, g, variant >= 1000 ? variant : 0, S(stream));
         return 0;
     }
@@ -502,7 +502,7 @@ int lmx_op_gemm_form(int32_t dtype, int32_t M, int32_t N, int32_t K, int32_t act
     LMX_REQUIRE(form && M > 0 && N > 0 && K > 0 && scratch_bytes >= 0, "gemm_form: bad arguments");
     void* const any = reinterpret_cast<void*>((uintptr_t)4096);              // aligned; nothing is read or launched
     GemmArgs g{any, any, any, nullptr, nullptr, M, N, K, K, K, act_gated(act) ? N / 2 : N, 0, act};
-    if (scratch_bytes > 0) { g.skw = any; g.skw_bytes = (size_t)scratch_bytes; g.sk_cnt = static_cast<int*>(any); }
+    if (scratch_bytes > 0) { g.scratch(any, (size_t)scratch_bytes); g.sk_cnt = static_cast<int*>(any); }
     form[0] = form[1] = form[2] = 0; form[3] = 1;
     if (batch) {
         const SkinnyForm f = skinny_form(g);

@@ -617,7 +617,7 @@ void Model::prefill(Seq* s, const void* embeds, int T, int chunk, void* logits, 
         LMX_CHECK_HIP(hipStreamSynchronize(st));
         s->skw.ensure((size_t)256 * 256 * 256 * sizeof(float));
     }
-    auto with_scratch = [&](GemmArgs g) { g.skw = s->skw.p; g.skw_bytes = s->skw.bytes; return g; };
+    auto with_scratch = [&](GemmArgs g) { g.scratch(s->skw.p, s->skw.bytes); return g; };
 
     for (int c0 = 0; c0 < T; c0 += chunk) {
         const int tc = (T - c0) < chunk ? (T - c0) : chunk;
@@ -771,7 +771,7 @@ void Model::prefill_multi(Seq* const* seqs, const void* const* embeds, const int
         LMX_CHECK_HIP(hipStreamSynchronize(st));
         s0->skw.ensure((size_t)256 * 256 * 256 * sizeof(float));
     }
-    auto with_scratch = [&](GemmArgs g) { g.skw = s0->skw.p; g.skw_bytes = s0->skw.bytes; return g; };
+    auto with_scratch = [&](GemmArgs g) { g.scratch(s0->skw.p, s0->skw.bytes); return g; };
     auto rows = [&](void* base, long r0, size_t width) { return static_cast<char*>(base) + (size_t)r0 * width * es; };
     struct Segment { int seq, src0, dst0, n, pos0; };    // rows [src0, src0 + n) of sequence `seq` sit at rows [dst0, ...) of the piece; first position pos0
     int cur = 0, cur_done = 0;                           // next sequence / rows of it already consumed
@@ -1045,7 +1045,7 @@ void Model::decode_batch(Batch* b, Seq* const* seqs, int n, const int64_t* token
             g.X = x_normed; g.ldx = g.K;
         }
         LMX_PROF("decode_batch.linear");
-        if (dt != kF32 && g.M <= 32) { g.Wsw = wsw; g.skw = b->sk_scratch.p; g.skw_bytes = b->sk_scratch.bytes; g.sk_cnt = b->sk_cnt.as<int>(); launch_skinny_gemm(dt, g, st); } else launch_gemm(dt, g, cfg.gemm_variant, st);
+        if (dt != kF32 && g.M <= 32) { g.Wsw = wsw; g.scratch(b->sk_scratch.p, b->sk_scratch.bytes); g.sk_cnt = b->sk_cnt.as<int>(); launch_skinny_gemm(dt, g, st); } else launch_gemm(dt, g, cfg.gemm_variant, st);
     };
     if (n == 1) {
         // a lone member takes the single-sequence step (GEMV with fused RMSNorm: fewer launches, full-rate weight stream)

@@ -678,7 +678,7 @@ static void launch_gemm_pipe(const GemmArgs& a, hipStream_t st) {
 
 int gemm_slices(const GemmArgs& a) {
     int s = a.skw ? gemm8p_pick_split(a.M, a.N, a.K) : 1;
-    while (s > 1 && gemm8p_splitk_ws_bytes(a.M, a.N, s) > a.skw_bytes) --s;
+    while (s > 1 && gemm8p_splitk_ws_bytes(a.M, a.N, s) > a.skw_bytes()) --s;
     return s;
 }
 

@@ -594,9 +594,9 @@ static void launch_gemm8p_t(GemmArgs a, hipStream_t st) {
             if (g_fb.ws) (void)hipFree(g_fb.ws);
             LMX_CHECK_HIP(hipMalloc(&g_fb.ws, need)); g_fb.ws_bytes = need;
         }
-        a.skw = g_fb.ws; a.skw_bytes = g_fb.ws_bytes;
+        a.scratch(g_fb.ws, g_fb.ws_bytes);
     }
-    if (S > 1) LMX_REQUIRE(gemm8p_splitk_ws_bytes(a.M, a.N, S) <= a.skw_bytes, "gemm8p: the partial tiles do not fit the scratch");
+    if (S > 1) LMX_REQUIRE(gemm8p_splitk_ws_bytes(a.M, a.N, S) <= a.skw_bytes(), "gemm8p: the partial tiles do not fit the scratch");
     // A K-sliced GEMM is TWO launches; an armed kernel timer (in-situ profile) then spans both: start stamped at the GEMM's begin, stop at the reduction's
     // end, so the reported duration includes the boundary between them.
     const bool two = S > 1;

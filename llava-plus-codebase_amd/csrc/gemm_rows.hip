@@ -359,7 +359,7 @@ RowsForm gemm_rows_form(int dtype, const GemmArgs& a) {
         const int bn = few ? 64 : 128, tiles = mt * cdiv(a.N, bn);
         if (tiles <= 256) {
             int s = std::min(256 / tiles, few ? 4 : mt == 2 ? 4 : 6);
-            while (s > 1 && (nk / s < 10 || !a.skw || a.pk_kc || gemm_rows_slab_bytes(a.M, a.N, s) > a.skw_bytes)) --s;
+            while (s > 1 && (nk / s < 10 || !a.skw || a.pk_kc || gemm_rows_slab_bytes(a.M, a.N, s) > a.skw_bytes())) --s;
             if (tiles * s >= 128 && (few || s <= 2 || nk >= 128 || (mt == 2 && a.M <= 384))) return RowsForm{mt, bn, s};
         }
     }
@@ -375,7 +375,7 @@ RowsForm gemm_rows_form(int dtype, const GemmArgs& a) {
 
 void launch_gemm_rows(int dtype, const GemmArgs& a, int mtiles, int BN, int S, hipStream_t st) {
     LMX_REQUIRE(gemm_rows_applies(dtype, a) && mtiles >= 1 && cdiv(a.M, mtiles) <= 256 && (BN == 64 || BN == 128), "gemm_rows: shape or alignment");
-    LMX_REQUIRE(S >= 1 && S <= a.K / GEMM_BK && (S == 1 || (a.skw && gemm_rows_slab_bytes(a.M, a.N, S) <= a.skw_bytes && !a.pk_kc)), "gemm_rows: K slices");
+    LMX_REQUIRE(S >= 1 && S <= a.K / GEMM_BK && (S == 1 || (a.skw && gemm_rows_slab_bytes(a.M, a.N, S) <= a.skw_bytes() && !a.pk_kc)), "gemm_rows: K slices");
     // every M tile covers cdiv(rows per tile, 32) * 32 rows: the tiles that start past M are left out
     mtiles = cdiv(a.M, cdiv(cdiv(a.M, mtiles), 32) * 32);
     if (dtype == kBF16) { if (BN == 64) launch_rows_n<bf16_t, 64>(a, mtiles, S, st); else launch_rows_n<bf16_t, 128>(a, mtiles, S, st); }

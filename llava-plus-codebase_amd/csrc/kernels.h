@@ -19,10 +19,13 @@ struct GemmArgs {
     int act;            // lmx::Act
     const void* Wsw = nullptr;   // skinny kernel only: W re-laid in MFMA-fragment order (skinny_swizzle), else null
     int split_k = 0;             // ping-pong kernel (gemm8p.hip): K slices per 256x256 tile (0 = let the launcher pick)
-    // fp32 scratch of the K slices and what it holds: every rule takes only as many slices as fit, every launcher refuses more.  Null: the ping-pong kernel takes the
-    // launcher's own (one stream at a time), the others do not slice
+    // fp32 scratch of the K slices and what it holds, in whole KiB: every rule takes only as many slices as fit, every launcher refuses more.  (Four bytes where the struct had a
+    // hole: with every later field eight bytes further the kernels' argument loads were grouped differently, and a decode step of 32 sequences took 2 % longer.)  Null: the
+    // ping-pong kernel takes the launcher's own (one stream at a time), the others do not slice
+    uint32_t skw_kib = 0;
     void* skw = nullptr;
-    size_t skw_bytes = 0;
+    void scratch(void* p, size_t bytes) { skw = p; skw_kib = (uint32_t)(bytes >> 10); }
+    size_t skw_bytes() const { return (size_t)skw_kib << 10; }
     int* sk_cnt = nullptr;       // skinny kernel's K slices across workgroups: one arrival ticket per workgroup of rows (N / 16 at most), zero before the first launch (the last arriver re-arms)
     // q|k|v projection of a prefill with RoPE and the KV-cache append in the EPILOGUE (gemm8p.hip: qkv_rope_epilogue; where gemm_fuses_qkv()
     // says so): the tile is rounded to T into LDS and leaves the workgroup as  q rows -> rotated, into C (the q columns; k | v columns of C are not

@@ -330,7 +330,7 @@ SkinnyForm skinny_form(const GemmArgs& a) {
         const int tiles = cdiv(a.N, 16 * rt);
         for (int ks = 1; ks <= (slices ? 4 : 1); ks *= 2) {
             if (ks > 1 && nsuper / ks < 8) break;                       // two super-steps for each of a slice's waves
-            if (ks > 1 && (size_t)tiles * ks * rt * ct * 1024 > a.skw_bytes) break;
+            if (ks > 1 && (size_t)tiles * ks * rt * ct * 1024 > a.skw_bytes()) break;
             const double even = (double)tiles * ks / (256.0 * cdiv(tiles * ks, 256));
             const double cost = (1 + 0.25 * ct / rt) * (1 + 0.42 * (1 / even - 1)) * (1 + (ks == 1 ? 0.0 : ks == 2 ? 0.15 : 0.30) / weights);
             if (cost < least) { least = cost; best = SkinnyForm{rt, ks}; }

@@ -398,7 +398,7 @@ void Model::stack_prefill(Seq* const* seqs, const void* const* embeds, const int
         LMX_CHECK_HIP(hipStreamSynchronize(st));
         s0->skw.ensure((size_t)256 * 256 * 256 * sizeof(float));
     }
-    auto with_scratch = [&](GemmArgs g) { g.skw = s0->skw.p; g.skw_bytes = s0->skw.bytes; return g; };
+    auto with_scratch = [&](GemmArgs g) { g.scratch(s0->skw.p, s0->skw.bytes); return g; };
     auto rows = [&](void* base, long r0, size_t width) { return static_cast<char*>(base) + (size_t)r0 * width * es; };
     auto residual = [&](const float* xi, const void* yy, int top, const void* post, const void* inject, const void* pre, bool cast, int nr) {
         LMX_PROF("prefill.residual_norm");
@@ -721,7 +721,7 @@ void Model::stack_decode_batch_step(Batch* b, Seq* const* seqs, int n, int64_t* 
 void Model::stack_batch_linear(Batch* b, GemmArgs g, const void* wsw, hipStream_t st) {
     if (cfg.dtype != kF32 && g.M <= 32) {
         g.Wsw = wsw;
-        if (!g.c_f32) { g.skw = b->sk_scratch.p; g.skw_bytes = b->sk_scratch.bytes; g.sk_cnt = b->sk_cnt.as<int>(); }
+        if (!g.c_f32) { g.scratch(b->sk_scratch.p, b->sk_scratch.bytes); g.sk_cnt = b->sk_cnt.as<int>(); }
         launch_skinny_gemm(cfg.dtype, g, st);
     } else launch_gemm(cfg.dtype, g, cfg.gemm_variant, st);
 }

@@ -64,7 +64,7 @@ void Model::stack_mix_prefill(int r, Seq* const* seqs, const std::vector<Segment
     auto gemm = [&](const char* name, GemmArgs g) { LMX_PROF_K(name);
         // inner sizes of a few K-steps: the time is the launch's fixed part and the output; the smaller tiles write it sooner than the large ones
         const int v = gv == 0 && dt != kF32 && g.K <= 512 ? (g.K <= 256 ? 5 : 18) : gv;
-        if (g.K >= 1024) { g.skw = skw.p; g.skw_bytes = skw.bytes; }
+        if (g.K >= 1024) g.scratch(skw.p, skw.bytes);
         launch_gemm(dt, g, v, st); };
     if (d.mixer == LMX_MIXER_DELTA) {
         DeltaPrefillArgs a{};

@@ -123,7 +123,17 @@ __device__ __forceinline__ void decode_fused_body(DecodeFusedArgs a, const int h
         __syncthreads();
         const float p_new = has_new ? red[4] : 0.f;
 
-        // ---- o = P · V from the registers loaded above ---------------------------------------------------------------------
+        // ---- o = P · V from the registers loaded above; behind the cached keys P is 0 and the values are cleared (never 0 x NaN) -----------------------------
+        if (nk_cached < DF_CHUNK) {
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const bool in = kb * 64 + s8 * 8 + e < nk_cached;
+#pragma unroll
+                    for (int db = 0; db < DB; ++db) vv[kb][db][e] = in ? vv[kb][db][e] : 0.f;
+                }
+        }
         float acc[DB];
 #pragma unroll
         for (int db = 0; db < DB; ++db) acc[db] = 0.f;

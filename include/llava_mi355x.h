@@ -377,6 +377,9 @@ int lmx_op_decode_win(int32_t dtype, int32_t D, const void* qkv, int32_t qkv_str
                       const int32_t* const* pos_devs, void* const* ws_devs, int32_t* const* counters_devs, int32_t n_seq, void* tab_dev, const void* q_norm, const void* k_norm,
                       const float* cos_sin_dev, int32_t n_heads, int32_t n_kv_heads, int32_t s_max, int32_t n_split, int32_t qk_dim, int32_t rot_dims, int32_t window, int32_t sink,
                       int32_t gate_off, float scale, float eps, void* stream);
+/* what a decode step takes, on the host alone: form[2] = {all query heads of a kv head in one workgroup, splits}; span: keys that the longest sequence may have to walk.
+ * (lmx_op_decode_win itself gives every batch that it can to the grouped kernel.) */
+int lmx_op_decode_win_form(int32_t dtype, int32_t D, int32_t n_heads, int32_t n_kv_heads, int32_t n_seq, int32_t span, int32_t* form);
 int lmx_op_argmax(int32_t dtype, const void* logits, int32_t V, int64_t* out_tok_dev, void* stream);
 int lmx_op_im2col(int32_t dtype, const void* pixels, void* out, int32_t N, int32_t S, int32_t patch, int32_t kpad, void* stream);
 

@@ -534,7 +534,7 @@ void Model::stack_prefill(Seq* const* seqs, const void* const* embeds, const int
 // ---------------------------------------------------------------------------------------------------------------
 // decode
 // ---------------------------------------------------------------------------------------------------------------
-static WinDecodeArgs decode_args(const Stack& S, const StackLayer& l, int dtype, const void* qkv, void* out, int n_seq, int max_len, int s_max) {
+static WinDecodeArgs decode_args(const Stack& S, const StackLayer& l, int dtype, const void* qkv, void* out, int n_seq, int max_len, int s_max, bool& grouped) {
     const lmx_layer_config& d = l.c;
     WinDecodeArgs a;
     a.qkv = qkv; a.out = out; a.q_norm = l.qn; a.k_norm = l.kn; a.cos_sin = d.rope_dims ? S.rope[(size_t)d.rope_table] : nullptr;
@@ -543,11 +543,8 @@ static WinDecodeArgs decode_args(const Stack& S, const StackLayer& l, int dtype,
     // chunks the longest member's window can touch; enough workgroups to fill the chip, no more
     int span = max_len + 1;
     if (d.window > 0 && d.window + 127 < span) span = d.window + 127;
-    const int chunks = std::max(1, std::min((span + 127) / 128, 32));
-    const bool grouped = decode_win_grouped(dtype, l.D, d.n_heads, d.n_kv_heads, n_seq);
-    const int wgs = (grouped ? d.n_kv_heads : d.n_heads) * n_seq, want = grouped ? 256 : 1024;       // workgroups of one split
-    const int fill = (want + wgs - 1) / wgs;
-    a.n_split = std::max(1, std::min(chunks, fill));
+    const WinForm f = decode_win_form(dtype, l.D, d.n_heads, d.n_kv_heads, n_seq, span);
+    a.n_split = f.n_split; grouped = f.grouped;
     return a;
 }
 
@@ -625,10 +622,11 @@ void Model::stack_decode_step(Seq* s, hipStream_t st, int64_t* id_out) {
         top = 0;
         if (l.c.mixer == LMX_MIXER_ATTENTION) {
             LMX_PROF_K("decode.attn");
-            WinDecodeArgs a = decode_args(S, l, dt, s->d_qkv, s->d_attn, 1, s->len, kv_pitch);
+            bool grouped;
+            WinDecodeArgs a = decode_args(S, l, dt, s->d_qkv, s->d_attn, 1, s->len, kv_pitch, grouped);
             a.one = stack_seq_ref(r, s);
             a.pos = s->len;
-            launch_decode_win(dt, l.D, a, st);
+            launch_decode_win(dt, l.D, a, grouped, st);
         } else stack_mix_decode(r, nullptr, stack_seq_ref(r, s), 1, s->len, s->d_qkv, s->d_attn, s->sw, nullptr, st);
         if (l.parallel() && l.dense()) plain("decode.gemv.gate_up", s->d_x, l.wgu, static_cast<char*>(s->d_attn) + (size_t)l.an * es, 2 * l.ff, H, l.act());
         plain("decode.gemv.o", s->d_attn, l.wo, s->d_y, H, l.out_k);
@@ -694,9 +692,10 @@ void Model::stack_decode_batch_step(Batch* b, Seq* const* seqs, int n, int64_t* 
         const DecodeFusedSeq* tab = b->d_attn_tab + (size_t)r * b->cap;
         if (l.c.mixer == LMX_MIXER_ATTENTION) {
             LMX_PROF("decode_batch.attn");
-            WinDecodeArgs a = decode_args(S, l, dt, b->qkv, b->attn, n, max_len, kv_pitch);
+            bool grouped;
+            WinDecodeArgs a = decode_args(S, l, dt, b->qkv, b->attn, n, max_len, kv_pitch, grouped);
             a.tab = tab;
-            launch_decode_win(dt, l.D, a, st);
+            launch_decode_win(dt, l.D, a, grouped, st);
         } else stack_mix_decode(r, tab, DecodeFusedSeq{}, n, max_len, b->qkv, b->attn, b->sw, b, st);
         if (l.parallel() && l.dense()) linear(GemmArgs{b->x, l.wgu, static_cast<char*>(b->attn) + (size_t)l.an * es, nullptr, nullptr, n, 2 * l.ff, H, H, H, l.out_k, 0, l.act()}, l.sw_gu);
         linear(GemmArgs{b->attn, l.wo, b->y, nullptr, nullptr, n, H, l.out_k, l.out_k, l.out_k, H, 0, kActNone}, l.sw_o);

@@ -9,6 +9,7 @@
 //
 // Head vectors are stored padded to D in {64, 128, 256} lanes: the padding weights are zero, so padded lanes of q, k and v are zero and add nothing; the query / key
 // norm divides by the true width.
+#include <algorithm>
 #include <type_traits>
 
 #include "common.h"
@@ -647,7 +648,8 @@ __global__ __launch_bounds__(256) void decode_win_kernel(WinDecodeArgs a) {
 // Scores = K tile (16 keys) x query heads (16 columns), the softmax over the lane's 16 keys and 4 lanes, then V^T rows x probabilities.  The C layout of the scores (lane = head,
 // 4 rows a tile) is the B layout of the probabilities when row 4 q + r of tile t is key 8 q + 4 t + r of 32, so no probability changes lanes.  Probabilities keep fp32's 24
 // bits: three 16-bit terms, three MFMAs; f16 terms of a probability times 2^15, because f16 ends at 2^-24: without the factor a probability of 2^-12 kept 12 bits and one below 2^-25
-// none, with it the sums are off by 2^-40 a key.  Bound: the cache stream (32 sequences x 1024 keys, 8 kv heads of 128: 134 MB a launch); figures: decode_win_grouped.
+// none, with it the sums are off by 2^-40 a key.  Bound: the cache stream (32 sequences x 1024 keys, 8 kv heads of 128: 134 MB a launch): straight operand loads 36.9 us, whole lines through LDS with the next piece on the
+// wire 32.0 (4.2 TB/s), with one split (straight: 2 splits 36.4, 4 43.3: the merge and a shorter walk cost more than a fuller chip gives); which launches: decode_win_form.
 template <typename T> struct WinMfma;
 template <> struct WinMfma<bf16_t> {
     static __device__ __forceinline__ f32x4 run(const uint4& a, const uint4& b, f32x4 c) {
@@ -900,21 +902,36 @@ __global__ __launch_bounds__(256) void decode_win_group_kernel(WinDecodeArgs a) 
     if (tid == 0) __hip_atomic_store(ticket, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);          // re-arm for the next launch
 }
 
-// 16-bit caches of heads up to 128 wide, up to 16 query heads a kv head, more than one sequence.  32 sequences of 568 - 1300 keys, window 1024, 32 heads on 8 kv heads of 128:
-// one head a workgroup 86.7 us; keys and values straight into the operands 36.9; whole lines through LDS, the next piece on the wire 32.0 (4.2 TB/s) — one split (straight: 2 splits
-// 36.4, 4 43.3: the merge and a shorter walk cost more than a fuller chip gives).  One sequence of 601 keys, 16 heads on 4:
-// 11.1 us either way, all of it latency, so the form with more workgroups stays.
-bool decode_win_grouped(int dtype, int D, int n_heads, int n_kv_heads, int n_seq) {
+bool decode_win_groups(int dtype, int D, int n_heads, int n_kv_heads, int n_seq) {
     return dtype != kF32 && D <= 128 && n_heads / n_kv_heads <= WIN_GROUP_MAX && n_seq > 1;
 }
+// Which kernel and how many splits.  The grouped one reads a cached key once instead of once per query head, but has a group-th of the workgroups, a longer start and, over splits,
+// one workgroup that merges all heads of the group.  us, one head a workgroup -> grouped, 16-bit:
+//   32 heads on  8 of 128   32 sequences of 1024 keys 97 -> 31   8 of 130  13.4 -> 11.2    2 of 600  13.3 -> 11.4    4 of 20  8.1 -> 8.7    16 of 20  11.1 -> 9.4
+//   24 heads on 12          32 of 1200  84 -> 52                 2 of 130  10.4 -> 9.8     32 of 60  14 -> 17
+//    8 heads on  1          32 of 600   32 -> 14                 8 of 600  13 -> 13        2 of 600  10 -> 13        8 of 60  8 -> 10        (16 on 1: 16 of 600  23 -> 19, 4 of 600  12 -> 17)
+//   32 heads on 32           8 of 1200  45 -> 31                 16 of 600 46 -> 40        3 of 600  14 -> 15        16 of 60  11 -> 19      (16 of 64: 16 of 600  16 -> 13, 6 of 600  10 -> 11)
+// so: by the bytes that one head a workgroup asks for, more of them where the group is larger (the merge), and for groups of 2 - 4 from one chunk of keys on.  One sequence of 601
+// keys, 16 heads on 4: 11.1 us either way, all of it latency, so the form with more workgroups stays.
+// Splits: as many as make ONE round of workgroups of the grouped kernel (its waves fill a CU: 96 x 3 and 160 x 2 workgroups took a second round, 15 -> 19 and 21 -> 25 us).
+WinForm decode_win_form(int dtype, int D, int n_heads, int n_kv_heads, int n_seq, int span) {
+    const int group = n_heads / n_kv_heads, chunks = std::max(1, std::min((span + 127) / 128, DF_MAX_SPLIT));
+    const double mb = (double)n_heads * n_seq * span * D * 4e-6;
+    bool grouped = decode_win_groups(dtype, D, n_heads, n_kv_heads, n_seq);
+    if (group == 1) grouped = grouped && span >= 512 && mb >= 48;
+    else if (group <= 4) grouped = grouped && (span >= 128 || (group >= 3 && mb >= 8));
+    else grouped = grouped && mb >= 0.6 * group * group;
+    const int wgs = (grouped ? n_kv_heads : n_heads) * n_seq;
+    return WinForm{grouped, std::max(1, std::min(chunks, grouped ? 256 / wgs : (1024 + wgs - 1) / wgs))};
+}
 
-void launch_decode_win(int dtype, int D, const WinDecodeArgs& a, hipStream_t st) {
+void launch_decode_win(int dtype, int D, const WinDecodeArgs& a, bool grouped, hipStream_t st) {
     LMX_REQUIRE(D == 64 || D == 128 || D == 256, "decode_win: padded head width must be 64, 128 or 256");
     LMX_REQUIRE(a.s_max % DF_CHUNK == 0 && a.n_split >= 1 && a.n_split <= DF_MAX_SPLIT && a.n_seq >= 1, "decode_win: cache in whole 128-key chunks, 1..32 splits");
     LMX_REQUIRE(a.n_heads >= 1 && a.n_kv_heads >= 1 && a.n_heads % a.n_kv_heads == 0 && a.qkv && a.out, "decode_win: bad arguments");
     LMX_REQUIRE(a.rot_dims % 2 == 0 && a.rot_dims <= a.qk_dim && a.qk_dim <= D && (a.rot_dims == 0 || a.cos_sin), "decode_win: bad rotation");
     LMX_REQUIRE(a.tab || (a.n_seq == 1 && a.one.K && a.one.VT && a.one.ws && a.one.counters && (a.pos >= 0 || a.one.pos_ptr)), "decode_win: bad sequence");
-    if (decode_win_grouped(dtype, D, a.n_heads, a.n_kv_heads, a.n_seq) && a.qkv_stride % 4 == 0 && reinterpret_cast<uintptr_t>(a.qkv) % 8 == 0) {
+    if (grouped && decode_win_groups(dtype, D, a.n_heads, a.n_kv_heads, a.n_seq) && a.qkv_stride % 4 == 0 && reinterpret_cast<uintptr_t>(a.qkv) % 8 == 0) {
         const dim3 grid(a.n_kv_heads, a.n_split, a.n_seq);
         const int smem = win_group_smem(a.n_heads / a.n_kv_heads, D);
 #define L(TT, DD)                                                                                                                                          \

@@ -315,16 +315,20 @@ size_t skinny_scratch_bytes(int N) { return (size_t)cdiv(N, 64) * 8 * (4 * 2 * 2
 
 // Row tiles per workgroup and K slices of a linear.  What a form costs is its weight stream, made longer by the x rows that every workgroup reads again (CT / RT of the weights, a
 // quarter of the price of as many weight bytes: they come from L2), by workgroups that do not divide evenly over the 256 CUs (less than in proportion: the CUs that are
-// done leave their bandwidth to the others), and by the hand-over between slices (about 2.5 us for two, 5 for four).  us at 16 / 32 rows, RT x slices, events' 2 us included:
-//   22016 x 4096 gated  2: 32.3 / 36.8   4: 36.8 / 42.8      4096 x 11008  1: 20.0 / 25.3   2 x 2: 20.5 / 23.3   4 x 4: 21.5 / 24.2
-//   27648 x 5120 gated  2: 52.7 / 61.2   4: 49.8 / 58.1      4096 x  4096  1: 11.4 / 13.0   2 x 2: 12.7 / 13.8
-//   12288 x 4096  1: 23.6 / 29.9   2: 25.0 / 28.3   4: 22.8 / 26.1       6208 x 4096  1: 16.9 / 19.3   2: 15.1 / 18.8   4 x 2: 16.4 / 18.1
+// done leave their bandwidth to the others), and by the hand-over between slices (about 2.5 us for two, 5 for four).  us at 16 / 32 rows, RT x slices, launches back to back:
+//   22016 x 4096 gated  2: 29.5 / 34.5   4: 34.2 / 40.0      12288 x 4096  1: 19.0 / 24.3   2: 20.2 / 23.9   4: 18.9 / 21.9
+//   27648 x 5120 gated  2: 47.3 / 55.6   4: 44.7 / 51.2       6208 x 4096  1: 13.2 / 16.7   2: 11.7 / 14.3   4: 16.1 / 19.5   2 x 2: 14.4 / 16.2   4 x 2: 13.4 / 15.7
+//   15360 x 5120        1: 30.0 / 39.1   2: 26.2 / 31.2   4: 26.1 / 28.7
+// (4096 x 11008, with the events' 2 us: 1: 20.0 / 25.3   2 x 2: 20.5 / 23.3   4 x 4: 21.5 / 24.2.)
+// Up to 8 rows x is next to nothing, and a wide linear is faster the smaller its workgroups (us at 2 / 8 rows, RT 1 : 4): 15360 x 5120 24.9 / 25.7 : 26.0 / 25.9, 12288 x 4096 17.0 / 17.1 :
+// 18.3 / 18.4, 32000 x 4096 38.8 / 39.2 : 41.3 / 41.6, 11008 x 4096 16.1 / 16.5 : 17.0 / 17.3, 9216 x 3072 12.0 / 12.5 : 12.8 / 13.1.
 SkinnyForm skinny_form(const GemmArgs& a) {
     const bool gated = act_gated(a.act), slices = !gated && a.skw && a.sk_cnt && a.N % 64 == 0 && a.N < SKINNY_SLICED_N;
     const int ct = a.M > 16 ? 2 : 1, nsuper = cdiv(a.K, SK_SUPER);
     const double weights = (double)a.N * a.K / (4096.0 * 11008.0);
     SkinnyForm best{gated ? 2 : 1, 1};
     double least = 1e30;
+    if (!gated && a.M <= 8 && a.N >= SKINNY_SLICED_N) return best;
     for (int rt = 4; rt >= (gated ? 2 : 1); rt /= 2) {
         if (a.N % (16 * rt) != 0 && rt > 1) continue;                   // the fragment-order copy ends with the last 16 rows
         const int tiles = cdiv(a.N, 16 * rt);

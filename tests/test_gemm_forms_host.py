@@ -34,6 +34,14 @@ def test_slices_of_a_decode_batch_fit_the_scratch(M, N, K):
     assert ops.gemm_form(torch.bfloat16, M, N, K, batch=True, scratch_bytes=0)[3] == 1
 
 
+@pytest.mark.parametrize("M,N,K,act,rt", [(2, 15360, 5120, 0, 1), (8, 12288, 4096, 0, 1), (8, 32000, 4096, 0, 1), (9, 12288, 4096, 0, 4), (32, 15360, 5120, 0, 4), (8, 22016, 4096, 3, 2),
+                                          (8, 27648, 5120, 3, 4), (16, 6208, 4096, 0, 2), (32, 6208, 4096, 0, 2)])
+def test_tiles_of_a_decode_batch(M, N, K, act, rt):
+    """The measured best at widths where the forms are a twentieth and more apart."""
+    from llava_mi355x import ops
+    assert ops.gemm_form(torch.bfloat16, M, N, K, act=act, batch=True)[1] == rt
+
+
 @pytest.mark.parametrize("dt,N,K,ldx,ldw,words", [(torch.bfloat16, 256, 128, 132, 128, "16-byte row alignment"), (torch.float16, 256, 128, 128, 129, "16-byte row alignment"),
                                                   (torch.bfloat16, 250, 128, 128, 128, "multiple of 8"), (torch.bfloat16, 256, 96, 96, 96, "multiple of 64"), (torch.float32, 256, 128, 128, 128, "16-bit dtypes")])
 @pytest.mark.parametrize("variant", [1101, 2201])

@@ -339,7 +339,7 @@ size_t gemm_rows_slab_bytes(int M, int N, int S) { return S > 1 ? (size_t)S * M 
 //    139   58.0 -> 33.7  17.4 (19.3)   70.8 -> 50.4  41.7 -> 34.9      128 weight rows, up to 6 slices; o stays where it was
 //    250   58.7 -> 43.1  20.8 (25.6)   78.5 -> 62.6  53.3 -> 50.9
 //    290   61.9 -> 45.4  31.7 -> 26.0  80.5 (90.4)   85.5 -> 46.5      two row tiles; gate|up (344 workgroups) stays
-//    512   74.1 -> 64.3  34.0 (36.1)   94.3 (128.7)  91.3 -> 69.7
+//    512   74.1 -> 64.3  33.6 -> 31.1  94.3 (128.7)  90.0 -> 76.0
 // so: 64 weight rows up to 128 rows, where the weights are the time; 128 above, where the rows' re-reads are; no more than one workgroup per CU; slices of at least 10 slabs,
 // and above 128 rows no slicing of a short K (the slabs of o cost what its weights cost).  Short products (K < 1024, under 4 M weights) are launch time on any form.
 //
@@ -349,10 +349,22 @@ size_t gemm_rows_slab_bytes(int M, int N, int S) { return S > 1 ? (size_t)S * M 
 //   2048 x 2048 x 5632  58.8 -> 56.6   2308 x 1024 x 4096  61.2 -> 37.0   4616 x 1024 x 4096  59.1 -> 56.9   577 x 4096 x 1024   17.3 -> 13.8   2308 x 1024 x 1024   17.9 -> 14.9
 // Not: long K under tiles of 160 rows and more (1087 x 4096 x 11008: 100.7 (116.4): three slices of 256 x 256 tiles read less), 160 and more tiles of 256 x 256, and the few small
 // tiles of 577 x 1024 and its like (7.4, 16.9 us on 64 x 64), whose time is their chain of K steps.
+//
+// Where the others are the faster ones (30 weights x 24 row counts, launches back to back, weights cold; other (here)):
+//   a short K in slices: the second launch costs what is saved.  257 x 3072 x 2048 10.7 (19.9), 128 x 4096 x 2048 11.9 (15.9), 256 x 8192 x 1536 16.5 (25.1); rows at 33 .. 64
+//     over up to 64 tiles of 64 x 64 stay here, and up to 256 rows over more than 640: 64 x 3072 x 2048 12.2 -> 10.9, 251 x 11456 x 2304 37.3 -> 31.9;
+//   one round of 64 x 64 tiles: 96 x 6656 x 4096 19.2 (21.3), 257 x 3072 x 3072 14.2 (19.7), 257 x 2560 x 5120 21.4 (24.6); two rounds: 257 x 4096 x 4096 30.4 -> 24.4;
+//   256 x 256 tiles in slices where one slice leaves CUs idle: 258 x 9792 x 7296 59.4 (75.8), 183 x 18176 x 7744 84.5 (96.4).  (Where it does not they win back to back, 512 x 12288 x
+//     4096 60.6 (63.5), 256 x 15360 x 5120 61.6 (65.3), 256 x 27648 x 5120 87.8 (96.7), and lose inside a prompt: 500 rows 12 us a layer of 4096, 250 rows 4 us a layer of 5120);
+//   tall tiles over a short K: 2048 x 4096 x 2048 42.6 (47.8), 2308 x 3072 x 1024 21.3 (26.1); 2048 x 3072 x 2048 39.9 -> 36.0.
+// Over all 720 products 1.135 times as fast as the others alone (1.115 without these lines).
 RowsForm gemm_rows_form(int dtype, const GemmArgs& a) {
     const RowsForm none{0, 0, 1};
     if (a.K < 1024 || (size_t)a.N * a.K < ((size_t)1 << 20) || !gemm_rows_applies(dtype, a)) return none;
     const int nk = a.K / GEMM_BK;
+    const int64_t t64 = (int64_t)cdiv(a.M, 64) * cdiv(a.N, 64);
+    const int t256 = cdiv(a.M, 256) * cdiv(a.N, 256), big = t256 * gemm_slices(a);       // workgroups of the ping-pong kernel
+    const bool plain = !act_gated(a.act) && !a.c_f32;                                   // (the others have one tile form for fp32 output and no small ones for gated)
     if (a.M <= 512 && (size_t)a.N * a.K >= ((size_t)4 << 20)) {
         const int mt = cdiv(a.M, 256);
         const bool few = a.M <= 128 && cdiv(a.N, 64) <= 256;
@@ -360,15 +372,22 @@ RowsForm gemm_rows_form(int dtype, const GemmArgs& a) {
         if (tiles <= 256) {
             int s = std::min(256 / tiles, few ? 4 : mt == 2 ? 4 : 6);
             while (s > 1 && (nk / s < 10 || !a.skw || a.pk_kc || gemm_rows_slab_bytes(a.M, a.N, s) > a.skw_bytes())) --s;
-            if (tiles * s >= 128 && (few || s <= 2 || nk >= 128 || (mt == 2 && a.M <= 384))) return RowsForm{mt, bn, s};
+            bool take = tiles * s >= 128 && (few || s <= 2 || nk >= 128 || (mt == 2 && a.M <= 384));
+            if (take && plain) {
+                if (a.K < 2560 && (s == 1 ? few && a.M <= 64 : (a.M <= 32 || a.M > 64 || t64 > 64) && (mt == 2 || t64 <= 640))) take = false;
+                else if (few && a.M > 64 && s == 2 && t64 <= 256 && a.K < 8192) take = false;
+                else if (mt == 2 && s > 1 && t64 <= (a.K <= 3072 ? 320 : 256)) take = false;
+            }
+            if (take && !a.c_f32 && s == 1 && a.M > 96 && tiles < (mt == 2 ? 176 : 160) && big >= 192) return none;
+            if (take) return RowsForm{mt, bn, s};
         }
     }
-    const int64_t t64 = (int64_t)cdiv(a.M, 64) * cdiv(a.N, 64);
-    if (a.M <= 384 || cdiv(a.M, 256) * cdiv(a.N, 256) >= 160 || t64 <= (a.K >= 2048 ? 320 : 512)) return none;
+    if (a.M <= (a.K < 2560 ? 256 : 384) || t256 >= 160 || t64 <= (a.K >= 2048 ? 320 : 512)) return none;
     const int nt = cdiv(a.N, 128), fit = 256 / nt;
     if (fit < 1 || cdiv(a.M, fit) > 256) return none;
     const int mt = cdiv(a.M, cdiv(cdiv(a.M, fit), 32) * 32), rows32 = cdiv(cdiv(a.M, mt), 32);
-    if (mt * nt < 144 || (rows32 > 4 && nk > 64)) return none;
+    if (mt * nt < 144 || (rows32 > 4 && nk > 64) || (rows32 > 3 && nk > 128)) return none;
+    if (rows32 >= 7 && (a.K <= 1024 || (a.K <= 2048 && (int64_t)cdiv(a.M, 128) * cdiv(a.N, 128) > 400))) return none;
     return RowsForm{mt, 128, 1};
 }
 

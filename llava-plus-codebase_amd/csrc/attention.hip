@@ -155,23 +155,6 @@ __global__ __launch_bounds__(512, D == 64 && !WIN ? 4 : 2) void flash_prefill2_k
     for (int r = 0; r < nrounds; ++r) {
         const int t = 2 * r + grp;
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // everything this wave staged for round r has landed
-        if (const int live = a.kv_len - (tile0 + t) * FA_KT; t < ntiles && live < FA_KT) {
-            // the tile with the last key: what the cache holds behind it (an earlier request's values, Inf and NaN among them) has probability 0, and 0 x NaN is NaN, so
-            // every wave clears it in the pieces of V^T that it staged itself
-            int ln = lane;
-            asm volatile("" : "+v"(ln));                       // no address of this branch is worth a register outside of it
-#pragma unroll
-            for (int i = 0; i < VPPW; ++i) {
-                const int p = wave + 4 * i, row = p * 8 + (ln >> 3), key = (((ln & 7) ^ (row >> 1)) & 7) * 8;
-                uint4* v = reinterpret_cast<uint4*>(smem + ((r % NRND) * 2 + grp) * BUF_BYTES + K_BYTES + p * 1024 + ln * 16);
-                if (key + 8 <= live) continue;
-                uint4 w = *v;
-                auto keep = [&](int k) { return (key + k < live ? 0x0000ffffu : 0u) | (key + k + 1 < live ? 0xffff0000u : 0u); };
-                w.x &= keep(0); w.y &= keep(2); w.z &= keep(4); w.w &= keep(6);
-                *v = w;
-            }
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        }
         __builtin_amdgcn_s_barrier();          // round r visible to every wave; everyone is done with round r - 1 (its slots are free)
         if (r + NRND - 1 < nrounds) stage_round(r + NRND - 1);
         if (t >= ntiles) continue;             // odd tile count: group 1 sits out the last round (it still takes the barriers)

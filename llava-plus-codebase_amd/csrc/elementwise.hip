@@ -192,7 +192,8 @@ void launch_layernorm(int dtype, const void* x, const void* w, const void* b, vo
 // RoPE + KV-cache write. grid = (ceil(T/64), n_heads + 2*n_kv_heads); 256 threads.
 //   head slot < n_heads                : q, rotated in place
 //   n_heads <= slot < n_heads + n_kv   : k, rotated, written to K cache [kvh][pos][D]
-//   otherwise                          : v, transposed through LDS into Vᵀ cache [kvh][d][pos] (128-byte key runs)
+//   otherwise                          : v, transposed through LDS into Vᵀ cache [kvh][d][pos] (128-byte key runs); Vᵀ behind the last row is cleared to the end of its 64 keys
+//                                        (the prompt attention reads whole tiles; an earlier sequence's Inf or NaN there would meet probability 0)
 // HF rounding chain (model dtype T): cos,sin -> T ; out = T( T(x*cos) + T(rot(x)*sin) ).
 // ---------------------------------------------------------------------------------------------------------------
 template <typename T, int D>
@@ -260,6 +261,11 @@ __global__ __launch_bounds__(256) void rope_kv_kernel(RopeKvArgs a) {
     if (t < ntok) {
         const int pos = pos0 + tok0 + t;
         for (int d = tid >> 6; d < D; d += 4) vt[(size_t)d * a.s_max + pos] = tile[t * PITCH + d];
+    }
+    if (tok0 + 64 >= a.T) {
+        const int end = pos0 + a.T, whole = (end + 63) & ~63, pos = end + t;
+        if (pos < (whole < a.s_max ? whole : a.s_max))
+            for (int d = tid >> 6; d < D; d += 4) vt[(size_t)d * a.s_max + pos] = from_f32<T>(0.f);
     }
 }
 

@@ -172,6 +172,12 @@ __device__ __forceinline__ void qkv_rope_epilogue(const GemmArgs& a, f32x16 (&ac
                 }
             }
         }
+        if (m0 + 256 >= a.M) {                                  // V^T behind the last row: cleared to the end of its 64 keys, as rope_kv_kernel does
+            const int end = a.qf_pos0 + a.M, whole = (end + 63) & ~63, pos = end + (tid & 63);
+            if (pos < (whole < a.qf_smax ? whole : a.qf_smax))
+                for (int c = tid >> 6; c < 256; c += 8)
+                    reinterpret_cast<uint16_t*>(vt)[((size_t)(kvh0 + c / D) * D + (c % D)) * a.qf_smax + pos] = 0;
+        }
     }
 }
 

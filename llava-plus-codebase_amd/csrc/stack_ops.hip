@@ -172,6 +172,7 @@ void launch_residual_norm(int dtype, const ResidualNormArgs& a, int rows, hipStr
 //   PAIRED (rot_dims % 16 == 0): D / 16 lanes own one head vector, two 8-element chunks each — a chunk of the rotated part with its partner half a rotation away, or two
 //   neighbouring chunks of the rest — so a lane rotates what it loaded: no LDS, no barrier.
 //   otherwise: D / 8 lanes, 8 consecutive elements each, the partner i +- rot_dims / 2 through LDS (any even number of rotated dimensions).
+// V^T behind the last row is cleared to the end of its 64 keys (or to zero_to).
 // ---------------------------------------------------------------------------------------------------------------
 template <typename T, int D, bool PAIRED>
 __global__ __launch_bounds__(256) void qkv_norm_rope_kv_kernel(QkvNormRopeArgs a) {
@@ -294,6 +295,11 @@ __global__ __launch_bounds__(256) void qkv_norm_rope_kv_kernel(QkvNormRopeArgs a
     if (t < ntok || t < nzero) {
         const int pos = a.pos0 + tok0 + t;
         for (int d = tid >> 6; d < D; d += 4) vt[(size_t)d * a.s_max + pos] = t < ntok ? tile[t * PITCH + d] : from_f32<T>(0.f);
+    }
+    if (ntok > 0 && tok0 + 64 >= a.T && a.zero_to == 0) {     // as in rope_kv_kernel: to the end of the last row's 64 keys
+        const int end = a.pos0 + a.T, whole = (end + 63) & ~63, pos = end + t;
+        if (pos < (whole < a.s_max ? whole : a.s_max))
+            for (int d = tid >> 6; d < D; d += 4) vt[(size_t)d * a.s_max + pos] = from_f32<T>(0.f);
     }
 }
 

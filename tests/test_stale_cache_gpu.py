@@ -1,5 +1,6 @@
-"""What a cache holds behind the last key (an earlier request's values, with Inf and NaN among them) never reaches a later request: every attention kernel that reads whole tiles of
-V^T clears it, because probability 0 times NaN is NaN.  The same launches on clean caches give the same bits."""
+"""What a cache holds behind the last key (an earlier request's values, with Inf and NaN among them) never reaches a later request, although probability 0 times NaN is NaN: the launches
+that append a portion's rows clear V^T to the end of the last row's 64 keys, and the kernels of a step clear what they loaded.  The same launches on clean caches give the same
+bits."""
 import pytest
 import torch
 
@@ -36,26 +37,64 @@ def test_a_sequence_after_one_of_nan(cuda, name, dt, context, rows):
     assert bool(outs[0].isfinite().all()) and torch.equal(outs[0], outs[2]) and torch.equal(outs[1], outs[3])
 
 
-@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+def test_a_layer_stack_sequence_after_one_of_nan(cuda, dt):
+    """The same for windowed layers: widths with and without whole rotation groups, windows that end inside a tile."""
+    from llava_mi355x import _C
+    from llava_mi355x.engine_lm import LmxKVCache
+    from siterax_util import build, tokens
+    for name in ("mixed", "odd"):
+        m = build(name, dt)
+        for n, more in ((2, 0), (70, 9), (129, 60)):
+            ids = torch.tensor([tokens(name, n + more + 1, n)], device=cuda)
+            outs = []
+            for stale in (False, True):
+                first = LmxKVCache(m, 1)
+                if stale:
+                    nan = torch.full((400, m.row_pitch), float("nan"), dtype=dt, device=cuda)
+                    _C.check(_C.lib.lmx_prefill(m._h, first.seqs[0], _C.ptr(nan), 400, 0, None, 0, 1, _C.stream_handle()))
+                _C.check(_C.lib.lmx_seq_truncate(first.seqs[0], 0, _C.stream_handle()))
+                o = m.forward(ids[:, :n], past_key_values=first)
+                got = [o.logits]
+                if more:
+                    got.append(m.forward(ids[:, n:n + more], past_key_values=first).logits)
+                got.append(m.forward(ids[:, n + more:], past_key_values=first).logits)
+                outs.append(got)
+            for a, b in zip(*outs):
+                assert bool(a.isfinite().all()) and torch.equal(a, b), (name, n, more)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("D", [64, 128])
-@pytest.mark.parametrize("form", ["causal", "whole", "window"])
-@pytest.mark.parametrize("kv_len", [1, 7, 8, 63, 64, 65, 120, 129, 577])
-def test_prompt_attention(cuda, dt, D, form, kv_len):
+@pytest.mark.parametrize("T,pos0", [(1, 0), (63, 0), (64, 0), (65, 8), (70, 56), (130, 120), (1, 255), (100, 156)])
+def test_appended_rows_clear_the_rest_of_their_tile(cuda, dt, D, T, pos0):
+    """rope_kv: V^T from the last row to the end of its 64 keys is 0, what lies before the portion and behind that tile stays."""
     from llava_mi355x import ops
-    H, G, s_max = 4, 2, 640
-    g = torch.Generator().manual_seed(kv_len)
-    q_len = min(kv_len, 33)
-    q = torch.randn(q_len, (H + 2 * G) * D, generator=g).to(dt).to(cuda)
-    k, v = torch.randn(G, s_max, D, generator=g).to(dt), torch.randn(G, D, s_max, generator=g).to(dt)
-    outs = []
-    for stale in (False, True):
-        k[:, kv_len:], v[:, :, kv_len:] = (float("nan"), float("inf")) if stale else (0, 0)
-        kc, vt = k.to(cuda), v.to(cuda)
-        if form == "window":
-            outs.append(ops.window_attn(q, kc, vt, kv_len - q_len, H, G, D ** -0.5, window=50))
-        else:
-            outs.append(ops.flash_attn(q, kc, vt, q_len, kv_len, kv_len - q_len, H, G, D, form == "causal"))
-    assert bool(outs[0].isfinite().all()) and torch.equal(outs[0], outs[1])
+    H, G, s_max = 2, 2, 256
+    g = torch.Generator().manual_seed(T + pos0)
+    qkv = torch.randn(T, (H + 2 * G) * D, generator=g).to(dt).to(cuda)
+    v = qkv[:, (H + G) * D:].reshape(T, G, D).permute(1, 2, 0).clone()
+    kc, vt = torch.zeros(G, s_max, D, dtype=dt, device=cuda), torch.full((G, D, s_max), float("nan"), dtype=dt, device=cuda)
+    ops.rope_kv(qkv, kc, vt, torch.ones(s_max, D, device=cuda), pos0, H, G, D)
+    end = pos0 + T
+    whole = -(-end // 64) * 64
+    assert torch.equal(vt[:, :, pos0:end], v) and not bool(vt[:, :, end:whole].any())
+    assert bool(vt[:, :, :pos0].isnan().all()) and bool(vt[:, :, whole:].isnan().all())
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D,H,G,T,pos0", [(128, 32, 32, 1087, 0), (128, 16, 16, 2000, 40), (64, 64, 16, 2001, 8), (128, 32, 32, 1088, 64)])
+def test_the_fused_projection_clears_it_too(cuda, dt, D, H, G, T, pos0):
+    from llava_mi355x import ops
+    s_max, K = 2176, 128
+    x, w = torch.randn(T, K, device=cuda).to(dt), torch.randn((H + 2 * G) * D, K, device=cuda).to(dt)
+    out = torch.empty(T, (H + 2 * G) * D, dtype=dt, device=cuda)
+    kc, vt = torch.zeros(G, s_max, D, dtype=dt, device=cuda), torch.full((G, D, s_max), float("nan"), dtype=dt, device=cuda)
+    ops.gemm_qkv_rope(x, w, out, kc, vt, torch.ones(s_max, D, device=cuda), pos0, H, G, D)
+    end = pos0 + T
+    whole = -(-end // 64) * 64
+    assert bool(vt[:, :, pos0:end].isfinite().all()) and not bool(vt[:, :, end:whole].any())
+    assert bool(vt[:, :, :pos0].isnan().all()) and bool(vt[:, :, whole:].isnan().all())
 
 
 @pytest.mark.parametrize("dt,D", [(torch.float32, 64), (torch.float32, 128), (torch.bfloat16, 64), (torch.float16, 64), (torch.bfloat16, 128)])

@@ -92,15 +92,15 @@ __global__ __launch_bounds__(BA_NW * 64) void decode_attn_wave_kernel(DecodeFuse
     rope8<T, D>(qkv + head * D, cs, sub * 8, qv);
     const uint32_t qp[4] = {pack2<T>(qv[0], qv[1]), pack2<T>(qv[2], qv[3]), pack2<T>(qv[4], qv[5]), pack2<T>(qv[6], qv[7])};      // exact: rotated q is rounded to T
 
-    load_k(wave * BA_PIECE, wave < n_piece);
-    asm volatile("" ::: "memory");                                          // keys before values: the order the loop's wait counts rely on
-    load_v(wave * BA_PIECE, wave < n_piece);
-    asm volatile("" ::: "memory");
-
     float m_run = -INFINITY, l_run = 0.f;                                   // m: of the wave; l: of this lane's keys
     float acc[16];
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+    if (wave < n_piece) {                                                   // (a wave without a piece asks for nothing: 32 loads of an empty view are 32 trips through the address unit)
+    load_k(wave * BA_PIECE, true);
+    asm volatile("" ::: "memory");                                          // keys before values: the order the loop's wait counts rely on
+    load_v(wave * BA_PIECE, true);
+    asm volatile("" ::: "memory");
     for (int pc = wave; pc < n_piece; pc += NW) {
         const int nk = pos - pc * BA_PIECE;                                            // >= 1 live keys
         // ---- scores: 16 partial sums per lane, reduced over the key's 16 lanes and dealt out: lane (kslot, sub) ends with key 4 sub + kslot ------------------------
@@ -164,6 +164,7 @@ __global__ __launch_bounds__(BA_NW * 64) void decode_attn_wave_kernel(DecodeFuse
 #pragma unroll
         for (int i = 0; i < 16; ++i) asm volatile("" : "+v"(acc[i]) :: "memory");
         load_v((pc + NW) * BA_PIECE, pc + NW < n_piece);
+    }
     }
     // ---- the wave's state: o[d] = sum over the 8 lanes of a d-row, then (o, m, l) into LDS ------------------------------------------------------------------
 #pragma unroll

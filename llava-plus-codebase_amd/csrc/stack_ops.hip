@@ -911,21 +911,20 @@ __global__ __launch_bounds__(256) void decode_win_group_kernel(WinDecodeArgs a) 
 bool decode_win_groups(int dtype, int D, int n_heads, int n_kv_heads, int n_seq) {
     return dtype != kF32 && D <= 128 && n_heads / n_kv_heads <= WIN_GROUP_MAX && n_seq > 1;
 }
-// Which kernel and how many splits.  The grouped one reads a cached key once instead of once per query head, but has a group-th of the workgroups, a longer start and, over splits,
-// one workgroup that merges all heads of the group.  us, one head a workgroup -> grouped, 16-bit:
-//   32 heads on  8 of 128   32 sequences of 1024 keys 97 -> 31   8 of 130  13.4 -> 11.2    2 of 600  13.3 -> 11.4    4 of 20  8.1 -> 8.7    16 of 20  11.1 -> 9.4
-//   24 heads on 12          32 of 1200  84 -> 52                 2 of 130  10.4 -> 9.8     32 of 60  14 -> 17
-//    8 heads on  1          32 of 600   32 -> 14                 8 of 600  13 -> 13        2 of 600  10 -> 13        8 of 60  8 -> 10        (16 on 1: 16 of 600  23 -> 19, 4 of 600  12 -> 17)
-//   32 heads on 32           8 of 1200  45 -> 31                 16 of 600 46 -> 40        3 of 600  14 -> 15        16 of 60  11 -> 19      (16 of 64: 16 of 600  16 -> 13, 6 of 600  10 -> 11)
-// so: by the bytes that one head a workgroup asks for, more of them where the group is larger (the merge), and for groups of 2 - 4 from one chunk of keys on.  One sequence of 601
-// keys, 16 heads on 4: 11.1 us either way, all of it latency, so the form with more workgroups stays.
+// Which kernel and how many splits.  The grouped one reads a cached key once instead of once per query head, in whole lines, but has a group-th of the workgroups, a longer start
+// and, over splits, one workgroup that merges all heads of the group.  us, one head a workgroup -> grouped, 16-bit, caches cold (in a step the weights pass between two layers):
+//   32 heads on  8 of 128   32 sequences of 1200 keys 116 -> 33   8 of 130  15 -> 12     2 of 600  14 -> 13     4 of 20  9 -> 11      16 of 60  13 -> 11
+//   24 heads on 12          32 of 1200 108 -> 53                  2 of 130  12 -> 11     32 of 60  17 -> 19
+//   32 heads on 32           8 of 1200  74 -> 32                  2 of 300  14 -> 12     16 of 130 33 -> 23     16 of 60  18 -> 20
+//    8 heads on  1          32 of 600   34 -> 15                  8 of 600  14 -> 15     2 of 600  12 -> 15      8 of 60  9 -> 12     (16 on 1: 16 of 600 25 -> 20, 4 of 600 13 -> 20)
+// so: up to groups of four from one chunk of keys on, larger groups by the bytes that one head a workgroup asks for (the merge grows with the group); shorter contexts only where
+// a group is three or four.  One sequence of 601 keys, 16 heads on 4: 11.1 us either way, all of it latency, so the form with more workgroups stays.
 // Splits: as many as make ONE round of workgroups of the grouped kernel (its waves fill a CU: 96 x 3 and 160 x 2 workgroups took a second round, 15 -> 19 and 21 -> 25 us).
 WinForm decode_win_form(int dtype, int D, int n_heads, int n_kv_heads, int n_seq, int span) {
     const int group = n_heads / n_kv_heads, chunks = std::max(1, std::min((span + 127) / 128, DF_MAX_SPLIT));
     const double mb = (double)n_heads * n_seq * span * D * 4e-6;
     bool grouped = decode_win_groups(dtype, D, n_heads, n_kv_heads, n_seq);
-    if (group == 1) grouped = grouped && span >= 512 && mb >= 48;
-    else if (group <= 4) grouped = grouped && (span >= 128 || (group >= 3 && mb >= 8));
+    if (group <= 4) grouped = grouped && (span >= 128 || (group >= 3 && mb >= 10));
     else grouped = grouped && mb >= 0.6 * group * group;
     const int wgs = (grouped ? n_kv_heads : n_heads) * n_seq;
     return WinForm{grouped, std::max(1, std::min(chunks, grouped ? 256 / wgs : (1024 + wgs - 1) / wgs))};

@@ -68,11 +68,12 @@ def test_skinny_gemm_bias_act_residual(cuda, M, act):
     assert _rel_err(r2, ref) < 1e-2
 
 
-@pytest.mark.parametrize("M,I", [(1, 352), (7, 352), (16, 352), (32, 352), (20, 8192), (32, 11008)])
-def test_skinny_gemm_silu_mul(cuda, M, I):
+@pytest.mark.parametrize("M,I,rt", [(1, 352, 2), (7, 352, 2), (16, 352, 2), (32, 352, 2), (20, 8192, 4), (32, 11008, 2), (16, 13824, 4), (3, 5632, 4)])
+def test_skinny_gemm_silu_mul(cuda, M, I, rt):
     from llava_mi355x import _C, ops
     torch.manual_seed(5 + M)
     K = 256
+    assert ops.gemm_form(torch.bfloat16, M, 2 * I, K, act=_C.ACT_SILU_MUL, batch=True) == (0, rt, 1 + (M > 16), 1)
     x = torch.randn(M, K, device=cuda).bfloat16()
     g = (torch.randn(I, K, device=cuda) / math.sqrt(K)).bfloat16(); u = (torch.randn(I, K, device=cuda) / math.sqrt(K)).bfloat16()
     fused = ops.interleave_gate_up(g, u)
@@ -83,16 +84,16 @@ def test_skinny_gemm_silu_mul(cuda, M, I):
 
 
 @pytest.mark.parametrize("dt", ["bf16", "f16"])
-@pytest.mark.parametrize("M,N,K", [(9, 4096, 4096), (16, 4096, 4096), (17, 4096, 11008), (32, 4096, 4096), (32, 4096, 11008), (32, 5120, 13824), (24, 4096, 1408),
-                                   (32, 4096, 512), (12, 1024, 4096), (32, 4160, 4096),
-                                   (32, 12288, 4096), (17, 12288, 4096), (24, 15360, 5120), (16, 12288, 4096)])     # q|k|v of 7B / 13B: two slices above 16 rows
+@pytest.mark.parametrize("M,N,K", [(2, 640, 13824), (8, 1024, 11008), (16, 640, 13824), (9, 1088, 11008), (16, 1664, 11008), (17, 640, 13824), (32, 1088, 11008), (17, 4096, 11008),
+                                   (32, 4096, 11008), (24, 3072, 11008), (32, 2048, 13824), (32, 5120, 13824), (20, 4416, 13824), (32, 4032, 13824)])
 def test_skinny_gemm_k_slices_across_workgroups(cuda, dt, M, N, K):
-    """Round 6: narrow layers (N = hidden) of a decode batch with more than 8 rows take 64 weight rows per workgroup and K SLICES ACROSS WORKGROUPS (variant 24: the
-    engine's form, with its scratch): every slice's fp32 partial tile leaves write-through, the last workgroup to arrive for a tile adds the slices in slice order and
-    runs the epilogue.  Checked against the float64 product rounded once (one ulp + fp32 accumulation noise), against the 16-rows-per-workgroup form (same tolerance:
+    """Linears of a decode batch below 8192 columns take K SLICES ACROSS WORKGROUPS where the cost rule says so (variant 24: the engine's form, with its scratch): every
+    slice's fp32 partial tile leaves write-through, the last workgroup to arrive for a tile adds the slices in slice order and runs the epilogue.  Two and four slices of
+    16, 32 and 64 weight rows.  Checked against the float64 product rounded once (one ulp + fp32 accumulation noise), against the form without scratch (same tolerance:
     the summation order differs), bit for bit from launch to launch on the SAME scratch and tickets (30 launches, alternating inputs: a stale partial tile or a ticket
     left armed would show), with bias / activation / residual aliasing the output."""
     from llava_mi355x import ops
+    assert ops.gemm_form(DT[dt], M, N, K, batch=True)[3] > 1 and ops.gemm_form(DT[dt], M, N, K, scratch_bytes=0, batch=True)[3] == 1
     from test_gemm8p_gpu import assert_one_ulp
     g = torch.Generator(device=cuda).manual_seed(M * 131 + N + K)
     T = DT[dt]
@@ -106,7 +107,7 @@ def test_skinny_gemm_k_slices_across_workgroups(cuda, dt, M, N, K):
         if first[i] is None:
             first[i] = got.clone()
             assert_one_ulp(got, refs[i], dt, 3e-5 * float(refs[i].abs().max()), f"K-slice form, input {i}")
-            assert_one_ulp(ops.gemm(xs[i], w, variant=21), refs[i], dt, 3e-5 * float(refs[i].abs().max()), "16-rows-per-workgroup form")
+            assert_one_ulp(ops.gemm(xs[i], w, variant=21), refs[i], dt, 3e-5 * float(refs[i].abs().max()), "one slice")
         else:
             assert torch.equal(got, first[i]), f"launch {it}: not the bits of the first launch on this input"
     b = torch.randn(N, device=cuda, generator=g).to(T); r = torch.randn(M, N, device=cuda, generator=g).to(T)

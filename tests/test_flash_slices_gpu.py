@@ -1,6 +1,6 @@
 """A short prompt portion on a long context: its attention's keys are cut into slices over the workgroups and merged by a second launch (csrc/attention.hip: flash_slices,
 flash_merge_kernel).  Every row against the one-token step of the same position (another kernel, its own merge), for contexts at the borders of the slices' tiles, one row
-and more than one query block; the tolerance is that of the other comparisons of two 16-bit forms of one step."""
+and more than one query block, heads of 128 and, two to a kv head, of 64; the tolerance is that of the other comparisons of two 16-bit forms of one step."""
 import pytest
 import torch
 
@@ -9,11 +9,12 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("context,rows", [(511, 1), (448, 64), (640, 33), (1343, 129), (1919, 5)])
-def test_rows_of_a_portion_as_single_steps(cuda, dt, context, rows):
+@pytest.mark.parametrize("name", ["tiny", "tiny_gqa"])
+def test_rows_of_a_portion_as_single_steps(cuda, name, dt, context, rows):
     from llava_mi355x import _C
     from llava_mi355x.model import LmxKVCache
     from synthetic import build as harness, recipes as synth
-    cfg = synth.CONFIGS["tiny"]
+    cfg = synth.CONFIGS[name]
     model = harness.build_model(cfg, dtype=dt, seed=0, max_position=2048)
     torch.manual_seed(context)
     V = cfg.vocab_size

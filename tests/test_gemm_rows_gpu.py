@@ -83,3 +83,19 @@ def test_slices_of_the_rule(cuda, dt, form, M, N, K):
     assert_one_ulp(got, ref, dt, 2e-5 * float(ref.abs().max()), f"{M}x{N}x{K}")
     ops.gemm(-x, w, residual=r, variant=_C.GEMM_SCRATCH)
     assert torch.equal(got, ops.gemm(x, w, residual=r, variant=_C.GEMM_SCRATCH))
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("M,N,K", [(5, 10248, 1024), (139, 32000, 1024), (300, 8200, 2048)])
+@pytest.mark.parametrize("cap", [0.0, 7.5])
+def test_fp32_output_with_a_soft_cap(cuda, dt, M, N, K, cap):
+    """An output head's logits.  Bound: an fp32 sum of K products (the cap's slope is at most 1), tanh and its division to 8 units in the last place."""
+    from llava_mi355x import ops
+    x, w = _mk(M, N, K, dt, cuda, M + N)
+    w = w * 4
+    want = x.double() @ w.double().t()
+    bound = K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
+    if cap:
+        want = cap * torch.tanh(want / cap)
+    got = ops.linear_f32(x, w, cap, 0)
+    assert got.dtype == torch.float32 and bool(((got.double() - want).abs() <= bound + want.abs() * 2.0 ** -20).all())

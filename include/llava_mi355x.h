@@ -207,7 +207,7 @@ int lmx_gather_embeds(lmx_model* m, const int32_t* src_dev, int32_t rows, const 
  * decode state; replaces the past_key_values tuple of the reference (llava_arch.py:105; a14 in SURVEY §8). */
 int lmx_seq_create(lmx_model* m, lmx_seq** out);
 int lmx_seq_destroy(lmx_seq* s);                     /* before or after lmx_destroy of its model; nothing else works on a sequence whose model is gone */
-int lmx_seq_reset(lmx_seq* s);                       /* length := 0 (cache contents stay finite) */
+int lmx_seq_reset(lmx_seq* s);                       /* length := 0 (cache contents stay; nothing reads behind the length) */
 int lmx_seq_length(const lmx_seq* s);                /* tokens currently in the cache (host mirror) */
 
 /* replaces: LlamaForCausalLM.forward with inputs_embeds (llava_llama.py:88-99 -> HF5:models/llama/modeling_llama.py:

@@ -747,7 +747,7 @@ void launch_cast_f32(int dtype, const float* src, void* dst, size_t n, hipStream
 
 // column sums of dy [rows][cols] -> fp32 [cols] (bias gradient).  A workgroup owns 64 columns (one 128-byte line of a 16-bit row): lanes of VEC columns side by side, the other
 // lanes take rows in turn, four of them on the wire; the row lanes' sums are added in lane order: deterministic.  Bound: the read of dy where cols / 64 workgroups can draw it.
-// (One thread per column and row after row: 2308 x 4096 530 us, 16 workgroups waiting for one 2-byte load each.)
+// (bf16, 2308 x 4096 / 5909 x 4096: 6.2 / 15.0 us, 3.0 / 3.2 TB/s; one thread per column and row after row, 16 workgroups waiting for one 2-byte load each: 224 / 1362.)
 template <typename T, int VEC>
 __global__ __launch_bounds__(1024) void col_sum_kernel(const T* __restrict__ dy, int ld, int rows, int cols, float* __restrict__ out) {
     constexpr int CL = 64 / VEC, RL = 1024 / CL;                           // column lanes, row lanes

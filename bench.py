@@ -226,7 +226,7 @@ def cpu_baseline_reference(cfg, ids, pix, new_tokens, decode_steps=0):
 
 def parity_record(model_name):
     """What the parity gate asserts for the kernels this line times, with the figures of the latest committed run of tests/test_full_depth_gpu.py
-    (profiles/r0N_full_depth_*.json; NOT re-measured by the bench: the fp32 oracle pass over 7B takes minutes of host time).  Every report carries the hash of the
+    (profiles/full_depth_*.json; NOT re-measured by the bench: the fp32 oracle pass over 7B takes minutes of host time).  Every report carries the hash of the
     kernel sources it was measured on (synthetic/treehash.py); `stale` says whether that is the tree this bench runs on — after a kernel change the committed
     figures are the previous build's until the suite has been re-run and its reports committed."""
     from synthetic.treehash import csrc_sha16
@@ -239,12 +239,11 @@ def parity_record(model_name):
            "source": "tests/test_full_depth_gpu.py, committed run under profiles/ (not re-measured here)", "csrc_sha16_of_this_run": here}
 
     def latest(stem):
-        for rnd in ("r06", "r05"):
-            p = os.path.join(ROOT, "profiles", f"{rnd}_{stem}.json")
-            if os.path.exists(p):
-                with open(p) as f:
-                    return json.load(f), os.path.basename(p)
-        return None, None
+        p = os.path.join(ROOT, "profiles", f"{stem}.json")
+        if not os.path.exists(p):
+            return None, None
+        with open(p) as f:
+            return json.load(f), os.path.basename(p)
     stamps = []
     try:
         rep, name = latest("full_depth_fp32_llava15_7b")

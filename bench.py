@@ -560,8 +560,7 @@ def pmc_traffic(root):
 def pmc_prefill_traffic(root, T, iters=4):
     """HBM-side bytes per launch of the four prefill GEMM shapes, measured NOW: two rocprofv3 passes (FETCH_SIZE, WRITE_SIZE; --pmc with
     --kernel-trace only) over tools/mb_gemm_prefill.py, which launches q|k|v, gate|up, o_proj, down_proj `iters` times each in that order.  Dispatches are told
-    apart by kernel instantiation and order: the un-split kernel serves q|k|v then gate|up; the K-sliced kernel + its reduction serve o_proj then down_proj
-    (their figure = GEMM + reduction: the fp32 partial tiles are written by one and read by the other).  gfx950 corrections as in pmc_traffic."""
+    apart by order; a K-sliced launch's figure includes the reduction behind it (the fp32 partial tiles are written by one and read by the other).  gfx950 corrections as in pmc_traffic."""
     import csv, glob, shutil, subprocess, tempfile
     exe = shutil.which("rocprofv3")
     if not exe:
@@ -576,15 +575,18 @@ def pmc_prefill_traffic(root, T, iters=4):
             f = glob.glob(os.path.join(d, "**", "*counter_collection.csv"), recursive=True)[0]
             rows = [r for r in csv.DictReader(open(f)) if r["Counter_Name"] == ctr]
             rows.sort(key=lambda r: int(r.get("Dispatch_Id", 0)))
-            # gemm8p_kernel<T, SPLIT>: SPLIT = 1 is the un-split launch (round 5's prune left these two template parameters)
-            unsplit = [float(r["Counter_Value"]) for r in rows if "gemm8p_kernel" in r["Kernel_Name"] and ", 1>" in r["Kernel_Name"]]
-            sliced = [float(r["Counter_Value"]) for r in rows if "gemm8p_kernel" in r["Kernel_Name"] and ", 1>" not in r["Kernel_Name"]]
-            reduce_ = [float(r["Counter_Value"]) for r in rows if "splitk_reduce" in r["Kernel_Name"]]
-            if len(unsplit) != 2 * iters or len(sliced) != 2 * iters or len(reduce_) != 2 * iters:
-                return {"error": f"unexpected dispatch counts {len(unsplit)} / {len(sliced)} / {len(reduce_)} for {ctr}"}
-            mean = lambda xs: sum(xs) / len(xs)
-            per[ctr] = {"qkv": mean(unsplit[:iters]), "gate_up": mean(unsplit[iters:]), "o_proj": mean(sliced[:iters]) + mean(reduce_[:iters]),
-                        "down": mean(sliced[iters:]) + mean(reduce_[iters:])}
+            # the four shapes in mb_gemm_prefill.py's order, `iters` launches each; a K-sliced launch is followed by the one that adds its partial tiles
+            launches = []
+            for r in rows:
+                name, value = r["Kernel_Name"], float(r["Counter_Value"])
+                if any(n in name for n in ("gemm4w_kernel", "gemm8p_kernel", "gemm_rows_kernel", "gemm_pipe_kernel", "gemm_mfma_kernel")):
+                    launches.append(value)
+                elif launches and any(n in name for n in ("gemm4w_reduce", "splitk_reduce", "rows_reduce")):
+                    launches[-1] += value
+            names = ("qkv", "gate_up", "o_proj", "down")
+            if len(launches) != len(names) * iters:
+                return {"error": f"unexpected dispatch count {len(launches)} for {ctr}"}
+            per[ctr] = {n: sum(launches[i * iters:(i + 1) * iters]) / iters for i, n in enumerate(names)}
         except Exception as ex:  # noqa: BLE001
             return {"error": repr(ex)[:200]}
         finally:
@@ -1269,7 +1271,7 @@ def main():
                                    "re-measured in this run); counted at the L2 -> fabric boundary, so Infinity-Cache hits are inside; o_proj / down_proj are K-sliced (3 slices): "
                                    "their figure includes the fp32 partial tiles written by the GEMM and read by the launch-boundary reduction; the rest above 1.0 is operand-tile "
                                    "re-reads (each X tile by every N-tile column, each W tile by the 5 M-tiles) that drift out of an XCD's 4 MB L2"}
-    roof_p = {"bound": "mfma", "kernel": "gemm8p_kernel<bf16,...> (q|k|v, gate|up whole tiles; o_proj, down_proj as 3 K slices + splitk_reduce_kernel, timed together): decoder prefill linears",
+    roof_p = {"bound": "mfma", "kernel": "gemm4w_kernel<bf16,...> (tiles and K slices by gemm4w_form; a sliced product timed with gemm4w_reduce_kernel): decoder prefill linears",
               # frac = the north_star quantity: ALL FLOPs of the prefill (tower + projector + decoder linears + attention) / the measured prefill time;
               # the GEMM family alone (kernel-only durations) is reported beside it
               "achieved": fl["total"] / (prefill_ms * 1e-3) / 1e12 / world, "peak": PEAK_BF16_TFLOPS,

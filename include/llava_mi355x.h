@@ -302,8 +302,10 @@ int lmx_model_set_option(lmx_model* m, const char* key, int32_t value);
 int lmx_op_gemm(int32_t dtype, const void* x, const void* w, void* c, const void* bias, const void* residual,
                 int32_t M, int32_t N, int32_t K, int32_t ldx, int32_t ldw, int32_t ldc, int32_t ldr, int32_t act, int32_t variant, void* stream);
 /* variant LMX_GEMM_SCRATCH: the choice a prefill makes, which brings scratch for K slices (this entry's own 64 MiB: one stream at a time); variant 0 chooses without.
- * lmx_op_gemm_form: that choice for contiguous 16-byte aligned operands and `scratch_bytes` of scratch, on the host alone.  form[4]: batch = 0: {1, row tiles, weight
- * rows of a workgroup, K slices} of the kernel for few row tiles, {0, 0, 0, K slices} of the others; batch = 1 (linears of a decode batch, M <= 32): {0, 16-row weight tiles of
+ * Products of more than 256 rows and more than 640 tiles of 64 x 64 go to the four-wave kernel in either (variant 100 mb + 10 nb + slices: its tiles of 32 mb x 32 nb by number).
+ * lmx_op_gemm_form: for contiguous 16-byte aligned operands and `scratch_bytes` of scratch, on the host alone.  form[4]: batch = 0: {1, row tiles, weight
+ * rows of a workgroup, K slices} where the rule of the kernel for few row tiles has a form (which the products above do not reach), else {0, 0, 0, K slices} of the
+ * four-wave kernel or the others; batch = 1 (linears of a decode batch, M <= 32): {0, 16-row weight tiles of
  * a workgroup, 16-row token tiles, K slices}. */
 #define LMX_GEMM_SCRATCH 40
 int lmx_op_gemm_form(int32_t dtype, int32_t M, int32_t N, int32_t K, int32_t act, int64_t scratch_bytes, int32_t batch, int32_t* form);
@@ -317,7 +319,7 @@ int lmx_op_rope_kv(int32_t dtype, int32_t head_dim, void* qkv, void* kcache, voi
  * per row, which is what the attention backward of the training step reads (lmx_op_attn_bwd with k / v = column windows of qkv: no gathered copies). */
 int lmx_op_rope_kv_rows(int32_t dtype, int32_t head_dim, void* qkv, void* kcache, void* vtcache, const float* cos_sin_dev, int32_t pos0,
                         int32_t T, int32_t n_heads, int32_t n_kv_heads, int32_t s_max, void* stream);
-/* q|k|v projection with RoPE + KV-cache append in the GEMM's epilogue (gemm8p.hip: qkv_rope_epilogue; what Model::prefill launches where
+/* q|k|v projection with RoPE + KV-cache append in the GEMM's epilogue (gemm4w.h: qkv_rope_epilogue4; what Model::prefill launches where
  * the shape allows it): qkv[:, :n_heads*D] <- rotated q, kcache / vtcache rows pos0 .. pos0 + T - 1 <- rotated k / v; the k | v columns of `qkv` are
  * left untouched.  Fails when the shape does not take the fused launch (same rule as the engine: un-split ping-pong GEMM, head-aligned tiles). */
 int lmx_op_gemm_qkv_rope(int32_t dtype, int32_t head_dim, const void* x, const void* w, void* qkv, void* kcache, void* vtcache, const float* cos_sin_dev,

@@ -512,7 +512,7 @@ int lmx_op_gemm_form(int32_t dtype, int32_t M, int32_t N, int32_t K, int32_t act
     }
     const RowsForm f = gemm_rows_form(dtype, g);
     if (f.mtiles) { form[0] = 1; form[1] = f.mtiles; form[2] = f.bn; form[3] = f.slices; }
-    else if (dtype != kF32) form[3] = gemm_slices(g);
+    else if (dtype != kF32) { const TileForm t = gemm4w_form(dtype, g); form[3] = t.mb ? t.slices : gemm_slices(g); }
     LMX_API_END
 }
 int lmx_op_gemv(int32_t dtype, const void* x, const void* w, void* c, const void* bias, const void* residual, const void* norm_w, float eps,

@@ -59,7 +59,7 @@ template <typename T> __device__ __forceinline__ float round_to(float f) { retur
 // One RoPE output with HF's rounding chain, T( T(x c) + T(r s) ) (HF5:models/llama/modeling_llama.py:130-160 on tensors of the model dtype: every
 // elementwise op rounds).  Contraction is switched OFF here: for fp16 hipcc narrows T(x c) with half operands to a half multiply (exact) and would then be
 // free to fuse it with the add into ONE half fma — skipping the rounding of the product — in one kernel and not in another (seen: rope_kv_kernel and the
-// q|k|v epilogue of gemm8p.hip disagreed in 25 % of the fp16 elements by one ulp).  With the pragma every kernel computes the same, HF's, bits.
+// q|k|v epilogue of the prompt GEMM disagreed in 25 % of the fp16 elements by one ulp).  With the pragma every kernel computes the same, HF's, bits.
 template <typename T> __device__ __forceinline__ float rope_term(float x, float c, float r, float s) {
 #pragma clang fp contract(off)
     const float p = round_to<T>(x * c);

@@ -610,9 +610,8 @@ void Model::prefill(Seq* s, const void* embeds, int T, int chunk, void* logits, 
     const float scale = 1.f / sqrtf((float)D);
     const int gv = cfg.gemm_variant;
     const bool lead = cfg.tp_rank == 0;
-    // N = hidden linears (o_proj, down_proj) give too few 256x256 tiles at prompt lengths around 1k: the ping-pong GEMM slices K
-    // over up to three workgroups per tile and reduces fp32 partial tiles in the launch (gemm8p.hip).  The scratch is per sequence
-    // (request threads prefill concurrently); <= 256 partial tiles = 64 MiB by construction of gemm8p_pick_split.
+    // N = hidden linears (o_proj, down_proj) give few tiles at prompt lengths around 1k: K is sliced over up to three workgroups per tile and a second
+    // launch adds the fp32 partial tiles (gemm4w.h).  The scratch is per sequence (request threads prefill concurrently); the rules take only as many slices as fit 64 MiB.
     if (dt != kF32 && !s->skw.p) {
         LMX_CHECK_HIP(hipStreamSynchronize(st));
         s->skw.ensure((size_t)256 * 256 * 256 * sizeof(float));

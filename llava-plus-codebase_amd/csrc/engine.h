@@ -219,7 +219,7 @@ struct Model {
     void stack_moe(const StackLayer& l, const void* x, int rows, const StackWs& w, const StackProf& pn, hipStream_t st);
     void stack_heads(const GroupGemvArgs& g, int n, hipStream_t st);
     // ---- options a caller may flip on a live model (lmx_model_set_option; defaults from the environment at creation) ----------------------------------
-    // fuse_rope: RoPE + KV append in the prefill's q|k|v GEMM epilogue (gemm8p.hip qkv_rope_epilogue) instead of a rope_kv launch — bit-identical, faster
+    // fuse_rope: RoPE + KV append in the prefill's q|k|v GEMM epilogue (gemm4w.h qkv_rope_epilogue4) instead of a rope_kv launch — bit-identical, faster
     // vis_pack:  CLIP K / V^T pack in the tower's q|k|v GEMM epilogue instead of a pack launch — bit-identical, launch count
     // splitq:    the decode step's q|k|v projection as q-launch + (k|v projection ∥ attention) launch (decode_attn.hip) — bit-identical
     bool opt_fuse_rope = true, opt_vis_pack = true, opt_splitq = true;

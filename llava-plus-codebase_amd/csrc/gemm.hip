@@ -687,14 +687,18 @@ static void launch_gemm16(const GemmArgs& a, int variant, hipStream_t st) {
     // variant: 0 = auto, 2 = 128x128 reg-staged (kept as an independent cross-check of the LDS-DMA path), 4 = 64x128 glds, 5 = 64x64 glds,
     //          7 / 9 = LDS-ring kernels with counted vmcnt (128x256x64 3-slot, 256x256x64 2-slot; 8 waves), 15 = 64x64 4-slot ring (4 waves),
     //          18 = 128x128x64 2-slot 4 waves.  (Round 5 removed the arms auto never picks: 1, 12, 14 and the deeper rings 23 - 26 of round 4, EXPERIMENTS.md r4-C.)
+    if (variant == 0 && gemm8p_enabled()) {                              // (LMX_GEMM8P=0: the ring kernels below as an A/B and cross-check)
+        const TileForm f = gemm4w_form(TypeInfo<T>::id, a);
+        if (f.mb) { launch_gemm4w(TypeInfo<T>::id, a, f, st); return; }
+    }
     if (variant == 0) {
         const RowsForm f = gemm_rows_form(TypeInfo<T>::id, a);
         if (f.mtiles) { launch_gemm_rows(TypeInfo<T>::id, a, f.mtiles, f.bn, f.slices, st); return; }
     }
     if (a.c_f32) { launch_gemm_cfg<T, 64, 128, 2, 2, true, true>(a, st); return; }      // fp32 logits of a few wanted rows: one tile form
     if (variant == 0) {
-        // Large problems: the ping-pong 256x256x64 kernel (gemm8p.hip), K-sliced when N = hidden leaves CUs idle and the caller brought
-        // the partial-tile scratch (the engine does, per sequence; LMX_GEMM8P=0 switches the kernel off: the ring kernels below as an A/B and cross-check).
+        // What is left of the large problems (up to 256 rows): the ping-pong 256x256x64 kernel (gemm8p.hip), K-sliced when the tiles leave CUs idle and the caller brought
+        // the partial-tile scratch (the engine does, per sequence; LMX_GEMM8P=0 switches the kernel off).
         if (gemm8p_enabled()) {
             const int tiles = cdiv(a.M, 256) * cdiv(a.N, 256);
             const int S = gemm_slices(a);
@@ -747,7 +751,12 @@ bool gemm_fuses_qkv(int dtype, int M, int K, int D, int nh, int nkv, int pos0, i
     const int N = (nh + 2 * nkv) * D;
     if (!gemm8p_enabled() || has_bias || M <= 0 || K % 64 != 0 || !(D == 64 || D == 128) || (nh * D) % 256 != 0 || (nkv * D) % 256 != 0 || pos0 % 8 != 0 || s_max % 8 != 0)
         return false;
-    return cdiv(M, 256) * cdiv(N, 256) >= 160 && gemm8p_pick_split(M, N, K) == 1;      // launch_gemm16's own rule for the un-split ping-pong kernel
+    if (cdiv(M, 256) * cdiv(N, 256) < 160 || gemm8p_pick_split(M, N, K) != 1) return false;
+    // un-split in launch_gemm16's own choice, so that the fused launch adds the same products in the same order
+    void* const any = reinterpret_cast<void*>((uintptr_t)4096);
+    GemmArgs g{any, any, any, nullptr, nullptr, M, N, K, K, K, N, 0, kActNone};
+    g.scratch(any, (size_t)64 << 20);
+    return gemm4w_form(dtype, g).slices == 1;
 }
 
 void launch_gemm(int dtype, const GemmArgs& a, int variant, hipStream_t st) {
@@ -755,6 +764,7 @@ void launch_gemm(int dtype, const GemmArgs& a, int variant, hipStream_t st) {
     if (a.qf_kc) LMX_REQUIRE(variant == 0 && gemm_fuses_qkv(dtype, a.M, a.K, a.qf_D, a.qf_nh, a.qf_nkv, a.qf_pos0, a.qf_smax, a.bias != nullptr),
                              "gemm: the fused q|k|v epilogue needs the un-split ping-pong launch (gemm_fuses_qkv)");
     if (variant == 20) { launch_skinny_gemm(dtype, a, st); return; }
+    if (variant >= 100 && variant < 1000) { launch_gemm4w(dtype, a, TileForm{variant / 100, variant / 10 % 10, variant % 10}, st); return; }
     // 30: ping-pong kernel, K slices chosen by gemm8p_pick_split; 33 / 34 / 35: 2 / 3 / 1 slices forced
     if (variant == 30 || (variant >= 33 && variant <= 35)) {
         GemmArgs b = a;

@@ -1,0 +1,116 @@
+// Host side of the four-wave GEMM (kernels: gemm4w.h): which tile and how many K slices, and the launch.
+#include <algorithm>
+#include <mutex>
+
+#include "gemm4w.h"
+
+namespace lmx {
+
+LMX_GEMM4W_LARGE(LMX_GEMM4W_EXTERN, bf16_t)
+LMX_GEMM4W_SMALL(LMX_GEMM4W_EXTERN, bf16_t)
+LMX_GEMM4W_LARGE(LMX_GEMM4W_EXTERN, f16_t)
+LMX_GEMM4W_SMALL(LMX_GEMM4W_EXTERN, f16_t)
+
+namespace {
+
+struct Tile { int8_t mb, nb; };
+#define LMX_GEMM4W_TILE(T, MB, NB) {MB, NB},
+constexpr Tile kTiles[] = {LMX_GEMM4W_LARGE(LMX_GEMM4W_TILE, ) LMX_GEMM4W_SMALL(LMX_GEMM4W_TILE, )};
+
+// Time of a launch (us), fitted to 3200 timings: 112 products of 139 .. 6528 rows x 256 .. 28000 weights x 512 .. 13824, every tile of 4 .. 8 x 4 .. 8 blocks, 1 .. 3 slices
+// (6 % rms; the form it picks is 1.2 % behind the best one of this table in the mean).  256 workgroups are a round, one a CU.
+//   a K-step:  0.24 us + 0.0129 a block of the tile + 0.0066 a block of its sides
+//   a round that leaves CUs idle has their power: its K-steps take 0.76 + 0.24 x (the share of CUs at work) of that
+//   an epilogue: 0.2 us a block, more with gating or an activation; a slice's plain stores half of that, then the reduction's launch and its reads
+float cost(const GemmArgs& a, int mb, int nb, int S) {
+    const int tiles = cdiv(a.M, 32 * mb) * cdiv(a.N, 32 * nb) * S, n = cdiv(a.K / 64, S), area = mb * nb;
+    const float steps = n * (0.24f + 0.0129f * area + 0.0066f * (mb + nb));
+    const float epi = S > 1 ? 0.108f * area - 0.5f : (act_gated(a.act) ? 0.34f : a.act != kActNone ? 0.64f : 0.215f) * area - 2.2f;
+    float t = (tiles / 256) * (steps + epi);
+    if (const int rem = tiles % 256) {
+        const float share = rem / 256.f;
+        t += steps * (0.76f + 0.24f * share) + epi * std::max(0.5f, share);
+    }
+    if (S > 1) t += 3.8f + 1.17e-6f * S * a.M * a.N;
+    return t;
+}
+
+// fallback K-slice scratch for callers that bring none and ask for slices (lmx_op_gemm: unit tests, microbenchmarks; ONE stream at a time).
+// The engine passes per-sequence scratch instead (Model::prefill), so concurrent request threads never share it.
+struct FallbackWs {
+    std::mutex mu;
+    void* ws = nullptr; size_t ws_bytes = 0;
+};
+FallbackWs g_fb;
+
+template <typename T> void launch_t(const GemmArgs& a, const TileForm& f, hipStream_t st) {
+#define LMX_GEMM4W_CASE(T_, MB, NB) case MB * 16 + NB: gemm4w_launch<T_, MB, NB>(a, f.slices, st); return;
+    switch (f.mb * 16 + f.nb) {
+        LMX_GEMM4W_LARGE(LMX_GEMM4W_CASE, T)
+        LMX_GEMM4W_SMALL(LMX_GEMM4W_CASE, T)
+        default: throw Error{"gemm4w: no such tile"};
+    }
+}
+
+}  // namespace
+
+// what the slices of a product may need at most: the scratch of any tile form (and of 256 x 256 tiles, which callers size theirs by)
+size_t gemm4w_slab_bytes(int M, int N, const TileForm& f) {
+    if (f.slices <= 1) return 0;
+    const size_t tile = (size_t)cdiv(M, 32 * f.mb) * cdiv(N, 32 * f.nb) * f.mb * f.nb * 1024, whole = (size_t)cdiv(M, 256) * cdiv(N, 256) * 65536;
+    return f.slices * std::max(tile, whole) * sizeof(float);
+}
+
+// Which products: more than 256 rows (below, the row tiles of gemm_rows.hip read every weight once) and more than 640 tiles of 64 x 64.  Below that the small tiles and row tiles
+// are the faster ones, us theirs / here:  800 x 1024 x 2048 10.3 / 14.1   2000 x 512 x 2048 12.9 / 14.8   257 x 6208 x 2048 15.1 / 17.1   330 x 4544 x 2304 15.9 / 17.3
+//   577 x 4096 x 1024 13.3 / 13.9   2308 x 1024 x 4096 30.5 / 27.2;  above:  700 x 3072 x 1024 11.4 / 9.8   500 x 12288 x 4096 64.8 / 48.6   400 x 22016 x 4096 gated 97 / 70
+//   1087 x 4096 x 4096 45.5 / 39.7   2048 x 2048 x 2048 23.6 / 18.4   2048 x 2048 x 5632 56.0 / 41.0   2308 x 3072 x 1024 22.0 / 17.5   1541 x 12544 x 4096 170.5 / 126.5.
+TileForm gemm4w_form(int dtype, const GemmArgs& a) {
+    const TileForm none{0, 0, 1};
+    if ((dtype != kBF16 && dtype != kF16) || a.c_f32 || a.K % 64 != 0 || a.N % 8 != 0 || (act_gated(a.act) && a.N % 64 != 0) || (a.pk_kc && a.pk_D % 8 != 0)) return none;
+    if ((size_t)a.M * a.ldx * 2 >= ((size_t)1 << 32) || (size_t)a.N * a.ldw * 2 >= ((size_t)1 << 32)) return none;
+    if (a.M <= 256 || (int64_t)cdiv(a.M, 64) * cdiv(a.N, 64) <= 640) return none;
+    TileForm best = none;
+    float least = 0.f;
+    for (const Tile& t : kTiles) {
+        if (a.qf_kc && t.nb != 8) continue;
+        const int64_t tiles = (int64_t)cdiv(a.M, 32 * t.mb) * cdiv(a.N, 32 * t.nb);
+        for (int S = 1; S <= 3; ++S) {
+            const TileForm f{t.mb, t.nb, S};
+            if (S > 1 && (!a.skw || a.pk_kc || a.qf_kc || tiles * S > 272 || a.K / 64 / S < 10 || gemm4w_slab_bytes(a.M, a.N, f) > a.skw_bytes())) break;
+            const float c = cost(a, t.mb, t.nb, S);
+            if (!best.mb || c < least) { best = f; least = c; }
+        }
+    }
+    return best;
+}
+
+void launch_gemm4w(int dtype, GemmArgs a, TileForm f, hipStream_t st) {
+    LMX_REQUIRE(a.K % 64 == 0, "gemm4w: K must be a multiple of 64");
+    LMX_REQUIRE((size_t)a.M * a.ldx * 2 < ((size_t)1 << 32) && (size_t)a.N * a.ldw * 2 < ((size_t)1 << 32), "gemm4w: operands must be addressable with 32-bit byte offsets");
+    LMX_REQUIRE(!act_gated(a.act) || a.N % 64 == 0, "gemm4w: SiLU·mul needs N % 64 == 0");
+    LMX_REQUIRE(a.N % 4 == 0 && a.ldc % 4 == 0 && (!a.R || a.ldr % 4 == 0) && !a.c_f32, "gemm4w: rows of 8 bytes, 16-bit output");
+    f.slices = std::max(1, std::min({f.slices, 3, cdiv(a.K / 64, 2)}));       // slices of whole pairs of K-steps
+    if (f.slices > 1 && !a.skw) {
+        std::lock_guard<std::mutex> lk(g_fb.mu);
+        const size_t need = (gemm4w_slab_bytes(a.M, a.N, f) + 1023) / 1024 * 1024;
+        if (need > g_fb.ws_bytes) {
+            LMX_CHECK_HIP(hipStreamSynchronize(st));
+            if (g_fb.ws) (void)hipFree(g_fb.ws);
+            g_fb.ws = nullptr; g_fb.ws_bytes = 0;
+            LMX_CHECK_HIP(hipMalloc(&g_fb.ws, need)); g_fb.ws_bytes = need;
+        }
+        a.scratch(g_fb.ws, g_fb.ws_bytes);
+    }
+    LMX_REQUIRE(f.slices == 1 || gemm4w_slab_bytes(a.M, a.N, f) <= a.skw_bytes(), "gemm4w: the partial tiles do not fit the scratch");
+    if (a.qf_kc) LMX_REQUIRE(f.slices == 1 && f.nb == 8 && a.qf_rope && a.qf_vt && (a.qf_D == 64 || a.qf_D == 128) && (a.qf_nh * a.qf_D) % 256 == 0 && (a.qf_nkv * a.qf_D) % 256 == 0 &&
+                             a.N == (a.qf_nh + 2 * a.qf_nkv) * a.qf_D && a.qf_pos0 % 8 == 0 && a.qf_smax % 8 == 0 && !a.bias && !a.R && a.act == kActNone && a.ldc % 8 == 0,
+                             "gemm4w: the fused q|k|v epilogue needs an un-split launch over head-aligned tiles (gemm_fuses_qkv)");
+    // the CLIP K / V^T pack lives in the un-split epilogue only: a K-sliced launch's reduction would write the k | v columns to C and leave the pack untouched
+    if (a.pk_kc) LMX_REQUIRE(f.slices == 1 && !act_gated(a.act) && a.pk_D % 8 == 0 && a.N % 8 == 0, "gemm4w: the K / V^T pack epilogue needs an un-split launch of a plain linear");
+    if (dtype == kBF16) launch_t<bf16_t>(a, f, st);
+    else if (dtype == kF16) launch_t<f16_t>(a, f, st);
+    else throw Error{"gemm4w: 16-bit dtypes only"};
+}
+
+}  // namespace lmx

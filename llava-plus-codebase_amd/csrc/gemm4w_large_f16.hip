@@ -1,0 +1,6 @@
+// f16 instantiations of the four-wave GEMM (gemm4w.h): large tiles
+#include "gemm4w.h"
+
+namespace lmx {
+LMX_GEMM4W_LARGE(LMX_GEMM4W_INST, f16_t)
+}  // namespace lmx

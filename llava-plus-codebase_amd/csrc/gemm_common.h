@@ -1,4 +1,4 @@
-// Pieces shared by the prefill GEMM kernels (gemm.hip, gemm8p.hip): MFMA wrappers, the LDS tile image / swizzle, and the
+// Pieces shared by the prefill GEMM kernels (gemm.hip, gemm8p.hip, gemm4w.h): MFMA wrappers, the LDS tile image / swizzle, and the
 // register epilogue (bias / activation / SiLU·mul / residual, 8-byte packed stores).
 #pragma once
 #include "common.h"

@@ -18,7 +18,7 @@ struct GemmArgs {
     int ldx, ldw, ldc, ldr;
     int act;            // lmx::Act
     const void* Wsw = nullptr;   // skinny kernel only: W re-laid in MFMA-fragment order (skinny_swizzle), else null
-    int split_k = 0;             // ping-pong kernel (gemm8p.hip): K slices per 256x256 tile (0 = let the launcher pick)
+    int split_k = 0;             // ping-pong kernel (gemm8p.hip): K slices per 256x256 tile (0 = let the launcher pick); four-wave kernel: set by its launcher
     // fp32 scratch of the K slices and what it holds, in whole KiB: every rule takes only as many slices as fit, every launcher refuses more.  (Four bytes where the struct had a
     // hole: with every later field eight bytes further the kernels' argument loads were grouped differently, and a decode step of 32 sequences took 2 % longer.)  Null: the
     // ping-pong kernel takes the launcher's own (one stream at a time), the others do not slice
@@ -27,7 +27,7 @@ struct GemmArgs {
     void scratch(void* p, size_t bytes) { skw = p; skw_kib = (uint32_t)(bytes >> 10); }
     size_t skw_bytes() const { return (size_t)skw_kib << 10; }
     int* sk_cnt = nullptr;       // skinny kernel's K slices across workgroups: one arrival ticket per workgroup of rows (N / 16 at most), zero before the first launch (the last arriver re-arms)
-    // q|k|v projection of a prefill with RoPE and the KV-cache append in the EPILOGUE (gemm8p.hip: qkv_rope_epilogue; where gemm_fuses_qkv()
+    // q|k|v projection of a prefill with RoPE and the KV-cache append in the EPILOGUE (gemm4w.h: qkv_rope_epilogue4; where gemm_fuses_qkv()
     // says so): the tile is rounded to T into LDS and leaves the workgroup as  q rows -> rotated, into C (the q columns; k | v columns of C are not
     // written)   k rows -> rotated, into the K cache [kv head][pos][D]   v rows -> the V^T cache [kv head][d][pos].  Same arithmetic and rounding points as
     // launch_gemm + launch_rope_kv (HF5:models/llama/modeling_llama.py:130-160,243-281).  qf_kc != null switches it on.
@@ -42,7 +42,7 @@ struct GemmArgs {
     int c_f32 = 0; float cap = 0.f;
 };
 void launch_gemm(int dtype, const GemmArgs& a, int variant, hipStream_t st);
-// true when launch_gemm(variant 0) of a [M, (nh + 2 nkv) D] x K projection runs as ONE un-split ping-pong launch whose tiles are head-aligned, i.e. can take
+// true when launch_gemm(variant 0) of a [M, (nh + 2 nkv) D] x K projection runs as ONE un-split launch whose tiles are head-aligned, i.e. can take
 // the qf_* fields (pos0 = first cache position of row 0)
 bool gemm_fuses_qkv(int dtype, int M, int K, int D, int nh, int nkv, int pos0, int s_max, bool has_bias);
 // ping-pong 256x256x64 kernel (gemm8p.hip): variant 30 of launch_gemm (33 / 34 / 35: 2 / 3 / 1 K slices forced); LMX_GEMM8P=0 keeps launch_gemm's auto choice off it
@@ -50,6 +50,11 @@ bool gemm8p_enabled();
 void launch_gemm8p(int dtype, const GemmArgs& a, hipStream_t st);
 size_t gemm8p_splitk_ws_bytes(int M, int N, int split_k);
 int gemm8p_pick_split(int M, int N, int K);
+// four-wave kernel (gemm4w.h, gemm4w.hip): tiles of 32 mb x 32 nb, K slices (> 1: fp32 partial tiles in a.skw and a second launch that adds them); variant 100 mb + 10 nb + slices
+struct TileForm { int mb, nb, slices; };
+TileForm gemm4w_form(int dtype, const GemmArgs& a);                   // the form variant 0 takes (mb 0: another kernel)
+size_t gemm4w_slab_bytes(int M, int N, const TileForm& f);
+void launch_gemm4w(int dtype, GemmArgs a, TileForm f, hipStream_t st);
 // linears of up to a few hundred rows (gemm_rows.hip): mtiles row tiles of <= 256 rows, BN = 64 / 128 weight rows a workgroup, S slices of K (S > 1: fp32 slabs in a.skw,
 // gemm_rows_slab_bytes, and a second launch that adds them); variant 1000 mtiles + 100 (BN / 64) + S of launch_gemm
 bool gemm_rows_applies(int dtype, const GemmArgs& a);

@@ -125,6 +125,33 @@ template <> __device__ __forceinline__ void store8<f16_t>(f16_t* p, const float 
     *reinterpret_cast<uint4*>(p) = u;
 }
 
+// 8 elements of T as they lie in memory: requested now, converted when they are needed
+template <typename T> struct Chunk8;
+template <> struct Chunk8<bf16_t> {
+    uint4 r;
+    __device__ __forceinline__ void load(const bf16_t* p) { r = *reinterpret_cast<const uint4*>(p); }
+    __device__ __forceinline__ void get(float (&v)[8]) const {
+        v[0] = unpack_lo<bf16_t>(r.x); v[1] = unpack_hi<bf16_t>(r.x); v[2] = unpack_lo<bf16_t>(r.y); v[3] = unpack_hi<bf16_t>(r.y);
+        v[4] = unpack_lo<bf16_t>(r.z); v[5] = unpack_hi<bf16_t>(r.z); v[6] = unpack_lo<bf16_t>(r.w); v[7] = unpack_hi<bf16_t>(r.w);
+    }
+};
+template <> struct Chunk8<f16_t> {
+    uint4 r;
+    __device__ __forceinline__ void load(const f16_t* p) { r = *reinterpret_cast<const uint4*>(p); }
+    __device__ __forceinline__ void get(float (&v)[8]) const {
+        v[0] = unpack_lo<f16_t>(r.x); v[1] = unpack_hi<f16_t>(r.x); v[2] = unpack_lo<f16_t>(r.y); v[3] = unpack_hi<f16_t>(r.y);
+        v[4] = unpack_lo<f16_t>(r.z); v[5] = unpack_hi<f16_t>(r.z); v[6] = unpack_lo<f16_t>(r.w); v[7] = unpack_hi<f16_t>(r.w);
+    }
+};
+template <> struct Chunk8<float> {
+    float r[8];
+    __device__ __forceinline__ void load(const float* p) { load8<float>(p, r); }
+    __device__ __forceinline__ void get(float (&v)[8]) const {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = r[e];
+    }
+};
+
 // ---- wave64 / block reductions --------------------------------------------------------------
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll

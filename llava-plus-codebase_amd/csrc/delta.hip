@@ -14,7 +14,8 @@
 // the products above.
 //
 // Decode: the read-out o = S^T q after the write equals (g S)^T q + (k . q) u, so both products of a token run over the decayed state at once and the state update is
-// off the critical path.
+// off the critical path.  What bounds one sequence is not bytes (2 MB on 16 heads) but memory latencies in a row: with every load requested ahead of the first wait
+// 12.9 -> 10.0 us at 16 heads of 128 x 128, 54 -> 39 us at 32 sequences of 32 heads (3.4 TB/s of state).
 #include <algorithm>
 #include <type_traits>
 
@@ -393,11 +394,11 @@ void launch_delta_gate(int dtype, const DeltaPrefillArgs& a, hipStream_t st) {
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// one new token per sequence: grid (heads, sequences), 1024 threads
+// one new token per sequence: grid (heads, sequences), NTH threads
 // ---------------------------------------------------------------------------------------------------------------
-template <typename T, int LPC>
-__global__ __launch_bounds__(1024) void delta_decode_kernel(DeltaDecodeArgs a) {
-    constexpr int DK = LPC * 8, NTH = 1024, CPP = NTH / LPC, PF = 2;      // columns of one pass over the state, passes in flight
+template <typename T, int LPC, int NTH>
+__global__ __launch_bounds__(NTH, NTH == 512 && sizeof(T) == 2 ? 4 : 1) void delta_decode_kernel(DeltaDecodeArgs a) {
+    constexpr int DK = LPC * 8, CPP = NTH / LPC, PF = 2048 / NTH, RP = 2048 / NTH;      // columns of one pass over the state, passes in flight, low-rank rows at a time
     extern __shared__ __attribute__((aligned(16))) float sm[];
     __shared__ float red[NTH / 64];
     const int tid = threadIdx.x;
@@ -410,56 +411,115 @@ __global__ __launch_bounds__(1024) void delta_decode_kernel(DeltaDecodeArgs a) {
     T* ring = reinterpret_cast<T*>(e.VT);
     const T* conv = reinterpret_cast<const T*>(a.w.conv);
     const int sub = tid % LPC, col = tid / LPC;
-    // everything that is read from memory is requested before anything waits
+    // Everything that is read from memory is requested before anything waits: state, the first pass over the low-rank rows, inputs and weights of the convolutions (every
+    // slot of the ring, so that no address waits for the position), biases, norm weights.  Addresses past an end are clamped and their values dropped.
     float S[PF][8];
 #pragma unroll
-    for (int p = 0; p < PF; ++p) if (p * CPP + col < DV) load8<float>(st + (size_t)(p * CPP + col) * DK + sub * 8, S[p]);
+    for (int p = 0; p < PF; ++p) {
+        const int c = p * CPP + col;
+        load8<float>(st + (size_t)(c < DV ? c : DV - 1) * DK + sub * 8, S[p]);
+    }
     const int pos = *e.pos_ptr;
+    const T* wdt = reinterpret_cast<const T*>(a.w.dt_bias) + h * DK;
+    // decays and output gates: 8 lanes per row of the second low-rank matrices, RP rows at a time.  Rows of a wave are on one side of DK and of DK + DV (multiples of 64)
+    auto low_rank = [&](int i, const T*& w, const T*& x, int& n) {
+        i = i < DK + DV ? i : DK + DV - 1;
+        const bool is_g = __builtin_amdgcn_readfirstlane(i) < DK;
+        w = reinterpret_cast<const T*>(a.wag) + (size_t)(is_g ? h * DK + i : H * DK + h * DV + i - DK) * a.wag_ld + (is_g ? 0 : a.ra);
+        x = row + a.a_off + (is_g ? 0 : a.ra);
+        n = is_g ? a.ra : a.rg;
+    };
+    const int c8 = (tid & 7) * 8;
+    Chunk8<T> wf[RP][2], xf[RP][2];
+    float bias[RP];
+#pragma unroll
+    for (int m = 0; m < RP; ++m) {
+        const T *w, *x;
+        int n;
+        low_rank((tid >> 3) + m * (NTH / 8), w, x, n);
+        const int c1 = n > 64 ? c8 + 64 : c8;
+        wf[m][0].load(w + c8); wf[m][1].load(w + c1); xf[m][0].load(x + c8); xf[m][1].load(x + c1);
+        const int i = (tid >> 3) + m * (NTH / 8);
+        bias[m] = to_f32(wdt[i < DK ? i : DK - 1]);
+    }
+    const int n_conv = 2 * DK + DV;
+    auto channel = [&](int i) { return i >= 2 * DK ? 2 * G * DK + h * DV + i - 2 * DK : (i < DK ? kh * DK + i : (G + kh) * DK + i - DK); };
+    constexpr int RT = 4;                                    // a ring of up to so many taps is read whole
+    const int ci = channel(tid < n_conv ? tid : n_conv - 1);
+    const T x_new = row[ci];
+    T rv[RT], cv[RT];
+#pragma unroll
+    for (int j = 0; j < RT; ++j) {
+        const int t = j < taps ? j : taps - 1;
+        rv[j] = ring[(size_t)t * C + ci];
+        cv[j] = conv[(size_t)t * C + ci];
+    }
+    const T beta_in = row[C + h], rate_in = reinterpret_cast<const T*>(a.w.A_log)[h], norm_w = reinterpret_cast<const T*>(a.w.norm)[tid < DV ? tid : DV - 1];
     const bool frozen = e.done && *e.done != 0;
-    const float beta = sigmoid_acc(to_f32(row[C + h]));
-    const float rate = expf(to_f32(reinterpret_cast<const T*>(a.w.A_log)[h]));
-    // ---- decays and output gates: 8 lanes per row of the second low-rank matrices
-    for (int i0 = tid >> 3; i0 < DK + DV; i0 += NTH / 4) {   // two rows at a time
-        const T *w[2], *x[2];
-        int n[2];
-        float s[2] = {0.f, 0.f};
+    const float beta = sigmoid_acc(to_f32(beta_in));
+    const float rate = expf(to_f32(rate_in));
+    for (int i0 = tid >> 3; i0 < DK + DV; i0 += 256) {
+        const bool first = i0 == tid >> 3;
+        const T *w[RP], *x[RP];
+        int n[RP];
+        float s[RP] = {};
 #pragma unroll
-        for (int m = 0; m < 2; ++m) {
-            const int i = i0 + m * (NTH / 8);
-            const bool is_g = i < DK;
-            w[m] = reinterpret_cast<const T*>(a.wag) + (size_t)(is_g ? h * DK + i : H * DK + h * DV + i - DK) * a.wag_ld + (is_g ? 0 : a.ra);
-            x[m] = row + a.a_off + (is_g ? 0 : a.ra);
-            n[m] = i >= DK + DV ? 0 : is_g ? a.ra : a.rg;
+        for (int m = 0; m < RP; ++m) low_rank(i0 + m * (NTH / 8), w[m], x[m], n[m]);
+        if (first) {
+#pragma unroll
+            for (int m = 0; m < RP; ++m)
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    if (u == 1 && n[m] <= 64) continue;
+                    float f[8], y[8]; wf[m][u].get(f); xf[m][u].get(y);
+#pragma unroll
+                    for (int e2 = 0; e2 < 8; ++e2) s[m] = fmaf(f[e2], y[e2], s[m]);
+                }
         }
-        const int most = n[0] > n[1] ? n[0] : n[1];
+        const int most = a.ra > a.rg ? a.ra : a.rg;
 #pragma unroll 2
-        for (int c = (tid & 7) * 8; c < most; c += 64)
+        for (int c = c8 + (first ? 128 : 0); c < most; c += 64)
 #pragma unroll
-            for (int m = 0; m < 2; ++m) {
+            for (int m = 0; m < RP; ++m) {
                 if (c >= n[m]) continue;
                 float f[8], y[8]; load8<T>(w[m] + c, f); load8<T>(x[m] + c, y);
 #pragma unroll
                 for (int e2 = 0; e2 < 8; ++e2) s[m] = fmaf(f[e2], y[e2], s[m]);
             }
 #pragma unroll
-        for (int m = 0; m < 2; ++m) {
+        for (int m = 0; m < RP; ++m) {
             const int i = i0 + m * (NTH / 8);
             s[m] = round_to<T>(lanes_sum<8>(s[m]));          // the prompt path stores this product in the model dtype
-            if ((tid & 7) != 0 || n[m] == 0) continue;
-            if (i < DK) g[i] = decay_f32(rate, s[m] + to_f32(reinterpret_cast<const T*>(a.w.dt_bias)[h * DK + i]));
+            if ((tid & 7) != 0 || i >= DK + DV) continue;
+            if (i < DK) g[i] = decay_f32(rate, s[m] + (first ? bias[m] : to_f32(wdt[i])));
             else gate[i - DK] = sigmoid_acc(s[m]);
         }
     }
     // ---- short convolutions: thread per channel; the ring slot of this position is not one that any tap reads
     const int slot = pos % taps;
-    for (int i = tid; i < 2 * DK + DV; i += NTH) {
+    for (int i = tid; i < n_conv; i += NTH) {
         const bool is_v = i >= 2 * DK;
-        const int c = is_v ? 2 * G * DK + h * DV + i - 2 * DK : (i < DK ? kh * DK + i : (G + kh) * DK + i - DK);
-        const T xin = row[c];
-        float s = to_f32(xin) * to_f32(conv[(size_t)(taps - 1) * C + c]);
-        for (int j = 1, sl = slot; j < taps; ++j) {
-            sl = sl == 0 ? taps - 1 : sl - 1;
-            if (pos - j >= 0) s = fmaf(to_f32(ring[(size_t)sl * C + c]), to_f32(conv[(size_t)(taps - 1 - j) * C + c]), s);
+        const int c = channel(i);
+        T xin;
+        float s;
+        if (i == tid && taps <= RT) {
+            xin = x_new;
+            const int last = taps - 1;
+            const float r0 = to_f32(rv[0]), r1 = to_f32(rv[1]), r2 = to_f32(rv[2]), r3 = to_f32(rv[3]), w0 = to_f32(cv[0]), w1 = to_f32(cv[1]), w2 = to_f32(cv[2]), w3 = to_f32(cv[3]);
+            s = to_f32(xin) * (last == 0 ? w0 : last == 1 ? w1 : last == 2 ? w2 : w3);
+#pragma unroll
+            for (int j = 1; j < RT; ++j) {
+                if (j >= taps || pos - j < 0) continue;
+                const int sl = slot >= j ? slot - j : slot - j + taps, t = last - j;
+                s = fmaf(sl == 0 ? r0 : sl == 1 ? r1 : sl == 2 ? r2 : r3, t == 0 ? w0 : t == 1 ? w1 : w2, s);
+            }
+        } else {
+            xin = row[c];
+            s = to_f32(xin) * to_f32(conv[(size_t)(taps - 1) * C + c]);
+            for (int j = 1, sl = slot; j < taps; ++j) {
+                sl = sl == 0 ? taps - 1 : sl - 1;
+                if (pos - j >= 0) s = fmaf(to_f32(ring[(size_t)sl * C + c]), to_f32(conv[(size_t)(taps - 1 - j) * C + c]), s);
+            }
         }
         if (is_v || h % rep == 0) ring[(size_t)slot * C + c] = xin;
         s = silu_acc(s);
@@ -508,7 +568,7 @@ __global__ __launch_bounds__(1024) void delta_decode_kernel(DeltaDecodeArgs a) {
     ss = block_sum<NTH / 64>(ss, red);                       // (its barriers also publish o)
     const float inv = 1.f / sqrtf(ss / (float)a.s.dv + a.eps);
     T* out = reinterpret_cast<T*>(a.out) + (size_t)z * a.out_ld + h * DV;
-    for (int c = tid; c < DV; c += NTH) out[c] = from_f32<T>(o[c] * inv * to_f32(reinterpret_cast<const T*>(a.w.norm)[c]) * gate[c]);
+    for (int c = tid; c < DV; c += NTH) out[c] = from_f32<T>(o[c] * inv * to_f32(c == tid ? norm_w : reinterpret_cast<const T*>(a.w.norm)[c]) * gate[c]);
 }
 
 void launch_delta_decode(int dtype, const DeltaDecodeArgs& a, hipStream_t st) {
@@ -519,9 +579,16 @@ void launch_delta_decode(int dtype, const DeltaDecodeArgs& a, hipStream_t st) {
     const dim3 grid(a.s.H, a.n_seq);
     const size_t smem = (size_t)(3 * a.s.DK + 3 * a.s.DV) * 4;
     LMX_REQUIRE(smem <= 60 * 1024 && a.a_off % 8 == 0, "delta_decode: head widths too large");
-    if (dtype == kBF16) { using TT = bf16_t; DELTA_KB(delta_decode_kernel, grid, 1024, smem, a); }
-    else if (dtype == kF16) { using TT = f16_t; DELTA_KB(delta_decode_kernel, grid, 1024, smem, a); }
-    else { using TT = float; DELTA_KB(delta_decode_kernel, grid, 1024, smem, a); }
+#define L(TT, NTH) do { if (a.s.DK == 64) LMX_LAUNCH((delta_decode_kernel<TT, 8, NTH>), grid, dim3(NTH), smem, st, a); \
+                        else if (a.s.DK == 128) LMX_LAUNCH((delta_decode_kernel<TT, 16, NTH>), grid, dim3(NTH), smem, st, a); \
+                        else LMX_LAUNCH((delta_decode_kernel<TT, 32, NTH>), grid, dim3(NTH), smem, st, a); } while (0)
+#define LN(TT) do { if (wide) L(TT, 1024); else L(TT, 512); } while (0)
+    // 1024 threads a head while every workgroup has a CU of its own; past that two workgroups of 512 on a CU, whose reads and arithmetic overlap.  us at 16 x 16 / 16 x 24 /
+    // 32 x 32 heads x sequences: 1024 threads 13.8 / 22.5 / 45.4, 512 threads 15.9 / 20.0 / 40.5
+    const bool wide = a.s.H * a.n_seq <= 256;
+    if (dtype == kBF16) LN(bf16_t); else if (dtype == kF16) LN(f16_t); else LN(float);
+#undef LN
+#undef L
     LMX_CHECK_HIP(hipGetLastError());
 }
 

@@ -421,32 +421,6 @@ void launch_rows_attn(int dtype, int D, const FlashArgs& a, hipStream_t st) {
 // norm and rotation.  The workgroup that walks the chunk of position `pos` takes the new key from the qkv row (and, for the first query head of a kv group, appends
 // it); it is never read back from the cache inside the launch.  Splits are merged by the last workgroup of a head to arrive (write-through partials, one ticket).
 // ---------------------------------------------------------------------------------------------------------------
-template <typename T> struct Chunk8;
-template <> struct Chunk8<bf16_t> {
-    uint4 r;
-    __device__ __forceinline__ void load(const bf16_t* p) { r = *reinterpret_cast<const uint4*>(p); }
-    __device__ __forceinline__ void get(float (&v)[8]) const {
-        v[0] = unpack_lo<bf16_t>(r.x); v[1] = unpack_hi<bf16_t>(r.x); v[2] = unpack_lo<bf16_t>(r.y); v[3] = unpack_hi<bf16_t>(r.y);
-        v[4] = unpack_lo<bf16_t>(r.z); v[5] = unpack_hi<bf16_t>(r.z); v[6] = unpack_lo<bf16_t>(r.w); v[7] = unpack_hi<bf16_t>(r.w);
-    }
-};
-template <> struct Chunk8<f16_t> {
-    uint4 r;
-    __device__ __forceinline__ void load(const f16_t* p) { r = *reinterpret_cast<const uint4*>(p); }
-    __device__ __forceinline__ void get(float (&v)[8]) const {
-        v[0] = unpack_lo<f16_t>(r.x); v[1] = unpack_hi<f16_t>(r.x); v[2] = unpack_lo<f16_t>(r.y); v[3] = unpack_hi<f16_t>(r.y);
-        v[4] = unpack_lo<f16_t>(r.z); v[5] = unpack_hi<f16_t>(r.z); v[6] = unpack_lo<f16_t>(r.w); v[7] = unpack_hi<f16_t>(r.w);
-    }
-};
-template <> struct Chunk8<float> {
-    float r[8];
-    __device__ __forceinline__ void load(const float* p) { load8<float>(p, r); }
-    __device__ __forceinline__ void get(float (&v)[8]) const {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = r[e];
-    }
-};
-
 // one head vector by one wave: norm over the true width, rotation, into out[D] (fp32 LDS); tmp[D] is scratch of this wave
 template <typename T, int D>
 __device__ __forceinline__ void norm_rope_vec(const T* __restrict__ x, const T* __restrict__ nw, float eps, int qk_dim, const float* __restrict__ cs, int rot_dims,

@@ -206,7 +206,7 @@ __device__ __forceinline__ f32x4 ldg4(const float* p) { return *reinterpret_cast
 // lanes: register i of lane l of an accumulator is row 4 (l / 16) + i, column l % 16, which as a B operand is k index l / 16 of the i-th of four products whose A operands
 // hold columns 4 (l / 16) + i.  The waves' parts of (D k) S and of o meet in LDS.
 template <typename T, int LPC>
-__global__ __launch_bounds__(256, 1) void delta_scan_kernel(DeltaPrefillArgs a) {
+__global__ __launch_bounds__(256, LPC <= 16 && sizeof(T) == 2 ? 2 : 1) void delta_scan_kernel(DeltaPrefillArgs a) {
     constexpr int DK = LPC * 8, NT = DK / 64, C = DELTA_C;
     __shared__ __attribute__((aligned(16))) f32x4 wb[2][4][64], ob[2][4][64];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -220,62 +220,87 @@ __global__ __launch_bounds__(256, 1) void delta_scan_kernel(DeltaPrefillArgs a) 
     for (int j = 0; j < NT; ++j) S[j] = sg.pos0 > 0 ? ldg4(st + j * 16) : f32x4{0.f, 0.f, 0.f, 0.f};
     using Raw = std::conditional_t<sizeof(T) == 2, uint2, f32x4>;
     struct Chunk { f32x4 kd[NT], qd[NT], kt[NT], dc[NT], tm; float pm; Raw v; };
+    // a chunk's base is uniform, a lane's place in it does not change: one 32-bit offset a lane for each array
+    const unsigned o_kd = r16 * DK + cb + q4, o_kt = (cb + r16) * C + q4, o_dc = cb + q4, o_tm = r16 * C + q4, o_v = (c0 + r16) * C + q4;
     auto fetch = [&](int n, Chunk& x) {
         const size_t ch = (size_t)(sg.chunk0 + n) * H + h;
+        const float *kd = a.kd + ch * C * DK, *qd = a.qd + ch * C * DK, *kt = a.kt + ch * DK * C, *dc = a.dc + ch * DK, *tm = a.tm + ch * C * C, *pm = a.pm + ch * C * C;
+        const T* v = reinterpret_cast<const T*>(a.v) + ch * DV * C;
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
-            const int c = cb + j * 16;
-            x.kd[j] = ldg4(a.kd + (ch * C + r16) * DK + c + q4);
-            x.qd[j] = ldg4(a.qd + (ch * C + r16) * DK + c + q4);
-            x.kt[j] = ldg4(a.kt + (ch * DK + c + r16) * C + q4);
-            x.dc[j] = ldg4(a.dc + ch * DK + c + q4);
+            x.kd[j] = ldg4(kd + o_kd + j * 16);
+            x.qd[j] = ldg4(qd + o_kd + j * 16);
+            x.kt[j] = ldg4(kt + o_kt + j * 16 * C);
+            x.dc[j] = ldg4(dc + o_dc + j * 16);
         }
-        x.tm = ldg4(a.tm + (ch * C + r16) * C + q4);
-        x.pm = a.pm[(ch * C + r16) * C + q4 + wave];
-        x.v = *reinterpret_cast<const Raw*>(reinterpret_cast<const T*>(a.v) + (ch * DV + c0 + r16) * C + q4);
+        x.tm = ldg4(tm + o_tm);
+        x.pm = pm[o_tm + wave];
+        x.v = *reinterpret_cast<const Raw*>(v + o_v);
     };
-    auto put_o = [&](int n) {                                // chunk n's read-out, one element a thread
-        const int t = ((tid >> 2) >> 4) * 4 + (tid & 3), col = (tid >> 2) & 15;
+    // a read-out of the chunk before, one element a thread; its parts are in LDS since the barrier of this step
+    const int ot = (tid >> 6) * 4 + (tid & 3), ocol = (tid >> 2) & 15;
+    float* const obase = a.o + (size_t)sg.row0 * H * DV + (size_t)h * DV + c0;
+    const unsigned o_o = (unsigned)ot * H * DV + ocol;
+    auto put_o = [&](int n, float v) { if (n * C + ot < sg.n) (obase + (size_t)n * C * H * DV)[o_o] = v; };
+    auto sum_o = [&](int n) {
         const float* p = reinterpret_cast<const float*>(&ob[n & 1][0][0]) + tid;
-        const float v = (p[0] + p[256]) + (p[512] + p[768]);
-        if (n * C + t < sg.n) a.o[((size_t)sg.row0 + n * C + t) * H * DV + (size_t)h * DV + c0 + col] = v;
+        return (p[0] + p[256]) + (p[512] + p[768]);
     };
     const int nc = (sg.n + C - 1) / C;
-    auto step = [&](int n, const Chunk& cur) {
+    // The chain of a chunk is W (8 products of 32 cycles), its way through LDS, U (4) and the new S (8); what does not hang on it fills the waits: O's products cover the
+    // write, the barrier and the reads.  The fences keep it in this order.
+    auto step = [&](int n, const Chunk& cur, auto fetch_next) {
         f32x4 W = {0.f, 0.f, 0.f, 0.f}, O = W, U = W, X;
 #pragma unroll
         for (int j = 0; j < NT; ++j)
 #pragma unroll
             for (int i = 0; i < 4; ++i) W = mfma4(cur.kd[j][i], S[j][i], W);
+        fetch_next();
+        __builtin_amdgcn_sched_barrier(0);
+        constexpr int NO = NT * 4;
+        auto part_o = [&](int k) { O = mfma4(cur.qd[k / 4][k % 4], S[k / 4][k % 4], O); };
+        part_o(0);
+        __builtin_amdgcn_sched_barrier(0);
         wb[n & 1][wave][lane] = W;
 #pragma unroll
-        for (int j = 0; j < NT; ++j)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) O = mfma4(cur.qd[j][i], S[j][i], O);
+        for (int k = 1; k < NO / 2; ++k) part_o(k);
+        __builtin_amdgcn_sched_barrier(0);
         // LDS only: a full barrier would also wait for the chunks that are on their way
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
         const f32x4 w0 = wb[n & 1][0][lane], w1 = wb[n & 1][1][lane], w2 = wb[n & 1][2][lane], w3 = wb[n & 1][3][lane];
+        float o_prev = 0.f;
+        if (n > 0) o_prev = sum_o(n - 1);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int k = NO / 2; k < NO; ++k) part_o(k);
         f32x4 v;
         if constexpr (sizeof(T) == 2) v = f32x4{unpack_lo<T>(cur.v.x), unpack_hi<T>(cur.v.x), unpack_lo<T>(cur.v.y), unpack_hi<T>(cur.v.y)}; else v = cur.v;
 #pragma unroll
         for (int i = 0; i < 4; ++i) X[i] = v[i] - ((w0[i] + w1[i]) + (w2[i] + w3[i]));
 #pragma unroll
-        for (int i = 0; i < 4; ++i) U = mfma4(cur.tm[i], X[i], U);
-#pragma unroll
-        for (int j = 0; j < NT; ++j) {
+        for (int j = 0; j < NT; ++j)
 #pragma unroll
             for (int i = 0; i < 4; ++i) S[j][i] *= cur.dc[j][i];
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) S[j] = mfma4(cur.kt[j][i], U[i], S[j]);
-        }
-        O = mfma4(cur.pm, wave == 0 ? U[0] : wave == 1 ? U[1] : wave == 2 ? U[2] : U[3], O);      // a quarter of P U per wave
+        for (int i = 0; i < 4; ++i) U = mfma4(cur.tm[i], X[i], U);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j) S[j] = mfma4(cur.kt[j][i], U[i], S[j]);
+        const float u = wave < 2 ? (wave == 0 ? U[0] : U[1]) : (wave == 2 ? U[2] : U[3]);
+        O = mfma4(cur.pm, u, O);                             // a quarter of P U per wave
         ob[n & 1][wave][lane] = O;
-        if (n > 0) put_o(n - 1);
+        if (n > 0) put_o(n - 1, o_prev);
+        __builtin_amdgcn_sched_barrier(0);
     };
-    // NB chunks in registers, NB - 1 of them on their way; past the last chunk the last one is read again
-    constexpr int NB = NT >= 4 ? 3 : 4;
+    // Two chunks in registers, one of them on its way; past the last chunk the last one is read again.  More of them gave nothing (the chain above bounds a step) and took the
+    // registers of a second workgroup on the CU, which short and many sequences need.  us at 16 heads x 1100 rows / 16 heads x (1100, 890, 680) / 32 heads x 16 sequences of
+    // about 50: four chunks and one workgroup 73.5 / 106 / 108, this 62 / 94 / 64
+    constexpr int NB = 2;
     Chunk buf[NB];
     auto at = [&](int n) { return n < nc ? n : nc - 1; };
 #pragma unroll
@@ -283,11 +308,11 @@ __global__ __launch_bounds__(256, 1) void delta_scan_kernel(DeltaPrefillArgs a) 
     int n = 0;
     for (; n + NB <= nc; n += NB)
 #pragma unroll
-        for (int u = 0; u < NB; ++u) { fetch(at(n + u + NB - 1), buf[(u + NB - 1) % NB]); step(n + u, buf[u]); }
+        for (int u = 0; u < NB; ++u) step(n + u, buf[u], [&] { fetch(at(n + u + NB - 1), buf[(u + NB - 1) % NB]); });
 #pragma unroll
-    for (int u = 0; u < NB - 1; ++u) if (n + u < nc) step(n + u, buf[u]);
+    for (int u = 0; u < NB - 1; ++u) if (n + u < nc) step(n + u, buf[u], [] {});
     __syncthreads();
-    put_o(nc - 1);
+    put_o(nc - 1, sum_o(nc - 1));
 #pragma unroll
     for (int j = 0; j < NT; ++j) *reinterpret_cast<f32x4*>(st + j * 16) = S[j];
     // the newest inputs of the convolutions: every channel once, spread over the segment's workgroups

@@ -719,6 +719,21 @@ int lmx_op_decode_win_form(int32_t dtype, int32_t D, int32_t n_heads, int32_t n_
     LMX_API_END
 }
 
+size_t lmx_op_group_plan_bytes(int32_t rows, int32_t per_row) { return rows > 0 && per_row > 0 ? group_plan_bytes(rows * per_row) : 0; }
+int lmx_op_group_gemm(int32_t dtype, const void* x, const void* w, void* c, const int32_t* ids, int32_t rows, int32_t per_row, int32_t groups, int32_t shared_x, int32_t N, int32_t K,
+                      int32_t act, int32_t bm, int32_t nb, void* plan, void* stream) {
+    LMX_API_BEGIN
+    LMX_REQUIRE(x && w && c && ids && plan && rows >= 1 && per_row >= 1 && groups >= 1, "group_gemm: bad arguments");
+    const int slots = rows * per_row;
+    GroupGemmArgs a{x, w, c, N, K, K, K, act == kActSiluMul || act == kActReluMul ? N / 2 : N, (size_t)N * K, slots, groups};
+    a.act = act; a.per_row = shared_x ? per_row : 1;
+    a.plan = group_plan_at(plan, slots);
+    if (bm == 0) bm = group_gemm_bm(&a, 1);
+    launch_group_plan(ids, slots, groups, bm, a.plan, S(stream));
+    launch_group_gemm(dtype, a, bm, S(stream), nb);
+    LMX_API_END
+}
+
 // ---- training-step slices (train.hip) ---------------------------------------------------------------------------------------------
 int lmx_op_ce_loss(int32_t dtype, const void* logits, int32_t ld, const int64_t* labels, int32_t B, int32_t T, int32_t V, int64_t ignore_index,
                    float* lse_scratch, float* row_loss_scratch, float* out_loss_count, float grad, void* dlogits_or_null, int32_t ldd, void* stream) {

@@ -89,6 +89,7 @@ template <int MB, int NB> struct Shape4w {
     static constexpr int OX0 = 0, OW0 = MB0 * 4096, OW1 = OW0 + NB0 * 4096, OX1 = OW1 + NB1 * 4096;
     static constexpr int NR = 160 * 1024 / STEP < 4 ? 160 * 1024 / STEP : 4;      // K-steps of the ring
     static constexpr int LDS = NR * STEP;
+    static_assert(LDS + BM * 4 <= 160 * 1024, "the grouped form keeps its rows' slots beside the ring");
 };
 constexpr int QF4_PITCH = 264;                               // elements per LDS row of the q|k|v epilogue
 
@@ -234,8 +235,9 @@ __device__ __forceinline__ void qkv_rope_epilogue4(const GemmArgs& a, f32x4 (&ac
     }
 }
 
-template <typename T, int MB, int NB>
-__device__ __forceinline__ void epilogue4(const GemmArgs& a, f32x4 (&acc)[NB][MB], int m0, int n0, int wm, int wn, int lane) {
+// out_row(m): row of C that row m of the tile's problem is written to
+template <typename T, int MB, int NB, typename F>
+__device__ __forceinline__ void epilogue4(const GemmArgs& a, f32x4 (&acc)[NB][MB], int m0, int n0, int wm, int wn, int lane, F&& out_row) {
     constexpr int P = (NB + 1) / 2;                                     // pairs of blocks
     T* C = reinterpret_cast<T*>(a.C);
     const T* bias = reinterpret_cast<const T*>(a.bias);
@@ -278,7 +280,7 @@ __device__ __forceinline__ void epilogue4(const GemmArgs& a, f32x4 (&acc)[NB][MB
 #pragma unroll
             for (int jj = 0; jj < MB; ++jj)
                 if (jj == j) take(t, jj);
-            T* row = C + (size_t)m * a.ldc + (nb >> 1);
+            T* row = C + (size_t)out_row(m) * a.ldc + (nb >> 1);
             uint32_t o2[2 * ((P + 1) / 2)][2];                           // four outputs a lane of pair p
 #pragma unroll
             for (int p = 0; p < P; ++p) {
@@ -352,7 +354,7 @@ __device__ __forceinline__ void epilogue4(const GemmArgs& a, f32x4 (&acc)[NB][MB
             columns(t, v);
             if (bias) add_bias(v);
             if (R) residual(v, rows[j]);
-            T* row = C + (size_t)m * a.ldc;
+            T* row = C + (size_t)out_row(m) * a.ldc;
 #pragma unroll
             for (int p = 0; p < P; ++p) {
                 const int c = 32 * p + cb, n = nb + c;
@@ -397,7 +399,7 @@ __device__ __forceinline__ void epilogue4(const GemmArgs& a, f32x4 (&acc)[NB][MB
             }
         }
         if (R) residual(v, rq);
-        T* row = C + (size_t)m * a.ldc;
+        T* row = C + (size_t)out_row(m) * a.ldc;
 #pragma unroll
         for (int p = 0; p < P; ++p) {
             const int c = 32 * p + cb, n = nb + c;
@@ -420,54 +422,23 @@ __device__ __forceinline__ void epilogue4(const GemmArgs& a, f32x4 (&acc)[NB][MB
     }
 }
 
-template <typename T, int MB, int NB, bool SPLIT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm4w_kernel(GemmArgs a) {
+// weight row behind buffer row rb + 32 i of a tile's W halves
+template <int NB> __device__ __forceinline__ int weight_row(int i, int rb, int n0, int N, bool gated) {
+    constexpr int NB0 = (NB + 1) / 2, NB1 = NB / 2;
+    const int half = i >= NB0, blocks = half ? NB1 : NB0, r = (half ? i - NB0 : i) * 32 + rb;      // buffer row of the half
+    const int w = r >= 16 * blocks, c = r - w * 16 * blocks;
+    int n = n0 + w * NB * 16 + half * NB0 * 16 + c;
+    if (gated) n = gated_row(n);
+    return n < N ? n : N - 1;
+}
+
+// the K-steps [kt_begin, kt_begin + nk) of one tile.  vx, vw: byte offsets of the thread's DMA pieces in the operands; x1_live: the tile has rows in X half 1 (without, its phases are skipped)
+template <typename T, int MB, int NB>
+__device__ __forceinline__ void product4(f32x4 (&acc)[NB][MB], char* smem, v4i_t rsX, v4i_t rsW, const uint32_t (&vx)[MB], const uint32_t (&vw)[NB], int kt_begin, int nk, bool x1_live,
+                                         int tid) {
     using SH = Shape4w<MB, NB>;
     constexpr int MB0 = SH::MB0, MB1 = SH::MB1, NB0 = SH::NB0, NB1 = SH::NB1;
-    extern __shared__ __attribute__((aligned(16))) char smem[];
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave & 1, wn = wave >> 1;
-    const int l15 = lane & 15, g4 = lane >> 4;
-
-    const int S = SPLIT ? a.split_k : 1;
-    const int mtiles = (a.M + SH::BM - 1) / SH::BM, ntiles = (a.N + SH::BN - 1) / SH::BN;
-    const int lid = xcd_remap(blockIdx.x, mtiles * ntiles * S);
-    const int tile = SPLIT ? lid / S : lid, slice = SPLIT ? lid - tile * S : 0;
-    int tile_m, tile_n;
-    if constexpr (!SPLIT) gemm_tile_of(tile, mtiles, ntiles, tile_m, tile_n);
-    else { tile_n = tile / mtiles; tile_m = tile - tile_n * mtiles; }
-    const int m0 = tile_m * SH::BM, n0 = tile_n * SH::BN;
-    const int nk_all = a.K >> 6;
-    const int pairs = (nk_all + 1) >> 1;                     // slices of whole pairs: only the last one can end on an odd K-step
-    const int kt_begin = SPLIT ? 2 * (int)((long)pairs * slice / S) : 0;
-    const int kt_end = SPLIT && slice + 1 < S ? 2 * (int)((long)pairs * (slice + 1) / S) : nk_all;
-    const int nk = kt_end - kt_begin;
-
-    // ---- LDS-DMA sources: piece i of a half covers buffer rows 8 (wave + 4 i) .. + 7 -----------------------------------------------
-    v4i_t rsX = make_rsrc(a.X, (uint32_t)((size_t)a.M * a.ldx * sizeof(T)));
-    v4i_t rsW = make_rsrc(a.W, (uint32_t)((size_t)a.N * a.ldw * sizeof(T)));
-    uint32_t vx[MB], vw[NB];
-    {
-        const int rb = 8 * wave + (lane >> 3);
-        const int chunk = ((lane & 7) ^ (rb >> 1)) & 7;
-        const bool gated = act_gated(a.act);
-#pragma unroll
-        for (int i = 0; i < MB; ++i) {
-            int m = m0 + i * 32 + rb;                        // tile rows in order: half 1 follows half 0
-            m = m < a.M ? m : a.M - 1;
-            vx[i] = (uint32_t)(((size_t)m * a.ldx + chunk * 8) * sizeof(T));
-        }
-#pragma unroll
-        for (int i = 0; i < NB; ++i) {
-            const int half = i >= NB0, blocks = half ? NB1 : NB0, r = (half ? i - NB0 : i) * 32 + rb;      // buffer row of the half
-            const int w = r >= 16 * blocks, c = r - w * 16 * blocks;
-            int n = n0 + w * NB * 16 + half * NB0 * 16 + c;
-            if (gated) n = gated_row(n);
-            n = n < a.N ? n : a.N - 1;
-            vw[i] = (uint32_t)(((size_t)n * a.ldw + chunk * 8) * sizeof(T));
-        }
-    }
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave & 1, wn = wave >> 1, l15 = lane & 15, g4 = lane >> 4;
     const unsigned lds_base = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
     const unsigned lds_wave = __builtin_amdgcn_readfirstlane(lds_base + wave * 1024);
 
@@ -489,7 +460,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
         }
     }
 
-    f32x4 acc[NB][MB];
 #pragma unroll
     for (int i = 0; i < NB; ++i)
 #pragma unroll
@@ -501,8 +471,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     auto rd_x1 = [&](int ring, int t) { const int ks = t / MB1, i = t % MB1; x1[ks][i] = at(ox[ks] + ring + SH::OX1 + i * 4096); };
     auto rd_w0 = [&](int ring, int t) { const int ks = t / NB0, i = t % NB0; w0[ks][i] = at(ow0[ks] + ring + i * 2048); };
     auto rd_w1 = [&](int ring, int t) { const int ks = t / NB1, i = t % NB1; w1[ks][i] = at(ow1[ks] + ring + i * 2048); };
-
-    const bool x1_live = a.M - m0 > 32 * MB0;                // a ragged tile without rows in X half 1 skips its phases
 
     auto main_loop = [&](auto live_c) {
         constexpr bool X1 = decltype(live_c)::value;
@@ -606,6 +574,54 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     else main_loop(IC<0>{});
     mfma_settle();
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");         // no LDS write is on its way when the workgroup, or its ring, ends
+}
+
+template <typename T, int MB, int NB, bool SPLIT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm4w_kernel(GemmArgs a) {
+    using SH = Shape4w<MB, NB>;
+    constexpr int MB0 = SH::MB0;
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave & 1, wn = wave >> 1;
+    const int l15 = lane & 15, g4 = lane >> 4;
+
+    const int S = SPLIT ? a.split_k : 1;
+    const int mtiles = (a.M + SH::BM - 1) / SH::BM, ntiles = (a.N + SH::BN - 1) / SH::BN;
+    const int lid = xcd_remap(blockIdx.x, mtiles * ntiles * S);
+    const int tile = SPLIT ? lid / S : lid, slice = SPLIT ? lid - tile * S : 0;
+    int tile_m, tile_n;
+    if constexpr (!SPLIT) gemm_tile_of(tile, mtiles, ntiles, tile_m, tile_n);
+    else { tile_n = tile / mtiles; tile_m = tile - tile_n * mtiles; }
+    const int m0 = tile_m * SH::BM, n0 = tile_n * SH::BN;
+    const int nk_all = a.K >> 6;
+    const int pairs = (nk_all + 1) >> 1;                     // slices of whole pairs: only the last one can end on an odd K-step
+    const int kt_begin = SPLIT ? 2 * (int)((long)pairs * slice / S) : 0;
+    const int kt_end = SPLIT && slice + 1 < S ? 2 * (int)((long)pairs * (slice + 1) / S) : nk_all;
+    const int nk = kt_end - kt_begin;
+
+    // ---- LDS-DMA sources: piece i of a half covers buffer rows 8 (wave + 4 i) .. + 7 -----------------------------------------------
+    v4i_t rsX = make_rsrc(a.X, (uint32_t)((size_t)a.M * a.ldx * sizeof(T)));
+    v4i_t rsW = make_rsrc(a.W, (uint32_t)((size_t)a.N * a.ldw * sizeof(T)));
+    uint32_t vx[MB], vw[NB];
+    {
+        const int rb = 8 * wave + (lane >> 3);
+        const int chunk = ((lane & 7) ^ (rb >> 1)) & 7;
+        const bool gated = act_gated(a.act);
+#pragma unroll
+        for (int i = 0; i < MB; ++i) {
+            int m = m0 + i * 32 + rb;                        // tile rows in order: half 1 follows half 0
+            m = m < a.M ? m : a.M - 1;
+            vx[i] = (uint32_t)(((size_t)m * a.ldx + chunk * 8) * sizeof(T));
+        }
+#pragma unroll
+        for (int i = 0; i < NB; ++i) {
+            const int n = weight_row<NB>(i, rb, n0, a.N, gated);
+            vw[i] = (uint32_t)(((size_t)n * a.ldw + chunk * 8) * sizeof(T));
+        }
+    }
+    f32x4 acc[NB][MB];
+    product4<T, MB, NB>(acc, smem, rsX, rsW, vx, vw, kt_begin, nk, a.M - m0 > 32 * MB0, tid);
 
     if constexpr (!SPLIT) {
         if constexpr (NB == 8) {
@@ -615,7 +631,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
                 return;
             }
         }
-        epilogue4<T, MB, NB>(a, acc, m0, n0, wm, wn, lane);
+        epilogue4<T, MB, NB>(a, acc, m0, n0, wm, wn, lane, [](int m) { return m; });
     } else {
         // fp32 partial tile in accumulator order: float4 number j NB + i of thread tid at ((j NB + i) 256 + tid) 16 of the slab
         f32x4* slab = reinterpret_cast<f32x4*>(a.skw) + ((size_t)tile * S + slice) * (SH::BM * SH::BN / 4) + tid;
@@ -626,6 +642,53 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
             for (int i = 0; i < NB; ++i) slab[(j * NB + i) * 256] = acc[i][j];
         }
     }
+}
+
+// The rows of a group times its weight (GroupGemmArgs with a plan; bound and figures: as the linears above, group_gemm_bm): tile rows are slots, their X rows gathered through the DMA offsets, their C rows scattered by the
+// epilogue.  Tiles run group by group, a group's row tiles next to each other for one panel of its weight.  The grid is an upper bound: workgroups past the plan's tiles leave.
+template <typename T, int MB, int NB>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void group_gemm4w_kernel(GroupGemmArgs a) {
+    using SH = Shape4w<MB, NB>;
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave & 1, wn = wave >> 1;
+    const int ntiles = (a.N + SH::BN - 1) / SH::BN, total = *a.plan.n_tiles * ntiles;
+    if ((int)blockIdx.x >= total) return;
+    const int lid = xcd_remap(blockIdx.x, total);
+    const GroupTile t = a.plan.tiles[lid / ntiles];
+    const int rel = lid - t.first * ntiles;
+    const GroupTile u = a.plan.tiles[t.first + rel % t.n_tiles];
+    const int grp = __builtin_amdgcn_readfirstlane(u.group), row0 = __builtin_amdgcn_readfirstlane(u.row0), rows = __builtin_amdgcn_readfirstlane(u.rows);
+    const int n0 = __builtin_amdgcn_readfirstlane(rel / t.n_tiles) * SH::BN;
+    const int* order = a.plan.order + row0;
+    __shared__ int slots[SH::BM];                            // (the product's first barriers stand between this and the epilogue)
+    if (tid < SH::BM) slots[tid] = order[tid < rows ? tid : rows - 1];
+    const v4i_t rsX = make_rsrc(a.X, (uint32_t)((size_t)(a.rows / a.per_row) * a.ldx * sizeof(T)));
+    const v4i_t rsW = make_rsrc(reinterpret_cast<const T*>(a.W) + (size_t)grp * a.w_group, (uint32_t)((size_t)a.N * a.ldw * sizeof(T)));
+    uint32_t vx[MB], vw[NB];
+    const int rb = 8 * wave + (lane >> 3), chunk = ((lane & 7) ^ (rb >> 1)) & 7;
+    const bool gated = act_gated(a.act);
+#pragma unroll
+    for (int i = 0; i < MB; ++i) {
+        const int r = i * 32 + rb;
+        vx[i] = (uint32_t)(((size_t)(order[r < rows ? r : rows - 1] / a.per_row) * a.ldx + chunk * 8) * sizeof(T));
+    }
+#pragma unroll
+    for (int i = 0; i < NB; ++i) vw[i] = (uint32_t)(((size_t)weight_row<NB>(i, rb, n0, a.N, gated) * a.ldw + chunk * 8) * sizeof(T));
+    f32x4 acc[NB][MB];
+    product4<T, MB, NB>(acc, smem, rsX, rsW, vx, vw, 0, a.K >> 6, rows > 32 * SH::MB0, tid);
+    GemmArgs e{};
+    e.C = a.C; e.ldc = a.ldc; e.M = rows; e.N = a.N; e.act = a.act;
+    epilogue4<T, MB, NB>(e, acc, 0, n0, wm, wn, lane, [&](int m) { return slots[m]; });
+}
+
+template <typename T, int MB, int NB>
+void group_gemm4w_launch(const GroupGemmArgs& a, int m_tiles, hipStream_t st) {
+    using SH = Shape4w<MB, NB>;
+    auto kern = group_gemm4w_kernel<T, MB, NB>;
+    static std::once_flag once;
+    std::call_once(once, [&] { LMX_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, SH::LDS)); });
+    LMX_LAUNCH(kern, dim3(m_tiles * cdiv(a.N, SH::BN)), dim3(256), SH::LDS, st, a);
+    LMX_CHECK_HIP(hipGetLastError());
 }
 
 // sum of the slices in slice order + epilogue, in row order through LDS: workgroup (tile, j) makes rows 32 j .. + 31 of the tile
@@ -746,7 +809,9 @@ void gemm4w_launch(GemmArgs a, int S, hipStream_t st) {
 // the tile forms, in the order of gemm4w.hip's table; each dtype's in two source files
 #define LMX_GEMM4W_LARGE(X, T) X(T, 8, 8) X(T, 7, 8) X(T, 7, 7) X(T, 8, 6)
 #define LMX_GEMM4W_SMALL(X, T) X(T, 5, 8) X(T, 6, 6) X(T, 5, 6) X(T, 5, 4) X(T, 4, 5) X(T, 4, 4)
-#define LMX_GEMM4W_EXTERN(T, MB, NB) extern template void gemm4w_launch<T, MB, NB>(GemmArgs, int, hipStream_t);
-#define LMX_GEMM4W_INST(T, MB, NB) template void gemm4w_launch<T, MB, NB>(GemmArgs, int, hipStream_t);
+#define LMX_GEMM4W_EXTERN(T, MB, NB) extern template void gemm4w_launch<T, MB, NB>(GemmArgs, int, hipStream_t); \
+                                     extern template void group_gemm4w_launch<T, MB, NB>(const GroupGemmArgs&, int, hipStream_t);
+#define LMX_GEMM4W_INST(T, MB, NB) template void gemm4w_launch<T, MB, NB>(GemmArgs, int, hipStream_t); \
+                                   template void group_gemm4w_launch<T, MB, NB>(const GroupGemmArgs&, int, hipStream_t);
 
 }  // namespace lmx

@@ -22,15 +22,19 @@ constexpr Tile kTiles[] = {LMX_GEMM4W_LARGE(LMX_GEMM4W_TILE, ) LMX_GEMM4W_SMALL(
 //   a K-step:  0.24 us + 0.0129 a block of the tile + 0.0066 a block of its sides
 //   a round that leaves CUs idle has their power: its K-steps take 0.76 + 0.24 x (the share of CUs at work) of that
 //   an epilogue: 0.2 us a block, more with gating or an activation; a slice's plain stores half of that, then the reduction's launch and its reads
-float cost(const GemmArgs& a, int mb, int nb, int S) {
-    const int tiles = cdiv(a.M, 32 * mb) * cdiv(a.N, 32 * nb) * S, n = cdiv(a.K / 64, S), area = mb * nb;
+float rounds(int tiles, int n, int act, int mb, int nb, bool slices) {
+    const int area = mb * nb;
     const float steps = n * (0.24f + 0.0129f * area + 0.0066f * (mb + nb));
-    const float epi = S > 1 ? 0.108f * area - 0.5f : (act_gated(a.act) ? 0.34f : a.act != kActNone ? 0.64f : 0.215f) * area - 2.2f;
+    const float epi = slices ? 0.108f * area - 0.5f : (act_gated(act) ? 0.34f : act != kActNone ? 0.64f : 0.215f) * area - 2.2f;
     float t = (tiles / 256) * (steps + epi);
     if (const int rem = tiles % 256) {
         const float share = rem / 256.f;
         t += steps * (0.76f + 0.24f * share) + epi * std::max(0.5f, share);
     }
+    return t;
+}
+float cost(const GemmArgs& a, int mb, int nb, int S) {
+    float t = rounds(cdiv(a.M, 32 * mb) * cdiv(a.N, 32 * nb) * S, cdiv(a.K / 64, S), a.act, mb, nb, S > 1);
     if (S > 1) t += 3.8f + 1.17e-6f * S * a.M * a.N;
     return t;
 }
@@ -52,7 +56,57 @@ template <typename T> void launch_t(const GemmArgs& a, const TileForm& f, hipStr
     }
 }
 
+// A grouped product on tiles of mb x nb blocks.  The host does not know the groups' rows: the mean over loads around the average.  Over 75 .. 670 rows a group of two
+// mixtures (16 groups, 2816 x 2048 and 2048 x 1408, 5504 x 4096 and 4096 x 2752, rows spread at random) the tile this picks is 2.5 % behind the best one in the mean
+float group_cost(const GroupGemmArgs& a, int mb, int nb) {
+    const float avg = (float)a.rows / a.groups;
+    float t = 0.f;
+    for (const float load : {0.85f, 0.92f, 1.f, 1.08f, 1.15f}) {
+        const int m_tiles = a.groups * std::max(1, cdiv((int)(avg * load), 32 * mb));
+        t += 0.2f * rounds(m_tiles * cdiv(a.N, 32 * nb), a.K / 64, a.act, mb, nb, false);
+    }
+    return t;
+}
+int group_nb(const GroupGemmArgs& a, int mb, float* least) {
+    int best = 0;
+    for (const Tile& t : kTiles) {
+        if (t.mb != mb) continue;
+        const float c = group_cost(a, mb, t.nb);
+        if (!best || c < *least) { best = t.nb; *least = c; }
+    }
+    return best;
+}
+template <typename T> void launch_group_t(const GroupGemmArgs& a, int mb, int nb, int m_tiles, hipStream_t st) {
+#define LMX_GROUP4W_CASE(T_, MB, NB) case MB * 16 + NB: group_gemm4w_launch<T_, MB, NB>(a, m_tiles, st); return;
+    switch (mb * 16 + nb) {
+        LMX_GEMM4W_LARGE(LMX_GROUP4W_CASE, T)
+        LMX_GEMM4W_SMALL(LMX_GROUP4W_CASE, T)
+        default: throw Error{"group_gemm: no such tile"};
+    }
+}
+
 }  // namespace
+
+bool group_gemm4w_applies(const GroupGemmArgs& a) {
+    return a.plan.n_tiles && a.rows % a.per_row == 0 && (size_t)(a.rows / a.per_row) * a.ldx * 2 < ((size_t)1 << 32) && (size_t)a.N * a.ldw * 2 < ((size_t)1 << 32);
+}
+int group_gemm4w_bm(const GroupGemmArgs* a, int n) {
+    int best = 0;
+    float least = 0.f;
+    for (int mb = 4; mb <= 8; ++mb) {
+        float sum = 0.f, c = 0.f;
+        for (int i = 0; i < n; ++i) { group_nb(a[i], mb, &c); sum += c; }
+        if (!best || sum < least) { best = mb; least = sum; }
+    }
+    return 32 * best;
+}
+void launch_group_gemm4w(int dtype, const GroupGemmArgs& a, int bm, int nb, int m_tiles, hipStream_t st) {
+    LMX_REQUIRE(bm % 32 == 0 && bm >= 128 && bm <= 256 && group_gemm4w_applies(a), "group_gemm: bad tiles");
+    float c = 0.f;
+    if (nb == 0) nb = group_nb(a, bm / 32, &c);
+    if (dtype == kBF16) launch_group_t<bf16_t>(a, bm / 32, nb, m_tiles, st);
+    else launch_group_t<f16_t>(a, bm / 32, nb, m_tiles, st);
+}
 
 // what the slices of a product may need at most: the scratch of any tile form (and of 256 x 256 tiles, which callers size theirs by)
 size_t gemm4w_slab_bytes(int M, int N, const TileForm& f) {

@@ -310,7 +310,6 @@ struct GroupTile { int group, row0, rows, first, n_tiles; int pad[3]; };      //
 struct GroupPlan { int* order = nullptr; GroupTile* tiles = nullptr; int* n_tiles = nullptr; };
 size_t group_plan_bytes(int slots);
 GroupPlan group_plan_at(void* base, int slots);
-int group_gemm_bm(int slots, int groups);                        // rows of a tile
 bool group_gemm_applies(int dtype, int slots, int groups);
 void launch_group_plan(const int* ids, int slots, int groups, int bm, const GroupPlan& p, hipStream_t st);
 struct GroupGemmArgs {
@@ -320,7 +319,12 @@ struct GroupGemmArgs {
     int x_group = 0, c_group = 0, act = 0, per_row = 1;
     GroupPlan plan{};
 };
-void launch_group_gemm(int dtype, const GroupGemmArgs& a, int bm, hipStream_t st);
+void launch_group_gemm(int dtype, const GroupGemmArgs& a, int bm, hipStream_t st, int nb = 0);
+int group_gemm_bm(const GroupGemmArgs* a, int n);                // rows of a tile for n products over one plan
+// the four-wave form (gemm4w.hip): tiles of 128, 160 .. 256 rows
+bool group_gemm4w_applies(const GroupGemmArgs& a);
+int group_gemm4w_bm(const GroupGemmArgs* a, int n);
+void launch_group_gemm4w(int dtype, const GroupGemmArgs& a, int bm, int nb, int m_tiles, hipStream_t st);      // nb: column blocks, 0 = the cheapest
 struct MoeRouterArgs { const void* x; const void* w; const void* bias; int ldx, K, E, top; int* ids; float* wt; };      // ids / wt [rows][top]: the largest logits and their softmax
 void launch_moe_router(int dtype, const MoeRouterArgs& a, int rows, hipStream_t st);
 

@@ -2,7 +2,7 @@
 //
 //   moe_router_kernel    fp32 router logits, the `top` largest and the softmax over them
 //   group_plan_kernel    rows of every expert side by side, cut into tiles
-//   group_gemm_kernel    the rows of a group times its weight on MFMA tiles (16-bit)
+//   group_gemm_kernel    the rows of a group times its weight on MFMA tiles (16-bit), groups of up to 64 rows (more of them: gemm4w.h)
 //   group_gemv_kernel    one row through the weight of its group (an expert, or a head), weights streamed straight into the vector ALUs
 #include <algorithm>
 
@@ -107,10 +107,15 @@ GroupPlan group_plan_at(void* base, int slots) {
     char* p = static_cast<char*>(base);
     return GroupPlan{reinterpret_cast<int*>(p + 256), reinterpret_cast<GroupTile*>(p + 256 + ((size_t)slots * 4 + 255) / 256 * 256), reinterpret_cast<int*>(p)};
 }
-// rows of a tile: what an average group fills
-int group_gemm_bm(int slots, int groups) {
-    const int avg = slots / groups;
-    return avg <= 24 ? 32 : avg <= 96 ? 64 : avg <= 160 ? 128 : 256;
+// Rows of a tile.  From 65 rows a group on the four-wave tiles (gemm4w.h) that make the cheapest rounds; below them 32 or 64 rows, what an average group fills.  us of both
+// products of a mixture of 16, tiles of 64 rows (or, the best before, 128 and 256 rows of eight waves and a ring of two) / four-wave tiles:
+//   2048 wide, experts of 1408: 50 rows a group 51 / 50   75: 62 / 51   130: 75 / 55   250: 103 / 81   385: 157 / 111   670: 239 / 184
+//   4096 wide, experts of 2752: 50 rows a group 215 / 212   75: 264 / 229   130: 316 / 249   250: 399 / 322   385: 516 / 384   670: 787 / 618
+int group_gemm_bm(const GroupGemmArgs* a, int n) {
+    const int avg = a->rows / a->groups;
+    bool four = avg > 64;
+    for (int i = 0; i < n; ++i) four = four && group_gemm4w_applies(a[i]);
+    return four ? group_gemm4w_bm(a, n) : avg <= 24 ? 32 : 64;
 }
 bool group_gemm_applies(int dtype, int slots, int groups) { return dtype != kF32 && slots >= 16 && slots >= groups; }
 void launch_group_plan(const int* ids, int slots, int E, int bm, const GroupPlan& p, hipStream_t st) {
@@ -238,15 +243,15 @@ static void launch_group_gemm_cfg(const GroupGemmArgs& a, int m_tiles, hipStream
     LMX_LAUNCH(kern, dim3(m_tiles * cdiv(a.N, BN)), dim3(WM * WN * 64), smem, st, a);
     LMX_CHECK_HIP(hipGetLastError());
 }
-void launch_group_gemm(int dtype, const GroupGemmArgs& a, int bm, hipStream_t st) {
+void launch_group_gemm(int dtype, const GroupGemmArgs& a, int bm, hipStream_t st, int nb) {
     LMX_REQUIRE(a.X && a.W && a.C && a.rows >= 1 && a.groups >= 1 && a.N >= 1 && a.K >= 64 && a.K % 64 == 0 && a.per_row >= 1, "group_gemm: bad arguments");
     LMX_REQUIRE(a.ldx % 8 == 0 && a.ldw % 8 == 0 && a.ldc % 4 == 0 && a.w_group % 8 == 0 && a.x_group % 8 == 0 && a.c_group % 4 == 0 && a.N % 4 == 0, "group_gemm: 16-byte rows");
     LMX_REQUIRE(!act_gated(a.act) || a.N % 64 == 0, "group_gemm: gated rows come in groups of 64");
     // with a plan: every group's last tile may be part empty; no more tiles than rows
     const int m_tiles = a.plan.n_tiles ? std::min(a.rows, a.rows / bm + a.groups) : a.groups * cdiv(a.rows, bm);
 #define L(TT) do { if (bm == 32) launch_group_gemm_cfg<TT, 32, 128, 1, 2, 4>(a, m_tiles, st); else if (bm == 64) launch_group_gemm_cfg<TT, 64, 128, 2, 2, 3>(a, m_tiles, st); \
-                   else if (bm == 128) launch_group_gemm_cfg<TT, 128, 128, 2, 2, 2>(a, m_tiles, st); else if (bm == 256) launch_group_gemm_cfg<TT, 256, 256, 2, 4, 2>(a, m_tiles, st); \
-                   else throw Error{"group_gemm: tiles of 32, 64, 128 or 256 rows"}; } while (0)
+                   else throw Error{"group_gemm: tiles of 32, 64 or 128 .. 256 rows"}; } while (0)
+    if (bm > 64 && dtype != kF32) { launch_group_gemm4w(dtype, a, bm, nb, m_tiles, st); return; }
     if (dtype == kBF16) L(bf16_t); else if (dtype == kF16) L(f16_t); else throw Error{"group_gemm: 16-bit models"};
 #undef L
 }

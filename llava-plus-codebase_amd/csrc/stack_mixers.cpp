@@ -185,15 +185,13 @@ void Model::stack_moe(const StackLayer& l, const void* x, int rows, const StackW
     const int dt = cfg.dtype, top = l.c.top_experts, E = l.c.experts, slots = rows * top;
     { LMX_PROF_K(pn.router); launch_moe_router(dt, MoeRouterArgs{x, l.wr, l.br, H, H, E, top, w.ids, w.wt}, rows, st); }
     if (group_gemm_applies(dt, slots, E)) {
-        const int bm = group_gemm_bm(slots, E);
-        const GroupPlan plan = group_plan_at(w.plan, slots);
-        { LMX_PROF_K(pn.plan); launch_group_plan(w.ids, slots, E, bm, plan, st); }
-        GroupGemmArgs g{x, l.wgu, w.act, 2 * l.ff, H, H, H, l.ff, (size_t)2 * l.ff * H, slots, E};
-        g.act = l.act(); g.per_row = top; g.plan = plan;
-        { LMX_PROF_K(pn.gate_up); launch_group_gemm(dt, g, bm, st); }
-        GroupGemmArgs o{w.act, l.wd, w.slots, H, l.ff, l.ff, l.ff, H, (size_t)H * l.ff, slots, E};
-        o.plan = plan;
-        { LMX_PROF_K(pn.down); launch_group_gemm(dt, o, bm, st); }
+        GroupGemmArgs p[2] = {{x, l.wgu, w.act, 2 * l.ff, H, H, H, l.ff, (size_t)2 * l.ff * H, slots, E}, {w.act, l.wd, w.slots, H, l.ff, l.ff, l.ff, H, (size_t)H * l.ff, slots, E}};
+        p[0].act = l.act(); p[0].per_row = top;
+        p[0].plan = p[1].plan = group_plan_at(w.plan, slots);
+        const int bm = group_gemm_bm(p, 2);
+        { LMX_PROF_K(pn.plan); launch_group_plan(w.ids, slots, E, bm, p[0].plan, st); }
+        { LMX_PROF_K(pn.gate_up); launch_group_gemm(dt, p[0], bm, st); }
+        { LMX_PROF_K(pn.down); launch_group_gemm(dt, p[1], bm, st); }
         return;
     }
     GroupGemvArgs g{x, l.wgu, w.act, 2 * l.ff, H, H, H, l.ff, (size_t)2 * l.ff * H};

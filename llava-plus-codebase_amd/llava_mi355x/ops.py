@@ -63,6 +63,19 @@ def gemv(x, w, bias=None, residual=None, norm_w=None, eps=1e-5, act=_C.ACT_NONE,
     return out
 
 
+def group_gemm(x, w, ids, act=_C.ACT_NONE, shared_x=True, bm=0, nb=0):
+    """act(x_row @ w[ids[row, j]].T) per slot (row, j), [rows * per_row, N]; x has a row per slot unless shared_x.  Gated w rows as in gemm."""
+    _need_cuda(x, w, ids)
+    rows, per_row = ids.shape
+    groups, N, K = w.shape
+    assert ids.dtype == torch.int32 and x.is_contiguous() and w.is_contiguous() and ids.is_contiguous() and x.shape == (rows if shared_x else rows * per_row, K)
+    out = torch.empty((rows * per_row, N // 2 if act in (_C.ACT_SILU_MUL, _C.ACT_RELU_MUL) else N), dtype=x.dtype, device=x.device)
+    plan = torch.empty(lib.lmx_op_group_plan_bytes(rows, per_row), dtype=torch.uint8, device=x.device)
+    check(lib.lmx_op_group_gemm(torch_dtype_code(x.dtype), ptr(x), ptr(w), ptr(out), ptr(ids), rows, per_row, groups, int(shared_x), N, K, act, bm, nb, ptr(plan), stream_handle()),
+          "group_gemm")
+    return out
+
+
 def rmsnorm(x, w, eps):
     _need_cuda(x, w)
     y = torch.empty_like(x)

@@ -260,7 +260,7 @@ void launch_group_gemm(int dtype, const GroupGemmArgs& a, int bm, hipStream_t st
 // grid (slots, ceil(outputs / outputs per workgroup)), 256 threads.  `lpr` lanes own one weight row (a power of two with 8 lpr <= K): short rows leave no lane idle.
 // Gated: a lane group takes the gate row and the up row of its output.
 // ---------------------------------------------------------------------------------------------------------------
-template <typename T>
+template <typename T, bool GATED>
 __global__ __launch_bounds__(256) void group_gemv_kernel(GroupGemvArgs a, int lpr, int opw) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     T* xs = reinterpret_cast<T*>(smem);
@@ -270,29 +270,45 @@ __global__ __launch_bounds__(256) void group_gemv_kernel(GroupGemvArgs a, int lp
     const T* x = reinterpret_cast<const T*>(a.X) + xr * a.ldx + (a.ids ? 0 : grp * a.x_group);
     const T* W = reinterpret_cast<const T*>(a.W) + (size_t)grp * a.w_group;
     T* C = reinterpret_cast<T*>(a.C) + cr * a.ldc + (a.ids ? 0 : grp * a.c_group);
-    for (int c = tid * 8; c < a.K; c += 2048) { float v[8]; load8<T>(x + c, v); store8<T>(xs + c, v); }
-    __syncthreads();
-    const bool gated = act_gated(a.act);
-    const int outs = gated ? a.N / 2 : a.N, sub = tid % lpr, per = 256 / lpr;
+    const int outs = GATED ? a.N / 2 : a.N, sub = tid % lpr, per = 256 / lpr;
     const int o0 = blockIdx.y * opw, o1 = o0 + opw < outs ? o0 + opw : outs;
+    // U pieces of a row (both rows, gated) are on their way together, the first ones ahead of the staging of x: piece by piece a row of 2048 was four memory latencies.  Pieces
+    // past the row's end re-read its first one and count as zeros.  (us a launch, four slots: 2 x 1408 rows of 2048 12.2 -> 11.6, 2048 rows of 1408 8.1 -> 6.7)
+    constexpr int U = 4;
+    Chunk8<T> g[U], u[GATED ? U : 1];
+    const int step = U * lpr * 8;
     for (int ob = o0; ob < o1; ob += per) {                  // every lane stays: the sums run over whole lane groups
         const int o = ob + tid / lpr, oc = o < o1 ? o : o1 - 1;
-        const int r0 = gated ? 64 * (oc >> 5) + (oc & 31) : oc;
-        const T* w0 = W + (size_t)r0 * a.ldw;
+        const T* w0 = W + (size_t)(GATED ? 64 * (oc >> 5) + (oc & 31) : oc) * a.ldw;
         const T* w1 = w0 + (size_t)32 * a.ldw;
         float s0 = 0.f, s1 = 0.f;
-        for (int c = sub * 8; c < a.K; c += lpr * 8) {
-            float v[8], f[8]; load8<T>(xs + c, v); load8<T>(w0 + c, f);
+        for (int cb = 0; cb < a.K; cb += step) {
 #pragma unroll
-            for (int i = 0; i < 8; ++i) s0 = fmaf(f[i], v[i], s0);
-            if (gated) {
-                load8<T>(w1 + c, f);
+            for (int k = 0; k < U; ++k) {
+                int c = cb + sub * 8 + k * lpr * 8; c = c < a.K ? c : 0;
+                g[k].load(w0 + c);
+                if (GATED) u[k].load(w1 + c);
+            }
+            if (ob == o0 && cb == 0) {
+                for (int c = tid * 8; c < a.K; c += 2048) { Chunk8<T> v; v.load(x + c); *reinterpret_cast<Chunk8<T>*>(xs + c) = v; }
+                __syncthreads();
+            }
 #pragma unroll
-                for (int i = 0; i < 8; ++i) s1 = fmaf(f[i], v[i], s1);
+            for (int k = 0; k < U; ++k) {
+                const int c = cb + sub * 8 + k * lpr * 8;
+                const bool in = c < a.K;
+                float v[8], f[8]; load8<T>(xs + (in ? c : 0), v); g[k].get(f);
+#pragma unroll
+                for (int i = 0; i < 8; ++i) s0 = in ? fmaf(f[i], v[i], s0) : s0;
+                if (GATED) {
+                    u[k].get(f);
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) s1 = in ? fmaf(f[i], v[i], s1) : s1;
+                }
             }
         }
-        for (int d = lpr >> 1; d > 0; d >>= 1) { s0 += __shfl_xor(s0, d, 64); if (gated) s1 += __shfl_xor(s1, d, 64); }
-        if (sub == 0 && o < o1) C[o] = from_f32<T>(gated ? gate_mul(a.act, s0, s1) : s0);
+        for (int d = lpr >> 1; d > 0; d >>= 1) { s0 += __shfl_xor(s0, d, 64); if (GATED) s1 += __shfl_xor(s1, d, 64); }
+        if (sub == 0 && o < o1) C[o] = from_f32<T>(GATED ? gate_mul(a.act, s0, s1) : s0);
     }
 }
 
@@ -307,7 +323,8 @@ void launch_group_gemv(int dtype, const GroupGemvArgs& a, int slots, hipStream_t
     int opw = per;                                           // outputs of a workgroup: more of them while the grid stays large enough
     while (opw < 64 && (long)slots * cdiv(outs, opw * 2) >= 1024) opw *= 2;
     const dim3 grid(slots, cdiv(outs, opw));
-#define L(TT) LMX_LAUNCH(group_gemv_kernel<TT>, grid, dim3(256), (size_t)a.K * sizeof(TT), st, a, lpr, opw)
+#define L(TT) do { if (act_gated(a.act)) LMX_LAUNCH((group_gemv_kernel<TT, true>), grid, dim3(256), (size_t)a.K * sizeof(TT), st, a, lpr, opw); \
+                   else LMX_LAUNCH((group_gemv_kernel<TT, false>), grid, dim3(256), (size_t)a.K * sizeof(TT), st, a, lpr, opw); } while (0)
     if (dtype == kBF16) L(bf16_t); else if (dtype == kF16) L(f16_t); else L(float);
 #undef L
     LMX_CHECK_HIP(hipGetLastError());

@@ -21,6 +21,7 @@
 
 #include "common.h"
 #include "kernels.h"
+#include "moe_pick.h"
 
 namespace lmx {
 
@@ -424,6 +425,7 @@ void launch_delta_gate(int dtype, const DeltaPrefillArgs& a, hipStream_t st) {
 template <typename T, int LPC, int NTH>
 __global__ __launch_bounds__(NTH, NTH == 512 && sizeof(T) == 2 ? 4 : 1) void delta_decode_kernel(DeltaDecodeArgs a) {
     constexpr int DK = LPC * 8, CPP = NTH / LPC, PF = 2048 / NTH, RP = 2048 / NTH;      // columns of one pass over the state, passes in flight, low-rank rows at a time
+    if ((int)blockIdx.x == a.s.H) { moe_router_row<T, NTH / 64>(a.router, blockIdx.y); return; }
     extern __shared__ __attribute__((aligned(16))) float sm[];
     __shared__ float red[NTH / 64];
     const int tid = threadIdx.x;
@@ -596,12 +598,16 @@ __global__ __launch_bounds__(NTH, NTH == 512 && sizeof(T) == 2 ? 4 : 1) void del
     for (int c = tid; c < DV; c += NTH) out[c] = from_f32<T>(o[c] * inv * to_f32(c == tid ? norm_w : reinterpret_cast<const T*>(a.w.norm)[c]) * gate[c]);
 }
 
+static bool one_round(const DeltaShape& s, int n_seq) { return s.H * n_seq <= 256; }
+// past one round the routers are a tail of their own: 32 x 32 heads x sequences 39.1 us without, 50.4 with them, 9.8 alone; in one round (16 x 1) 9.9 either way, 8.1 alone
+bool delta_decode_routes(const DeltaShape& s, int n_seq) { return one_round(s, n_seq); }
 void launch_delta_decode(int dtype, const DeltaDecodeArgs& a, hipStream_t st) {
     delta_check(a.s);
     LMX_REQUIRE(a.ra % 64 == 0 && a.rg % 64 == 0 && a.ra >= 64 && a.rg >= 64 && a.wag_ld >= a.ra + a.rg && a.wag_ld % 8 == 0, "delta_decode: low-rank widths in whole 64-column groups");
     LMX_REQUIRE(a.a_off >= a.s.channels() + a.s.H && a.ld >= a.a_off + a.ra + a.rg, "delta_decode: bad row pitch");
     LMX_REQUIRE(a.n_seq >= 1 && (a.tab || (a.n_seq == 1 && a.one.K && a.one.VT && a.one.pos_ptr)), "delta_decode: bad sequence");
-    const dim3 grid(a.s.H, a.n_seq);
+    check_router(a.router);
+    const dim3 grid(a.s.H + (a.router.x ? 1 : 0), a.n_seq);
     const size_t smem = (size_t)(3 * a.s.DK + 3 * a.s.DV) * 4;
     LMX_REQUIRE(smem <= 60 * 1024 && a.a_off % 8 == 0, "delta_decode: head widths too large");
 #define L(TT, NTH) do { if (a.s.DK == 64) LMX_LAUNCH((delta_decode_kernel<TT, 8, NTH>), grid, dim3(NTH), smem, st, a); \
@@ -610,7 +616,8 @@ void launch_delta_decode(int dtype, const DeltaDecodeArgs& a, hipStream_t st) {
 #define LN(TT) do { if (wide) L(TT, 1024); else L(TT, 512); } while (0)
     // 1024 threads a head while every workgroup has a CU of its own; past that two workgroups of 512 on a CU, whose reads and arithmetic overlap.  us at 16 x 16 / 16 x 24 /
     // 32 x 32 heads x sequences: 1024 threads 13.8 / 22.5 / 45.4, 512 threads 15.9 / 20.0 / 40.5
-    const bool wide = a.s.H * a.n_seq <= 256;
+    const bool wide = one_round(a.s, a.n_seq);
+    LMX_REQUIRE(wide || !a.router.x, "delta_decode: no router here");
     if (dtype == kBF16) LN(bf16_t); else if (dtype == kF16) LN(f16_t); else LN(float);
 #undef LN
 #undef L

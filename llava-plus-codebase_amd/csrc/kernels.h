@@ -243,6 +243,7 @@ WinForm decode_win_form(int dtype, int D, int n_heads, int n_kv_heads, int n_seq
 // Projection rows of a layer: q [G][DK] | k [G][DK] | v [H][DV] | beta [H] | ...; DK in {64, 128, 256} and DV (a multiple of 64) are padded head widths, the padding is
 // zero.  q, k, v pass a causal convolution of `taps` inputs per channel and silu; q and k are unit vectors; the decay is one per head and key channel.
 // State of a sequence and layer run: S transposed, [H][DV][DK] floats, and a ring of the last `taps` projection rows (row of position p at p % taps), [taps][channels].
+struct MoeRouterArgs { const void* x; const void* w; const void* bias; int ldx, K, E, top; int* ids; float* wt; };      // ids / wt [rows][top]: the largest logits and their softmax
 struct DeltaShape {
     int H = 0, G = 0, DK = 0, DV = 0, dk = 0, dv = 0, taps = 1;      // heads, key heads, padded and true widths
     __host__ __device__ int channels() const { return 2 * G * DK + H * DV; }
@@ -274,7 +275,9 @@ struct DeltaDecodeArgs {                 // one new token per sequence, everythi
     const DecodeFusedSeq* tab = nullptr; DecodeFusedSeq one{};      // K = state, VT = ring
     int n_seq = 1;
     float eps;
+    MoeRouterArgs router{};              // x set: a parallel layer's mixture chooses its experts in the same launch (where delta_decode_routes)
 };
+bool delta_decode_routes(const DeltaShape& s, int n_seq);
 void launch_delta_decode(int dtype, const DeltaDecodeArgs& a, hipStream_t st);
 
 // ---- latent attention (latent.hip): keys and values are linear in a normalised latent row, the only thing that is cached: [s_max][R] ---------------------------------
@@ -291,8 +294,10 @@ struct LatentDecodeArgs {                // queries already in the latent space,
     const DecodeFusedSeq* tab = nullptr; DecodeFusedSeq one{};
     int n_seq = 1, H = 0, R = 0, s_max = 0, n_split = 1, window = 0;
     float scale = 1.f;
+    MoeRouterArgs router{};              // as DeltaDecodeArgs; where latent_decode_routes
 };
 void launch_latent_decode(int dtype, const LatentDecodeArgs& a, hipStream_t st);
+bool latent_decode_routes(int dtype, int R);
 int latent_decode_split(int dtype, int R, int H, int n_seq, int span);      // n_split for a context of `span` keys
 
 // ---- grouped linears and mixtures of experts (moe.hip) -----------------------------------------------------------------------------------------------------------
@@ -325,7 +330,6 @@ int group_gemm_bm(const GroupGemmArgs* a, int n);                // rows of a ti
 bool group_gemm4w_applies(const GroupGemmArgs& a);
 int group_gemm4w_bm(const GroupGemmArgs* a, int n);
 void launch_group_gemm4w(int dtype, const GroupGemmArgs& a, int bm, int nb, int m_tiles, hipStream_t st);      // nb: column blocks, 0 = the cheapest
-struct MoeRouterArgs { const void* x; const void* w; const void* bias; int ldx, K, E, top; int* ids; float* wt; };      // ids / wt [rows][top]: the largest logits and their softmax
 void launch_moe_router(int dtype, const MoeRouterArgs& a, int rows, hipStream_t st);
 
 // ---- decode-step attention of a single request (decode_attn.hip; 16-bit models) ---------------------------------------------------------------------

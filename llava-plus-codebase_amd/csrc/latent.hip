@@ -10,6 +10,7 @@
 
 #include "common.h"
 #include "kernels.h"
+#include "moe_pick.h"
 #include "attention_decode.h"
 
 namespace lmx {
@@ -178,6 +179,10 @@ template <> __device__ __forceinline__ f32x4 mfma16<f16_t>(const uint4& a, const
 template <typename T, int R>
 __global__ __launch_bounds__(256, 1) void latent_mfma_kernel(LatentDecodeArgs a) {
     static_assert(R <= 512, "one column block per wave");
+    if ((int)blockIdx.y * 16 >= a.H) {                       // the last row of workgroups: a router
+        if (blockIdx.x == 0) moe_router_row<T, 4>(a.router, blockIdx.z);
+        return;
+    }
     constexpr int KT = 128, PITCH = KT + 4, NQ = R / 32;
     __shared__ __attribute__((aligned(16))) float ss[2][16][PITCH];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -302,6 +307,7 @@ __global__ __launch_bounds__(R / 4) void latent_merge_kernel(LatentDecodeArgs a)
 
 // workgroups along a context of `span` keys: enough of them to fill the chip, no more
 static bool latent_mfma(int dtype, int R) { return dtype != kF32 && R >= 128; }
+bool latent_decode_routes(int dtype, int R) { return latent_mfma(dtype, R); }
 int latent_decode_split(int dtype, int R, int H, int n_seq, int span) {
     const bool mf = latent_mfma(dtype, R);
     const int wgs = mf ? cdiv(H, 16) * n_seq : H * n_seq;
@@ -313,7 +319,8 @@ void launch_latent_decode(int dtype, const LatentDecodeArgs& a, hipStream_t st) 
     LMX_REQUIRE(a.H >= 1 && a.n_split >= 1 && a.n_split <= DF_MAX_SPLIT && a.n_seq >= 1 && a.q && a.out && a.s_max >= 1, "latent_decode: bad arguments");
     LMX_REQUIRE(a.tab || (a.n_seq == 1 && a.one.K && a.one.pos_ptr && a.one.ws && a.one.counters), "latent_decode: bad sequence");
     if (latent_mfma(dtype, a.R)) {
-        const dim3 grid(a.n_split, cdiv(a.H, 16), a.n_seq);
+        check_router(a.router);
+        const dim3 grid(a.n_split, cdiv(a.H, 16) + (a.router.x ? 1 : 0), a.n_seq);
 #define M1(TT, RR) do { LMX_LAUNCH((latent_mfma_kernel<TT, RR>), grid, dim3(256), 0, st, a); if (a.n_split > 1) LMX_LAUNCH((latent_merge_kernel<TT, RR>), dim3(a.H, a.n_seq), dim3(RR / 4), 0, st, a); } while (0)
 #define M(TT) do { if (a.R == 128) M1(TT, 128); else if (a.R == 256) M1(TT, 256); else M1(TT, 512); } while (0)
         if (dtype == kBF16) M(bf16_t); else M(f16_t);
@@ -322,6 +329,7 @@ void launch_latent_decode(int dtype, const LatentDecodeArgs& a, hipStream_t st) 
         LMX_CHECK_HIP(hipGetLastError());
         return;
     }
+    LMX_REQUIRE(!a.router.x, "latent_decode: no router here");
     const dim3 grid(a.H, a.n_split, a.n_seq);
 #define L(TT, KK) LMX_LAUNCH((latent_decode_kernel<TT, KK>), grid, dim3(256), 0, st, a)
 #define LR(TT) do { if (a.R == 64) L(TT, 8); else if (a.R == 128) L(TT, 16); else if (a.R == 256) L(TT, 32); else L(TT, 64); } while (0)

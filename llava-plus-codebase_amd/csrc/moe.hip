@@ -9,62 +9,17 @@
 #include "common.h"
 #include "kernels.h"
 #include "gemm_common.h"
+#include "moe_pick.h"
 
 namespace lmx {
 
-constexpr int MOE_MAX_E = 256, MOE_MAX_TOP = 32;
-
-// the `top` largest of z[0, E) (lowest index first among equals) and their softmax, by one wave: an expert's place is the number of experts ahead of it.
-// z is padded with -inf to a multiple of 4
-__device__ __forceinline__ void pick_top(const float* z, int E, int top, int lane, int* place, int* ids, float* wt) {
-    float v[MOE_MAX_E / 64]; int rank[MOE_MAX_E / 64];
-    if (lane < top) place[lane] = lane;                      // only non-finite logits leave a place empty
-#pragma unroll
-    for (int i = 0; i < MOE_MAX_E / 64; ++i) { v[i] = lane + 64 * i < E ? z[lane + 64 * i] : -INFINITY; rank[i] = 0; }
-    for (int j = 0; j < E; j += 4) {
-        const float4 q = *reinterpret_cast<const float4*>(z + j);
-        const float o[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-        for (int n = 0; n < 4; ++n)
-#pragma unroll
-            for (int i = 0; i < MOE_MAX_E / 64; ++i) rank[i] += o[n] > v[i] || (o[n] == v[i] && j + n < lane + 64 * i);
-    }
-#pragma unroll
-    for (int i = 0; i < MOE_MAX_E / 64; ++i) if (lane + 64 * i < E && rank[i] < top) place[rank[i]] = lane + 64 * i;
-    __builtin_amdgcn_wave_barrier();
-    const int id = lane < top ? place[lane] : 0;
-    const float e = lane < top ? expf(z[id] - z[place[0]]) : 0.f;
-    const float sum = wave_sum(e);
-    if (lane < top) { ids[lane] = id; wt[lane] = e / sum; }
-}
-
-// grid (rows), 64 NW threads: a wave per expert at a time
+// grid (rows), 64 NW threads
 template <typename T, int NW>
-__global__ __launch_bounds__(64 * NW) void moe_router_kernel(MoeRouterArgs a) {
-    __shared__ __attribute__((aligned(16))) float z[MOE_MAX_E];
-    __shared__ int place[MOE_MAX_TOP];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const T* x = reinterpret_cast<const T*>(a.x) + (size_t)blockIdx.x * a.ldx;
-    if (tid < MOE_MAX_E && tid >= a.E) z[tid] = -INFINITY;
-    for (int e = wave; e < a.E; e += NW) {
-        const T* w = reinterpret_cast<const T*>(a.w) + (size_t)e * a.K;
-        float s = 0.f;
-#pragma unroll 4
-        for (int c = lane * 8; c < a.K; c += 512) {
-            float f[8], v[8]; load8<T>(w + c, f); load8<T>(x + c, v);
-#pragma unroll
-            for (int i = 0; i < 8; ++i) s = fmaf(f[i], v[i], s);
-        }
-        s = wave_sum(s);
-        if (lane == 0) z[e] = s + (a.bias ? to_f32(reinterpret_cast<const T*>(a.bias)[e]) : 0.f);
-    }
-    __syncthreads();
-    if (wave == 0) pick_top(z, a.E, a.top, lane, place, a.ids + (size_t)blockIdx.x * a.top, a.wt + (size_t)blockIdx.x * a.top);
-}
+__global__ __launch_bounds__(64 * NW) void moe_router_kernel(MoeRouterArgs a) { moe_router_row<T, NW>(a, blockIdx.x); }
 
 void launch_moe_router(int dtype, const MoeRouterArgs& a, int rows, hipStream_t st) {
-    LMX_REQUIRE(a.E >= 1 && a.E <= MOE_MAX_E && a.top >= 1 && a.top <= a.E && a.top <= MOE_MAX_TOP, "moe_router: 1..256 experts, at most 32 of them per row");
-    LMX_REQUIRE(a.K % 8 == 0 && a.ldx % 8 == 0 && a.x && a.w && a.ids && a.wt, "moe_router: bad arguments");
+    LMX_REQUIRE(a.x, "moe_router: bad arguments");
+    check_router(a);
     if (rows <= 0) return;
 #define L(TT) do { if (rows <= 64) LMX_LAUNCH((moe_router_kernel<TT, 16>), dim3(rows), dim3(1024), 0, st, a); else LMX_LAUNCH((moe_router_kernel<TT, 4>), dim3(rows), dim3(256), 0, st, a); } while (0)
     if (dtype == kBF16) L(bf16_t); else if (dtype == kF16) L(f16_t); else L(float);

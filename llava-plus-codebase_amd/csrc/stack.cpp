@@ -620,6 +620,7 @@ void Model::stack_decode_step(Seq* s, hipStream_t st, int64_t* id_out) {
         const GemvArgs g{nullptr, l.wqkv, s->d_qkv, l.bqkv, nullptr, nullptr, 0.f, l.qkv_n, H, H, H, l.qkv_n, 0, kActNone};
         linear("decode.gemv.qkv", before, y, top, g, !(l.parallel() && l.ff));      // a parallel layer's other linears read the same row
         top = 0;
+        bool routed = false;
         if (l.c.mixer == LMX_MIXER_ATTENTION) {
             LMX_PROF_K("decode.attn");
             bool grouped;
@@ -627,7 +628,7 @@ void Model::stack_decode_step(Seq* s, hipStream_t st, int64_t* id_out) {
             a.one = stack_seq_ref(r, s);
             a.pos = s->len;
             launch_decode_win(dt, l.D, a, grouped, st);
-        } else stack_mix_decode(r, nullptr, stack_seq_ref(r, s), 1, s->len, s->d_qkv, s->d_attn, s->sw, nullptr, st);
+        } else routed = stack_mix_decode(r, nullptr, stack_seq_ref(r, s), 1, s->len, s->d_x, s->d_qkv, s->d_attn, s->sw, nullptr, st);
         if (l.parallel() && l.dense()) plain("decode.gemv.gate_up", s->d_x, l.wgu, static_cast<char*>(s->d_attn) + (size_t)l.an * es, 2 * l.ff, H, l.act());
         plain("decode.gemv.o", s->d_attn, l.wo, s->d_y, H, l.out_k);
         y = s->d_y;
@@ -638,7 +639,7 @@ void Model::stack_decode_step(Seq* s, hipStream_t st, int64_t* id_out) {
                 plain("decode.gemv.down", s->d_act, l.wd, s->d_y, H, l.ff);
             } else { residual(sp, y, 0, false); y = nullptr; }
         }
-        if (l.moe()) { stack_moe(l, s->d_x, 1, s->sw, stack_prof_decode, st); top = l.c.top_experts; }
+        if (l.moe()) { stack_moe(l, s->d_x, 1, s->sw, stack_prof_decode, st, routed); top = l.c.top_experts; }
         before = stack_step(S, r, l.ff && !l.parallel() ? 1 : 0, final_norm);
     }
     {
@@ -690,13 +691,14 @@ void Model::stack_decode_batch_step(Batch* b, Seq* const* seqs, int n, int64_t* 
         const StackLayer& l = S.layers[(size_t)S.runs[(size_t)r].layer];
         linear(GemmArgs{b->x, l.wqkv, b->qkv, l.bqkv, nullptr, n, l.qkv_n, H, H, H, l.qkv_n, 0, kActNone}, l.sw_qkv);
         const DecodeFusedSeq* tab = b->d_attn_tab + (size_t)r * b->cap;
+        bool routed = false;
         if (l.c.mixer == LMX_MIXER_ATTENTION) {
             LMX_PROF("decode_batch.attn");
             bool grouped;
             WinDecodeArgs a = decode_args(S, l, dt, b->qkv, b->attn, n, max_len, kv_pitch, grouped);
             a.tab = tab;
             launch_decode_win(dt, l.D, a, grouped, st);
-        } else stack_mix_decode(r, tab, DecodeFusedSeq{}, n, max_len, b->qkv, b->attn, b->sw, b, st);
+        } else routed = stack_mix_decode(r, tab, DecodeFusedSeq{}, n, max_len, b->x, b->qkv, b->attn, b->sw, b, st);
         if (l.parallel() && l.dense()) linear(GemmArgs{b->x, l.wgu, static_cast<char*>(b->attn) + (size_t)l.an * es, nullptr, nullptr, n, 2 * l.ff, H, H, H, l.out_k, 0, l.act()}, l.sw_gu);
         linear(GemmArgs{b->attn, l.wo, b->y, nullptr, nullptr, n, H, l.out_k, l.out_k, l.out_k, H, 0, kActNone}, l.sw_o);
         const void* yy = b->y;
@@ -707,7 +709,7 @@ void Model::stack_decode_batch_step(Batch* b, Seq* const* seqs, int n, int64_t* 
                 linear(GemmArgs{b->act, l.wd, b->y, nullptr, nullptr, n, H, l.ff, l.ff, l.ff, H, 0, kActNone}, l.sw_d);
             } else yy = nullptr;
         }
-        if (l.moe()) stack_moe(l, b->x, n, b->sw, stack_prof_batch, st);
+        if (l.moe()) stack_moe(l, b->x, n, b->sw, stack_prof_batch, st, routed);
         norm(b->xr, yy, l.moe() ? l.c.top_experts : 0, stack_step(S, r, l.ff && !l.parallel() ? 1 : 0, final_norm));
     }
     GemmArgs ga{b->x, lm_head, b->logits, nullptr, nullptr, n, V, H, H, H, V, 0, kActNone};

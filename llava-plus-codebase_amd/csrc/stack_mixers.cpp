@@ -124,22 +124,26 @@ void Model::stack_mix_prefill(int r, Seq* const* seqs, const std::vector<Segment
 // ---------------------------------------------------------------------------------------------------------------
 // one new token per sequence
 // ---------------------------------------------------------------------------------------------------------------
-void Model::stack_mix_decode(int r, const DecodeFusedSeq* tab, const DecodeFusedSeq& one, int n, int max_len, void* qkv, void* mix, const StackWs& w, Batch* b, hipStream_t st) {
+bool Model::stack_mix_decode(int r, const DecodeFusedSeq* tab, const DecodeFusedSeq& one, int n, int max_len, const void* x, void* qkv, void* mix, const StackWs& w, Batch* b, hipStream_t st) {
     Stack& S = *stk;
     const StackLayer& l = S.layers[(size_t)S.runs[(size_t)r].layer];
     const lmx_layer_config& d = l.c;
     const int dt = cfg.dtype;
     const StackProf& pn = b ? stack_prof_batch : stack_prof_decode;
+    // a parallel layer's mixture reads the mixer's input row: its choice is one workgroup more of the mixer's longest launch.  A launch of its own takes 8 us for 64 KB of router rows
+    const MoeRouterArgs router = l.parallel() && l.moe() && opt_stack_fuse ? stack_router(l, x, w) : MoeRouterArgs{};
     if (d.mixer == LMX_MIXER_DELTA) {
         DeltaDecodeArgs a{};
         a.s = l.ds; a.w = DeltaWeights{l.conv, l.a_log, l.dt_bias, l.onorm};
         a.proj = qkv; a.ld = l.qkv_n; a.a_off = l.a_off(); a.ra = l.ra; a.rg = l.rg;
         a.wag = l.wag; a.wag_ld = l.ra + l.rg; a.out = mix; a.out_ld = l.out_k;
         a.tab = tab; a.one = one; a.n_seq = n; a.eps = S.c.norm_eps;
+        if (delta_decode_routes(l.ds, n)) a.router = router;
         LMX_PROF_K(pn.delta);
         launch_delta_decode(dt, a, st);
-        return;
+        return a.router.x;
     }
+    const bool routes = router.x && latent_decode_routes(dt, l.R);
     {
         LMX_PROF_K(pn.norm);
         LatentNormArgs a{qkv, l.qkv_n, l.Q, d.q_rank, l.R, d.kv_rank, l.qn_lat, l.kn_lat, one.K, 0};
@@ -162,11 +166,13 @@ void Model::stack_mix_decode(int r, const DecodeFusedSeq* tab, const DecodeFused
         int span = max_len + 1;
         if (d.window > 0 && d.window < span) span = d.window;
         a.n_split = latent_decode_split(dt, l.R, d.n_heads, n, span);
+        if (routes) a.router = router;
         launch_latent_decode(dt, a, st);
     }
     GroupGemvArgs o{w.olat, static_cast<char*>(l.wukv) + (size_t)l.an * l.R * es, mix, l.D, l.R, d.n_heads * l.R, l.R, l.out_k, (size_t)l.D * l.R};
     o.groups = d.n_heads; o.x_group = l.R; o.c_group = l.D;
     { LMX_PROF_K(pn.olat); stack_heads(o, n, st); }
+    return routes;
 }
 
 // every head's rows through the head's own weight
@@ -181,9 +187,10 @@ void Model::stack_heads(const GroupGemvArgs& g, int n, hipStream_t st) {
 // ---------------------------------------------------------------------------------------------------------------
 // mixture of experts: choices, then both products with the rows as they are (few: weights streamed per row) or sorted by expert (MFMA tiles)
 // ---------------------------------------------------------------------------------------------------------------
-void Model::stack_moe(const StackLayer& l, const void* x, int rows, const StackWs& w, const StackProf& pn, hipStream_t st) {
+MoeRouterArgs Model::stack_router(const StackLayer& l, const void* x, const StackWs& w) const { return MoeRouterArgs{x, l.wr, l.br, H, H, l.c.experts, l.c.top_experts, w.ids, w.wt}; }
+void Model::stack_moe(const StackLayer& l, const void* x, int rows, const StackWs& w, const StackProf& pn, hipStream_t st, bool routed) {
     const int dt = cfg.dtype, top = l.c.top_experts, E = l.c.experts, slots = rows * top;
-    { LMX_PROF_K(pn.router); launch_moe_router(dt, MoeRouterArgs{x, l.wr, l.br, H, H, E, top, w.ids, w.wt}, rows, st); }
+    if (!routed) { LMX_PROF_K(pn.router); launch_moe_router(dt, stack_router(l, x, w), rows, st); }
     if (group_gemm_applies(dt, slots, E)) {
         GroupGemmArgs p[2] = {{x, l.wgu, w.act, 2 * l.ff, H, H, H, l.ff, (size_t)2 * l.ff * H, slots, E}, {w.act, l.wd, w.slots, H, l.ff, l.ff, l.ff, H, (size_t)H * l.ff, slots, E}};
         p[0].act = l.act(); p[0].per_row = top;

@@ -93,8 +93,7 @@ __device__ __forceinline__ void decode_fused_body(DecodeFusedArgs a, const int h
             float sdot = 0.f;
 #pragma unroll
             for (int e = 0; e < 8; ++e) sdot = fmaf(qv[e], kv[u][e], sdot);
-#pragma unroll
-            for (int o = LPK / 2; o > 0; o >>= 1) sdot += __shfl_xor(sdot, o, 64);
+            sdot = group_sum<LPK>(sdot);
             if (sub == 0) sc_lds[kl] = kl < nk_cached ? sdot * scl : -INFINITY;
         }
         __syncthreads();
@@ -105,8 +104,7 @@ __device__ __forceinline__ void decode_fused_body(DecodeFusedArgs a, const int h
             float sdot = 0.f;
 #pragma unroll
             for (int e = 0; e < 8; ++e) sdot = fmaf(qv[e], kr[e], sdot);
-#pragma unroll
-            for (int o = LPK / 2; o > 0; o >>= 1) sdot += __shfl_xor(sdot, o, 64);
+            sdot = group_sum<LPK>(sdot);
             if (sub == 0) sc_lds[nk - 1] = sdot * scl;
             if (head % group == 0) store8<T>(Kc + (size_t)pos * D + sub * 8, kr);
         }
@@ -152,7 +150,7 @@ __device__ __forceinline__ void decode_fused_body(DecodeFusedArgs a, const int h
 #pragma unroll
         for (int db = 0; db < DB; ++db) {
             float t = acc[db];
-            t += __shfl_xor(t, 1, 64); t += __shfl_xor(t, 2, 64); t += __shfl_xor(t, 4, 64);
+            t = sum8(t);
             if (s8 == 0) {
                 const int d = db * 32 + drow;
                 if (has_new) t = fmaf(p_new, to_f32(vnew[d]), t);

@@ -116,8 +116,7 @@ __device__ __forceinline__ void dec_attn_chunk(const DecAttnArgs& a, int item, c
         float sdot = 0.f;
 #pragma unroll
         for (int e = 0; e < 8; ++e) sdot = fmaf(qv[e], kv[e], sdot);
-#pragma unroll
-        for (int o = LPK / 2; o > 0; o >>= 1) sdot += __shfl_xor(sdot, o, 64);
+        sdot = group_sum<LPK>(sdot);
         if (sub == 0) sc_lds[kl] = kl < nk ? sdot * scl : -INFINITY;
     }
     __syncthreads();
@@ -154,7 +153,7 @@ __device__ __forceinline__ void dec_attn_chunk(const DecAttnArgs& a, int item, c
 #pragma unroll
     for (int db = 0; db < DB; ++db) {
         float t = acc[db];
-        t += __shfl_xor(t, 1, 64); t += __shfl_xor(t, 2, 64); t += __shfl_xor(t, 4, 64);
+        t = sum8(t);
         if (s8 == 0) {
             const int d = db * 32 + drow;
             if (merger) mg_o[d] = t;                                       // the merger keeps its own partial in LDS
@@ -263,8 +262,7 @@ __device__ __forceinline__ void dec_attn_chunk(const DecAttnArgs& a, int item, c
         float sdot = 0.f;
 #pragma unroll
         for (int e2 = 0; e2 < 8; ++e2) sdot = fmaf(qv[e2], kr[e2], sdot);
-#pragma unroll
-        for (int o2 = LPK / 2; o2 > 0; o2 >>= 1) sdot += __shfl_xor(sdot, o2, 64);
+        sdot = group_sum<LPK>(sdot);
         if (sub == 0) red[4] = sdot * scl;
         if (head % group == 0) store8<T>(Kc + (size_t)pos * D + sub * 8, kr);
     }

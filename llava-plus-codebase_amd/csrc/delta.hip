@@ -26,14 +26,9 @@
 namespace lmx {
 
 // sum over the LPC lanes of a column (8, 16 or 32 consecutive lanes); every lane gets it
-template <int CTRL> __device__ __forceinline__ float dpp_add(float v) {
-    return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
-}
 template <int LPC> __device__ __forceinline__ float lanes_sum(float v) {
-    v = dpp_add<0xB1>(v);                                  // lane ^ 1
-    v = dpp_add<0x4E>(v);                                  // lane ^ 2
-    v = dpp_add<0x141>(v);                                 // mirror in 8
-    if constexpr (LPC >= 16) v = dpp_add<0x140>(v);        // mirror in 16
+    v = sum8(v);
+    if constexpr (LPC >= 16) v += dpp_get<0x140>(v);       // mirror in 16
     if constexpr (LPC >= 32) v += __shfl_xor(v, 16, 64);
     return v;
 }

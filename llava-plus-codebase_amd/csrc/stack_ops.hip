@@ -363,8 +363,7 @@ __global__ __launch_bounds__(256) void rows_attn_kernel(FlashArgs a) {
             float s = 0.f;
 #pragma unroll
             for (int e = 0; e < 8; ++e) s = fmaf(qv[e], kv[e], s);
-#pragma unroll
-            for (int o = LPK / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+            s = group_sum<LPK>(s);
             if (sub == 0) p_lds[b + kslot] = key >= lo && key <= pos ? s * scl : -INFINITY;
         }
     }
@@ -390,7 +389,7 @@ __global__ __launch_bounds__(256) void rows_attn_kernel(FlashArgs a) {
 #pragma unroll
             for (int e = 0; e < 8; ++e) acc = fmaf(pv[e], pv[e] != 0.f ? vv[e] : 0.f, acc);
         }
-        acc += __shfl_xor(acc, 1, 64); acc += __shfl_xor(acc, 2, 64); acc += __shfl_xor(acc, 4, 64);
+        acc = sum8(acc);
         if (sub == 0) O[d] = from_f32<T>(acc * out);
     }
 }
@@ -528,8 +527,7 @@ __global__ __launch_bounds__(256) void decode_win_kernel(WinDecodeArgs a) {
             float s = 0.f;
 #pragma unroll
             for (int i = 0; i < 8; ++i) s = fmaf(qv[i], kv[i], s);
-#pragma unroll
-            for (int o = LPK / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+            s = group_sum<LPK>(s);
             if (sub == 0) sc[kl] = key == pos ? red[6] : (key >= lo && key < pos ? s * scl : -INFINITY);
         }
         __syncthreads();
@@ -572,7 +570,7 @@ __global__ __launch_bounds__(256) void decode_win_kernel(WinDecodeArgs a) {
 #pragma unroll
     for (int db = 0; db < DB; ++db) {
         float t = acc[db];
-        t += __shfl_xor(t, 1, 64); t += __shfl_xor(t, 2, 64); t += __shfl_xor(t, 4, 64);
+        t = sum8(t);
         if (s8 == 0) {
             const int d = db * 32 + drow;
             if (a.n_split == 1) out[d] = from_f32<T>(t * fin);

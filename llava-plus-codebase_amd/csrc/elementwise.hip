@@ -420,8 +420,8 @@ void launch_copy_rows(int dtype, const void* src, void* dst, int N, int Ttot, in
 // ---------------------------------------------------------------------------------------------------------------
 // greedy sampling + decode-loop bookkeeping
 // ---------------------------------------------------------------------------------------------------------------
-template <typename T>
-__global__ __launch_bounds__(1024) void argmax_kernel(const T* __restrict__ logits, int V, int64_t* __restrict__ out) {
+// 1024 threads; thread 0 gets the id
+template <typename T> __device__ __forceinline__ int64_t argmax_row(const T* __restrict__ logits, int V) {
     __shared__ float bv[16];
     __shared__ int bi[16];
     float best = -INFINITY; int idx = 0x7fffffff;
@@ -444,11 +444,15 @@ __global__ __launch_bounds__(1024) void argmax_kernel(const T* __restrict__ logi
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     if (lane == 0) { bv[w] = best; bi[w] = idx; }
     __syncthreads();
-    if (threadIdx.x == 0) {
+    if (threadIdx.x == 0)
         for (int i = 1; i < 16; ++i)
             if (bv[i] > best || (bv[i] == best && bi[i] < idx)) { best = bv[i]; idx = bi[i]; }
-        *out = idx == 0x7fffffff ? 0 : idx;
-    }
+    return idx == 0x7fffffff ? 0 : idx;
+}
+template <typename T>
+__global__ __launch_bounds__(1024) void argmax_kernel(const T* __restrict__ logits, int V, int64_t* __restrict__ out) {
+    const int64_t t = argmax_row<T>(logits, V);
+    if (threadIdx.x == 0) *out = t;
 }
 
 void launch_argmax(int dtype, const void* logits, int V, int64_t* out_tok, hipStream_t st) {
@@ -590,15 +594,42 @@ void launch_set_stop(StopSpec* dst, const StopSpec& v, hipStream_t st) {
 }
 
 // the pick of a prefill (launch_argmax / launch_sample left it in *tok_ptr) joins the sequence's token log; its stop rule (may be null) is applied to it
+__device__ __forceinline__ void log_token(int64_t t, int64_t* log, int* n_out_ptr, int max_out, StopSpec* stop) {
+    if (stop && stop->done != 0) return;
+    const int n = *n_out_ptr;
+    if (n < max_out) log[n] = t;
+    *n_out_ptr = n + 1;
+    if (stop && stop_rule_fires(stop, t, log, n + 1, max_out)) stop->done = 1;
+}
 __global__ void log_token_kernel(const int64_t* tok_ptr, int64_t* log, int* n_out_ptr, int max_out, StopSpec* stop) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        if (stop && stop->done != 0) return;
-        const int n = *n_out_ptr;
-        const int64_t t = *tok_ptr;
-        if (n < max_out) log[n] = t;
-        *n_out_ptr = n + 1;
-        if (stop && stop_rule_fires(stop, t, log, n + 1, max_out)) stop->done = 1;
-    }
+    if (threadIdx.x == 0 && blockIdx.x == 0) log_token(*tok_ptr, log, n_out_ptr, max_out, stop);
+}
+// a workgroup a sequence: argmax_kernel and log_token_kernel
+__global__ __launch_bounds__(1024) void first_token_rows_kernel(FirstTokens a, int V) {
+    const FirstToken f = a.s[blockIdx.x];
+    const int64_t t = argmax_row<float>(f.logits, V);
+    if (threadIdx.x == 0) { *f.tok = t; log_token(t, f.log, f.n_out, f.max_out, f.stop); }
+}
+void launch_first_tokens(const FirstTokens& a, int n, int V, hipStream_t st) {
+    LMX_REQUIRE(n >= 0 && n <= HEAD_ROWS, "first_tokens: too many sequences");
+    if (n == 0) return;
+    hipLaunchKernelGGL(first_token_rows_kernel, dim3(n), dim3(1024), 0, st, a, V);
+    LMX_CHECK_HIP(hipGetLastError());
+}
+template <typename T>
+__global__ __launch_bounds__(256) void gather_rows_kernel(const T* __restrict__ src, T* __restrict__ dst, RowList rows, int W) {
+    const T* s = src + (size_t)rows.at[blockIdx.x] * W;
+    T* d = dst + (size_t)blockIdx.x * W;
+    constexpr int VE = 16 / sizeof(T);
+    for (int c = threadIdx.x; c < W / VE; c += 256) reinterpret_cast<uint4*>(d)[c] = reinterpret_cast<const uint4*>(s)[c];
+}
+void launch_gather_rows(int dtype, const void* src, void* dst, const RowList& rows, int n, int W, hipStream_t st) {
+    LMX_REQUIRE(n >= 0 && n <= HEAD_ROWS && W % 8 == 0, "gather_rows: bad rows");
+    if (n == 0) return;
+#define L(TT) hipLaunchKernelGGL(gather_rows_kernel<TT>, dim3(n), dim3(256), 0, st, (const TT*)src, (TT*)dst, rows, W)
+    if (dtype == kBF16) L(bf16_t); else if (dtype == kF16) L(f16_t); else L(float);
+#undef L
+    LMX_CHECK_HIP(hipGetLastError());
 }
 void launch_log_token(const int64_t* tok_ptr, int64_t* log, int* n_out_ptr, int max_out, StopSpec* stop, hipStream_t st) {
     hipLaunchKernelGGL(log_token_kernel, dim3(1), dim3(64), 0, st, tok_ptr, log, n_out_ptr, max_out, stop);

@@ -346,5 +346,12 @@ void launch_set_stop(StopSpec* dst, const StopSpec& v, hipStream_t st);
 void launch_hash128(const void* base, size_t bytes_per_item, int items, uint64_t* out_dev, hipStream_t st);      // out_dev[2 * item + {0, 1}]      // *dst = v on the stream (v travels as a kernel argument; re-arms done = v.done)
 void launch_interleave_half(int dtype, const void* src, void* dst, int I, int K, int half, hipStream_t st);
 void launch_log_token(const int64_t* tok_ptr, int64_t* log, int* n_out_ptr, int max_out, StopSpec* stop, hipStream_t st);
+// prompts that end together: their last rows side by side, one product with the head, one launch for all greedy picks
+constexpr int HEAD_ROWS = 32;
+struct RowList { int at[HEAD_ROWS]; };
+void launch_gather_rows(int dtype, const void* src, void* dst, const RowList& rows, int n, int W, hipStream_t st);
+struct FirstToken { const float* logits; int64_t* tok; int64_t* log; int* n_out; int max_out; StopSpec* stop; };
+struct FirstTokens { FirstToken s[HEAD_ROWS]; };
+void launch_first_tokens(const FirstTokens& a, int n, int V, hipStream_t st);
 
 }  // namespace lmx

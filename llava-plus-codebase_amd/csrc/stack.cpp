@@ -387,7 +387,7 @@ void Model::stack_prefill(Seq* const* seqs, const void* const* embeds, const int
     for (int i = 0; i < n; ++i) max_end = std::max(max_end, seqs[i]->len + Ts[i]);
     const size_t o_h = carve(S.ids_in() ? 0 : (size_t)block_rows * H * es), o_xr = carve((size_t)block_rows * H * 4), o_x = carve((size_t)block_rows * H * es),
                  o_y = carve((size_t)block_rows * H * es), o_qkv = carve((size_t)block_rows * qkv_n * es), o_attn = carve((size_t)block_rows * S.mix_n * es),
-                 o_act = carve((size_t)block_rows * I_l * es), o_log = carve((size_t)V * 4), o_want = carve((size_t)std::min(block_rows, LOGIT_ROWS) * H * es),
+                 o_act = carve((size_t)block_rows * I_l * es), o_log = carve((size_t)std::min(n, HEAD_ROWS) * V * 4), o_want = carve((size_t)std::min(block_rows, LOGIT_ROWS) * H * es),
                  o_ws = carve(S.ws_bytes(block_rows, H, es, false)), o_scratch = carve(stack_mix_scratch(block_rows, max_end));
     if (off > s0->pws.bytes) { LMX_CHECK_HIP(hipStreamSynchronize(st)); s0->pws.ensure(off); }
     char* Wk = s0->pws.as<char>();
@@ -511,17 +511,40 @@ void Model::stack_prefill(Seq* const* seqs, const void* const* embeds, const int
                     want_next[(size_t)g.seq] += nr;
                 }
             }
-        for (const Segment& g : seg) {
-            if (g.src0 + g.n != Ts[g.seq] || !(greedy || out.last_logits)) continue;
-            Seq* s = seqs[g.seq];
-            float* dst = out.last_logits ? out.last_logits + (size_t)g.seq * V : last_logits;
-            GemvArgs ga{rows(x, g.dst0 + g.n - 1, H), lm_head, dst, nullptr, nullptr, nullptr, 0.f, V, H, H, H, V, 0, kActNone};
-            ga.c_f32 = 1; ga.cap = S.c.logit_softcap;
-            { LMX_PROF_K("prefill.gemv.lm_head"); launch_gemv(dt, ga, 1, st); }
+        // the sequences that end in this piece (neighbours): one row alone through the GEMV, several through one product with the head (32 rows of 4096 one by one 1265 us)
+        std::vector<Segment> ends;
+        if (greedy || out.last_logits)
+            for (const Segment& g : seg) if (g.src0 + g.n == Ts[g.seq]) ends.push_back(g);
+        for (size_t i0 = 0; i0 < ends.size(); i0 += HEAD_ROWS) {
+            const int nr = (int)std::min(ends.size() - i0, (size_t)HEAD_ROWS);
+            const Segment* e = ends.data() + i0;
+            float* dst = out.last_logits ? out.last_logits + (size_t)e[0].seq * V : last_logits;
+            if (nr > 1 && dt != kF32) {
+                RowList list{};
+                for (int i = 0; i < nr; ++i) list.at[i] = e[i].dst0 + e[i].n - 1;
+                LMX_PROF("prefill.gemm.lm_head");
+                launch_gather_rows(dt, x, want, list, nr, H, st);
+                GemmArgs ga{want, lm_head, dst, nullptr, nullptr, nr, V, H, H, H, V, 0, kActNone};
+                ga.c_f32 = 1; ga.cap = S.c.logit_softcap;
+                launch_gemm(dt, ga, gv, st);
+            } else for (int i = 0; i < nr; ++i) {
+                GemvArgs ga{rows(x, e[i].dst0 + e[i].n - 1, H), lm_head, dst + (size_t)i * V, nullptr, nullptr, nullptr, 0.f, V, H, H, H, V, 0, kActNone};
+                ga.c_f32 = 1; ga.cap = S.c.logit_softcap;
+                LMX_PROF_K("prefill.gemv.lm_head");
+                launch_gemv(dt, ga, 1, st);
+            }
             if (!greedy) continue;
-            if (s->samp.temperature > 0.f) launch_sample(kF32, dst, Vr, s->samp, s->d_nout, s->d_tok, nullptr, nullptr, st);
-            else launch_argmax(kF32, dst, Vr, s->d_tok, st);
-            launch_log_token(s->d_tok, s->d_log, s->d_nout, s->log_cap, s->d_stop, st);
+            FirstTokens ft{};
+            int nf = 0;
+            for (int i = 0; i < nr; ++i) {
+                Seq* s = seqs[e[i].seq];
+                const float* z = dst + (size_t)i * V;
+                if (s->samp.temperature > 0.f) {
+                    launch_sample(kF32, z, Vr, s->samp, s->d_nout, s->d_tok, nullptr, nullptr, st);
+                    launch_log_token(s->d_tok, s->d_log, s->d_nout, s->log_cap, s->d_stop, st);
+                } else ft.s[nf++] = FirstToken{z, s->d_tok, s->d_log, s->d_nout, s->log_cap, s->d_stop};
+            }
+            launch_first_tokens(ft, nf, Vr, st);
         }
     }
     for (int i = 0; i < n; ++i) {

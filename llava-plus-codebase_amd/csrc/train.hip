@@ -196,10 +196,11 @@ template <typename T> __device__ __forceinline__ void unpack8(const uint4& u, fl
     v[0] = unpack_lo<T>(u.x); v[1] = unpack_hi<T>(u.x); v[2] = unpack_lo<T>(u.y); v[3] = unpack_hi<T>(u.y);
     v[4] = unpack_lo<T>(u.z); v[5] = unpack_hi<T>(u.z); v[6] = unpack_lo<T>(u.w); v[7] = unpack_hi<T>(u.w);
 }
-template <typename T, int NCH>
+// RPW 16: as above.  RPW 1 (dx alone, `inv` gets the rows' inverse norms): a wave a row, for row counts whose blocks of 128 leave CUs idle.
+template <typename T, int NCH, int RPW>
 __global__ __launch_bounds__(512) void rmsnorm_bwd_fused_kernel(const T* __restrict__ x, const T* __restrict__ w, const T* __restrict__ dy, const T* __restrict__ res,
-                                                                T* __restrict__ dx, float* __restrict__ part, int rows, float eps) {
-    constexpr int H = NCH * 512, RPB = 128, RPW = 16;
+                                                                T* __restrict__ dx, float* __restrict__ part, float* __restrict__ inv_out, int rows, float eps) {
+    constexpr int H = NCH * 512, RPB = 8 * RPW;
     __shared__ float sums[H];
     __shared__ __attribute__((aligned(16))) T wl[H];                       // the weight row, read back per chunk (registers go to the dw accumulators)
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -228,6 +229,7 @@ __global__ __launch_bounds__(512) void rmsnorm_bwd_fused_kernel(const T* __restr
         }
         ss = wave_sum(ss);
         const float inv = rsqrtf(ss / (float)H + eps);
+        if (RPW == 1 && inv_out && lane == 0) inv_out[r] = inv;
         // the packed words stay the only copy of the row between the passes: without these the compiler keeps the unpacked floats of one pass alive for the next
         // (128 more registers: spills)
 #define LMX_OPAQUE(v) asm volatile("" : "+v"((v).x), "+v"((v).y), "+v"((v).z), "+v"((v).w))
@@ -253,7 +255,7 @@ __global__ __launch_bounds__(512) void rmsnorm_bwd_fused_kernel(const T* __restr
             for (int e = 0; e < 8; ++e) {
                 const float xh = xf[e] * inv;
                 o[e] = inv * (gf[e] * wf[e] - xh * dot);
-                acc[j][e] += gf[e] * xf[e] * inv;
+                if (RPW > 1) acc[j][e] += gf[e] * xf[e] * inv;
             }
             if (res) {
                 float rf[8]; unpack8<T>(*reinterpret_cast<const uint4*>(res + off + j * 512), rf);
@@ -265,7 +267,7 @@ __global__ __launch_bounds__(512) void rmsnorm_bwd_fused_kernel(const T* __restr
             *reinterpret_cast<uint4*>(dx + off + j * 512) = u;
         }
     }
-    if (!part) return;                                                     // uniform: dx only
+    if (RPW == 1 || !part) return;                                         // uniform: dx only
     // the workgroup's partial row of dw: waves add their accumulators in wave order (deterministic)
 #pragma unroll 1
     for (int wv_ = 0; wv_ < 8; ++wv_) {
@@ -283,18 +285,54 @@ __global__ __launch_bounds__(512) void rmsnorm_bwd_fused_kernel(const T* __restr
     for (int c = threadIdx.x; c < H; c += 512) part[(size_t)blockIdx.x * H + c] = sums[c];
 }
 
+// dw's partial rows from 16-byte pieces: 64 columns x 128 rows a workgroup, 8 lanes a row, four rows a lane group requested together; the 32 groups' sums in order
+template <typename T>
+__global__ __launch_bounds__(256) void rmsnorm_bwd_dw_part8_kernel(const T* __restrict__ x, const T* __restrict__ dy, const float* __restrict__ inv, float* __restrict__ part, int rows, int H) {
+    __shared__ float red[32][65];
+    const int c = (threadIdx.x & 7) * 8, g = threadIdx.x >> 3, r0 = blockIdx.y * 128 + g;
+    Chunk8<T> xv[4], gv[4];
+    float iv[4], s[8] = {};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const int r = r0 + 32 * k < rows ? r0 + 32 * k : rows - 1;
+        xv[k].load(x + (size_t)r * H + blockIdx.x * 64 + c); gv[k].load(dy + (size_t)r * H + blockIdx.x * 64 + c); iv[k] = inv[r];
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        if (r0 + 32 * k >= rows) continue;
+        float a[8], b[8]; xv[k].get(a); gv[k].get(b);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s[e] += b[e] * a[e] * iv[k];
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) red[g][c + e] = s[e];
+    __syncthreads();
+    if (threadIdx.x < 64) {
+        float t[8] = {};                                                  // short chains: one of 32 rounds more than the one-pass form does
+#pragma unroll
+        for (int i = 0; i < 32; ++i) t[i % 8] += red[i][threadIdx.x];
+        part[(size_t)blockIdx.y * H + blockIdx.x * 64 + threadIdx.x] = ((t[0] + t[1]) + (t[2] + t[3])) + ((t[4] + t[5]) + (t[6] + t[7]));
+    }
+}
+
 void launch_rmsnorm_bwd(int dtype, const void* x, const void* w, const void* dy, const void* residual, void* dx, float* dw, float* inv_scratch, int rows, int H,
                         float eps, hipStream_t st) {
     if (rows <= 0) return;
     // partial rows of the weight gradient live in the CALLER's scratch, behind the [rows] inverse norms: inv_scratch holds
     // rows + cdiv(rows, 128) * H floats (lmx_op_rmsnorm_bwd's contract) — nothing process-wide, so steps on different streams / devices cannot meet
-    constexpr int RPB = 128;
+    constexpr int RPB = 128, RMS_BWD_ONE_PASS = 144;
     const int nblk = cdiv(rows, RPB);
     float* part = dw ? inv_scratch + (((size_t)rows + 63) / 64) * 64 : nullptr;
     const bool aligned = (((uintptr_t)x | (uintptr_t)w | (uintptr_t)dy | (uintptr_t)dx | (uintptr_t)residual) & 15) == 0;
     if (dtype != kF32 && aligned && (H == 1024 || H == 2048 || H == 4096)) {
-#define F(TT, NC) hipLaunchKernelGGL((rmsnorm_bwd_fused_kernel<TT, NC>), dim3(nblk), dim3(512), 0, st, (const TT*)x, (const TT*)w, (const TT*)dy, (const TT*)residual, \
-                                     (TT*)dx, part, rows, eps)
+        // Blocks of 128 rows are one pass over x and dy, and the faster form once they fill the chip; below that a row a wave, and the weight gradient reads both again.
+        // us with the residual, one pass / two: 1000 x 4096 100 / 20, 6528 x 4096 129 / 71, 16384 x 4096 202 / 191, 20000 x 4096 226 / 242; 6528 x 2048 74 / 41, 24576 x 2048 147 / 142
+        const bool two = nblk < RMS_BWD_ONE_PASS;
+#define F(TT, NC) do { if (two) hipLaunchKernelGGL((rmsnorm_bwd_fused_kernel<TT, NC, 1>), dim3(cdiv(rows, 8)), dim3(512), 0, st, (const TT*)x, (const TT*)w, (const TT*)dy, \
+                                                   (const TT*)residual, (TT*)dx, nullptr, dw ? inv_scratch : nullptr, rows, eps);                                        \
+                       else hipLaunchKernelGGL((rmsnorm_bwd_fused_kernel<TT, NC, 16>), dim3(nblk), dim3(512), 0, st, (const TT*)x, (const TT*)w, (const TT*)dy,          \
+                                               (const TT*)residual, (TT*)dx, part, nullptr, rows, eps);                                                                  \
+                       if (two && dw) hipLaunchKernelGGL(rmsnorm_bwd_dw_part8_kernel<TT>, dim3(H / 64, nblk), dim3(256), 0, st, (const TT*)x, (const TT*)dy, inv_scratch, part, rows, H); } while (0)
 #define FT(TT) do { if (H == 1024) F(TT, 2); else if (H == 2048) F(TT, 4); else F(TT, 8); } while (0)
         if (dtype == kBF16) FT(bf16_t); else FT(f16_t);
 #undef FT

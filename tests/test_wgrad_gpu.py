@@ -184,6 +184,21 @@ def test_rmsnorm_bwd_one_pass_form(cuda, rows, H, dtype, with_res):
     assert torch.equal(dx3, dx) and torch.equal(dw3, dw)                 # deterministic: partial rows are added in a fixed order
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows", [18304, 18305])
+def test_rmsnorm_bwd_on_both_sides_of_its_line(cuda, rows, dtype):
+    """143 blocks of 128 rows: dx by a wave a row, dw in a second pass; 144: both in one pass.  A term of dw passes at
+    most 16 + 8 + 144 additions, three products and the rounding of rsqrt: under 180 fp32 roundings of the sum of magnitudes."""
+    ops = _ops()
+    x, dy, w = _rand((rows, 1024), dtype, cuda, 21), _rand((rows, 1024), dtype, cuda, 22), (1 + 0.1 * _rand((1024,), torch.float32, cuda, 23)).to(dtype)
+    dx, dw = ops.rmsnorm_bwd(x, w, dy, 1e-5)
+    inv = torch.rsqrt(x.double().pow(2).mean(-1, keepdim=True) + 1e-5)
+    xh, g = x.double() * inv, dy.double() * w.double()
+    dx_ref, dw_ref = inv * (g - xh * (g * xh).mean(-1, keepdim=True)), (dy.double() * xh).sum(0)
+    assert (dx.double() - dx_ref).abs().max().item() <= 1.01 * (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11) * dx_ref.abs().max().item()
+    assert bool(((dw.double() - dw_ref).abs() <= 180 * 2.0 ** -24 * (dy.double() * xh).abs().sum(0)).all())
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("nh,nkv,D", [(32, 32, 128), (4, 2, 64)])
 def test_rope_kv_rows_leaves_rotated_k_in_the_rows(cuda, nh, nkv, D, dtype):

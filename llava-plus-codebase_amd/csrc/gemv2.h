@@ -271,7 +271,7 @@ __device__ __forceinline__ void gemv2_body(const GemvArgs& a, int bid, char* sme
     }
 }
 
-// x' of one row to rn.x_out by the 256 threads of the calling workgroup (see RES above)
+// x' of one row to rn.x_out by the 256 threads of the calling workgroup (see RES above) and, where other launches read it too, its normalised row to rn.xn
 template <typename T>
 __device__ __forceinline__ void residual_row_store(const ResidualNormArgs& rn, float* red) {
     const T* y = reinterpret_cast<const T*>(rn.y);
@@ -288,6 +288,7 @@ __device__ __forceinline__ void residual_row_store(const ResidualNormArgs& rn, f
         }
         inv1 = post ? rn.mult / sqrtf(block_sum<4>(ss, red) * (1.f / (float)rn.H_real) + rn.eps) : rn.mult;
     }
+    float s2 = 0.f;
     for (int c = tid; c < HC; c += 256) {
         float x[8], v[8], g[8];
         if (rn.x_in) load8<float>(rn.x_in + c * 8, x);
@@ -307,6 +308,17 @@ __device__ __forceinline__ void residual_row_store(const ResidualNormArgs& rn, f
             for (int e = 0; e < 8; ++e) x[e] += g[e];
         }
         store8<float>(rn.x_out + c * 8, x);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s2 += x[e] * x[e];
+    }
+    if (!rn.xn) return;
+    const float inv2 = 1.f / sqrtf(block_sum<4>(s2, red) * (1.f / (float)rn.H_real) + rn.eps);
+    for (int c = tid; c < HC; c += 256) {                    // (every thread reads back what it wrote)
+        float x[8], g[8];
+        load8<float>(rn.x_out + c * 8, x); load8<T>(reinterpret_cast<const T*>(rn.pre_w) + c * 8, g);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = x[e] * inv2 * g[e];
+        store8<T>(reinterpret_cast<T*>(rn.xn) + c * 8, x);
     }
 }
 

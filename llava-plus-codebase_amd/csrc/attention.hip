@@ -207,7 +207,7 @@ __global__ __launch_bounds__(512, D == 64 && !WIN ? 4 : 2) void flash_prefill2_k
                     tmax = fmaxf(tmax, v);
                 }
         }
-        tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
+        tmax = fold32(tmax, OpMax{});
         // defer-max: keep the old running max (no O / l rescale) while no row of the wave grew by more than 2^FA_DEFER;
         // P is then bounded by 2^FA_DEFER instead of 1, which fp32 sums and 16-bit P fragments absorb.  m_run starts at
         // -1e30, so the first tile always takes the rescale branch (alpha = 0 on zero accumulators).
@@ -284,7 +284,7 @@ __global__ __launch_bounds__(512, D == 64 && !WIN ? 4 : 2) void flash_prefill2_k
 #pragma unroll
             for (int r = 0; r < 16; ++r) oacc[i][r] = oacc[i][r] * a0 + mg[(i * 16 + r) * 64 + lane] * a1;
     }
-    const float l_tot = l_run + __shfl_xor(l_run, 32, 64);
+    const float l_tot = fold32(l_run, OpSum{});
     if (a.part) {                                        // sums as they are, with their maximum: flash_merge_kernel
         if (qrow >= a.q_len) return;
         float* pp = a.part + (((size_t)blockIdx.z * a.q_len + qrow) * a.n_heads + head) * (D + 4);
@@ -452,8 +452,7 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(DecodeAttnArgs a) {
             float s = 0.f;
 #pragma unroll
             for (int e = 0; e < 8; ++e) s = fmaf(qv[e], kv[e], s);
-#pragma unroll
-            for (int o = LPK / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+            s = group_sum<LPK>(s);
             if (sub == 0 && kl < nk) sc_lds[kl] = s * scl;
         }
     }
@@ -494,9 +493,7 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(DecodeAttnArgs a) {
                 acc = fmaf(p1.x, vv[4], acc); acc = fmaf(p1.y, vv[5], acc);
                 acc = fmaf(p1.z, vv[6], acc); acc = fmaf(p1.w, vv[7], acc);
             }
-            acc += __shfl_xor(acc, 1, 64);
-            acc += __shfl_xor(acc, 2, 64);
-            acc += __shfl_xor(acc, 4, 64);
+            acc = sum8(acc);
             if (sub == 0) ws[2 + d] = acc;
         }
     }

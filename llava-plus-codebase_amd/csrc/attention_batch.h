@@ -128,7 +128,7 @@ __global__ __launch_bounds__(BA_NW * 64) void decode_attn_wave_kernel(DecodeFuse
         // ---- online softmax over the piece --------------------------------------------------------------------------------------------------------------
         float mx = fmaxf(s, ba_dpp<0x140>(s));
         mx = fmaxf(mx, ba_dpp<0x141>(mx)); mx = fmaxf(mx, ba_dpp<0x1B>(mx)); mx = fmaxf(mx, ba_dpp<0xB1>(mx));
-        mx = fmaxf(mx, __shfl_xor(mx, 16, 64)); mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        mx = fold16(mx, OpMax{}); mx = fold32(mx, OpMax{});
         const float m_new = fmaxf(m_run, mx);                               // finite: the piece has at least one live key
         const float p = live ? __builtin_amdgcn_exp2f(s - m_new) : 0.f;
         const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);          // first piece: exp2(-inf) = 0 on zero accumulators
@@ -182,7 +182,7 @@ __global__ __launch_bounds__(BA_NW * 64) void decode_attn_wave_kernel(DecodeFuse
         float dot = 0.f;
 #pragma unroll
         for (int c = 0; c < 8; ++c) dot = fmaf(qv[c], kr[c], dot);
-        dot += __shfl_xor(dot, 8, 64); dot += __shfl_xor(dot, 4, 64); dot += __shfl_xor(dot, 2, 64); dot += __shfl_xor(dot, 1, 64);
+        dot = group_sum<16>(dot);
         if (lane == 0) { part[NW][D] = dot * scl; part[NW][D + 1] = 1.f; }
         if (head % group == 0 && kslot == 0) store8<T>(Kc + (size_t)pos * D + sub * 8, kr);          // one workgroup per kv head appends
     }

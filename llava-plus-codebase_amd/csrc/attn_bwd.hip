@@ -215,7 +215,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_mfma_kernel(BwdArgs a) {
                     sv[kb][r] = v;
                     tmax = fmaxf(tmax, v);
                 }
-            tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
+            tmax = fold32(tmax, OpMax{});
             const float m_new = fmaxf(m_run, tmax);                  // finite from the first tile on: key 0 is visible to every row
             const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
             float ps = 0.f, pds = 0.f;
@@ -231,8 +231,8 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_mfma_kernel(BwdArgs a) {
             pd_run = pd_run * alpha + pds;
             m_run = m_new;
         }
-        const float l_tot = l_run + __shfl_xor(l_run, 32, 64);
-        const float pd_tot = pd_run + __shfl_xor(pd_run, 32, 64);
+        const float l_tot = fold32(l_run, OpSum{});
+        const float pd_tot = fold32(pd_run, OpSum{});
         lse2 = m_run + __builtin_amdgcn_logf(l_tot);                  // v_log_f32 = log2
         delta = pd_tot / l_tot;
         if (hi == 0 && qrow < a.T) { a.lse[(size_t)head * a.lse_stride + qrow] = lse2; a.delta[(size_t)head * a.Tp + qrow] = delta; }

@@ -156,18 +156,28 @@ template <> struct Chunk8<float> {
 // Lanes meet in DPP moves and, past a row of 16, permlane swaps (a few cycles each; through LDS, as a shuffle goes, every step is a round trip of some 70).  The pairs are those of
 // xor shuffles with N/2 .. 1: behind the step of 8 a row is periodic, so rotations are as good as the xor.  Whole waves only.  (decode_win_kernel, 16 heads x 600 keys: 11.95 -> 9.7 us; a gated linear of 11264 x 2048 with its norms 12.9 -> 11.9)
 template <int CTRL> __device__ __forceinline__ float dpp_get(float v) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true)); }
+template <typename OP> __device__ __forceinline__ float fold32(float v, OP op) {      // lanes l and l ^ 32
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+template <typename OP> __device__ __forceinline__ float fold16(float v, OP op) {      // lanes l and l ^ 16
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+struct OpSum { __device__ __forceinline__ float operator()(float x, float y) const { return x + y; } };
+struct OpMax { __device__ __forceinline__ float operator()(float x, float y) const { return fmaxf(x, y); } };
 template <int N, typename OP> __device__ __forceinline__ float group_fold(float v, OP op) {
     static_assert(N == 8 || N == 16 || N == 32 || N == 64, "lanes of a group");
-    if constexpr (N >= 64) { const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false); v = op(__uint_as_float(r[0]), __uint_as_float(r[1])); }
-    if constexpr (N >= 32) { const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false); v = op(__uint_as_float(r[0]), __uint_as_float(r[1])); }
+    if constexpr (N >= 64) v = fold32(v, op);
+    if constexpr (N >= 32) v = fold16(v, op);
     if constexpr (N >= 16) { v = op(v, dpp_get<0x128>(v)); v = op(v, dpp_get<0x124>(v)); }
     else v = op(v, __shfl_xor(v, 4, 64));
     v = op(v, dpp_get<0x4E>(v));
     return op(v, dpp_get<0xB1>(v));
 }
-template <int N> __device__ __forceinline__ float group_sum(float v) { return group_fold<N>(v, [](float x, float y) { return x + y; }); }
+template <int N> __device__ __forceinline__ float group_sum(float v) { return group_fold<N>(v, OpSum{}); }
 __device__ __forceinline__ float wave_sum(float v) { return group_sum<64>(v); }
-__device__ __forceinline__ float wave_max(float v) { return group_fold<64>(v, [](float x, float y) { return fmaxf(x, y); }); }
+__device__ __forceinline__ float wave_max(float v) { return group_fold<64>(v, OpMax{}); }
 // sum over 8 consecutive lanes, neighbours first
 __device__ __forceinline__ float sum8(float v) {
     v += dpp_get<0xB1>(v);                                  // lane ^ 1

@@ -29,7 +29,7 @@ namespace lmx {
 template <int LPC> __device__ __forceinline__ float lanes_sum(float v) {
     v = sum8(v);
     if constexpr (LPC >= 16) v += dpp_get<0x140>(v);       // mirror in 16
-    if constexpr (LPC >= 32) v += __shfl_xor(v, 16, 64);
+    if constexpr (LPC >= 32) v = fold16(v, OpSum{});
     return v;
 }
 __device__ __forceinline__ float softplus_f32(float z) { return z > 20.f ? z : log1pf(expf(z)); }

@@ -96,8 +96,7 @@ __global__ __launch_bounds__(256) void latent_decode_kernel(LatentDecodeArgs a) 
             float t = 0.f;
 #pragma unroll
             for (int i = 0; i < 8; ++i) t = fmaf(q[i], c[u][i], t);
-#pragma unroll
-            for (int o = LPK / 2; o > 0; o >>= 1) t += __shfl_xor(t, o, 64);
+            t = group_sum<LPK>(t);
             s[u] = j0 + u * step <= pos ? t * scl : -INFINITY;
             mx = fmaxf(mx, s[u]);
         }
@@ -238,7 +237,7 @@ __global__ __launch_bounds__(256, 1) void latent_mfma_kernel(LatentDecodeArgs a)
 #pragma unroll
             for (int i = 0; i < 8; ++i) mx = fmaxf(mx, p[t][i]);
         }
-        mx = fmaxf(mx, __shfl_xor(mx, 16, 64)); mx = fmaxf(mx, __shfl_xor(mx, 32, 64));      // finite: the tile's first key is seen
+        mx = fold16(mx, OpMax{}); mx = fold32(mx, OpMax{});      // finite: the tile's first key is seen
         const float alpha = __builtin_amdgcn_exp2f(m - mx);
         m = mx; l *= alpha;
         uint4 pf[4];
@@ -266,7 +265,7 @@ __global__ __launch_bounds__(256, 1) void latent_mfma_kernel(LatentDecodeArgs a)
             }
         }
     }
-    l += __shfl_xor(l, 16, 64); l += __shfl_xor(l, 32, 64);
+    l = fold16(l, OpSum{}); l = fold32(l, OpSum{});
     // one split: the output; several: accumulators [head][split][R + 4] with maximum and sum behind them, for latent_merge_kernel
     T* out = reinterpret_cast<T*>(a.out) + ((size_t)z * a.H + h0) * R;
     float* ws = a.n_split > 1 ? e.ws + ((size_t)h0 * a.n_split + split) * (R + 4) : nullptr;

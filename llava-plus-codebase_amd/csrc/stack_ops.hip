@@ -741,7 +741,7 @@ __global__ __launch_bounds__(256) void decode_win_group_kernel(WinDecodeArgs a) 
                 s[g][r] = !edge || (key >= lo && key < pos) ? s[g][r] * scl : -INFINITY;
                 mx = fmaxf(mx, s[g][r]);
             }
-        mx = fmaxf(mx, __shfl_xor(mx, 16, 64)); mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        mx = fold16(mx, OpMax{}); mx = fold32(mx, OpMax{});
         const float m_new = fmaxf(m, mx), ms = m_new == -INFINITY ? 0.f : m_new;
         const float alpha = __builtin_amdgcn_exp2f(m - ms);
         m = m_new;
@@ -809,7 +809,7 @@ __global__ __launch_bounds__(256) void decode_win_group_kernel(WinDecodeArgs a) 
         }
     }
     // ---- the four waves, then the splits ----
-    l += __shfl_xor(l, 16, 64); l += __shfl_xor(l, 32, 64);
+    l = fold16(l, OpSum{}); l = fold32(l, OpSum{});
     if (q4 == 0) { wm[wave * 16 + i16] = m; wl[wave * 16 + i16] = l; }
     __syncthreads();                                           // every wave is done with its tile: the partial rows take their place
     if (i16 < group) {

@@ -890,7 +890,7 @@ bool decode_win_groups(int dtype, int D, int n_heads, int n_kv_heads, int n_seq)
 //   32 heads on 32           8 of 1200  74 -> 32                  2 of 300  14 -> 12     16 of 130 33 -> 23     16 of 60  18 -> 20
 //    8 heads on  1          32 of 600   34 -> 15                  8 of 600  14 -> 15     2 of 600  12 -> 15      8 of 60  9 -> 12     (16 on 1: 16 of 600 25 -> 20, 4 of 600 13 -> 20)
 // so: up to groups of four from one chunk of keys on, larger groups by the bytes that one head a workgroup asks for (the merge grows with the group); shorter contexts only where
-// a group is three or four.  One sequence of 601 keys, 16 heads on 4: 11.1 us either way, all of it latency, so the form with more workgroups stays.
+// a group is three or four.  One sequence of 601 keys, 16 heads on 4: 11.1 us either way (9.7 since sums over lanes pass LDS by), all of it latency, so the form with more workgroups stays.
 // Splits: as many as make ONE round of workgroups of the grouped kernel (its waves fill a CU: 96 x 3 and 160 x 2 workgroups took a second round, 15 -> 19 and 21 -> 25 us).
 WinForm decode_win_form(int dtype, int D, int n_heads, int n_kv_heads, int n_seq, int span) {
     const int group = n_heads / n_kv_heads, chunks = std::max(1, std::min((span + 127) / 128, DF_MAX_SPLIT));

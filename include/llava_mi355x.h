@@ -382,7 +382,7 @@ int lmx_op_decode_win(int32_t dtype, int32_t D, const void* qkv, int32_t qkv_str
 /* what a decode step takes, on the host alone: form[2] = {all query heads of a kv head in one workgroup, splits}; span: keys that the longest sequence may have to walk.
  * (lmx_op_decode_win itself gives every batch that it can to the grouped kernel.) */
 int lmx_op_decode_win_form(int32_t dtype, int32_t D, int32_t n_heads, int32_t n_kv_heads, int32_t n_seq, int32_t span, int32_t* form);
-/* act(x_row W_g^T) of every slot (row, choice): g = ids[slot] picks one of the groups' weights w [groups][N][K]; x row = slot / per_row (shared_x) or slot, c row = slot.
+/* act(x_row W_g^T) of every slot (row, choice): g = ids[slot], in [0, groups), picks one of the groups' weights w [groups][N][K]; x row = slot / per_row (shared_x) or slot, c row = slot.
  * bm: rows of a tile, 0 = as the engine chooses; 32, 64 or, 16-bit four-wave tiles, 128 .. 256 in steps of 32, those with nb blocks of 32 columns (0 = as the engine chooses).
  * plan: lmx_op_group_plan_bytes(rows, per_row) bytes of scratch. */
 size_t lmx_op_group_plan_bytes(int32_t rows, int32_t per_row);

@@ -397,7 +397,8 @@ int lmx_op_im2col(int32_t dtype, const void* pixels, void* out, int32_t N, int32
  *   positions; scratch: B*(T-1) floats each; dlogits (optional, [B*T][ldd]) = grad * d(loss)/d(logits).
  * lmx_op_rmsnorm_bwd / swiglu_bwd / rope_bwd: autograd of LlamaRMSNorm, silu(gate)*up and apply_rotary_pos_emb
  *   (HF5:models/llama/modeling_llama.py:53-67, 163-176, 138-160); rmsnorm_bwd's inv_scratch holds round_up(rows, 64) + ceil(rows / 128) * H floats
- *   (inverse norms, then the weight gradient's partial rows: the caller owns every byte of scratch).  lmx_op_transpose: operand re-layout so that dgrad / wgrad run on lmx_op_gemm.
+ *   (inverse norms, then the weight gradient's partial rows: the caller owns every byte of scratch); its dx may be x or dy itself for 16-bit rows of 1024, 2048 or 4096
+ *   from 16-byte addresses, and is another buffer otherwise.  lmx_op_transpose: operand re-layout so that dgrad / wgrad run on lmx_op_gemm.
  * lmx_op_attn_bwd: causal attention backward (contract of llava/train/llama_flash_attn_monkey_patch.py:68-91): q / k / v / d_out as
  *   [T][heads][head_dim] rows of stride ldq / ldk / ldo elements; dk32 / dv32: T*kv_heads*head_dim fp32 scratch. */
 int lmx_op_ce_loss(int32_t dtype, const void* logits, int32_t ld, const int64_t* labels, int32_t B, int32_t T, int32_t V, int64_t ignore_index,

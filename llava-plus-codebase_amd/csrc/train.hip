@@ -319,7 +319,7 @@ void launch_rmsnorm_bwd(int dtype, const void* x, const void* w, const void* dy,
                         float eps, hipStream_t st) {
     if (rows <= 0) return;
     // partial rows of the weight gradient live in the CALLER's scratch, behind the [rows] inverse norms: inv_scratch holds
-    // rows + cdiv(rows, 128) * H floats (lmx_op_rmsnorm_bwd's contract) — nothing process-wide, so steps on different streams / devices cannot meet
+    // round_up(rows, 64) + cdiv(rows, 128) * H floats (lmx_op_rmsnorm_bwd's contract) — nothing process-wide, so steps on different streams / devices cannot meet
     constexpr int RPB = 128, RMS_BWD_ONE_PASS = 144;
     const int nblk = cdiv(rows, RPB);
     float* part = dw ? inv_scratch + (((size_t)rows + 63) / 64) * 64 : nullptr;
@@ -327,7 +327,8 @@ void launch_rmsnorm_bwd(int dtype, const void* x, const void* w, const void* dy,
     if (dtype != kF32 && aligned && (H == 1024 || H == 2048 || H == 4096)) {
         // Blocks of 128 rows are one pass over x and dy, and the faster form once they fill the chip; below that a row a wave, and the weight gradient reads both again.
         // us with the residual, one pass / two: 1000 x 4096 100 / 20, 6528 x 4096 129 / 71, 16384 x 4096 202 / 191, 20000 x 4096 226 / 242; 6528 x 2048 74 / 41, 24576 x 2048 147 / 142
-        const bool two = nblk < RMS_BWD_ONE_PASS;
+        // A dx that lies on x or dy, with a weight gradient: one pass whatever the size, which has read a row when it writes it; the second of two would read what the first has written.
+        const bool two = nblk < RMS_BWD_ONE_PASS && !(dw && (dx == x || dx == dy));
 #define F(TT, NC) do { if (two) hipLaunchKernelGGL((rmsnorm_bwd_fused_kernel<TT, NC, 1>), dim3(cdiv(rows, 8)), dim3(512), 0, st, (const TT*)x, (const TT*)w, (const TT*)dy, \
                                                    (const TT*)residual, (TT*)dx, nullptr, dw ? inv_scratch : nullptr, rows, eps);                                        \
                        else hipLaunchKernelGGL((rmsnorm_bwd_fused_kernel<TT, NC, 16>), dim3(nblk), dim3(512), 0, st, (const TT*)x, (const TT*)w, (const TT*)dy,          \

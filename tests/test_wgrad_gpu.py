@@ -199,6 +199,29 @@ def test_rmsnorm_bwd_on_both_sides_of_its_line(cuda, rows, dtype):
     assert bool(((dw.double() - dw_ref).abs() <= 180 * 2.0 ** -24 * (dy.double() * xh).abs().sum(0)).all())
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H", [1024, 2048, 4096])
+@pytest.mark.parametrize("over", ["x", "dy"])
+@pytest.mark.parametrize("with_res", [False, True])
+def test_rmsnorm_bwd_over_one_of_its_inputs(cuda, over, H, dtype, with_res):
+    """dx written over x or dy, row counts far below the one-pass line: dx has the bits of a call with a buffer of its own, dw is the float64 sum over what x and dy were.  A term of dw
+    passes at most 16 + 8 + 2 additions, three products and the rounding of rsqrt: under 32 fp32 roundings of the sum of magnitudes."""
+    from llava_mi355x import _C
+    ops = _ops()
+    rows, eps = 200, 1e-5
+    x, dy, w = _rand((rows, H), dtype, cuda, 31), _rand((rows, H), dtype, cuda, 32, 0.7), (1 + 0.1 * _rand((H,), torch.float32, cuda, 33)).to(dtype)
+    res = _rand((rows, H), dtype, cuda, 34) if with_res else None
+    want, _ = ops.rmsnorm_bwd(x, w, dy, eps, residual=res)
+    xh = x.double() * torch.rsqrt(x.double().pow(2).mean(-1, keepdim=True) + eps)
+    terms = dy.double() * xh
+    dx = x if over == "x" else dy
+    dw, scratch = torch.empty(H, device=cuda), torch.empty(256 + 2 * H, device=cuda)
+    args = [_C.torch_dtype_code(dtype), _C.ptr(x), _C.ptr(w), _C.ptr(dy)] + ([_C.ptr(res)] if with_res else []) + [_C.ptr(dx), _C.ptr(dw), _C.ptr(scratch), rows, H, eps, _C.stream_handle()]
+    _C.check((_C.lib.lmx_op_rmsnorm_bwd_add if with_res else _C.lib.lmx_op_rmsnorm_bwd)(*args), "rmsnorm_bwd")
+    assert torch.equal(dx, want)
+    assert bool(((dw.double() - terms.sum(0)).abs() <= 32 * 2.0 ** -24 * terms.abs().sum(0)).all())
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("nh,nkv,D", [(32, 32, 128), (4, 2, 64)])
 def test_rope_kv_rows_leaves_rotated_k_in_the_rows(cuda, nh, nkv, D, dtype):

@@ -1,5 +1,6 @@
 // Host side of the four-wave GEMM (kernels: gemm4w.h): which tile and how many K slices, and the launch.
 #include <algorithm>
+#include <iterator>
 #include <mutex>
 
 #include "gemm4w.h"
@@ -140,6 +141,8 @@ TileForm gemm4w_form(int dtype, const GemmArgs& a) {
 }
 
 void launch_gemm4w(int dtype, GemmArgs a, TileForm f, hipStream_t st) {
+    LMX_REQUIRE(dtype == kBF16 || dtype == kF16, "gemm4w: 16-bit dtypes only");
+    LMX_REQUIRE(std::any_of(std::begin(kTiles), std::end(kTiles), [&](const Tile& t) { return t.mb == f.mb && t.nb == f.nb; }), "gemm4w: no such tile");
     LMX_REQUIRE(a.K % 64 == 0, "gemm4w: K must be a multiple of 64");
     LMX_REQUIRE((size_t)a.M * a.ldx * 2 < ((size_t)1 << 32) && (size_t)a.N * a.ldw * 2 < ((size_t)1 << 32), "gemm4w: operands must be addressable with 32-bit byte offsets");
     LMX_REQUIRE(!act_gated(a.act) || a.N % 64 == 0, "gemm4w: SiLU·mul needs N % 64 == 0");
@@ -163,8 +166,7 @@ void launch_gemm4w(int dtype, GemmArgs a, TileForm f, hipStream_t st) {
     // the CLIP K / V^T pack lives in the un-split epilogue only: a K-sliced launch's reduction would write the k | v columns to C and leave the pack untouched
     if (a.pk_kc) LMX_REQUIRE(f.slices == 1 && !act_gated(a.act) && a.pk_D % 8 == 0 && a.N % 8 == 0, "gemm4w: the K / V^T pack epilogue needs an un-split launch of a plain linear");
     if (dtype == kBF16) launch_t<bf16_t>(a, f, st);
-    else if (dtype == kF16) launch_t<f16_t>(a, f, st);
-    else throw Error{"gemm4w: 16-bit dtypes only"};
+    else launch_t<f16_t>(a, f, st);
 }
 
 }  // namespace lmx

@@ -65,3 +65,13 @@ def test_a_form_by_number_checks_what_the_choice_checks(dt, N, K, ldx, ldw, word
     any_ = ctypes.c_void_p(4096)
     assert _C.lib.lmx_op_gemm(_C.torch_dtype_code(dt), any_, any_, any_, None, None, 64, N, K, ldx, ldw, N, 0, 0, variant, None) != 0
     assert words in _C.last_error()
+
+
+@pytest.mark.parametrize("variant", [100, 102, 109, 331, 492, 802, 803, 902])
+def test_a_four_wave_tile_that_is_not_there(variant):
+    """No tile of 0 blocks, none outside the table: an error before anything is computed from its sizes."""
+    import ctypes
+    from llava_mi355x import _C
+    any_ = ctypes.c_void_p(4096)
+    assert _C.lib.lmx_op_gemm(_C.torch_dtype_code(torch.bfloat16), any_, any_, any_, None, None, 64, 256, 256, 256, 256, 256, 0, 0, variant, None) != 0
+    assert "no such tile" in _C.last_error()

@@ -141,9 +141,11 @@ TileForm gemm4w_form(int dtype, const GemmArgs& a) {
 }
 
 void launch_gemm4w(int dtype, GemmArgs a, TileForm f, hipStream_t st) {
+    // (forms by number come here without launch_gemm's and gemm4w_form's checks)
     LMX_REQUIRE(dtype == kBF16 || dtype == kF16, "gemm4w: 16-bit dtypes only");
     LMX_REQUIRE(std::any_of(std::begin(kTiles), std::end(kTiles), [&](const Tile& t) { return t.mb == f.mb && t.nb == f.nb; }), "gemm4w: no such tile");
     LMX_REQUIRE(a.K % 64 == 0, "gemm4w: K must be a multiple of 64");
+    LMX_REQUIRE(a.ldx % 8 == 0 && a.ldw % 8 == 0, "gemm4w: leading dims must keep 16-byte row alignment");
     LMX_REQUIRE((size_t)a.M * a.ldx * 2 < ((size_t)1 << 32) && (size_t)a.N * a.ldw * 2 < ((size_t)1 << 32), "gemm4w: operands must be addressable with 32-bit byte offsets");
     LMX_REQUIRE(!act_gated(a.act) || a.N % 64 == 0, "gemm4w: SiLU·mul needs N % 64 == 0");
     LMX_REQUIRE(a.N % 4 == 0 && a.ldc % 4 == 0 && (!a.R || a.ldr % 4 == 0) && !a.c_f32, "gemm4w: rows of 8 bytes, 16-bit output");

@@ -67,6 +67,17 @@ def test_a_form_by_number_checks_what_the_choice_checks(dt, N, K, ldx, ldw, word
     assert words in _C.last_error()
 
 
+@pytest.mark.parametrize("dt,K,ldx,ldw,words", [(torch.bfloat16, 256, 260, 256, "16-byte row alignment"), (torch.float16, 256, 256, 257, "16-byte row alignment"), (torch.bfloat16, 96, 96, 96, "multiple of 64"),
+                                                (torch.float32, 256, 256, 256, "16-bit dtypes")])
+@pytest.mark.parametrize("variant", [881, 882, 443])
+def test_a_four_wave_form_by_number_checks_what_the_choice_checks(dt, K, ldx, ldw, words, variant):
+    import ctypes
+    from llava_mi355x import _C
+    any_ = ctypes.c_void_p(4096)
+    assert _C.lib.lmx_op_gemm(_C.torch_dtype_code(dt), any_, any_, any_, None, None, 64, 256, K, ldx, ldw, 256, 0, 0, variant, None) != 0
+    assert words in _C.last_error()
+
+
 @pytest.mark.parametrize("variant", [100, 102, 109, 331, 492, 802, 803, 902])
 def test_a_four_wave_tile_that_is_not_there(variant):
     """No tile of 0 blocks, none outside the table: an error before anything is computed from its sizes."""

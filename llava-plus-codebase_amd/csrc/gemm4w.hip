@@ -123,6 +123,7 @@ size_t gemm4w_slab_bytes(int M, int N, const TileForm& f) {
 TileForm gemm4w_form(int dtype, const GemmArgs& a) {
     const TileForm none{0, 0, 1};
     if ((dtype != kBF16 && dtype != kF16) || a.c_f32 || a.K % 64 != 0 || a.N % 8 != 0 || (act_gated(a.act) && a.N % 64 != 0) || (a.pk_kc && a.pk_D % 8 != 0)) return none;
+    if (a.R && a.ldr % 4 != 0) return none;                  // residual rows of any pitch: another kernel's
     if ((size_t)a.M * a.ldx * 2 >= ((size_t)1 << 32) || (size_t)a.N * a.ldw * 2 >= ((size_t)1 << 32)) return none;
     if (a.M <= 256 || (int64_t)cdiv(a.M, 64) * cdiv(a.N, 64) <= 640) return none;
     TileForm best = none;

@@ -91,6 +91,22 @@ def test_choice(cuda, M, N, K, act):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+@pytest.mark.parametrize("M,N,K", [(513, 4672, 640), (1087, 4096, 4096), (2048, 5120, 1024)])
+@pytest.mark.parametrize("odd", [1, 2, 3])
+def test_residual_rows_of_any_pitch(cuda, dt, M, N, K, odd):
+    """A residual whose rows are not multiples of 8 bytes apart, on the large side of the rule's lines: taken by another kernel, not refused."""
+    from llava_mi355x import _C
+    x, w = _mk(M, N, K, dt, cuda, M + odd)
+    r = torch.randn(M, N + odd, device=cuda).to(DT[dt])
+    ref = x.double() @ w.double().t() + r[:, :N].double()
+    out = torch.empty(M, N, device=cuda, dtype=DT[dt])
+    for v in (0, _C.GEMM_SCRATCH):
+        _C.check(_C.lib.lmx_op_gemm(_C.torch_dtype_code(DT[dt]), _C.ptr(x), _C.ptr(w), _C.ptr(out), None, _C.ptr(r), M, N, K, K, K, N, N + odd, 0, v, _C.stream_handle()), "gemm")
+        assert_one_ulp(out, ref, dt, 2e-5 * float(ref.abs().max()), f"{M}x{N}x{K} pitch {N + odd} variant {v}")
+
+
+@pytest.mark.gpu
 def test_refusals(cuda):
     from llava_mi355x import ops
     from llava_mi355x._C import LmxError

@@ -510,9 +510,10 @@ int lmx_op_gemm_form(int32_t dtype, int32_t M, int32_t N, int32_t K, int32_t act
         form[1] = f.rt; form[2] = M > 16 ? 2 : 1; form[3] = f.ks;
         return 0;
     }
-    const RowsForm f = gemm_rows_form(dtype, g);
-    if (f.mtiles) { form[0] = 1; form[1] = f.mtiles; form[2] = f.bn; form[3] = f.slices; }
-    else if (dtype != kF32) { const TileForm t = gemm4w_form(dtype, g); form[3] = t.mb ? t.slices : gemm_slices(g); }
+    const LinearForm f = linear_form(dtype, g);
+    form[3] = f.slices;
+    if (f.kernel == LinearForm::kRows) { form[0] = 1; form[1] = f.rows.mtiles; form[2] = f.rows.bn; }
+    else if (f.kernel == LinearForm::kTiles) { form[0] = 2; form[1] = f.tile.mb; form[2] = f.tile.nb; }
     LMX_API_END
 }
 int lmx_op_gemv(int32_t dtype, const void* x, const void* w, void* c, const void* bias, const void* residual, const void* norm_w, float eps,

@@ -682,28 +682,36 @@ int gemm_slices(const GemmArgs& a) {
     return s;
 }
 
+// Four waves' tiles (gemm4w.hip), row tiles (gemm_rows.hip), and of what is left of the large problems (up to 256 rows) the ping-pong 256x256x64 kernel (gemm8p.hip), K-sliced when its
+// tiles leave CUs idle and the caller brought the partial-tile scratch (the engine does, per sequence).  LMX_GEMM8P=0: the row tiles and the ring kernels alone, as an A/B and cross-check.
+LinearForm linear_form(int dtype, const GemmArgs& a) {
+    LinearForm f;
+    if (dtype != kBF16 && dtype != kF16) return f;
+    if (gemm8p_enabled()) {
+        f.tile = gemm4w_form(dtype, a);
+        if (f.tile.mb) { f.kernel = LinearForm::kTiles; f.slices = f.tile.slices; return f; }
+    }
+    f.rows = gemm_rows_form(dtype, a);
+    if (f.rows.mtiles) { f.kernel = LinearForm::kRows; f.slices = f.rows.slices; return f; }
+    if (a.c_f32 || !gemm8p_enabled()) return f;
+    const int S = gemm_slices(a);
+    if (cdiv(a.M, 256) * cdiv(a.N, 256) * S >= 160) { f.kernel = LinearForm::kPingPong; f.slices = S; }
+    return f;
+}
+
 template <typename T>
 static void launch_gemm16(const GemmArgs& a, int variant, hipStream_t st) {
     // variant: 0 = auto, 2 = 128x128 reg-staged (kept as an independent cross-check of the LDS-DMA path), 4 = 64x128 glds, 5 = 64x64 glds,
     //          7 / 9 = LDS-ring kernels with counted vmcnt (128x256x64 3-slot, 256x256x64 2-slot; 8 waves), 15 = 64x64 4-slot ring (4 waves),
     //          18 = 128x128x64 2-slot 4 waves.  (Round 5 removed the arms auto never picks: 1, 12, 14 and the deeper rings 23 - 26 of round 4, EXPERIMENTS.md r4-C.)
-    if (variant == 0 && gemm8p_enabled()) {                              // (LMX_GEMM8P=0: the ring kernels below as an A/B and cross-check)
-        const TileForm f = gemm4w_form(TypeInfo<T>::id, a);
-        if (f.mb) { launch_gemm4w(TypeInfo<T>::id, a, f, st); return; }
-    }
     if (variant == 0) {
-        const RowsForm f = gemm_rows_form(TypeInfo<T>::id, a);
-        if (f.mtiles) { launch_gemm_rows(TypeInfo<T>::id, a, f.mtiles, f.bn, f.slices, st); return; }
+        const LinearForm f = linear_form(TypeInfo<T>::id, a);
+        if (f.kernel == LinearForm::kTiles) { launch_gemm4w(TypeInfo<T>::id, a, f.tile, st); return; }
+        if (f.kernel == LinearForm::kRows) { launch_gemm_rows(TypeInfo<T>::id, a, f.rows.mtiles, f.rows.bn, f.rows.slices, st); return; }
+        if (f.kernel == LinearForm::kPingPong) { GemmArgs b = a; b.split_k = f.slices; launch_gemm8p(TypeInfo<T>::id, b, st); return; }
     }
     if (a.c_f32) { launch_gemm_cfg<T, 64, 128, 2, 2, true, true>(a, st); return; }      // fp32 logits of a few wanted rows: one tile form
     if (variant == 0) {
-        // What is left of the large problems (up to 256 rows): the ping-pong 256x256x64 kernel (gemm8p.hip), K-sliced when the tiles leave CUs idle and the caller brought
-        // the partial-tile scratch (the engine does, per sequence; LMX_GEMM8P=0 switches the kernel off).
-        if (gemm8p_enabled()) {
-            const int tiles = cdiv(a.M, 256) * cdiv(a.N, 256);
-            const int S = gemm_slices(a);
-            if (tiles * S >= 160) { GemmArgs b = a; b.split_k = S; launch_gemm8p(TypeInfo<T>::id, b, st); return; }
-        }
         // Tile choice from the round-1 microbenchmarks (profiles/r01_microbench.jsonl).  The pipelined ring kernels are
         // bound by L2->LDS bandwidth (~12 TB/s), so the biggest tile that still fills the chip wins; when even 128-row
         // tiles cannot give every CU work (CLIP-sized problems) fall back to the small-tile kernels.

@@ -60,6 +60,13 @@ void launch_gemm4w(int dtype, GemmArgs a, TileForm f, hipStream_t st);
 bool gemm_rows_applies(int dtype, const GemmArgs& a);
 struct RowsForm { int mtiles, bn, slices; };
 RowsForm gemm_rows_form(int dtype, const GemmArgs& a);                // the form variant 0 takes (mtiles 0: another kernel)
+// what launch_gemm takes for variant 0
+struct LinearForm {
+    enum Kernel { kRing = 0, kRows = 1, kTiles = 2, kPingPong = 3 } kernel = kRing;
+    TileForm tile{0, 0, 1}; RowsForm rows{0, 0, 1};
+    int slices = 1;
+};
+LinearForm linear_form(int dtype, const GemmArgs& a);
 size_t gemm_rows_slab_bytes(int M, int N, int S);
 void launch_gemm_rows(int dtype, const GemmArgs& a, int mtiles, int BN, int S, hipStream_t st);
 // decode-batch linear (skinny.hip): M <= 32 rows, 16-bit, weights streamed once straight into MFMA operands; variant 20 of launch_gemm

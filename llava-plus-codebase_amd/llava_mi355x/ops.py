@@ -43,7 +43,7 @@ def gemm(x, w, bias=None, residual=None, act=_C.ACT_NONE, variant=0, out=None):
 
 
 def gemm_form(dtype, M, N, K, act=_C.ACT_NONE, scratch_bytes=64 << 20, batch=False):
-    """The form that the rules of the row-tile kernel, else the K slices (batch: those of the decode batch's linears) have for such a product and scratch, as lmx_op_gemm_form describes it.  No GPU needed."""
+    """What launch_gemm (batch: the decode batch's linears) takes for such a product and scratch, as lmx_op_gemm_form describes it.  No GPU needed."""
     form = (ctypes.c_int32 * 4)()
     check(lib.lmx_op_gemm_form(torch_dtype_code(dtype), M, N, K, act, scratch_bytes, int(batch), form), "gemm_form")
     return tuple(form)

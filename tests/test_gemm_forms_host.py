@@ -36,8 +36,12 @@ def test_slices_of_a_decode_batch_fit_the_scratch(M, N, K):
 
 # rows, weights, K: where a row-tile form measured at least a twentieth slower / faster than the other kernels
 OTHERS = [(257, 3072, 2048, 0), (300, 3072, 3072, 0), (128, 4096, 2048, 0), (256, 8192, 1536, 0), (96, 6656, 4096, 0), (257, 2560, 5120, 0), (258, 9792, 7296, 0), (183, 18176, 7744, 0), (2048, 4096, 2048, 0), (2308, 3072, 1024, 0), (33, 10240, 2048, 0)]
-ROW_TILES = [(20, 4096, 11008, 0), (64, 3072, 2048, 0), (139, 12288, 4096, 0), (139, 22016, 4096, 3), (251, 11456, 2304, 0), (257, 4096, 4096, 0), (384, 5120, 13824, 0), (484, 14720, 2816, 0),
-             (512, 16384, 3072, 3), (500, 12288, 4096, 0), (500, 15360, 5120, 0), (250, 27648, 5120, 3), (257, 6208, 2048, 0), (600, 4096, 4096, 0), (1087, 4096, 2048, 0), (2048, 3072, 2048, 0), (2308, 1024, 4096, 0), (25, 26816, 1216, 0), (11, 18048, 4224, 0)]
+ROW_TILES = [(20, 4096, 11008, 0), (64, 3072, 2048, 0), (139, 12288, 4096, 0), (139, 22016, 4096, 3), (251, 11456, 2304, 0), (257, 4096, 4096, 0), (384, 5120, 13824, 0), (250, 27648, 5120, 3), (257, 6208, 2048, 0), (600, 4096, 4096, 0), (2308, 1024, 4096, 0), (25, 26816, 1216, 0), (11, 18048, 4224, 0)]
+
+
+# past 256 rows and 640 tiles of 64 x 64, where the four-wave tiles measured faster than both: mb, nb, K slices
+FOUR_WAVES = {(484, 14720, 2816, 0): (6, 6, 1), (512, 16384, 3072, 3): (8, 6, 1), (500, 12288, 4096, 0): (5, 6, 1), (500, 15360, 5120, 0): (6, 6, 1), (1087, 4096, 2048, 0): (5, 4, 1),
+              (2048, 3072, 2048, 0): (5, 6, 1), (1087, 4096, 11008, 0): (7, 8, 3), (258, 9792, 7296, 0): (5, 8, 3)}
 
 
 @pytest.mark.parametrize("case", OTHERS + ROW_TILES)
@@ -45,6 +49,20 @@ def test_the_faster_kernel(case):
     from llava_mi355x import ops
     M, N, K, act = case
     assert (ops.gemm_form(torch.bfloat16, M, N, K, act=act)[0] == 1) == (case in ROW_TILES)
+
+
+@pytest.mark.parametrize("case", list(FOUR_WAVES))
+def test_four_wave_tiles(case):
+    from llava_mi355x import ops
+    M, N, K, act = case
+    assert ops.gemm_form(torch.bfloat16, M, N, K, act=act) == (2,) + FOUR_WAVES[case]
+
+
+@pytest.mark.parametrize("M,N", [(256, 12288), (257, 8192), (257, 8256), (640, 4096), (641, 4096)])
+def test_the_line_of_the_four_wave_tiles(M, N):
+    """256 rows, 640 tiles of 64 x 64: on the line another kernel, past it the four-wave tiles."""
+    from llava_mi355x import ops
+    assert (ops.gemm_form(torch.float16, M, N, 2048)[0] == 2) == ((M, N) in ((257, 8256), (641, 4096)))
 
 
 @pytest.mark.parametrize("M,N,K,act,rt", [(2, 15360, 5120, 0, 1), (8, 12288, 4096, 0, 1), (8, 32000, 4096, 0, 1), (9, 12288, 4096, 0, 4), (32, 15360, 5120, 0, 4), (8, 22016, 4096, 3, 2),

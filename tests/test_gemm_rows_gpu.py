@@ -46,10 +46,13 @@ def test_epilogues(cuda, variant, act):
 
 
 @pytest.mark.parametrize("M,N,K,res", [(385, 2048, 2048, False), (577, 4096, 1024, False), (640, 2112, 4096, True), (1087, 4096, 4096, True), (1087, 4096, 4160, True), (2308, 1024, 1024, True),
-                                       (2679, 1280, 2048, False), (4616, 1024, 1024, False), (1153, 1024, 2048, True)])
+                                       (2679, 1280, 2048, False), (4616, 1024, 1024, False), (1153, 1024, 2048, True), (600, 4096, 4096, True), (2308, 1024, 4096, False), (1200, 2048, 2048, True),
+                                       (257, 6208, 2048, False)])
 def test_one_round_of_tiles(cuda, M, N, K, res):
-    """The other part of the rule: row tiles of a height that makes one round of workgroups."""
+    """The other part of the rule: row tiles of a height that makes one round of workgroups, and both sides of its lines: small tiles below, four-wave tiles past 640 tiles of 64 x 64."""
     from llava_mi355x import ops
+    form = ops.gemm_form(torch.bfloat16, M, N, K, scratch_bytes=0)
+    assert form[0] == {(385, 2048): 0, (1153, 1024): 0, (1087, 4096): 2, (2679, 1280): 2, (4616, 1024): 2}.get((M, N), 1) and (form[0] != 1 or form[1] > 1)
     x, w = _mk(M, N, K, "bf16", cuda, M + N)
     r = torch.randn(M, N, device=cuda).bfloat16() if res else None
     ref = x.double() @ w.double().t() + (r.double() if res else 0)
@@ -57,9 +60,10 @@ def test_one_round_of_tiles(cuda, M, N, K, res):
 
 
 @pytest.mark.parametrize("M", [2, 32, 128, 129, 256, 257, 384, 385, 512, 513])
-@pytest.mark.parametrize("N,K,ldc", [(12288, 1024, 12288), (22016, 1024, 22016), (12288, 1024, 12292)])
+@pytest.mark.parametrize("N,K,ldc", [(12288, 1024, 12288), (22016, 1024, 22016), (12288, 1024, 12292), (4096, 4096, 4096)])
 def test_rule(cuda, M, N, K, ldc):
-    """What variant 0 takes, on both sides of every line of the rule and with rows that are not 16-byte aligned (another kernel's)."""
+    """What variant 0 takes, on both sides of every line of the rule (past 256 rows: of the width that the four-wave tiles leave to it) and with rows that are not 16-byte aligned
+    (another kernel's)."""
     from llava_mi355x import ops
     x, w = _mk(M, N, K, "bf16", cuda, M)
     out = torch.zeros(M, ldc, device=cuda, dtype=DT["bf16"])

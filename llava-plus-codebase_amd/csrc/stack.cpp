@@ -526,7 +526,7 @@ void Model::stack_prefill(Seq* const* seqs, const void* const* embeds, const int
                 launch_gather_rows(dt, x, want, list, nr, H, st);
                 GemmArgs ga{want, lm_head, dst, nullptr, nullptr, nr, V, H, H, H, V, 0, kActNone};
                 ga.c_f32 = 1; ga.cap = S.c.logit_softcap;
-                launch_gemm(dt, ga, gv, st);
+                launch_gemm(dt, ga, 0, st);                  // (its own choice, as the GEMV's: a tile by number, gv, need not have fp32 output)
             } else for (int i = 0; i < nr; ++i) {
                 GemvArgs ga{rows(x, e[i].dst0 + e[i].n - 1, H), lm_head, dst + (size_t)i * V, nullptr, nullptr, nullptr, 0.f, V, H, H, H, V, 0, kActNone};
                 ga.c_f32 = 1; ga.cap = S.c.logit_softcap;

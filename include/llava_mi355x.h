@@ -320,7 +320,7 @@ int lmx_op_rope_kv_rows(int32_t dtype, int32_t head_dim, void* qkv, void* kcache
                         int32_t T, int32_t n_heads, int32_t n_kv_heads, int32_t s_max, void* stream);
 /* q|k|v projection with RoPE + KV-cache append in the GEMM's epilogue (gemm4w.h: qkv_rope_epilogue4; what Model::prefill launches where
  * the shape allows it): qkv[:, :n_heads*D] <- rotated q, kcache / vtcache rows pos0 .. pos0 + T - 1 <- rotated k / v; the k | v columns of `qkv` are
- * left untouched.  Fails when the shape does not take the fused launch (same rule as the engine: un-split ping-pong GEMM, head-aligned tiles). */
+ * left untouched.  Fails when the shape does not take the fused launch (same rule as the engine: 160 tiles of 256 x 256, head-aligned; no K slices). */
 int lmx_op_gemm_qkv_rope(int32_t dtype, int32_t head_dim, const void* x, const void* w, void* qkv, void* kcache, void* vtcache, const float* cos_sin_dev,
                          int32_t pos0, int32_t T, int32_t K, int32_t n_heads, int32_t n_kv_heads, int32_t s_max, void* stream);
 int lmx_op_flash_attn(int32_t dtype, int32_t head_dim, const void* q, void* o, const void* kcache, const void* vtcache,

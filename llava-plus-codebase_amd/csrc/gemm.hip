@@ -760,17 +760,18 @@ bool gemm_fuses_qkv(int dtype, int M, int K, int D, int nh, int nkv, int pos0, i
     if (!gemm8p_enabled() || has_bias || M <= 0 || K % 64 != 0 || !(D == 64 || D == 128) || (nh * D) % 256 != 0 || (nkv * D) % 256 != 0 || pos0 % 8 != 0 || s_max % 8 != 0)
         return false;
     if (cdiv(M, 256) * cdiv(N, 256) < 160 || gemm8p_pick_split(M, N, K) != 1) return false;
-    // un-split in launch_gemm16's own choice, so that the fused launch adds the same products in the same order
+    // 160 tiles of 256 x 256 leave the four-wave kernel no K slices (gemm4w_form) and, up to 256 rows, the ping-pong kernel none either: the launch without the epilogue adds the same
+    // products in the same order
     void* const any = reinterpret_cast<void*>((uintptr_t)4096);
     GemmArgs g{any, any, any, nullptr, nullptr, M, N, K, K, K, N, 0, kActNone};
-    g.scratch(any, (size_t)64 << 20);
-    return gemm4w_form(dtype, g).slices == 1;
+    g.qf_kc = any; g.qf_D = D;
+    return gemm4w_form(dtype, g).mb != 0;
 }
 
 void launch_gemm(int dtype, const GemmArgs& a, int variant, hipStream_t st) {
     LMX_REQUIRE(a.M > 0 && a.N > 0 && a.K > 0, "gemm: empty problem");
     if (a.qf_kc) LMX_REQUIRE(variant == 0 && gemm_fuses_qkv(dtype, a.M, a.K, a.qf_D, a.qf_nh, a.qf_nkv, a.qf_pos0, a.qf_smax, a.bias != nullptr),
-                             "gemm: the fused q|k|v epilogue needs the un-split ping-pong launch (gemm_fuses_qkv)");
+                             "gemm: this shape does not take the q|k|v epilogue (gemm_fuses_qkv)");
     if (variant == 20) { launch_skinny_gemm(dtype, a, st); return; }
     if (variant >= 100 && variant < 1000) { launch_gemm4w(dtype, a, TileForm{variant / 100, variant / 10 % 10, variant % 10}, st); return; }
     // 30: ping-pong kernel, K slices chosen by gemm8p_pick_split; 33 / 34 / 35: 2 / 3 / 1 slices forced

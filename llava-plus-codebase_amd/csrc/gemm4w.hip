@@ -125,7 +125,7 @@ TileForm gemm4w_form(int dtype, const GemmArgs& a) {
     if ((dtype != kBF16 && dtype != kF16) || a.c_f32 || a.K % 64 != 0 || a.N % 8 != 0 || (act_gated(a.act) && a.N % 64 != 0) || (a.pk_kc && a.pk_D % 8 != 0)) return none;
     if (a.R && a.ldr % 4 != 0) return none;                  // residual rows of any pitch: another kernel's
     if ((size_t)a.M * a.ldx * 2 >= ((size_t)1 << 32) || (size_t)a.N * a.ldw * 2 >= ((size_t)1 << 32)) return none;
-    if (a.M <= 256 || (int64_t)cdiv(a.M, 64) * cdiv(a.N, 64) <= 640) return none;
+    if (!a.qf_kc && (a.M <= 256 || (int64_t)cdiv(a.M, 64) * cdiv(a.N, 64) <= 640)) return none;      // (the q|k|v epilogue is here alone: gemm_fuses_qkv's lines)
     TileForm best = none;
     float least = 0.f;
     for (const Tile& t : kTiles) {

@@ -68,119 +68,6 @@ __device__ __forceinline__ v4i_t make_rsrc(const void* p, uint32_t bytes) {
 
 }  // namespace
 
-// ---------------------------------------------------------------------------------------------------------------------------
-// q|k|v epilogue with RoPE + KV-cache append (GemmArgs::qf_*).  The 256 x 256 tile covers whole heads of ONE of the three regions (the launcher checks the
-// alignment).  It is rounded to T — the rounding point of the unfused path, where the GEMM stores T and rope_kv_kernel reads it back — into the LDS the
-// operand ring no longer needs (256 x 264 elements), then leaves row-wise:
-//   q / k tile: LDS image [row][col]; work item = (row, head, group of 8 rotation pairs): x1 = cols d .. d + 7, x2 = cols d + D/2 ..; cos / sin of the row's
-//               position from the fp32 table, rounded to T; out = T( T(x cos) + T(rot(x) sin) ) as rope_kv_kernel; 16-byte stores into the q columns of C /
-//               the K-cache row of the position.
-//   v tile:     LDS image TRANSPOSED [col][row] (2-byte LDS writes: a lane owns one row), so that a work item (d, 8 consecutive positions) is one 16-byte
-//               LDS read and one 16-byte store into V^T[kv head][d][pos ..] (pos0 and the row group are multiples of 8).
-// ---------------------------------------------------------------------------------------------------------------------------
-constexpr int QF_PITCH = 264;                               // elements per LDS row (528 B: 16-byte aligned rows, 4-bank shift per row)
-constexpr int QF_LDS = 256 * QF_PITCH * 2;                  // bytes (16-bit T)
-
-template <typename T>
-__device__ __forceinline__ void qkv_rope_epilogue(const GemmArgs& a, f32x16 (&acc)[2][4], char* smem, int m0, int n0, int wm, int wn, int l31, int hi, int tid) {
-    T* tile = reinterpret_cast<T*>(smem);
-    const int D = a.qf_D, HALF = D >> 1;
-    const int q_cols = a.qf_nh * D, k_cols = a.qf_nkv * D;
-    const int region = n0 < q_cols ? 0 : (n0 < q_cols + k_cols ? 1 : 2);
-    __syncthreads();                                        // every wave has left the operand ring
-    if (region < 2) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const int row = wm * 128 + j * 32 + l31, col = wn * 64 + i * 32 + 8 * q + 4 * hi;
-                    uint2 u;
-                    u.x = pack2<T>(acc[i][j][4 * q], acc[i][j][4 * q + 1]); u.y = pack2<T>(acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]);
-                    *reinterpret_cast<uint2*>(tile + row * QF_PITCH + col) = u;
-                }
-        __syncthreads();
-        const int GPR = HALF >> 3, HPT = 256 / D;            // groups of 8 pairs per head row, heads per tile
-        // 256 x HPT x GPR = 4096 items, 8 per thread: item = tid + 512 it -> the same pair group g and head hh every time, rows 32 apart.  The cos / sin
-        // values of four rows at a time are requested BEFORE the batch's first store (round 4): in the one-item-at-a-time loop every item's table loads waited behind
-        // the previous item's stores (possible aliasing), eight dependent L2 round trips = ~10 us at the tail of every q|k|v workgroup.
-        constexpr int NIT = 4;                               // items per batch (two batches: 64 registers of table values at a time)
-        const int g = tid % GPR, hh = (tid / GPR) % HPT, i0 = g * 8;
-        const int rstep = 512 / (GPR * HPT);                 // 32
-#pragma unroll 1
-        for (int half = 0; half < 2; ++half) {
-        const int r0 = tid / (GPR * HPT) + half * NIT * rstep;
-        f32x4 cs4[NIT][4];
-#pragma unroll
-        for (int it = 0; it < NIT; ++it) {
-            int m = m0 + r0 + it * rstep; m = m < a.M ? m : a.M - 1;
-            const float* cs = a.qf_rope + (size_t)(a.qf_pos0 + m) * D;
-            cs4[it][0] = *reinterpret_cast<const f32x4*>(cs + i0); cs4[it][1] = *reinterpret_cast<const f32x4*>(cs + i0 + 4);
-            cs4[it][2] = *reinterpret_cast<const f32x4*>(cs + HALF + i0); cs4[it][3] = *reinterpret_cast<const f32x4*>(cs + HALF + i0 + 4);
-        }
-#pragma unroll
-        for (int it = 0; it < NIT; ++it) {
-            const int r = r0 + it * rstep;
-            const int m = m0 + r;
-            if (m >= a.M) continue;
-            const int pos = a.qf_pos0 + m;
-            float x1[8], x2[8], o1[8], o2[8];
-            load8<T>(tile + r * QF_PITCH + hh * D + i0, x1);
-            load8<T>(tile + r * QF_PITCH + hh * D + HALF + i0, x2);
-            const float cv[8] = {cs4[it][0].x, cs4[it][0].y, cs4[it][0].z, cs4[it][0].w, cs4[it][1].x, cs4[it][1].y, cs4[it][1].z, cs4[it][1].w};
-            const float sv[8] = {cs4[it][2].x, cs4[it][2].y, cs4[it][2].z, cs4[it][2].w, cs4[it][3].x, cs4[it][3].y, cs4[it][3].z, cs4[it][3].w};
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const float c = round_to<T>(cv[e]), sn = round_to<T>(sv[e]);
-                o1[e] = rope_term<T>(x1[e], c, -x2[e], sn);
-                o2[e] = rope_term<T>(x2[e], c, x1[e], sn);
-            }
-            T* dst;
-            if (region == 0) dst = reinterpret_cast<T*>(a.C) + (size_t)m * a.ldc + n0 + hh * D;
-            else dst = reinterpret_cast<T*>(a.qf_kc) + ((size_t)((n0 - q_cols) / D + hh) * a.qf_smax + pos) * D;
-            store8<T>(dst + i0, o1);
-            store8<T>(dst + HALF + i0, o2);
-        }
-        }
-    } else {
-        uint16_t* tt = reinterpret_cast<uint16_t*>(smem);     // [col][row]
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int row = wm * 128 + j * 32 + l31, col = wn * 64 + i * 32 + 8 * (r >> 2) + 4 * hi + (r & 3);
-                    tt[col * QF_PITCH + row] = (uint16_t)(pack2<T>(acc[i][j][r], 0.f) & 0xffffu);      // the conversion gemm_epilogue's store4 uses
-                }
-        __syncthreads();
-        T* vt = reinterpret_cast<T*>(a.qf_vt);
-        const int kvh0 = (n0 - q_cols - k_cols) / D;
-        for (int item = tid; item < 256 * 32; item += 512) {
-            const int rg = item & 31, c = item >> 5;
-            const int m = m0 + rg * 8;
-            if (m >= a.M) continue;
-            T* dst = vt + ((size_t)(kvh0 + c / D) * D + (c % D)) * a.qf_smax + a.qf_pos0 + m;
-            const uint4 v = *reinterpret_cast<const uint4*>(tt + c * QF_PITCH + rg * 8);
-            if (m + 8 <= a.M) *reinterpret_cast<uint4*>(dst) = v;
-            else {
-#pragma unroll
-                for (int k = 0; k < 8; ++k) {                   // the last, partial row group of the prompt
-                    const uint32_t wk = k < 2 ? v.x : (k < 4 ? v.y : (k < 6 ? v.z : v.w));
-                    if (m + k < a.M) reinterpret_cast<uint16_t*>(dst)[k] = (uint16_t)((k & 1) ? (wk >> 16) : (wk & 0xffffu));
-                }
-            }
-        }
-        if (m0 + 256 >= a.M) {                                  // V^T behind the last row: cleared to the end of its 64 keys, as rope_kv_kernel does
-            const int end = a.qf_pos0 + a.M, whole = (end + 63) & ~63, pos = end + (tid & 63);
-            if (pos < (whole < a.qf_smax ? whole : a.qf_smax))
-                for (int c = tid >> 6; c < 256; c += 8)
-                    reinterpret_cast<uint16_t*>(vt)[((size_t)(kvh0 + c / D) * D + (c % D)) * a.qf_smax + pos] = 0;
-        }
-    }
-}
-
 // SPLIT: K slices per tile (1, 2 or 3).  A K-sliced workgroup stores its fp32 partial tile and exits; the kernel boundary publishes the slabs and
 // splitk_reduce_rows_kernel / splitk_reduce_kernel sum them (launch-boundary split-K, EXPERIMENTS.md r3-E).  The in-launch reduction by the last arriver, the
 // tail-split / M-tail tile orders and the fused-RMSNorm reductions of rounds 2 - 4 measured slower or equal and were removed in round 5 (EXPERIMENTS.md r2-I,
@@ -396,7 +283,6 @@ __global__ __launch_bounds__(512) void gemm8p_kernel(GemmArgs a) {
     const int m_base = mw, n_base = n0 + wn * 64;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     if constexpr (SPLIT == 1) {
-        if (a.qf_kc) { qkv_rope_epilogue<T>(a, acc, smem, m0, n0, wm, wn, l31, hi, tid); return; }
         // (the operand ring is dead: every half-tile has landed and been read before the balancing barrier)
         gemm_epilogue<T, 4, 2>(a, acc, m_base, n_base, lane, smem + wave * epilogue_wave_bytes<2>());
     } else {
@@ -614,18 +500,15 @@ static void launch_gemm8p_t(GemmArgs a, hipStream_t st) {
         {
             std::lock_guard<std::mutex> lk(mu);
             if (!done.count(reinterpret_cast<const void*>(kern))) {
-                LMX_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, QF_LDS > P8_LDS ? QF_LDS : P8_LDS));
+                LMX_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, P8_LDS));
                 done.insert(reinterpret_cast<const void*>(kern));
             }
         }
-        const int lds = a.qf_kc ? (QF_LDS > P8_LDS ? QF_LDS : P8_LDS) : P8_LDS;
-        if (two && timed) { kt->used = true; hipExtLaunchKernelGGL(kern, dim3(tiles * S), dim3(512), lds, st, kt->e0, nullptr, 0, a); }
-        else LMX_LAUNCH(kern, dim3(tiles * S), dim3(512), lds, st, a);
+        if (two && timed) { kt->used = true; hipExtLaunchKernelGGL(kern, dim3(tiles * S), dim3(512), P8_LDS, st, kt->e0, nullptr, 0, a); }
+        else LMX_LAUNCH(kern, dim3(tiles * S), dim3(512), P8_LDS, st, a);
         LMX_CHECK_HIP(hipGetLastError());
     };
-    if (a.qf_kc) LMX_REQUIRE(S == 1 && a.qf_rope && a.qf_vt && (a.qf_D == 64 || a.qf_D == 128) && (a.qf_nh * a.qf_D) % 256 == 0 &&
-                             (a.qf_nkv * a.qf_D) % 256 == 0 && a.N == (a.qf_nh + 2 * a.qf_nkv) * a.qf_D && a.qf_pos0 % 8 == 0 && a.qf_smax % 8 == 0 && !a.bias && !a.R &&
-                             a.act == kActNone && a.ldc % 8 == 0, "gemm8p: the fused q|k|v epilogue needs an un-split launch over head-aligned tiles (gemm_fuses_qkv)");
+    LMX_REQUIRE(!a.qf_kc, "gemm8p: the q|k|v epilogue is the four-wave kernel's");
     // the CLIP K / V^T pack lives in gemm_epilogue only: the K-sliced launches' reduction kernels would write the k | v columns to C and leave the pack untouched
     if (a.pk_kc) LMX_REQUIRE(S == 1 && !act_gated(a.act) && a.pk_D % 4 == 0, "gemm8p: the K / V^T pack epilogue needs an un-split launch of a plain linear");
     if (S == 3) launch(gemm8p_kernel<T, 3>);

@@ -1,9 +1,9 @@
-"""RoPE + KV-cache append in the q|k|v GEMM's epilogue (csrc/gemm8p.hip: qkv_rope_epilogue) against the two launches it replaces
+"""RoPE + KV-cache append in the q|k|v GEMM's epilogue (csrc/gemm4w.h: qkv_rope_epilogue4) against the two launches it replaces
 (launch_gemm + rope_kv_kernel).  Both are LlamaAttention's q_proj / k_proj / v_proj, apply_rotary_pos_emb and the cache update of a prefill
 (HF5:models/llama/modeling_llama.py:130-160, 243-281) with the same arithmetic and the same rounding points (the tile is rounded to the model dtype
 before the rotation, as a stored-and-reloaded q|k|v row would be), so logits and generated ids must be BIT-IDENTICAL — the ids also prove the caches:
 every decode step reads the K / V^T rows the prefill wrote.  7B and 13B widths, prompts whose last row group is partial (1087 = 135 x 8 + 7 rows),
-bf16 and fp16; a prompt too short for the ping-pong kernel and a chunk that starts at a position that is not a multiple of 8 keep the two launches."""
+bf16 and fp16; a prompt of too few tiles and a chunk that starts at a position that is not a multiple of 8 keep the two launches."""
 import pytest
 import torch
 
@@ -44,7 +44,7 @@ def test_shapes_that_keep_the_two_launches(cuda):
     cfg = synth.with_layers(synth.CONFIGS["llava15_7b"], 2, 1)
     model = harness.build_model(cfg, dtype=torch.bfloat16, seed=0, device_rng=True, max_position=2048)
     pix = torch.from_numpy(synth.make_pixels(cfg, 1, seed=1)).to(cuda, torch.bfloat16)
-    # 40 + 575 rows: too few 256 x 256 tiles for the ping-pong kernel
+    # 40 + 575 rows: too few 256 x 256 tiles
     ids = torch.from_numpy(synth.make_prompt(cfg, 40, image_positions=(5,), seed=3))[None].to(cuda)
     _, _, names = _run(model, ids, pix, True, n_new=2)
     assert "prefill.rope_kv" in names
@@ -57,10 +57,11 @@ def test_shapes_that_keep_the_two_launches(cuda):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("D,nh,nkv,T,pos0", [(128, 32, 32, 1087, 0), (128, 16, 16, 2000, 40), (64, 64, 16, 2000, 8)])
+@pytest.mark.parametrize("D,nh,nkv,T,pos0", [(128, 32, 32, 1087, 0), (128, 16, 16, 2000, 40), (64, 64, 16, 2000, 8), (128, 32, 32, 1200, 8), (64, 64, 64, 1253, 16), (128, 40, 40, 1087, 0),
+                                             (128, 128, 96, 200, 8), (128, 128, 96, 256, 0)])
 def test_fused_projection_op_equals_gemm_then_rope_kv(cuda, dtype, D, nh, nkv, T, pos0):
     """The two forms on the same operands: rotated q, the K-cache rows and the V^T columns must be the same BITS (GQA head_dim 64 included: four heads per
-    tile, rotation partner inside the wave's own 64 columns)."""
+    tile, rotation partner inside the wave's own 64 columns).  Tiles of 7, 8 and 5 x 8 blocks; up to 256 rows the launch without the epilogue is the ping-pong kernel's."""
     from llava_mi355x import ops
     from test_ops_gpu import _rope_table
     torch.manual_seed(3)

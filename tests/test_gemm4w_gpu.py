@@ -74,6 +74,32 @@ def test_gated(cuda, form, M):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("act", [0, 1, 2, 3, 4])
+def test_three_slices(cuda, form, act):
+    """Seven K-steps in slices of 2, 2 and 3 (one, one and two pairs): bias, activations, gating with a bias, the residual; row and column tails.  Against the un-sliced tiles' bound."""
+    from llava_mi355x import _C, ops
+    M, N, K = 290, 448, 448
+    x, w = _mk(M, N, K, "bf16", cuda, act + form)
+    b = torch.randn(N, device=cuda).bfloat16()
+    y = x.double() @ w.double().t() + b.double()
+    v = 10 * form + 3
+    if act >= 3:
+        y = y.view(M, N // 64, 2, 32)
+        ref = ((torch.nn.functional.silu(y[:, :, 0]) if act == _C.ACT_SILU_MUL else torch.relu(y[:, :, 0])) * y[:, :, 1]).reshape(M, N // 2)
+        got = ops.gemm(x, w, bias=b, act=act, variant=v, out=torch.empty(M, N // 2, device=cuda, dtype=torch.bfloat16))
+        assert_one_ulp(got, ref, "bf16", 6e-5 * float(ref.abs().max()), f"variant {v} act {act}")
+        return
+    y = y * torch.sigmoid(1.702 * y) if act == 1 else torch.nn.functional.gelu(y) if act == 2 else y
+    r = torch.randn(M, N, device=cuda).bfloat16()
+    ref = y + r.double()
+    got = ops.gemm(x, w, bias=b, residual=r, act=act, variant=v)
+    assert_one_ulp(got, ref, "bf16", 3e-5 * float(ref.abs().max()), f"variant {v} act {act}")
+    ops.gemm(x, w, bias=b, residual=r, act=act, variant=v, out=r)        # in place
+    assert torch.equal(r, got)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K,act", [(257, 10304, 1024, 0), (513, 4672, 640, 1), (700, 3072, 1024, 0), (1087, 4096, 4096, 0), (1087, 22016, 1024, 3), (2048, 2048, 5632, 0), (2679, 6400, 2048, 0), (6528, 4096, 1088, 0)])
 def test_choice(cuda, M, N, K, act):
     """What variant 0 and a prefill's call take, on the large side of the rule's lines."""

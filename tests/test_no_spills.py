@@ -1,6 +1,7 @@
-"""The prefill GEMM's hot instantiations must stay free of scratch (register spills): gemm8p_kernel sits at 251 of 256 VGPRs, and a few more live values in a
+"""The prefill GEMMs' hot instantiations must stay free of scratch (register spills): gemm4w_kernel keeps up to 256 accumulators and 217 other registers a lane at one wave a SIMD,
+gemm8p_kernel sits at 251 of 256 VGPRs, and a few more live values in a
 rarely taken branch once doubled the whole prefill (round 4: a runtime `skip X half 1` flag in the ragged loop -> 88 bytes of spills per lane -> ragged tiles
-took two tile-times).  hipcc reports the numbers at compile time; this test recompiles the one file (~1 min, no GPU needed)."""
+took two tile-times).  hipcc reports the numbers at compile time; these tests recompile the files (~1 min, no GPU needed)."""
 import os
 import re
 import shutil
@@ -10,6 +11,24 @@ import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CSRC = os.path.join(ROOT, "llava-plus-codebase_amd", "csrc")
+
+
+def scratch_sizes(source, tmp_path):
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    r = subprocess.run([hipcc, "-O3", "-std=c++17", "-fPIC", "--offload-arch=gfx950", "-I.", "-I../../include",
+                        "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-c", source, "-o", str(tmp_path / "g.o"),
+                        "-Rpass-analysis=kernel-resource-usage"], cwd=CSRC, capture_output=True, text=True, timeout=900)
+    assert r.returncode == 0, r.stderr[-2000:]
+    return {m[1]: int(m[2]) for m in re.finditer(r"Function Name: (\S+).*?ScratchSize \[bytes/lane\]: (\d+)", r.stderr, re.S)}
+
+
+@pytest.mark.skipif(shutil.which("hipcc") is None and not os.path.exists("/opt/rocm/bin/hipcc"), reason="hipcc not available")
+@pytest.mark.parametrize("source,tiles", [("gemm4w_large_bf16.hip", 4), ("gemm4w_small_f16.hip", 6)])
+def test_four_wave_tiles_have_no_scratch(tmp_path, source, tiles):
+    """Each tile un-sliced, sliced and grouped, and its reductions of two and three slices."""
+    usage = scratch_sizes(source, tmp_path)
+    assert len([k for k in usage if "gemm4w" in k]) == 5 * tiles, sorted(usage)
+    assert not {k: v for k, v in usage.items() if v}, usage
 
 
 @pytest.mark.skipif(shutil.which("hipcc") is None and not os.path.exists("/opt/rocm/bin/hipcc"), reason="hipcc not available")

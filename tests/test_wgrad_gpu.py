@@ -155,11 +155,11 @@ def test_transpose_padded_is_exact(cuda, rows, cols, dtype):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("rows,H", [(1, 4096), (16, 4096), (129, 4096), (200, 2048), (640, 1024), (2048, 4096), (37, 512)])
 @pytest.mark.parametrize("with_res", [False, True])
-def test_rmsnorm_bwd_one_pass_form(cuda, rows, H, dtype, with_res):
-    """lmx_op_rmsnorm_bwd / lmx_op_rmsnorm_bwd_add (csrc/train.hip rmsnorm_bwd_fused_kernel for 16-bit rows of 1024 / 2048 / 4096; H = 512: the three-launch form)
-    against the fp64 formula of LlamaRMSNorm's autograd (HF5:models/llama/modeling_llama.py:53-67) on the 16-bit inputs:
+def test_rmsnorm_bwd_of_few_rows(cuda, rows, H, dtype, with_res):
+    """lmx_op_rmsnorm_bwd / lmx_op_rmsnorm_bwd_add (csrc/train.hip rmsnorm_bwd_fused_kernel, a wave a row, and rmsnorm_bwd_dw_part8_kernel for 16-bit rows of 1024 / 2048 / 4096;
+    H = 512: the three-launch form) against the fp64 formula of LlamaRMSNorm's autograd (HF5:models/llama/modeling_llama.py:53-67) on the 16-bit inputs:
         inv = rsqrt(mean(x^2) + eps), xhat = x inv, g = dy w, dx = inv (g - xhat mean(g xhat)), dw = sum_rows dy xhat;   with a residual: dx = T(res + T(dx)).
-    Row counts that are not multiples of the 16 rows a wave walks or the 128 a workgroup owns; dx-only calls (no dw) too."""
+    Row counts that are not multiples of the 8 rows of a workgroup or the 128 of a partial row of dw; dx-only calls (no dw) too."""
     ops = _ops()
     eps = 1e-5
     x = _rand((rows, H), dtype, cuda, 11, 1.3); dy = _rand((rows, H), dtype, cuda, 12, 0.7)
@@ -186,29 +186,43 @@ def test_rmsnorm_bwd_one_pass_form(cuda, rows, H, dtype, with_res):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("rows", [18304, 18305])
-def test_rmsnorm_bwd_on_both_sides_of_its_line(cuda, rows, dtype):
-    """143 blocks of 128 rows: dx by a wave a row, dw in a second pass; 144: both in one pass.  A term of dw passes at
+@pytest.mark.parametrize("H,with_res", [(1024, False), (2048, True), (4096, False), (4096, True)])
+def test_rmsnorm_bwd_on_both_sides_of_its_line(cuda, rows, H, with_res, dtype):
+    """143 blocks of 128 rows: dx by a wave a row, dw in a second pass; 144, the last of one row: both in one pass of a wave over 16 rows.  A term of dw passes at
     most 16 + 8 + 144 additions, three products and the rounding of rsqrt: under 180 fp32 roundings of the sum of magnitudes."""
     ops = _ops()
-    x, dy, w = _rand((rows, 1024), dtype, cuda, 21), _rand((rows, 1024), dtype, cuda, 22), (1 + 0.1 * _rand((1024,), torch.float32, cuda, 23)).to(dtype)
-    dx, dw = ops.rmsnorm_bwd(x, w, dy, 1e-5)
-    inv = torch.rsqrt(x.double().pow(2).mean(-1, keepdim=True) + 1e-5)
-    xh, g = x.double() * inv, dy.double() * w.double()
-    dx_ref, dw_ref = inv * (g - xh * (g * xh).mean(-1, keepdim=True)), (dy.double() * xh).sum(0)
-    assert (dx.double() - dx_ref).abs().max().item() <= 1.01 * (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11) * dx_ref.abs().max().item()
-    assert bool(((dw.double() - dw_ref).abs() <= 180 * 2.0 ** -24 * (dy.double() * xh).abs().sum(0)).all())
+    x, dy, w = _rand((rows, H), dtype, cuda, 21), _rand((rows, H), dtype, cuda, 22), (1 + 0.1 * _rand((H,), torch.float32, cuda, 23)).to(dtype)
+    res = _rand((rows, H), dtype, cuda, 24) if with_res else None
+    dx, dw = ops.rmsnorm_bwd(x, w, dy, 1e-5, residual=res)
+    ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    dw_ref, mag = torch.zeros(H, dtype=torch.float64, device=cuda), torch.zeros(H, dtype=torch.float64, device=cuda)
+    for a in range(0, rows, 4096):
+        b = min(a + 4096, rows)
+        inv = torch.rsqrt(x[a:b].double().pow(2).mean(-1, keepdim=True) + 1e-5)
+        xh, g = x[a:b].double() * inv, dy[a:b].double() * w.double()
+        want = inv * (g - xh * (g * xh).mean(-1, keepdim=True))
+        if with_res:
+            want = res[a:b].double() + want.to(dtype).double()
+        assert (dx[a:b].double() - want).abs().max().item() <= (2 if with_res else 1.01) * ulp * want.abs().max().item()
+        dw_ref += (dy[a:b].double() * xh).sum(0)
+        mag += (dy[a:b].double() * xh).abs().sum(0)
+    assert bool(((dw.double() - dw_ref).abs() <= 180 * 2.0 ** -24 * mag).all())
+    only, none = ops.rmsnorm_bwd(x, w, dy, 1e-5, want_dw=False, residual=res)
+    again, dw2 = ops.rmsnorm_bwd(x, w, dy, 1e-5, residual=res)
+    assert none is None and torch.equal(only, dx) and torch.equal(again, dx) and torch.equal(dw2, dw)      # deterministic: partial rows are added in a fixed order
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("H", [1024, 2048, 4096])
 @pytest.mark.parametrize("over", ["x", "dy"])
 @pytest.mark.parametrize("with_res", [False, True])
-def test_rmsnorm_bwd_over_one_of_its_inputs(cuda, over, H, dtype, with_res):
+@pytest.mark.parametrize("rows", [1, 200, 256])
+def test_rmsnorm_bwd_over_one_of_its_inputs(cuda, rows, over, H, dtype, with_res):
     """dx written over x or dy, row counts far below the one-pass line: dx has the bits of a call with a buffer of its own, dw is the float64 sum over what x and dy were.  A term of dw
-    passes at most 16 + 8 + 2 additions, three products and the rounding of rsqrt: under 32 fp32 roundings of the sum of magnitudes."""
+    passes at most 16 + 8 + 2 additions, three products and the rounding of rsqrt: under 32 fp32 roundings of the sum of magnitudes.  One row; rows that fill no wave's 16; whole blocks."""
     from llava_mi355x import _C
     ops = _ops()
-    rows, eps = 200, 1e-5
+    eps = 1e-5
     x, dy, w = _rand((rows, H), dtype, cuda, 31), _rand((rows, H), dtype, cuda, 32, 0.7), (1 + 0.1 * _rand((H,), torch.float32, cuda, 33)).to(dtype)
     res = _rand((rows, H), dtype, cuda, 34) if with_res else None
     want, _ = ops.rmsnorm_bwd(x, w, dy, eps, residual=res)

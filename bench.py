@@ -1238,14 +1238,12 @@ def main():
     n_gemm = sum(prof[k][1] for k in gemm_flops if k in prof)
     gt_k = gt
     mfma_busy, pmc_file = None, None
-    for cand in ("r06_pmc.json", "r05_pmc.json", "r04_pmc.json", "r03_pmc.json", "r02_pmc_gemm.json"):
-        try:
-            with open(os.path.join(ROOT, "profiles", cand)) as f:
-                mfma_busy = json.load(f).get("summary")
-            pmc_file = cand
-            break
-        except Exception:  # noqa: BLE001
-            continue
+    try:
+        with open(os.path.join(ROOT, "profiles", "gemm_prefill_counters.json")) as f:
+            mfma_busy = json.load(f)["kernels"]
+        pmc_file = "gemm_prefill_counters.json"
+    except Exception:  # noqa: BLE001
+        pass
     # HBM-side bytes per GEMM launch: PMC passes (FETCH_SIZE + WRITE_SIZE with the guide's gfx950 corrections) over the single-kernel drivers, committed digest
     gemm_traffic = None
     live_gemm = None
@@ -1257,8 +1255,8 @@ def main():
         per = {k: {"hbm_side_bytes": live_gemm[k], "algorithmic_bytes": algo[k], "ratio": live_gemm[k] / algo[k]} for k in algo}
         gemm_traffic = {"per_launch_avg_bytes": sum(v["hbm_side_bytes"] for v in per.values()) / len(per), "by_shape": per,
                         "how": "rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE, THIS run (tools/mb_gemm_prefill.py: the four shapes as the engine launches them); counted at the L2 -> fabric "
-                               "boundary, so Infinity-Cache hits are inside; o_proj / down_proj are K-sliced (3 slices): their figure includes the fp32 partial tiles written by the "
-                               "GEMM and read by the launch-boundary reduction; the rest above 1.0 is operand-tile re-reads that drift out of an XCD's 4 MB L2"}
+                               "boundary, so Infinity-Cache hits are inside; down_proj is K-sliced (3 slices): its figure includes the fp32 partial tiles written by the "
+                               "GEMM and read by the launch-boundary reduction; the rest above 1.0 is X, which each of the 8 XCDs' L2 reads (gate|up: in both rounds of its tiles)"}
     elif mfma_busy and world == 1 and a.model == "llava15_7b":
         algo = {"qkv": (T * H + 3 * H * H + T * 3 * H) * es, "o_proj": (T * H + H * H + 2 * T * H) * es, "gate_up": (T * H + 2 * H * I + T * I) * es,
                 "down": (T * I + H * I + 2 * T * H) * es}
@@ -1267,10 +1265,10 @@ def main():
         if per:
             gemm_traffic = {"per_launch_avg_bytes": sum(v["hbm_side_bytes"] for v in per.values()) / len(per), "by_shape": per,
                             "live_error": live_gemm,
-                            "how": f"profiles/{pmc_file} (rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE passes of tools/gpu_pmc_r3.sh over the single-shape drivers; committed digest, not "
-                                   "re-measured in this run); counted at the L2 -> fabric boundary, so Infinity-Cache hits are inside; o_proj / down_proj are K-sliced (3 slices): "
-                                   "their figure includes the fp32 partial tiles written by the GEMM and read by the launch-boundary reduction; the rest above 1.0 is operand-tile "
-                                   "re-reads (each X tile by every N-tile column, each W tile by the 5 M-tiles) that drift out of an XCD's 4 MB L2"}
+                            "how": f"profiles/{pmc_file} (rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE passes over tools/mb_gemm_prefill.py; committed digest, not "
+                                   "re-measured in this run); counted at the L2 -> fabric boundary, so Infinity-Cache hits are inside; down_proj is K-sliced (3 slices): "
+                                   "its figure includes the fp32 partial tiles written by the GEMM and read by the launch-boundary reduction; the rest above 1.0 is X, which "
+                                   "each of the 8 XCDs' L2 reads (gate|up: in both rounds of its tiles)"}
     roof_p = {"bound": "mfma", "kernel": "gemm4w_kernel<bf16,...> (tiles and K slices by gemm4w_form; a sliced product timed with gemm4w_reduce_kernel): decoder prefill linears",
               # frac = the north_star quantity: ALL FLOPs of the prefill (tower + projector + decoder linears + attention) / the measured prefill time;
               # the GEMM family alone (kernel-only durations) is reported beside it

@@ -473,7 +473,8 @@ int lmx_seq_truncate(lmx_seq* s, int32_t n_rows, void* stream);
 /* Packed prefill of several requests (serving; the reference prefills each request alone inside its own generate() thread, model_worker.py:174-185):
  * the rows of all sequences are processed as ONE row block in pieces of block_rows (0 = everything at once), every linear as a single GEMM over
  * the piece; RoPE / KV append / causal attention per sequence against its own cache; each sequence's last row gets the lm_head and its pick
- * (greedy != 0), exactly as lmx_prefill does.  embeds[i]: [n_tokens[i], hidden] rows of request i (output of lmx_gather_embeds). */
+ * (greedy != 0), as lmx_prefill does.  The products' tiles, and with them the order of their fp32 sums, follow the rows that are read together (layer-stack decoders: the head's too,
+ * where several sequences end in one piece), so a sequence's logits agree with those of lmx_prefill to rounding, and a near-tie can be picked otherwise.  embeds[i]: [n_tokens[i], hidden] rows of request i (output of lmx_gather_embeds). */
 /* The same, with the logits of chosen rows (layer-stack decoders): n_want[i] ascending row indices of sequence i's portion, concatenated in want_rows;
  * logits_dev receives [sum n_want][vocab pitch] floats. */
 int lmx_prefill_batch_logits(lmx_model* m, lmx_seq* const* seqs, int32_t n, const void* const* embeds, const int32_t* n_tokens, int32_t block_rows, const int32_t* n_want,

@@ -594,7 +594,9 @@ __global__ __launch_bounds__(NTH, NTH == 512 && sizeof(T) == 2 ? 4 : 1) void del
 }
 
 static bool one_round(const DeltaShape& s, int n_seq) { return s.H * n_seq <= 256; }
-// past one round the routers are a tail of their own: 32 x 32 heads x sequences 39.1 us without, 50.4 with them, 9.8 alone; in one round (16 x 1) 9.9 either way, 8.1 alone
+// past one round the routers are a tail of their own: 32 x 32 heads x sequences 39.1 us without, 50.4 with them, 9.8 alone; in one round (16 x 1) 9.9 either way, 8.1 alone.  On the line,
+// where the routers' own workgroups are the ones past the round, they still cost less than their launches: a decode step with two of them, 16 x 16 728 us in the step's launch, 734 in
+// their own; 32 x 8 1458, 1461
 bool delta_decode_routes(const DeltaShape& s, int n_seq) { return one_round(s, n_seq); }
 void launch_delta_decode(int dtype, const DeltaDecodeArgs& a, hipStream_t st) {
     delta_check(a.s);
@@ -610,7 +612,7 @@ void launch_delta_decode(int dtype, const DeltaDecodeArgs& a, hipStream_t st) {
                         else LMX_LAUNCH((delta_decode_kernel<TT, 32, NTH>), grid, dim3(NTH), smem, st, a); } while (0)
 #define LN(TT) do { if (wide) L(TT, 1024); else L(TT, 512); } while (0)
     // 1024 threads a head while every workgroup has a CU of its own; past that two workgroups of 512 on a CU, whose reads and arithmetic overlap.  us at 16 x 16 / 16 x 24 /
-    // 32 x 32 heads x sequences: 1024 threads 13.8 / 22.5 / 45.4, 512 threads 15.9 / 20.0 / 40.5
+    // 32 x 32 heads x sequences: 1024 threads 13.8 / 22.5 / 45.4, 512 threads 15.9 / 20.0 / 40.5 (bf16 at 128 registers: 20 bytes a lane in scratch at DK 128, 8 at 256, f16 none)
     const bool wide = one_round(a.s, a.n_seq);
     LMX_REQUIRE(wide || !a.router.x, "delta_decode: no router here");
     if (dtype == kBF16) LN(bf16_t); else if (dtype == kF16) LN(f16_t); else LN(float);

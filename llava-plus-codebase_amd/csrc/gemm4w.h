@@ -3,10 +3,14 @@
 // Replaces the same torch.nn.Linear calls as gemm.hip (HF5:models/llama/modeling_llama.py:163-176,243-281) for every prompt-sized linear: the decoder's q|k|v, gate|up, o and
 // down, the CLIP tower's, the training step's forward and data gradients.
 //
-// Bound: power.  With random operands the chip's matrix cores run at the clock their power allows, so a form is as fast as it is frugal, and a launch as fast as its tiles divide
-// over the CUs.  Both decide the shape (4096 x 4096 x 8192, one round of 256 tiles, us on random operands / on zeros, where the clock stays up):
-//   * one wave a SIMD with a 128 x 128 piece of the tile: a K-step of 256 x 256 x 64 reads 128 KB of fragments from LDS (eight waves of 128 x 64: 192 KB, as many cycles as the
-//     MFMAs take).  204 / 137 with eight waves of v_mfma_f32_32x32x16, 174 / 136 here;
+// Bound: power in a full round.  With random operands the chip's matrix cores run at the clock their power allows: 4096 x 4096 x 8192, one round of 256 tiles, takes 187 us at 1.85 GHz
+// with the matrix cores 76 % busy, the same on zeros 146 us at 2.30 GHz and 78 % (eight waves of 32x32x16: 208 us at 1.63 GHz, 145 at 2.26; by counters).  So a form is as fast as it is
+// frugal, and a launch as fast as its tiles divide over the CUs: q|k|v, gate|up and down of a 7B prompt of 1087 rows hold 2.03 .. 2.13 GHz at 59 .. 61 % busy; o, 224 tiles with 0.24 us
+// of fixed cost in a K-step of 0.56, is not bound by power: 2.4 GHz at 34 %.  From memory, every XCD's L2 reads X once and the weights once between them: 199 MB at q|k|v are 8 x 8.9 of
+// X, 101 of W and 27 of output; 123 at o, 335 at down with its partial tiles; 371 at gate|up, whose second round reads X once more.
+// Both decide the shape (4096 x 4096 x 8192, us on random operands / on zeros):
+//   * one wave a SIMD with a 128 x 128 piece of the tile: a K-step of 256 x 256 x 64 reads 128 KB of fragments from LDS (eight waves of 128 x 64: 192 KB; LDS is busy
+//     in 19 % of the cycles against 30).  204 / 137 with eight waves of v_mfma_f32_32x32x16, 174 / 136 here;
 //   * v_mfma_f32_16x16x32, not 32x32x16: 177 / 126 against 192 / 121 without the epilogue.  The larger instruction is the better one on zeros and takes more power on numbers;
 //   * both K halves of an accumulator back to back: 178 / 138 -> 174 / 136;
 //   * tiles of 32 MB x 32 NB for many MB, NB, because the power limit makes the time of a K-step follow the tile's area (0.12 + 0.018 us x MB NB): whichever divides

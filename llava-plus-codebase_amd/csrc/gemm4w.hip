@@ -19,7 +19,8 @@ struct Tile { int8_t mb, nb; };
 constexpr Tile kTiles[] = {LMX_GEMM4W_LARGE(LMX_GEMM4W_TILE, ) LMX_GEMM4W_SMALL(LMX_GEMM4W_TILE, )};
 
 // Time of a launch (us), fitted to 3200 timings: 112 products of 139 .. 6528 rows x 256 .. 28000 weights x 512 .. 13824, every tile of 4 .. 8 x 4 .. 8 blocks, 1 .. 3 slices
-// (6 % rms; the form it picks is 1.2 % behind the best one of this table in the mean).  256 workgroups are a round, one a CU.
+// (6 % rms; the form it picks is 1.2 % behind the best one of this table in the mean).  Over 140 products of another run, 300 .. 6528 rows of 17 linears: 4 % low, 7.5 % rms about that, the
+// pick 0.7 % behind in the mean and 16 % at most (300 x 12288 x 4096: 45.8 us for 39.3).  256 workgroups are a round, one a CU.
 //   a K-step:  0.24 us + 0.0129 a block of the tile + 0.0066 a block of its sides
 //   a round that leaves CUs idle has their power: its K-steps take 0.76 + 0.24 x (the share of CUs at work) of that
 //   an epilogue: 0.2 us a block, more with gating or an activation; a slice's plain stores half of that, then the reduction's launch and its reads
@@ -116,10 +117,12 @@ size_t gemm4w_slab_bytes(int M, int N, const TileForm& f) {
     return f.slices * std::max(tile, whole) * sizeof(float);
 }
 
-// Which products: more than 256 rows (below, the row tiles of gemm_rows.hip read every weight once) and more than 640 tiles of 64 x 64.  Below that the small tiles and row tiles
-// are the faster ones, us theirs / here:  800 x 1024 x 2048 10.3 / 14.1   2000 x 512 x 2048 12.9 / 14.8   257 x 6208 x 2048 15.1 / 17.1   330 x 4544 x 2304 15.9 / 17.3
-//   577 x 4096 x 1024 13.3 / 13.9   2308 x 1024 x 4096 30.5 / 27.2;  above:  700 x 3072 x 1024 11.4 / 9.8   500 x 12288 x 4096 64.8 / 48.6   400 x 22016 x 4096 gated 97 / 70
-//   1087 x 4096 x 4096 45.5 / 39.7   2048 x 2048 x 2048 23.6 / 18.4   2048 x 2048 x 5632 56.0 / 41.0   2308 x 3072 x 1024 22.0 / 17.5   1541 x 12544 x 4096 170.5 / 126.5.
+// Which products: more than 256 rows (below, the row tiles of gemm_rows.hip read every weight once) and more than 640 tiles of 64 x 64, us theirs / here.
+//   Past that line none of the other forms was the faster one in 140 products:  500 x 12288 x 4096 64.8 / 48.6   400 x 22016 x 4096 gated 97 / 70   1087 x 4096 x 4096 45.5 / 39.7
+//     2048 x 2048 x 2048 23.6 / 18.4   2048 x 2048 x 5632 56.0 / 41.0   2308 x 3072 x 1024 22.0 / 17.5   1541 x 12544 x 4096 170.5 / 126.5.
+//   Below it, by shape:  800 x 1024 x 2048 10.3 / 14.1   2000 x 512 x 2048 12.9 / 14.8   257 x 6208 x 2048 15.1 / 17.1   330 x 4544 x 2304 15.9 / 17.3   577 x 4096 x 1024 13.3 / 13.9,
+//     but  700 x 3072 x 1024 11.4 / 9.8   2308 x 1024 x 4096 30.5 / 27.2   500 x 4096 x 11008 74.3 / 63.3.  Of 31 products of 300 .. 640 tiles the form taken is ahead of the tile of the
+//     cost above in 11, the tile by more than a tenth in 12: a line that follows K as well would stand lower for a long one.
 TileForm gemm4w_form(int dtype, const GemmArgs& a) {
     const TileForm none{0, 0, 1};
     if ((dtype != kBF16 && dtype != kF16) || a.c_f32 || a.K % 64 != 0 || a.N % 8 != 0 || (act_gated(a.act) && a.N % 64 != 0) || (a.pk_kc && a.pk_D % 8 != 0)) return none;

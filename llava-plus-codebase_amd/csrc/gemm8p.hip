@@ -1,7 +1,8 @@
 // Ping-pong prefill GEMM for gfx950: C[M,N] = act(X[M,K] · W[N,K]ᵀ + bias) (+ residual), 16-bit operands, fp32 accumulate.
 //
-// Replaces the same torch.nn.Linear calls as gemm.hip (HF5:models/llama/modeling_llama.py:163-176,243-281) for the large
-// decoder linears of a prefill (q|k|v, gate|up, o_proj, down_proj at T ~ 1k).
+// Replaces the same torch.nn.Linear calls as gemm.hip (HF5:models/llama/modeling_llama.py:163-176,243-281) for wide
+// linears of up to 256 rows that the row tiles leave (183 x 18176 x 7744), K-sliced where the caller brings scratch;
+// past 256 rows the four-wave kernel (gemm4w.h) is the faster one.
 //
 // Structure (one 512-thread workgroup per 256x256 output tile, one workgroup per CU, 128 KiB of LDS):
 //   * 8 waves = 2 (M) x 4 (N); a wave owns a 128 (M) x 64 (N) sub-tile = 4 x 2 accumulators of v_mfma_f32_32x32x16.

@@ -343,6 +343,8 @@ size_t gemm_rows_slab_bytes(int M, int N, int S) { return S > 1 ? (size_t)S * M 
 // so: 64 weight rows up to 128 rows, where the weights are the time; 128 above, where the rows' re-reads are; no more than one workgroup per CU; slices of at least 10 slabs,
 // and above 128 rows no slicing of a short K (the slabs of o cost what its weights cost).  Short products (K < 1024, under 4 M weights) are launch time on any form.
 //
+// Of products of more than 256 rows and 640 tiles of 64 x 64 only those with fp32 output come here (and all with LMX_GEMM8P=0): the four-wave tiles take the others (gemm4w.hip, linear_form).
+//
 // More rows (or what the slices above do not take): tiles of 32 .. 256 rows x 128 weight rows, as many as make ONE round of workgroups, where 256 x 256 tiles would be too few and
 // small tiles several rounds (us, best other form -> here; 16-bit, weights cold):
 //   2048 x 2048 x 2048  33.6 -> 23.9   1400 x 2048 x 2048  30.9 -> 20.0   2679 x 1280 x 2048  30.9 -> 22.9   600 x 4096 x 4096  40.5 -> 32.8   1087 x 4096 x 4096  51.9 -> 47.1
@@ -390,7 +392,6 @@ RowsForm gemm_rows_form(int dtype, const GemmArgs& a) {
     if (rows32 >= 7 && (a.K <= 1024 || (a.K <= 2048 && (int64_t)cdiv(a.M, 128) * cdiv(a.N, 128) > 400))) return none;
     return RowsForm{mt, 128, 1};
 }
-
 
 void launch_gemm_rows(int dtype, const GemmArgs& a, int mtiles, int BN, int S, hipStream_t st) {
     LMX_REQUIRE(gemm_rows_applies(dtype, a) && mtiles >= 1 && cdiv(a.M, mtiles) <= 256 && (BN == 64 || BN == 128), "gemm_rows: shape or alignment");

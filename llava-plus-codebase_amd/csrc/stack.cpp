@@ -511,7 +511,8 @@ void Model::stack_prefill(Seq* const* seqs, const void* const* embeds, const int
                     want_next[(size_t)g.seq] += nr;
                 }
             }
-        // the sequences that end in this piece (neighbours): one row alone through the GEMV, several through one product with the head (32 rows of 4096 one by one 1265 us)
+        // the sequences that end in this piece (neighbours): one row alone through the GEMV, several through one product with the head (32 rows of 4096 one by one 1265 us).  Both have fp32
+        // sums, in another order, as the other linears of a piece have by its rows
         std::vector<Segment> ends;
         if (greedy || out.last_logits)
             for (const Segment& g : seg) if (g.src0 + g.n == Ts[g.seq]) ends.push_back(g);

@@ -682,20 +682,77 @@ int gemm_slices(const GemmArgs& a) {
     return s;
 }
 
-// Four waves' tiles (gemm4w.hip), row tiles (gemm_rows.hip), and of what is left of the large problems (up to 256 rows) the ping-pong 256x256x64 kernel (gemm8p.hip), K-sliced when its
-// tiles leave CUs idle and the caller brought the partial-tile scratch (the engine does, per sequence).  LMX_GEMM8P=0: the row tiles and the ring kernels alone, as an A/B and cross-check.
+// Tile choice from microbenchmarks (profiles/r01_microbench.jsonl).  The pipelined ring kernels are
+// bound by L2->LDS bandwidth (~12 TB/s), so the biggest tile that still fills the chip wins; when even 128-row
+// tiles cannot give every CU work (CLIP-sized problems) fall back to the small-tile kernels.
+static int ring_variant(const GemmArgs& a) {
+    const long t256 = (long)cdiv(a.M, 256) * cdiv(a.N, 256);
+    const long t128x256 = (long)cdiv(a.M, 128) * cdiv(a.N, 256);
+    const long t64 = (long)cdiv(a.M, 64) * cdiv(a.N, 128);
+    const long t128 = (long)cdiv(a.M, 128) * cdiv(a.N, 128);
+    if (t256 >= 200) return 9;                             // 256x256, 2-slot ring   (qkv, gate|up at T~1k; TP=2 gate|up: 215 tiles)
+    if (t128 >= 192 && t128 <= 512) return 18;             // 128x128, 64 KB: 192..512 tiles, all co-resident (two per CU), beat fewer big
+                                                           // tiles (o_proj 58 vs 64 us, down_proj 146 vs 152 us at T=1087; TP-rank shapes
+                                                           // 1087x3072x4096 44 vs 52 us, 1087x2816x4096 46 vs 51 us: profiles/EXPERIMENTS.md)
+    if (t128x256 >= 128) return 7;                         // 128x256, 3-slot ring   (o_proj, down_proj)
+    if (t64 <= 320 && !act_gated(a.act)) {                 // (<= : CLIP fc1 577 x 4096 x 1024 has exactly 320 -> 64x64 2-slot kernel, 14.6 vs 16.5 us for 64x128)
+        // CLIP-sized problems are latency-bound: with few 64x64 tiles (<= 2 per CU) keep three K-slabs in flight per
+        // workgroup (4-slot ring, 64 KB LDS); with more tiles the 2-slot kernel's higher occupancy (32 KB) wins.
+        const long t64x64 = (long)cdiv(a.M, 64) * cdiv(a.N, 64);
+        // fewer tiles than CUs and a long K (CLIP fc2: 577 x 1024 x 4096, 160 tiles x 64 K-steps): two K groups per workgroup — 20.5 -> 18.2 us
+        // (profiles/r05_vis_gemm_ksplit.jsonl; at K = 1024 the forms tie, with more tiles than CUs the 8-wave workgroups lose)
+        return t64x64 <= 256 && a.K >= 2048 ? 16 : (t64x64 <= 512 ? 15 : 5);
+    }
+    return 4;
+}
+
+// Time of a launch (us) on the forms that the four-wave tiles compete with, fitted to 2200 timings as theirs is (`cost` of gemm4w.hip; ping-pong 6 % rms, row tiles 5, rings 2 .. 5).
+// `places` workgroups are a round; a round that is not full takes `idle` (its K-steps) and `part` (its epilogues) of a full one at least.  Row tiles: a tile of 256 x 128.
+struct FormTime { int bm, bn, places; float act[4], res, bias, step, idle, part, launch, slice_mn; };      // act: none, quick GELU, GELU, gated
+static float form_time(const GemmArgs& a, const LinearForm& f) {
+    static constexpr FormTime rows{0, 0, 256, {3.2f, 7.3f, 9.7f, 3.7f}, 2.70f, 0.95f, 1.006f, 0.688f, 1.f, 3.8f, 1.99e-6f},
+        ping_pong{256, 256, 256, {6.9f, 16.9f, 24.5f, 10.0f}, 4.43f, 0.18f, 1.519f, 0.486f, 0.794f, 2.6f, 1.62e-6f},
+        ring18{128, 128, 512, {6.5f, 12.3f, 16.6f, 7.7f}, 1.51f, 0.25f, 1.075f, 0.648f, 0.599f, 0.f, 0.f},
+        ring7{128, 256, 256, {5.9f, 11.4f, 15.9f, 7.6f}, 1.61f, 0.05f, 0.814f, 0.971f, 0.693f, 0.f, 0.f},
+        ring4{64, 128, 768, {6.3f, 10.6f, 13.2f, 6.7f}, 0.09f, 0.68f, 1.055f, 0.886f, 0.254f, 0.f, 0.f};
+    const FormTime& t = f.kernel == LinearForm::kRows ? rows : f.kernel == LinearForm::kPingPong ? ping_pong : f.ring == 18 ? ring18 : f.ring == 7 ? ring7 : ring4;
+    const int kind = act_gated(a.act) ? 3 : a.act == kActQuickGelu ? 1 : a.act != kActNone ? 2 : 0;
+    float step = t.step, area = 1.f;
+    int tiles;
+    if (f.kernel == LinearForm::kRows) {
+        const int r32 = cdiv(cdiv(a.M, f.rows.mtiles), 32), mt = cdiv(a.M, 32 * r32);
+        area = r32 / 8.f * (f.rows.bn / 128.f);
+        step += 0.877f * (area - 1.f) + 0.001f * mt;
+        tiles = mt * cdiv(a.N, f.rows.bn) * f.slices;
+    } else tiles = cdiv(a.M, t.bm) * cdiv(a.N, t.bn) * f.slices;
+    const float steps = cdiv(a.K / 64, f.slices) * step;
+    const float epi = f.slices > 1 ? 0.f : (t.act[kind] + (a.R ? t.res : 0.f) + (a.bias && (kind == 0 || kind == 3) ? t.bias : 0.f)) * area;
+    const float share = (float)(tiles % t.places) / t.places;
+    float us = t.launch + (tiles / t.places) * (steps + epi);
+    if (share > 0.f) us += steps * (t.idle + (1.f - t.idle) * share) + epi * (t.part + (1.f - t.part) * share);
+    if (f.slices > 1) us += t.slice_mn * f.slices * a.M * a.N;
+    return us;
+}
+
+// Row tiles (gemm_rows.hip), wide products that they leave on the ping-pong 256x256x64 kernel (gemm8p.hip), K-sliced when its tiles leave CUs idle and the caller brought the partial-tile
+// scratch (the engine does, per sequence), the ring kernels, and past gemm4w_form's line the four-wave tiles (gemm4w.hip) where they take less time than whichever of these it would be.
+// Of 2200 products past the line, mean time 0.901 of the others' (the better of both by measurement: 0.893), more than a twentieth slower than them in 2 %.  The four-wave tiles
+//   everywhere 1.00, and by K and activation (none, none with a residual, GELU):  64 .. 256 1.26 1.44 1.37   257 .. 512 1.04 1.22 1.28   513 .. 800 0.85 1.05 1.08
+//   1201 .. 2000 0.78 0.90 1.09   from 4001 0.74 0.78 0.80.  us others / four-wave tiles:  2308 x 3072 x 64 with a residual 8.3 / 13.7   1087 x 12288 x 192 quick GELU 24.9 / 32.0
+//   1152 x 5120 x 1024 GELU 28.8 / 32.7   2304 x 4096 x 1024 GELU 52.7 / 41.8   2308 x 4096 x 1024 quick GELU 36.1 / 33.0.
+// LMX_GEMM8P=0: the row tiles and the ring kernels alone, as an A/B and cross-check.
 LinearForm linear_form(int dtype, const GemmArgs& a) {
     LinearForm f;
     if (dtype != kBF16 && dtype != kF16) return f;
-    if (gemm8p_enabled()) {
-        f.tile = gemm4w_form(dtype, a);
-        if (f.tile.mb) { f.kernel = LinearForm::kTiles; f.slices = f.tile.slices; return f; }
-    }
     f.rows = gemm_rows_form(dtype, a);
-    if (f.rows.mtiles) { f.kernel = LinearForm::kRows; f.slices = f.rows.slices; return f; }
-    if (a.c_f32 || !gemm8p_enabled()) return f;
     const int S = gemm_slices(a);
-    if (cdiv(a.M, 256) * cdiv(a.N, 256) * S >= 160) { f.kernel = LinearForm::kPingPong; f.slices = S; }
+    if (f.rows.mtiles) { f.kernel = LinearForm::kRows; f.slices = f.rows.slices; }
+    else if (!a.c_f32 && gemm8p_enabled() && cdiv(a.M, 256) * cdiv(a.N, 256) * S >= 160) { f.kernel = LinearForm::kPingPong; f.slices = S; }
+    else f.ring = ring_variant(a);
+    if (!gemm8p_enabled()) return f;
+    float us = 0.f;
+    f.tile = gemm4w_form(dtype, a, &us);
+    if (f.tile.mb && (a.qf_kc || us < form_time(a, f))) { f.kernel = LinearForm::kTiles; f.slices = f.tile.slices; }      // (the q|k|v epilogue is the four-wave kernel's alone)
     return f;
 }
 
@@ -711,30 +768,7 @@ static void launch_gemm16(const GemmArgs& a, int variant, hipStream_t st) {
         if (f.kernel == LinearForm::kPingPong) { GemmArgs b = a; b.split_k = f.slices; launch_gemm8p(TypeInfo<T>::id, b, st); return; }
     }
     if (a.c_f32) { launch_gemm_cfg<T, 64, 128, 2, 2, true, true>(a, st); return; }      // fp32 logits of a few wanted rows: one tile form
-    if (variant == 0) {
-        // Tile choice from the round-1 microbenchmarks (profiles/r01_microbench.jsonl).  The pipelined ring kernels are
-        // bound by L2->LDS bandwidth (~12 TB/s), so the biggest tile that still fills the chip wins; when even 128-row
-        // tiles cannot give every CU work (CLIP-sized problems) fall back to the small-tile kernels.
-        const long t256 = (long)cdiv(a.M, 256) * cdiv(a.N, 256);
-        const long t128x256 = (long)cdiv(a.M, 128) * cdiv(a.N, 256);
-        const long t64 = (long)cdiv(a.M, 64) * cdiv(a.N, 128);
-        const long t128 = (long)cdiv(a.M, 128) * cdiv(a.N, 128);
-        if (t256 >= 200) variant = 9;                          // 256x256, 2-slot ring   (qkv, gate|up at T~1k; TP=2 gate|up: 215 tiles)
-        else if (t128 >= 192 && t128 <= 512)
-            variant = 18;                                      // 128x128, 64 KB: 192..512 tiles, all co-resident (two per CU), beat fewer big
-                                                               // tiles (o_proj 58 vs 64 us, down_proj 146 vs 152 us at T=1087; TP-rank shapes
-                                                               // 1087x3072x4096 44 vs 52 us, 1087x2816x4096 46 vs 51 us: profiles/EXPERIMENTS.md)
-        else if (t128x256 >= 128) variant = 7;                 // 128x256, 3-slot ring   (o_proj, down_proj)
-        else if (t64 <= 320 && !act_gated(a.act)) {                  // (<= : CLIP fc1 577 x 4096 x 1024 has exactly 320 -> 64x64 2-slot kernel, 14.6 vs 16.5 us for 64x128)
-            // CLIP-sized problems are latency-bound: with few 64x64 tiles (<= 2 per CU) keep three K-slabs in flight per
-            // workgroup (4-slot ring, 64 KB LDS); with more tiles the 2-slot kernel's higher occupancy (32 KB) wins.
-            const long t64x64 = (long)cdiv(a.M, 64) * cdiv(a.N, 64);
-            // fewer tiles than CUs and a long K (CLIP fc2: 577 x 1024 x 4096, 160 tiles x 64 K-steps): two K groups per workgroup — 20.5 -> 18.2 us
-            // (profiles/r05_vis_gemm_ksplit.jsonl; at K = 1024 the forms tie, with more tiles than CUs the 8-wave workgroups lose)
-            variant = t64x64 <= 256 && a.K >= 2048 ? 16 : (t64x64 <= 512 ? 15 : 5);
-        }
-        else variant = 4;
-    }
+    if (variant == 0) variant = ring_variant(a);
     switch (variant) {
         case 2: launch_gemm_cfg<T, 128, 128, 2, 2, false>(a, st); break;
         case 4: launch_gemm_cfg<T, 64, 128, 2, 2, true>(a, st); break;

@@ -18,27 +18,24 @@ struct Tile { int8_t mb, nb; };
 #define LMX_GEMM4W_TILE(T, MB, NB) {MB, NB},
 constexpr Tile kTiles[] = {LMX_GEMM4W_LARGE(LMX_GEMM4W_TILE, ) LMX_GEMM4W_SMALL(LMX_GEMM4W_TILE, )};
 
-// Time of a launch (us), fitted to 3200 timings: 112 products of 139 .. 6528 rows x 256 .. 28000 weights x 512 .. 13824, every tile of 4 .. 8 x 4 .. 8 blocks, 1 .. 3 slices
-// (6 % rms; the form it picks is 1.2 % behind the best one of this table in the mean).  Over 140 products of another run, 300 .. 6528 rows of 17 linears: 4 % low, 7.5 % rms about that, the
-// pick 0.7 % behind in the mean and 16 % at most (300 x 12288 x 4096: 45.8 us for 39.3).  256 workgroups are a round, one a CU.
+// Time of a launch (us).  K-steps fitted to 112 linears back to back; epilogues, slices and the rest to 900 products of 257 .. 8000 rows x 512 .. 28000 weights x 64 .. 14000, every
+// activation, with and without residual and bias, every tile of the table, 1 .. 3 slices, each form for 3.5 ms ahead of its timing (the chip at its power limit) on weights from memory
+// (1.6 GB of them in turn).  7 % rms at the form it picks, which is 0.9 % behind the best one of the table in the mean, 30 % at most.  256 workgroups are a round, one a CU.
 //   a K-step:  0.24 us + 0.0129 a block of the tile + 0.0066 a block of its sides
 //   a round that leaves CUs idle has their power: its K-steps take 0.76 + 0.24 x (the share of CUs at work) of that
-//   an epilogue: 0.2 us a block, more with gating or an activation; a slice's plain stores half of that, then the reduction's launch and its reads
-float rounds(int tiles, int n, int act, int mb, int nb, bool slices) {
-    const int area = mb * nb;
-    const float steps = n * (0.24f + 0.0129f * area + 0.0066f * (mb + nb));
-    const float epi = slices ? 0.108f * area - 0.5f : (act_gated(act) ? 0.34f : act != kActNone ? 0.64f : 0.215f) * area - 2.2f;
-    float t = (tiles / 256) * (steps + epi);
-    if (const int rem = tiles % 256) {
-        const float share = rem / 256.f;
-        t += steps * (0.76f + 0.24f * share) + epi * std::max(0.5f, share);
-    }
-    return t;
-}
+//   an epilogue:  2 us + 0.093 a block, more with an activation (vector ALUs at one wave a SIMD), a residual or a bias; of a slice 5 us, then the reduction's launch and its reads
 float cost(const GemmArgs& a, int mb, int nb, int S) {
-    float t = rounds(cdiv(a.M, 32 * mb) * cdiv(a.N, 32 * nb) * S, cdiv(a.K / 64, S), a.act, mb, nb, S > 1);
-    if (S > 1) t += 3.8f + 1.17e-6f * S * a.M * a.N;
-    return t;
+    const int area = mb * nb, tiles = cdiv(a.M, 32 * mb) * cdiv(a.N, 32 * nb) * S;
+    const bool gated = act_gated(a.act);
+    const float steps = cdiv(a.K / 64, S) * (0.24f + 0.0129f * area + 0.0066f * (mb + nb));
+    float block = gated ? 0.187f : a.act == kActQuickGelu ? 0.429f : a.act != kActNone ? 0.642f : 0.093f;
+    if (a.R) block += 0.152f;
+    if (a.bias && (gated || a.act == kActNone)) block += 0.077f;      // (the other activations were timed with theirs)
+    const float epi = S > 1 ? 5.1f : block * area + 2.06f;
+    float t = (tiles / 256) * (steps + epi);
+    if (const int rem = tiles % 256) t += steps * (0.76f + 0.24f * (rem / 256.f)) + epi;
+    if (S > 1) t += 4.5f + 1.27e-6f * S * a.M * a.N;
+    return 1.6f + 1.03f * t;
 }
 
 // fallback K-slice scratch for callers that bring none and ask for slices (lmx_op_gemm: unit tests, microbenchmarks; ONE stream at a time).
@@ -58,14 +55,25 @@ template <typename T> void launch_t(const GemmArgs& a, const TileForm& f, hipStr
     }
 }
 
-// A grouped product on tiles of mb x nb blocks.  The host does not know the groups' rows: the mean over loads around the average.  Over 75 .. 670 rows a group of two
-// mixtures (16 groups, 2816 x 2048 and 2048 x 1408, 5504 x 4096 and 4096 x 2752, rows spread at random) the tile this picks is 2.5 % behind the best one in the mean
+// A grouped product on tiles of mb x nb blocks, by rounds fitted to back-to-back launches of 112 linears of 139 .. 6528 rows (6 % rms).  The host does not know the groups' rows: the mean
+// over loads around the average.  Over 75 .. 670 rows a group of two mixtures (16 groups, 2816 x 2048 and 2048 x 1408, 5504 x 4096 and 4096 x 2752, rows spread at random) the tile this
+// picks is 2.5 % behind the best one in the mean; over ten grouped products of 70 .. 900 rows a group 3.1 %
+float group_rounds(int tiles, int n, int act, int mb, int nb) {
+    const int area = mb * nb;
+    const float steps = n * (0.24f + 0.0129f * area + 0.0066f * (mb + nb)), epi = (act_gated(act) ? 0.34f : act != kActNone ? 0.64f : 0.215f) * area - 2.2f;
+    float t = (tiles / 256) * (steps + epi);
+    if (const int rem = tiles % 256) {
+        const float share = rem / 256.f;
+        t += steps * (0.76f + 0.24f * share) + epi * std::max(0.5f, share);
+    }
+    return t;
+}
 float group_cost(const GroupGemmArgs& a, int mb, int nb) {
     const float avg = (float)a.rows / a.groups;
     float t = 0.f;
     for (const float load : {0.85f, 0.92f, 1.f, 1.08f, 1.15f}) {
         const int m_tiles = a.groups * std::max(1, cdiv((int)(avg * load), 32 * mb));
-        t += 0.2f * rounds(m_tiles * cdiv(a.N, 32 * nb), a.K / 64, a.act, mb, nb, false);
+        t += 0.2f * group_rounds(m_tiles * cdiv(a.N, 32 * nb), a.K / 64, a.act, mb, nb);
     }
     return t;
 }
@@ -117,13 +125,10 @@ size_t gemm4w_slab_bytes(int M, int N, const TileForm& f) {
     return f.slices * std::max(tile, whole) * sizeof(float);
 }
 
-// Which products: more than 256 rows (below, the row tiles of gemm_rows.hip read every weight once) and more than 640 tiles of 64 x 64, us theirs / here.
-//   Past that line none of the other forms was the faster one in 140 products:  500 x 12288 x 4096 64.8 / 48.6   400 x 22016 x 4096 gated 97 / 70   1087 x 4096 x 4096 45.5 / 39.7
-//     2048 x 2048 x 2048 23.6 / 18.4   2048 x 2048 x 5632 56.0 / 41.0   2308 x 3072 x 1024 22.0 / 17.5   1541 x 12544 x 4096 170.5 / 126.5.
-//   Below it, by shape:  800 x 1024 x 2048 10.3 / 14.1   2000 x 512 x 2048 12.9 / 14.8   257 x 6208 x 2048 15.1 / 17.1   330 x 4544 x 2304 15.9 / 17.3   577 x 4096 x 1024 13.3 / 13.9,
-//     but  700 x 3072 x 1024 11.4 / 9.8   2308 x 1024 x 4096 30.5 / 27.2   500 x 4096 x 11008 74.3 / 63.3.  Of 31 products of 300 .. 640 tiles the form taken is ahead of the tile of the
-//     cost above in 11, the tile by more than a tenth in 12: a line that follows K as well would stand lower for a long one.
-TileForm gemm4w_form(int dtype, const GemmArgs& a) {
+// Which products: more than 256 rows (below, the row tiles of gemm_rows.hip read every weight once) and more than 640 tiles of 64 x 64, and of these those that no other form makes in
+// less time (linear_form).  Below the line, us theirs / here, by shape:  800 x 1024 x 2048 10.3 / 14.1   2000 x 512 x 2048 12.9 / 14.8   257 x 6208 x 2048 15.1 / 17.1
+//   330 x 4544 x 2304 15.9 / 17.3   577 x 4096 x 1024 13.3 / 13.9,  but  700 x 3072 x 1024 11.4 / 9.8   2308 x 1024 x 4096 30.5 / 27.2   500 x 4096 x 11008 74.3 / 63.3.
+TileForm gemm4w_form(int dtype, const GemmArgs& a, float* us) {
     const TileForm none{0, 0, 1};
     if ((dtype != kBF16 && dtype != kF16) || a.c_f32 || a.K % 64 != 0 || a.N % 8 != 0 || (act_gated(a.act) && a.N % 64 != 0) || (a.pk_kc && a.pk_D % 8 != 0)) return none;
     if (a.R && a.ldr % 4 != 0) return none;                  // residual rows of any pitch: another kernel's
@@ -141,6 +146,7 @@ TileForm gemm4w_form(int dtype, const GemmArgs& a) {
             if (!best.mb || c < least) { best = f; least = c; }
         }
     }
+    if (us) *us = least;
     return best;
 }
 

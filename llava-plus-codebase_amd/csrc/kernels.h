@@ -52,7 +52,7 @@ size_t gemm8p_splitk_ws_bytes(int M, int N, int split_k);
 int gemm8p_pick_split(int M, int N, int K);
 // four-wave kernel (gemm4w.h, gemm4w.hip): tiles of 32 mb x 32 nb, K slices (> 1: fp32 partial tiles in a.skw and a second launch that adds them); variant 100 mb + 10 nb + slices
 struct TileForm { int mb, nb, slices; };
-TileForm gemm4w_form(int dtype, const GemmArgs& a);                   // the form variant 0 takes (mb 0: another kernel)
+TileForm gemm4w_form(int dtype, const GemmArgs& a, float* us = nullptr);      // the cheapest form and its time (mb 0: not here); what is taken: linear_form
 size_t gemm4w_slab_bytes(int M, int N, const TileForm& f);
 void launch_gemm4w(int dtype, GemmArgs a, TileForm f, hipStream_t st);
 // linears of up to a few hundred rows (gemm_rows.hip): mtiles row tiles of <= 256 rows, BN = 64 / 128 weight rows a workgroup, S slices of K (S > 1: fp32 slabs in a.skw,
@@ -64,7 +64,7 @@ RowsForm gemm_rows_form(int dtype, const GemmArgs& a);                // the for
 struct LinearForm {
     enum Kernel { kRing = 0, kRows = 1, kTiles = 2, kPingPong = 3 } kernel = kRing;
     TileForm tile{0, 0, 1}; RowsForm rows{0, 0, 1};
-    int slices = 1;
+    int slices = 1, ring = 0;            // ring: variant of the ring kernels
 };
 LinearForm linear_form(int dtype, const GemmArgs& a);
 size_t gemm_rows_slab_bytes(int M, int N, int S);

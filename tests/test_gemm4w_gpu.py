@@ -100,10 +100,13 @@ def test_three_slices(cuda, form, act):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K,act", [(257, 10304, 1024, 0), (513, 4672, 640, 1), (700, 3072, 1024, 0), (1087, 4096, 4096, 0), (1087, 22016, 1024, 3), (2048, 2048, 5632, 0), (2679, 6400, 2048, 0), (6528, 4096, 1088, 0)])
+@pytest.mark.parametrize("M,N,K,act", [(257, 10304, 1024, 0), (513, 4672, 640, 1), (700, 3072, 1024, 0), (1087, 4096, 4096, 0), (1087, 22016, 1024, 3), (2048, 2048, 5632, 0), (2679, 6400, 2048, 0), (6528, 4096, 1088, 0),
+                                       (2693, 2048, 128, 0), (1348, 21056, 448, 3), (1200, 4096, 1024, 1), (1348, 21056, 1024, 3)])
 def test_choice(cuda, M, N, K, act):
-    """What variant 0 and a prefill's call take, on the large side of the rule's lines."""
+    """What variant 0 and a prefill's call take past the rule's line, the four-wave tiles and the forms that are cheaper there."""
     from llava_mi355x import _C, ops
+    form = ops.gemm_form(torch.bfloat16, M, N, K, act=act)[0]
+    assert form == {(700, 1024): 1, (2693, 128): 0, (1348, 448): 0, (1200, 1024): 1}.get((M, K), 2)
     x, w = _mk(M, N, K, "bf16", cuda, M + N)
     y = x.double() @ w.double().t()
     if act == 3:

@@ -215,7 +215,7 @@ void launch_group_gemm(int dtype, const GroupGemmArgs& a, int bm, hipStream_t st
 // grid (slots, ceil(outputs / outputs per workgroup)), 256 threads.  `lpr` lanes own one weight row (a power of two with 8 lpr <= K): short rows leave no lane idle.
 // Gated: a lane group takes the gate row and the up row of its output.
 // ---------------------------------------------------------------------------------------------------------------
-template <typename T, bool GATED>
+template <typename T, bool GATED, int U>
 __global__ __launch_bounds__(256) void group_gemv_kernel(GroupGemvArgs a, int lpr, int opw) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     T* xs = reinterpret_cast<T*>(smem);
@@ -229,7 +229,6 @@ __global__ __launch_bounds__(256) void group_gemv_kernel(GroupGemvArgs a, int lp
     const int o0 = blockIdx.y * opw, o1 = o0 + opw < outs ? o0 + opw : outs;
     // U pieces of a row (both rows, gated) are on their way together, the first ones ahead of the staging of x: piece by piece a row of 2048 was four memory latencies.  Pieces
     // past the row's end re-read its first one and count as zeros.  (us a launch, four slots: 2 x 1408 rows of 2048 12.2 -> 11.6, 2048 rows of 1408 8.1 -> 6.7)
-    constexpr int U = 4;
     Chunk8<T> g[U], u[GATED ? U : 1];
     const int step = U * lpr * 8;
     for (int ob = o0; ob < o1; ob += per) {                  // every lane stays: the sums run over whole lane groups
@@ -279,10 +278,19 @@ void launch_group_gemv(int dtype, const GroupGemvArgs& a, int slots, hipStream_t
     int opw = per;                                           // outputs of a workgroup: more of them while the grid stays large enough
     while (opw < 64 && (long)slots * cdiv(outs, opw * 2) >= 1024) opw *= 2;
     const dim3 grid(slots, cdiv(outs, opw));
-#define L(TT) do { if (act_gated(a.act)) LMX_LAUNCH((group_gemv_kernel<TT, true>), grid, dim3(256), (size_t)a.K * sizeof(TT), st, a, lpr, opw); \
-                   else LMX_LAUNCH((group_gemv_kernel<TT, false>), grid, dim3(256), (size_t)a.K * sizeof(TT), st, a, lpr, opw); } while (0)
+    // pieces together: up to four, as many as leave the fewest past the end of a row of this length, and one by one where so many workgroups follow each other that their latencies do not
+    // count.  us a launch one by one / four always / now, fp32 (16-bit models have few slots here): 16 rows x 16 heads of 512 columns 10.9 / 12.6 / 8.5 and of 128 8.2 / 13.8 / 8.3,
+    // 32 rows x 32 heads 22 / 40 / 16.5 and 24 / 40 / 23, 128 slots x 4096 rows of 2752 576 / 618 / 599, 3600 slots x 2048 rows of 1408 1925 / 2128 / 1950 and x 2 x 1408 rows
+    // of 2048 7934 / 8181 / 7916
+    const int pieces = cdiv(a.K, lpr * 8);
+    const int U = (long)grid.x * grid.y > 4096 ? 1 : pieces <= 4 ? pieces : cdiv(pieces, 3) * 3 < cdiv(pieces, 4) * 4 ? 3 : 4;
+#define L1(TT, G, UU) LMX_LAUNCH((group_gemv_kernel<TT, G, UU>), grid, dim3(256), (size_t)a.K * sizeof(TT), st, a, lpr, opw)
+#define LU(TT, G) do { if (U == 4) L1(TT, G, 4); else if (U == 3) L1(TT, G, 3); else if (U == 2) L1(TT, G, 2); else L1(TT, G, 1); } while (0)
+#define L(TT) do { if (act_gated(a.act)) LU(TT, true); else LU(TT, false); } while (0)
     if (dtype == kBF16) L(bf16_t); else if (dtype == kF16) L(f16_t); else L(float);
 #undef L
+#undef LU
+#undef L1
     LMX_CHECK_HIP(hipGetLastError());
 }
 

@@ -66,10 +66,10 @@ def test_the_line_of_the_four_wave_tiles(M, N):
 
 
 # products past that line that the four-wave tiles make in a tenth more time than another form, or half as much again (a short K, an activation behind a K of up to some 2000), and the
-# same products with a longer K or without the activation
+# same products with a longer K or without the activation; three that one round of small tiles makes in less time than the row tiles
 SHORT = [(1087, 12288, 192, 1), (2693, 2048, 128, 0), (3303, 13824, 576, 1), (722, 8824, 512, 2), (1152, 5120, 1024, 2), (1348, 21056, 448, 3), (1620, 20648, 448, 2)]
 LONG = [(1087, 12288, 4096, 1), (2693, 2048, 1024, 0), (3303, 13824, 4096, 1), (722, 8824, 4096, 2), (1152, 5120, 8192, 0), (1348, 21056, 1024, 3), (1620, 20648, 1024, 0),
-        (2304, 4096, 1024, 2), (2308, 4096, 1024, 1)]
+        (2304, 4096, 1024, 2), (2308, 4096, 1024, 1), (2200, 1280, 2048, 0), (680, 4096, 4096, 0), (520, 4640, 3072, 0)]
 
 
 @pytest.mark.parametrize("case", SHORT + LONG)

@@ -321,7 +321,7 @@ def cpu_baseline(cfg, T, new_tokens, n_layers):
 
 def tp_projection(cfg, dtype, dev, ids, pix, new_tokens, worlds=(2, 4, 8), batch=32):
     """What the request and a serving batch should look like at TP = 2 / 4 / 8 — a PROJECTION, printed so that the first real multi-GPU run has a prediction to be
-    judged against (no multi-GPU node was available to the builder).  Measured part: ONE engine instance holds rank 0's shard of a TP = W group (the
+    compared with (none was available when it was written).  Measured part: ONE engine instance holds rank 0's shard of a TP = W group (the
     production shard selection of Model::load_weight: the rank-local GEMM / GEMV / attention shapes are the real ones) and the all-reduce is replaced
     through lmx_tp_set_allreduce_hook by a no-op that counts calls, so the timed sections are the rank's compute incl. every launch boundary:
       rank_compute_prefill_ms           the WHOLE prefill as a rank runs it: replicated CLIP tower + projector + splice (not sharded) and the sharded decoder,

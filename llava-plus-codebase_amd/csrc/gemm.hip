@@ -752,9 +752,9 @@ LinearForm linear_form(int dtype, const GemmArgs& a) {
     if (!gemm8p_enabled()) return f;
     float us = 0.f;
     f.tile = gemm4w_form(dtype, a, &us);
-    // Near the line both times err by a tenth or more (2200 x 1280 x 2048: 17.8 us for 17.3 on the tiles, under that for 21.2 on the row tiles), and long K-loops without an activation to
-    // compute are where the tiles win.  767 such products, a twentieth slower than the tiles / than the other form: 3 / 11 with this margin, 16 / 5 without; 1044
-    // of widths 2048 .. 5120 and 264 .. 7500 rows: 3 a fiftieth slower than the tiles or more with it, 27 without.
+    // Near the line both times err by a tenth or more (2200 x 1280 x 2048: 17.8 us for 17.3 on the tiles, under that for 21.2 on the row tiles), and long K-loops whose epilogue computes no
+    // activation, or a gated one of half the outputs, are where the tiles win.  767 such products, a twentieth slower than the tiles / than the other form: 3 / 11 with this margin,
+    // 16 / 5 without; 1044 of widths 2048 .. 5120 and 264 .. 7500 rows: 3 a fiftieth slower than the tiles or more with it, 27 without.
     const float margin = a.K >= 1024 && (a.act == kActNone || act_gated(a.act)) ? 1.08f : 1.f;
     if (f.tile.mb && (a.qf_kc || us < margin * form_time(a, f))) { f.kernel = LinearForm::kTiles; f.slices = f.tile.slices; }      // (the q|k|v epilogue is the four-wave kernel's alone)
     return f;

@@ -709,7 +709,8 @@ int lmx_op_decode_win(int32_t dtype, int32_t D, const void* qkv, int32_t qkv_str
     a.qkv = qkv; a.out = out; a.q_norm = q_norm; a.k_norm = k_norm; a.cos_sin = cos_sin_dev; a.tab = static_cast<const DecodeFusedSeq*>(tab_dev);
     a.n_seq = n_seq; a.qkv_stride = qkv_stride; a.out_stride = out_stride; a.n_heads = n_heads; a.n_kv_heads = n_kv_heads; a.s_max = s_max; a.n_split = n_split;
     a.qk_dim = qk_dim; a.rot_dims = rot_dims; a.window = window; a.sink = sink; a.gate_off = gate_off; a.scale = scale; a.eps = eps;
-    launch_decode_win(dtype, D, a, /*grouped=*/true, S(stream));      // every batch that the grouped kernel can take; the engine: decode_win_form
+    const int keys = window > 0 && window < s_max ? window : s_max;
+    launch_decode_win(dtype, D, a, /*grouped=*/true, /*wide=*/keys > 8 * 64 * n_split, S(stream));      // every batch that the grouped kernel can take; the engine: decode_win_form
     LMX_API_END
 }
 int lmx_op_decode_win_form(int32_t dtype, int32_t D, int32_t n_heads, int32_t n_kv_heads, int32_t n_seq, int32_t span, int32_t* form) {

@@ -240,10 +240,10 @@ struct WinDecodeArgs {
     int qk_dim = 0, rot_dims = 0, window = 0, sink = 0, gate_off = -1;      // gate_off: column of head 0's gate in the row, -1 = no gates
     float scale = 1.f, eps = 0.f;
 };
-// grouped: one workgroup per kv head and split (where decode_win_groups says that it can) instead of one per query head and split
-void launch_decode_win(int dtype, int D, const WinDecodeArgs& a, bool grouped, hipStream_t st);
+// grouped: one workgroup per kv head and split (where decode_win_groups says that it can) instead of one per query head and split; wide: of eight waves instead of four
+void launch_decode_win(int dtype, int D, const WinDecodeArgs& a, bool grouped, bool wide, hipStream_t st);
 bool decode_win_groups(int dtype, int D, int n_heads, int n_kv_heads, int n_seq);
-struct WinForm { bool grouped; int n_split; };
+struct WinForm { bool grouped; int n_split; bool wide; };
 WinForm decode_win_form(int dtype, int D, int n_heads, int n_kv_heads, int n_seq, int span);      // what a step takes; span: keys that the longest sequence may have to walk
 
 // ---- gated delta rule (delta.hip): per head a state S [key channel][value channel] in fp32, S <- g S;  u = beta (v - S^T k);  S <- S + k u^T;  o = S^T q -----------------

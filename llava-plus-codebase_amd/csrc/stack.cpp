@@ -558,7 +558,7 @@ void Model::stack_prefill(Seq* const* seqs, const void* const* embeds, const int
 // ---------------------------------------------------------------------------------------------------------------
 // decode
 // ---------------------------------------------------------------------------------------------------------------
-static WinDecodeArgs decode_args(const Stack& S, const StackLayer& l, int dtype, const void* qkv, void* out, int n_seq, int max_len, int s_max, bool& grouped) {
+static WinDecodeArgs decode_args(const Stack& S, const StackLayer& l, int dtype, const void* qkv, void* out, int n_seq, int max_len, int s_max, WinForm& f) {
     const lmx_layer_config& d = l.c;
     WinDecodeArgs a;
     a.qkv = qkv; a.out = out; a.q_norm = l.qn; a.k_norm = l.kn; a.cos_sin = d.rope_dims ? S.rope[(size_t)d.rope_table] : nullptr;
@@ -567,8 +567,8 @@ static WinDecodeArgs decode_args(const Stack& S, const StackLayer& l, int dtype,
     // chunks the longest member's window can touch; enough workgroups to fill the chip, no more
     int span = max_len + 1;
     if (d.window > 0 && d.window + 127 < span) span = d.window + 127;
-    const WinForm f = decode_win_form(dtype, l.D, d.n_heads, d.n_kv_heads, n_seq, span);
-    a.n_split = f.n_split; grouped = f.grouped;
+    f = decode_win_form(dtype, l.D, d.n_heads, d.n_kv_heads, n_seq, span);
+    a.n_split = f.n_split;
     return a;
 }
 
@@ -648,11 +648,11 @@ void Model::stack_decode_step(Seq* s, hipStream_t st, int64_t* id_out) {
         bool routed = false;
         if (l.c.mixer == LMX_MIXER_ATTENTION) {
             LMX_PROF_K("decode.attn");
-            bool grouped;
-            WinDecodeArgs a = decode_args(S, l, dt, s->d_qkv, s->d_attn, 1, s->len, kv_pitch, grouped);
+            WinForm f;
+            WinDecodeArgs a = decode_args(S, l, dt, s->d_qkv, s->d_attn, 1, s->len, kv_pitch, f);
             a.one = stack_seq_ref(r, s);
             a.pos = s->len;
-            launch_decode_win(dt, l.D, a, grouped, st);
+            launch_decode_win(dt, l.D, a, f.grouped, f.wide, st);
         } else routed = stack_mix_decode(r, nullptr, stack_seq_ref(r, s), 1, s->len, s->d_x, s->d_qkv, s->d_attn, s->sw, nullptr, st);
         if (l.parallel() && l.dense()) plain("decode.gemv.gate_up", s->d_x, l.wgu, static_cast<char*>(s->d_attn) + (size_t)l.an * es, 2 * l.ff, H, l.act());
         plain("decode.gemv.o", s->d_attn, l.wo, s->d_y, H, l.out_k);
@@ -719,10 +719,10 @@ void Model::stack_decode_batch_step(Batch* b, Seq* const* seqs, int n, int64_t* 
         bool routed = false;
         if (l.c.mixer == LMX_MIXER_ATTENTION) {
             LMX_PROF("decode_batch.attn");
-            bool grouped;
-            WinDecodeArgs a = decode_args(S, l, dt, b->qkv, b->attn, n, max_len, kv_pitch, grouped);
+            WinForm f;
+            WinDecodeArgs a = decode_args(S, l, dt, b->qkv, b->attn, n, max_len, kv_pitch, f);
             a.tab = tab;
-            launch_decode_win(dt, l.D, a, grouped, st);
+            launch_decode_win(dt, l.D, a, f.grouped, f.wide, st);
         } else routed = stack_mix_decode(r, tab, DecodeFusedSeq{}, n, max_len, b->x, b->qkv, b->attn, b->sw, b, st);
         if (l.parallel() && l.dense()) linear(GemmArgs{b->x, l.wgu, static_cast<char*>(b->attn) + (size_t)l.an * es, nullptr, nullptr, n, 2 * l.ff, H, H, H, l.out_k, 0, l.act()}, l.sw_gu);
         linear(GemmArgs{b->attn, l.wo, b->y, nullptr, nullptr, n, H, l.out_k, l.out_k, l.out_k, H, 0, kActNone}, l.sw_o);

@@ -641,13 +641,13 @@ template <> struct WinMfma<f16_t> {
 };
 constexpr int WIN_GROUP_MAX = 16;                              // query heads of a kv head: the columns of a tile
 // q heads, new key, one row of scratch per wave | the waves' partial rows [wave][head][D], statistics | the waves' tiles (the partial rows take their place after the walk)
-static int win_group_smem(int group, int D) { return ((group + 5) * D + 2 * 4 * 16 + 8 + std::max(4 * 64 * D / 2, 4 * group * D)) * (int)sizeof(float); }
+static int win_group_smem(int group, int D, int nw) { return ((group + 1 + nw) * D + 2 * nw * 16 + 8 + std::max(nw * 64 * D / 2, nw * group * D)) * (int)sizeof(float); }
 
-template <typename T, int D>
-__global__ __launch_bounds__(256) void decode_win_group_kernel(WinDecodeArgs a) {
+template <typename T, int D, int NW>
+__global__ __launch_bounds__(NW * 64) void decode_win_group_kernel(WinDecodeArgs a) {
     extern __shared__ __attribute__((aligned(16))) float wsm[];
     const int group = a.n_heads / a.n_kv_heads;
-    float *qs = wsm, *ks = qs + group * D, *tmp = ks + D, *wm = tmp + 4 * D, *wl = wm + 64, *flag = wl + 64, *wo = flag + 8;      // wo: [wave][head][D] after the walk, [wave] tiles of 64 keys before
+    float *qs = wsm, *ks = qs + group * D, *tmp = ks + D, *wm = tmp + NW * D, *wl = wm + NW * 16, *flag = wl + NW * 16, *wo = flag + 8;      // wo: [wave][head][D] after the walk, [wave] tiles of 64 keys before
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int i16 = lane & 15, q4 = lane >> 4;
     const int kvh = blockIdx.x, split = blockIdx.y, z = blockIdx.z;
@@ -655,7 +655,7 @@ __global__ __launch_bounds__(256) void decode_win_group_kernel(WinDecodeArgs a) 
     int pos = a.pos >= 0 ? a.pos : *e.pos_ptr;
     pos = __builtin_amdgcn_readfirstlane(pos < a.s_max ? pos : a.s_max - 1);
     const int lo = a.window > 0 && pos - a.window + 1 > 0 ? pos - a.window + 1 : 0;
-    const int p0 = lo / 64, np = (pos + 63) / 64 - p0;         // 64-key pieces with a cached key that is seen (np <= 0: none); split's wave w takes 4 split + w, + 4 n_split, ...
+    const int p0 = lo / 64, np = (pos + 63) / 64 - p0;         // 64-key pieces with a cached key that is seen (np <= 0: none); split's wave w takes NW split + w, + NW n_split, ...
     const T* row = reinterpret_cast<const T*>(a.qkv) + (size_t)z * a.qkv_stride;
     T* Kc = reinterpret_cast<T*>(e.K) + (size_t)kvh * a.s_max * D;
     T* Vt = reinterpret_cast<T*>(e.VT) + (size_t)kvh * D * a.s_max;
@@ -695,12 +695,12 @@ __global__ __launch_bounds__(256) void decode_win_group_kernel(WinDecodeArgs a) 
         for (int u = 0; u < NL; ++u) *reinterpret_cast<uint4*>(tile + u * 1024 + lane * 16) = r[u];
         asm volatile("" ::: "memory");                         // the wave's LDS operations retire in order; the compiler must not turn them round either
     };
-    const int first = 4 * split + wave, step = 4 * a.n_split;
+    const int first = NW * split + wave, step = NW * a.n_split;
     load_k(p0 + first, first < np);
     asm volatile("" ::: "memory");                             // keys before values: the order of the walk
     load_v(p0 + first, first < np);
     asm volatile("" ::: "memory");
-    for (int h = wave; h < group + (owner ? 1 : 0); h += 4) {  // the query heads, then the new key
+    for (int h = wave; h < group + (owner ? 1 : 0); h += NW) {  // the query heads, then the new key
         const bool isk = h == group;
         norm_rope_vec<T, D>(row + (isk ? a.n_heads + kvh : kvh * group + h) * D, reinterpret_cast<const T*>(isk ? a.k_norm : a.q_norm), a.eps, a.qk_dim, cs, a.rot_dims, tmp + wave * D,
                             qs + h * D, lane);
@@ -788,7 +788,7 @@ __global__ __launch_bounds__(256) void decode_win_group_kernel(WinDecodeArgs a) 
     }
     // into the caches after the walk: a store in flight (to a pointer out of the table) makes every wait of the walk one for everything
     if (owner) {
-        for (int d = tid; d < D; d += 256) {
+        for (int d = tid; d < D; d += NW * 64) {
             Kc[(size_t)pos * D + d] = from_f32<T>(ks[d]);
             Vt[(size_t)d * a.s_max + pos] = vnew[d];
         }
@@ -808,7 +808,7 @@ __global__ __launch_bounds__(256) void decode_win_group_kernel(WinDecodeArgs a) 
             acc[d] = acc[d] * alpha + vv * (pn * UP);
         }
     }
-    // ---- the four waves, then the splits ----
+    // ---- the waves, then the splits ----
     l = fold16(l, OpSum{}); l = fold32(l, OpSum{});
     if (q4 == 0) { wm[wave * 16 + i16] = m; wl[wave * 16 + i16] = l; }
     __syncthreads();                                           // every wave is done with its tile: the partial rows take their place
@@ -820,14 +820,14 @@ __global__ __launch_bounds__(256) void decode_win_group_kernel(WinDecodeArgs a) 
     constexpr int WS = D + 4;
     T* out = reinterpret_cast<T*>(a.out) + (size_t)z * a.out_stride + kvh * group * D;
     auto gate = [&](int h) { return a.gate_off >= 0 ? sigmoid_f32(to_f32(row[a.gate_off + kvh * group + h])) : 1.f; };
-    for (int i = tid; i < group * D; i += 256) {
+    for (int i = tid; i < group * D; i += NW * 64) {
         const int h = i / D, d = i % D;
         float M = -INFINITY, lt = 0.f, o = 0.f;
 #pragma unroll
-        for (int w = 0; w < 4; ++w) M = fmaxf(M, wm[w * 16 + h]);
+        for (int w = 0; w < NW; ++w) M = fmaxf(M, wm[w * 16 + h]);
         const float Ms = M == -INFINITY ? 0.f : M;
 #pragma unroll
-        for (int w = 0; w < 4; ++w) {
+        for (int w = 0; w < NW; ++w) {
             const float f = __builtin_amdgcn_exp2f(wm[w * 16 + h] - Ms);
             lt += f * wl[w * 16 + h]; o += f * wo[(w * group + h) * D + d];
         }
@@ -849,7 +849,7 @@ __global__ __launch_bounds__(256) void decode_win_group_kernel(WinDecodeArgs a) 
     if (tid == 0) flag[0] = __hip_atomic_fetch_add(ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == a.n_split - 1 ? 1.f : 0.f;
     __syncthreads();
     if (flag[0] == 0.f) return;
-    for (int i = tid; i < group * D; i += 256) {
+    for (int i = tid; i < group * D; i += NW * 64) {
         const int h = i / D, d = i % D;
         const float* wsh = e.ws + (size_t)(kvh * group + h) * a.n_split * WS;
         float M = -INFINITY, lt = 0.f, o = 0.f;
@@ -891,6 +891,8 @@ bool decode_win_groups(int dtype, int D, int n_heads, int n_kv_heads, int n_seq)
 //    8 heads on  1          32 of 600   34 -> 15                  8 of 600  14 -> 15     2 of 600  12 -> 15      8 of 60  9 -> 12     (16 on 1: 16 of 600 25 -> 20, 4 of 600 13 -> 20)
 // so: up to groups of four from one chunk of keys on, larger groups by the bytes that one head a workgroup asks for (the merge grows with the group); shorter contexts only where
 // a group is three or four.  One sequence of 601 keys, 16 heads on 4: 11.1 us either way (9.7 since sums over lanes pass LDS by), all of it latency, so the form with more workgroups stays.
+// Eight waves instead of four: where a workgroup has a CU to itself and each of eight still walks more than one piece.  32 sequences of 600 .. 1024 keys, 8 kv heads: 31.4 -> 29.3 us
+// a launch (4.6 TB/s of keys and values); steps of 4 layers at up to 8 pieces a workgroup are 0 .. 1.5 % slower with eight (a longer merge for the same walk).
 // Splits: as many as make ONE round of workgroups of the grouped kernel (its waves fill a CU: 96 x 3 and 160 x 2 workgroups took a second round, 15 -> 19 and 21 -> 25 us).
 WinForm decode_win_form(int dtype, int D, int n_heads, int n_kv_heads, int n_seq, int span) {
     const int group = n_heads / n_kv_heads, chunks = std::max(1, std::min((span + 127) / 128, DF_MAX_SPLIT));
@@ -898,11 +900,11 @@ WinForm decode_win_form(int dtype, int D, int n_heads, int n_kv_heads, int n_seq
     bool grouped = decode_win_groups(dtype, D, n_heads, n_kv_heads, n_seq);
     if (group <= 4) grouped = grouped && (span >= 128 || (group >= 3 && mb >= 10));
     else grouped = grouped && mb >= 0.6 * group * group;
-    const int wgs = (grouped ? n_kv_heads : n_heads) * n_seq;
-    return WinForm{grouped, std::max(1, std::min(chunks, grouped ? 256 / wgs : (1024 + wgs - 1) / wgs))};
+    const int wgs = (grouped ? n_kv_heads : n_heads) * n_seq, n_split = std::max(1, std::min(chunks, grouped ? 256 / wgs : (1024 + wgs - 1) / wgs));
+    return WinForm{grouped, n_split, grouped && wgs * n_split <= 256 && span > 8 * 64 * n_split};
 }
 
-void launch_decode_win(int dtype, int D, const WinDecodeArgs& a, bool grouped, hipStream_t st) {
+void launch_decode_win(int dtype, int D, const WinDecodeArgs& a, bool grouped, bool wide, hipStream_t st) {
     LMX_REQUIRE(D == 64 || D == 128 || D == 256, "decode_win: padded head width must be 64, 128 or 256");
     LMX_REQUIRE(a.s_max % DF_CHUNK == 0 && a.n_split >= 1 && a.n_split <= DF_MAX_SPLIT && a.n_seq >= 1, "decode_win: cache in whole 128-key chunks, 1..32 splits");
     LMX_REQUIRE(a.n_heads >= 1 && a.n_kv_heads >= 1 && a.n_heads % a.n_kv_heads == 0 && a.qkv && a.out, "decode_win: bad arguments");
@@ -910,17 +912,19 @@ void launch_decode_win(int dtype, int D, const WinDecodeArgs& a, bool grouped, h
     LMX_REQUIRE(a.tab || (a.n_seq == 1 && a.one.K && a.one.VT && a.one.ws && a.one.counters && (a.pos >= 0 || a.one.pos_ptr)), "decode_win: bad sequence");
     if (grouped && decode_win_groups(dtype, D, a.n_heads, a.n_kv_heads, a.n_seq) && a.qkv_stride % 4 == 0 && reinterpret_cast<uintptr_t>(a.qkv) % 8 == 0) {
         const dim3 grid(a.n_kv_heads, a.n_split, a.n_seq);
-        const int smem = win_group_smem(a.n_heads / a.n_kv_heads, D);
-#define L(TT, DD)                                                                                                                                          \
+        const int group = a.n_heads / a.n_kv_heads;
+#define L(TT, DD, NWV)                                                                                                                                     \
     do {                                                                                                                                                   \
         static bool attr_set = false;                                                                                                                      \
         if (!attr_set) {                                                                                                                                   \
-            LMX_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&decode_win_group_kernel<TT, DD>), hipFuncAttributeMaxDynamicSharedMemorySize, win_group_smem(WIN_GROUP_MAX, DD))); \
+            LMX_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&decode_win_group_kernel<TT, DD, NWV>), hipFuncAttributeMaxDynamicSharedMemorySize, win_group_smem(WIN_GROUP_MAX, DD, NWV))); \
             attr_set = true;                                                                                                                               \
         }                                                                                                                                                  \
-        LMX_LAUNCH((decode_win_group_kernel<TT, DD>), grid, dim3(256), smem, st, a);                                                                       \
+        LMX_LAUNCH((decode_win_group_kernel<TT, DD, NWV>), grid, dim3(NWV * 64), win_group_smem(group, DD, NWV), st, a);                                   \
     } while (0)
-        if (dtype == kBF16) { if (D == 128) L(bf16_t, 128); else L(bf16_t, 64); } else { if (D == 128) L(f16_t, 128); else L(f16_t, 64); }
+#define LD(TT) do { if (wide) { if (D == 128) L(TT, 128, 8); else L(TT, 64, 8); } else if (D == 128) L(TT, 128, 4); else L(TT, 64, 4); } while (0)
+        if (dtype == kBF16) LD(bf16_t); else LD(f16_t);
+#undef LD
 #undef L
         LMX_CHECK_HIP(hipGetLastError());
         return;

@@ -18,7 +18,8 @@
 // lane offset + scalar offset): as 64-bit pointers the 32 addresses of a piece cost 64 registers.  After the loop: one barrier, the four wave states + the NEW key (rotated
 // from the qkv row, value from the qkv row) are merged by threads d < D, and one workgroup per kv head appends the new key / value to the caches.
 // Bound: the cache stream.  16 sequences of 516 - 1090 keys, 32 heads: 48.3 us a launch with a piece's loads requested together and plain, rows of V^T 4 KiB apart; 47.6 with
-// the prefetch and the dealt-out sums; 43.2 (4.9 TB/s) with loads marked streaming and rows 4.25 KiB apart (Model::kv_pitch).  The same loads with no arithmetic: 38.7.
+// the prefetch and the dealt-out sums; 43.2 (4.9 TB/s) with loads marked streaming and rows 4.25 KiB apart (Model::kv_pitch); 40.9 with the sequences in
+// batch_attn_order.  The same loads with no arithmetic, sequences as they come: 38.7.
 #pragma once
 #include "common.h"
 #include "kernels.h"
@@ -50,11 +51,11 @@ constexpr int BA_NW = 4;          // waves per workgroup
 // decode batch: grid (heads, sequences); K / V^T / position of sequence z from the per-layer table, q|k|v and output rows by stride
 // NT: the loads are marked streaming, where no other workgroup reads the same keys
 template <typename T, bool NT>
-__global__ __launch_bounds__(BA_NW * 64) void decode_attn_wave_kernel(DecodeFusedArgs a) {
+__global__ __launch_bounds__(BA_NW * 64) void decode_attn_wave_kernel(DecodeFusedArgs a, BatchOrder order) {
     constexpr int D = 128, NW = BA_NW;
     __shared__ __attribute__((aligned(16))) float p_lds[NW][BA_PIECE];      // wave-private: probabilities of the current piece, by key
     __shared__ float part[NW + 1][D + 2];                                    // wave states (o[D], m, l) + the new key's
-    const int zseq = blockIdx.y, head = blockIdx.x;
+    const int zseq = order.z[blockIdx.y], head = blockIdx.x;
     const DecodeFusedSeq e = a.tab[zseq];
     int pos = *e.pos_ptr;                                                   // keys [0, pos) are cached; this token's key goes to row pos
     pos = pos < a.s_max ? pos : a.s_max - 1;                                // the host keeps len + steps <= s_max; never index past the cache whatever the device word holds
@@ -215,9 +216,19 @@ __global__ __launch_bounds__(BA_NW * 64) void decode_attn_wave_kernel(DecodeFuse
 // 7.62**, 4 or 8 waves x 4 heads 25 - 30 % slower: two independent 4-wave workgroups per CU, one head each, drift apart, so one's merge tail and start-up run under the
 // other's stream; walking several heads per workgroup only lengthens the tail.
 template <typename T>
-inline void launch_decode_attn_wave_t(const DecodeFusedArgs& a, hipStream_t st) {
-    if (a.n_heads == a.n_kv_heads) hipLaunchKernelGGL((decode_attn_wave_kernel<T, true>), dim3(a.n_heads, a.n_seq), dim3(BA_NW * 64), 0, st, a);
-    else hipLaunchKernelGGL((decode_attn_wave_kernel<T, false>), dim3(a.n_heads, a.n_seq), dim3(BA_NW * 64), 0, st, a);
+inline void launch_decode_attn_wave_t(const DecodeFusedArgs& all, hipStream_t st) {
+    constexpr int MOST = (int)sizeof(BatchOrder::z);
+    for (int z0 = 0; z0 < all.n_seq; z0 += MOST) {                          // (an engine's batch is one launch)
+        DecodeFusedArgs a = all;
+        a.n_seq = all.n_seq - z0 < MOST ? all.n_seq - z0 : MOST;
+        a.tab = all.tab + z0;
+        a.QKV = static_cast<const T*>(all.QKV) + (size_t)z0 * all.qkv_stride;
+        a.O = static_cast<T*>(all.O) + (size_t)z0 * all.o_stride;
+        BatchOrder o;
+        for (int z = 0; z < a.n_seq; ++z) o.z[z] = all.order && all.n_seq <= MOST ? all.order[z] : (uint8_t)z;
+        if (a.n_heads == a.n_kv_heads) hipLaunchKernelGGL((decode_attn_wave_kernel<T, true>), dim3(a.n_heads, a.n_seq), dim3(BA_NW * 64), 0, st, a, o);
+        else hipLaunchKernelGGL((decode_attn_wave_kernel<T, false>), dim3(a.n_heads, a.n_seq), dim3(BA_NW * 64), 0, st, a, o);
+    }
 }
 
 }  // namespace lmx

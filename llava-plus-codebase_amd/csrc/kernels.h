@@ -165,6 +165,7 @@ void launch_attn_probs(int dtype, int D, const AttnProbsArgs& a, hipStream_t st)
 // launch (agent-scope counter protocol), so there is no separate combine launch.
 // decode batch (continuous batching): per-sequence pointers of ONE layer; workgroup (head, split, z) serves sequence z
 struct DecodeFusedSeq { void* K; void* VT; const int* pos_ptr; float* ws; int* counters; const int* done = nullptr; };      // done: the sequence's stop flag (recurrent state stands still once it is set)
+struct BatchOrder { uint8_t z[256]; };        // sequence of each row of workgroups, by value (a decode batch holds 256 at most)
 struct DecodeFusedArgs {
     const void* QKV;       // [qkv_n] row of this token: q heads | k heads | v heads (pre-RoPE)
     void* K;               // caches of this layer (the new key/value are appended at *pos_ptr)
@@ -180,9 +181,11 @@ struct DecodeFusedArgs {
     // batch form: tab != null => n_seq sequences in one launch; K / VT / pos_ptr / ws / counters come from tab[z], QKV and O are
     // [n_seq] rows with the given element strides
     const DecodeFusedSeq* tab = nullptr;
+    const uint8_t* order = nullptr;      // host: n_seq sequence indices in the order of launch (null: as they are)
     int n_seq = 1, qkv_stride = 0, o_stride = 0;
 };
 void launch_decode_fused(int dtype, int D, const DecodeFusedArgs& a, hipStream_t st);
+void batch_attn_order(const int* len, int n_seq, int n_heads, uint8_t* order);      // DecodeFusedArgs::order for sequences of these lengths (256 at most)
 size_t decode_fused_ws_floats(int n_heads, int n_split, int D);
 size_t decode_attn_ws_floats(int n_rows, int n_heads, int n_split, int D);
 

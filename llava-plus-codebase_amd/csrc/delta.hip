@@ -22,6 +22,7 @@
 #include "common.h"
 #include "kernels.h"
 #include "moe_pick.h"
+#include "gemv2.h"
 
 namespace lmx {
 
@@ -418,14 +419,11 @@ void launch_delta_gate(int dtype, const DeltaPrefillArgs& a, hipStream_t st) {
 // one new token per sequence: grid (heads, sequences), NTH threads
 // ---------------------------------------------------------------------------------------------------------------
 template <typename T, int LPC, int NTH>
-__global__ __launch_bounds__(NTH, NTH == 512 && sizeof(T) == 2 ? 4 : 1) void delta_decode_kernel(DeltaDecodeArgs a) {
+__device__ __forceinline__ void delta_decode_head(const DeltaDecodeArgs& a, int h, int z, float* sm, float* red) {
     constexpr int DK = LPC * 8, CPP = NTH / LPC, PF = 2048 / NTH, RP = 2048 / NTH;      // columns of one pass over the state, passes in flight, low-rank rows at a time
-    if ((int)blockIdx.x == a.s.H) { moe_router_row<T, NTH / 64>(a.router, blockIdx.y); return; }
-    extern __shared__ __attribute__((aligned(16))) float sm[];
-    __shared__ float red[NTH / 64];
     const int tid = threadIdx.x;
     const int H = a.s.H, G = a.s.G, DV = a.s.DV, taps = a.s.taps, C = a.s.channels();
-    const int h = blockIdx.x, z = blockIdx.y, rep = H / G, kh = h / rep;
+    const int rep = H / G, kh = h / rep;
     float *q = sm, *k = q + DK, *g = k + DK, *v = g + DK, *gate = v + DV, *o = gate + DV;
     const DecodeFusedSeq e = a.tab ? a.tab[z] : a.one;
     const T* row = reinterpret_cast<const T*>(a.proj) + (size_t)z * a.ld;
@@ -593,20 +591,42 @@ __global__ __launch_bounds__(NTH, NTH == 512 && sizeof(T) == 2 ? 4 : 1) void del
     for (int c = tid; c < DV; c += NTH) out[c] = from_f32<T>(o[c] * inv * to_f32(c == tid ? norm_w : reinterpret_cast<const T*>(a.w.norm)[c]) * gate[c]);
 }
 
+template <typename T, int LPC, int NTH>
+__global__ __launch_bounds__(NTH, NTH == 512 && sizeof(T) == 2 ? 4 : 1) void delta_decode_kernel(DeltaDecodeArgs a) {
+    extern __shared__ __attribute__((aligned(16))) float sm[];
+    __shared__ float red[NTH / 64];
+    if ((int)blockIdx.x == a.s.H) { moe_router_row<T, NTH / 64>(a.router, blockIdx.y); return; }
+    delta_decode_head<T, LPC, NTH>(a, blockIdx.x, blockIdx.y, sm, red);
+}
+
+// One sequence's step beside a linear that reads the layer's normalised row too (a parallel layer's gate | up): the heads' workgroups are the first of the launch, the linear's, sixteen
+// waves of R rows, follow.  The step is a chain of latencies on 16 .. 32 CUs, the linear a stream that wants the others; in launches of their own each waits for the other's end.
+template <typename T, int LPC, int R>
+__global__ __launch_bounds__(1024) void delta_decode_linear_kernel(DeltaDecodeArgs a, GemvArgs g) {
+    extern __shared__ __attribute__((aligned(16))) float sm[];
+    __shared__ float red[16];
+    if ((int)blockIdx.x < a.s.H) delta_decode_head<T, LPC, 1024>(a, blockIdx.x, 0, sm, red);
+    else gemv2_body<T, R, 4, 1, false, false, 16>(g, (int)blockIdx.x - a.s.H, reinterpret_cast<char*>(sm), nullptr, 0u);
+}
+
 static bool one_round(const DeltaShape& s, int n_seq) { return s.H * n_seq <= 256; }
 // past one round the routers are a tail of their own: 32 x 32 heads x sequences 39.1 us without, 50.4 with them, 9.8 alone; in one round (16 x 1) 9.9 either way, 8.1 alone.  On the line,
 // where the routers' own workgroups are the ones past the round, they still cost less than their launches: a decode step with two of them, 16 x 16 728 us in the step's launch, 734 in
 // their own; 32 x 8 1458, 1461
 bool delta_decode_routes(const DeltaShape& s, int n_seq) { return one_round(s, n_seq); }
-void launch_delta_decode(int dtype, const DeltaDecodeArgs& a, hipStream_t st) {
+static size_t delta_decode_smem(const DeltaShape& s) { return (size_t)(3 * s.DK + 3 * s.DV) * 4; }
+static void delta_decode_check(const DeltaDecodeArgs& a) {
     delta_check(a.s);
     LMX_REQUIRE(a.ra % 64 == 0 && a.rg % 64 == 0 && a.ra >= 64 && a.rg >= 64 && a.wag_ld >= a.ra + a.rg && a.wag_ld % 8 == 0, "delta_decode: low-rank widths in whole 64-column groups");
     LMX_REQUIRE(a.a_off >= a.s.channels() + a.s.H && a.ld >= a.a_off + a.ra + a.rg, "delta_decode: bad row pitch");
     LMX_REQUIRE(a.n_seq >= 1 && (a.tab || (a.n_seq == 1 && a.one.K && a.one.VT && a.one.pos_ptr)), "delta_decode: bad sequence");
+    LMX_REQUIRE(delta_decode_smem(a.s) <= 60 * 1024 && a.a_off % 8 == 0, "delta_decode: head widths too large");
+}
+void launch_delta_decode(int dtype, const DeltaDecodeArgs& a, hipStream_t st) {
+    delta_decode_check(a);
     check_router(a.router);
     const dim3 grid(a.s.H + (a.router.x ? 1 : 0), a.n_seq);
-    const size_t smem = (size_t)(3 * a.s.DK + 3 * a.s.DV) * 4;
-    LMX_REQUIRE(smem <= 60 * 1024 && a.a_off % 8 == 0, "delta_decode: head widths too large");
+    const size_t smem = delta_decode_smem(a.s);
 #define L(TT, NTH) do { if (a.s.DK == 64) LMX_LAUNCH((delta_decode_kernel<TT, 8, NTH>), grid, dim3(NTH), smem, st, a); \
                         else if (a.s.DK == 128) LMX_LAUNCH((delta_decode_kernel<TT, 16, NTH>), grid, dim3(NTH), smem, st, a); \
                         else LMX_LAUNCH((delta_decode_kernel<TT, 32, NTH>), grid, dim3(NTH), smem, st, a); } while (0)
@@ -617,6 +637,24 @@ void launch_delta_decode(int dtype, const DeltaDecodeArgs& a, hipStream_t st) {
     LMX_REQUIRE(wide || !a.router.x, "delta_decode: no router here");
     if (dtype == kBF16) LN(bf16_t); else if (dtype == kF16) LN(f16_t); else LN(float);
 #undef LN
+#undef L
+    LMX_CHECK_HIP(hipGetLastError());
+}
+
+bool delta_decode_joins(int dtype, const DeltaShape& s, const GemvArgs& g) { return s.H <= 64 && g.K <= 8192 && gemv2_applies(dtype, g); }
+void launch_delta_decode_linear(int dtype, const DeltaDecodeArgs& a, const GemvArgs& g, hipStream_t st) {
+    delta_decode_check(a);
+    LMX_REQUIRE(a.n_seq == 1 && !a.tab && !a.router.x && delta_decode_joins(dtype, a.s, g) && !g.norm_w, "delta_decode_linear: one sequence, a plain linear of the weight stream");
+    LMX_REQUIRE(!act_gated(g.act) || g.N % 64 == 0, "delta_decode_linear: gated rows come in groups of 64");
+    // four rows a wave where that leaves every workgroup a CU of its own (all of a row of 2048 is on the wire at once), two where the workgroups come in rounds
+    const bool four = cdiv(g.N, 64) + a.s.H <= 256;
+    const size_t smem = std::max(delta_decode_smem(a.s), gemv2_smem_bytes(g.K, 2, 16));
+    const dim3 grid(a.s.H + cdiv(g.N, four ? 64 : 32));
+#define L(TT, LPC) do { if (four) LMX_LAUNCH((delta_decode_linear_kernel<TT, LPC, 4>), grid, dim3(1024), smem, st, a, g); \
+                        else LMX_LAUNCH((delta_decode_linear_kernel<TT, LPC, 2>), grid, dim3(1024), smem, st, a, g); } while (0)
+#define LD(TT) do { if (a.s.DK == 64) L(TT, 8); else if (a.s.DK == 128) L(TT, 16); else L(TT, 32); } while (0)
+    if (dtype == kBF16) LD(bf16_t); else LD(f16_t);
+#undef LD
 #undef L
     LMX_CHECK_HIP(hipGetLastError());
 }

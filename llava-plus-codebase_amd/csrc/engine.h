@@ -215,8 +215,8 @@ struct Model {
     void stack_mix_prefill(int r, Seq* const* seqs, const std::vector<Segment>& seg, int fill, const void* x, void* qkv, void* mix, void* scratch, const DevBuf& skw, hipStream_t st);
     size_t stack_mix_scratch(int rows, int keys) const;
     // the same over one new token of every sequence (tab: batch; else `one`), projection rows already there
-    bool stack_mix_decode(int r, const DecodeFusedSeq* tab, const DecodeFusedSeq& one, int n, int max_len, const void* x, void* qkv, void* mix, const StackWs& w, Batch* b, hipStream_t st);
-    void stack_moe(const StackLayer& l, const void* x, int rows, const StackWs& w, const StackProf& pn, hipStream_t st, bool routed = false);      // routed: the mixer's launch chose the experts
+    bool stack_mix_decode(int r, const DecodeFusedSeq* tab, const DecodeFusedSeq& one, int n, int max_len, const void* x, void* qkv, void* mix, const StackWs& w, Batch* b, hipStream_t st, const GemvArgs* beside = nullptr);
+    void stack_moe(const StackLayer& l, const void* x, int rows, const StackWs& w, const StackProf& pn, hipStream_t st, bool routed = false, const GemvArgs* beside = nullptr);      // routed: the mixer's launch chose the experts; beside: a linear in the launch of the first product (few rows)
     MoeRouterArgs stack_router(const StackLayer& l, const void* x, const StackWs& w) const;
     void stack_heads(const GroupGemvArgs& g, int n, hipStream_t st);
     // ---- options a caller may flip on a live model (lmx_model_set_option; defaults from the environment at creation) ----------------------------------

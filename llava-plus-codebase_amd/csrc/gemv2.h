@@ -7,7 +7,7 @@
 // A __device__ body so that two kernels can carry it: gemv2_kernel (gemm.hip: one linear per launch) and decode_kv_attn_kernel (decode_attn.hip: the k|v
 // projection of a decode step next to that step's attention workgroups).  `bid` = this workgroup's index among the linear's workgroups (4 waves x R rows
 // each); PUBLISH: the outputs leave as tagged 8-byte granules (gran[n] = {bits of T, tag}) for a consumer inside the SAME launch instead of as C[n].
-// GEMV2_NX: 16-byte chunks of x per thread (K <= 2048 NX): 2 for the hidden-width inputs of the 7B model, 4 / 6 / 8 up to 8192 / 12288 / 16384.
+// GEMV2_NX: 16-byte chunks of x per thread (K <= 512 NW NX): with four waves 2 for the hidden-width inputs of the 7B model, 4 / 6 / 8 up to 8192 / 12288 / 16384.
 #pragma once
 #include "common.h"
 #include "gemm_common.h"
@@ -16,18 +16,18 @@
 
 namespace lmx {
 
-constexpr size_t gemv2_smem_bytes(int K, int es) { return (size_t)K * es + 16; }
+constexpr size_t gemv2_smem_bytes(int K, int es, int nw = 4) { return (size_t)K * es + 4 * nw; }
 
 // RES (the layer-stack decoders' linears): the input row is not a stored vector but what residual_norm_kernel (stack_ops.hip) would have written — xn = rms_norm(x') pre_w with
 // x' = x_in + mult rms_norm(y) post_w + inject, y = a.X — computed by every workgroup while its first weight rounds are on the wire; one workgroup past the linear's own
 // (residual_row_store) stores x' for the launches that follow, so nobody stores inside the counted stream.
-template <typename T, int R, int P, int GEMV2_NX, bool PUBLISH, bool RES = false>
+template <typename T, int R, int P, int GEMV2_NX, bool PUBLISH, bool RES = false, int NW = 4>
 __device__ __forceinline__ void gemv2_body(const GemvArgs& a, int bid, char* smem, unsigned long long* gran, unsigned tag, unsigned long long* ts = nullptr,
                                            const ResidualNormArgs* rn = nullptr) {
     if (ts && threadIdx.x == 0 && (bid & 31) == 0) __hip_atomic_fetch_min(ts + 6, (unsigned long long)__builtin_amdgcn_s_memrealtime(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);      // debug timeline (decode_attn.hip)
     static_assert(sizeof(T) == 2, "gemv2: 16-bit weights");
     T* xs = reinterpret_cast<T*>(smem);                       // [K]
-    float* red = reinterpret_cast<float*>(smem + (size_t)a.K * sizeof(T));   // 4 floats
+    float* red = reinterpret_cast<float*>(smem + (size_t)a.K * sizeof(T));   // NW floats
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -36,7 +36,7 @@ __device__ __forceinline__ void gemv2_body(const GemvArgs& a, int bid, char* sme
     const T* __restrict__ X = reinterpret_cast<const T*>(a.X);
     const bool silu = act_gated(a.act);
 
-    const int slot0 = (bid * 4 + wave) * R;            // first "row slot" of this wave
+    const int slot0 = (bid * NW + wave) * R;            // first "row slot" of this wave
     int rows[R];
     uint32_t roff[R];                                         // byte offset of each row (wave-uniform: scalar registers)
 #pragma unroll
@@ -66,7 +66,7 @@ __device__ __forceinline__ void gemv2_body(const GemvArgs& a, int bid, char* sme
     if (has_x) {
 #pragma unroll
         for (int i = 0; i < GEMV2_NX; ++i) {
-            const int c = tid + 256 * i;
+            const int c = tid + 64 * NW * i;
             if (c < KC) ws_load_plain(xraw[i], (uint32_t)c * 16u, rsX, 0u);
         }
     }
@@ -76,7 +76,7 @@ __device__ __forceinline__ void gemv2_body(const GemvArgs& a, int bid, char* sme
                      rsR0 = ws_make_rsrc(rn->x_in ? static_cast<const void*>(rn->x_in) : a.W, 0x7fffffffu);
 #pragma unroll
         for (int i = 0; i < GEMV2_NX; ++i) {
-            const int c = tid + 256 * i;
+            const int c = tid + 64 * NW * i;
             if (c >= KC) continue;
             if (has_post) ws_load_plain(praw[i], (uint32_t)c * 16u, rsP, 0u);
             if (rn->inject) ws_load_plain(iraw[i], (uint32_t)c * 16u, rsI, 0u);
@@ -88,7 +88,7 @@ __device__ __forceinline__ void gemv2_body(const GemvArgs& a, int bid, char* sme
     if (a.norm_w) {
 #pragma unroll
         for (int i = 0; i < GEMV2_NX; ++i) {
-            const int c = tid + 256 * i;
+            const int c = tid + 64 * NW * i;
             if (c < KC) ws_load_plain(graw[i], (uint32_t)c * 16u, rsG, 0u);
         }
     }
@@ -114,7 +114,7 @@ __device__ __forceinline__ void gemv2_body(const GemvArgs& a, int bid, char* sme
             float ss = 0.f;
 #pragma unroll
             for (int i = 0; i < GEMV2_NX; ++i) {
-                const int c = tid + 256 * i;
+                const int c = tid + 64 * NW * i;
                 if (c < KC) {
                     ws_wait1<P * R>(xraw[i]);
                     float v[8]; ws_unpack8<T>(xraw[i], v);
@@ -122,12 +122,12 @@ __device__ __forceinline__ void gemv2_body(const GemvArgs& a, int bid, char* sme
                     for (int e = 0; e < 8; ++e) ss += v[e] * v[e];
                 }
             }
-            inv1 = has_post ? rn->mult / sqrtf(block_sum<4>(ss, red) * rH + rn->eps) : rn->mult;
+            inv1 = has_post ? rn->mult / sqrtf(block_sum<NW>(ss, red) * rH + rn->eps) : rn->mult;
         }
         float s2 = 0.f;
 #pragma unroll
         for (int i = 0; i < GEMV2_NX; ++i) {
-            const int c = tid + 256 * i;
+            const int c = tid + 64 * NW * i;
             if (c < KC) {
 #pragma unroll
                 for (int e = 0; e < 8; ++e) xv[i][e] = 0.f;
@@ -157,10 +157,10 @@ __device__ __forceinline__ void gemv2_body(const GemvArgs& a, int bid, char* sme
                 for (int e = 0; e < 8; ++e) s2 += xv[i][e] * xv[i][e];
             }
         }
-        const float inv2 = 1.f / sqrtf(block_sum<4>(s2, red) * rH + rn->eps);
+        const float inv2 = 1.f / sqrtf(block_sum<NW>(s2, red) * rH + rn->eps);
 #pragma unroll
         for (int i = 0; i < GEMV2_NX; ++i) {
-            const int c = tid + 256 * i;
+            const int c = tid + 64 * NW * i;
             if (c < KC) {
                 float g[8];
                 ws_wait1<P * R>(graw[i]); ws_unpack8<T>(graw[i], g);
@@ -174,7 +174,7 @@ __device__ __forceinline__ void gemv2_body(const GemvArgs& a, int bid, char* sme
         float ss = 0.f;
 #pragma unroll
         for (int i = 0; i < GEMV2_NX; ++i) {
-            const int c = tid + 256 * i;
+            const int c = tid + 64 * NW * i;
             if (c < KC) {
                 ws_wait1<P * R>(xraw[i]);                     // everything older than the P x R weight loads = every x load
                 const ws_u32x4 raw = xraw[i];
@@ -187,11 +187,11 @@ __device__ __forceinline__ void gemv2_body(const GemvArgs& a, int bid, char* sme
             }
         }
         if (g) {
-            ss = block_sum<4>(ss, red);
+            ss = block_sum<NW>(ss, red);
             const float inv = rsqrtf(ss / (float)K + a.eps);
 #pragma unroll
             for (int i = 0; i < GEMV2_NX; ++i) {
-                const int c = tid + 256 * i;
+                const int c = tid + 64 * NW * i;
                 if (c < KC) {
                     float v[8], gv[8];
                     load8<T>(xs + c * 8, v);

@@ -289,6 +289,9 @@ struct DeltaDecodeArgs {                 // one new token per sequence, everythi
 };
 bool delta_decode_routes(const DeltaShape& s, int n_seq);
 void launch_delta_decode(int dtype, const DeltaDecodeArgs& a, hipStream_t st);
+// one sequence's step and a linear of the same input row in one launch (16-bit; the router stays out)
+bool delta_decode_joins(int dtype, const DeltaShape& s, const GemvArgs& g);
+void launch_delta_decode_linear(int dtype, const DeltaDecodeArgs& a, const GemvArgs& g, hipStream_t st);
 
 // ---- latent attention (latent.hip): keys and values are linear in a normalised latent row, the only thing that is cached: [s_max][R] ---------------------------------
 struct LatentNormArgs {                  // rows: c_q <- rms_norm(c_q) in place, cache[pos] <- rms_norm(c)
@@ -319,6 +322,9 @@ struct GroupGemvArgs {                   // slot = blockIdx.y.  ids: group = ids
     const int* ids = nullptr; int per_row = 1, groups = 1;
 };
 void launch_group_gemv(int dtype, const GroupGemvArgs& a, int slots, hipStream_t st);
+// a gated grouped product and an independent small linear in one launch (16-bit)
+bool group_gemv_joins(int dtype, const GemvArgs& g);
+void launch_group_gemv_linear(int dtype, const GroupGemvArgs& a, int slots, const GemvArgs& g, hipStream_t st);
 // many rows per group: MFMA tiles.  With a plan (mixtures) tile rows are slots: x row slot / per_row, c row slot; without one every group takes rows [0, rows)
 constexpr int GROUP_MIN_BM = 32;
 struct GroupTile { int group, row0, rows, first, n_tiles; int pad[3]; };      // rows [row0, row0 + rows) of `order`; the group's first tile and tile count

@@ -10,6 +10,7 @@
 #include "kernels.h"
 #include "gemm_common.h"
 #include "moe_pick.h"
+#include "gemv2.h"
 
 namespace lmx {
 
@@ -216,17 +217,16 @@ void launch_group_gemm(int dtype, const GroupGemmArgs& a, int bm, hipStream_t st
 // Gated: a lane group takes the gate row and the up row of its output.
 // ---------------------------------------------------------------------------------------------------------------
 template <typename T, bool GATED, int U>
-__global__ __launch_bounds__(256) void group_gemv_kernel(GroupGemvArgs a, int lpr, int opw) {
-    extern __shared__ __attribute__((aligned(16))) char smem[];
+__device__ __forceinline__ void group_gemv_body(const GroupGemvArgs& a, int lpr, int opw, int slot, int part, char* smem) {
     T* xs = reinterpret_cast<T*>(smem);
-    const int tid = threadIdx.x, slot = blockIdx.x;
+    const int tid = threadIdx.x;
     const int grp = a.ids ? a.ids[slot] : slot % a.groups;
     const size_t xr = a.ids ? slot / a.per_row : slot / a.groups, cr = a.ids ? slot : slot / a.groups;
     const T* x = reinterpret_cast<const T*>(a.X) + xr * a.ldx + (a.ids ? 0 : grp * a.x_group);
     const T* W = reinterpret_cast<const T*>(a.W) + (size_t)grp * a.w_group;
     T* C = reinterpret_cast<T*>(a.C) + cr * a.ldc + (a.ids ? 0 : grp * a.c_group);
     const int outs = GATED ? a.N / 2 : a.N, sub = tid % lpr, per = 256 / lpr;
-    const int o0 = blockIdx.y * opw, o1 = o0 + opw < outs ? o0 + opw : outs;
+    const int o0 = part * opw, o1 = o0 + opw < outs ? o0 + opw : outs;
     // U pieces of a row (both rows, gated) are on their way together, the first ones ahead of the staging of x: piece by piece a row of 2048 was four memory latencies.  Pieces
     // past the row's end re-read its first one and count as zeros.  (us a launch, four slots: 2 x 1408 rows of 2048 12.2 -> 11.6, 2048 rows of 1408 8.1 -> 6.7)
     Chunk8<T> g[U], u[GATED ? U : 1];
@@ -266,30 +266,69 @@ __global__ __launch_bounds__(256) void group_gemv_kernel(GroupGemvArgs a, int lp
         if (sub == 0 && o < o1) C[o] = from_f32<T>(GATED ? gate_mul(a.act, s0, s1) : s0);
     }
 }
+template <typename T, bool GATED, int U>
+__global__ __launch_bounds__(256) void group_gemv_kernel(GroupGemvArgs a, int lpr, int opw) {
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    group_gemv_body<T, GATED, U>(a, lpr, opw, blockIdx.x, blockIdx.y, smem);
+}
 
-void launch_group_gemv(int dtype, const GroupGemvArgs& a, int slots, hipStream_t st) {
-    LMX_REQUIRE(a.X && a.W && a.C && a.N >= 1 && a.K >= 64 && a.K % 8 == 0 && a.ldx % 8 == 0 && a.ldw % 8 == 0 && a.w_group % 8 == 0 && a.x_group % 8 == 0, "group_gemv: bad arguments");
-    LMX_REQUIRE(!act_gated(a.act) || a.N % 64 == 0, "group_gemv: gated rows come in groups of 64");
-    LMX_REQUIRE(a.per_row >= 1 && a.groups >= 1 && (size_t)a.K * dtype_size(dtype) <= 64 * 1024, "group_gemv: bad groups");
-    if (slots <= 0) return;
+// The same beside a small linear that neither reads nor writes what it does (a parallel layer's output projection beside its experts): the linear's workgroups first
+template <typename T, bool GATED, int U>
+__global__ __launch_bounds__(256) void group_gemv_linear_kernel(GroupGemvArgs a, int lpr, int opw, int slots, GemvArgs g, int linear_wgs) {
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int b = (int)blockIdx.x - linear_wgs;
+    if (b < 0) gemv2_body<T, 1, 2, 2, false>(g, blockIdx.x, smem, nullptr, 0u);
+    else group_gemv_body<T, GATED, U>(a, lpr, opw, b % slots, b / slots, smem);
+}
+
+struct GroupGemvForm { int lpr, opw, parts, U; };
+static GroupGemvForm group_gemv_form(const GroupGemvArgs& a, int slots) {
     int lpr = 64;
     while (lpr > 1 && lpr * 8 > a.K) lpr >>= 1;
     const int outs = act_gated(a.act) ? a.N / 2 : a.N, per = 256 / lpr;
     int opw = per;                                           // outputs of a workgroup: more of them while the grid stays large enough
     while (opw < 64 && (long)slots * cdiv(outs, opw * 2) >= 1024) opw *= 2;
-    const dim3 grid(slots, cdiv(outs, opw));
+    const int parts = cdiv(outs, opw);
     // pieces together: up to four, as many as leave the fewest past the end of a row of this length, and one by one where so many workgroups follow each other that their latencies do not
     // count.  us a launch one by one / four always / now, fp32 (16-bit models have few slots here): 16 rows x 16 heads of 512 columns 10.9 / 12.6 / 8.5 and of 128 8.2 / 13.8 / 8.3,
     // 32 rows x 32 heads 22 / 40 / 16.5 and 24 / 40 / 23, 128 slots x 4096 rows of 2752 576 / 618 / 599, 3600 slots x 2048 rows of 1408 1925 / 2128 / 1950 and x 2 x 1408 rows
     // of 2048 7934 / 8181 / 7916
     const int pieces = cdiv(a.K, lpr * 8);
-    const int U = (long)grid.x * grid.y > 4096 ? 1 : pieces <= 4 ? pieces : cdiv(pieces, 3) * 3 < cdiv(pieces, 4) * 4 ? 3 : 4;
-#define L1(TT, G, UU) LMX_LAUNCH((group_gemv_kernel<TT, G, UU>), grid, dim3(256), (size_t)a.K * sizeof(TT), st, a, lpr, opw)
-#define LU(TT, G) do { if (U == 4) L1(TT, G, 4); else if (U == 3) L1(TT, G, 3); else if (U == 2) L1(TT, G, 2); else L1(TT, G, 1); } while (0)
+    const int U = (long)slots * parts > 4096 ? 1 : pieces <= 4 ? pieces : cdiv(pieces, 3) * 3 < cdiv(pieces, 4) * 4 ? 3 : 4;
+    return GroupGemvForm{lpr, opw, parts, U};
+}
+static void group_gemv_check(int dtype, const GroupGemvArgs& a) {
+    LMX_REQUIRE(a.X && a.W && a.C && a.N >= 1 && a.K >= 64 && a.K % 8 == 0 && a.ldx % 8 == 0 && a.ldw % 8 == 0 && a.w_group % 8 == 0 && a.x_group % 8 == 0, "group_gemv: bad arguments");
+    LMX_REQUIRE(!act_gated(a.act) || a.N % 64 == 0, "group_gemv: gated rows come in groups of 64");
+    LMX_REQUIRE(a.per_row >= 1 && a.groups >= 1 && (size_t)a.K * dtype_size(dtype) <= 64 * 1024, "group_gemv: bad groups");
+}
+void launch_group_gemv(int dtype, const GroupGemvArgs& a, int slots, hipStream_t st) {
+    group_gemv_check(dtype, a);
+    if (slots <= 0) return;
+    const GroupGemvForm f = group_gemv_form(a, slots);
+    const dim3 grid(slots, f.parts);
+#define L1(TT, G, UU) LMX_LAUNCH((group_gemv_kernel<TT, G, UU>), grid, dim3(256), (size_t)a.K * sizeof(TT), st, a, f.lpr, f.opw)
+#define LU(TT, G) do { if (f.U == 4) L1(TT, G, 4); else if (f.U == 3) L1(TT, G, 3); else if (f.U == 2) L1(TT, G, 2); else L1(TT, G, 1); } while (0)
 #define L(TT) do { if (act_gated(a.act)) LU(TT, true); else LU(TT, false); } while (0)
     if (dtype == kBF16) L(bf16_t); else if (dtype == kF16) L(f16_t); else L(float);
 #undef L
 #undef LU
+#undef L1
+    LMX_CHECK_HIP(hipGetLastError());
+}
+
+bool group_gemv_joins(int dtype, const GemvArgs& g) { return g.K <= 4096 && g.K % 8 == 0 && (size_t)g.N * g.K <= ((size_t)1 << 25) && !g.norm_w && gemv2_applies(dtype, g); }
+void launch_group_gemv_linear(int dtype, const GroupGemvArgs& a, int slots, const GemvArgs& g, hipStream_t st) {
+    group_gemv_check(dtype, a);
+    LMX_REQUIRE(slots >= 1 && act_gated(a.act) && !act_gated(g.act) && group_gemv_joins(dtype, g), "group_gemv_linear: a gated grouped product and a small plain linear");
+    const GroupGemvForm f = group_gemv_form(a, slots);
+    const int linear_wgs = cdiv(g.N, 4);
+    const dim3 grid(linear_wgs + slots * f.parts);
+    const size_t smem = std::max((size_t)a.K * 2, gemv2_smem_bytes(g.K, 2));
+#define L1(TT, UU) LMX_LAUNCH((group_gemv_linear_kernel<TT, true, UU>), grid, dim3(256), smem, st, a, f.lpr, f.opw, slots, g, linear_wgs)
+#define L(TT) do { if (f.U == 4) L1(TT, 4); else if (f.U == 3) L1(TT, 3); else if (f.U == 2) L1(TT, 2); else L1(TT, 1); } while (0)
+    if (dtype == kBF16) L(bf16_t); else L(f16_t);
+#undef L
 #undef L1
     LMX_CHECK_HIP(hipGetLastError());
 }

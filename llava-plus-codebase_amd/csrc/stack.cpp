@@ -646,6 +646,11 @@ void Model::stack_decode_step(Seq* s, hipStream_t st, int64_t* id_out) {
         linear("decode.gemv.qkv", before, y, top, g, true, l.parallel() && l.ff);      // a parallel layer's other linears read the same row
         top = 0;
         bool routed = false;
+        // a parallel layer's gate | up beside the delta step, its output projection beside the experts' first product: neither waits for the other
+        const GemvArgs gu{s->d_x, l.wgu, static_cast<char*>(s->d_attn) + (size_t)l.an * es, nullptr, nullptr, nullptr, 0.f, 2 * l.ff, H, H, H, l.ff, 0, l.act()};
+        const GemvArgs go{s->d_attn, l.wo, s->d_y, nullptr, nullptr, nullptr, 0.f, H, l.out_k, l.out_k, l.out_k, H, 0, kActNone};
+        const bool par = l.parallel() && opt_stack_fuse, join_gu = par && l.dense() && l.c.mixer == LMX_MIXER_DELTA && delta_decode_joins(dt, l.ds, gu);
+        const bool join_o = par && l.moe() && act_gated(l.act()) && !group_gemm_applies(dt, l.c.top_experts, l.c.experts) && group_gemv_joins(dt, go);
         if (l.c.mixer == LMX_MIXER_ATTENTION) {
             LMX_PROF_K("decode.attn");
             WinForm f;
@@ -653,9 +658,9 @@ void Model::stack_decode_step(Seq* s, hipStream_t st, int64_t* id_out) {
             a.one = stack_seq_ref(r, s);
             a.pos = s->len;
             launch_decode_win(dt, l.D, a, f.grouped, f.wide, st);
-        } else routed = stack_mix_decode(r, nullptr, stack_seq_ref(r, s), 1, s->len, s->d_x, s->d_qkv, s->d_attn, s->sw, nullptr, st);
-        if (l.parallel() && l.dense()) plain("decode.gemv.gate_up", s->d_x, l.wgu, static_cast<char*>(s->d_attn) + (size_t)l.an * es, 2 * l.ff, H, l.act());
-        plain("decode.gemv.o", s->d_attn, l.wo, s->d_y, H, l.out_k);
+        } else routed = stack_mix_decode(r, nullptr, stack_seq_ref(r, s), 1, s->len, s->d_x, s->d_qkv, s->d_attn, s->sw, nullptr, st, join_gu ? &gu : nullptr);
+        if (l.parallel() && l.dense() && !join_gu) { LMX_PROF_K("decode.gemv.gate_up"); launch_gemv(dt, gu, 1, st); }
+        if (!join_o) { LMX_PROF_K("decode.gemv.o"); launch_gemv(dt, go, 1, st); }
         y = s->d_y;
         if (l.ff && !l.parallel()) {
             const StackStep sp = stack_step(S, r, 0, final_norm);
@@ -664,7 +669,7 @@ void Model::stack_decode_step(Seq* s, hipStream_t st, int64_t* id_out) {
                 plain("decode.gemv.down", s->d_act, l.wd, s->d_y, H, l.ff);
             } else { residual(sp, y, 0, false); y = nullptr; }
         }
-        if (l.moe()) { stack_moe(l, s->d_x, 1, s->sw, stack_prof_decode, st, routed); top = l.c.top_experts; }
+        if (l.moe()) { stack_moe(l, s->d_x, 1, s->sw, stack_prof_decode, st, routed, join_o ? &go : nullptr); top = l.c.top_experts; }
         before = stack_step(S, r, l.ff && !l.parallel() ? 1 : 0, final_norm);
     }
     {

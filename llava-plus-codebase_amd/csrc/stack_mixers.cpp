@@ -124,7 +124,7 @@ void Model::stack_mix_prefill(int r, Seq* const* seqs, const std::vector<Segment
 // ---------------------------------------------------------------------------------------------------------------
 // one new token per sequence
 // ---------------------------------------------------------------------------------------------------------------
-bool Model::stack_mix_decode(int r, const DecodeFusedSeq* tab, const DecodeFusedSeq& one, int n, int max_len, const void* x, void* qkv, void* mix, const StackWs& w, Batch* b, hipStream_t st) {
+bool Model::stack_mix_decode(int r, const DecodeFusedSeq* tab, const DecodeFusedSeq& one, int n, int max_len, const void* x, void* qkv, void* mix, const StackWs& w, Batch* b, hipStream_t st, const GemvArgs* beside) {
     Stack& S = *stk;
     const StackLayer& l = S.layers[(size_t)S.runs[(size_t)r].layer];
     const lmx_layer_config& d = l.c;
@@ -140,7 +140,7 @@ bool Model::stack_mix_decode(int r, const DecodeFusedSeq* tab, const DecodeFused
         a.tab = tab; a.one = one; a.n_seq = n; a.eps = S.c.norm_eps;
         if (delta_decode_routes(l.ds, n)) a.router = router;
         LMX_PROF_K(pn.delta);
-        launch_delta_decode(dt, a, st);
+        if (beside) launch_delta_decode_linear(dt, a, *beside, st); else launch_delta_decode(dt, a, st);
         return a.router.x;
     }
     const bool routes = router.x && latent_decode_routes(dt, l.R);
@@ -188,7 +188,7 @@ void Model::stack_heads(const GroupGemvArgs& g, int n, hipStream_t st) {
 // mixture of experts: choices, then both products with the rows as they are (few: weights streamed per row) or sorted by expert (MFMA tiles)
 // ---------------------------------------------------------------------------------------------------------------
 MoeRouterArgs Model::stack_router(const StackLayer& l, const void* x, const StackWs& w) const { return MoeRouterArgs{x, l.wr, l.br, H, H, l.c.experts, l.c.top_experts, w.ids, w.wt}; }
-void Model::stack_moe(const StackLayer& l, const void* x, int rows, const StackWs& w, const StackProf& pn, hipStream_t st, bool routed) {
+void Model::stack_moe(const StackLayer& l, const void* x, int rows, const StackWs& w, const StackProf& pn, hipStream_t st, bool routed, const GemvArgs* beside) {
     const int dt = cfg.dtype, top = l.c.top_experts, E = l.c.experts, slots = rows * top;
     if (!routed) { LMX_PROF_K(pn.router); launch_moe_router(dt, stack_router(l, x, w), rows, st); }
     if (group_gemm_applies(dt, slots, E)) {
@@ -203,7 +203,7 @@ void Model::stack_moe(const StackLayer& l, const void* x, int rows, const StackW
     }
     GroupGemvArgs g{x, l.wgu, w.act, 2 * l.ff, H, H, H, l.ff, (size_t)2 * l.ff * H};
     g.act = l.act(); g.ids = w.ids; g.per_row = top;
-    { LMX_PROF_K(pn.gate_up); launch_group_gemv(dt, g, slots, st); }
+    { LMX_PROF_K(pn.gate_up); if (beside) launch_group_gemv_linear(dt, g, slots, *beside, st); else launch_group_gemv(dt, g, slots, st); }
     GroupGemvArgs o{w.act, l.wd, w.slots, H, l.ff, l.ff, l.ff, H, (size_t)H * l.ff};
     o.ids = w.ids;
     { LMX_PROF_K(pn.down); launch_group_gemv(dt, o, slots, st); }

@@ -302,7 +302,7 @@ int lmx_model_set_option(lmx_model* m, const char* key, int32_t value);
 int lmx_op_gemm(int32_t dtype, const void* x, const void* w, void* c, const void* bias, const void* residual,
                 int32_t M, int32_t N, int32_t K, int32_t ldx, int32_t ldw, int32_t ldc, int32_t ldr, int32_t act, int32_t variant, void* stream);
 /* variant LMX_GEMM_SCRATCH: the choice a prefill makes, which brings scratch for K slices (this entry's own 64 MiB: one stream at a time); variant 0 chooses without.
- * Products of more than 256 rows and more than 640 tiles of 64 x 64 go to the four-wave kernel in either (variant 100 mb + 10 nb + slices: its tiles of 32 mb x 32 nb by number).
+ * Products of more than 256 rows and more than 640 tiles of 64 x 64 (160 .. 256 where K is long) that it makes in the least time go to the four-wave kernel in either (variant 100 mb + 10 nb + slices: its tiles of 32 mb x 32 nb by number).
  * lmx_op_gemm_form: what is launched for contiguous 16-byte aligned operands and `scratch_bytes` of scratch, on the host alone.  form[4]: batch = 0: {2, mb, nb, K slices} of the
  * four-wave kernel, {1, row tiles, weight rows of a workgroup, K slices} of the kernel for few row tiles, {0, 0, 0, K slices} of the others; batch = 1 (linears of a decode
  * batch, M <= 32): {0, 16-row weight tiles of a workgroup, 16-row token tiles, K slices}. */

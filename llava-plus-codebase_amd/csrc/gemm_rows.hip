@@ -343,7 +343,7 @@ size_t gemm_rows_slab_bytes(int M, int N, int S) { return S > 1 ? (size_t)S * M 
 // so: 64 weight rows up to 128 rows, where the weights are the time; 128 above, where the rows' re-reads are; no more than one workgroup per CU; slices of at least 10 slabs,
 // and above 128 rows no slicing of a short K (the slabs of o cost what its weights cost).  Short products (K < 1024, under 4 M weights) are launch time on any form.
 //
-// Of products of more than 256 rows and 640 tiles of 64 x 64 only those with fp32 output come here (and all with LMX_GEMM8P=0): the four-wave tiles take the others (gemm4w.hip, linear_form).
+// Of products past the lines of the four-wave tiles (gemm4w_form) come here those with fp32 output, those that these tiles make in less time (linear_form) and all with LMX_GEMM8P=0.
 //
 // More rows (or what the slices above do not take): tiles of 32 .. 256 rows x 128 weight rows, as many as make ONE round of workgroups, where 256 x 256 tiles would be too few and
 // small tiles several rounds (us, best other form -> here; 16-bit, weights cold):

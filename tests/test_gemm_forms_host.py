@@ -118,3 +118,11 @@ def test_a_four_wave_tile_that_is_not_there(variant):
     any_ = ctypes.c_void_p(4096)
     assert _C.lib.lmx_op_gemm(_C.torch_dtype_code(torch.bfloat16), any_, any_, any_, None, None, 64, 256, 256, 256, 256, 256, 0, 0, variant, None) != 0
     assert "no such tile" in _C.last_error()
+
+
+@pytest.mark.parametrize("M,N,K,tiles", [(385, 2048, 8192, True), (384, 2048, 8192, False), (385, 1472, 8192, True), (385, 1408, 8192, False), (1100, 1024, 5120, True), (1100, 896, 5120, False),
+                                         (1024, 1024, 5120, False), (1100, 1024, 5056, False)])
+def test_a_long_k_moves_the_line(M, N, K, tiles):
+    """Past 384 rows more than 160 tiles of 64 x 64 from a K of 8192 on, more than 256 (and 1024 weights) from 5120 on."""
+    from llava_mi355x import ops
+    assert (ops.gemm_form(torch.bfloat16, M, N, K)[0] == 2) == tiles

@@ -636,11 +636,11 @@ __global__ __launch_bounds__(256) void gemv2_kernel(GemvArgs a) {
 }
 
 // the same linear on a row that is formed in front of it: residual addition and both norms of the layer-stack decoders (gemv2.h RES).  The last workgroup stores x'.
-template <typename T, int R, int P, int GEMV2_NX>
-__global__ __launch_bounds__(256) void gemv2_res_kernel(GemvArgs a, ResidualNormArgs rn) {
+template <typename T, int R, int P, int GEMV2_NX, int NW>
+__global__ __launch_bounds__(64 * NW) void gemv2_res_kernel(GemvArgs a, ResidualNormArgs rn) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    if (blockIdx.x == gridDim.x - 1) { residual_row_store<T>(rn, reinterpret_cast<float*>(smem)); return; }
-    gemv2_body<T, R, P, GEMV2_NX, false, true>(a, (int)blockIdx.x, smem, nullptr, 0u, nullptr, &rn);
+    if (blockIdx.x == gridDim.x - 1) { residual_row_store<T, NW>(rn, reinterpret_cast<float*>(smem)); return; }
+    gemv2_body<T, R, P, GEMV2_NX, false, true, NW>(a, (int)blockIdx.x, smem, nullptr, 0u, nullptr, &rn);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -873,19 +873,25 @@ bool gemv2_applies(int dtype, const GemvArgs& a) {
     return a.K <= 16384 && reinterpret_cast<uintptr_t>(a.X) % 16 == 0;
 }
 
-template <typename T, int R, int P, int NX>
+template <typename T, int R, int P, int NX, int NW>
 static void launch_gemv2_res_rx(const GemvArgs& a, const ResidualNormArgs& rn, hipStream_t st) {
-    auto kern = gemv2_res_kernel<T, R, P, NX>;
+    auto kern = gemv2_res_kernel<T, R, P, NX, NW>;
     static bool attr_set = false;
     if (!attr_set) { LMX_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024)); attr_set = true; }
-    LMX_LAUNCH(kern, dim3(cdiv(a.N, 4 * R) + 1), dim3(256), gemv2_smem_bytes(a.K, (int)sizeof(T)), st, a, rn);
+    LMX_LAUNCH(kern, dim3(cdiv(a.N, NW * R) + 1), dim3(64 * NW), gemv2_smem_bytes(a.K, (int)sizeof(T), NW), st, a, rn);
     LMX_CHECK_HIP(hipGetLastError());
 }
+// Every workgroup forms the row again (20 bytes of it for 16 of a weight row at a width of 2048), so eight waves share it, two rows each; products of few rows, where that leaves CUs idle,
+// take a row a wave, and those of long rows besides four waves as the plain linear.  us a launch, weights cold, four waves of two rows -> here:  3088 x 2048 5.59 -> 5.02
+//   6464 x 2048 8.53 -> 7.96   11264 x 2048 gated 11.74 -> 10.66   7000 x 3072 11.40 -> 9.14   16384 x 3072 gated 20.1 -> 17.1   22016 x 4096 gated 31.2 -> 29.6   (2048 x 2048 3.92: 4.69,
+//   4096 x 4096 8.50: 8.75);  a row a wave  1280 x 2048 3.74 -> 3.46   2048 x 2048 3.92 -> 3.81   4096 x 4096 8.50 -> 7.76   (2048 x 3072 5.09: 5.23, 2048 x 4096 5.72: 5.86).
 template <typename T>
 static void launch_gemv2_res(const GemvArgs& a, const ResidualNormArgs& rn, hipStream_t st) {
-    if (a.K <= 2048) launch_gemv2_res_rx<T, 2, 4, 1>(a, rn, st);
-    else if (a.K <= 4096) launch_gemv2_res_rx<T, 2, 4, 2>(a, rn, st);
-    else launch_gemv2_res_rx<T, 2, 4, 4>(a, rn, st);
+    if (a.K > 4096) { launch_gemv2_res_rx<T, 2, 4, 4, 4>(a, rn, st); return; }
+    if (a.N >= 2560 && (a.K <= 3072 || a.N >= 6144)) launch_gemv2_res_rx<T, 2, 2, 1, 8>(a, rn, st);
+    else if (!act_gated(a.act) && (a.K <= 2048 || a.N >= 4096)) launch_gemv2_res_rx<T, 1, 4, 1, 8>(a, rn, st);
+    else if (a.K <= 2048) launch_gemv2_res_rx<T, 2, 4, 1, 4>(a, rn, st);
+    else launch_gemv2_res_rx<T, 2, 4, 2, 4>(a, rn, st);
 }
 
 bool gemv_residual_applies(int dtype, const GemvArgs& a) {
@@ -903,7 +909,7 @@ void launch_gemv_residual(int dtype, GemvArgs a, const ResidualNormArgs& rn, hip
 
 // The single-row decode linears of 16-bit models take the hand-counted stream.  (R rows per wave, P rounds in flight) per shape from the in-situ sweep
 // of round 3 (tools/mb_decode.py, LLaVA-1.5-7B, per launch incl. ~1.4 us of event pair; gemv_kernel -> gemv2_kernel): q|k|v 20.5 -> 19.1 us (R 2, P 4),
-// gate|up 30.9 -> 29.5 (2, 4), down 19.9 -> 17.8 (1, 8: K = 11008 keeps 8 KB per wave on the wire), lm_head 45.8 -> 42.2 (2, 4), o_proj 8.7 -> 8.8 (1, 2).
+// gate|up 30.9 -> 29.5 (2, 4), down 19.9 -> 17.8 (1, 8: K = 11008 keeps 8 KB per wave on the wire), lm_head 45.8 -> 42.2 (2, 4), o_proj 8.7 -> 8.8 (1, 2; now 1, 4).
 template <typename T>
 static bool launch_gemv2(const GemvArgs& a, hipStream_t st) {
     if constexpr (sizeof(T) != 2) return false;
@@ -912,8 +918,9 @@ static bool launch_gemv2(const GemvArgs& a, hipStream_t st) {
         if (act_gated(a.act)) launch_gemv2_r<T, 2, 4>(a, st);
         else if (a.K >= 8192) launch_gemv2_r<T, 1, 8>(a, st);
         // small linears (<= 32 M weights): o_proj keeps one row per wave (1024 short-lived workgroups); with the RMSNorm fused — the split-q step's q projection — every
-        // workgroup also normalises the whole input row, so half as many workgroups with two rows per wave win: 8.1 -> 7.5 us (profiles/r05_small_gemv_rp.txt)
-        else if ((size_t)a.N * a.K <= ((size_t)1 << 25)) { if (a.norm_w) launch_gemv2_r<T, 2, 4>(a, st); else launch_gemv2_r<T, 1, 2>(a, st); }
+        // workgroup also normalises the whole input row, so half as many workgroups with two rows per wave win: 8.1 -> 7.5 us (profiles/r05_small_gemv_rp.txt).  Four loads of a row
+        // ahead instead of two: 2048 x 5632 6.55 -> 5.72 us, 2048 x 7680 7.97 -> 7.10, rows of 2048 .. 4096 as before (3.82, 5.08, 7.1)
+        else if ((size_t)a.N * a.K <= ((size_t)1 << 25)) { if (a.norm_w) launch_gemv2_r<T, 2, 4>(a, st); else launch_gemv2_r<T, 1, 4>(a, st); }
         else launch_gemv2_r<T, 2, 4>(a, st);
         return true;
     }

@@ -271,8 +271,8 @@ __device__ __forceinline__ void gemv2_body(const GemvArgs& a, int bid, char* sme
     }
 }
 
-// x' of one row to rn.x_out by the 256 threads of the calling workgroup (see RES above) and, where other launches read it too, its normalised row to rn.xn
-template <typename T>
+// x' of one row to rn.x_out by the 64 NW threads of the calling workgroup (see RES above) and, where other launches read it too, its normalised row to rn.xn
+template <typename T, int NW = 4>
 __device__ __forceinline__ void residual_row_store(const ResidualNormArgs& rn, float* red) {
     const T* y = reinterpret_cast<const T*>(rn.y);
     const T* post = reinterpret_cast<const T*>(rn.post_w);
@@ -281,15 +281,15 @@ __device__ __forceinline__ void residual_row_store(const ResidualNormArgs& rn, f
     float inv1 = 0.f;
     if (y) {
         float ss = 0.f;
-        for (int c = tid; c < HC; c += 256) {
+        for (int c = tid; c < HC; c += 64 * NW) {
             float v[8]; load8<T>(y + c * 8, v);
 #pragma unroll
             for (int e = 0; e < 8; ++e) ss += v[e] * v[e];
         }
-        inv1 = post ? rn.mult / sqrtf(block_sum<4>(ss, red) * (1.f / (float)rn.H_real) + rn.eps) : rn.mult;
+        inv1 = post ? rn.mult / sqrtf(block_sum<NW>(ss, red) * (1.f / (float)rn.H_real) + rn.eps) : rn.mult;
     }
     float s2 = 0.f;
-    for (int c = tid; c < HC; c += 256) {
+    for (int c = tid; c < HC; c += 64 * NW) {
         float x[8], v[8], g[8];
         if (rn.x_in) load8<float>(rn.x_in + c * 8, x);
         else {
@@ -312,8 +312,8 @@ __device__ __forceinline__ void residual_row_store(const ResidualNormArgs& rn, f
         for (int e = 0; e < 8; ++e) s2 += x[e] * x[e];
     }
     if (!rn.xn) return;
-    const float inv2 = 1.f / sqrtf(block_sum<4>(s2, red) * (1.f / (float)rn.H_real) + rn.eps);
-    for (int c = tid; c < HC; c += 256) {                    // (every thread reads back what it wrote)
+    const float inv2 = 1.f / sqrtf(block_sum<NW>(s2, red) * (1.f / (float)rn.H_real) + rn.eps);
+    for (int c = tid; c < HC; c += 64 * NW) {                    // (every thread reads back what it wrote)
         float x[8], g[8];
         load8<float>(rn.x_out + c * 8, x); load8<T>(reinterpret_cast<const T*>(rn.pre_w) + c * 8, g);
 #pragma unroll

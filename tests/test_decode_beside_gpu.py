@@ -1,0 +1,61 @@
+"""One sequence's decode step: launches that two products share (csrc/delta.hip: delta_decode_linear_kernel, csrc/moe.hip: group_gemv_linear_kernel) against the launches of their own,
+and the forms of the linear that forms its own row (csrc/gemm.hip: launch_gemv2_res) on both sides of their lines."""
+import ctypes
+
+import pytest
+import torch
+
+from oracle import vizosun_oracle as O
+from vizosun_util import build_config, config, delta, dense, latent, moe, rel, steady_routing
+
+pytestmark = pytest.mark.gpu
+DT = {"bf16": torch.bfloat16, "f16": torch.float16}
+TOL = {"bf16": 4e-2, "f16": 6e-3}
+
+
+def _steps(m, first, n):
+    """logits of n steps, one at a time, behind a prompt of 5 tokens"""
+    from llava_mi355x._C import check, lib, ptr, stream_handle
+    from llava_mi355x.engine_lm import LmxKVCache
+    cache, out = LmxKVCache(m, 1), []
+    e = m.get_model().embed_tokens(torch.tensor(first, device="cuda"))
+    check(lib.lmx_prefill(m._h, cache.seqs[0], ptr(e), len(first), 0, None, 0, 1, stream_handle()), "lmx_prefill")
+    for i in range(n):
+        z = torch.empty((1, m._vocab_cap), dtype=m.logits_dtype, device="cuda")
+        check(lib.lmx_decode(m._h, cache.seqs[0], 3 + i, 1, ptr(z), 1, stream_handle()), "lmx_decode")
+        out.append(z)
+    torch.cuda.synchronize()
+    cache.close()
+    return torch.cat(out)
+
+
+@pytest.mark.parametrize("dt", list(DT))
+@pytest.mark.parametrize("dim", [40, 128, 200])
+@pytest.mark.parametrize("ff", [33, 88, 8064, 8200])
+def test_products_beside_each_other(cuda, dt, dim, ff):
+    """Gate | up in less than one workgroup of 64 rows, in several, on the line between four rows a wave and two, and past it; experts of two layers, one behind latent attention."""
+    cfg = config([delta(4, 2, dim, 40, 3, dense(ff)), delta(3, 3, 64, 48, 4, moe(72, 6, 2)), latent(3, 40, 20, 50, 36, 24, moe(40, 5, 3)), delta(4, 4, dim, dim, 4, dense(ff))], 136, 211)
+    w = steady_routing(cfg, O.make_weights(cfg, 3, (18, 70)))
+    m = build_config(cfg, w, DT[dt], 64)
+    a = _steps(m, [5, 9, 2, 7, 1], 6)
+    m.set_option("stack_fuse", 0)
+    b = _steps(m, [5, 9, 2, 7, 1], 6)
+    assert torch.isfinite(a.float()).all() and rel(a, b.double().cpu()) < TOL[dt] / 8
+
+
+@pytest.mark.parametrize("dt", list(DT))
+@pytest.mark.parametrize("N,H,act", [(8, 2048, 0), (2552, 2048, 0), (2560, 2048, 0), (2560, 3072, 0), (2552, 3072, 0), (2568, 3136, 0), (4088, 4096, 0), (4096, 4096, 0), (6136, 3136, 0),
+                                     (6144, 3136, 0), (6152, 4096, 0), (2496, 2048, 3), (2560, 2048, 3), (2560, 3136, 3), (6144, 4096, 3), (2560, 4160, 0)])
+def test_the_row_and_its_linear(cuda, dt, N, H, act):
+    from llava_mi355x import ops
+    g = torch.Generator(device="cuda").manual_seed(N + H)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    x, y, inj, post, pre = r(1, H), r(1, H).to(DT[dt]), r(1, H).to(DT[dt]), r(H).to(DT[dt]), r(H).to(DT[dt])
+    w, b = (r(N, H) / H ** 0.5).to(DT[dt]), r(N).to(DT[dt])
+    x1, xn = ops.residual_norm(x, y, post, inj, pre, 0.37, 1e-5, dtype=DT[dt])
+    x2, one = ops.gemv_residual(x, y, post, inj, pre, w, 0.37, 1e-5, bias=b, act=act)
+    z = xn.double() @ w.double().t() + b.double()
+    if act:
+        z = z.view(1, -1, 2, 32)
+        z = (z[:, :, 0] * torch.sigmoid(z[:, :, 0]) * z[:, :, 1]).reshape(1, -1)
+    assert rel(x2, x1.double().cpu()) < 1e-6 and rel(one, z.cpu()) < 2 * 2.0 ** (-8 if dt == "bf16" else -11)      # (an element of xn may round the other way)

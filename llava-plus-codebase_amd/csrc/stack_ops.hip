@@ -33,6 +33,16 @@ __global__ __launch_bounds__(256) void residual_norm_kernel(ResidualNormArgs a) 
     const T* post = y || a.top > 0 ? reinterpret_cast<const T*>(a.post_w) : nullptr;
     const T* pre = reinterpret_cast<const T*>(a.pre_w);
     float x[NP][8], yv[NP][8];
+    // Both norms' weights and the injected row are on their way with the rows, four experts' rows at a time: each behind the sum in front of it was a trip to memory of its own
+    Chunk8<T> gp[NP], gn[NP], gi[NP];
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+        const int c = tid + i * 256;
+        if (c >= HC) continue;
+        if (post) gp[i].load(post + c * 8);
+        if (pre) gn[i].load(pre + c * 8);
+        if (inj) gi[i].load(inj + c * 8);
+    }
     float ss = 0.f;
 #pragma unroll
     for (int i = 0; i < NP; ++i) {
@@ -48,11 +58,22 @@ __global__ __launch_bounds__(256) void residual_norm_kernel(ResidualNormArgs a) 
 #pragma unroll
             for (int e = 0; e < 8; ++e) yv[i][e] = 0.f;
         }
-        for (int k = 0; k < a.top; ++k) {
-            const float wk = a.moe_w[(size_t)row * a.top + k];
-            float v[8]; load8<T>(reinterpret_cast<const T*>(a.moe_y) + ((size_t)row * a.top + k) * a.H + c * 8, v);
+        for (int k0 = 0; k0 < a.top; k0 += 4) {
+            Chunk8<T> m[4];
+            float wk[4];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) yv[i][e] = fmaf(wk, v[e], yv[i][e]);
+            for (int k = 0; k < 4; ++k) {
+                const size_t slot = (size_t)row * a.top + (k0 + k < a.top ? k0 + k : k0);
+                wk[k] = a.moe_w[slot];
+                m[k].load(reinterpret_cast<const T*>(a.moe_y) + slot * a.H + c * 8);
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                if (k0 + k >= a.top) continue;
+                float v[8]; m[k].get(v);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) yv[i][e] = fmaf(wk[k], v[e], yv[i][e]);
+            }
         }
         if (post) {
 #pragma unroll
@@ -69,7 +90,7 @@ __global__ __launch_bounds__(256) void residual_norm_kernel(ResidualNormArgs a) 
         for (int i = 0; i < NP; ++i) {
             const int c = tid + i * 256;
             if (c >= HC) continue;
-            float g[8]; load8<T>(post + c * 8, g);
+            float g[8]; gp[i].get(g);
 #pragma unroll
             for (int e = 0; e < 8; ++e) x[i][e] += yv[i][e] * inv * g[e];
         }
@@ -80,7 +101,7 @@ __global__ __launch_bounds__(256) void residual_norm_kernel(ResidualNormArgs a) 
         const int c = tid + i * 256;
         if (c >= HC) continue;
         if (inj) {
-            float g[8]; load8<T>(inj + c * 8, g);
+            float g[8]; gi[i].get(g);
 #pragma unroll
             for (int e = 0; e < 8; ++e) x[i][e] += g[e];
         }
@@ -101,7 +122,7 @@ __global__ __launch_bounds__(256) void residual_norm_kernel(ResidualNormArgs a) 
     for (int i = 0; i < NP; ++i) {
         const int c = tid + i * 256;
         if (c >= HC) continue;
-        float g[8], o[8]; load8<T>(pre + c * 8, g);
+        float g[8], o[8]; gn[i].get(g);
 #pragma unroll
         for (int e = 0; e < 8; ++e) o[e] = x[i][e] * inv2 * g[e];
         store8<T>(xn + c * 8, o);

@@ -133,14 +133,25 @@ __global__ __launch_bounds__(WM * WN * 64) void group_gemm_kernel(GroupGemmArgs 
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
     const int nk = a.K / GEMM_BK;
     const unsigned lds_base = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
+    // Tiles walk K from different places (in step, all of them ask for the same 128 bytes of every weight row at a time), and weights that nearly always have one reader, groups filling
+    // four fifths of a tile in the mean or less, are marked streaming so that the rows stay in L2.  32 rows x 4 of 16 experts, weights cold, us: 5504 x 4096 gated 135 -> 120, 4096 x 2752
+    // 66 -> 56, 2816 x 2048 gated 43 -> 33.5, 2048 x 1408 18 -> 16.5; with two slabs where more than 512 tiles come, all of them resident, 110 (6.5 TB/s of weights) and 54.5.  Tiles of
+    // 64 rows, 5504 x 4096: 50 rows a group 138 -> 119, 64 rows 149: 162.
+    const bool lone = a.plan.n_tiles ? a.rows * 5 <= a.groups * BM * 4 : a.rows <= BM;
+    const int rot = (tile_n * 5 + grp * 3) % nk;
     auto stage = [&](int kt, unsigned buf_off) {             // (inline asm for the reason given in gemm_pipe_kernel: ordering is the counted vmcnt + s_barrier below)
+        int k = kt + rot; k = k < nk ? k : k - nk;
 #pragma unroll
         for (int i = 0; i < PPW; ++i) {
             const unsigned dst = __builtin_amdgcn_readfirstlane(lds_base + buf_off + (wave + NW * i) * 1024);
-            const T* src = gsrc[i] + (size_t)kt * GEMM_BK;
+            const T* src = gsrc[i] + (size_t)k * GEMM_BK;
             unsigned keep;
-            asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
-                         : "=&s"(keep) : "v"(src), "s"(dst) : "memory");
+            if (lone && (wave + NW * i) * 8 >= BM)           // (wave-uniform)
+                asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt\n\ts_mov_b32 m0, %0"
+                             : "=&s"(keep) : "v"(src), "s"(dst) : "memory");
+            else
+                asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
+                             : "=&s"(keep) : "v"(src), "s"(dst) : "memory");
         }
     };
 #pragma unroll
@@ -205,7 +216,9 @@ void launch_group_gemm(int dtype, const GroupGemmArgs& a, int bm, hipStream_t st
     LMX_REQUIRE(!act_gated(a.act) || a.N % 64 == 0, "group_gemm: gated rows come in groups of 64");
     // with a plan: every group's last tile may be part empty; no more tiles than rows
     const int m_tiles = a.plan.n_tiles ? std::min(a.rows, a.rows / bm + a.groups) : a.groups * cdiv(a.rows, bm);
-#define L(TT) do { if (bm == 32) launch_group_gemm_cfg<TT, 32, 128, 1, 2, 4>(a, m_tiles, st); else if (bm == 64) launch_group_gemm_cfg<TT, 64, 128, 2, 2, 3>(a, m_tiles, st); \
+    // two slabs: 2048 x 1408 of 288 tiles 16.5 -> 25.5 us, 2816 x 2048 of 440 33.5 -> 34; 5504 x 4096 at 20 / 24 / 32 rows a group, two tiles for most, 121 / 122 / 154 -> 110 / 111 / 197
+    const bool many = a.plan.n_tiles && a.rows <= 24 * a.groups && m_tiles * cdiv(a.N, 128) > 512;
+#define L(TT) do { if (bm == 32 && many) launch_group_gemm_cfg<TT, 32, 128, 1, 2, 2>(a, m_tiles, st); else if (bm == 32) launch_group_gemm_cfg<TT, 32, 128, 1, 2, 4>(a, m_tiles, st); else if (bm == 64) launch_group_gemm_cfg<TT, 64, 128, 2, 2, 3>(a, m_tiles, st); \
                    else throw Error{"group_gemm: tiles of 32, 64 or 128 .. 256 rows"}; } while (0)
     if (bm > 64 && dtype != kF32) { launch_group_gemm4w(dtype, a, bm, nb, m_tiles, st); return; }
     if (dtype == kBF16) L(bf16_t); else if (dtype == kF16) L(f16_t); else throw Error{"group_gemm: 16-bit models"};

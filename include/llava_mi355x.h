@@ -290,9 +290,10 @@ int lmx_seq_read_tokens(lmx_seq* s, int64_t* host_out, int32_t max_n, int32_t* n
  * bench.py derives its `roofline` objects from this. */
 int lmx_profile_enable(lmx_model* m, int32_t on);
 int lmx_profile_read(lmx_model* m, char* names_buf, int32_t names_cap, double* ms, int64_t* counts, int32_t max_n, int32_t* n_out);
-/* Options of a live model (defaults come from the environment at lmx_create: LMX_FUSE_ROPE, LMX_VIS_PACK, LMX_DECODE_SPLITQ; all default 1).  Every one selects
+/* Options of a live model (defaults come from the environment at lmx_create: LMX_FUSE_ROPE, LMX_FUSE_SLICES, LMX_VIS_PACK, LMX_DECODE_SPLITQ; all default 1).  Every one selects
  * between two launch forms with bit-identical results — the switch exists for A/B timing and for the tests that prove the identity:
  *   "fuse_rope"     RoPE + KV-cache append in the prefill's q|k|v GEMM epilogue (HF5:models/llama/modeling_llama.py:130-160,243-281) vs. a rope_kv launch
+ *   "fuse_slices"   the K slices of a prompt's q|k|v, o and down linears added by the launch that reads their rows (rope_kv, RMSNorm) vs. by a launch of their own
  *   "vis_pack"      CLIP K / V^T pack in the tower's q|k|v GEMM epilogue (HF5:models/clip/modeling_clip.py:295-340) vs. a pack launch
  *   "decode_splitq" decode step of 16-bit models as q launch + (k|v projection with the attention workgroups) launch vs. q|k|v launch + attention launch
  * Unknown keys are an error.  Not to be flipped while requests are in flight on other threads. */

@@ -417,6 +417,7 @@ int lmx_model_set_option(lmx_model* m, const char* key, int32_t value) {
     LMX_REQUIRE(m && key, "null argument");
     const std::string k(key);
     if (k == "fuse_rope") m->impl.opt_fuse_rope = value != 0;
+    else if (k == "fuse_slices") m->impl.opt_fuse_slices = value != 0;
     else if (k == "vis_pack") m->impl.opt_vis_pack = value != 0;
     else if (k == "decode_splitq") m->impl.opt_splitq = value != 0;
     else if (k == "stack_fuse") m->impl.opt_stack_fuse = value != 0;

@@ -194,9 +194,10 @@ void launch_layernorm(int dtype, const void* x, const void* w, const void* b, vo
 //   n_heads <= slot < n_heads + n_kv   : k, rotated, written to K cache [kvh][pos][D]
 //   otherwise                          : v, transposed through LDS into Vᵀ cache [kvh][d][pos] (128-byte key runs); Vᵀ behind the last row is cleared to the end of its 64 keys
 //                                        (the prompt attention reads whole tiles; an earlier sequence's Inf or NaN there would meet probability 0)
+// SLABS: the rows are still the projection's K slices; added here in rows_reduce_kernel's order (139 rows of 32 + 32 + 32 heads in two slices: 5.1 + 5.9 us in two launches -> 6.9).
 // HF rounding chain (model dtype T): cos,sin -> T ; out = T( T(x*cos) + T(rot(x)*sin) ).
 // ---------------------------------------------------------------------------------------------------------------
-template <typename T, int D>
+template <typename T, int D, bool SLABS>
 __global__ __launch_bounds__(256) void rope_kv_kernel(RopeKvArgs a) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int tid = threadIdx.x;
@@ -207,6 +208,21 @@ __global__ __launch_bounds__(256) void rope_kv_kernel(RopeKvArgs a) {
     constexpr int HALF = D / 2;
     constexpr int GPR = HALF / 8;              // 8-pair groups per token row
     const int ntok = (a.T - tok0) < 64 ? (a.T - tok0) : 64;
+    auto row8 = [&](int t, int col, float (&v)[8]) {         // 8 columns of token tok0 + t
+        if constexpr (SLABS) {
+            const float* p = a.slabs + (size_t)(tok0 + t) * a.qkv_stride + col;
+            const size_t step = (size_t)a.T * a.qkv_stride;
+            load8<float>(p, v);
+#pragma unroll 2
+            for (int s = 1; s < a.slices; ++s) {
+                float u[8]; load8<float>(p + s * step, u);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[e] += u[e];
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = round_to<T>(v[e]);
+        } else load8<T>(qkv + (size_t)(tok0 + t) * a.qkv_stride + col, v);
+    };
 
     if (slot < a.n_heads + a.n_kv_heads) {
         const bool is_k = slot >= a.n_heads;
@@ -218,7 +234,7 @@ __global__ __launch_bounds__(256) void rope_kv_kernel(RopeKvArgs a) {
             const int pos = pos0 + tok0 + t;
             T* xp = qkv + (size_t)(tok0 + t) * a.qkv_stride + col0;
             float x1[8], x2[8];
-            load8<T>(xp + i0, x1); load8<T>(xp + HALF + i0, x2);
+            row8(t, col0 + i0, x1); row8(t, col0 + HALF + i0, x2);
             float o1[8], o2[8];
             if (a.cos_sin) {
                 const float* cs = a.cos_sin + (size_t)pos * D;
@@ -236,7 +252,7 @@ __global__ __launch_bounds__(256) void rope_kv_kernel(RopeKvArgs a) {
                 T* kp = kc + (size_t)pos * D;
                 store8<T>(kp + i0, o1); store8<T>(kp + HALF + i0, o2);
                 if (a.k_inplace && a.cos_sin) { store8<T>(xp + i0, o1); store8<T>(xp + HALF + i0, o2); }
-            } else if (a.cos_sin) {
+            } else if (a.cos_sin || SLABS) {
                 store8<T>(xp + i0, o1); store8<T>(xp + HALF + i0, o2);
             }
         }
@@ -251,7 +267,7 @@ __global__ __launch_bounds__(256) void rope_kv_kernel(RopeKvArgs a) {
     for (int g = tid; g < 64 * (D / 8); g += 256) {
         const int t = g / (D / 8), c = (g % (D / 8)) * 8;
         if (t >= ntok) continue;
-        float v[8]; load8<T>(qkv + (size_t)(tok0 + t) * a.qkv_stride + col0 + c, v);
+        float v[8]; row8(t, col0 + c, v);
 #pragma unroll
         for (int e = 0; e < 8; ++e) tile[t * PITCH + c + e] = from_f32<T>(v[e]);
     }
@@ -275,10 +291,13 @@ void launch_rope_kv(int dtype, int D, const RopeKvArgs& a, hipStream_t st) {
     if (a.T <= 0) return;
     const dim3 grid(cdiv(a.T, 64), a.n_heads + 2 * a.n_kv_heads);
     const size_t smem = (size_t)64 * (D + 2) * dtype_size(dtype);
-#define L(TT, DD) hipLaunchKernelGGL((rope_kv_kernel<TT, DD>), grid, dim3(256), smem, st, a)
-    if (dtype == kBF16) { if (D == 128) L(bf16_t, 128); else L(bf16_t, 64); }
-    else if (dtype == kF16) { if (D == 128) L(f16_t, 128); else L(f16_t, 64); }
-    else { if (D == 128) L(float, 128); else L(float, 64); }
+#define L(TT, DD, SL) hipLaunchKernelGGL((rope_kv_kernel<TT, DD, SL>), grid, dim3(256), smem, st, a)
+#define LS(TT, DD) do { if (a.slabs) L(TT, DD, true); else L(TT, DD, false); } while (0)
+    if (a.slabs) LMX_REQUIRE(a.slices >= 1 && !a.k_inplace && dtype != kF32, "rope_kv: slices of a 16-bit projection");
+    if (dtype == kBF16) { if (D == 128) LS(bf16_t, 128); else LS(bf16_t, 64); }
+    else if (dtype == kF16) { if (D == 128) LS(f16_t, 128); else LS(f16_t, 64); }
+    else { if (D == 128) L(float, 128, false); else L(float, 64, false); }
+#undef LS
 #undef L
     LMX_CHECK_HIP(hipGetLastError());
 }

@@ -44,6 +44,7 @@ Model::Model(const lmx_config& c) : cfg(c) {
     es = les = (int)dtype_size(c.dtype);
     // defaults of the options lmx_model_set_option can flip later (A/B runs and the bit-identity tests of the fused forms)
     { const char* e = getenv("LMX_FUSE_ROPE"); if (e) opt_fuse_rope = atoi(e) != 0; }
+    { const char* e = getenv("LMX_FUSE_SLICES"); if (e) opt_fuse_slices = atoi(e) != 0; }
     { const char* e = getenv("LMX_VIS_PACK"); if (e) opt_vis_pack = atoi(e) != 0; }
     { const char* e = getenv("LMX_DECODE_SPLITQ"); if (e) opt_splitq = atoi(e) != 0; }
     { const char* e = getenv("LMX_TP_OVERLAP"); if (e) { tp_overlap = atoi(e) != 0; tp_overlap_force = atoi(e) == 2; } }
@@ -625,21 +626,37 @@ void Model::prefill(Seq* s, const void* embeds, int T, int chunk, void* logits, 
         // rows [r0, r0+n) of this chunk through the attention block / the MLP block of layer l (partial sums land in h)
         auto rows = [&](void* base, int r0, size_t width) { return static_cast<char*>(base) + (size_t)r0 * width * es; };
         const bool tp_active = cfg.tp_world > 1 || comm != nullptr;
-        auto attn_block = [&](int l, int r0, int n) {
+        // the linear that closes a block, and the norm of its rows if its K slices are still to be added (next: that norm; null: the sum is not this launch's to finish)
+        auto close_block = [&](const GemmArgs& g, const void* next, void* xr, const char* name) {
+            int slices = 0;
+            { LMX_PROF_K(name); if (next) slices = launch_gemm_slices(dt, g, gv, st); else launch_gemm(dt, g, gv, st); }
+            if (slices) { LMX_PROF("prefill.rmsnorm"); launch_rows_reduce_norm(dt, g, slices, next, xr, cfg.rms_eps, st); }
+            return slices > 0;
+        };
+        // normed: x holds the block's normed rows already; returns that for the next block
+        auto attn_block = [&](int l, int r0, int n, const void* next = nullptr, bool normed = false) {
             const DecLayerW& w = dec[l];
             void* kc = s->kc.as<char>() + (size_t)l * s->layer_stride;
             void* vt = s->vt.as<char>() + (size_t)l * s->layer_stride;
             void *hr = rows(h, r0, H), *xr = rows(x, r0, H), *qr = rows(qkv, r0, qkv_n), *ar = rows(attn, r0, (size_t)nh_l * D);
-            { LMX_PROF("prefill.rmsnorm"); launch_rmsnorm(dt, hr, w.ln1, xr, n, H, H, H, cfg.rms_eps, st); }
+            if (!normed) { LMX_PROF("prefill.rmsnorm"); launch_rmsnorm(dt, hr, w.ln1, xr, n, H, H, H, cfg.rms_eps, st); }
             // RoPE + KV-cache append ride in the q|k|v GEMM's epilogue where that launch is the un-split ping-pong kernel over head-aligned tiles
             const bool qf = gv == 0 && opt_fuse_rope && gemm_fuses_qkv(dt, n, H, D, nh_l, nkv_l, pos0 + r0, kv_pitch, false);
+            int slices = 0;
             {
                 LMX_PROF_K("prefill.gemm.qkv");
                 GemmArgs g = with_scratch(GemmArgs{xr, w.wqkv, qr, nullptr, nullptr, n, qkv_n, H, H, H, qkv_n, 0, kActNone});
-                if (qf) { g.qf_rope = rope; g.qf_kc = kc; g.qf_vt = vt; g.qf_pos0 = pos0 + r0; g.qf_nh = nh_l; g.qf_nkv = nkv_l; g.qf_smax = kv_pitch; g.qf_D = D; }
-                launch_gemm(dt, g, gv, st);
+                if (qf) {
+                    g.qf_rope = rope; g.qf_kc = kc; g.qf_vt = vt; g.qf_pos0 = pos0 + r0; g.qf_nh = nh_l; g.qf_nkv = nkv_l; g.qf_smax = kv_pitch; g.qf_D = D;
+                    launch_gemm(dt, g, gv, st);
+                } else if (opt_fuse_slices) slices = launch_gemm_slices(dt, g, gv, st);
+                else launch_gemm(dt, g, gv, st);
             }
-            if (!qf) { LMX_PROF("prefill.rope_kv"); launch_rope_kv(dt, D, RopeKvArgs{qr, kc, vt, rope, nullptr, pos0 + r0, n, qkv_n, nh_l, nkv_l, kv_pitch}, st); }
+            if (!qf) {
+                RopeKvArgs rk{qr, kc, vt, rope, nullptr, pos0 + r0, n, qkv_n, nh_l, nkv_l, kv_pitch};
+                if (slices) { rk.slabs = s->skw.as<float>(); rk.slices = slices; }
+                LMX_PROF("prefill.rope_kv"); launch_rope_kv(dt, D, rk, st);
+            }
             if (attn_probs) {
                 void* pl = static_cast<char*>(attn_probs) + (size_t)l * nh_l * T * kv_after * es;
                 launch_attn_probs(dt, D, AttnProbsArgs{qr, kc, pl, n, c0 + r0, T, pos0 + r0, kv_after, qkv_n, nh_l, nkv_l, kv_pitch, scale}, st);
@@ -651,14 +668,14 @@ void Model::prefill(Seq* s, const void* embeds, int T, int chunk, void* logits, 
                 fa.part = s->skw.as<float>(); fa.part_bytes = s->skw.bytes;
                 { LMX_PROF("prefill.attn"); launch_flash_prefill(dt, D, fa, st); }
             }
-            { LMX_PROF_K("prefill.gemm.o"); launch_gemm(dt, with_scratch(GemmArgs{ar, w.wo, hr, nullptr, lead ? hr : nullptr, n, H, nh_l * D, nh_l * D, nh_l * D, H, H, kActNone}), gv, st); }
+            return close_block(with_scratch(GemmArgs{ar, w.wo, hr, nullptr, lead ? hr : nullptr, n, H, nh_l * D, nh_l * D, nh_l * D, H, H, kActNone}), next, xr, "prefill.gemm.o");
         };
-        auto mlp_block = [&](int l, int r0, int n) {
+        auto mlp_block = [&](int l, int r0, int n, const void* next = nullptr, bool normed = false) {
             const DecLayerW& w = dec[l];
             void *hr = rows(h, r0, H), *xr = rows(x, r0, H), *cr = rows(act, r0, I_l);
-            { LMX_PROF("prefill.rmsnorm"); launch_rmsnorm(dt, hr, w.ln2, xr, n, H, H, H, cfg.rms_eps, st); }
+            if (!normed) { LMX_PROF("prefill.rmsnorm"); launch_rmsnorm(dt, hr, w.ln2, xr, n, H, H, H, cfg.rms_eps, st); }
             { LMX_PROF_K("prefill.gemm.gate_up"); launch_gemm(dt, with_scratch(GemmArgs{xr, w.wgu, cr, nullptr, nullptr, n, 2 * I_l, H, H, H, I_l, 0, kActSiluMul}), gv, st); }
-            { LMX_PROF_K("prefill.gemm.down"); launch_gemm(dt, with_scratch(GemmArgs{cr, w.wd, hr, nullptr, lead ? hr : nullptr, n, H, I_l, I_l, I_l, H, H, kActNone}), gv, st); }
+            return close_block(with_scratch(GemmArgs{cr, w.wd, hr, nullptr, lead ? hr : nullptr, n, H, I_l, I_l, I_l, H, H, kActNone}), next, xr, "prefill.gemm.down");
         };
         // The two-half pipeline hides 35-55 % of the all-reduce time but costs GEMM efficiency (each half alone cannot fill the chip): measured with a
         // timed stand-in all-reduce (tools/mb_tp_overlap.py, 7B shards) it wins from rows x ranks >= 4096 on — TP=2 at 2048 rows, TP=8 at 1087 —
@@ -695,11 +712,13 @@ void Model::prefill(Seq* s, const void* embeds, int T, int chunk, void* logits, 
             }
             for (int i = 0; i < 2; ++i) LMX_CHECK_HIP(hipStreamWaitEvent(st, s->ev_r[i], 0));
         } else {
+            const bool whole = opt_fuse_slices && !tp_active && !ar_hook && H <= 8192;       // whole: no sum over ranks between a block and the norm behind it
+            bool normed = false;
             for (int l = 0; l < L; ++l) {
                 if (hidden) LMX_CHECK_HIP(hipMemcpyAsync(hidden_rows(l), h, (size_t)tc * H * es, hipMemcpyDeviceToDevice, st));      // the layer's input rows
-                attn_block(l, 0, tc);
+                normed = attn_block(l, 0, tc, whole ? dec[l].ln2 : nullptr, normed);
                 allreduce(h, (size_t)tc * H, st);
-                mlp_block(l, 0, tc);
+                normed = mlp_block(l, 0, tc, whole && l + 1 < L ? dec[l + 1].ln1 : nullptr, normed);
                 { LMX_PROF_AR("prefill.allreduce"); allreduce(h, (size_t)tc * H, st); }
             }
             if (hidden) launch_rmsnorm(dt, h, final_norm, hidden_rows(L), tc, H, H, H, cfg.rms_eps, st);       // the tuple's last entry is normalised

@@ -221,9 +221,10 @@ struct Model {
     void stack_heads(const GroupGemvArgs& g, int n, hipStream_t st);
     // ---- options a caller may flip on a live model (lmx_model_set_option; defaults from the environment at creation) ----------------------------------
     // fuse_rope: RoPE + KV append in the prefill's q|k|v GEMM epilogue (gemm4w.h qkv_rope_epilogue4) instead of a rope_kv launch — bit-identical, faster
+    // fuse_slices: the K slices of a prompt's q|k|v, o and down linears are added by the launch that reads their rows (rope_kv, the norm) — bit-identical, faster
     // vis_pack:  CLIP K / V^T pack in the tower's q|k|v GEMM epilogue instead of a pack launch — bit-identical, launch count
     // splitq:    the decode step's q|k|v projection as q-launch + (k|v projection ∥ attention) launch (decode_attn.hip) — bit-identical
-    bool opt_fuse_rope = true, opt_vis_pack = true, opt_splitq = true;
+    bool opt_fuse_rope = true, opt_fuse_slices = true, opt_vis_pack = true, opt_splitq = true;
     bool opt_stack_fuse = true;         // stack_fuse: a layer-stack decode step's residual addition and norms inside the linear's launch (equal up to rounding)
     // Sequences in existence (lmx_seq_create .. lmx_seq_destroy).  The split-q launch parks one waiting workgroup per head until its own launch's projection has
     // run; launches of DIFFERENT sequences (request threads on their own streams) may be resident together, so the form is only taken while all sequences'

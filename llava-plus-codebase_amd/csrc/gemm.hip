@@ -839,6 +839,21 @@ void launch_gemm(int dtype, const GemmArgs& a, int variant, hipStream_t st) {
     else throw Error{"gemm: bad dtype"};
 }
 
+// The forms are launch_gemm's: a linear is not sliced for its reader's sake.  (It could: o of 5120 at 192 rows 264 -> 260 us a layer, at 256 326 -> 309; o of 4096 does not move, and the
+// sum over K would then depend on who reads it.)
+int launch_gemm_slices(int dtype, const GemmArgs& g, int variant, hipStream_t st) {
+    if (variant == 0 && dtype != kF32 && !g.bias && g.act == kActNone && !g.c_f32 && !g.pk_kc && !g.qf_kc && g.N % 8 == 0 && g.K % GEMM_BK == 0 && g.ldx % 8 == 0 && g.ldw % 8 == 0 && g.ldc % 8 == 0 &&
+        (!g.R || g.ldr % 8 == 0)) {
+        const LinearForm f = linear_form(dtype, g);
+        if (f.kernel == LinearForm::kRows && f.slices > 1) {
+            launch_gemm_rows(dtype, g, f.rows.mtiles, f.rows.bn, f.slices, st, /*keep=*/true);
+            return f.slices;
+        }
+    }
+    launch_gemm(dtype, g, variant, st);
+    return 0;
+}
+
 template <typename T, int MB, int R>
 static void launch_gemv_r(const GemvArgs& a, hipStream_t st) {
     const size_t smem = (size_t)MB * a.K * sizeof(T) + 16;

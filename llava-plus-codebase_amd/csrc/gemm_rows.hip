@@ -282,8 +282,69 @@ __global__ __launch_bounds__(256) void rows_reduce_kernel(GemmArgs a, int S) {
     }
 }
 
+// The same sum with residual rows, and the RMSNorm of the finished row in the same launch: a workgroup owns a row (rmsnorm_reg_kernel's order of its sum, so its bits).  Its time is the
+// launch, one slice's round trip behind the other and the row's sum: 139 rows of 4096 in six slices (13.7 MB from L2) 4.8 + 4.8 us in two launches -> 5.8.  A layer of prompts of 33 .. 384
+// rows, hidden 4096, 2 .. 4 us less of 125 .. 255 for down, and as much for o where that is sliced.
+template <typename T, int NP>
+__global__ __launch_bounds__(256) void rows_reduce_norm_kernel(GemmArgs a, int S, const T* __restrict__ w, T* __restrict__ xn, float eps) {
+    __shared__ float red[4];
+    const int m = blockIdx.x, tid = threadIdx.x, HC = a.N >> 3;
+    const float* slab = static_cast<const float*>(a.skw) + (size_t)m * a.N;
+    const size_t step = (size_t)a.M * a.N;
+    const T* R = static_cast<const T*>(a.R);
+    float v[NP][8], r[NP][8];
+    Chunk8<T> g[NP];
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+        const int c = tid + i * 256;
+        if (c >= HC) continue;
+        load8<float>(slab + c * 8, v[i]);
+        if (R) load8<T>(R + (size_t)m * a.ldr + c * 8, r[i]);
+        g[i].load(w + c * 8);
+    }
+    for (int s = 1; s < S; ++s) {
+        float t[NP][8];
+#pragma unroll
+        for (int i = 0; i < NP; ++i) { const int c = tid + i * 256; if (c < HC) load8<float>(slab + s * step + c * 8, t[i]); }
+#pragma unroll
+        for (int i = 0; i < NP; ++i)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[i][e] += t[i][e];
+    }
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+        const int c = tid + i * 256;
+        if (c >= HC) continue;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) { v[i][e] = round_to<T>(R ? v[i][e] + r[i][e] : v[i][e]); ss += v[i][e] * v[i][e]; }
+        store8<T>(static_cast<T*>(a.C) + (size_t)m * a.ldc + c * 8, v[i]);
+    }
+    ss = block_sum<4>(ss, red);
+    const float inv = rsqrtf(ss / (float)a.N + eps);
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+        const int c = tid + i * 256;
+        if (c >= HC) continue;
+        float o[8]; g[i].get(o);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e] = round_to<T>(v[i][e] * inv) * o[e];
+        store8<T>(xn + (size_t)m * a.N + c * 8, o);
+    }
+}
+void launch_rows_reduce_norm(int dtype, const GemmArgs& a, int S, const void* norm_w, void* xn, float eps, hipStream_t st) {
+    LMX_REQUIRE(dtype != kF32 && a.N <= 8192 && !a.bias && a.act == kActNone && !a.c_f32 && !a.pk_kc, "rows_reduce_norm: a plain 16-bit linear of up to 8192 outputs");
+    const int np = cdiv(a.N / 8, 256);
+#define R(TT, NPV) hipLaunchKernelGGL((rows_reduce_norm_kernel<TT, NPV>), dim3(a.M), dim3(256), 0, st, a, S, (const TT*)norm_w, (TT*)xn, eps)
+#define RT(TT) do { if (np == 1) R(TT, 1); else if (np == 2) R(TT, 2); else if (np == 3) R(TT, 3); else R(TT, 4); } while (0)
+    if (dtype == kBF16) RT(bf16_t); else RT(f16_t);
+#undef RT
+#undef R
+    LMX_CHECK_HIP(hipGetLastError());
+}
+
 template <typename T, int MT, int BN>
-static void launch_rows_cfg(const GemmArgs& a, int mtiles, int S, hipStream_t st) {
+static void launch_rows_cfg(const GemmArgs& a, int mtiles, int S, hipStream_t st, bool keep) {
     constexpr int smem = rows_smem<MT, BN>();
     static_assert(smem <= 160 * 1024, "LDS");
     auto kern = gemm_rows_kernel<T, MT, BN>;
@@ -294,14 +355,14 @@ static void launch_rows_cfg(const GemmArgs& a, int mtiles, int S, hipStream_t st
     }
     const dim3 grid(mtiles * cdiv(a.N, BN) * S);
     KernelTimer* kt = g_kernel_timer;
-    if (S > 1 && kt && !kt->used) {              // an armed kernel timer spans both launches, the boundary between them included
+    if (S > 1 && !keep && kt && !kt->used) {              // an armed kernel timer spans both launches, the boundary between them included
         const dim3 rg((unsigned)cdiv64((int64_t)a.M * (act_gated(a.act) ? a.N / 2 : a.N) / 8, 256));
         kt->used = true;
         hipExtLaunchKernelGGL(kern, grid, dim3(512), smem, st, kt->e0, nullptr, 0, a, mtiles, S);
         hipExtLaunchKernelGGL(rows_reduce_kernel<T>, rg, dim3(256), 0, st, nullptr, kt->e1, 0, a, S);
     } else {
         LMX_LAUNCH(kern, grid, dim3(512), smem, st, a, mtiles, S);
-        if (S > 1) {
+        if (S > 1 && !keep) {
             const dim3 rg((unsigned)cdiv64((int64_t)a.M * (act_gated(a.act) ? a.N / 2 : a.N) / 8, 256));
             hipLaunchKernelGGL(rows_reduce_kernel<T>, rg, dim3(256), 0, st, a, S);
         }
@@ -310,16 +371,16 @@ static void launch_rows_cfg(const GemmArgs& a, int mtiles, int S, hipStream_t st
 }
 
 template <typename T, int BN>
-static void launch_rows_n(const GemmArgs& a, int mtiles, int S, hipStream_t st) {
+static void launch_rows_n(const GemmArgs& a, int mtiles, int S, hipStream_t st, bool keep) {
     switch (cdiv(cdiv(a.M, mtiles), 32)) {
-        case 1: launch_rows_cfg<T, 1, BN>(a, mtiles, S, st); break;
-        case 2: launch_rows_cfg<T, 2, BN>(a, mtiles, S, st); break;
-        case 3: launch_rows_cfg<T, 3, BN>(a, mtiles, S, st); break;
-        case 4: launch_rows_cfg<T, 4, BN>(a, mtiles, S, st); break;
-        case 5: launch_rows_cfg<T, 5, BN>(a, mtiles, S, st); break;
-        case 6: launch_rows_cfg<T, 6, BN>(a, mtiles, S, st); break;
-        case 7: launch_rows_cfg<T, 7, BN>(a, mtiles, S, st); break;
-        default: launch_rows_cfg<T, 8, BN>(a, mtiles, S, st); break;
+        case 1: launch_rows_cfg<T, 1, BN>(a, mtiles, S, st, keep); break;
+        case 2: launch_rows_cfg<T, 2, BN>(a, mtiles, S, st, keep); break;
+        case 3: launch_rows_cfg<T, 3, BN>(a, mtiles, S, st, keep); break;
+        case 4: launch_rows_cfg<T, 4, BN>(a, mtiles, S, st, keep); break;
+        case 5: launch_rows_cfg<T, 5, BN>(a, mtiles, S, st, keep); break;
+        case 6: launch_rows_cfg<T, 6, BN>(a, mtiles, S, st, keep); break;
+        case 7: launch_rows_cfg<T, 7, BN>(a, mtiles, S, st, keep); break;
+        default: launch_rows_cfg<T, 8, BN>(a, mtiles, S, st, keep); break;
     }
 }
 
@@ -393,13 +454,13 @@ RowsForm gemm_rows_form(int dtype, const GemmArgs& a) {
     return RowsForm{mt, 128, 1};
 }
 
-void launch_gemm_rows(int dtype, const GemmArgs& a, int mtiles, int BN, int S, hipStream_t st) {
+void launch_gemm_rows(int dtype, const GemmArgs& a, int mtiles, int BN, int S, hipStream_t st, bool keep) {
     LMX_REQUIRE(gemm_rows_applies(dtype, a) && mtiles >= 1 && cdiv(a.M, mtiles) <= 256 && (BN == 64 || BN == 128), "gemm_rows: shape or alignment");
     LMX_REQUIRE(S >= 1 && S <= a.K / GEMM_BK && (S == 1 || (a.skw && gemm_rows_slab_bytes(a.M, a.N, S) <= a.skw_bytes() && !a.pk_kc)), "gemm_rows: K slices");
     // every M tile covers cdiv(rows per tile, 32) * 32 rows: the tiles that start past M are left out
     mtiles = cdiv(a.M, cdiv(cdiv(a.M, mtiles), 32) * 32);
-    if (dtype == kBF16) { if (BN == 64) launch_rows_n<bf16_t, 64>(a, mtiles, S, st); else launch_rows_n<bf16_t, 128>(a, mtiles, S, st); }
-    else { if (BN == 64) launch_rows_n<f16_t, 64>(a, mtiles, S, st); else launch_rows_n<f16_t, 128>(a, mtiles, S, st); }
+    if (dtype == kBF16) { if (BN == 64) launch_rows_n<bf16_t, 64>(a, mtiles, S, st, keep); else launch_rows_n<bf16_t, 128>(a, mtiles, S, st, keep); }
+    else { if (BN == 64) launch_rows_n<f16_t, 64>(a, mtiles, S, st, keep); else launch_rows_n<f16_t, 128>(a, mtiles, S, st, keep); }
 }
 
 }  // namespace lmx

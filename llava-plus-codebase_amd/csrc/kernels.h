@@ -68,7 +68,8 @@ struct LinearForm {
 };
 LinearForm linear_form(int dtype, const GemmArgs& a);
 size_t gemm_rows_slab_bytes(int M, int N, int S);
-void launch_gemm_rows(int dtype, const GemmArgs& a, int mtiles, int BN, int S, hipStream_t st);
+void launch_gemm_rows(int dtype, const GemmArgs& a, int mtiles, int BN, int S, hipStream_t st, bool keep = false);      // keep: the fp32 slabs [slice][M][N] stay as they are
+void launch_rows_reduce_norm(int dtype, const GemmArgs& a, int S, const void* norm_w, void* xn, float eps, hipStream_t st);
 // decode-batch linear (skinny.hip): M <= 32 rows, 16-bit, weights streamed once straight into MFMA operands; variant 20 of launch_gemm
 void launch_skinny_gemm(int dtype, const GemmArgs& a, hipStream_t st);
 constexpr int SKINNY_SLICED_N = 8192;              // linears this wide and wider fill the CUs without K slices
@@ -404,8 +405,12 @@ struct RopeKvArgs {
     int qkv_stride;
     int n_heads, n_kv_heads, s_max;
     int k_inplace = 0;    // the rotated k ALSO replaces the k columns of QKV (the training step's backward reads k from there: no gathered copy)
+    // the projection in K slices instead of QKV rows: fp32 [slices][T][qkv_stride], added in slice order and rounded; QKV then receives the rotated q alone
+    const float* slabs = nullptr; int slices = 0;
 };
 void launch_rope_kv(int dtype, int D, const RopeKvArgs& a, hipStream_t st);
+// launch_gemm, but the K slices of a plain linear in row tiles may stay as they are for the rows' next launch to add: their number, fp32 [slices][M][N] in g.skw (0: the rows are whole in g.C)
+int launch_gemm_slices(int dtype, const GemmArgs& g, int variant, hipStream_t st);
 
 // token-embedding gather + image-feature splice: out[r] = src[r] >= 0 ? table[src[r]] : src[r] == -1 ? 0 : feats[-2 - src[r]]
 void launch_gather_embed(int dtype, const int* src, const void* table, const void* feats, void* out, int rows, int H, hipStream_t st);

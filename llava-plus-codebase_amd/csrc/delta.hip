@@ -632,7 +632,7 @@ void launch_delta_decode(int dtype, const DeltaDecodeArgs& a, hipStream_t st) {
                         else LMX_LAUNCH((delta_decode_kernel<TT, 32, NTH>), grid, dim3(NTH), smem, st, a); } while (0)
 #define LN(TT) do { if (wide) L(TT, 1024); else L(TT, 512); } while (0)
     // 1024 threads a head while every workgroup has a CU of its own; past that two workgroups of 512 on a CU, whose reads and arithmetic overlap.  us at 16 x 16 / 16 x 24 /
-    // 32 x 32 heads x sequences: 1024 threads 13.8 / 22.5 / 45.4, 512 threads 15.9 / 20.0 / 40.5 (bf16 at 128 registers: 20 bytes a lane in scratch at DK 128, 8 at 256, f16 none)
+    // 32 x 32 heads x sequences: 1024 threads 13.8 / 22.5 / 45.4, 512 threads 15.9 / 20.0 / 40.5 (bf16 at 128 registers: 20 bytes a lane in scratch at DK 256, none at 128; f16 none)
     const bool wide = one_round(a.s, a.n_seq);
     LMX_REQUIRE(wide || !a.router.x, "delta_decode: no router here");
     if (dtype == kBF16) LN(bf16_t); else if (dtype == kF16) LN(f16_t); else LN(float);

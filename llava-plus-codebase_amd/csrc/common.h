@@ -213,17 +213,13 @@ enum Act : int { kActNone = 0, kActQuickGelu = 1, kActGeluErf = 2, kActSiluMul =
 // gated forms: the weight's rows come in [32 gate | 32 up] groups and the output is f(gate) * up
 __host__ __device__ __forceinline__ bool act_gated(int act) { return act == kActSiluMul || act == kActReluMul; }
 
-// x / (1 + e^-cx).  Outputs of 16 bits take the reciprocal instruction (one unit in the last place of 32 bits; a division is ten more instructions: quick GELU of
-// 2308 x 4096 x 1024 34.2 -> 31.8 us, gate | up of 1087 x 22016 x 4096 151.1 -> 148.6; the error against 64 bits is that of the 16-bit result, 1.662440e-3 and 2.0765e-4, either way).
-// A quarter of numerator and denominator: the reciprocal of 2^126 and more is a subnormal number, which the instruction makes zero (x from -87.4 down, whose results bf16 holds).
-template <typename T = bf16_t> __device__ __forceinline__ float over_one_plus_exp(float x, float cx) {
-    if constexpr (sizeof(T) == 4) return x / (1.f + __expf(-cx));
-    else return 0.25f * x * __builtin_amdgcn_rcpf(fmaf(0.25f, __expf(-cx), 0.25f));
-}
-template <typename T = bf16_t> __device__ __forceinline__ float act_quick_gelu(float x) { return over_one_plus_exp<T>(x, 1.702f * x); }
+// x / (1 + e^-cx) by the exact division in every type.  The reciprocal instruction (one unit in the last place of 32 bits) saves ten instructions an output: quick GELU of
+// 2308 x 4096 x 1024 34.2 -> 31.8 us, gate | up of 1087 x 22016 x 4096 151.1 -> 148.6, but more 16-bit results are rounded the other way than 64 bits have them: 1.262 -> 1.500 % (quick GELU) and
+// 0.144 -> 0.170 % (SiLU) over wide arguments.
+__device__ __forceinline__ float act_quick_gelu(float x) { return x / (1.f + __expf(-1.702f * x)); }
 __device__ __forceinline__ float act_gelu_erf(float x) { return 0.5f * x * (1.f + erff(x * 0.70710678118654752f)); }
-template <typename T = bf16_t> __device__ __forceinline__ float act_silu(float x) { return over_one_plus_exp<T>(x, x); }
-template <typename T = bf16_t> __device__ __forceinline__ float gate_mul(int act, float g, float u) { return (act == kActReluMul ? fmaxf(g, 0.f) : act_silu<T>(g)) * u; }
+__device__ __forceinline__ float act_silu(float x) { return x / (1.f + __expf(-x)); }
+__device__ __forceinline__ float gate_mul(int act, float g, float u) { return (act == kActReluMul ? fmaxf(g, 0.f) : act_silu(g)) * u; }
 
 // logits <- cap tanh(logits / cap); cap <= 0: unchanged
 __device__ __forceinline__ float soft_cap(float v, float cap) { return cap > 0.f ? cap * tanhf(v / cap) : v; }

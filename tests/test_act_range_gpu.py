@@ -30,3 +30,27 @@ def test_the_whole_range(cuda, dt, act, M):
     tol = ref.abs() * ((2.0 ** -8 if dt == torch.bfloat16 else 2.0 ** -24) + (cx.abs() + 4) * 2.0 ** -23)
     tol = torch.where(cx < -88.7, torch.full_like(tol, 2.0 ** -120), tol)
     assert torch.isfinite(got).all() and ((got - ref).abs() <= tol).all(), ((got - ref).abs() / tol.clamp_min(1e-300)).max()
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("act", [1, 3])
+@pytest.mark.parametrize("M", [1, 12, 139, 300, 1200])
+def test_sixteen_bits_are_the_rounded_thirty_two(cuda, dt, act, M):
+    """The epilogue is computed in 32 bits whatever the output: a 16-bit result is the fp32 model's for the same argument, rounded once.  The arguments are sums of two operands, exact in 32
+    bits, 1024 a row."""
+    from llava_mi355x import ops
+    g = torch.Generator(device="cuda").manual_seed(act + M)
+    outs = {}
+    z = (4 * torch.randn(M, 1, generator=g, device="cuda")).clamp(-15, 15).mul(16).round().div(16).to(dt)          # eight bits, and six more behind them: their sum has no more than 15
+    lo = (torch.randint(-63, 64, (1024,), generator=g, device="cuda") / 2048).to(dt)
+    for t in (dt, torch.float32):
+        x = torch.zeros(M, 1024, device=cuda, dtype=t)
+        x[:, :1], x[:, 1] = z.to(t), 1.0
+        w = torch.zeros(1024 * (2 if act == 3 else 1), 1024, device=cuda, dtype=t)
+        gate = w if act == 1 else w.view(32, 2, 32, 1024)[:, 0].reshape(1024, 1024).clone()
+        gate[:, 0], gate[:, 1] = 1.0, lo.to(t)
+        if act == 3:
+            w.view(32, 2, 32, 1024)[:, 0] = gate.view(32, 32, 1024)
+            w.view(32, 2, 32, 1024)[:, 1, :, 1] = 1.0
+        outs[t] = ops.gemm(x, w, act=act, out=torch.empty(M, 1024, device=cuda, dtype=t))
+    assert torch.equal(outs[dt], outs[torch.float32].to(dt)), int((outs[dt] != outs[torch.float32].to(dt)).sum())

@@ -976,8 +976,9 @@ def _vizosun_model(size, dev, dtype, max_position):
     return _random_weights(VizosunForCausalLM(c, dtype=dtype, device=dev, max_position=max_position), shapes, dev, dtype)
 
 
-def _vizosun_floors(size, T, ctx, n_batch, dec_steps, batch_steps):
-    """Roofline time of everything a kernel group does in the profiled passes (one prefill of T rows, dec_steps single and batch_steps batched steps)."""
+def _vizosun_floors(size, T, ctx, n_batch, dec_steps, batch_steps, timed=()):
+    """Roofline time of everything a kernel group does in the profiled passes (one prefill of T rows, dec_steps single and batch_steps batched steps).  timed: the groups of the
+    profile; a launch that two linears share is a group of its own and has the floors of both."""
     W, H, D, Q, R, F, (E, top, EF), L, V, win = size
     A, hd = VIZOSUN_RANK, H * D
     hbm = lambda by: by / (PEAK_HBM_GBS * 1e9)
@@ -990,6 +991,7 @@ def _vizosun_floors(size, T, ctx, n_batch, dec_steps, batch_steps):
     add("prefill.embed", hbm(8.0 * T * W))
     for i in range(L):
         lat, mix = i % 4 == 3, i % 2 == 1
+        share_gu, share_o = not lat and not mix and "decode.delta_gate_up" in timed, mix and "decode.moe.gate_up_o" in timed
         n_in = Q + R if lat else 3 * hd + H + 2 * A
         add("prefill.gemm.qkv", lin(T, n_in, W))
         add("decode.gemv.qkv", hbm(2.0 * n_in * W) * dec_steps)
@@ -1008,19 +1010,19 @@ def _vizosun_floors(size, T, ctx, n_batch, dec_steps, batch_steps):
             add("prefill.delta.scan", max(hbm(T * hd * (12.0 + 2 + 4)), 7.0 * T * hd * D / (PEAK_FP32_TFLOPS * 1e12)))
             add("prefill.delta.gate", hbm(T * hd * 8.0))
             for pre, n, steps in (("decode", 1, dec_steps), ("decode_batch", n_batch, batch_steps)):
-                add(pre + ".delta", hbm(8.0 * hd * D * n + 4.0 * hd * A) * steps)
+                add("decode.delta_gate_up" if share_gu and pre == "decode" else pre + ".delta", hbm(8.0 * hd * D * n + 4.0 * hd * A) * steps)
         add("prefill.gemm.o", lin(T, W, hd + (0 if mix else F)))
-        add("decode.gemv.o", hbm(2.0 * W * (hd + (0 if mix else F))) * dec_steps)
+        add("decode.moe.gate_up_o" if share_o else "decode.gemv.o", hbm(2.0 * W * (hd + (0 if mix else F))) * dec_steps)
         add("prefill.residual_norm", hbm(12.0 * T * W + (2.0 * top * T * W if mix else 0)))
         if mix:
             add("prefill.moe.router", hbm(2.0 * T * W)); add("prefill.moe.gate_up", lin(T * top, 2 * EF, W, 2 * EF * E)); add("prefill.moe.down", lin(T * top, W, EF, W * E))
             for pre, n, steps in (("decode", 1, dec_steps), ("decode_batch", n_batch, batch_steps)):
                 hit = E * (1 - (1 - top / E) ** n)      # experts that n rows choose at random
                 add(pre + ".moe.router", hbm(2.0 * E * W) * steps)
-                add(pre + ".moe.gate_up", hbm(4.0 * EF * W * hit) * steps); add(pre + ".moe.down", hbm(2.0 * EF * W * hit) * steps)
+                add("decode.moe.gate_up_o" if share_o and pre == "decode" else pre + ".moe.gate_up", hbm(4.0 * EF * W * hit) * steps); add(pre + ".moe.down", hbm(2.0 * EF * W * hit) * steps)
         else:
             add("prefill.gemm.gate_up", lin(T, 2 * F, W))
-            add("decode.gemv.gate_up", hbm(4.0 * W * F) * dec_steps)
+            add("decode.delta_gate_up" if share_gu else "decode.gemv.gate_up", hbm(4.0 * W * F) * dec_steps)
     add("prefill.residual_norm", hbm(6.0 * T * W))
     add("decode.gemv.lm_head", hbm(2.0 * V * W) * dec_steps)
     return f
@@ -1038,7 +1040,7 @@ def run_vizosun(a, dev):
             model = _vizosun_model(size, dev, dtype, 4096) if kind == "vizosun" else _siterax_model(sx, dev, dtype, 4096)
             fig, prof, bprof = _time_decoder(model, T, ctx, new, a.steps, a.warmup)
             if kind == "vizosun":
-                floors = _vizosun_floors(size, T, ctx, 32, 8, 4)
+                floors = _vizosun_floors(size, T, ctx, 32, 8, 4, {**prof, **bprof})
                 fig["kernels"] = {k: {"us": round(ms * 1e3 / max(1, n), 2), "launches": n, "total_us": round(ms * 1e3, 1), **({"roofline_frac": round(floors[k] * 1e3 / ms, 3)} if k in floors and ms > 0 else {})}
                                   for k, (ms, n) in sorted({**prof, **bprof}.items())}
             else:

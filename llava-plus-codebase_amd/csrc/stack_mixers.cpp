@@ -139,7 +139,7 @@ bool Model::stack_mix_decode(int r, const DecodeFusedSeq* tab, const DecodeFused
         a.wag = l.wag; a.wag_ld = l.ra + l.rg; a.out = mix; a.out_ld = l.out_k;
         a.tab = tab; a.one = one; a.n_seq = n; a.eps = S.c.norm_eps;
         if (delta_decode_routes(l.ds, n)) a.router = router;
-        LMX_PROF_K(pn.delta);
+        LMX_PROF_K(beside ? "decode.delta_gate_up" : pn.delta);
         if (beside) launch_delta_decode_linear(dt, a, *beside, st); else launch_delta_decode(dt, a, st);
         return a.router.x;
     }
@@ -203,7 +203,7 @@ void Model::stack_moe(const StackLayer& l, const void* x, int rows, const StackW
     }
     GroupGemvArgs g{x, l.wgu, w.act, 2 * l.ff, H, H, H, l.ff, (size_t)2 * l.ff * H};
     g.act = l.act(); g.ids = w.ids; g.per_row = top;
-    { LMX_PROF_K(pn.gate_up); if (beside) launch_group_gemv_linear(dt, g, slots, *beside, st); else launch_group_gemv(dt, g, slots, st); }
+    { LMX_PROF_K(beside ? "decode.moe.gate_up_o" : pn.gate_up); if (beside) launch_group_gemv_linear(dt, g, slots, *beside, st); else launch_group_gemv(dt, g, slots, st); }
     GroupGemvArgs o{w.act, l.wd, w.slots, H, l.ff, l.ff, l.ff, H, (size_t)H * l.ff};
     o.ids = w.ids;
     { LMX_PROF_K(pn.down); launch_group_gemv(dt, o, slots, st); }

@@ -52,3 +52,21 @@ def test_oracle_is_only_imported_by_the_cpu_baseline_leg():
             if f.endswith((".py", ".cpp", ".hip", ".h")):
                 text = open(os.path.join(d, f), errors="replace").read()
                 assert "import oracle" not in text and "from oracle" not in text and "/root/reference" not in text, os.path.join(d, f)
+
+
+def test_a_shared_launch_has_the_floors_of_both_linears():
+    """Two linears in one launch are one group of the profile: their floors move there together, nothing is counted twice or under a name whose launches no longer hold it."""
+    import bench
+    for size in bench.VIZOSUN_SIZES.values():
+        W, H, D, Q, R, F, (E, top, EF), L, V, win = size
+        apart = bench._vizosun_floors(size, 2048, 2048, 32, 8, 4)
+        both = bench._vizosun_floors(size, 2048, 2048, 32, 8, 4, ("decode.delta_gate_up", "decode.moe.gate_up_o"))
+        assert not {"decode.gemv.gate_up", "decode.moe.gate_up"} & set(both) and not {"decode.delta_gate_up", "decode.moe.gate_up_o"} & set(apart)
+        assert abs(sum(apart.values()) - sum(both.values())) < 1e-9 * sum(apart.values())
+        us = lambda by: 8 * by / (bench.PEAK_HBM_GBS * 1e9)
+        dense = sum(i % 2 == 0 for i in range(L))
+        # what the remaining o launches read: the dense layers' [heads | feed-forward] columns
+        assert abs(both["decode.gemv.o"] - dense * us(2.0 * W * (H * D + F))) < 1e-12
+        assert abs(both["decode.delta_gate_up"] - dense * us(8.0 * H * D * D + 4.0 * H * D * bench.VIZOSUN_RANK + 4.0 * W * F)) < 1e-12
+        assert abs(both["decode.delta"] - sum(i % 4 == 1 for i in range(L)) * us(8.0 * H * D * D + 4.0 * H * D * bench.VIZOSUN_RANK)) < 1e-12
+        assert abs(both["decode.moe.gate_up_o"] - (L - dense) * us(4.0 * EF * W * E * (1 - (1 - top / E)) + 2.0 * W * H * D)) < 1e-12

@@ -43,6 +43,23 @@ def test_products_beside_each_other(cuda, dt, dim, ff):
     assert torch.isfinite(a.float()).all() and rel(a, b.double().cpu()) < TOL[dt] / 8
 
 
+def test_a_shared_launch_is_a_group_of_its_own(cuda):
+    """Launches by profile group, of 6 steps: what runs in a shared launch is under neither linear's own name."""
+    cfg = config([delta(4, 2, 128, 40, 3, dense(88)), delta(3, 3, 64, 48, 4, moe(72, 6, 2)), latent(3, 40, 20, 50, 36, 24, moe(40, 5, 3)), delta(4, 4, 128, 128, 4, dense(88))], 136, 211)
+    m = build_config(cfg, steady_routing(cfg, O.make_weights(cfg, 3, (18, 70))), torch.bfloat16, 64)
+    names = ("decode.delta", "decode.delta_gate_up", "decode.gemv.gate_up", "decode.moe.gate_up", "decode.moe.gate_up_o", "decode.gemv.o")
+
+    def launches():
+        m.profile(True)
+        _steps(m, [5, 9, 2, 7, 1], 6)
+        prof = m.profile_read()
+        m.profile(False)
+        return [prof[k][1] if k in prof else 0 for k in names]
+    assert launches() == [6, 12, 0, 0, 12, 12]
+    m.set_option("stack_fuse", 0)
+    assert launches() == [18, 0, 12, 12, 0, 24]
+
+
 @pytest.mark.parametrize("dt", list(DT))
 @pytest.mark.parametrize("N,H,act", [(8, 2048, 0), (2552, 2048, 0), (2560, 2048, 0), (2560, 3072, 0), (2552, 3072, 0), (2568, 3136, 0), (4088, 4096, 0), (4096, 4096, 0), (6136, 3136, 0),
                                      (6144, 3136, 0), (6152, 4096, 0), (2496, 2048, 3), (2560, 2048, 3), (2560, 3136, 3), (6144, 4096, 3), (2560, 4160, 0)])

@@ -728,6 +728,18 @@ int lmx_op_decode_win_form(int32_t dtype, int32_t D, int32_t n_heads, int32_t n_
     LMX_API_END
 }
 
+static GemvArgs plain_row(int32_t N, int32_t K) { return GemvArgs{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0.f, N, K, K, K, N, 0, kActNone}; }
+int lmx_op_delta_joins(int32_t dtype, int32_t heads, int32_t head_dim, int32_t N, int32_t K, int32_t* joins) {
+    LMX_API_BEGIN
+    LMX_REQUIRE(joins && heads >= 1 && (head_dim == 64 || head_dim == 128 || head_dim == 256) && N >= 1 && K >= 64, "delta_joins: bad arguments");
+    DeltaShape s{};
+    s.H = heads; s.DK = head_dim;
+    GemvArgs g = plain_row(N, K);
+    g.act = kActSiluMul;
+    *joins = delta_decode_joins(dtype, s, g);
+    LMX_API_END
+}
+
 size_t lmx_op_group_plan_bytes(int32_t rows, int32_t per_row) { return rows > 0 && per_row > 0 ? group_plan_bytes(rows * per_row) : 0; }
 int lmx_op_group_gemm(int32_t dtype, const void* x, const void* w, void* c, const int32_t* ids, int32_t rows, int32_t per_row, int32_t groups, int32_t shared_x, int32_t N, int32_t K,
                       int32_t act, int32_t bm, int32_t nb, void* plan, void* stream) {

@@ -609,6 +609,7 @@ __global__ __launch_bounds__(1024) void delta_decode_linear_kernel(DeltaDecodeAr
     else gemv2_body<T, R, 4, 1, false, false, 16>(g, (int)blockIdx.x - a.s.H, reinterpret_cast<char*>(sm), nullptr, 0u);
 }
 
+static bool joined_one_round(int heads, int rows) { return cdiv(rows, 64) + heads <= 256; }      // four rows a wave of the linear beside the step
 static bool one_round(const DeltaShape& s, int n_seq) { return s.H * n_seq <= 256; }
 // past one round the routers are a tail of their own: 32 x 32 heads x sequences 39.1 us without, 50.4 with them, 9.8 alone; in one round (16 x 1) 9.9 either way, 8.1 alone.  On the line,
 // where the routers' own workgroups are the ones past the round, they still cost less than their launches: a decode step with two of them, 16 x 16 728 us in the step's launch, 734 in
@@ -641,13 +642,28 @@ void launch_delta_decode(int dtype, const DeltaDecodeArgs& a, hipStream_t st) {
     LMX_CHECK_HIP(hipGetLastError());
 }
 
-bool delta_decode_joins(int dtype, const DeltaShape& s, const GemvArgs& g) { return s.H <= 64 && g.K <= 8192 && gemv2_applies(dtype, g); }
+// Where the shared launch takes less than the two (us a layer of one token, two launches -> one; heads of 128):
+//   one round of workgroups (four rows a wave)   N x K  8192 x 2048 31.3 -> 26.8   11264 x 4096 64.0 -> 58.6   11264 x 8192 154.3 -> 150.7,
+//     but few workgroups with long rows are the longer of the two:   1024 x 4096 44.4 : 45.8   5632 x 5120 67.8 : 68.1   1024 x 8192 118.2 : 126.1   (5632 x 4096 53.3 : 51.3, 1024 x 3072 32.7 : 32.4)
+//   several rounds (two rows a wave)   16384 x 2048 39.0 -> 36.0   22016 x 3072 63.2 -> 58.3   18432 x 4608 91.0 -> 87.4   22016 x 6144 134.9 -> 132.0   18432 x 7168 148.6 -> 148.1,
+//     but the launch of its own streams faster, by more than the step the more there is:   32768 x 6144 165.4 : 166.0   22016 x 7168 161.8 : 164.6, and with rows a multiple of 8 KiB apart at
+//     once:   16384 x 4096 73.7 : 74.8   32768 x 4096 108.3 : 112.4   22016 x 8192 197.9 : 204.3
+//   heads of 256, whose step is twice as long   11264 x 2048 43.5 -> 35.5   22016 x 4096 95.1 -> 87.7   1024 x 4096 55.8 -> 51.6;   32768 x 8192 250 : 254
+// More than 64 heads: 96 of 64 beside 22016 x 4096 93.4 either way.
+bool delta_decode_joins(int dtype, const DeltaShape& s, const GemvArgs& g) {
+    if (s.H > 64 || g.K > 8192 || !gemv2_applies(dtype, g)) return false;
+    const bool bounded = (size_t)g.N * g.K <= ((size_t)1 << 27);
+    if (s.DK == 256 && g.K <= 4096) return bounded;
+    if (joined_one_round(s.H, g.N)) return g.K <= 3072 || g.N >= 6144;
+    return bounded && g.K % 4096 != 0;
+}
 void launch_delta_decode_linear(int dtype, const DeltaDecodeArgs& a, const GemvArgs& g, hipStream_t st) {
     delta_decode_check(a);
     LMX_REQUIRE(a.n_seq == 1 && !a.tab && !a.router.x && delta_decode_joins(dtype, a.s, g) && !g.norm_w, "delta_decode_linear: one sequence, a plain linear of the weight stream");
     LMX_REQUIRE(!act_gated(g.act) || g.N % 64 == 0, "delta_decode_linear: gated rows come in groups of 64");
-    // four rows a wave where that leaves every workgroup a CU of its own (all of a row of 2048 is on the wire at once), two where the workgroups come in rounds
-    const bool four = cdiv(g.N, 64) + a.s.H <= 256;
+    // four rows a wave where that leaves every workgroup a CU of its own (all of a row of 2048 is on the wire at once), two where the workgroups come in rounds: a layer of one token at four
+    // rows / two  11264 x 2048 29.5 / 29.9 us   16384 x 3072 51.4 / 51.9   22016 x 4096 82.7 / 83.1, but  32768 x 6144 165.4 / 163.3
+    const bool four = joined_one_round(a.s.H, g.N);
     const size_t smem = std::max(delta_decode_smem(a.s), gemv2_smem_bytes(g.K, 2, 16));
     const dim3 grid(a.s.H + cdiv(g.N, four ? 64 : 32));
 #define L(TT, LPC) do { if (four) LMX_LAUNCH((delta_decode_linear_kernel<TT, LPC, 4>), grid, dim3(1024), smem, st, a, g); \

@@ -386,6 +386,8 @@ int lmx_op_decode_win(int32_t dtype, int32_t D, const void* qkv, int32_t qkv_str
 int lmx_op_decode_win_form(int32_t dtype, int32_t D, int32_t n_heads, int32_t n_kv_heads, int32_t n_seq, int32_t span, int32_t* form);
 /* a parallel layer's gate | up of N rows over width K beside its delta step of `heads` heads of 64, 128 or 256 (head_dim) in one launch, one sequence: joins = 1 where a decode step does so */
 int lmx_op_delta_joins(int32_t dtype, int32_t heads, int32_t head_dim, int32_t N, int32_t K, int32_t* joins);
+/* its output projection of out_k columns over width K beside its `slots` experts' first product of 2 ff rows, one sequence: as above */
+int lmx_op_moe_joins(int32_t dtype, int32_t slots, int32_t ff, int32_t K, int32_t out_k, int32_t* joins);
 /* act(x_row W_g^T) of every slot (row, choice): g = ids[slot], in [0, groups), picks one of the groups' weights w [groups][N][K]; x row = slot / per_row (shared_x) or slot, c row = slot.
  * bm: rows of a tile, 0 = as the engine chooses; 32, 64 or, 16-bit four-wave tiles, 128 .. 256 in steps of 32, those with nb blocks of 32 columns (0 = as the engine chooses).
  * plan: lmx_op_group_plan_bytes(rows, per_row) bytes of scratch. */

@@ -740,6 +740,15 @@ int lmx_op_delta_joins(int32_t dtype, int32_t heads, int32_t head_dim, int32_t N
     LMX_API_END
 }
 
+int lmx_op_moe_joins(int32_t dtype, int32_t slots, int32_t ff, int32_t K, int32_t out_k, int32_t* joins) {
+    LMX_API_BEGIN
+    LMX_REQUIRE(joins && slots >= 1 && ff >= 32 && ff % 32 == 0 && K >= 64 && out_k >= 64, "moe_joins: bad arguments");
+    GroupGemvArgs a{nullptr, nullptr, nullptr, 2 * ff, K, K, K, ff, (size_t)2 * ff * K};
+    a.act = kActSiluMul; a.per_row = slots;
+    *joins = group_gemv_joins(dtype, a, slots, plain_row(K, out_k));
+    LMX_API_END
+}
+
 size_t lmx_op_group_plan_bytes(int32_t rows, int32_t per_row) { return rows > 0 && per_row > 0 ? group_plan_bytes(rows * per_row) : 0; }
 int lmx_op_group_gemm(int32_t dtype, const void* x, const void* w, void* c, const int32_t* ids, int32_t rows, int32_t per_row, int32_t groups, int32_t shared_x, int32_t N, int32_t K,
                       int32_t act, int32_t bm, int32_t nb, void* plan, void* stream) {

@@ -217,6 +217,7 @@ struct Model {
     // the same over one new token of every sequence (tab: batch; else `one`), projection rows already there
     bool stack_mix_decode(int r, const DecodeFusedSeq* tab, const DecodeFusedSeq& one, int n, int max_len, const void* x, void* qkv, void* mix, const StackWs& w, Batch* b, hipStream_t st, const GemvArgs* beside = nullptr);
     void stack_moe(const StackLayer& l, const void* x, int rows, const StackWs& w, const StackProf& pn, hipStream_t st, bool routed = false, const GemvArgs* beside = nullptr);      // routed: the mixer's launch chose the experts; beside: a linear in the launch of the first product (few rows)
+    GroupGemvArgs stack_moe_first(const StackLayer& l, const void* x, const StackWs& w) const;      // the experts' first product, rows as they are
     MoeRouterArgs stack_router(const StackLayer& l, const void* x, const StackWs& w) const;
     void stack_heads(const GroupGemvArgs& g, int n, hipStream_t st);
     // ---- options a caller may flip on a live model (lmx_model_set_option; defaults from the environment at creation) ----------------------------------

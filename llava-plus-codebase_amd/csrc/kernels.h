@@ -324,7 +324,7 @@ struct GroupGemvArgs {                   // slot = blockIdx.y.  ids: group = ids
 };
 void launch_group_gemv(int dtype, const GroupGemvArgs& a, int slots, hipStream_t st);
 // a gated grouped product and an independent small linear in one launch (16-bit)
-bool group_gemv_joins(int dtype, const GemvArgs& g);
+bool group_gemv_joins(int dtype, const GroupGemvArgs& a, int slots, const GemvArgs& g);
 void launch_group_gemv_linear(int dtype, const GroupGemvArgs& a, int slots, const GemvArgs& g, hipStream_t st);
 // many rows per group: MFMA tiles.  With a plan (mixtures) tile rows are slots: x row slot / per_row, c row slot; without one every group takes rows [0, rows)
 constexpr int GROUP_MIN_BM = 32;

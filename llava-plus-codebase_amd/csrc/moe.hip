@@ -330,10 +330,19 @@ void launch_group_gemv(int dtype, const GroupGemvArgs& a, int slots, hipStream_t
     LMX_CHECK_HIP(hipGetLastError());
 }
 
-bool group_gemv_joins(int dtype, const GemvArgs& g) { return g.K <= 4096 && g.K % 8 == 0 && (size_t)g.N * g.K <= ((size_t)1 << 25) && !g.norm_w && gemv2_applies(dtype, g); }
+// Where the shared launch takes less than the two (us a layer of one token, two launches -> one):  rows of up to 3072  4 slots of 2 x 1408 x 2048 42.7 -> 39.8, 2 x 4096 x 2048 72.6 -> 68.7,
+// 2 x 4096 x 3072 96.6 -> 94.0, 8 slots 149.2 -> 146.3.  Longer rows while a workgroup has few of them and there are more than four workgroups a CU (the linear's go first, and what follows
+// in one even round ends as late as they began): 4 slots of 2 x 2752 x 4096 106.4 -> 104.4, 2 x 3328 x 4096 115.0 -> 111.6, 8 of 2 x 1408 103.5 -> 102.2, 2 of 2 x 5632 106.9 -> 104.6, but
+// 4 of 2 x 4096 128.1 : 131.9, 2 x 8192 197.9 : 208.5, 2 of 2 x 4096 92.7 : 94.5, 8 of 2 x 2048 133.2 : 134.2; rows of 6144 .. 8192 99 .. 283 us, 0.9 % less to 5.6 % more.
+bool group_gemv_joins(int dtype, const GroupGemvArgs& a, int slots, const GemvArgs& g) {
+    if (g.K > 4096 || g.K % 8 != 0 || (size_t)g.N * g.K > ((size_t)1 << 25) || g.norm_w || !gemv2_applies(dtype, g)) return false;
+    if (a.K <= 3072) return true;
+    const GroupGemvForm f = group_gemv_form(a, slots);
+    return a.K <= 4096 && (f.opw <= 4 || (f.opw <= 8 && slots * f.parts > 1024));
+}
 void launch_group_gemv_linear(int dtype, const GroupGemvArgs& a, int slots, const GemvArgs& g, hipStream_t st) {
     group_gemv_check(dtype, a);
-    LMX_REQUIRE(slots >= 1 && act_gated(a.act) && !act_gated(g.act) && group_gemv_joins(dtype, g), "group_gemv_linear: a gated grouped product and a small plain linear");
+    LMX_REQUIRE(slots >= 1 && act_gated(a.act) && !act_gated(g.act) && group_gemv_joins(dtype, a, slots, g), "group_gemv_linear: a gated grouped product and a small plain linear");
     const GroupGemvForm f = group_gemv_form(a, slots);
     const int linear_wgs = cdiv(g.N, 4);
     const dim3 grid(linear_wgs + slots * f.parts);

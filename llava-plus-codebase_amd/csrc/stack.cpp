@@ -650,7 +650,7 @@ void Model::stack_decode_step(Seq* s, hipStream_t st, int64_t* id_out) {
         const GemvArgs gu{s->d_x, l.wgu, static_cast<char*>(s->d_attn) + (size_t)l.an * es, nullptr, nullptr, nullptr, 0.f, 2 * l.ff, H, H, H, l.ff, 0, l.act()};
         const GemvArgs go{s->d_attn, l.wo, s->d_y, nullptr, nullptr, nullptr, 0.f, H, l.out_k, l.out_k, l.out_k, H, 0, kActNone};
         const bool par = l.parallel() && opt_stack_fuse, join_gu = par && l.dense() && l.c.mixer == LMX_MIXER_DELTA && delta_decode_joins(dt, l.ds, gu);
-        const bool join_o = par && l.moe() && act_gated(l.act()) && !group_gemm_applies(dt, l.c.top_experts, l.c.experts) && group_gemv_joins(dt, go);
+        const bool join_o = par && l.moe() && act_gated(l.act()) && !group_gemm_applies(dt, l.c.top_experts, l.c.experts) && group_gemv_joins(dt, stack_moe_first(l, s->d_x, s->sw), l.c.top_experts, go);
         if (l.c.mixer == LMX_MIXER_ATTENTION) {
             LMX_PROF_K("decode.attn");
             WinForm f;

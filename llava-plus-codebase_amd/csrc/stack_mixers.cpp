@@ -188,6 +188,11 @@ void Model::stack_heads(const GroupGemvArgs& g, int n, hipStream_t st) {
 // mixture of experts: choices, then both products with the rows as they are (few: weights streamed per row) or sorted by expert (MFMA tiles)
 // ---------------------------------------------------------------------------------------------------------------
 MoeRouterArgs Model::stack_router(const StackLayer& l, const void* x, const StackWs& w) const { return MoeRouterArgs{x, l.wr, l.br, H, H, l.c.experts, l.c.top_experts, w.ids, w.wt}; }
+GroupGemvArgs Model::stack_moe_first(const StackLayer& l, const void* x, const StackWs& w) const {
+    GroupGemvArgs g{x, l.wgu, w.act, 2 * l.ff, H, H, H, l.ff, (size_t)2 * l.ff * H};
+    g.act = l.act(); g.ids = w.ids; g.per_row = l.c.top_experts;
+    return g;
+}
 void Model::stack_moe(const StackLayer& l, const void* x, int rows, const StackWs& w, const StackProf& pn, hipStream_t st, bool routed, const GemvArgs* beside) {
     const int dt = cfg.dtype, top = l.c.top_experts, E = l.c.experts, slots = rows * top;
     if (!routed) { LMX_PROF_K(pn.router); launch_moe_router(dt, stack_router(l, x, w), rows, st); }
@@ -201,8 +206,7 @@ void Model::stack_moe(const StackLayer& l, const void* x, int rows, const StackW
         { LMX_PROF_K(pn.down); launch_group_gemm(dt, p[1], bm, st); }
         return;
     }
-    GroupGemvArgs g{x, l.wgu, w.act, 2 * l.ff, H, H, H, l.ff, (size_t)2 * l.ff * H};
-    g.act = l.act(); g.ids = w.ids; g.per_row = top;
+    const GroupGemvArgs g = stack_moe_first(l, x, w);
     { LMX_PROF_K(beside ? "decode.moe.gate_up_o" : pn.gate_up); if (beside) launch_group_gemv_linear(dt, g, slots, *beside, st); else launch_group_gemv(dt, g, slots, st); }
     GroupGemvArgs o{w.act, l.wd, w.slots, H, l.ff, l.ff, l.ff, H, (size_t)H * l.ff};
     o.ids = w.ids;

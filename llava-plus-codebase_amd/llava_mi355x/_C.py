@@ -158,6 +158,7 @@ _SIGS = {
     "lmx_op_group_plan_bytes": (c_size_t, [c_int32] * 2),
     "lmx_op_group_gemm": (c_int32, [c_int32] + [c_void_p] * 4 + [c_int32] * 9 + [c_void_p] * 2),
     "lmx_op_delta_joins": (c_int32, [c_int32] * 5 + [POINTER(c_int32)]),
+    "lmx_op_moe_joins": (c_int32, [c_int32] * 5 + [POINTER(c_int32)]),
     "lmx_op_decode_win_form": (c_int32, [c_int32] * 6 + [POINTER(c_int32)]),
     "lmx_op_argmax": (c_int32, [c_int32, c_void_p, c_int32, c_void_p, c_void_p]),
     "lmx_op_ce_loss": (c_int32, [c_int32, c_void_p, c_int32, c_void_p, c_int32, c_int32, c_int32, c_int64, c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_int32, c_void_p]),

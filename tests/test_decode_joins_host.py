@@ -1,5 +1,5 @@
 """Which linears of one token share a launch with the work beside them, asked of the library on the host.  Every case was timed both ways: the shared launch is taken where it is the shorter
-one (csrc/delta.hip: delta_decode_joins)."""
+one (csrc/delta.hip: delta_decode_joins, csrc/moe.hip: group_gemv_joins)."""
 import ctypes
 
 import pytest
@@ -30,3 +30,26 @@ def test_gate_up_beside_the_delta_step(case):
 @pytest.mark.parametrize("dim", [64, 128, 256])
 def test_never_what_the_launch_cannot_take(dim):
     assert not _delta(16, dim, 1024, 1024, torch.float32) and not _delta(16, dim, 8192, 8256) and not _delta(16, dim, 1024, 1028)
+
+
+def _moe(slots, ff, K, out_k, dt=torch.bfloat16):
+    from llava_mi355x import _C
+    f = ctypes.c_int32()
+    _C.check(_C.lib.lmx_op_moe_joins(_C.torch_dtype_code(dt), slots, ff, K, out_k, f))
+    return bool(f.value)
+
+
+# experts of a row, their width, the layer's width, the output projection's columns
+BESIDE = [(4, 704, 1024, 1024), (4, 1408, 2048, 2048), (4, 4096, 2048, 2048), (8, 4096, 2048, 2048), (4, 4096, 3072, 3072), (8, 4096, 3072, 3072), (4, 256, 4096, 4096), (4, 1408, 4096, 4096),
+          (4, 2752, 3584, 3584), (4, 2752, 4096, 4096), (4, 3328, 4096, 4096), (2, 2048, 4096, 4096), (2, 5632, 4096, 4096), (8, 1408, 4096, 4096), (8, 704, 3584, 3584)]
+ALONE = [(4, 4096, 4096, 4096), (4, 8192, 4096, 4096), (2, 4096, 4096, 4096), (8, 2048, 3584, 3584), (8, 2048, 4096, 4096), (8, 4096, 4096, 4096), (4, 4096, 3584, 3584), (8, 5632, 4096, 4096),
+         (4, 4096, 5120, 4096), (4, 2048, 6144, 4096), (4, 4096, 6144, 4096), (4, 2048, 7168, 4096), (4, 4096, 8192, 4096)]
+
+
+@pytest.mark.parametrize("case", BESIDE + ALONE)
+def test_output_projection_beside_the_experts(case):
+    assert _moe(*case) == (case in BESIDE)
+
+
+def test_never_more_columns_than_the_launch_stages():
+    assert not _moe(4, 1408, 2048, 4160) and not _moe(4, 1408, 2048, 2048, torch.float32) and not _moe(4, 1408, 2048, 2052)

@@ -381,6 +381,11 @@ int lmx_op_decode_win(int32_t dtype, int32_t D, const void* qkv, int32_t qkv_str
                       const int32_t* const* pos_devs, void* const* ws_devs, int32_t* const* counters_devs, int32_t n_seq, void* tab_dev, const void* q_norm, const void* k_norm,
                       const float* cos_sin_dev, int32_t n_heads, int32_t n_kv_heads, int32_t s_max, int32_t n_split, int32_t qk_dim, int32_t rot_dims, int32_t window, int32_t sink,
                       int32_t gate_off, float scale, float eps, void* stream);
+/* the same with workgroups of 4 (as lmx_op_decode_win) or 8 waves where the grouped kernel takes the batch */
+int lmx_op_decode_win_waves(int32_t dtype, int32_t D, const void* qkv, int32_t qkv_stride, void* out, int32_t out_stride, void* const* kcaches, void* const* vtcaches,
+                      const int32_t* const* pos_devs, void* const* ws_devs, int32_t* const* counters_devs, int32_t n_seq, void* tab_dev, const void* q_norm, const void* k_norm,
+                      const float* cos_sin_dev, int32_t n_heads, int32_t n_kv_heads, int32_t s_max, int32_t n_split, int32_t qk_dim, int32_t rot_dims, int32_t window, int32_t sink,
+                      int32_t gate_off, float scale, float eps, int32_t waves, void* stream);
 /* what a decode step takes, on the host alone: form[2] = {all query heads of a kv head in one workgroup, splits}; span: keys that the longest sequence may have to walk.
  * (lmx_op_decode_win itself gives every batch that it can to the grouped kernel.) */
 int lmx_op_decode_win_form(int32_t dtype, int32_t D, int32_t n_heads, int32_t n_kv_heads, int32_t n_seq, int32_t span, int32_t* form);

@@ -702,11 +702,12 @@ int lmx_op_window_attn(int32_t dtype, int32_t D, const void* q, int32_t q_stride
     if (rows_form || dtype == kF32 || D > 128) launch_rows_attn(dtype, D, a, S(stream)); else launch_flash_prefill(dtype, D, a, S(stream));
     LMX_API_END
 }
-int lmx_op_decode_win(int32_t dtype, int32_t D, const void* qkv, int32_t qkv_stride, void* out, int32_t out_stride, void* const* kcaches, void* const* vtcaches,
+int lmx_op_decode_win_waves(int32_t dtype, int32_t D, const void* qkv, int32_t qkv_stride, void* out, int32_t out_stride, void* const* kcaches, void* const* vtcaches,
                       const int32_t* const* pos_devs, void* const* ws_devs, int32_t* const* counters_devs, int32_t n_seq, void* tab_dev, const void* q_norm, const void* k_norm,
                       const float* cos_sin_dev, int32_t n_heads, int32_t n_kv_heads, int32_t s_max, int32_t n_split, int32_t qk_dim, int32_t rot_dims, int32_t window, int32_t sink,
-                      int32_t gate_off, float scale, float eps, void* stream) {
+                      int32_t gate_off, float scale, float eps, int32_t waves, void* stream) {
     LMX_API_BEGIN
+    LMX_REQUIRE(waves == 4 || waves == 8, "decode_win: workgroups of four or eight waves");
     LMX_REQUIRE(n_seq >= 1 && kcaches && vtcaches && pos_devs && ws_devs && counters_devs && tab_dev, "decode_win: bad arguments");
     std::vector<DecodeFusedSeq> tab((size_t)n_seq);
     for (int i = 0; i < n_seq; ++i) tab[(size_t)i] = DecodeFusedSeq{kcaches[i], vtcaches[i], pos_devs[i], static_cast<float*>(ws_devs[i]), counters_devs[i]};
@@ -716,9 +717,15 @@ int lmx_op_decode_win(int32_t dtype, int32_t D, const void* qkv, int32_t qkv_str
     a.qkv = qkv; a.out = out; a.q_norm = q_norm; a.k_norm = k_norm; a.cos_sin = cos_sin_dev; a.tab = static_cast<const DecodeFusedSeq*>(tab_dev);
     a.n_seq = n_seq; a.qkv_stride = qkv_stride; a.out_stride = out_stride; a.n_heads = n_heads; a.n_kv_heads = n_kv_heads; a.s_max = s_max; a.n_split = n_split;
     a.qk_dim = qk_dim; a.rot_dims = rot_dims; a.window = window; a.sink = sink; a.gate_off = gate_off; a.scale = scale; a.eps = eps;
-    const int keys = window > 0 && window < s_max ? window : s_max;
-    launch_decode_win(dtype, D, a, /*grouped=*/true, /*wide=*/keys > 8 * 64 * n_split, S(stream));      // every batch that the grouped kernel can take; the engine: decode_win_form
+    launch_decode_win(dtype, D, a, /*grouped=*/true, /*wide=*/waves == 8, S(stream));      // every batch that the grouped kernel can take; the engine: decode_win_form
     LMX_API_END
+}
+int lmx_op_decode_win(int32_t dtype, int32_t D, const void* qkv, int32_t qkv_stride, void* out, int32_t out_stride, void* const* kcaches, void* const* vtcaches,
+                      const int32_t* const* pos_devs, void* const* ws_devs, int32_t* const* counters_devs, int32_t n_seq, void* tab_dev, const void* q_norm, const void* k_norm,
+                      const float* cos_sin_dev, int32_t n_heads, int32_t n_kv_heads, int32_t s_max, int32_t n_split, int32_t qk_dim, int32_t rot_dims, int32_t window, int32_t sink,
+                      int32_t gate_off, float scale, float eps, void* stream) {
+    return lmx_op_decode_win_waves(dtype, D, qkv, qkv_stride, out, out_stride, kcaches, vtcaches, pos_devs, ws_devs, counters_devs, n_seq, tab_dev, q_norm, k_norm, cos_sin_dev, n_heads, n_kv_heads,
+                                   s_max, n_split, qk_dim, rot_dims, window, sink, gate_off, scale, eps, 4, stream);
 }
 int lmx_op_decode_win_form(int32_t dtype, int32_t D, int32_t n_heads, int32_t n_kv_heads, int32_t n_seq, int32_t span, int32_t* form) {
     LMX_API_BEGIN

@@ -266,8 +266,9 @@ def window_attn(qkv, kcache, vtcache, q_pos0, n_heads, n_kv_heads, scale, window
     return out
 
 
-def decode_win(qkv, kcaches, vtcaches, pos_words, cos_sin, n_heads, n_kv_heads, qk_dim, rot_dims, scale, eps, q_norm=None, k_norm=None, window=0, sink=True, gate_off=-1, n_split=1):
-    """One new token per sequence (row i of qkv, pre-norm, pre-rotation): append to cache i at its position word, windowed attention.  Returns [n_seq, n_heads * D]."""
+def decode_win(qkv, kcaches, vtcaches, pos_words, cos_sin, n_heads, n_kv_heads, qk_dim, rot_dims, scale, eps, q_norm=None, k_norm=None, window=0, sink=True, gate_off=-1, n_split=1, waves=4):
+    """One new token per sequence (row i of qkv, pre-norm, pre-rotation): append to cache i at its position word, windowed attention.  waves: of a workgroup of the grouped kernel, 4 or 8.
+    Returns [n_seq, n_heads * D]."""
     import ctypes
     _need_cuda(qkv, cos_sin, q_norm, k_norm, *kcaches, *vtcaches, *pos_words)
     n = qkv.shape[0]
@@ -277,8 +278,8 @@ def decode_win(qkv, kcaches, vtcaches, pos_words, cos_sin, n_heads, n_kv_heads, 
     cnt = [torch.zeros(n_heads, dtype=torch.int32, device=qkv.device) for _ in range(n)]
     tab = torch.empty(lib.lmx_op_decode_attn_batch_tab_bytes(n), dtype=torch.uint8, device=qkv.device)
     arr = lambda ts: (ctypes.c_void_p * n)(*[t.data_ptr() for t in ts])
-    check(lib.lmx_op_decode_win(torch_dtype_code(qkv.dtype), D, ptr(qkv), qkv.stride(0), ptr(out), out.stride(0), arr(kcaches), arr(vtcaches), arr(pos_words), arr(ws), arr(cnt), n, ptr(tab),
-                                ptr(q_norm), ptr(k_norm), ptr(cos_sin), n_heads, n_kv_heads, s_max, n_split, qk_dim, rot_dims, window, int(sink), gate_off, scale, eps, stream_handle()),
+    check(lib.lmx_op_decode_win_waves(torch_dtype_code(qkv.dtype), D, ptr(qkv), qkv.stride(0), ptr(out), out.stride(0), arr(kcaches), arr(vtcaches), arr(pos_words), arr(ws), arr(cnt), n, ptr(tab),
+                                ptr(q_norm), ptr(k_norm), ptr(cos_sin), n_heads, n_kv_heads, s_max, n_split, qk_dim, rot_dims, window, int(sink), gate_off, scale, eps, waves, stream_handle()),
           "decode_win")
     return out
 

@@ -389,6 +389,7 @@ int lmx_op_decode_win_waves(int32_t dtype, int32_t D, const void* qkv, int32_t q
 /* what a decode step takes, on the host alone: form[2] = {all query heads of a kv head in one workgroup, splits}; span: keys that the longest sequence may have to walk.
  * (lmx_op_decode_win itself gives every batch that it can to the grouped kernel.) */
 int lmx_op_decode_win_form(int32_t dtype, int32_t D, int32_t n_heads, int32_t n_kv_heads, int32_t n_seq, int32_t span, int32_t* form);
+int lmx_op_decode_win_form_waves(int32_t dtype, int32_t D, int32_t n_heads, int32_t n_kv_heads, int32_t n_seq, int32_t max_len, int32_t window, int32_t* waves);      /* the grouped kernel's: 4 or 8; max_len: cached keys of the longest sequence */
 /* a parallel layer's gate | up of N rows over width K beside its delta step of `heads` heads of 64, 128 or 256 (head_dim) in one launch, one sequence: joins = 1 where a decode step does so */
 int lmx_op_delta_joins(int32_t dtype, int32_t heads, int32_t head_dim, int32_t N, int32_t K, int32_t* joins);
 /* its output projection of out_k columns over width K beside its `slots` experts' first product of 2 ff rows, one sequence: as above */

@@ -730,8 +730,14 @@ int lmx_op_decode_win(int32_t dtype, int32_t D, const void* qkv, int32_t qkv_str
 int lmx_op_decode_win_form(int32_t dtype, int32_t D, int32_t n_heads, int32_t n_kv_heads, int32_t n_seq, int32_t span, int32_t* form) {
     LMX_API_BEGIN
     LMX_REQUIRE(form && n_heads >= 1 && n_kv_heads >= 1 && n_heads % n_kv_heads == 0 && n_seq >= 1 && span >= 1, "decode_win_form: bad arguments");
-    const WinForm f = decode_win_form(dtype, D, n_heads, n_kv_heads, n_seq, span);
+    const WinForm f = decode_win_form(dtype, D, n_heads, n_kv_heads, n_seq, span - 1, 0);
     form[0] = f.grouped; form[1] = f.n_split;
+    LMX_API_END
+}
+int lmx_op_decode_win_form_waves(int32_t dtype, int32_t D, int32_t n_heads, int32_t n_kv_heads, int32_t n_seq, int32_t max_len, int32_t window, int32_t* waves) {
+    LMX_API_BEGIN
+    LMX_REQUIRE(waves && n_heads >= 1 && n_kv_heads >= 1 && n_heads % n_kv_heads == 0 && n_seq >= 1 && max_len >= 0 && window >= 0, "decode_win_form: bad arguments");
+    *waves = decode_win_form(dtype, D, n_heads, n_kv_heads, n_seq, max_len, window).wide ? 8 : 4;
     LMX_API_END
 }
 

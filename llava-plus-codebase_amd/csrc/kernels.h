@@ -248,7 +248,7 @@ struct WinDecodeArgs {
 void launch_decode_win(int dtype, int D, const WinDecodeArgs& a, bool grouped, bool wide, hipStream_t st);
 bool decode_win_groups(int dtype, int D, int n_heads, int n_kv_heads, int n_seq);
 struct WinForm { bool grouped; int n_split; bool wide; };
-WinForm decode_win_form(int dtype, int D, int n_heads, int n_kv_heads, int n_seq, int span);      // what a step takes; span: keys that the longest sequence may have to walk
+WinForm decode_win_form(int dtype, int D, int n_heads, int n_kv_heads, int n_seq, int max_len, int window);      // what a step takes; max_len: cached keys of the longest sequence
 
 // ---- gated delta rule (delta.hip): per head a state S [key channel][value channel] in fp32, S <- g S;  u = beta (v - S^T k);  S <- S + k u^T;  o = S^T q -----------------
 // Projection rows of a layer: q [G][DK] | k [G][DK] | v [H][DV] | beta [H] | ...; DK in {64, 128, 256} and DV (a multiple of 64) are padded head widths, the padding is

@@ -564,10 +564,7 @@ static WinDecodeArgs decode_args(const Stack& S, const StackLayer& l, int dtype,
     a.qkv = qkv; a.out = out; a.q_norm = l.qn; a.k_norm = l.kn; a.cos_sin = d.rope_dims ? S.rope[(size_t)d.rope_table] : nullptr;
     a.n_seq = n_seq; a.qkv_stride = l.qkv_n; a.out_stride = l.out_k; a.n_heads = d.n_heads; a.n_kv_heads = d.n_kv_heads; a.s_max = s_max;
     a.qk_dim = d.qk_dim; a.rot_dims = d.rope_dims; a.window = d.window; a.sink = d.softmax_sink; a.gate_off = l.gate_off; a.scale = d.attn_scale; a.eps = S.c.norm_eps;
-    // chunks the longest member's window can touch; enough workgroups to fill the chip, no more
-    int span = max_len + 1;
-    if (d.window > 0 && d.window + 127 < span) span = d.window + 127;
-    f = decode_win_form(dtype, l.D, d.n_heads, d.n_kv_heads, n_seq, span);
+    f = decode_win_form(dtype, l.D, d.n_heads, d.n_kv_heads, n_seq, max_len, d.window);
     a.n_split = f.n_split;
     return a;
 }

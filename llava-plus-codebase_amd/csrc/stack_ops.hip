@@ -912,17 +912,29 @@ bool decode_win_groups(int dtype, int D, int n_heads, int n_kv_heads, int n_seq)
 //    8 heads on  1          32 of 600   34 -> 15                  8 of 600  14 -> 15     2 of 600  12 -> 15      8 of 60  9 -> 12     (16 on 1: 16 of 600 25 -> 20, 4 of 600 13 -> 20)
 // so: up to groups of four from one chunk of keys on, larger groups by the bytes that one head a workgroup asks for (the merge grows with the group); shorter contexts only where
 // a group is three or four.  One sequence of 601 keys, 16 heads on 4: 11.1 us either way (9.7 since sums over lanes pass LDS by), all of it latency, so the form with more workgroups stays.
-// Eight waves instead of four: where a workgroup has a CU to itself and each of eight still walks more than one piece.  32 sequences of 600 .. 1024 keys, 8 kv heads: 31.4 -> 29.3 us
-// a launch (4.6 TB/s of keys and values); steps of 4 layers at up to 8 pieces a workgroup are 0 .. 1.5 % slower with eight (a longer merge for the same walk).
+// Eight waves instead of four: where a workgroup has a CU to itself, some of eight waves get a second piece, and the busiest workgroup takes no more pieces than with four (24 pieces in two
+// splits are 16 + 8 for 12 + 12).  A step of 10 layers of small linears, 5 .. 32 sequences, 4 or 8 kv heads, contexts of 260 .. 4000, four waves -> eight, us a layer:  one split, 8 pieces
+// 52.5 -> 51.9, 12 60.7 -> 59.6, 16 68.0 -> 65.8, 32 85.6 -> 83.4, 63 110.1 -> 109.5;  two, 17 48.6 -> 47.5, 34 59.0 -> 57.4, 52 67.9 -> 67.0, but 24 49.2 : 50.8 and 53.2 : 54.8, 41 56.1 : 57.1;
+// three, 48 58.9 -> 57.8, but 34 52.2 : 54.1;  four, 34 49.1 -> 47.9, but 42 50.2 : 52.1;  five, 42 44.8 -> 44.0, but 52 46.1 : 48.8.  Level where the busiest takes as many either way and more
+// workgroups are as busy (52 pieces in four splits 51.0 : 51.4).  Groups of two in one split 2 % more to 4 % less, in two 46.1 : 45.9, 59.7 : 60.4; a head a group 50.8 : 51.1, 58.7 : 57.8,
+// 63.7 : 64.9.  Five to eight pieces stay with four waves: 1 .. 4 % less with groups of three and more, 1 .. 2 % more with two.  32 sequences of 600 .. 1024 keys, 8 kv heads: 31.4 -> 29.3 us
+// a launch (4.6 TB/s of keys and values).
 // Splits: as many as make ONE round of workgroups of the grouped kernel (its waves fill a CU: 96 x 3 and 160 x 2 workgroups took a second round, 15 -> 19 and 21 -> 25 us).
-WinForm decode_win_form(int dtype, int D, int n_heads, int n_kv_heads, int n_seq, int span) {
+// pieces of 64 keys that the busiest of `splits` workgroups of nw waves takes of np
+static int win_most_pieces(int np, int splits, int nw) { return np / (nw * splits) * nw + std::min(nw, np % (nw * splits)); }
+WinForm decode_win_form(int dtype, int D, int n_heads, int n_kv_heads, int n_seq, int max_len, int window) {
+    // chunks the longest member's window can touch; enough workgroups to fill the chip, no more
+    const int span = window > 0 && window + 127 < max_len + 1 ? window + 127 : max_len + 1;
     const int group = n_heads / n_kv_heads, chunks = std::max(1, std::min((span + 127) / 128, DF_MAX_SPLIT));
     const double mb = (double)n_heads * n_seq * span * D * 4e-6;
     bool grouped = decode_win_groups(dtype, D, n_heads, n_kv_heads, n_seq);
     if (group <= 4) grouped = grouped && (span >= 128 || (group >= 3 && mb >= 10));
     else grouped = grouped && mb >= 0.6 * group * group;
     const int wgs = (grouped ? n_kv_heads : n_heads) * n_seq, n_split = std::max(1, std::min(chunks, grouped ? 256 / wgs : (1024 + wgs - 1) / wgs));
-    return WinForm{grouped, n_split, grouped && wgs * n_split <= 256 && span > 8 * 64 * n_split};
+    // cached keys in sight, wherever in a piece the window begins
+    const int np = window > 0 && window <= max_len ? std::min((max_len + 63) / 64, (window + 61) / 64 + 1) : (max_len + 63) / 64;
+    const bool wide = grouped && wgs * n_split <= 256 && np > 8 * n_split && win_most_pieces(np, n_split, 8) <= win_most_pieces(np, n_split, 4) && group >= (n_split > 1 ? 3 : 2);
+    return WinForm{grouped, n_split, wide};
 }
 
 void launch_decode_win(int dtype, int D, const WinDecodeArgs& a, bool grouped, bool wide, hipStream_t st) {

@@ -161,6 +161,7 @@ _SIGS = {
     "lmx_op_delta_joins": (c_int32, [c_int32] * 5 + [POINTER(c_int32)]),
     "lmx_op_moe_joins": (c_int32, [c_int32] * 5 + [POINTER(c_int32)]),
     "lmx_op_decode_win_form": (c_int32, [c_int32] * 6 + [POINTER(c_int32)]),
+    "lmx_op_decode_win_form_waves": (c_int32, [c_int32] * 7 + [POINTER(c_int32)]),
     "lmx_op_argmax": (c_int32, [c_int32, c_void_p, c_int32, c_void_p, c_void_p]),
     "lmx_op_ce_loss": (c_int32, [c_int32, c_void_p, c_int32, c_void_p, c_int32, c_int32, c_int32, c_int64, c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_int32, c_void_p]),
     "lmx_op_rmsnorm_bwd": (c_int32, [c_int32, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int32, c_int32, c_float, c_void_p]),

@@ -397,6 +397,8 @@ int lmx_op_moe_joins(int32_t dtype, int32_t slots, int32_t ff, int32_t K, int32_
 /* act(x_row W_g^T) of every slot (row, choice): g = ids[slot], in [0, groups), picks one of the groups' weights w [groups][N][K]; x row = slot / per_row (shared_x) or slot, c row = slot.
  * bm: rows of a tile, 0 = as the engine chooses; 32, 64 or, 16-bit four-wave tiles, 128 .. 256 in steps of 32, those with nb blocks of 32 columns (0 = as the engine chooses).
  * plan: lmx_op_group_plan_bytes(rows, per_row) bytes of scratch. */
+/* tiles of bm = 32 or 64 rows, on the host alone: form[2] = {weights marked streaming, slabs of the ring}; rows: of all groups together (planned) or of each */
+int lmx_op_group_gemm_form(int32_t rows, int32_t groups, int32_t planned, int32_t N, int32_t K, int32_t bm, int32_t* form);
 size_t lmx_op_group_plan_bytes(int32_t rows, int32_t per_row);
 int lmx_op_group_gemm(int32_t dtype, const void* x, const void* w, void* c, const int32_t* ids, int32_t rows, int32_t per_row, int32_t groups, int32_t shared_x, int32_t N, int32_t K,
                       int32_t act, int32_t bm, int32_t nb, void* plan, void* stream);

@@ -762,6 +762,17 @@ int lmx_op_moe_joins(int32_t dtype, int32_t slots, int32_t ff, int32_t K, int32_
     LMX_API_END
 }
 
+int lmx_op_group_gemm_form(int32_t rows, int32_t groups, int32_t planned, int32_t N, int32_t K, int32_t bm, int32_t* form) {
+    LMX_API_BEGIN
+    LMX_REQUIRE(form && rows >= 1 && groups >= 1 && N >= 1 && K >= 64 && (bm == 32 || bm == 64), "group_gemm_form: bad arguments");
+    GroupGemmArgs a{};
+    a.rows = rows; a.groups = groups; a.N = N; a.K = K;
+    if (planned) a.plan.n_tiles = form;                               // (asked for, never read)
+    const GroupGemmForm f = group_gemm_form(a, bm);
+    form[0] = f.stream; form[1] = f.slabs;
+    LMX_API_END
+}
+
 size_t lmx_op_group_plan_bytes(int32_t rows, int32_t per_row) { return rows > 0 && per_row > 0 ? group_plan_bytes(rows * per_row) : 0; }
 int lmx_op_group_gemm(int32_t dtype, const void* x, const void* w, void* c, const int32_t* ids, int32_t rows, int32_t per_row, int32_t groups, int32_t shared_x, int32_t N, int32_t K,
                       int32_t act, int32_t bm, int32_t nb, void* plan, void* stream) {

@@ -341,6 +341,8 @@ struct GroupGemmArgs {
     int x_group = 0, c_group = 0, act = 0, per_row = 1;
     GroupPlan plan{};
 };
+struct GroupGemmForm { bool stream; int slabs; };
+GroupGemmForm group_gemm_form(const GroupGemmArgs& a, int bm);      // tiles of 32 and 64 rows: weights marked streaming, slabs of the ring
 void launch_group_gemm(int dtype, const GroupGemmArgs& a, int bm, hipStream_t st, int nb = 0);
 int group_gemm_bm(const GroupGemmArgs* a, int n);                // rows of a tile for n products over one plan
 // the four-wave form (gemm4w.hip): tiles of 128, 160 .. 256 rows

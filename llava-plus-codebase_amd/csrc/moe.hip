@@ -84,7 +84,7 @@ void launch_group_plan(const int* ids, int slots, int E, int bm, const GroupPlan
 // MFMA tiles of a grouped product: the LDS ring of gemm_pipe_kernel (gemm.hip) with a row list.  Logical tiles run group by group, a group's row tiles next to each
 // other for one panel of its weight.  The grid is an upper bound: workgroups past the plan's tile count leave at once.
 // ---------------------------------------------------------------------------------------------------------------
-template <typename T, int BM, int BN, int WM, int WN, int NSTAGE>
+template <typename T, int BM, int BN, int WM, int WN, int NSTAGE, bool STREAM>
 __global__ __launch_bounds__(WM * WN * 64) void group_gemm_kernel(GroupGemmArgs a) {
     constexpr int NW = WM * WN, TM = BM / WM, TN = BN / WN, MT = TM / 32, NTL = TN / 32, PIECES = (BM + BN) / 8, PPW = PIECES / NW;
     constexpr int BUF_BYTES = (BM + BN) * GEMM_ROWB;
@@ -133,20 +133,16 @@ __global__ __launch_bounds__(WM * WN * 64) void group_gemm_kernel(GroupGemmArgs 
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
     const int nk = a.K / GEMM_BK;
     const unsigned lds_base = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
-    // Tiles walk K from different places (in step, all of them ask for the same 128 bytes of every weight row at a time), and weights that nearly always have one reader, groups filling
-    // four fifths of a tile in the mean or less, are marked streaming so that the rows stay in L2.  32 rows x 4 of 16 experts, weights cold, us: 5504 x 4096 gated 135 -> 120, 4096 x 2752
-    // 66 -> 56, 2816 x 2048 gated 43 -> 33.5, 2048 x 1408 18 -> 16.5; with two slabs where more than 512 tiles come, all of them resident, 110 (6.5 TB/s of weights) and 54.5.  Tiles of
-    // 64 rows, 5504 x 4096: 50 rows a group 138 -> 119, 64 rows 149: 162.
-    const bool lone = a.plan.n_tiles ? a.rows * 5 <= a.groups * BM * 4 : a.rows <= BM;
-    const int rot = (tile_n * 5 + grp * 3) % nk;
+    const int rot = STREAM ? (tile_n * 5 + grp * 3) % nk : 0;      // (in step, all tiles ask for the same 128 bytes of every weight row at a time)
     auto stage = [&](int kt, unsigned buf_off) {             // (inline asm for the reason given in gemm_pipe_kernel: ordering is the counted vmcnt + s_barrier below)
-        int k = kt + rot; k = k < nk ? k : k - nk;
+        int k = kt;
+        if constexpr (STREAM) { k += rot; k = k < nk ? k : k - nk; }
 #pragma unroll
         for (int i = 0; i < PPW; ++i) {
             const unsigned dst = __builtin_amdgcn_readfirstlane(lds_base + buf_off + (wave + NW * i) * 1024);
             const T* src = gsrc[i] + (size_t)k * GEMM_BK;
             unsigned keep;
-            if (lone && (wave + NW * i) * 8 >= BM)           // (wave-uniform)
+            if (STREAM && (wave + NW * i) * 8 >= BM)         // (wave-uniform)
                 asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt\n\ts_mov_b32 m0, %0"
                              : "=&s"(keep) : "v"(src), "s"(dst) : "memory");
             else
@@ -200,15 +196,29 @@ __global__ __launch_bounds__(WM * WN * 64) void group_gemm_kernel(GroupGemmArgs 
     }
 }
 
-template <typename T, int BM, int BN, int WM, int WN, int NSTAGE>
+template <typename T, int BM, int BN, int WM, int WN, int NSTAGE, bool STREAM>
 static void launch_group_gemm_cfg(const GroupGemmArgs& a, int m_tiles, hipStream_t st) {
     constexpr int smem = NSTAGE * (BM + BN) * GEMM_ROWB;
     static_assert(smem <= 160 * 1024, "LDS ring does not fit");
-    auto kern = group_gemm_kernel<T, BM, BN, WM, WN, NSTAGE>;
+    auto kern = group_gemm_kernel<T, BM, BN, WM, WN, NSTAGE, STREAM>;
     static bool attr_set = false;
     if (!attr_set) { LMX_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, smem)); attr_set = true; }
     LMX_LAUNCH(kern, dim3(m_tiles * cdiv(a.N, BN)), dim3(WM * WN * 64), smem, st, a);
     LMX_CHECK_HIP(hipGetLastError());
+}
+// Tiles of 32 and 64 rows.  Weights that nearly always have one reader, groups filling four fifths of a tile in the mean or less, are marked streaming, so that the rows stay in L2, and every
+// workgroup walks K from a place of its own.  Both pay where the workgroups fill the chip (counted as if the rows were spread evenly: the grid itself is an upper bound); a few of them wait
+// longer for a line that is fetched again for its second half.  320 products of 4 .. 64 groups at 3 .. 63 rows a group, weights cold, time of plain loads over streaming:  528 .. 1024
+// workgroups 1.04 .. 1.43, 240 .. 512 1.03 .. 1.39, 224 0.98 .. 1.25, 208 0.97, 192 1.03 .. 1.17 with K a multiple of 2048 (rows on the same channels) and 0.93 .. 1.05 without, fewer
+// 0.69 .. 1.02 (704 x 6528 in 4 groups 46 us : 67, 576 x 6144 in 6 43 : 62).  32 rows x 4 of 16 experts: 5504 x 4096 gated 135 -> 120 us, 2816 x 2048 43 -> 33.5.
+// Two slabs instead of four: past what four let reside (512 workgroups) up to all that two do (1024).  5504 x 4096 (688) 120 -> 110 us, 6.5 TB/s of weights; two / four of 320 .. 416
+// workgroups 0.89 .. 0.95, of 528 .. 992 1.00 .. 1.23, of 1040 .. 1536 0.85 .. 0.96, from 1800 on level.
+GroupGemmForm group_gemm_form(const GroupGemmArgs& a, int bm) {
+    if (bm > 64) return GroupGemmForm{false, 0};
+    const int nt = cdiv(a.N, 128), wgs = a.groups * cdiv(a.rows, a.plan.n_tiles ? a.groups * bm : bm) * nt;
+    const bool lone = a.plan.n_tiles ? a.rows * 5 <= a.groups * bm * 4 : a.rows <= bm;
+    const bool stream = lone && wgs >= (a.K % 2048 == 0 ? 192 : 224);
+    return GroupGemmForm{stream, bm == 64 ? 3 : a.plan.n_tiles && stream && wgs > 512 && wgs <= 1024 ? 2 : 4};
 }
 void launch_group_gemm(int dtype, const GroupGemmArgs& a, int bm, hipStream_t st, int nb) {
     LMX_REQUIRE(a.X && a.W && a.C && a.rows >= 1 && a.groups >= 1 && a.N >= 1 && a.K >= 64 && a.K % 64 == 0 && a.per_row >= 1, "group_gemm: bad arguments");
@@ -216,10 +226,12 @@ void launch_group_gemm(int dtype, const GroupGemmArgs& a, int bm, hipStream_t st
     LMX_REQUIRE(!act_gated(a.act) || a.N % 64 == 0, "group_gemm: gated rows come in groups of 64");
     // with a plan: every group's last tile may be part empty; no more tiles than rows
     const int m_tiles = a.plan.n_tiles ? std::min(a.rows, a.rows / bm + a.groups) : a.groups * cdiv(a.rows, bm);
-    // two slabs: 2048 x 1408 of 288 tiles 16.5 -> 25.5 us, 2816 x 2048 of 440 33.5 -> 34; 5504 x 4096 at 20 / 24 / 32 rows a group, two tiles for most, 121 / 122 / 154 -> 110 / 111 / 197
-    const bool many = a.plan.n_tiles && a.rows <= 24 * a.groups && m_tiles * cdiv(a.N, 128) > 512;
-#define L(TT) do { if (bm == 32 && many) launch_group_gemm_cfg<TT, 32, 128, 1, 2, 2>(a, m_tiles, st); else if (bm == 32) launch_group_gemm_cfg<TT, 32, 128, 1, 2, 4>(a, m_tiles, st); else if (bm == 64) launch_group_gemm_cfg<TT, 64, 128, 2, 2, 3>(a, m_tiles, st); \
-                   else throw Error{"group_gemm: tiles of 32, 64 or 128 .. 256 rows"}; } while (0)
+    const GroupGemmForm f = group_gemm_form(a, bm);
+    const bool stream = f.stream, two = f.slabs == 2;
+#define L(TT) do { if (bm == 32 && two) launch_group_gemm_cfg<TT, 32, 128, 1, 2, 2, true>(a, m_tiles, st); \
+                    else if (bm == 32) { if (stream) launch_group_gemm_cfg<TT, 32, 128, 1, 2, 4, true>(a, m_tiles, st); else launch_group_gemm_cfg<TT, 32, 128, 1, 2, 4, false>(a, m_tiles, st); } \
+                    else if (bm == 64) { if (stream) launch_group_gemm_cfg<TT, 64, 128, 2, 2, 3, true>(a, m_tiles, st); else launch_group_gemm_cfg<TT, 64, 128, 2, 2, 3, false>(a, m_tiles, st); } \
+                    else throw Error{"group_gemm: tiles of 32, 64 or 128 .. 256 rows"}; } while (0)
     if (bm > 64 && dtype != kF32) { launch_group_gemm4w(dtype, a, bm, nb, m_tiles, st); return; }
     if (dtype == kBF16) L(bf16_t); else if (dtype == kF16) L(f16_t); else throw Error{"group_gemm: 16-bit models"};
 #undef L

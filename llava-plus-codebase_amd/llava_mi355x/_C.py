@@ -156,6 +156,7 @@ _SIGS = {
     "lmx_op_window_attn": (c_int32, [c_int32, c_int32, c_void_p, c_int32, c_void_p, c_int32, c_void_p, c_void_p] + [c_int32] * 5 + [c_float, c_int32, c_int32, c_void_p, c_int32, c_void_p]),
     "lmx_op_decode_win": (c_int32, [c_int32, c_int32, c_void_p, c_int32, c_void_p, c_int32] + [POINTER(c_void_p)] * 5 + [c_int32] + [c_void_p] * 4 + [c_int32] * 9 + [c_float, c_float, c_void_p]),
     "lmx_op_decode_win_waves": (c_int32, [c_int32, c_int32, c_void_p, c_int32, c_void_p, c_int32] + [POINTER(c_void_p)] * 5 + [c_int32] + [c_void_p] * 4 + [c_int32] * 9 + [c_float, c_float, c_int32, c_void_p]),
+    "lmx_op_group_gemm_form": (c_int32, [c_int32] * 6 + [POINTER(c_int32)]),
     "lmx_op_group_plan_bytes": (c_size_t, [c_int32] * 2),
     "lmx_op_group_gemm": (c_int32, [c_int32] + [c_void_p] * 4 + [c_int32] * 9 + [c_void_p] * 2),
     "lmx_op_delta_joins": (c_int32, [c_int32] * 5 + [POINTER(c_int32)]),

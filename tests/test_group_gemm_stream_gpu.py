@@ -1,5 +1,5 @@
-"""Grouped products on tiles of 32 and 64 rows (csrc/moe.hip: group_gemm_kernel): two slabs from 513 tiles on, weights marked streaming up to four fifths of a tile a group in the mean, every
-tile's walk over K begun somewhere else."""
+"""Grouped products on tiles of 32 and 64 rows (csrc/moe.hip: group_gemm_kernel): plain loads, weights marked streaming with every
+tile's walk over K begun somewhere else, and two slabs (group_gemm_form: from 224 and from 513 to 1024 workgroups with work), on both sides of each line."""
 import pytest
 import torch
 
@@ -9,7 +9,8 @@ DT = {"bf16": torch.bfloat16, "f16": torch.float16}
 
 @pytest.mark.parametrize("dt", list(DT))
 @pytest.mark.parametrize("bm,rows,per_row,E,N", [(32, 32, 4, 16, 3264), (32, 32, 4, 16, 3328), (32, 96, 4, 16, 2560), (32, 97, 4, 16, 2560), (32, 104, 4, 16, 264), (64, 204, 4, 16, 264),
-                                                 (64, 205, 4, 16, 264), (32, 5, 3, 15, 4480), (32, 16, 1, 16, 4096)])
+                                                 (64, 205, 4, 16, 264), (32, 5, 3, 15, 4480), (32, 16, 1, 16, 4096), (32, 24, 4, 16, 1664), (32, 24, 4, 16, 1792), (32, 32, 4, 16, 4096),
+                                                 (32, 32, 4, 16, 4104), (32, 12, 4, 16, 8192), (32, 12, 4, 16, 8200), (64, 80, 4, 16, 1664), (64, 80, 4, 16, 1792)])
 @pytest.mark.parametrize("K", [64, 128, 192, 704])
 def test_products(cuda, dt, bm, rows, per_row, E, N, K):
     from llava_mi355x import ops

@@ -370,6 +370,8 @@ int lmx_op_sample(int32_t dtype, const void* logits_dev, int32_t V, float temper
  * decode_win: per-sequence pointers as lmx_op_decode_attn_batch (tab_dev: lmx_op_decode_attn_batch_tab_bytes(n_seq) bytes). */
 int lmx_op_residual_norm(int32_t dtype, const float* x_in, const void* y, const void* post_w, const void* inject, const void* pre_w, float* x_out, void* xn, int32_t rows,
                          int32_t H, int32_t H_real, float mult, float eps, void* stream);
+/* on the host alone: ahead = 1 where the norms' weights and the injected row are loaded with the rows */
+int lmx_op_residual_norm_form(int32_t dtype, int32_t rows, int32_t H, int32_t inject, int32_t* ahead);
 int lmx_op_gemv_residual(int32_t dtype, const float* x_in, const void* y, const void* post_w, const void* inject, const void* pre_w, float* x_out, const void* w, const void* bias,
                          void* c, int32_t N, int32_t H, int32_t H_real, float mult, float eps, int32_t act, void* stream);
 int lmx_op_linear_f32(int32_t dtype, const void* x, const void* w, float* c, int32_t M, int32_t N, int32_t K, float cap, int32_t form, void* stream);

@@ -660,6 +660,14 @@ int lmx_op_im2col(int32_t dtype, const void* pixels, void* out, int32_t N, int32
 }
 
 // ---- layer-stack decoders (stack_ops.hip) ----------------------------------------------------------------------------------------
+int lmx_op_residual_norm_form(int32_t dtype, int32_t rows, int32_t H, int32_t inject, int32_t* ahead) {
+    LMX_API_BEGIN
+    LMX_REQUIRE(ahead && rows >= 1 && H >= 8 && H <= 8192, "residual_norm_form: bad arguments");
+    ResidualNormArgs a{};
+    a.H = H; a.inject = inject ? ahead : nullptr;                     // (asked for, never read)
+    *ahead = residual_norm_ahead(dtype, a, rows);
+    LMX_API_END
+}
 int lmx_op_residual_norm(int32_t dtype, const float* x_in, const void* y, const void* post_w, const void* inject, const void* pre_w, float* x_out, void* xn, int32_t rows,
                          int32_t H, int32_t H_real, float mult, float eps, void* stream) {
     LMX_API_BEGIN

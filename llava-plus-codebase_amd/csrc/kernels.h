@@ -202,6 +202,7 @@ struct ResidualNormArgs {
     const void* moe_y = nullptr; const float* moe_w = nullptr; int top = 0;
     int xn_ld = 0, cast = 0;             // row pitch of xn (0: H)
 };
+bool residual_norm_ahead(int dtype, const ResidualNormArgs& a, int rows);
 void launch_residual_norm(int dtype, const ResidualNormArgs& a, int rows, hipStream_t st);
 // input rows of a model with a bigram embedding: from a portion's ids, from one sequence's state words or from a decode batch's table
 struct SeqStateRef;

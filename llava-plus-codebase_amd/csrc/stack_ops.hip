@@ -22,7 +22,8 @@ namespace lmx {
 // ---------------------------------------------------------------------------------------------------------------
 // residual + norms
 // ---------------------------------------------------------------------------------------------------------------
-template <typename T, int NP>
+// AHEAD: both norms' weights and the injected row are on their way with the rows, four experts' rows at a time (each behind the sum in front of it was a trip to memory of its own)
+template <typename T, int NP, bool AHEAD>
 __global__ __launch_bounds__(256) void residual_norm_kernel(ResidualNormArgs a) {
     __shared__ float red[4];
     const int row = blockIdx.x, tid = threadIdx.x, HC = a.H >> 3;
@@ -33,12 +34,11 @@ __global__ __launch_bounds__(256) void residual_norm_kernel(ResidualNormArgs a) 
     const T* post = y || a.top > 0 ? reinterpret_cast<const T*>(a.post_w) : nullptr;
     const T* pre = reinterpret_cast<const T*>(a.pre_w);
     float x[NP][8], yv[NP][8];
-    // Both norms' weights and the injected row are on their way with the rows, four experts' rows at a time: each behind the sum in front of it was a trip to memory of its own
     Chunk8<T> gp[NP], gn[NP], gi[NP];
 #pragma unroll
     for (int i = 0; i < NP; ++i) {
         const int c = tid + i * 256;
-        if (c >= HC) continue;
+        if (!AHEAD || c >= HC) continue;
         if (post) gp[i].load(post + c * 8);
         if (pre) gn[i].load(pre + c * 8);
         if (inj) gi[i].load(inj + c * 8);
@@ -58,17 +58,18 @@ __global__ __launch_bounds__(256) void residual_norm_kernel(ResidualNormArgs a) 
 #pragma unroll
             for (int e = 0; e < 8; ++e) yv[i][e] = 0.f;
         }
-        for (int k0 = 0; k0 < a.top; k0 += 4) {
-            Chunk8<T> m[4];
-            float wk[4];
+        constexpr int KE = AHEAD ? 4 : 1;
+        for (int k0 = 0; k0 < a.top; k0 += KE) {
+            Chunk8<T> m[KE];
+            float wk[KE];
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
+            for (int k = 0; k < KE; ++k) {
                 const size_t slot = (size_t)row * a.top + (k0 + k < a.top ? k0 + k : k0);
                 wk[k] = a.moe_w[slot];
                 m[k].load(reinterpret_cast<const T*>(a.moe_y) + slot * a.H + c * 8);
             }
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
+            for (int k = 0; k < KE; ++k) {
                 if (k0 + k >= a.top) continue;
                 float v[8]; m[k].get(v);
 #pragma unroll
@@ -90,6 +91,7 @@ __global__ __launch_bounds__(256) void residual_norm_kernel(ResidualNormArgs a) 
         for (int i = 0; i < NP; ++i) {
             const int c = tid + i * 256;
             if (c >= HC) continue;
+            if (!AHEAD) gp[i].load(post + c * 8);
             float g[8]; gp[i].get(g);
 #pragma unroll
             for (int e = 0; e < 8; ++e) x[i][e] += yv[i][e] * inv * g[e];
@@ -101,6 +103,7 @@ __global__ __launch_bounds__(256) void residual_norm_kernel(ResidualNormArgs a) 
         const int c = tid + i * 256;
         if (c >= HC) continue;
         if (inj) {
+            if (!AHEAD) gi[i].load(inj + c * 8);
             float g[8]; gi[i].get(g);
 #pragma unroll
             for (int e = 0; e < 8; ++e) x[i][e] += g[e];
@@ -122,6 +125,7 @@ __global__ __launch_bounds__(256) void residual_norm_kernel(ResidualNormArgs a) 
     for (int i = 0; i < NP; ++i) {
         const int c = tid + i * 256;
         if (c >= HC) continue;
+        if (!AHEAD) gn[i].load(pre + c * 8);
         float g[8], o[8]; gn[i].get(g);
 #pragma unroll
         for (int e = 0; e < 8; ++e) o[e] = x[i][e] * inv2 * g[e];
@@ -173,6 +177,18 @@ void launch_embed_rows(int dtype, const EmbedRowsArgs& a, int rows, hipStream_t 
     LMX_CHECK_HIP(hipGetLastError());
 }
 
+// Loads ahead: fewer trips to memory a row, but registers for fewer rows on a CU.  16-bit rows of up to 2048 either way eight, of up to 4096 six for eight, of up to 8192 three for six: not
+// where the rows are one round without and two with it, past 4096 nor where they are few rounds (with an injected row, one trip more, a round fewer; from 3073 to 4096 always).  us without /
+// with, rows from L2 and, in brackets, from memory:  128 x 4096 4.2 / 3.5, 512 x 4096 6.4 / 5.8 (8.0 / 7.3), 1700 x 3072 11.9 / 12.1 (13.8 / 14.7), 1664 x 2560 10.6 / 11.1 and injected
+// 10.4 / 11.1, 2560 x 4096 21.7 / 20.6 (25.1 / 23.7), 1664 x 4096 injected 15.5 / 14.3;  512 x 8192 11.4 / 10.6, 1024 x 8192 18.6 / 19.0, 1536 x 8192 24.4 / 26.7 (888 x 8192 18.7 / 19.9),
+// 2560 x 8192 40.7 / 42.2 and injected 44.1 / 43.0, 4096 x 8192 84.3 / 80.5.  fp32 rows keep twice as much on the way: ahead only in one round.
+bool residual_norm_ahead(int dtype, const ResidualNormArgs& a, int rows) {
+    const int np = (a.H / 8 + 255) / 256;
+    if (dtype == kF32) return rows <= (np == 1 ? 1792 : np == 2 ? 1024 : 512);
+    if (np == 1) return true;
+    if (np == 2) return rows <= 1536 || rows > 2048 || (a.inject && a.H > 3072);
+    return rows <= 768 || rows > (a.inject ? 1536 : 2560);
+}
 void launch_residual_norm(int dtype, const ResidualNormArgs& a, int rows, hipStream_t st) {
     LMX_REQUIRE(a.H % 8 == 0 && a.H > 0 && a.H <= 8192 && a.H_real >= 1 && a.H_real <= a.H, "residual_norm: width must be a multiple of 8, at most 8192");
     LMX_REQUIRE(a.top >= 0 && (a.top == 0 || (a.moe_y && a.moe_w)), "residual_norm: expert outputs need their weights");
@@ -180,7 +196,8 @@ void launch_residual_norm(int dtype, const ResidualNormArgs& a, int rows, hipStr
     LMX_REQUIRE(!(a.pre_w && a.cast) && a.xn_ld % 8 == 0, "residual_norm: norm or cast, in 16-byte rows");
     if (rows <= 0) return;
     const int np = (a.H / 8 + 255) / 256;
-#define R(TT, NPV) LMX_LAUNCH((residual_norm_kernel<TT, NPV>), dim3(rows), dim3(256), 0, st, a)
+#define R(TT, NPV) do { if (residual_norm_ahead(dtype, a, rows)) LMX_LAUNCH((residual_norm_kernel<TT, NPV, true>), dim3(rows), dim3(256), 0, st, a); \
+                        else LMX_LAUNCH((residual_norm_kernel<TT, NPV, false>), dim3(rows), dim3(256), 0, st, a); } while (0)
 #define RT(TT) do { if (np == 1) R(TT, 1); else if (np == 2) R(TT, 2); else R(TT, 4); } while (0)
     if (dtype == kBF16) RT(bf16_t); else if (dtype == kF16) RT(f16_t); else RT(float);
 #undef RT

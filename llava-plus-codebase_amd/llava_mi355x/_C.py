@@ -149,6 +149,7 @@ _SIGS = {
     "lmx_op_decode_attn_batch_tab_bytes": (c_size_t, [c_int32]),
     "lmx_op_decode_attn_ws_bytes": (c_size_t, [c_int32] * 4),
     "lmx_op_sample": (c_int32, [c_int32, c_void_p, c_int32, c_float, c_float, c_int32, ctypes.c_uint64, c_void_p, POINTER(ctypes.c_uint32), c_void_p, c_void_p, c_void_p]),
+    "lmx_op_residual_norm_form": (c_int32, [c_int32] * 4 + [POINTER(c_int32)]),
     "lmx_op_residual_norm": (c_int32, [c_int32] + [c_void_p] * 7 + [c_int32] * 3 + [c_float, c_float, c_void_p]),
     "lmx_op_gemv_residual": (c_int32, [c_int32] + [c_void_p] * 9 + [c_int32] * 3 + [c_float, c_float, c_int32, c_void_p]),
     "lmx_op_linear_f32": (c_int32, [c_int32] + [c_void_p] * 3 + [c_int32] * 3 + [c_float, c_int32, c_void_p]),

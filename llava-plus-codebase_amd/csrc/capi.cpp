@@ -750,6 +750,16 @@ int lmx_op_decode_win_form_waves(int32_t dtype, int32_t D, int32_t n_heads, int3
 }
 
 static GemvArgs plain_row(int32_t N, int32_t K) { return GemvArgs{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0.f, N, K, K, K, N, 0, kActNone}; }
+int lmx_op_gemv_form(int32_t N, int32_t K, int32_t act, int32_t norm, int32_t* form) {
+    LMX_API_BEGIN
+    LMX_REQUIRE(form && N >= 1 && K >= 8 && K <= 16384 && K % 8 == 0, "gemv_form: bad arguments");
+    GemvArgs g = plain_row(N, K);
+    g.act = act;
+    if (norm) g.norm_w = form;                                        // (asked for, never read)
+    const GemvForm f = gemv2_form(g);
+    form[0] = f.rows; form[1] = f.ahead;
+    LMX_API_END
+}
 int lmx_op_delta_joins(int32_t dtype, int32_t heads, int32_t head_dim, int32_t N, int32_t K, int32_t* joins) {
     LMX_API_BEGIN
     LMX_REQUIRE(joins && heads >= 1 && (head_dim == 64 || head_dim == 128 || head_dim == 256) && N >= 1 && K >= 64, "delta_joins: bad arguments");

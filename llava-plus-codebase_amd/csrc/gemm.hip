@@ -925,18 +925,28 @@ void launch_gemv_residual(int dtype, GemvArgs a, const ResidualNormArgs& rn, hip
 // The single-row decode linears of 16-bit models take the hand-counted stream.  (R rows per wave, P rounds in flight) per shape from the in-situ sweep
 // of round 3 (tools/mb_decode.py, LLaVA-1.5-7B, per launch incl. ~1.4 us of event pair; gemv_kernel -> gemv2_kernel): q|k|v 20.5 -> 19.1 us (R 2, P 4),
 // gate|up 30.9 -> 29.5 (2, 4), down 19.9 -> 17.8 (1, 8: K = 11008 keeps 8 KB per wave on the wire), lm_head 45.8 -> 42.2 (2, 4), o_proj 8.7 -> 8.8 (1, 2; now 1, 4).
+// Small linears (<= 32 M weights): o_proj keeps one row per wave (1024 short-lived workgroups); with the RMSNorm fused — the split-q step's q projection — every
+// workgroup also normalises the whole input row, so half as many workgroups with two rows per wave win: 8.1 -> 7.5 us (profiles/r05_small_gemv_rp.txt).
+// Four loads of a row ahead instead of two: 2048 x 5632 6.55 -> 5.72 us, 2048 x 7680 7.97 -> 7.10, 1024 x 2048 and 2048 x 1152 a tenth less; but a row of up to 1024 has no more than two and
+// waits for those past its end (8192 x 512 3.71 : 4.42, 13152 x 640 6.53 : 7.25), and of up to 2048 only the products of one round, or of so many that they hide each other's starts, gain:
+// 2048 x 2048 1.5 % less, 12288 x 1408 7 %, 5120 x 2048 5.41 : 5.83, 6144 x 1792 5.82 : 6.28, 8192 x 1408 6.07 : 6.46.
+GemvForm gemv2_form(const GemvArgs& a) {
+    const size_t weights = (size_t)a.N * a.K;
+    if (act_gated(a.act)) return GemvForm{2, 4};
+    if (a.K >= 8192) return GemvForm{1, 8};
+    if (weights > ((size_t)1 << 25) || a.norm_w) return GemvForm{2, 4};
+    return GemvForm{1, a.K <= 1024 || (a.K <= 2048 && weights > ((size_t)1 << 22) && a.N < 11776) ? 2 : 4};
+}
 template <typename T>
 static bool launch_gemv2(const GemvArgs& a, hipStream_t st) {
     if constexpr (sizeof(T) != 2) return false;
     else {
         if (!gemv2_applies(TypeInfo<T>::id, a)) return false;
-        if (act_gated(a.act)) launch_gemv2_r<T, 2, 4>(a, st);
-        else if (a.K >= 8192) launch_gemv2_r<T, 1, 8>(a, st);
-        // small linears (<= 32 M weights): o_proj keeps one row per wave (1024 short-lived workgroups); with the RMSNorm fused — the split-q step's q projection — every
-        // workgroup also normalises the whole input row, so half as many workgroups with two rows per wave win: 8.1 -> 7.5 us (profiles/r05_small_gemv_rp.txt).  Four loads of a row
-        // ahead instead of two: 2048 x 5632 6.55 -> 5.72 us, 2048 x 7680 7.97 -> 7.10, rows of 2048 .. 4096 as before (3.82, 5.08, 7.1)
-        else if ((size_t)a.N * a.K <= ((size_t)1 << 25)) { if (a.norm_w) launch_gemv2_r<T, 2, 4>(a, st); else launch_gemv2_r<T, 1, 4>(a, st); }
-        else launch_gemv2_r<T, 2, 4>(a, st);
+        const GemvForm f = gemv2_form(a);
+        if (f.rows == 2) launch_gemv2_r<T, 2, 4>(a, st);
+        else if (f.ahead == 8) launch_gemv2_r<T, 1, 8>(a, st);
+        else if (f.ahead == 4) launch_gemv2_r<T, 1, 4>(a, st);
+        else launch_gemv2_r<T, 1, 2>(a, st);
         return true;
     }
 }

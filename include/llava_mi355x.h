@@ -313,6 +313,7 @@ int lmx_op_gemv(int32_t dtype, const void* x, const void* w, void* c, const void
                 int32_t MB, int32_t N, int32_t K, int32_t ldx, int32_t ldw, int32_t ldc, int32_t ldr, int32_t act, void* stream);
 /* one row of a 16-bit model, on the host alone: form[2] = {weight rows of a wave, 16-byte loads of each on the way}; norm: with the input row's norm in the launch */
 int lmx_op_gemv_form(int32_t N, int32_t K, int32_t act, int32_t norm, int32_t* form);
+int lmx_op_gemv_residual_form(int32_t N, int32_t K, int32_t act, int32_t* form);      /* of lmx_op_gemv_residual: form[3], the third the waves of a workgroup */
 int lmx_op_rmsnorm(int32_t dtype, const void* x, const void* w, void* y, int32_t rows, int32_t H, float eps, void* stream);
 int lmx_op_layernorm(int32_t dtype, const void* x, const void* w, const void* b, void* y, int32_t rows, int32_t H, float eps, void* stream);
 int lmx_op_rope_kv(int32_t dtype, int32_t head_dim, void* qkv, void* kcache, void* vtcache, const float* cos_sin_dev, int32_t pos0,

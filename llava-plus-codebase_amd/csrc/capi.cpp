@@ -760,6 +760,15 @@ int lmx_op_gemv_form(int32_t N, int32_t K, int32_t act, int32_t norm, int32_t* f
     form[0] = f.rows; form[1] = f.ahead;
     LMX_API_END
 }
+int lmx_op_gemv_residual_form(int32_t N, int32_t K, int32_t act, int32_t* form) {
+    LMX_API_BEGIN
+    LMX_REQUIRE(form && N >= 1 && K >= 8 && K <= 8192 && K % 8 == 0, "gemv_residual_form: bad arguments");
+    GemvArgs g = plain_row(N, K);
+    g.act = act;
+    const GemvForm f = gemv2_res_form(g);
+    form[0] = f.rows; form[1] = f.ahead; form[2] = f.waves;
+    LMX_API_END
+}
 int lmx_op_delta_joins(int32_t dtype, int32_t heads, int32_t head_dim, int32_t N, int32_t K, int32_t* joins) {
     LMX_API_BEGIN
     LMX_REQUIRE(joins && heads >= 1 && (head_dim == 64 || head_dim == 128 || head_dim == 256) && N >= 1 && K >= 64, "delta_joins: bad arguments");

@@ -900,11 +900,21 @@ static void launch_gemv2_res_rx(const GemvArgs& a, const ResidualNormArgs& rn, h
 // take a row a wave, and those of long rows besides four waves as the plain linear.  us a launch, weights cold, four waves of two rows -> here:  3088 x 2048 5.59 -> 5.02
 //   6464 x 2048 8.53 -> 7.96   11264 x 2048 gated 11.74 -> 10.66   7000 x 3072 11.40 -> 9.14   16384 x 3072 gated 20.1 -> 17.1   22016 x 4096 gated 31.2 -> 29.6   (2048 x 2048 3.92: 4.69,
 //   4096 x 4096 8.50: 8.75);  a row a wave  1280 x 2048 3.74 -> 3.46   2048 x 2048 3.92 -> 3.81   4096 x 4096 8.50 -> 7.76   (2048 x 3072 5.09: 5.23, 2048 x 4096 5.72: 5.86).
+// Rows of 2048 in one to one and a half rounds of eight waves stay with four: 4096 6.66 -> 6.44, but 4128 6.66: 6.85, 5120 7.30: 7.66, 6144 7.71: 8.05, 6400 8.17 -> 7.92 (of 1536 1 .. 4 % less,
+// of 2560 7 .. 10 %).
+GemvForm gemv2_res_form(const GemvArgs& a) {
+    const bool between = a.K > 1536 && a.K <= 2048 && a.N > 4096 && a.N <= 6144;
+    if (a.K > 4096 || between) return GemvForm{2, 4, 4};
+    if (a.N >= 2560 && (a.K <= 3072 || a.N >= 6144)) return GemvForm{2, 2, 8};
+    if (!act_gated(a.act) && (a.K <= 2048 || a.N >= 4096)) return GemvForm{1, 4, 8};
+    return GemvForm{2, 4, 4};
+}
 template <typename T>
 static void launch_gemv2_res(const GemvArgs& a, const ResidualNormArgs& rn, hipStream_t st) {
-    if (a.K > 4096) { launch_gemv2_res_rx<T, 2, 4, 4, 4>(a, rn, st); return; }
-    if (a.N >= 2560 && (a.K <= 3072 || a.N >= 6144)) launch_gemv2_res_rx<T, 2, 2, 1, 8>(a, rn, st);
-    else if (!act_gated(a.act) && (a.K <= 2048 || a.N >= 4096)) launch_gemv2_res_rx<T, 1, 4, 1, 8>(a, rn, st);
+    const GemvForm f = gemv2_res_form(a);
+    if (a.K > 4096) launch_gemv2_res_rx<T, 2, 4, 4, 4>(a, rn, st);
+    else if (f.waves == 8 && f.rows == 2) launch_gemv2_res_rx<T, 2, 2, 1, 8>(a, rn, st);
+    else if (f.waves == 8) launch_gemv2_res_rx<T, 1, 4, 1, 8>(a, rn, st);
     else if (a.K <= 2048) launch_gemv2_res_rx<T, 2, 4, 1, 4>(a, rn, st);
     else launch_gemv2_res_rx<T, 2, 4, 2, 4>(a, rn, st);
 }

@@ -95,8 +95,9 @@ struct GemvArgs {
     int act;
     int c_f32 = 0; float cap = 0.f;   // fp32 output with an optional soft cap, as GemmArgs::c_f32 (no SiLU*mul)
 };
-struct GemvForm { int rows, ahead; };       // rows of a wave, loads of each on the way
+struct GemvForm { int rows, ahead, waves = 4; };       // rows of a wave, loads of each on the way, waves of a workgroup
 GemvForm gemv2_form(const GemvArgs& a);     // of a linear on the weight stream (gemv2.h)
+GemvForm gemv2_res_form(const GemvArgs& a); // of one whose row is formed in front of it
 void launch_gemv(int dtype, const GemvArgs& a, int MB, hipStream_t st);
 // does launch_gemv(MB = 1) of this shape take the hand-counted weight stream (gemv2.h)?
 bool gemv2_applies(int dtype, const GemvArgs& a);

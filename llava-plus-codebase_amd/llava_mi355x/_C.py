@@ -128,6 +128,7 @@ _SIGS = {
     "lmx_op_gemm": (c_int32, [c_int32, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p] + [c_int32] * 9 + [c_void_p]),
     "lmx_op_gemm_form": (c_int32, [c_int32] * 5 + [c_int64, c_int32, POINTER(c_int32)]),
     "lmx_op_gemv_form": (c_int32, [c_int32] * 4 + [POINTER(c_int32)]),
+    "lmx_op_gemv_residual_form": (c_int32, [c_int32] * 3 + [POINTER(c_int32)]),
     "lmx_op_gemv": (c_int32, [c_int32, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_float] + [c_int32] * 8 + [c_void_p]),
     "lmx_op_rmsnorm": (c_int32, [c_int32, c_void_p, c_void_p, c_void_p, c_int32, c_int32, c_float, c_void_p]),
     "lmx_op_layernorm": (c_int32, [c_int32, c_void_p, c_void_p, c_void_p, c_void_p, c_int32, c_int32, c_float, c_void_p]),

@@ -62,7 +62,7 @@ def test_a_shared_launch_is_a_group_of_its_own(cuda):
 
 @pytest.mark.parametrize("dt", list(DT))
 @pytest.mark.parametrize("N,H,act", [(8, 2048, 0), (2552, 2048, 0), (2560, 2048, 0), (2560, 3072, 0), (2552, 3072, 0), (2568, 3136, 0), (4088, 4096, 0), (4096, 4096, 0), (6136, 3136, 0),
-                                     (6144, 3136, 0), (6152, 4096, 0), (2496, 2048, 3), (2560, 2048, 3), (2560, 3136, 3), (6144, 4096, 3), (2560, 4160, 0)])
+                                     (6144, 3136, 0), (6152, 4096, 0), (2496, 2048, 3), (2560, 2048, 3), (4096, 2048, 0), (4104, 1544, 0), (5632, 2048, 3), (6144, 2048, 0), (6152, 2048, 0), (2560, 3136, 3), (6144, 4096, 3), (2560, 4160, 0)])
 def test_the_row_and_its_linear(cuda, dt, N, H, act):
     from llava_mi355x import ops
     g = torch.Generator(device="cuda").manual_seed(N + H)

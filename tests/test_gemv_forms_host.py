@@ -1,4 +1,4 @@
-"""How a linear of one row streams its weights (csrc/gemm.hip: gemv2_form), asked of the library on the host.  Cases of one row a wave were timed with two and with four loads of it on the way."""
+"""How a linear of one row streams its weights (csrc/gemm.hip: gemv2_form, gemv2_res_form), asked of the library on the host.  Cases of one row a wave were timed with two and with four loads of it on the way."""
 import ctypes
 
 import pytest
@@ -19,3 +19,14 @@ def test_loads_of_a_row_ahead(N, K, ahead):
 
 def test_two_rows_a_wave():
     assert _form(4096, 4096, norm=1) == (2, 4) and _form(8200, 4096) == (2, 4) and _form(1024, 512, act=3) == (2, 4) and _form(22016, 4096, act=3) == (2, 4)
+
+
+@pytest.mark.parametrize("N,K,act,form", [(2552, 2048, 0, (1, 4, 8)), (2560, 2048, 0, (2, 2, 8)), (4096, 2048, 0, (2, 2, 8)), (4104, 2048, 0, (2, 4, 4)), (6144, 2048, 0, (2, 4, 4)), (6152, 2048, 0, (2, 2, 8)),
+                                          (5120, 1536, 0, (2, 2, 8)), (5120, 2056, 0, (2, 2, 8)), (5632, 2048, 3, (2, 4, 4)), (11264, 2048, 3, (2, 2, 8)), (2496, 2048, 3, (2, 4, 4)),
+                                          (4096, 4096, 0, (1, 4, 8)), (6144, 4096, 0, (2, 2, 8)), (4088, 4096, 0, (2, 4, 4)), (8192, 4104, 0, (2, 4, 4))])
+def test_a_row_formed_in_front(N, K, act, form):
+    """Eight waves share the row where that takes less time than four."""
+    from llava_mi355x import _C
+    f = (ctypes.c_int32 * 3)()
+    _C.check(_C.lib.lmx_op_gemv_residual_form(N, K, act, f))
+    assert tuple(f) == form

@@ -365,6 +365,7 @@ int lmx_op_decode_attn_batch(int32_t dtype, int32_t head_dim, const void* qkv, i
 size_t lmx_op_decode_attn_batch_tab_bytes(int32_t n_seq);
 /* the order in which a decode batch launches sequences of these lengths (1 .. 256 of them), n_heads workgroups each, on the host alone */
 int lmx_op_batch_attn_order(const int32_t* len, int32_t n_seq, int32_t n_heads, uint8_t* order);
+int lmx_op_batch_attn_ordered(int32_t n_seq, int32_t n_heads, int32_t* ordered);      /* 0: that many are launched as they come */
 size_t lmx_op_decode_attn_ws_bytes(int32_t n_rows, int32_t n_heads, int32_t n_split, int32_t head_dim);
 int lmx_op_sample(int32_t dtype, const void* logits_dev, int32_t V, float temperature, float top_p, int32_t top_k, uint64_t seed,
                   const int32_t* offset_dev, const uint32_t* u32_override_host, int64_t* out_tok_dev, uint8_t* keep_out_dev, void* stream);

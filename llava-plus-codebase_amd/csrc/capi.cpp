@@ -644,6 +644,12 @@ int lmx_op_batch_attn_order(const int32_t* len, int32_t n_seq, int32_t n_heads, 
     batch_attn_order(len, n_seq, n_heads, order);
     LMX_API_END
 }
+int lmx_op_batch_attn_ordered(int32_t n_seq, int32_t n_heads, int32_t* ordered) {
+    LMX_API_BEGIN
+    LMX_REQUIRE(ordered && n_seq >= 1 && n_seq <= 256 && n_heads >= 1, "batch_attn_ordered: 1..256 sequences");
+    *ordered = batch_attn_ordered(n_seq, n_heads);
+    LMX_API_END
+}
 size_t lmx_op_decode_attn_batch_tab_bytes(int32_t n_seq) { return sizeof(DecodeFusedSeq) * (size_t)(n_seq > 0 ? n_seq : 0); }
 size_t lmx_op_decode_attn_ws_bytes(int32_t n_rows, int32_t n_heads, int32_t n_split, int32_t head_dim) {
     return decode_attn_ws_floats(n_rows, n_heads, n_split, head_dim) * sizeof(float);

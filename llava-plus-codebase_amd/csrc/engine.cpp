@@ -1078,8 +1078,11 @@ void Model::decode_batch(Batch* b, Seq* const* seqs, int n, const int64_t* token
     if (!stk || !stk->ids_in()) { LMX_PROF("decode_batch.embed"); launch_gather_tokens_batch(dt, b->d_state_tab, n, embed, b->h, H, V, st); }
     uint8_t order[256];
     int lens[256];
-    for (int i = 0; i < n; ++i) lens[i] = seqs[i]->len;                  // (all of them grow by one a step)
-    batch_attn_order(lens, n, nh_l, order);
+    const bool ordered = !stk && batch_attn_ordered(n, nh_l);
+    if (ordered) {
+        for (int i = 0; i < n; ++i) lens[i] = seqs[i]->len;              // (all of them grow by one a step)
+        batch_attn_order(lens, n, nh_l, order);
+    }
     for (int step = 0; step < n_steps; ++step) {
         if (stk) {
             stack_decode_batch_step(b, seqs, n, d_ids + (size_t)step * b->cap, st);
@@ -1096,7 +1099,7 @@ void Model::decode_batch(Batch* b, Seq* const* seqs, int n, const int64_t* token
                 for (int i = 0; i < n; ++i) max_len = std::max(max_len, seqs[i]->len);
                 // live 128-key chunks of the longest member (the host mirrors every position); shorter members' surplus workgroups only take their ticket
                 DecodeFusedArgs a{b->qkv, nullptr, nullptr, rope, nullptr, nh_l, nkv_l, kv_pitch, max_len / 128 + 1, scale, nullptr, nullptr, b->attn};
-                a.tab = b->d_attn_tab + (size_t)l * b->cap; a.order = order; a.n_seq = n; a.qkv_stride = qkv_n; a.o_stride = nh_l * D;
+                a.tab = b->d_attn_tab + (size_t)l * b->cap; a.order = ordered ? order : nullptr; a.n_seq = n; a.qkv_stride = qkv_n; a.o_stride = nh_l * D;
                 launch_decode_fused(dt, D, a, st);
             }
             linear(b->attn, nullptr, nullptr, GemmArgs{b->attn, w.wo, b->h, nullptr, lead ? b->h : nullptr, n, H, nh_l * D, nh_l * D, nh_l * D, H, H, kActNone}, w.sw_o);

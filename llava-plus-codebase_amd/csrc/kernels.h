@@ -190,6 +190,7 @@ struct DecodeFusedArgs {
 };
 void launch_decode_fused(int dtype, int D, const DecodeFusedArgs& a, hipStream_t st);
 void batch_attn_order(const int* len, int n_seq, int n_heads, uint8_t* order);      // DecodeFusedArgs::order for sequences of these lengths (256 at most)
+bool batch_attn_ordered(int n_seq, int n_heads);        // is a launch of them in that order, or as they come
 size_t decode_fused_ws_floats(int n_heads, int n_split, int D);
 size_t decode_attn_ws_floats(int n_rows, int n_heads, int n_split, int D);
 

@@ -148,6 +148,7 @@ _SIGS = {
     "lmx_op_decode_attn_batch": (c_int32, [c_int32, c_int32, c_void_p, c_int32, POINTER(c_void_p), POINTER(c_void_p), POINTER(c_void_p), POINTER(c_void_p),
                                            POINTER(c_void_p), c_int32, c_void_p, c_int32, c_int32, c_int32, c_int32, c_float, c_void_p, c_void_p, c_int32, c_void_p]),
     "lmx_op_batch_attn_order": (c_int32, [POINTER(c_int32), c_int32, c_int32, POINTER(c_uint8)]),
+    "lmx_op_batch_attn_ordered": (c_int32, [c_int32, c_int32, POINTER(c_int32)]),
     "lmx_op_decode_attn_batch_tab_bytes": (c_size_t, [c_int32]),
     "lmx_op_decode_attn_ws_bytes": (c_size_t, [c_int32] * 4),
     "lmx_op_sample": (c_int32, [c_int32, c_void_p, c_int32, c_float, c_float, c_int32, ctypes.c_uint64, c_void_p, POINTER(ctypes.c_uint32), c_void_p, c_void_p, c_void_p]),

@@ -32,3 +32,13 @@ def test_equal_lengths_stay_in_place_and_bad_arguments_raise():
     for n, heads in [(0, 32), (257, 32), (4, 0)]:
         with pytest.raises(_C.LmxError):
             _C.check(_C.lib.lmx_op_batch_attn_order((ctypes.c_int32 * 257)(), n, heads, (ctypes.c_uint8 * 257)()))
+
+
+@pytest.mark.parametrize("n,heads,want", [(12, 40, True), (13, 40, False), (14, 40, False), (15, 40, True), (25, 20, True), (26, 20, False), (27, 20, True), (16, 32, True), (17, 32, True), (16, 31, True),
+                                          (17, 31, False), (18, 31, False), (19, 31, True), (1, 600, False), (3, 300, True), (256, 1, True), (256, 256, True)])
+def test_no_long_one_last(n, heads, want):
+    """The reversed ones end within the first 512 workgroups, or others follow them."""
+    from llava_mi355x import _C
+    f = ctypes.c_int32()
+    _C.check(_C.lib.lmx_op_batch_attn_ordered(n, heads, f))
+    assert bool(f.value) == want

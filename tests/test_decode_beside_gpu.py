@@ -60,6 +60,28 @@ def test_a_shared_launch_is_a_group_of_its_own(cuda):
     assert launches() == [18, 0, 12, 12, 0, 24]
 
 
+def _joined(m, steps):
+    m.profile(True)
+    out = _steps(m, [5, 9, 2, 7, 1], steps)
+    prof = m.profile_read()
+    m.profile(False)
+    return out, tuple(prof[k][1] if k in prof else 0 for k in ("decode.delta_gate_up", "decode.moe.gate_up_o"))
+
+
+@pytest.mark.parametrize("dt", list(DT))
+@pytest.mark.parametrize("width,heads,ff", [(1088, 17, 200), (2048, 32, 200), (2112, 33, 1500), (2112, 33, 9000), (4160, 4, 3200)])
+def test_rows_of_several_loads(cuda, dt, width, heads, ff):
+    """Rows of the gate | up shorter than, as long as and longer than what a wave has on the way, the last load in part; output projections of 3, 4 and 5 loads of two beside experts."""
+    layers = [delta(2, 2, 64, 64, 4, dense(ff))] + ([delta(heads, heads, 64, 64, 4, moe(72, 6, 2))] if width <= 3072 else [])
+    cfg = config(layers, width, 211)
+    m = build_config(cfg, steady_routing(cfg, O.make_weights(cfg, 3, (18, 70))), DT[dt], 64)
+    a, n = _joined(m, 4)
+    assert n == (4, 4 if width <= 3072 else 0)
+    m.set_option("stack_fuse", 0)
+    b, n = _joined(m, 4)
+    assert n == (0, 0) and torch.isfinite(a.float()).all() and rel(a, b.double().cpu()) < TOL[dt] / 8
+
+
 @pytest.mark.parametrize("dt", list(DT))
 @pytest.mark.parametrize("N,H,act", [(8, 2048, 0), (2552, 2048, 0), (2560, 2048, 0), (2560, 3072, 0), (2552, 3072, 0), (2568, 3136, 0), (4088, 4096, 0), (4096, 4096, 0), (6136, 3136, 0),
                                      (6144, 3136, 0), (6152, 4096, 0), (2496, 2048, 3), (2560, 2048, 3), (4096, 2048, 0), (4104, 1544, 0), (5632, 2048, 3), (6144, 2048, 0), (6152, 2048, 0), (2560, 3136, 3), (6144, 4096, 3), (2560, 4160, 0)])

@@ -186,3 +186,8 @@ def test_sixteen_requests_decode_together_vs_oracle(cuda, n_req):
     bt.close()
     for c in caches:
         c.close()
+
+
+def test_more_sequences_than_one_launch_takes(cuda):
+    """256 sequences and the rest in launches of their own (csrc/attention_batch.h): every row against float64, at positions of both launches."""
+    _check(cuda, "bf16", 259, 2, 1, "nonfinite", seed=5)

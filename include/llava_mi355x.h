@@ -291,11 +291,14 @@ int lmx_seq_read_tokens(lmx_seq* s, int64_t* host_out, int32_t max_n, int32_t* n
 int lmx_profile_enable(lmx_model* m, int32_t on);
 int lmx_profile_read(lmx_model* m, char* names_buf, int32_t names_cap, double* ms, int64_t* counts, int32_t max_n, int32_t* n_out);
 /* Options of a live model (defaults come from the environment at lmx_create: LMX_FUSE_ROPE, LMX_FUSE_SLICES, LMX_VIS_PACK, LMX_DECODE_SPLITQ; all default 1).  Every one selects
- * between two launch forms with bit-identical results — the switch exists for A/B timing and for the tests that prove the identity:
+ * between two launch forms, of the first four with bit-identical results — the switch exists for A/B timing and for the tests that compare both:
  *   "fuse_rope"     RoPE + KV-cache append in the prefill's q|k|v GEMM epilogue (HF5:models/llama/modeling_llama.py:130-160,243-281) vs. a rope_kv launch
- *   "fuse_slices"   the K slices of a prompt's q|k|v, o and down linears added by the launch that reads their rows (rope_kv, RMSNorm) vs. by a launch of their own
+ *   "fuse_slices"   the K slices of a prompt's q|k|v, o and down linears added by the launch that reads their rows (rope_kv, RMSNorm) vs. by a launch of their own (prompts read one by one;
+ *                   o and down without tensor parallelism)
  *   "vis_pack"      CLIP K / V^T pack in the tower's q|k|v GEMM epilogue (HF5:models/clip/modeling_clip.py:295-340) vs. a pack launch
  *   "decode_splitq" decode step of 16-bit models as q launch + (k|v projection with the attention workgroups) launch vs. q|k|v launch + attention launch
+ *   "stack_fuse"    (default 1, no environment variable; equal up to rounding) a layer-stack decode step's residual addition and norms inside the linear that reads them, a parallel layer's
+ *                   router in its mixer's launch, and its gate|up and output projection beside the delta step and the experts vs. launches of their own
  * Unknown keys are an error.  Not to be flipped while requests are in flight on other threads. */
 int lmx_model_set_option(lmx_model* m, const char* key, int32_t value);
 
@@ -303,7 +306,7 @@ int lmx_model_set_option(lmx_model* m, const char* key, int32_t value);
 int lmx_op_gemm(int32_t dtype, const void* x, const void* w, void* c, const void* bias, const void* residual,
                 int32_t M, int32_t N, int32_t K, int32_t ldx, int32_t ldw, int32_t ldc, int32_t ldr, int32_t act, int32_t variant, void* stream);
 /* variant LMX_GEMM_SCRATCH: the choice a prefill makes, which brings scratch for K slices (this entry's own 64 MiB: one stream at a time); variant 0 chooses without.
- * Products of more than 256 rows and more than 640 tiles of 64 x 64 (160 .. 256 where K is long) that it makes in the least time go to the four-wave kernel in either (variant 100 mb + 10 nb + slices: its tiles of 32 mb x 32 nb by number).
+ * Products of more than 256 rows and more than 640 tiles of 64 x 64 (past 384 rows 160 with a K from 8192 on, 256 with one from 5120 on and 1024 weights) that it makes in the least time go to the four-wave kernel in either (variant 100 mb + 10 nb + slices: its tiles of 32 mb x 32 nb by number).
  * lmx_op_gemm_form: what is launched for contiguous 16-byte aligned operands and `scratch_bytes` of scratch, on the host alone.  form[4]: batch = 0: {2, mb, nb, K slices} of the
  * four-wave kernel, {1, row tiles, weight rows of a workgroup, K slices} of the kernel for few row tiles, {0, 0, 0, K slices} of the others; batch = 1 (linears of a decode
  * batch, M <= 32): {0, 16-row weight tiles of a workgroup, 16-row token tiles, K slices}. */

@@ -125,11 +125,14 @@ size_t gemm4w_slab_bytes(int M, int N, const TileForm& f) {
     return f.slices * std::max(tile, whole) * sizeof(float);
 }
 
-// Which products: more than 256 rows (below, the row tiles of gemm_rows.hip read every weight once) and more than 640 tiles of 64 x 64, past 384 rows with a K from 5120 on more than 256
-// and from 8192 on more than 160, and of these those that no other form makes in less time (linear_form).  Long K under the line of 640: 144 products of 385 .. 3000 rows x 768 .. 5504
-// weights, time of the form before / here 1.24 in the mean, 0.975 .. 1.6 (957 x 1280 x 11008 69.8 / 46.1 us, 800 x 1536 x 5632 32.2 / 25.2); up to 384 rows, where the row tiles come in
-// slices, 1.07 (351 x 2816 x 11008 42.4 / 43.8); K of 4096 0.83 .. 1.13, of 1024 .. 2560 0.64 .. 1.13; 2622 x 768 x 5120 31.3 / 35.0.  Below the line otherwise, us theirs / here, by shape:  800 x 1024 x 2048 10.3 / 14.1   2000 x 512 x 2048 12.9 / 14.8   257 x 6208 x 2048 15.1 / 17.1
-//   330 x 4544 x 2304 15.9 / 17.3   577 x 4096 x 1024 13.3 / 13.9,  but  700 x 3072 x 1024 11.4 / 9.8   2308 x 1024 x 4096 30.5 / 27.2   500 x 4096 x 11008 74.3 / 63.3.
+// Which products: more than 256 rows (below, the row tiles of gemm_rows.hip read every weight once) and more than 640 tiles of 64 x 64; past 384 rows, with a K from 8192 on, more than 160
+// and, with a K from 5120 on and 1024 weights or more, more than 256; of these those that no other form makes in less time (linear_form).  Long K under the line of 640: 144 products of
+// 385 .. 3000 rows x 768 .. 5504 weights, time of the form before / here 1.24 in the mean, 0.975 .. 1.6 (957 x 1280 x 11008 69.8 / 46.1 us, 800 x 1536 x 5632 32.2 / 25.2), 90 with SiLU, GELU
+// or quick GELU 1.33, 0.98 .. 2.2; up to 384 rows, where the row tiles come in slices, 1.07 (351 x 2816 x 11008 42.4 / 43.8).  Under 1024 weights and a K of 8192 the times err most, both
+// ways: 2878 x 832 x 5120 with a residual 38.6 / 44.1, 2622 x 768 x 5120 31.3 / 35.0, 3068 x 512 x 5824 30.1 / 33.5, but 2638 x 960 x 6144 49.6 / 40.2, 1641 x 768 x 7680 55.4 / 35.4.
+// K of 4096 0.83 .. 1.13, of 1024 .. 2560 0.64 .. 1.13.  Below the line otherwise, us theirs / here, by shape:  800 x 1024 x 2048 10.3 / 14.1   2000 x 512 x 2048 12.9 / 14.8
+//   257 x 6208 x 2048 15.1 / 17.1   330 x 4544 x 2304 15.9 / 17.3   577 x 4096 x 1024 13.3 / 13.9,  but  700 x 3072 x 1024 11.4 / 9.8   2308 x 1024 x 4096 30.5 / 27.2
+//   500 x 4096 x 11008 74.3 / 63.3.
 TileForm gemm4w_form(int dtype, const GemmArgs& a, float* us) {
     const TileForm none{0, 0, 1};
     if ((dtype != kBF16 && dtype != kF16) || a.c_f32 || a.K % 64 != 0 || a.N % 8 != 0 || (act_gated(a.act) && a.N % 64 != 0) || (a.pk_kc && a.pk_D % 8 != 0)) return none;

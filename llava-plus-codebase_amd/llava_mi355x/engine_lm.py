@@ -153,7 +153,7 @@ class EngineCausalLM:
             self.finalize_weights()
 
     def set_option(self, key: str, value: int) -> None:
-        """Flip one of the engine's launch-form options ("fuse_rope", "fuse_slices", "vis_pack", "decode_splitq": bit-identical forms; include/llava_mi355x.h)."""
+        """Flip one of the engine's launch-form options ("fuse_rope", "fuse_slices", "vis_pack", "decode_splitq": bit-identical forms; "stack_fuse": equal up to rounding; include/llava_mi355x.h)."""
         check(lib.lmx_model_set_option(self._h, key.encode(), int(value)), "lmx_model_set_option")
 
     def profile(self, enable: bool) -> None:

@@ -1,5 +1,5 @@
-"""SiLU and quick GELU over the whole range of their exponential (csrc/common.h: over_one_plus_exp): results down to 2^-120, where the denominator is 2^126 and more, against
-float64.  The argument reaches the epilogue exactly (one weight of 1 a row, zeros).  Tolerance: the result's rounding (half a unit in the last place: 2^-9, 2^-25), and the exponential's,
+"""SiLU and quick GELU over the whole range of their exponential (csrc/common.h: act_silu, act_quick_gelu): results down to 2^-120, where the denominator is 2^126 and more, against
+float64.  The argument reaches the epilogue exactly (one weight of 1 a row, zeros).  Tolerance: the result's rounding (half a unit in the last place: 2^-8, 2^-24), and the exponential's,
 whose argument is rounded in 32 bits: (|cx| + 4) 2^-23.  Past the largest 32-bit exponential the result is 0, at most 2^-120 away."""
 import pytest
 import torch

@@ -400,7 +400,7 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(GemmArgs a) {
                 acc[i][j] = v;
                 continue;
             }
-            v = apply_act(v, act);
+            v = apply_act<float>(v, act);
             if (R) v += R[(size_t)m * a.ldr + n];
             if (a.c_f32) v = soft_cap(v, a.cap);
             C[(size_t)m * a.ldc + n] = v;
@@ -425,7 +425,7 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(GemmArgs a) {
                     const int nl = tx * 4 + j;          // 0..31 gate column inside this 64 group
                     if (n0 + nl >= a.N) continue;
                     const float g = Ts[ty * 4 + i][nl], u = Ts[ty * 4 + i][nl + 32];
-                    C[(size_t)m * a.ldc + n0 / 2 + nl] = gate_mul(a.act, g, u);
+                    C[(size_t)m * a.ldc + n0 / 2 + nl] = gate_mul<float>(a.act, g, u);
                 }
             }
         }
@@ -604,7 +604,7 @@ __global__ __launch_bounds__(256) void gemv_kernel(GemvArgs a) {
             for (int mb = 0; mb < MB; ++mb) {
                 float g = acc[r][mb], u = acc[r + 1][mb];
                 if (bias) { g += to_f32(bias[rows[r]]); u += to_f32(bias[rows[r + 1]]); }
-                C[(size_t)mb * a.ldc + j] = from_f32<T>(gate_mul(a.act, g, u));
+                C[(size_t)mb * a.ldc + j] = from_f32<T>(gate_mul<T>(a.act, g, u));
             }
         }
         return;
@@ -617,7 +617,7 @@ __global__ __launch_bounds__(256) void gemv_kernel(GemvArgs a) {
         for (int mb = 0; mb < MB; ++mb) {
             float v = acc[r][mb];
             if (bias) v += to_f32(bias[n]);
-            v = apply_act(v, a.act);
+            v = apply_act<T>(v, a.act);
             if (Rr) v += to_f32(Rr[(size_t)mb * a.ldr + n]);
             if (a.c_f32) reinterpret_cast<float*>(a.C)[(size_t)mb * a.ldc + n] = soft_cap(v, a.cap);
             else C[(size_t)mb * a.ldc + n] = from_f32<T>(v);

@@ -24,8 +24,8 @@ template <> struct Mfma32x32x16<f16_t> {
 // ---------------------------------------------------------------------------------------------
 // shared epilogue math
 // ---------------------------------------------------------------------------------------------
-__device__ __forceinline__ float apply_act(float v, int act) {
-    if (act == kActQuickGelu) return act_quick_gelu(v);
+template <typename T = bf16_t> __device__ __forceinline__ float apply_act(float v, int act) {
+    if (act == kActQuickGelu) return act_quick_gelu<T>(v);
     if (act == kActGeluErf) return act_gelu_erf(v);
     return v;
 }

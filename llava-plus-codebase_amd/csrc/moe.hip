@@ -288,7 +288,7 @@ __device__ __forceinline__ void group_gemv_body(const GroupGemvArgs& a, int lpr,
         }
         if (lpr == 64) { s0 = group_sum<64>(s0); if (GATED) s1 = group_sum<64>(s1); }
         else for (int d = lpr >> 1; d > 0; d >>= 1) { s0 += __shfl_xor(s0, d, 64); if (GATED) s1 += __shfl_xor(s1, d, 64); }
-        if (sub == 0 && o < o1) C[o] = from_f32<T>(GATED ? gate_mul(a.act, s0, s1) : s0);
+        if (sub == 0 && o < o1) C[o] = from_f32<T>(GATED ? gate_mul<T>(a.act, s0, s1) : s0);
     }
 }
 template <typename T, bool GATED, int U>

@@ -1,8 +1,8 @@
 /* llava_mi355x.h — C ABI of libllava_mi355x.so (MI355X / gfx950 native LLaVA forward path)
  *
  * The reference (LLaVA-VL/LLaVA-Plus-Codebase) has no FFI: its seam is a Python class API whose arithmetic lives in
- * third-party torch/transformers code.  This header is the boundary a maintainer binds (ctypes stub in
- * INTEGRATION.md) to run that API on hand-written HIP kernels.  Each entry point cites the reference interface it
+ * third-party torch/transformers code.  This header is the boundary a maintainer binds (by ctypes,
+ * say) to run that API on hand-written HIP kernels.  Each entry point cites the reference interface it
  * replaces (paths relative to the reference repo; HF5: = transformers 5.15 sources the reference calls into).
  *
  * Conventions
@@ -204,7 +204,7 @@ int lmx_gather_embeds(lmx_model* m, const int32_t* src_dev, int32_t rows, const 
 
 /* ---- decoder ---------------------------------------------------------------------------------------------------
  * A sequence owns its KV cache (K [layer][kv_head][pos][d], Vᵀ [layer][kv_head][d][pos]) and the device-resident
- * decode state; replaces the past_key_values tuple of the reference (llava_arch.py:105; a14 in SURVEY §8). */
+ * decode state; replaces the past_key_values tuple of the reference (llava_arch.py:105). */
 int lmx_seq_create(lmx_model* m, lmx_seq** out);
 int lmx_seq_destroy(lmx_seq* s);                     /* before or after lmx_destroy of its model; nothing else works on a sequence whose model is gone */
 int lmx_seq_reset(lmx_seq* s);                       /* length := 0 (cache contents stay; nothing reads behind the length) */
@@ -260,7 +260,7 @@ int lmx_seq_set_stop(lmx_seq* s, const int64_t* eos_ids, int32_t n_eos, const in
 /* out = 1 once the sequence's stop rule has fired (synchronises `stream`) */
 int lmx_seq_stopped(lmx_seq* s, int32_t* out, void* stream);
 
-/* ---- decode batch: continuous batching (SURVEY §8f-1) --------------------------------------------------------------
+/* ---- decode batch: continuous batching --------------------------------------------------------------
  * new in this build: the reference serves up to --limit-model-concurrency requests as independent generate() threads with no
  * batching (llava/serve/model_worker.py:174-185, :264); here the decode steps of those requests share ONE pass over the
  * weights.  A batch owns the workspaces for up to `capacity` sequences; which sequences take part is decided per call, so
@@ -414,7 +414,7 @@ int lmx_op_group_gemm(int32_t dtype, const void* x, const void* w, void* c, cons
 int lmx_op_argmax(int32_t dtype, const void* logits, int32_t V, int64_t* out_tok_dev, void* stream);
 int lmx_op_im2col(int32_t dtype, const void* pixels, void* out, int32_t N, int32_t S, int32_t patch, int32_t kpad, void* stream);
 
-/* ---- training-step slices (csrc/train.hip; SURVEY 8 f-3): parity-first kernels for the finetuning step of llava/train/train.py:805-1000.
+/* ---- training-step slices (csrc/train.hip): parity-first kernels for the finetuning step of llava/train/train.py:805-1000.
  * lmx_op_ce_loss: LlamaForCausalLM's shifted cross-entropy with ignore_index (labels from llava_arch.py:181,200; IGNORE_INDEX = -100):
  *   logits [B*T][ld], labels [B][T] int64 (position t is scored against labels[t + 1]); out_loss_count[0] = mean loss, [1] = counted
  *   positions; scratch: B*(T-1) floats each; dlogits (optional, [B*T][ldd]) = grad * d(loss)/d(logits).
@@ -460,7 +460,7 @@ int lmx_op_attn_bwd_lse(int32_t dtype, int32_t head_dim, const void* q, const vo
                         int32_t lse_stride, void* dq, void* dk, void* dv, int32_t T, int32_t heads, int32_t kv_heads, int32_t ldq, int32_t ldk, int32_t ldo,
                         int32_t ldout, float scale, void* stream);
 
-/* ---- one optimisation step (SURVEY §8 f-3, BASELINE config 5; composed by llava_mi355x/train.py) ------------------------------------------
+/* ---- one optimisation step (composed by llava_mi355x/train.py) ------------------------------------------
  * Replaces, for the trainable part of the model (LLM + mm_projector; the CLIP tower is frozen, clip_encoder.py:25), what the HF Trainer +
  * DeepSpeed run per step under llava/train/train.py:805-1000 with scripts/zero2.json:
  *   lmx_op_elementwise   op 0: silu(gate) * up with HF's rounding points (LlamaMLP, HF5:models/llama/modeling_llama.py:163-176);

@@ -10,7 +10,7 @@
 //   ring.  Both products keep the query index on the MFMA *column* (lane&31): Sᵀ = K·Qᵀ and Oᵀ = Vᵀ·Pᵀ, so the running max /
 //   sum / rescale are per-lane scalars and P goes from the score accumulators straight into the next MFMA's B operand
 //   with no cross-lane traffic (the key order inside each 16-key MFMA step is permuted identically for P and Vᵀ).
-//   (The 4-wave first-generation kernel, 36.8 vs 27.5 us per layer, was removed in round 5.)
+//   (A 4-wave form took 36.8 us a layer where this takes 27.5.)
 // decode_attn_kernel    (any dtype, VALU): one workgroup per (row, head, key-split); used for single-token decode
 //   (HBM-bound KV streaming) and as the fp32 verification-mode attention for whole prompts.
 #include <algorithm>
@@ -78,7 +78,7 @@ __global__ __launch_bounds__(512, D == 64 && !WIN ? 4 : 2) void flash_prefill2_k
         for (int s = 0; s < KSTEPS; ++s) qf[s] = *reinterpret_cast<const uint4*>(qp + s * 16);
         // These are the only vector-memory loads the COMPILER knows of (the tile DMAs below are inline asm).  Left pending into the key loop, its wait-count
         // pass guards their first use there with s_waitcnt vmcnt(KSTEPS - 1) ... vmcnt(0) — counts that, on the hardware's single in-order counter, also cover
-        // the DMAs of the NEXT round issued just before: every round waited for its own prefetch inside the S = K Q chain (seen in the ISA, EXPERIMENTS r5-I).
+        // the DMAs of the NEXT round issued just before: every round waited for its own prefetch inside the S = K Q chain (seen in the ISA).
         // Waiting here, with an instruction the pass sees, leaves the loop with the one vmcnt wait per round that is meant.  (Time: unchanged — the tiles come
         // from L2 faster than a round computes — but the ring now works as written.)
         __builtin_amdgcn_s_waitcnt(0x0F70);          // vmcnt(0); expcnt / lgkmcnt untouched

@@ -33,7 +33,7 @@ template <int D> __device__ __forceinline__ int k_lds_off(int row, int chunk) {
 __device__ __forceinline__ int vt_lds_chunk(int row, int chunk) { return row * 128 + (((chunk ^ (row >> 1)) & 7) << 4); }
 // Key order inside a 32-key block.  The 32x32 accumulator of Sᵀ = K Qᵀ holds tile row (r & 3) + 8 (r >> 2) + 4 hi in register r of lane half hi, and the
 // P·V step (kb, s2) takes registers 8 s2 .. + 7 as its 8 k-values: with K fed in natural order those are keys {4 hi .. + 3} and {8 + 4 hi .. + 3} (+ 16 s2),
-// i.e. the Vᵀ operand needs TWO 8-byte LDS reads, 2-way bank-conflicted (1.46 M conflict cycles per launch in round 2's PMC).  Feeding K row pi(l31) =
+// i.e. the Vᵀ operand needs TWO 8-byte LDS reads, 2-way bank-conflicted (1.46 M conflict cycles per launch in the counters).  Feeding K row pi(l31) =
 // l31 with bits 2 and 3 swapped as tile row l31 makes them the 8 CONSECUTIVE keys 16 s2 + 8 hi .. + 7: one conflict-free 16-byte read.  (pi maps each
 // 16-lane service group of ds_read_b128 onto itself, so the K fragment reads stay conflict-free.)
 __device__ __forceinline__ int fa_key_perm(int l31) { return (l31 & 0x13) | ((l31 & 4) << 1) | ((l31 & 8) >> 1); }

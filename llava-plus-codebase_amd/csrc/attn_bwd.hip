@@ -16,7 +16,7 @@
 //       (row-major), lse / delta of the tile's 64 rows.   S = Q K^T, dP = dO V^T (rows = queries, in registers),  P, dS with the row's lse / delta,
 //       dV^T += (dO tile)^T . P,  dK^T += (Q tile)^T . dS.
 //
-// Round 6: NO transposed copies.  Through round 5 K^T, Q^T and dO^T were made by three launch_transpose calls per sample and staged as tiles of their own beside
+// NO transposed copies.  Before, K^T, Q^T and dO^T were made by three launch_transpose calls per sample and staged as tiles of their own beside
 // the row-major ones (3 / 4 tiles per ring slot: 144 / 132 KiB of LDS, ONE 4-wave workgroup per CU, one wave per SIMD — every exp / pack / LDS phase of a wave
 // left its matrix pipe idle: 0.16 of peak).  The second products' A operands (rows = d, contraction = the tile's 64 rows) now come out of the ROW-MAJOR tile the
 // first products already use, through ds_read_b64_tr_b16 (tools/probes/tr_b16_probe.hip: 16 lanes read a [4 rows][16 columns] block, lane i receives column i).

@@ -6,10 +6,10 @@
 //
 //   decode_attn_step_kernel   grid = heads x live chunks.  q | k_new | v_new come from the q|k|v row a preceding GEMV launch wrote.
 //
-//   decode_kv_attn_kernel     (round 5, "split-q" decode step)  The step's q|k|v projection is cut in two: a first launch computes q alone (4096 of the 12288
+//   decode_kv_attn_kernel     ("split-q" decode step)  The step's q|k|v projection is cut in two: a first launch computes q alone (4096 of the 12288
 //       rows at 7B); THIS launch holds the attention workgroups (lowest block ids: dispatched first) AND the workgroups of the k|v projection (gemv2_body).
-//       Why: as its own launch the attention is a latency chain — 19 MB of K / V^T land after ~5 us, partial at ~7, merged row stored at ~13 (EXPERIMENTS
-//       r3-D) — during which the HBM idles, and every form of "make the chain shorter" was measured equal (r3-D, r4-F, r4-G, r5-A).  Here the chain runs UNDER
+//       Why: as its own launch the attention is a latency chain — 19 MB of K / V^T land after ~5 us, partial at ~7, merged row stored at ~13
+//       — during which the HBM idles, and every form of "make the chain shorter" was measured equal.  Here the chain runs UNDER
 //       the k|v weight stream (67 MB, ~13 us): the cached keys need only q, which is ready at launch; the newest key / value are the one thing that depends on
 //       the k|v rows, and they reach the head's last chunk (the workgroup that owns position `pos`, which is also the one that appends to the caches) as
 //       tagged 8-byte granules published by the GEMV workgroups of the same launch.  That workgroup takes its ticket last — its partial waits for the
@@ -18,8 +18,8 @@
 //       Arithmetic is dec_attn_chunk's in both launches and the GEMV rows are gemv2_body's: ids and logits are bit-identical to the three-launch form
 //       (tests/test_decode_splitq_gpu.py).
 //
-// History: this file replaces decode_flow.hip (one launch per token without grid barriers, r3-B; attention + o_proj in one launch, r3-C; one workgroup per
-// head, r4-F; tagged-granule merge, r3-D) — built, bit-identical, measured slower or equal, removed in round 5; profiles/EXPERIMENTS.md names the commits.
+// Built, bit-identical, measured slower or equal and gone: one launch per token without grid barriers; attention + o_proj in one launch; one workgroup per head; a merge over tagged
+// granules alone.
 #include "attention_decode.h"
 #include "common.h"
 #include "gemv2.h"

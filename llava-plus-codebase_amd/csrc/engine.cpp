@@ -1,7 +1,7 @@
 // Engine: weights in kernel-optimal layouts, per-sequence KV caches (K rows + Vᵀ columns), prefill / decode
 // orchestration, device-resident decode loop, RCCL all-reduce for the tensor-parallel decoder.
 //
-// Reference call stacks this replaces (SURVEY §3): llava/model/llava_arch.py:94-97 (encode_images),
+// Reference call stacks this replaces: llava/model/llava_arch.py:94-97 (encode_images),
 // llava/model/language_model/llava_llama.py:88-99 -> HF5:models/llama/modeling_llama.py:367-494 (decoder forward),
 // HF5:models/clip/modeling_clip.py:594-657 (CLIP vision transformer).
 #include "engine.h"
@@ -60,7 +60,7 @@ Model::Model(const lmx_config& c) : cfg(c) {
     // k-slab granularity (7B at TP=8: 1376 -> 1408).  Padded gate|up rows are zero => silu(0)*0 = 0 => no contribution.
     I_sh = c.intermediate_size / c.tp_world; I_l = round_up(I_sh, 64);
     qkv_n = (nh_l + 2 * nkv_l) * D;
-    // vocabulary-parallel lm_head (SURVEY §8e): each rank streams V / world rows per token instead of all of them (262 MB at 7B: 8 % of
+    // vocabulary-parallel lm_head: each rank streams V / world rows per token instead of all of them (262 MB at 7B: 8 % of
     // a TP=1 token, 40 % of a TP=8 token if replicated); replicated when the vocabulary does not split into 8-row-aligned shards
     if (c.tp_world > 1 && V % (8 * c.tp_world) == 0) { V_l = V / c.tp_world; v_off = c.tp_rank * V_l; } else { V_l = V; v_off = 0; }
     s_max = round_up(c.max_position > 0 ? c.max_position : 2048, 128);   // decode attention works in 128-key chunks
@@ -640,7 +640,7 @@ void Model::prefill(Seq* s, const void* embeds, int T, int chunk, void* logits, 
             void* vt = s->vt.as<char>() + (size_t)l * s->layer_stride;
             void *hr = rows(h, r0, H), *xr = rows(x, r0, H), *qr = rows(qkv, r0, qkv_n), *ar = rows(attn, r0, (size_t)nh_l * D);
             if (!normed) { LMX_PROF("prefill.rmsnorm"); launch_rmsnorm(dt, hr, w.ln1, xr, n, H, H, H, cfg.rms_eps, st); }
-            // RoPE + KV-cache append ride in the q|k|v GEMM's epilogue where that launch is the un-split ping-pong kernel over head-aligned tiles
+            // RoPE + KV-cache append ride in the q|k|v GEMM's epilogue where that launch is un-split four-wave tiles (gemm4w.h, qkv_rope_epilogue4)
             const bool qf = gv == 0 && opt_fuse_rope && gemm_fuses_qkv(dt, n, H, D, nh_l, nkv_l, pos0 + r0, kv_pitch, false);
             int slices = 0;
             {
@@ -751,7 +751,7 @@ void Model::prefill(Seq* s, const void* embeds, int T, int chunk, void* logits, 
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// packed prefill of several sequences (serving: BASELINE configs 3 / 4 prefill many requests at once)
+// packed prefill of several sequences (serving: many requests at once)
 // ---------------------------------------------------------------------------------------------------------------
 // The rows of all sequences are walked as ONE packed row block in pieces of `block_rows`: every linear of a piece is a single GEMM over the piece's
 // rows (a 512-row chunk of one request reaches ~0.19 of the MFMA peak, 4096 packed rows ~0.4), RoPE / KV append / causal attention run per
@@ -940,7 +940,7 @@ void Model::decode(Seq* s, int64_t token, int n_steps, void* logits, bool greedy
     s->last_stream = st; s->used = true;
     if (token >= 0) launch_set_state(s->d_len, -1, s->d_tok, token, 1, s->d_nout, -1, st);
     // Plain stream launches: the ~160 kernels of a step average >20 us each against ~3.5 us of host launch cost, so the
-    // host runs far ahead of the GPU; a captured hipGraph measured no faster (3.57 vs 3.56 ms/token, profiles/EXPERIMENTS.md)
+    // host runs far ahead of the GPU; a captured hipGraph measured no faster (3.57 vs 3.56 ms/token)
     // and stream capture is not safe next to other threads using the legacy stream (model_worker runs 5 request threads).
     if (!stk || !stk->ids_in()) { LMX_PROF("decode.embed"); launch_gather_token(cfg.dtype, s->d_tok, embed, s->d_h, H, V, st); }      // (otherwise every step begins with its own row)
     for (int i = 0; i < n_steps; ++i) {
@@ -951,7 +951,7 @@ void Model::decode(Seq* s, int64_t token, int n_steps, void* logits, bool greedy
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// decode batch (continuous batching; SURVEY §8f-1): several sequences, each with its own KV cache and position, advance
+// decode batch (continuous batching): several sequences, each with its own KV cache and position, advance
 // one token per step and share ONE pass over the weights.
 // ---------------------------------------------------------------------------------------------------------------
 // Decode-batch weights: the skinny MFMA kernel loads its A fragments per lane, so from the [N][K] layout every 16-lane group of a load

@@ -70,9 +70,9 @@ __device__ __forceinline__ v4i_t make_rsrc(const void* p, uint32_t bytes) {
 }  // namespace
 
 // SPLIT: K slices per tile (1, 2 or 3).  A K-sliced workgroup stores its fp32 partial tile and exits; the kernel boundary publishes the slabs and
-// splitk_reduce_rows_kernel / splitk_reduce_kernel sum them (launch-boundary split-K, EXPERIMENTS.md r3-E).  The in-launch reduction by the last arriver, the
-// tail-split / M-tail tile orders and the fused-RMSNorm reductions of rounds 2 - 4 measured slower or equal and were removed in round 5 (EXPERIMENTS.md r2-I,
-// r2-T, r3-M, r4-B, r4-H name them and the commits that hold them).  The two levers of the schedule are fixed on: s_setprio around the MFMA segments and the
+// splitk_reduce_rows_kernel / splitk_reduce_kernel sum them (launch-boundary split-K).  The in-launch reduction by the last arriver, the
+// tail-split / M-tail tile orders and the fused-RMSNorm reductions measured slower or equal and are gone.
+// The two levers of the schedule are fixed on: s_setprio around the MFMA segments and the
 // one-barrier stagger of the two wave groups (without either: 830 / 838 TF against 1016 TF on the q|k|v shape).
 template <typename T, int SPLIT>
 __global__ __launch_bounds__(512) void gemm8p_kernel(GemmArgs a) {
@@ -205,8 +205,8 @@ __global__ __launch_bounds__(512) void gemm8p_kernel(GemmArgs a) {
     // the checks into one loop cost the full tiles 15 % (register pressure 218 -> 250, accumulator copies) — so the loop is instantiated
     // twice and chosen once per workgroup.
     // A ragged tile with at most 64 valid rows (T = 1087: the 63 rows of the fifth M-tile) never multiplies X half 1 (tile rows 64..127, 192..255): its ragged loop
-    // neither stages nor reads that half, so phases 2 and 3 of its K-steps shrink to their barriers (round 4: such a tile cost 0.9 of a full one because every
-    // interval lasts as long as its load side, EXPERIMENTS.md r3-M; the counted waits stay valid — fewer loads are in flight than they allow for).
+    // neither stages nor reads that half, so phases 2 and 3 of its K-steps shrink to their barriers (such a tile cost 0.9 of a full one because every
+    // interval lasts as long as its load side; the counted waits stay valid — fewer loads are in flight than they allow for).
     const bool x1_needed = a.M - m0 > 64;
     const int mw = m0 + wm * 128;                     // first row of this wave's 128-row block
     const bool live[4] = {mw < a.M, mw + 32 < a.M, mw + 64 < a.M, mw + 96 < a.M};
@@ -312,7 +312,7 @@ __global__ __launch_bounds__(512) void gemm8p_kernel(GemmArgs a) {
 
 // ---------------------------------------------------------------------------------------------------------------------------
 // Launch-boundary split-K reduction (the form every K-sliced launch takes).
-// In the in-launch form of round 2 ONE workgroup per tile reads S x 256 KiB of partials back through one CU (~10 us at the ~60-100 GB/s a single CU pulls) after an
+// In an in-launch form ONE workgroup per tile reads S x 256 KiB of partials back through one CU (~10 us at the ~60-100 GB/s a single CU pulls) after an
 // agent-scope release / ticket / acquire: ~45 us of the 142 us down_proj launch.  Here the GEMM workgroups store their slabs (plain stores: the kernel
 // boundary publishes them) and exit; this kernel spreads the same sums over 8 workgroups per tile — workgroup (tile, wm, j) owns the 32 x 256 block that
 // accumulator column j of the GEMM's wave row wm held, so thread t re-reads exactly the float4s GEMM thread wm * 256 + t wrote (4 KiB contiguous per

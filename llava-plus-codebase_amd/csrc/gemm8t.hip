@@ -2,7 +2,7 @@
 // (X = dY [rows][M], W = the layer's input [rows][N], C = dW [M = out features][N = in features]; 16-bit operands, fp32 accumulate).
 //
 // Replaces the weight half of torch.nn.Linear's backward (grad_weight = grad_output^T @ input) under the reference's training step
-// (llava/train/train.py:780-1000 -> transformers Trainer -> torch autograd).  Through round 5 the step transposed both operands
+// (llava/train/train.py:780-1000 -> transformers Trainer -> torch autograd).  Before, the step transposed both operands
 // ([rows][M] -> [M][rows], [rows][N] -> [N][rows]: two activation-sized read + write passes per linear) to feed the forward's NT kernel (gemm8p.hip); the
 // transposes were 6.3 % of a 16 x 2048 step (profiles/r06_config5_kernel_stats.csv).  Here the contraction index is the SLOW index of both operands in
 // memory and the MFMA fragments (8 consecutive contraction values per lane) come out of LDS through the gfx950 transpose read, ds_read_b64_tr_b16.

@@ -32,7 +32,7 @@ struct GemmArgs {
     // written)   k rows -> rotated, into the K cache [kv head][pos][D]   v rows -> the V^T cache [kv head][d][pos].  Same arithmetic and rounding points as
     // launch_gemm + launch_rope_kv (HF5:models/llama/modeling_llama.py:130-160,243-281).  qf_kc != null switches it on.
     const float* qf_rope = nullptr; void* qf_kc = nullptr; void* qf_vt = nullptr; int qf_pos0 = 0, qf_nh = 0, qf_nkv = 0, qf_smax = 0, qf_D = 0;
-    // CLIP q|k|v projection with the K / V^T pack in the epilogue (round 4; HF5:models/clip/modeling_clip.py:295-340 reshapes q, k, v per head; here the attention
+    // CLIP q|k|v projection with the K / V^T pack in the epilogue (HF5:models/clip/modeling_clip.py:295-340 reshapes q, k, v per head; here the attention
     // kernel wants K rows [head][pos][D] and V^T [head][d][pos]): columns [0, pk_heads * pk_D) go to C as usual, the k columns to pk_kc, the v columns
     // transposed to pk_vt (2-byte stores, 64-byte runs per register across the wave's 32 rows), same bias and the same rounding as GEMM + pack launch.  Row m
     // belongs to image m / pk_rows at position m % pk_rows; per-image cache stride pk_img_stride elements.  pk_kc != null switches it on (any 16-bit GEMM
@@ -480,7 +480,7 @@ struct P2PLaunch {
     uint32_t seq;                    // 1, 2, 3, ... identical on every rank for the same all-reduce
     void* peer[P2P_MAX_WORLD];       // exchange buffers as mapped in this process
     int last_len = 0;                // elements of the last row when the message is not a whole number of [H] rows (0 = H)
-    // LlamaRMSNorm of the summed rows inside the same launch (round 6; whole rows only): x_out [rows][H] <- rmsnorm(sum) * norm_w — the workgroup that owns a row has it
+    // LlamaRMSNorm of the summed rows inside the same launch (whole rows only): x_out [rows][H] <- rmsnorm(sum) * norm_w — the workgroup that owns a row has it
     // complete, so the decode batch's next linear needs no rmsnorm launch (65 of a tensor-parallel batched step's 227 launches).  rmsnorm_kernel's arithmetic, bit for bit
     const void* norm_w = nullptr; void* x_out = nullptr; float eps = 0.f;
 };
@@ -488,7 +488,7 @@ void launch_p2p_allreduce(int dtype, const P2PLaunch& l, hipStream_t st);
 size_t p2p_buffer_bytes(int world, int H, int es);
 size_t p2p_flags_offset(int world, int H, int es);
 
-// ---- two-shot peer-to-peer all-reduce for PREFILL-sized messages (p2p.hip, round 4): reduce-scatter + all-gather over all links at once ------------------
+// ---- two-shot peer-to-peer all-reduce for PREFILL-sized messages (p2p.hip): reduce-scatter + all-gather over all links at once ------------------
 // xGMI is point-to-point: a ring keeps one link per direction busy (2 (W - 1) / W x message over ONE 153 GB/s link: ~114 us for the 8.9 MB of a 1087-row
 // 7B prefill at W = 8).  Here rank r owns chunk r of the message: every rank pushes chunk p of its partial sums straight into rank p's exchange buffer (W - 1
 // links busy at once), the owner adds the W versions in rank order and pushes the finished chunk to every peer.  One launch, message / W per link and
@@ -528,7 +528,7 @@ int preprocess_coeffs(int in_size, int out_size, int o0, int on, int* bounds_out
 size_t launch_preprocess(int dtype, const uint8_t* rgb, int H, int W, int size, int pad_to_square, const float* mean, const float* std,
                          void* out, void* scratch, size_t scratch_bytes, hipStream_t st);
 
-// ---- training-step slices (train.hip; SURVEY §8 f-3): parity-first kernels, see the file header for the reference lines ------------------
+// ---- training-step slices (train.hip): parity-first kernels, see the file header for the reference lines ------------------
 // shifted cross-entropy over logits [B*T][ld] vs labels [B][T] (label of position t = labels[t + 1]); lse / row_loss: [B*(T-1)] floats;
 // out2[0] = mean loss over the counted positions, out2[1] = their number
 void launch_ce_loss_fwd(int dtype, const void* logits, int ld, const int64_t* labels, int B, int Tlen, int V, int64_t ignore, float* lse,

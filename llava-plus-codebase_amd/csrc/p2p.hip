@@ -184,7 +184,7 @@ __global__ __launch_bounds__(256) void p2p_allreduce_big_kernel(P2PBigArgs a) {
     constexpr int VE = 16 / sizeof(T);
     // workgroup g walks slices g, g + G, ... of every chunk; its flags are indexed by g: ONE release / acquire pair per phase and workgroup, not per slice —
     // a system-scope fence walks the L2, and the 544 x 4 of them of a 1087 x 4096 message cost 346 us between two processes on one MI355X where the data
-    // itself moves in ~10 us (profiles/EXPERIMENTS.md r4-K).  Every rank derives the same G from the message size, so flag g of a peer covers the same slices.
+    // itself moves in ~10 us.  Every rank derives the same G from the message size, so flag g of a peer covers the same slices.
     const int g = blockIdx.x, G = gridDim.x, tid = threadIdx.x;
     const int nv = P2P_BIG_SLICE / VE;                                    // 16-byte vectors per slice
     const int n_slices = (int)(a.chunk / P2P_BIG_SLICE);

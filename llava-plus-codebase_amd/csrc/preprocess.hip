@@ -1,4 +1,4 @@
-// Image preprocessing on the device (SURVEY §8f-4): process_images / expand2square (llava/mm_utils.py:16-44) + HF's
+// Image preprocessing on the device: process_images / expand2square (llava/mm_utils.py:16-44) + HF's
 // CLIPImageProcessor (resize shortest edge with PIL BICUBIC -> center crop -> rescale 1/255 -> normalise) for one decoded RGB
 // image already in HBM as uint8 [H][W][3].  The CPU path costs 10-20 ms per image on the host (PIL resize + numpy), in front of
 // every multimodal request's prefill; here it is two small launches.

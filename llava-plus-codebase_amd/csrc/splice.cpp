@@ -1,6 +1,6 @@
 // Host (integer) half of prepare_inputs_labels_for_multimodal — llava/model/llava_arch.py:99-240.
 //
-// Bit-exact contract (SURVEY §3.2, Appendix A/B2):
+// Bit-exact contract:
 //   :144-145  padding stripped per row with attention_mask
 //   :150-159  a row without IMAGE_TOKEN_INDEX still consumes one image-feature slot (zero-length slice)
 //   :161-187  text pieces and image slots interleaved; image positions get label IGNORE_INDEX

@@ -1,4 +1,4 @@
-// Training-step slices for the visual-instruction-tuning path (SURVEY §8 f-3, BASELINE config 5) — parity-first versions.
+// Training-step slices for the visual-instruction-tuning path — parity-first versions.
 //
 // What the reference runs in a finetuning step (llava/train/train.py:805-1000 -> HF Trainer -> LlavaLlamaForCausalLM.forward with labels,
 // llava_llama.py:56-99 -> LlamaForCausalLM's shifted cross-entropy; attention through llava/train/llama_flash_attn_monkey_patch.py:68-91)
@@ -186,7 +186,7 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_dw_sum_kernel(const float* __
     dw[c] = s;
 }
 
-// One pass over x and dy for 16-bit rows of H = NCH * 512 (round 6; the three launches above read x three times and dy twice: 774 us per norm at 32768 x 4096,
+// One pass over x and dy for 16-bit rows of H = NCH * 512 (the three launches above read x three times and dy twice: 774 us per norm at 32768 x 4096,
 // 2.8 % of a 16 x 2048 training step, profiles/r06_config5_kernel_stats_wgrad.csv).  One wave per row, 16 rows per wave in turn, 8 waves = 128 rows per workgroup:
 // a lane holds its 8 NCH elements of x, dy (and the residual) packed, computes inv, mean(g * xhat), dx, and keeps the row's dy * x * inv in NCH * 8 fp32
 // accumulators; after its rows the eight waves add their accumulators in wave order through LDS and the workgroup writes ONE partial row of dw (the same

@@ -1,4 +1,4 @@
-"""Continuous batching of decode steps (SURVEY §8f-1).
+"""Continuous batching of decode steps.
 
 The reference serves concurrent requests as independent `model.generate` threads with no batching
 (llava/serve/model_worker.py:174-185, `--limit-model-concurrency` :264): every request streams all weights from HBM for
@@ -105,7 +105,7 @@ class DecodeBatcher:
         self._step_status = None        # tensor parallel: pending ok / fail exchange of the last announced decode step (CommandChannel.agree_begin)
         self.scheduler_prefill = bool(scheduler_prefill) or channel is not None      # requests are prefilled by the scheduler, several at a time
         # single process: the packed prefills run on a thread and a stream of their own, so a new request neither waits behind the decode
-        # step in flight nor holds the live requests' next step back (VERDICT r4 item 9).  Under tensor parallelism every call that carries a collective must
+        # step in flight nor holds the live requests' next step back.  Under tensor parallelism every call that carries a collective must
         # be issued in ONE order on every rank: there the prefills stay between two decode steps on the leader's stream
         self.prefill_thread = bool(prefill_thread) and self.scheduler_prefill and channel is None
         # ... and the rank-local half of a request's prefill (image encode or feature-cache hit, splice, prefix-cache take: model._prepare_request) runs on the
@@ -116,7 +116,7 @@ class DecodeBatcher:
         self.max_prefill_batch = max(1, int(max_prefill_batch))
         # rows (prompt positions after the image splice) one packed prefill may hold: bounds how long the live requests wait between two of their
         # decode steps (a packed prefill runs between steps on the scheduler's stream; ~18 ms per 1k rows at 7B) and the packed workspace.  At least one
-        # request is always taken, whatever its length; 0 = unbounded (round 2's behaviour: up to max_prefill_batch requests whatever their size)
+        # request is always taken, whatever its length; 0 = unbounded (up to max_prefill_batch requests whatever their size)
         self.max_prefill_rows = max(0, int(max_prefill_rows))
         self.max_backlog_hold_s = 1.0   # longest the decode loop stands back for a burst's prefills (see _backlogged)
         self._hold_t0 = None
@@ -290,7 +290,7 @@ class DecodeBatcher:
                         if self.channel is not None:
                             # tensor parallel: every rank has seen (or will see at its next exchange) the failed step and the followers leave serve_follower.
                             # Any further send / agree would be a gloo collective against exited ranks: the batcher is dead from here on — fail everything
-                            # queued, refuse new work, never touch the channel again (ADVICE r3)
+                            # queued, refuse new work, never touch the channel again
                             self._break(live, e)
                             return
                         self._fail(live, e)
@@ -473,7 +473,7 @@ class DecodeBatcher:
         for m in self._requests:
             rows += self._request_rows(m.request)
             if rows > max(self.max_prefill_rows, 1):
-                # the hold is BOUNDED (ADVICE r5): under sustained arrivals the backlog never drains, and live requests must not wait for it for seconds — after
+                # the hold is BOUNDED: under sustained arrivals the backlog never drains, and live requests must not wait for it for seconds — after
                 # `max_backlog_hold_s` of standing back the decode steps run beside the prefills again until the backlog has been worked off once
                 now = time.monotonic()
                 if self._hold_t0 is None:

@@ -1,10 +1,10 @@
-"""Prompt templates: the host-side data format on the input side of the hot path (SURVEY §8 f-3 / f-4).
+"""Prompt templates: the host-side data format on the input side of the hot path.
 
 Mirror of the part of llava/conversation.py the training entry (llava/train/train.py:254-665 builds every training prompt through
 `conversation_lib.default_conversation` / `conv_templates[--version]`) and the serving clients (gradio_web_server_llava_plus.py:444-637,
 tools/config4_harness.py) use: the `Conversation` record, its five separator styles and `get_prompt()` (llava/conversation.py:54-148), `append_message`,
 `copy`, and the templates the reference's scripts select (`v1` / `plain` / `llava_llama_2`, plus the other text templates of llava/conversation.py:516-622).
-The Gradio rendering half of that file (HTML, image thumbnails, tool-output folding) is the web UI — out of scope (SURVEY §2).
+The Gradio rendering half of that file (HTML, image thumbnails, tool-output folding) is the web UI — out of scope.
 
 Same names, same fields, same strings out (tests/test_train_data_vs_reference.py compares every template and style against the reference's own module).
 """

@@ -265,7 +265,7 @@ class EngineCausalLM:
         prefill_thread (single process only) = 2 (default): the packed prefills run on their own thread and stream beside the decode steps instead
         of between two of them — a new request does not wait behind the step in flight, the live requests do not wait for its prefill — and each request's
         rank-local half (image encode / feature-cache hit, splice, prefix-cache take) runs on the request's own thread before it queues; 1 = that half on the
-        prefill thread too; 0 = round 4's order (one loop: prefill, then step)."""
+        prefill thread too; 0 = one loop: prefill, then step."""
         from .batching import DecodeBatcher
         if self.tp_world > 1:
             # tensor parallel: only the leader schedules, and it needs the command channel to its followers (tp_serving.py)

@@ -1,4 +1,4 @@
-"""Host-side pre/post-processing that produces the hot path's inputs (boundary-adjacent, SURVEY §2 row 6).
+"""Host-side pre/post-processing that produces the hot path's inputs (boundary-adjacent).
 
 Behavioural mirror of the reference's llava/mm_utils.py (same names, arguments and results) so the serving code that
 imports these helpers keeps working when this package stands in for `llava`:

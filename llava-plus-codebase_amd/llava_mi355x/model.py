@@ -1,7 +1,7 @@
 """Python mirror of the reference's model API over the MI355X engine (C ABI in include/llava_mi355x.h).
 
 Same names / argument meaning / results / error behaviour as the reference classes, so `llava.serve.model_worker`,
-`cli.py`, `predict.py` and the eval drivers keep working on top of it (SURVEY §8b):
+`cli.py`, `predict.py` and the eval drivers keep working on top of it:
   LlavaConfig, LlavaLlamaModel, LlavaLlamaForCausalLM     llava/model/language_model/llava_llama.py:31-111
   LlavaMetaForCausalLM.encode_images / prepare_inputs_labels_for_multimodal   llava/model/llava_arch.py:94-240
   CLIPVisionTower (attributes callers touch)                                  llava/model/multimodal_encoder/clip_encoder.py:7-78
@@ -378,8 +378,8 @@ class LlavaLlamaForCausalLM(EngineCausalLM):
 
     def _run_tower(self, x: torch.Tensor, out: torch.Tensor, sharded: bool) -> None:
         """Tower + projector over x [n,3,S,S] into out [n,P,H].  sharded (tensor parallel, n >= 2; a COLLECTIVE — every rank calls it with the same
-        pixels at the same point of its call sequence): the tower is data parallel over the images ("split images across ranks for B > 1,
-        then all-gather features") — rank r runs images r, r + W, ..., the other rows of `out` stay zero and the decoder's all-reduce sums the ranks'
+        pixels at the same point of its call sequence): the tower is data parallel over the images (images split across ranks, features
+        gathered) — rank r runs images r, r + W, ..., the other rows of `out` stay zero and the decoder's all-reduce sums the ranks'
         buffers, which IS the all-gather (every element has one non-zero contributor: exact in every dtype, like the vocabulary-parallel logits row)."""
         n = x.shape[0]
         if not sharded:

@@ -1,4 +1,4 @@
-"""Reuse across the turns of one conversation (SURVEY §8 f-1 / f-4; VERDICT r3 item 6).
+"""Reuse across the turns of one conversation.
 
 The LLaVA-Plus tool loop (llava/serve/gradio_web_server_llava_plus.py:498-637) answers a question in two `generate` calls: the second prompt is the first
 one — system text, the SAME image, the question — followed by the model's own first answer and the tool's output.  The reference worker

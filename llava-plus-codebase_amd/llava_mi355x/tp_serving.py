@@ -1,4 +1,4 @@
-"""Tensor-parallel serving: one process per GPU, rank 0 serves, the others follow (SURVEY §8e, BASELINE config 4).
+"""Tensor-parallel serving: one process per GPU, rank 0 serves, the others follow.
 
 The reference spreads a model over GPUs inside ONE process (`device_map="auto"`, llava/model/builder.py:26-34) and its worker threads
 call `model.generate` concurrently (llava/serve/model_worker.py:174-185).  With one process per GPU and tensor-parallel shards every
@@ -105,7 +105,7 @@ def prefill_symmetric(model, channel: CommandChannel, reqs, chunk: int) -> list:
          every rank, and the ranks agree once more on its outcome (an error there is raised by argument checks BEFORE any launch, i.e. on every rank
          or on none; the second exchange turns the remaining case into a symmetric failure instead of a hang at the next collective)."""
     # 0. several requests with images: ONE tower pass over all of them, the images split over the ranks and the features all-gathered
-    #    (model._preencode_requests; SURVEY §8e).  It carries a collective, so it is bracketed like step 3: first agree which requests' pixel
+    #    (model._preencode_requests).  It carries a collective, so it is bracketed like step 3: first agree which requests' pixel
     #    tensors every rank holds with the tower's geometry, run the pass over exactly those, agree on its outcome.
     feats = [None] * len(reqs)
     if getattr(model, "tp_world", 1) > 1 and len(reqs) > 1:

@@ -1,4 +1,4 @@
-"""One visual-instruction-tuning step on the MI355X kernels (SURVEY §8 f-3, BASELINE config 5).
+"""One visual-instruction-tuning step on the MI355X kernels.
 
 What the reference runs per step (llava/train/train.py:805-1000 -> HF Trainer.training_step -> LlavaLlamaForCausalLM.forward with labels,
 llava_llama.py:56-99; attention through llava/train/llama_flash_attn_monkey_patch.py:68-91; DeepSpeed ZeRO-2 per scripts/zero2.json:16-22;
@@ -19,7 +19,7 @@ AdamW, max_grad_norm 1.0 from the HF TrainingArguments defaults the launch scrip
 
 This is the parity-first version: fp32-engine runs match torch autograd + torch.optim.AdamW on the oracle (tests/test_train_step_gpu.py).
 `checkpoint=True` keeps only each layer's input and recomputes the layer in the backward pass (the reference's gradient_checkpointing).
-`keep_layers` / `keep_budget_bytes` (round 6): with 288 GB per GPU the LAST k layers keep their activations anyway — as many as the budget holds — and are
+`keep_layers` / `keep_budget_bytes`: with 288 GB per GPU the LAST k layers keep their activations anyway — as many as the budget holds — and are
 not recomputed: every kept layer takes one forward (a quarter of its GEMM FLOPs) out of the step; gradients are the same bits either way.
 """
 from __future__ import annotations
@@ -206,7 +206,7 @@ class TrainStep:
             raise KeyError(f"weights missing for the trainable part: {missing[:4]}...")
         self.shapes = {n: tuple(w[n].shape) for n in order}
         if bucket_elems is None:
-            bucket_elems = self.H * self.H                       # DeepSpeed's "auto" reduce_bucket_size = hidden_size^2 (SURVEY §2b)
+            bucket_elems = self.H * self.H                       # DeepSpeed's "auto" reduce_bucket_size = hidden_size^2
         # q | k | v of a layer form one fused operand of the step: no bucket boundary (padding) between them, whatever the world size
         fused = [f"model.layers.{l}.self_attn.{p}_proj.weight" for l in range(self.L) for p in ("q", "k")]
         self.part = ZeroPartition([(n, int(np.prod(self.shapes[n]))) for n in order], self.world, self.rank, bucket_elems, no_close_after=fused)

@@ -1,5 +1,5 @@
 """Training data pipeline of visual instruction tuning: conversations + image -> (input_ids, labels, image) samples -> padded batches
-(SURVEY §8 f-3, BASELINE config 5: the data format on the input side of the training step, llava_mi355x/train.py).
+(the data format on the input side of the training step, llava_mi355x/train.py).
 
 Mirror of the data half of llava/train/train.py — same names, same arguments, same tensors out:
 
@@ -59,7 +59,7 @@ class DataArguments:
 @dataclass
 class TrainingArguments:
     """The fields of the reference's TrainingArguments (a transformers.TrainingArguments subclass, train.py:83-111) that this package's training entry reads;
-    the HF Trainer / DeepSpeed / bitsandbytes / LoRA knobs have no counterpart here (out of scope)."""
+    the HF Trainer / DeepSpeed / bitsandbytes / LoRA knobs have no counterpart here."""
     output_dir: str = "./checkpoints"
     model_max_length: int = field(default=512, metadata={"help": "Maximum sequence length. Sequences will be right padded (and possibly truncated)."})
     per_device_train_batch_size: int = 16

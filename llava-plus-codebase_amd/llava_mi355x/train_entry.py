@@ -1,4 +1,4 @@
-"""Training entry of visual instruction tuning on the MI355X training step (SURVEY §8 f-3, BASELINE config 5): what llava/train/train.py:805-1000 does around
+"""Training entry of visual instruction tuning on the MI355X training step: what llava/train/train.py:805-1000 does around
 the HF Trainer, around llava_mi355x/train.py: TrainStep instead.
 
     initialize_vision_modules      llava/model/llava_arch.py:42-82     config fields of the vision side, a fresh mm_projector (torch.nn.Linear's own initialiser,
@@ -12,7 +12,7 @@ the HF Trainer, around llava_mi355x/train.py: TrainStep instead.
 
 Here a model is a (config, HF-named weight dict) pair — TrainStep owns the parameters in its flat ZeRO-2 buffers, the CLIP tower is the frozen inference tower of
 llava_mi355x/model.py (clip_encoder.py:25: `requires_grad_(False)`), its output enters the step as data.  Freezing (tune_mm_mlp_adapter, freeze_backbone,
-freeze_mm_mlp_adapter) = the frozen tensors' gradients never reach the optimiser (TrainStep.set_trainable).  Out of scope, as SURVEY §2 has it: DeepSpeed / HF
+freeze_mm_mlp_adapter) = the frozen tensors' gradients never reach the optimiser (TrainStep.set_trainable).  Out of scope: DeepSpeed / HF
 Trainer plumbing, bitsandbytes, LoRA, MPT, checkpoint resumption."""
 from __future__ import annotations
 

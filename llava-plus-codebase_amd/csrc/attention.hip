@@ -6,15 +6,15 @@
 //   HF5:models/clip/modeling_clip.py:259-335  (CLIP attention, non-causal, d=64)
 //   llava/train/llama_flash_attn_monkey_patch.py:79-91 (causal=True, softmax_scale=1/sqrt(d), dropout 0)
 //
-// flash_prefill2_kernel (16-bit, MFMA 32x32x16): one workgroup = 8 waves on 128 query rows; 64-key tiles of K and Vᵀ go by LDS-DMA into an XOR-swizzled
+// flash_prefill2_kernel (16-bit, MFMA 32x32x16): one workgroup = 4 waves on 64 query rows or 8 on 128; tiles of K and Vᵀ go by LDS-DMA into an XOR-swizzled
 //   ring.  Both products keep the query index on the MFMA *column* (lane&31): Sᵀ = K·Qᵀ and Oᵀ = Vᵀ·Pᵀ, so the running max /
 //   sum / rescale are per-lane scalars and P goes from the score accumulators straight into the next MFMA's B operand
 //   with no cross-lane traffic (the key order inside each 16-key MFMA step is permuted identically for P and Vᵀ).
-//   (A 4-wave form took 36.8 us a layer where this takes 27.5.)
 // decode_attn_kernel    (any dtype, VALU): one workgroup per (row, head, key-split); used for single-token decode
 //   (HBM-bound KV streaming) and as the fp32 verification-mode attention for whole prompts.
 #include <algorithm>
 #include <cstdlib>
+#include <type_traits>
 #include "common.h"
 #include "kernels.h"
 #include "attention_decode.h"
@@ -23,36 +23,46 @@
 
 namespace lmx {
 
-// flash_prefill2_kernel: the KEYS of a query block split over two wave groups.
-// One workgroup = 8 waves: wave w works on query rows 32 (w & 3) .. +32 and on the key tiles of parity w >> 2.  The heaviest causal block of a 1087-row
-// prompt walks 17 key tiles alone in the 4-wave kernel (34-39 us per layer while the MFMA work of the launch is ~7 us: one wave per SIMD cannot overlap
-// its softmax VALU work, LDS reads and barrier waits with anything); here every wave walks half the tiles and each SIMD holds two waves — one of each
-// group — whose MFMA and VALU phases interleave.  Tiles are staged in ROUNDS (tile 2r for group 0, 2r + 1 for group 1; each group's four waves DMA
-// their own tile) into a ring of NRND rounds, one workgroup barrier per round.  At the end group 1 hands its (O, m, l) to group 0 through the (then
-// free) ring and group 0 merges the two online-softmax states per lane: m = max(m0, m1), O = O0 2^(m0 - m) + O1 2^(m1 - m), l likewise.
+// flash_prefill2_kernel: the KEYS of a query block split over two wave groups: group g walks the key tiles of parity g, RW waves over the query rows, 32 each.  Tiles are staged in rounds
+// (a tile of each group, by the group's own waves) into a ring of two rounds, one workgroup barrier a round.  At the end group 1 hands its (O, m, l) to group 0 through the (then free)
+// ring and group 0 merges the two online-softmax states per lane: m = max(m0, m1), O = O0 2^(m0 - m) + O1 2^(m1 - m), l likewise.
+// Bound: neither matrix cores nor memory alone.  128 rows x 128 keys of D = 128 take a CU 0.9 us of products, as much of exponentials and their sums and 0.6 - 1.2 us of LDS (fragments; the
+// L2s would deliver the tiles four times as fast), and waves that a barrier keeps in step take them one after the other: 2.0 us.  So
+//   * D = 128 takes K a round ahead of Vᵀ: a tile's exponentials stand between the next tile's score products, whose results they do not wait for, in one instruction stream (turn), with
+//     the LDS reads some products ahead.  8 waves on 128 rows, 64-key tiles: 2.0 -> 1.85 us;
+//   * where blocks of 128 rows leave CUs idle (flash_wide), 64 rows and 32-key tiles: four waves, two workgroups a CU, in step with nobody but themselves.
+// 1087 causal rows of 32 heads 25.0 -> 22.5 us, 139 rows on 1347 keys (with the merge of their slices) 26.8 -> 20.0, 2048 rows of 16 heads with 4 kv heads 39.6 -> 33.2, D = 64: four images of
+// 577 rows, 16 heads, 18.6 -> 17.7 (the scale in the exponential's own multiply-add).  Behind 9216 keys, 256 heads, 128 rows: 163 -> 153.
 // WIN (FlashArgs::win): sliding window, softmax sink and output gate of the windowed decoders.  Only the key tiles a query block can see are walked: the tile
 // range starts at the tile of the first row's oldest visible key, so the work per block is bounded by the window.
-// Without a causal limit every row's position lies behind the last key (launch_flash_prefill): the same code, and fewer registers than a form of its own took (D = 64: 125, 177).
-// D = 64: two workgroups a CU (a ring of two rounds, 128 registers); four images of 577 rows, 16 heads: 24.2 us with one workgroup a CU and a ring of three -> 19.5.
+// Without a causal limit every row's position lies behind the last key (launch_flash_prefill): the same code, and fewer registers than a form of its own took.
+// D = 64: two workgroups a CU (128 registers), which leaves no room for the next tile's scores.
 constexpr int FA_SLICES_MAX = 8;
-template <typename T, int D, bool WIN = false>
-__global__ __launch_bounds__(512, D == 64 && !WIN ? 4 : 2) void flash_prefill2_kernel(FlashArgs a) {
+template <int D, int RW> struct FlashShape {
+    static constexpr int KT = D == 128 && RW == 2 ? 32 : 64;     // keys of a tile
+    static constexpr int QB = 32 * RW, THREADS = 128 * RW;       // query rows, threads of a workgroup: RW waves over the rows, 32 each, in two key groups
+    static constexpr int TILE = 2 * KT * D;                      // bytes of a K or a Vᵀ tile
+    static constexpr int LDS = 2 * 2 * 2 * TILE;                 // two rounds, a round being a tile of each key group
+};
+template <typename T, int D, int RW, bool WIN>
+__global__ __launch_bounds__((FlashShape<D, RW>::THREADS), D == 64 && !WIN ? 4 : 2) void flash_prefill2_kernel(FlashArgs a) {
+    using SH = FlashShape<D, RW>;
+    constexpr int KT = SH::KT, KB = KT / 32;
     constexpr int KSTEPS = D / 16;        // MFMA k-steps over the head dim (QKᵀ)
     constexpr int DB = D / 32;            // 32-row blocks of Oᵀ
-    constexpr int K_BYTES = FA_KT * D * 2;
-    constexpr int V_BYTES = D * FA_KT * 2;
-    constexpr int BUF_BYTES = K_BYTES + V_BYTES;
-    constexpr int NRND = 2;                       // rounds in the ring: 2 x 2 x 32 KiB (D = 128) / 2 x 2 x 16 KiB (D = 64)
     constexpr int KROWS_PP = 1024 / (D * 2);      // K rows per 1-KiB DMA piece (4 for D=128, 8 for D=64)
     constexpr int KCPR = D / 8;                   // 16-byte chunks per K row
-    constexpr int KPPW = K_BYTES / 1024 / 4;      // K pieces per wave per tile
-    constexpr int VPPW = V_BYTES / 1024 / 4;      // Vᵀ pieces per wave per tile (8 rows each)
+    constexpr int KPPW = SH::TILE / 1024 / RW;    // K pieces per wave per tile
+    constexpr int VPPW = SH::TILE / 1024 / RW;    // Vᵀ pieces per wave per tile
+    constexpr int VROWS_PP = 1024 / (KT * 2);     // Vᵀ rows per piece
+    constexpr int VCPR = KT / 8;                  // 16-byte chunks per Vᵀ row
+    constexpr bool PIPE = D == 128;               // the next tile's scores beside this tile's exponentials
 
     extern __shared__ __attribute__((aligned(16))) char smem[];
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave8 = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wave = wave8 & 3, grp = wave8 >> 2;        // query-row wave, key group
+    const int wave = wave8 % RW, grp = wave8 / RW;        // query-row wave, key group
     const int hi = lane >> 5, l31 = lane & 31;
     // 1-D grid ordered by work: ALL heads' heaviest (latest) causal query block first, then the next one, ... so the workgroups
     // that do not fit the first round (grid > CUs) are the lightest ones, not a few heads' full set
@@ -60,9 +70,12 @@ __global__ __launch_bounds__(512, D == 64 && !WIN ? 4 : 2) void flash_prefill2_k
     const int head = blockIdx.x % a.n_heads;
     const int kvh = head / (a.n_heads / a.n_kv_heads);
     const int qb = nqb - 1 - blockIdx.x / a.n_heads;
-    const int q0 = qb * FA_QB + wave * 32;               // this wave's first query row
+    const int q0 = qb * SH::QB + wave * 32;               // this wave's first query row
     const int qrow = q0 + l31;                           // this lane's query row (column of both products)
     const int krow_pi = fa_key_perm(l31);                // key row this lane feeds to QKᵀ as tile row l31
+
+    // scores in the log2 domain: factor behind the products
+    const float sc = (a.scale != 0.f ? fabsf(a.scale) : 1.f) * 1.4426950408889634f;
 
     const size_t bz = blockIdx.y;                        // problem of the batch
     const T* __restrict__ Q = reinterpret_cast<const T*>(a.Q) + bz * a.q_batch;
@@ -76,146 +89,119 @@ __global__ __launch_bounds__(512, D == 64 && !WIN ? 4 : 2) void flash_prefill2_k
         const T* qp = Q + (size_t)qr * a.q_stride + head * D + hi * 8;
 #pragma unroll
         for (int s = 0; s < KSTEPS; ++s) qf[s] = *reinterpret_cast<const uint4*>(qp + s * 16);
-        // These are the only vector-memory loads the COMPILER knows of (the tile DMAs below are inline asm).  Left pending into the key loop, its wait-count
-        // pass guards their first use there with s_waitcnt vmcnt(KSTEPS - 1) ... vmcnt(0) — counts that, on the hardware's single in-order counter, also cover
-        // the DMAs of the NEXT round issued just before: every round waited for its own prefetch inside the S = K Q chain (seen in the ISA).
-        // Waiting here, with an instruction the pass sees, leaves the loop with the one vmcnt wait per round that is meant.  (Time: unchanged — the tiles come
-        // from L2 faster than a round computes — but the ring now works as written.)
-        __builtin_amdgcn_s_waitcnt(0x0F70);          // vmcnt(0); expcnt / lgkmcnt untouched
+        // the products need a positive factor behind the maximum; others turn the queries' signs, or take them as zeros
+        if (a.scale <= 0.f) {
+#pragma unroll
+            for (int s = 0; s < KSTEPS; ++s) {
+                const uint32_t keep = a.scale < 0.f ? 0xffffffffu : 0u, turn = a.scale < 0.f ? 0x80008000u : 0u;
+                qf[s] = uint4{(qf[s].x & keep) ^ turn, (qf[s].y & keep) ^ turn, (qf[s].z & keep) ^ turn, (qf[s].w & keep) ^ turn};
+            }
+        }
     }
 
     // number of key tiles this workgroup needs
     int kv_end = a.kv_len;
     {
-        const int last_q = qb * FA_QB + FA_QB - 1;
+        const int last_q = qb * SH::QB + SH::QB - 1;
         const int lim = a.q_pos0 + (last_q < a.q_len ? last_q : a.q_len - 1) + 1;
         kv_end = lim < kv_end ? lim : kv_end;
     }
     // first tile of the walk (tile indices below are relative to it)
     int tile0 = 0;
     if constexpr (WIN) {
-        const int oldest = a.window > 0 ? a.q_pos0 + qb * FA_QB - a.window + 1 : 0;
-        tile0 = oldest > 0 ? oldest / FA_KT : 0;
+        const int oldest = a.window > 0 ? a.q_pos0 + qb * SH::QB - a.window + 1 : 0;
+        tile0 = oldest > 0 ? oldest / KT : 0;
     }
-    int ntiles = (kv_end + FA_KT - 1) / FA_KT - tile0;
+    int ntiles = (kv_end + KT - 1) / KT - tile0;
     if (a.part) {                                        // this workgroup's slice of the keys (blockIdx.z); 0 tiles: a partial row of weight 0
         const int lo = ntiles * (int)blockIdx.z / (int)gridDim.z;
         ntiles = ntiles * ((int)blockIdx.z + 1) / (int)gridDim.z - lo;
         tile0 += lo;
     }
+    const int nrounds = (ntiles + 1) / 2;
 
     f32x16 oacc[DB];
 #pragma unroll
     for (int i = 0; i < DB; ++i)
 #pragma unroll
         for (int r = 0; r < 16; ++r) oacc[i][r] = 0.f;
+    // running maximum, in units of log2 (scores times sc), and sum
     float m_run = -1e30f, l_run = 0.f;
-    const float sc = a.scale * 1.4426950408889634f;      // work in the log2 domain
     const int my_pos = a.q_pos0 + qrow;                   // causal limit of this lane's row
 
     // ---- K / Vᵀ tiles by LDS-DMA into a ring of two rounds (inline asm: see gemm_pipe_kernel for why) -----------------------
-    // per-lane source offsets (elements) inside a tile; the swizzle lives in the SOURCE address, the LDS image is lane-linear
-    int ksrc[KPPW], vsrc[VPPW];
+    // per-lane source offsets (bytes) inside a tile; the swizzle lives in the SOURCE address, the LDS image is lane-linear
+    uint32_t ksrc[KPPW], vsrc[VPPW];
 #pragma unroll
     for (int i = 0; i < KPPW; ++i) {
-        const int p = wave + 4 * i;
-        const int row = p * KROWS_PP + lane / KCPR;                       // key row inside the tile
-        const int sw = D == 128 ? row : (row >> 1);
-        const int chunk = ((lane % KCPR) ^ sw) & (KCPR - 1);
-        ksrc[i] = row * D + chunk * 8;
+        const int row = (wave + RW * i) * KROWS_PP + lane / KCPR;         // key row inside the tile
+        ksrc[i] = (uint32_t)(row * D + (((lane % KCPR) ^ (D == 128 ? row : row >> 1)) & (KCPR - 1)) * 8) * 2u;
     }
 #pragma unroll
     for (int i = 0; i < VPPW; ++i) {
-        const int p = wave + 4 * i;
-        const int row = p * 8 + (lane >> 3);                              // d row
-        const int chunk = ((lane & 7) ^ (row >> 1)) & 7;                  // 8-key group
-        vsrc[i] = row * a.s_max + chunk * 8;
+        const int row = (wave + RW * i) * VROWS_PP + lane / VCPR;         // d row
+        vsrc[i] = ((uint32_t)row * (uint32_t)a.s_max + (((lane % VCPR) ^ (row / (16 / VCPR))) & (VCPR - 1)) * 8) * 2u;
     }
-    const unsigned lds_base = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
-    auto dma = [&](const T* src, unsigned dst) {
-        unsigned keep;
-        asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
-                     : "=&s"(keep) : "v"(src), "s"(dst) : "memory");
+    const unsigned lds_base = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)smem + wave * 1024);
+    auto dma = [&](const T* src, uint32_t off, unsigned dst) {
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(src), "s"(dst) : "memory");
     };
-    auto stage = [&](int t, int slot) {
-        const unsigned base = lds_base + slot * BUF_BYTES;
-        const T* kt = Kc + (size_t)(tile0 + t) * FA_KT * D;
-        const T* vt = Vt + (size_t)(tile0 + t) * FA_KT;
-#pragma unroll
-        for (int i = 0; i < KPPW; ++i) dma(kt + ksrc[i], __builtin_amdgcn_readfirstlane(base + (wave + 4 * i) * 1024));
-#pragma unroll
-        for (int i = 0; i < VPPW; ++i) dma(vt + vsrc[i], __builtin_amdgcn_readfirstlane(base + K_BYTES + (wave + 4 * i) * 1024));
-    };
-
-    const int nrounds = (ntiles + 1) >> 1;
-    // this wave's group stages tile 2 r + grp of round r into slot (r % NRND) * 2 + grp (nothing if that tile does not exist)
-    auto stage_round = [&](int r) { const int t = 2 * r + grp; if (t < ntiles) stage(t, (r % NRND) * 2 + grp); };
-#pragma unroll
-    for (int r = 0; r < NRND - 1; ++r)
-        if (r < nrounds) stage_round(r);
-    for (int r = 0; r < nrounds; ++r) {
+    // this wave's group stages its tile 2 r + grp of round r into slot 2 (r % 2) + grp of the ring (nothing if that tile does not exist)
+    auto stage_k = [&](int r) {
         const int t = 2 * r + grp;
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // everything this wave staged for round r has landed
-        __builtin_amdgcn_s_barrier();          // round r visible to every wave; everyone is done with round r - 1 (its slots are free)
-        if (r + NRND - 1 < nrounds) stage_round(r + NRND - 1);
-        if (t >= ntiles) continue;             // odd tile count: group 1 sits out the last round (it still takes the barriers)
-        const char* kb_ = smem + ((r % NRND) * 2 + grp) * BUF_BYTES;
-        const char* vb_ = kb_ + K_BYTES;
+        if (t >= ntiles) return;
+        const T* kt = Kc + (size_t)(tile0 + t) * KT * D;
+        const unsigned base = lds_base + ((r & 1) * 2 + grp) * 2 * SH::TILE;
+#pragma unroll
+        for (int i = 0; i < KPPW; ++i) dma(kt, ksrc[i], base + i * RW * 1024);
+    };
+    auto stage_v = [&](int r) {
+        const int t = 2 * r + grp;
+        if (t >= ntiles) return;
+        const T* vt = Vt + (size_t)(tile0 + t) * KT;
+        const unsigned base = lds_base + ((r & 1) * 2 + grp) * 2 * SH::TILE + SH::TILE;
+#pragma unroll
+        for (int i = 0; i < VPPW; ++i) dma(vt, vsrc[i], base + i * RW * 1024);
+    };
+    auto ring_at = [&](int r) { return ((r & 1) * 2 + grp) * 2 * SH::TILE; };
 
-        // ---- Sᵀ = K · Qᵀ : sacc[kb][r] = S[key = t*64 + kb*32 + (r&3) + 8*(r>>2) + 4*hi][q = qrow] ------------
-        f32x16 sacc[2];
+    // fragment f of the stream that a tile's products read: Sᵀ = K · Qᵀ takes K rows kb 32 .. + 31, dims 16 s .. + 15 (f = 2 s + kb: two accumulator chains), Oᵀ += Vᵀ · Pᵀ takes
+    // Vᵀ rows db 32 .. + 31, keys 16 step .. + 15 (f = DB step + db: DB chains; slot e of step is key 16 step + 8 hi + e of the tile, see fa_key_perm: one 16-byte read).  The chunk of
+    // s or step is an xor of address bits that nothing else sets: one register of address for K and one for Vᵀ
+    const int k_lane = k_lds_off<D>(krow_pi, hi), v_lane = SH::TILE + l31 * KT * 2 + (((hi ^ (l31 / (16 / VCPR))) & (VCPR - 1)) << 4);
+    auto k_frag = [&](int ring, int f) { return *reinterpret_cast<const uint4*>(smem + ((ring + k_lane) ^ ((f / KB) << 5)) + f % KB * 64 * D); };
+    auto v_frag = [&](int ring, int f) { return *reinterpret_cast<const uint4*>(smem + ((ring + v_lane) ^ ((f / DB) << 5)) + (f % DB) * 64 * KT); };
+    auto scores = [&](f32x16 (&s)[KB], int f, const uint4& kf) { s[f % KB] = Mfma32<T>::run(kf, qf[f / KB], f < KB ? f32x16{} : s[f % KB]); };
+
+    // s[kb][r] = score of key = tile * 64 + kb * 32 + 16 (r >> 3) + 8 hi + (r & 7) and row qrow, before the scale.  What a row does not see becomes -inf (masking only on tiles that
+    // can hold an invisible key for some row of this wave: a wave-uniform test); the running maximum follows.
+    auto see = [&](f32x16 (&s)[KB], int t) {
+        const int tile_first = (tile0 + t) * KT, tile_last = tile_first + KT - 1;
+        if (tile_last >= a.kv_len || tile_last > a.q_pos0 + q0) {
+            const int last = (my_pos < a.kv_len - 1 ? my_pos : a.kv_len - 1) - tile_first - 8 * hi;      // of the lane's keys
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
+            for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) sacc[kb][r] = 0.f;
-        // the two 32-key blocks are independent accumulator chains: alternate them so back-to-back MFMAs never depend
+                for (int r = 0; r < 16; ++r) s[kb][r] = kb * 32 + 16 * (r >> 3) + (r & 7) <= last ? s[kb][r] : -INFINITY;
+        }
+        if constexpr (WIN) {
+            if (a.window > 0 && tile_first <= a.q_pos0 + q0 + 31 - a.window) {
+                const int first = my_pos - a.window + 1 - tile_first - 8 * hi;
 #pragma unroll
-        for (int s = 0; s < KSTEPS; ++s) {
+                for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
-            for (int kb = 0; kb < 2; ++kb) {
-                const uint4 kf = *reinterpret_cast<const uint4*>(kb_ + k_lds_off<D>(kb * 32 + krow_pi, s * 2 + hi));
-                sacc[kb] = Mfma32<T>::run(kf, qf[s], sacc[kb]);
+                    for (int r = 0; r < 16; ++r) s[kb][r] = kb * 32 + 16 * (r >> 3) + (r & 7) >= first ? s[kb][r] : -INFINITY;
             }
         }
-
-        // ---- online softmax (per lane = per query row) -------------------------------------------------------
-        // masking only on tiles that can contain an invisible key for some row of this wave (wave-uniform test)
-        float p[2][16];
-        float tmax = -INFINITY;
-        const int tile_first = (tile0 + t) * FA_KT, tile_last = tile_first + FA_KT - 1;
-        bool need_mask = tile_last >= a.kv_len || tile_last > a.q_pos0 + q0;
-        if constexpr (WIN) need_mask = need_mask || (a.window > 0 && tile_first <= a.q_pos0 + q0 + 31 - a.window);
-        if (need_mask) {
+        float tmax = s[0][0];
 #pragma unroll
-            for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int key = tile_first + kb * 32 + (r & 3) + 4 * ((r >> 2) & 1) + 8 * hi + 16 * (r >> 3);
-                    bool ok = key < a.kv_len;
-                    ok = ok && key <= my_pos;
-                    if constexpr (WIN) ok = ok && (a.window <= 0 || my_pos - key < a.window);
-                    const float v = ok ? sacc[kb][r] * sc : -INFINITY;
-                    p[kb][r] = v;
-                    tmax = fmaxf(tmax, v);
-                }
-        } else {
-#pragma unroll
-            for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const float v = sacc[kb][r] * sc;
-                    p[kb][r] = v;
-                    tmax = fmaxf(tmax, v);
-                }
-        }
-        tmax = fold32(tmax, OpMax{});
+        for (int i = 1; i < KT / 2; ++i) tmax = fmaxf(tmax, s[i >> 4][i & 15]);
+        tmax = fold32(tmax, OpMax{}) * sc;
         // defer-max: keep the old running max (no O / l rescale) while no row of the wave grew by more than 2^FA_DEFER;
         // P is then bounded by 2^FA_DEFER instead of 1, which fp32 sums and 16-bit P fragments absorb.  m_run starts at
         // -1e30, so the first tile always takes the rescale branch (alpha = 0 on zero accumulators).
-        float m_new = m_run;
         if (!__all(tmax - m_run <= FA_DEFER)) {
-            m_new = fmaxf(m_run, tmax);
-            const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+            const float m_new = fmaxf(m_run, tmax), alpha = __builtin_amdgcn_exp2f(m_run - m_new);
             l_run *= alpha;
 #pragma unroll
             for (int i = 0; i < DB; ++i)
@@ -223,42 +209,122 @@ __global__ __launch_bounds__(512, D == 64 && !WIN ? 4 : 2) void flash_prefill2_k
                 for (int r = 0; r < 16; ++r) oacc[i][r] *= alpha;
             m_run = m_new;
         }
-        float psum = 0.f;
-#pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const float e = __builtin_amdgcn_exp2f(p[kb][r] - m_new);
-                p[kb][r] = e;
-                psum += e;
-            }
-        l_run += psum;
+    };
 
-        // ---- P -> 16-bit B fragments: slot e of step (kb, s2) = p[kb][8*s2 + e] ---------------------------------
-        uint4 pf[2][2];
+    // Probabilities of a tile from its scores, Oᵀ += Vᵀ Pᵀ, and (NEXT) the scores of the group's next tile, as one stream of 32 slots: an exponential each, beside products of the
+    // matrix cores that do not wait for it (the next tile's scores, then the products of probabilities at least a slot back), each with the LDS read of the fragment AHEAD products on.
+    constexpr int AHEAD = 4;
+    uint4 fr[AHEAD];
+    auto read = [&](auto next_c, int kn, int vr, int m) {
+        constexpr int NS = decltype(next_c)::value ? KB * KSTEPS : 0;
+        if (m < NS + 2 * KB * DB) fr[m % AHEAD] = m < NS ? k_frag(kn, m) : v_frag(vr, m - NS);
+    };
+    auto read_ahead = [&](auto next_c, int kn, int vr) {
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
+        for (int m = 0; m < AHEAD; ++m) read(next_c, kn, vr, m);
+    };
+    auto turn = [&](auto next_c, const f32x16 (&s)[KB], f32x16 (&sn)[KB], int kn, int vr) {
+        constexpr bool NEXT = decltype(next_c)::value;
+        constexpr int NS = NEXT ? KB * KSTEPS : 0, NP = 2 * KB * DB;
+        uint4 pf[2 * KB];
+        auto product = [&](int m) {
+            if (m < NS) scores(sn, m, fr[m % AHEAD]);
+            else oacc[(m - NS) % DB] = Mfma32<T>::run(fr[m % AHEAD], pf[(m - NS) / DB], oacc[(m - NS) % DB]);
+            read(next_c, kn, vr, m + AHEAD);
+        };
+        float psum = 0.f, e[KT / 2];
+        auto pack = [&](int j) { pf[j] = uint4{pack2<T>(e[8 * j], e[8 * j + 1]), pack2<T>(e[8 * j + 2], e[8 * j + 3]), pack2<T>(e[8 * j + 4], e[8 * j + 5]), pack2<T>(e[8 * j + 6], e[8 * j + 7])}; };
+        if constexpr (PIPE) {
+            static_assert(KSTEPS == 8 && DB == 4, "slots and products of the stream");
 #pragma unroll
-            for (int s2 = 0; s2 < 2; ++s2) {
-                pf[kb][s2].x = pack2<T>(p[kb][8 * s2 + 0], p[kb][8 * s2 + 1]);
-                pf[kb][s2].y = pack2<T>(p[kb][8 * s2 + 2], p[kb][8 * s2 + 3]);
-                pf[kb][s2].z = pack2<T>(p[kb][8 * s2 + 4], p[kb][8 * s2 + 5]);
-                pf[kb][s2].w = pack2<T>(p[kb][8 * s2 + 6], p[kb][8 * s2 + 7]);
-            }
-
-        // ---- Oᵀ += Vᵀ · Pᵀ : A slot e of step (kb,s2) is key kb*32 + 16*s2 + 8*hi + e (see fa_key_perm: one 16-byte read) -------
-        // key steps outer, d blocks inner: DB independent accumulator chains per step
+            for (int i = 0; i <= KT / 2; ++i) {
+                // products of slot i: the next tile's scores one a slot, then those of the probabilities 8 j .. + 7 from slot 8 j + 9 on, one a slot or one in two, the last step's behind the
+                // last slot
+                if (i < KT / 2) e[i] = __builtin_amdgcn_exp2f(fmaf(s[i >> 4][i & 15], sc, -m_run));
+                if (i > 0) psum += e[i - 1];                 // (a slot behind the exponential)
+                if (i > 0 && i % 8 == 0) pack(i / 8 - 1);
+                if (i < KT / 2) {
+                    if (NEXT && i < NS) product(i);
+                    else if (NEXT && KB == 2 && i < 24) product(i);
+                    else if (i > 8 && (i & 1)) product(KB == 2 ? (NEXT ? 24 + (i - 25) / 2 : (i - 9) / 2) : NS + (i - 9) / 2);
+                } else {
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-            for (int s2 = 0; s2 < 2; ++s2) {
-                const int chunk = kb * 4 + s2 * 2 + hi;          // 16-byte chunk = this lane's 8 consecutive keys
-#pragma unroll
-                for (int db = 0; db < DB; ++db) {
-                    const uint4 vf = *reinterpret_cast<const uint4*>(vb_ + vt_lds_chunk(db * 32 + l31, chunk));
-                    oacc[db] = Mfma32<T>::run(vf, pf[kb][s2], oacc[db]);
+                    for (int m = NS + NP - DB; m < NS + NP; ++m) product(m);
                 }
+                __builtin_amdgcn_sched_barrier(0);
             }
+        } else {
+#pragma unroll
+            for (int i = 0; i < KT / 2; ++i) {
+                e[i] = __builtin_amdgcn_exp2f(fmaf(s[i >> 4][i & 15], sc, -m_run));
+                psum += e[i];
+                if (i % 8 == 7) pack(i / 8);
+            }
+#pragma unroll
+            for (int m = 0; m < NP; ++m) oacc[m % DB] = Mfma32<T>::run(v_frag(vr, m), pf[m / DB], oacc[m % DB]);
+        }
+        l_run += psum;
+    };
+
+    stage_k(0);
+    stage_v(0);
+    if constexpr (PIPE) stage_k(1);
+    // Q's are the only vector-memory loads the COMPILER knows of (the DMAs are inline asm).  Waited for here, with an instruction that its wait-count pass sees, they leave the loop with
+    // the one wait a round that is meant: left pending, their first use there would carry counts that also cover the DMAs on their way.
+    __builtin_amdgcn_s_waitcnt(0x0F70);              // vmcnt(0); expcnt / lgkmcnt untouched
+    if constexpr (PIPE) {
+        // In round r K of round r + 1 and Vᵀ of round r have landed and the scores of round r are in registers: K runs a round ahead of Vᵀ in its two slots
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        f32x16 sa[KB], sb[KB];
+        if (grp < ntiles) {
+#pragma unroll
+            for (int f = 0; f < KB * KSTEPS; ++f) scores(sa, f, k_frag(ring_at(0), f));
+        }
+        auto round = [&](auto next_c, f32x16 (&s)[KB], f32x16 (&sn)[KB], int r) {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // everything this wave staged in the round before has landed
+            __builtin_amdgcn_s_barrier();      // ... and every wave's; everyone is done with K of round r and Vᵀ of round r - 1, whose slots are free
+            asm volatile("" ::: "memory");
+            stage_v(r + 1);
+            stage_k(r + 2);
+            if constexpr (KB == 1) read_ahead(next_c, ring_at(r + 1), ring_at(r));      // on their way while the maximum is found
+            see(s, 2 * r + grp);
+            if constexpr (KB == 2) read_ahead(next_c, ring_at(r + 1), ring_at(r));
+            turn(next_c, s, sn, ring_at(r + 1), ring_at(r));
+        };
+        const int mine = (ntiles + 1 - grp) / 2;              // rounds in which this wave's group has a tile
+        const std::true_type next{};
+        const std::false_type last{};
+        int r = 0;
+#pragma unroll 1
+        for (; r + 2 < mine; r += 2) {
+            round(next, sa, sb, r);
+            round(next, sb, sa, r + 1);
+        }
+        if (r + 1 < mine) {
+            round(next, sa, sb, r);
+            round(last, sb, sa, r + 1);
+        } else if (r < mine) round(last, sa, sb, r);
+        if (mine < nrounds) {                  // an odd tile count: group 1 sits out the last round
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+        }
+    } else {
+#pragma unroll 1
+        for (int r = 0; r < nrounds; ++r) {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // everything this wave staged for round r has landed
+            __builtin_amdgcn_s_barrier();      // round r visible to every wave; everyone is done with round r - 1 (its slots are free)
+            asm volatile("" ::: "memory");
+            stage_k(r + 1);
+            stage_v(r + 1);
+            const int t = 2 * r + grp;
+            if (t >= ntiles) continue;
+            f32x16 s[KB];
+#pragma unroll
+            for (int f = 0; f < KB * KSTEPS; ++f) scores(s, f, k_frag(ring_at(r), f));
+            see(s, t);
+            turn(std::false_type{}, s, s, 0, ring_at(r));
+        }
     }
 
     // ---- merge the two key groups (group 1 -> LDS -> group 0), then O[q][d] = oacc / l ---------------------------------------------------
@@ -353,13 +419,36 @@ __global__ __launch_bounds__(256) void flash_merge_kernel(FlashArgs a, int slice
     *reinterpret_cast<uint2*>(reinterpret_cast<T*>(a.O) + (size_t)(pair / a.n_heads) * a.o_stride + (pair % a.n_heads) * D + d) = u;
 }
 
-// Key slices of a launch: where its workgroups leave half of the CUs idle or more, as many as fill them, of at least four 64-key tiles (two rounds) each.
+// Key slices of a launch: where its workgroups leave half of the places on the CUs empty or more, as many as fill them, of at least four 64-key tiles each.
 // 139 rows on 1347 keys, 32 heads of 128 (64 workgroups of 11 rounds): 30.5 us -> 17.5 with four slices and 5.0 for the merge.
-static int flash_slices(int D, const FlashArgs& a, int workgroups) {
+static int flash_slices(int D, const FlashArgs& a, int workgroups, bool wide) {
     if (!a.part || a.win || a.lse || a.n_batch != 1) return 1;
-    int s = std::min(std::min(256 / workgroups, cdiv(a.kv_len, FA_KT) / 4), FA_SLICES_MAX);
+    int s = std::min(std::min((D == 128 && wide ? 256 : 512) / workgroups, cdiv(a.kv_len, FA_KT) / 4), FA_SLICES_MAX);
     while (s > 1 && (size_t)s * a.q_len * a.n_heads * (D + 4) * sizeof(float) > a.part_bytes) --s;
     return std::max(s, 1);
+}
+
+// Which query blocks, D = 128.  128 rows (eight waves, a workgroup a CU) read K and Vᵀ from L2 and LDS for twice the rows, 64 rows (four waves, two workgroups a CU whose barriers are
+// their own) divide the work twice as finely, and the matrix cores of one workgroup run beside the exponentials of the other.  The larger blocks where they keep the chip busy to the end:
+// their work over 256 CUs against what the busiest CU has, the block with the most tiles or, in a second round (heaviest first), what the last of the first and the first of the second
+// take together.  us, 128 -> 64 rows:  1087 causal rows, 32 heads (0.65 of the time busy) 25.0 -> 22.5;  1100, 16 heads (0.31) 22.6 -> 19.8;  2048, 16 heads (0.53) 36.6 -> 33.2;  2048 in a
+// window of 1024, 32 heads (0.79) 50.5 -> 45.5;  2048, 32 heads (1.0) 52.9 -> 55.8;  128 rows behind 9216, 256 heads (1.0) 159 -> 172.
+static bool flash_wide(int D, const FlashArgs& a) {
+    if (D != 128) return true;
+    const int nqb = cdiv(a.q_len, 128);
+    auto tiles = [&](int qb) {                               // 64-key tiles of a block
+        int end = a.kv_len, first = 0;
+        if (a.causal) end = std::min(end, a.q_pos0 + std::min(128 * (qb + 1), a.q_len));
+        if (a.win && a.window > 0) first = std::max(0, a.q_pos0 + qb * 128 - a.window + 1) / FA_KT;
+        return cdiv(end, FA_KT) - first;
+    };
+    const long heads = (long)a.n_heads * a.n_batch, blocks = nqb * heads;
+    if (blocks < 256) return false;
+    long all = 0;
+    for (int qb = 0; qb < nqb; ++qb) all += tiles(qb) * heads;
+    auto nth = [&](long i) { return i < blocks ? tiles(nqb - 1 - (int)(i / heads)) : 0; };
+    const int busiest = blocks > 512 ? 0 : std::max(nth(0), nth(255) + nth(256));
+    return all >= 0.9 * 256 * busiest;
 }
 
 void launch_flash_prefill(int dtype, int D, const FlashArgs& a, hipStream_t st) {
@@ -369,22 +458,22 @@ void launch_flash_prefill(int dtype, int D, const FlashArgs& a, hipStream_t st) 
     LMX_REQUIRE(a.kv_len <= a.s_max && a.q_len > 0, "bad lengths");
     LMX_REQUIRE(a.q_stride % 8 == 0 && a.o_stride % 4 == 0, "q/o strides must keep 16-byte alignment");
     LMX_REQUIRE(a.n_batch >= 1 && (a.n_batch == 1 || (!a.win && !a.lse && a.q_batch % 8 == 0 && a.o_batch % 4 == 0 && a.kv_batch % 8 == 0)), "flash prefill: a batch is of plain problems, 16 bytes apart");
-    const int slices = flash_slices(D, a, cdiv(a.q_len, FA_QB) * a.n_heads);
-    const dim3 grid(cdiv(a.q_len, FA_QB) * a.n_heads, a.n_batch, slices);
+    const bool wide = flash_wide(D, a);
+    const int qblocks = cdiv(a.q_len, wide ? 128 : 64), slices = flash_slices(D, a, qblocks * a.n_heads, wide);
+    const dim3 grid(qblocks * a.n_heads, a.n_batch, slices);
     {
-        // two key groups per query block (flash_prefill2_kernel): 8 waves, ring of 2 rounds of two tiles
-        const int smem2 = 2 * 2 * (FA_KT * D * 2 + D * FA_KT * 2);
-#define LMX_FA2_LAUNCH(TT, DD, WW)                                                                                  \
+#define LMX_FA2_LAUNCH(TT, DD, RW, WW)                                                                              \
     do {                                                                                                            \
-        auto kern = flash_prefill2_kernel<TT, DD, WW>;                                                                \
+        using SH = FlashShape<DD, RW>;                                                                              \
+        auto kern = flash_prefill2_kernel<TT, DD, RW, WW>;                                                          \
         static bool attr_set = false;                                                                               \
         if (!attr_set) {                                                                                            \
-            LMX_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, smem2)); \
+            LMX_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, SH::LDS)); \
             attr_set = true;                                                                                        \
         }                                                                                                           \
-        hipLaunchKernelGGL(kern, grid, dim3(512), smem2, st, b);                                                    \
+        hipLaunchKernelGGL(kern, grid, dim3(SH::THREADS), SH::LDS, st, b);                                          \
     } while (0)
-#define LMX_FA2_D(TT, WW) do { if (D == 128) LMX_FA2_LAUNCH(TT, 128, WW); else LMX_FA2_LAUNCH(TT, 64, WW); } while (0)
+#define LMX_FA2_D(TT, WW) do { if (D == 64) LMX_FA2_LAUNCH(TT, 64, 4, WW); else if (wide) LMX_FA2_LAUNCH(TT, 128, 4, WW); else LMX_FA2_LAUNCH(TT, 128, 2, WW); } while (0)
         FlashArgs b = a;
         if (!a.causal) b.q_pos0 = a.kv_len;                  // every row sees every key
         if (slices == 1) b.part = nullptr;

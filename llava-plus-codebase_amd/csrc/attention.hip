@@ -44,8 +44,9 @@ template <int D, int RW> struct FlashShape {
     static constexpr int TILE = 2 * KT * D;                      // bytes of a K or a Vᵀ tile
     static constexpr int LDS = 2 * 2 * 2 * TILE;                 // two rounds, a round being a tile of each key group
 };
+// block: of the launch's query blocks of every head (a.q_len rows); bz: problem of a batch
 template <typename T, int D, int RW, bool WIN>
-__global__ __launch_bounds__((FlashShape<D, RW>::THREADS), D == 64 && !WIN ? 4 : 2) void flash_prefill2_kernel(FlashArgs a) {
+__device__ __forceinline__ void flash_body(const FlashArgs& a, const int block, const int nqb, const size_t bz, char* smem) {
     using SH = FlashShape<D, RW>;
     constexpr int KT = SH::KT, KB = KT / 32;
     constexpr int KSTEPS = D / 16;        // MFMA k-steps over the head dim (QKᵀ)
@@ -58,18 +59,15 @@ __global__ __launch_bounds__((FlashShape<D, RW>::THREADS), D == 64 && !WIN ? 4 :
     constexpr int VCPR = KT / 8;                  // 16-byte chunks per Vᵀ row
     constexpr bool PIPE = D == 128;               // the next tile's scores beside this tile's exponentials
 
-    extern __shared__ __attribute__((aligned(16))) char smem[];
-
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave8 = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wave = wave8 % RW, grp = wave8 / RW;        // query-row wave, key group
     const int hi = lane >> 5, l31 = lane & 31;
     // 1-D grid ordered by work: ALL heads' heaviest (latest) causal query block first, then the next one, ... so the workgroups
     // that do not fit the first round (grid > CUs) are the lightest ones, not a few heads' full set
-    const int nqb = gridDim.x / a.n_heads;
-    const int head = blockIdx.x % a.n_heads;
+    const int head = block % a.n_heads;
     const int kvh = head / (a.n_heads / a.n_kv_heads);
-    const int qb = nqb - 1 - blockIdx.x / a.n_heads;
+    const int qb = nqb - 1 - block / a.n_heads;
     const int q0 = qb * SH::QB + wave * 32;               // this wave's first query row
     const int qrow = q0 + l31;                           // this lane's query row (column of both products)
     const int krow_pi = fa_key_perm(l31);                // key row this lane feeds to QKᵀ as tile row l31
@@ -77,7 +75,6 @@ __global__ __launch_bounds__((FlashShape<D, RW>::THREADS), D == 64 && !WIN ? 4 :
     // scores in the log2 domain: factor behind the products
     const float sc = (a.scale != 0.f ? fabsf(a.scale) : 1.f) * 1.4426950408889634f;
 
-    const size_t bz = blockIdx.y;                        // problem of the batch
     const T* __restrict__ Q = reinterpret_cast<const T*>(a.Q) + bz * a.q_batch;
     const T* __restrict__ Kc = reinterpret_cast<const T*>(a.K) + bz * a.kv_batch + (size_t)kvh * a.s_max * D;
     const T* __restrict__ Vt = reinterpret_cast<const T*>(a.VT) + bz * a.kv_batch + (size_t)kvh * D * a.s_max;
@@ -390,6 +387,27 @@ __global__ __launch_bounds__((FlashShape<D, RW>::THREADS), D == 64 && !WIN ? 4 :
     }
 }
 
+template <typename T, int D, int RW, bool WIN>
+__global__ __launch_bounds__((FlashShape<D, RW>::THREADS), D == 64 && !WIN ? 4 : 2) void flash_prefill2_kernel(FlashArgs a) {
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    flash_body<T, D, RW, WIN>(a, blockIdx.x, gridDim.x / a.n_heads, blockIdx.y, smem);
+}
+
+// blockIdx.y: the segment.  Bound: a launch of one short prompt leaves most CUs idle.  32 prompts of 29 .. 64 rows, 32 heads: 8.4 us each, 268 in all -> 19.2 together; three of 1100, 894
+// and 688, 16 heads: 54 -> 29
+template <typename T, int D, int RW>
+__global__ __launch_bounds__((FlashShape<D, RW>::THREADS), 2) void flash_segs_kernel(FlashArgs a, RowSegs g) {
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const RowSeg& s = g.s[blockIdx.y];
+    const int nqb = (s.n + FlashShape<D, RW>::QB - 1) / FlashShape<D, RW>::QB;
+    if ((int)blockIdx.x >= nqb * a.n_heads) return;
+    a.Q = reinterpret_cast<const T*>(a.Q) + (size_t)s.row0 * a.q_stride;
+    a.O = reinterpret_cast<T*>(a.O) + (size_t)s.row0 * a.o_stride;
+    if (a.gate) a.gate = reinterpret_cast<const T*>(a.gate) + (size_t)s.row0 * a.q_stride;
+    a.K = s.K; a.VT = s.VT; a.q_len = s.n; a.kv_len = s.pos0 + s.n; a.q_pos0 = s.pos0; a.s_max = s.s_max;
+    flash_body<T, D, RW, true>(a, blockIdx.x, nqb, 0, smem);
+}
+
 // the slices' partial rows of one (query row, head), in slice order: four dims a thread
 template <typename T, int D>
 __global__ __launch_bounds__(256) void flash_merge_kernel(FlashArgs a, int slices) {
@@ -493,6 +511,33 @@ void launch_flash_prefill(int dtype, int D, const FlashArgs& a, hipStream_t st) 
         LMX_CHECK_HIP(hipGetLastError());
         return;
     }
+}
+
+void launch_flash_segs(int dtype, int D, const FlashArgs& a, const RowSegs& g, hipStream_t st) {
+    LMX_REQUIRE(dtype == kBF16 || dtype == kF16, "flash prefill is the 16-bit path");
+    LMX_REQUIRE(D == 64 || D == 128, "head_dim must be 64 or 128");
+    LMX_REQUIRE(a.win && a.causal && !a.lse && !a.part && a.n_batch == 1, "flash segments: the windowed form");
+    LMX_REQUIRE(a.q_stride % 8 == 0 && a.o_stride % 4 == 0, "q/o strides must keep 16-byte alignment");
+    LMX_REQUIRE(g.n >= 0 && g.n <= ROW_SEGS, "flash segments: too many");
+    int most = 0;
+    for (int i = 0; i < g.n; ++i) {
+        const RowSeg& s = g.s[i];
+        LMX_REQUIRE(s.K && s.VT && s.n >= 1 && s.row0 >= 0 && s.pos0 >= 0 && s.s_max % 64 == 0 && s.pos0 + s.n <= s.s_max, "flash segments: bad lengths");
+        most = std::max(most, s.n);
+    }
+    if (g.n == 0) return;
+#define L(TT, DD, RW) do {                                                                                                               \
+        using SH = FlashShape<DD, RW>;                                                                                                   \
+        auto kern = flash_segs_kernel<TT, DD, RW>;                                                                                       \
+        static bool attr_set = false;                                                                                                    \
+        if (!attr_set) { LMX_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, SH::LDS)); attr_set = true; } \
+        hipLaunchKernelGGL(kern, dim3(cdiv(most, SH::QB) * a.n_heads, g.n), dim3(SH::THREADS), SH::LDS, st, a, g);                       \
+    } while (0)
+#define LD(TT) do { if (D == 128) L(TT, 128, 2); else L(TT, 64, 4); } while (0)
+    if (dtype == kBF16) LD(bf16_t); else LD(f16_t);
+#undef LD
+#undef L
+    LMX_CHECK_HIP(hipGetLastError());
 }
 
 // ---------------------------------------------------------------------------------------------------------------

@@ -213,7 +213,7 @@ struct Model {
     struct Segment { int seq, src0, dst0, n, pos0; };    // rows [src0, src0 + n) of sequence `seq` sit at rows [dst0, ...) of the piece; first position pos0
     // a mixer over the normed rows x of a piece -> rows [an] of pitch out_k; qkv: its projection rows
     void stack_mix_prefill(int r, Seq* const* seqs, const std::vector<Segment>& seg, int fill, const void* x, void* qkv, void* mix, void* scratch, const DevBuf& skw, hipStream_t st);
-    size_t stack_mix_scratch(int rows, int keys) const;
+    size_t stack_mix_scratch(int rows, int keys, int n) const;      // n: sequences of the call
     // the same over one new token of every sequence (tab: batch; else `one`), projection rows already there
     bool stack_mix_decode(int r, const DecodeFusedSeq* tab, const DecodeFusedSeq& one, int n, int max_len, const void* x, void* qkv, void* mix, const StackWs& w, Batch* b, hipStream_t st, const GemvArgs* beside = nullptr);
     void stack_moe(const StackLayer& l, const void* x, int rows, const StackWs& w, const StackProf& pn, hipStream_t st, bool routed = false, const GemvArgs* beside = nullptr);      // routed: the mixer's launch chose the experts; beside: a linear in the launch of the first product (few rows)

@@ -105,6 +105,10 @@ bool gemv2_applies(int dtype, const GemvArgs& a);
 // ---- attention (attention.hip) ------------------------------------------------------------------------------
 // K cache layout  : [n_kv_heads][s_max][D]      (key rows, post-RoPE)
 // Vᵀ cache layout : [n_kv_heads][D][s_max]      (value columns; keys contiguous so P·V fragments are 8-byte reads)
+// rows of several sequences in one launch: rows [row0, row0 + n) of a piece are positions pos0 .. of a sequence with these caches of the layer (latents: K alone)
+constexpr int ROW_SEGS = 32;
+struct RowSeg { int row0, n, pos0, s_max, zero_to; void* K; void* VT; };
+struct RowSegs { int n; RowSeg s[ROW_SEGS]; };
 struct FlashArgs {
     const void* Q;      // [q_len rows][q_stride] ; head h at column h*D
     void* O;            // [q_len rows][o_stride] ; head h at column h*D
@@ -130,6 +134,8 @@ struct FlashArgs {
     size_t part_bytes = 0;
 };
 void launch_flash_prefill(int dtype, int D, const FlashArgs& a, hipStream_t st);
+// the windowed form over the rows of several sequences: Q, O and gate are row 0 of the piece; lengths, positions and caches are the segments'
+void launch_flash_segs(int dtype, int D, const FlashArgs& a, const RowSegs& g, hipStream_t st);
 
 struct DecodeAttnArgs {
     const void* Q;         // [n_rows][q_stride]; head h at h*D  (already rotated)
@@ -235,6 +241,8 @@ struct QkvNormRopeArgs {
     int zero_to = 0;                      // cache rows [pos0 + T, pos0 + zero_to) become zero (caches whose memory held something else before)
 };
 void launch_qkv_norm_rope_kv(int dtype, int D, const QkvNormRopeArgs& a, hipStream_t st);
+// over the rows of several sequences (qkv: row 0 of the piece); rotations of whole 16-byte groups
+void launch_qkv_norm_rope_segs(int dtype, int D, const QkvNormRopeArgs& a, const RowSegs& g, hipStream_t st);
 // attention of prompt rows on the vector ALUs (any dtype; FlashArgs' windowed causal form)
 void launch_rows_attn(int dtype, int D, const FlashArgs& a, hipStream_t st);
 
@@ -306,8 +314,10 @@ struct LatentNormArgs {                  // rows: c_q <- rms_norm(c_q) in place,
     void* cache; int pos0;               // row i goes to position pos0 + i; with tab: one row per sequence at *pos_ptr (cache = K)
     const DecodeFusedSeq* tab = nullptr; const int* pos_ptr = nullptr;
     int s_max; float eps;
+    void* lat = nullptr;                 // optional [rows][R]: the normalised latents once more, row by row
 };
 void launch_latent_norm(int dtype, const LatentNormArgs& a, int rows, hipStream_t st);
+void launch_latent_norm_segs(int dtype, const LatentNormArgs& a, const RowSegs& g, hipStream_t st);      // rows of several sequences: segment i's to its K
 struct LatentDecodeArgs {                // queries already in the latent space, [n_seq][H][R]; out the attention-weighted latents, same layout
     const void* q; void* out;
     const DecodeFusedSeq* tab = nullptr; DecodeFusedSeq one{};

@@ -15,20 +15,16 @@
 
 namespace lmx {
 
-// grid (rows), 256 threads: waves 0, 1 own the query latent, waves 2, 3 the other one
+// row `row` of the projection by 256 threads: waves 0, 1 own the query latent, waves 2, 3 the other one, which goes to cache row `to`
 template <typename T>
-__global__ __launch_bounds__(256) void latent_norm_kernel(LatentNormArgs a) {
+__device__ __forceinline__ void latent_norm_row(const LatentNormArgs& a, int row, T* to) {
     __shared__ float red[4];
-    const int row = blockIdx.x, tid = threadIdx.x, wave = tid >> 6, half = wave >> 1, lt = tid & 127;
+    const int tid = threadIdx.x, wave = tid >> 6, half = wave >> 1, lt = tid & 127;
     T* src = reinterpret_cast<T*>(a.proj) + (size_t)row * a.ld + (half ? a.Q : 0);
     const T* w = reinterpret_cast<const T*>(half ? a.r_w : a.q_w);
     const int n = half ? a.R : a.Q;
-    T* dst = src;
-    if (half) {
-        int pos = a.tab ? *a.tab[row].pos_ptr : a.pos_ptr ? *a.pos_ptr : a.pos0 + row;
-        pos = pos < a.s_max ? pos : a.s_max - 1;
-        dst = reinterpret_cast<T*>(a.tab ? a.tab[row].K : a.cache) + (size_t)pos * a.R;
-    }
+    T* dst = half ? to : src;
+    T* lat = half && a.lat ? reinterpret_cast<T*>(a.lat) + (size_t)row * a.R : nullptr;
     float ss = 0.f;
     for (int c = lt * 8; c < n; c += 1024) {
         float v[8]; load8<T>(src + c, v);
@@ -44,7 +40,42 @@ __global__ __launch_bounds__(256) void latent_norm_kernel(LatentNormArgs a) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] *= inv * g[e];
         store8<T>(dst + c, v);
+        if (lat) store8<T>(lat + c, v);
     }
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void latent_norm_kernel(LatentNormArgs a) {
+    const int row = blockIdx.x;
+    int pos = a.tab ? *a.tab[row].pos_ptr : a.pos_ptr ? *a.pos_ptr : a.pos0 + row;
+    pos = pos < a.s_max ? pos : a.s_max - 1;
+    latent_norm_row<T>(a, row, reinterpret_cast<T*>(a.tab ? a.tab[row].K : a.cache) + (size_t)pos * a.R);
+}
+
+// grid (rows of the longest segment, segments)
+template <typename T>
+__global__ __launch_bounds__(256) void latent_norm_segs_kernel(LatentNormArgs a, RowSegs g) {
+    const RowSeg& s = g.s[blockIdx.y];
+    if ((int)blockIdx.x >= s.n) return;
+    latent_norm_row<T>(a, s.row0 + blockIdx.x, reinterpret_cast<T*>(s.K) + (size_t)(s.pos0 + blockIdx.x) * a.R);
+}
+
+static int longest(const RowSegs& g) {
+    int n = 0;
+    for (int i = 0; i < g.n; ++i) n = std::max(n, g.s[i].n);
+    return n;
+}
+
+void launch_latent_norm_segs(int dtype, const LatentNormArgs& a, const RowSegs& g, hipStream_t st) {
+    LMX_REQUIRE(a.Q % 64 == 0 && a.R % 64 == 0 && a.q_n >= 1 && a.q_n <= a.Q && a.r_n >= 1 && a.r_n <= a.R && a.ld % 8 == 0 && a.ld >= a.Q + a.R, "latent_norm: bad widths");
+    LMX_REQUIRE(a.proj && a.q_w && a.r_w && g.n >= 0 && g.n <= ROW_SEGS, "latent_norm: bad arguments");
+    for (int i = 0; i < g.n; ++i) LMX_REQUIRE(g.s[i].K && g.s[i].n >= 1 && g.s[i].row0 >= 0 && g.s[i].pos0 >= 0 && g.s[i].pos0 + g.s[i].n <= g.s[i].s_max, "latent_norm: bad cache rows");
+    if (g.n == 0) return;
+    const dim3 grid(longest(g), g.n);
+#define L(TT) LMX_LAUNCH(latent_norm_segs_kernel<TT>, grid, dim3(256), 0, st, a, g)
+    if (dtype == kBF16) L(bf16_t); else if (dtype == kF16) L(f16_t); else L(float);
+#undef L
+    LMX_CHECK_HIP(hipGetLastError());
 }
 
 void launch_latent_norm(int dtype, const LatentNormArgs& a, int rows, hipStream_t st) {

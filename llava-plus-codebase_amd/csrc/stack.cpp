@@ -388,7 +388,7 @@ void Model::stack_prefill(Seq* const* seqs, const void* const* embeds, const int
     const size_t o_h = carve(S.ids_in() ? 0 : (size_t)block_rows * H * es), o_xr = carve((size_t)block_rows * H * 4), o_x = carve((size_t)block_rows * H * es),
                  o_y = carve((size_t)block_rows * H * es), o_qkv = carve((size_t)block_rows * qkv_n * es), o_attn = carve((size_t)block_rows * S.mix_n * es),
                  o_act = carve((size_t)block_rows * I_l * es), o_log = carve((size_t)std::min(n, HEAD_ROWS) * V * 4), o_want = carve((size_t)std::min(block_rows, LOGIT_ROWS) * H * es),
-                 o_ws = carve(S.ws_bytes(block_rows, H, es, false)), o_scratch = carve(stack_mix_scratch(block_rows, max_end));
+                 o_ws = carve(S.ws_bytes(block_rows, H, es, false)), o_scratch = carve(stack_mix_scratch(block_rows, max_end, n));
     if (off > s0->pws.bytes) { LMX_CHECK_HIP(hipStreamSynchronize(st)); s0->pws.ensure(off); }
     char* Wk = s0->pws.as<char>();
     void *h = Wk + o_h, *x = Wk + o_x, *y = Wk + o_y, *qkv = Wk + o_qkv, *attn = Wk + o_attn, *act = Wk + o_act, *want = Wk + o_want, *scratch = Wk + o_scratch;
@@ -457,7 +457,21 @@ void Model::stack_prefill(Seq* const* seqs, const void* const* embeds, const int
             const int an = l.an;
             { LMX_PROF_K("prefill.gemm.qkv"); launch_gemm(dt, with_scratch(GemmArgs{x, l.wqkv, qkv, l.bqkv, nullptr, fill, l.qkv_n, H, H, H, l.qkv_n, 0, kActNone}), gv, st); }
             if (d.mixer != LMX_MIXER_ATTENTION) stack_mix_prefill(r, seqs, seg, fill, x, qkv, attn, scratch, s0->skw, st);
-            else for (const Segment& g : seg) {
+            else if (seg.size() > 1 && dt != kF32 && l.D <= 128 && d.rope_dims % 16 == 0) {      // rows of several sequences: one launch for up to ROW_SEGS of them
+                for (size_t s0 = 0; s0 < seg.size(); s0 += ROW_SEGS) {
+                    RowSegs g{};
+                    g.n = (int)std::min(seg.size() - s0, (size_t)ROW_SEGS);
+                    for (int i = 0; i < g.n; ++i) {
+                        const Segment& e = seg[s0 + (size_t)i];
+                        g.s[i] = RowSeg{e.dst0, e.n, e.pos0, kv_pitch, 0, seqs[e.seq]->kc.as<char>() + S.runs[(size_t)r].k_off, seqs[e.seq]->vt.as<char>() + S.runs[(size_t)r].v_off};
+                    }
+                    { LMX_PROF("prefill.norm_rope_kv"); launch_qkv_norm_rope_segs(dt, l.D, rope_args(S, l, qkv, nullptr, nullptr, 0, 0, kv_pitch), g, st); }
+                    LMX_PROF("prefill.attn");
+                    FlashArgs fa{qkv, attn, nullptr, nullptr, 0, 0, 0, l.qkv_n, l.out_k, d.n_heads, d.n_kv_heads, kv_pitch, d.attn_scale, 1};
+                    fa.win = 1; fa.window = d.window; fa.sink = d.softmax_sink; fa.gate = l.gate_off >= 0 ? static_cast<char*>(qkv) + (size_t)l.gate_off * es : nullptr;
+                    launch_flash_segs(dt, l.D, fa, g, st);
+                }
+            } else for (const Segment& g : seg) {
                 Seq* s = seqs[g.seq];
                 void *kc = s->kc.as<char>() + S.runs[(size_t)r].k_off, *vt = s->vt.as<char>() + S.runs[(size_t)r].v_off;
                 void *qr = rows(qkv, g.dst0, l.qkv_n), *ar = rows(attn, g.dst0, l.out_k);

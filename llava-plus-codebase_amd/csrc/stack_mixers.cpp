@@ -39,14 +39,25 @@ StackWs Stack::ws(void* base, int rows, int H, int es, bool decode) const {
 // keys [k0, end) that the rows of a segment can see, k0 on a 64-key boundary
 static int first_key(const lmx_layer_config& d, int pos0) { return d.window > 0 && pos0 - d.window + 1 > 0 ? (pos0 - d.window + 1) & ~63 : 0; }
 
-// scratch of the widest mixer; keys: longest context of the call
-size_t Model::stack_mix_scratch(int rows, int keys) const {
+// several prompts from their first rows on, all in one launch each of norm, expansion, caches and attention (32 prompts of 29 .. 64 rows, a latent layer of 4096: 32 x (3.4 + 9.7 + 4.6 +
+// 8.4) us -> 6.5 + 27.7 + 18.0 + 19.2).  Rows that go on behind cached ones see keys that are no rows of the piece: those pieces take the segments one after the other
+static bool fresh_together(int dtype, int D, const std::vector<Model::Segment>& seg) {
+    if (dtype == kF32 || D > 128 || seg.size() < 2) return false;
+    for (const Model::Segment& g : seg) if (g.pos0) return false;
+    return true;
+}
+
+// scratch of the widest mixer; keys: longest context of the call, n: sequences
+size_t Model::stack_mix_scratch(int rows, int keys, int n) const {
     size_t most = 0;
     for (const StackLayer& l : stk->layers) {
         size_t b = 0;
         if (l.c.mixer == LMX_MIXER_LATENT) {
             const int nk = l.c.window > 0 ? std::min(keys, rows + l.c.window + 64) : keys;
             b = up256((size_t)rows * l.an * es) + up256((size_t)nk * 2 * l.an * es) + 2 * up256((size_t)round_up(nk, 128) * l.an * es);
+            if (n > 1)                                       // together (fresh_together): latents and their keys and values by row, caches of whole 128 keys each
+                b = std::max(b, up256((size_t)rows * l.an * es) + up256((size_t)rows * l.R * es) + up256((size_t)rows * 2 * l.an * es) +
+                                    2 * up256((size_t)(rows + 127 * std::min(n, ROW_SEGS)) * l.an * es));
         } else if (l.c.mixer == LMX_MIXER_DELTA) b = up256((size_t)rows * l.ds.H * (l.ds.DK + l.ds.DV) * es) + delta_scratch_bytes(l.ds, rows, es);
         most = std::max(most, b);
     }
@@ -88,6 +99,47 @@ void Model::stack_mix_prefill(int r, Seq* const* seqs, const std::vector<Segment
             { LMX_PROF_K("prefill.delta.scan"); launch_delta_scan(dt, a, st); }
             { LMX_PROF_K("prefill.delta.gate"); launch_delta_gate(dt, a, st); }
         }
+        return;
+    }
+    if (fresh_together(dt, l.D, seg)) {
+        // every key is a row of this piece: one product makes all keys and values
+        void* q = take((size_t)fill * l.an * es);
+        void* lat = take((size_t)fill * l.R * es);
+        char* kv = take((size_t)fill * 2 * l.an * es);
+        const size_t cache = (size_t)(fill + 127 * std::min((int)seg.size(), ROW_SEGS)) * l.an * es;
+        char *kc = take(cache), *vt = take(cache);
+        auto groups = [&](auto&& f) {
+            for (size_t s0 = 0; s0 < seg.size(); s0 += ROW_SEGS) {
+                RowSegs g{};
+                g.n = (int)std::min(seg.size() - s0, (size_t)ROW_SEGS);
+                f(g, seg.data() + s0);
+            }
+        };
+        groups([&](RowSegs& g, const Segment* s) {
+            LMX_PROF("prefill.latent_norm");
+            for (int i = 0; i < g.n; ++i) g.s[i] = RowSeg{s[i].dst0, s[i].n, 0, s_max, 0, seqs[s[i].seq]->kc.as<char>() + run.k_off, nullptr};
+            LatentNormArgs n{qkv, l.qkv_n, l.Q, d.q_rank, l.R, d.kv_rank, l.qn_lat, l.kn_lat, nullptr, 0};
+            n.eps = S.c.norm_eps; n.lat = lat;
+            launch_latent_norm_segs(dt, n, g, st);
+        });
+        gemm("prefill.gemm.uq", GemmArgs{qkv, l.wuq, q, nullptr, nullptr, fill, l.an, l.Q, l.qkv_n, l.Q, l.an, 0, kActNone});
+        gemm("prefill.gemm.ukv", GemmArgs{lat, l.wukv, kv, nullptr, nullptr, fill, 2 * l.an, l.R, l.R, l.R, 2 * l.an, 0, kActNone});
+        groups([&](RowSegs& g, const Segment* s) {
+            size_t at = 0;
+            for (int i = 0; i < g.n; ++i) {
+                const int cap = round_up(s[i].n, 128);
+                g.s[i] = RowSeg{s[i].dst0, s[i].n, 0, cap, cap, kc + at, vt + at};      // the attention tiles are whole: what lies behind the last key must not be NaN bits
+                at += (size_t)cap * l.an * es;
+            }
+            {
+                LMX_PROF("prefill.kv_rows");
+                launch_qkv_norm_rope_segs(dt, l.D, QkvNormRopeArgs{kv, nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, 2 * l.an, 0, d.n_heads, 0, l.D, 0, S.c.norm_eps}, g, st);
+            }
+            LMX_PROF("prefill.attn");
+            FlashArgs fa{q, mix, nullptr, nullptr, 0, 0, 0, l.an, l.out_k, d.n_heads, d.n_heads, 0, d.attn_scale, 1};
+            fa.win = 1; fa.window = d.window; fa.sink = d.softmax_sink;
+            launch_flash_segs(dt, l.D, fa, g, st);
+        });
         return;
     }
     // latent attention: latents into the cache, queries, then per segment the keys and values its rows can see

@@ -47,3 +47,21 @@ def test_more_sequences_than_one_launch_takes(cuda, family):
     assert max(family.rel(g, oracle(t)) for t, g in zip(ts, rows)) < family.TOL["bf16"]
     for c in caches:
         c.close()
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+def test_chosen_rows_of_several_sequences(cuda, dt):
+    """Single rows (more than a gather takes), pairs, whole stretches and a sequence without any, in one call: the rows of the call that asks for all of them."""
+    from llava_mi355x.engine_lm import LmxKVCache
+    m = siterax.model("mixed", dt)
+    n = [129, 70, 1, 200, 33]
+    ts = [siterax.tokens("mixed", k, 600 + i) for i, k in enumerate(n)]
+    chosen = [list(range(0, 129, 2)), [0, 1, 7, 8, 69], [0], list(range(10, 75)) + [199], [31, 32]]
+    oracle = [siterax.oracle("mixed", t) for t in ts]
+    caches = [LmxKVCache(m, 1) for _ in ts]
+    got = m.prefill_logits(caches, [m.get_model().embed_tokens(torch.tensor(t)) for t in ts], chosen)
+    torch.cuda.synchronize()
+    got = got[:, : m.config.vocab_size].split([len(c) for c in chosen])
+    assert max(siterax.rel(g, o[c]) for g, o, c in zip(got, oracle, chosen)) < siterax.TOL[dt]
+    for c in caches:
+        c.close()

@@ -298,7 +298,8 @@ int lmx_profile_read(lmx_model* m, char* names_buf, int32_t names_cap, double* m
  *   "vis_pack"      CLIP K / V^T pack in the tower's q|k|v GEMM epilogue (HF5:models/clip/modeling_clip.py:295-340) vs. a pack launch
  *   "decode_splitq" decode step of 16-bit models as q launch + (k|v projection with the attention workgroups) launch vs. q|k|v launch + attention launch
  *   "stack_fuse"    (default 1, no environment variable; equal up to rounding) a layer-stack decode step's residual addition and norms inside the linear that reads them, a parallel layer's
- *                   router in its mixer's launch, and its gate|up and output projection beside the delta step and the experts vs. launches of their own
+ *                   router in its mixer's launch, its gate|up and output projection beside the delta step and the experts, and the splits of its attention added by the linear behind it
+ *                   vs. launches of their own
  * Unknown keys are an error.  Not to be flipped while requests are in flight on other threads. */
 int lmx_model_set_option(lmx_model* m, const char* key, int32_t value);
 

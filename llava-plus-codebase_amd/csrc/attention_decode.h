@@ -22,6 +22,14 @@ __device__ __forceinline__ void rope8(const T* __restrict__ x, const float* __re
     }
 }
 
+// softmax end of one (row, head): unnormalised o, sum l and log2-domain maximum M -> output value.  A sink is one more key of score 0 without a value.
+__device__ __forceinline__ float softmax_scale(float l, float M, bool sink) {
+    if (!sink) return l > 0.f ? 1.f / l : 0.f;
+    const float m2 = fmaxf(M, 0.f), f = __builtin_amdgcn_exp2f(M - m2);
+    return f / (l * f + __builtin_amdgcn_exp2f(-m2));
+}
+__device__ __forceinline__ float sigmoid_f32(float g) { return 1.f / (1.f + __expf(-g)); }
+
 constexpr int DF_CHUNK = 128;     // keys per workgroup (fixed: every K / Vᵀ load of the chunk is issued up front)
 constexpr int DF_MAX_SPLIT = 32;
 

@@ -227,7 +227,7 @@ struct Model {
     // splitq:    the decode step's q|k|v projection as q-launch + (k|v projection ∥ attention) launch (decode_attn.hip) — bit-identical
     bool opt_fuse_rope = true, opt_fuse_slices = true, opt_vis_pack = true, opt_splitq = true;
     // stack_fuse: a layer-stack decode step's residual addition and norms inside the linear's launch, a parallel layer's router in its mixer's launch, its gate | up and output projection
-    //             beside the delta step and the experts — equal up to rounding, faster
+    //             beside the delta step and the experts, the splits of its attention added by the output projection — equal up to rounding, faster
     bool opt_stack_fuse = true;
     // Sequences in existence (lmx_seq_create .. lmx_seq_destroy).  The split-q launch parks one waiting workgroup per head until its own launch's projection has
     // run; launches of DIFFERENT sequences (request threads on their own streams) may be resident together, so the form is only taken while all sequences'

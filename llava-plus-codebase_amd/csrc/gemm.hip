@@ -643,6 +643,13 @@ __global__ __launch_bounds__(64 * NW) void gemv2_res_kernel(GemvArgs a, Residual
     gemv2_body<T, R, P, GEMV2_NX, false, true, NW>(a, (int)blockIdx.x, smem, nullptr, 0u, nullptr, &rn);
 }
 
+// the output projection behind a split decode attention (gemv2.h SPLITS)
+template <typename T, int R, int SPLITS>
+__global__ __launch_bounds__(512) void gemv2_heads_kernel(GemvArgs a, HeadSplitArgs h) {
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    gemv2_body<T, R, 4, 1, false, false, 8, SPLITS>(a, (int)blockIdx.x, smem, nullptr, 0u, nullptr, nullptr, &h);
+}
+
 // ---------------------------------------------------------------------------------------------
 // host launchers
 // ---------------------------------------------------------------------------------------------
@@ -930,6 +937,28 @@ void launch_gemv_residual(int dtype, GemvArgs a, const ResidualNormArgs& rn, hip
     LMX_REQUIRE(!a.R && (!act_gated(a.act) || a.N % 64 == 0), "gemv_residual: no second residual; SiLU*mul needs N % 64 == 0");
     a.X = rn.y; a.norm_w = rn.pre_w;
     if (dtype == kBF16) launch_gemv2_res<bf16_t>(a, rn, st); else launch_gemv2_res<f16_t>(a, rn, st);
+}
+
+// Eight waves share a row of up to 4096 (a chunk of eight a thread); one weight row a wave, two where that would be more than a workgroup for every CU.  Every workgroup reads all partials:
+// attention + linear, 8 heads x 128 behind 600 keys 13.4 -> 11.3 us, 16 x 128 behind 600 / 1000 13.2 -> 11.4 / 13.8 -> 12.1, 32 x 128 behind 600 / 1000 (32 KB a split) 16.3 -> 15.8 /
+// 17.3 -> 17.1: past 32768 values what the merge saves is gone.  More splits than that stay with the attention's merge (fewer of them: 16 x 256 behind 2000 keys 21.3 -> 23.0).
+int gemv_heads_splits(int dtype, const GemvArgs& a, int heads, int D) {
+    if (!gemv2_applies(dtype, a) || a.K != heads * D || D % 8 != 0 || a.K > 4096 || a.norm_w || a.R || a.act != kActNone || a.c_f32) return 0;
+    return std::min(16, 32768 / a.K);
+}
+void launch_gemv_heads(int dtype, GemvArgs a, const HeadSplitArgs& h, hipStream_t st) {
+    a.X = nullptr;
+    LMX_REQUIRE(h.ws && h.n_split >= 2 && h.n_split <= gemv_heads_splits(dtype, a, h.heads, h.D), "gemv_heads: a plain linear of up to 4096 inputs behind 2..16 splits, 32768 values at most");
+    const size_t smem = gemv2_smem_bytes(a.K, 2, 8);
+    const bool two = a.N > 8 * 256;
+#define L(TT, R, S) LMX_LAUNCH((gemv2_heads_kernel<TT, R, S>), dim3(cdiv(a.N, 8 * R)), dim3(512), smem, st, a, h)
+#define LS(TT, R) do { if (h.n_split <= 4) L(TT, R, 4); else if (h.n_split <= 6) L(TT, R, 6); else if (h.n_split <= 8) L(TT, R, 8); else L(TT, R, 16); } while (0)
+#define LR(TT) do { if (two) LS(TT, 2); else LS(TT, 1); } while (0)
+    if (dtype == kBF16) LR(bf16_t); else LR(f16_t);
+#undef LR
+#undef LS
+#undef L
+    LMX_CHECK_HIP(hipGetLastError());
 }
 
 // The single-row decode linears of 16-bit models take the hand-counted stream.  (R rows per wave, P rounds in flight) per shape from an in-situ sweep

@@ -99,6 +99,10 @@ struct GemvForm { int rows, ahead, waves = 4; };       // rows of a wave, loads 
 GemvForm gemv2_form(const GemvArgs& a);     // of a linear on the weight stream (gemv2.h)
 GemvForm gemv2_res_form(const GemvArgs& a); // of one whose row is formed in front of it
 void launch_gemv(int dtype, const GemvArgs& a, int MB, hipStream_t st);
+// a linear whose input row is a split decode attention's (WinDecodeArgs::leave): partials [heads][n_split][D + 4] as that launch leaves them, gate: head 0's gate or null
+struct HeadSplitArgs { const float* ws; const void* gate; int heads, n_split, D, sink; };
+int gemv_heads_splits(int dtype, const GemvArgs& a, int heads, int D);      // splits it takes at most; 0: not this linear
+void launch_gemv_heads(int dtype, GemvArgs a, const HeadSplitArgs& h, hipStream_t st);
 // does launch_gemv(MB = 1) of this shape take the hand-counted weight stream (gemv2.h)?
 bool gemv2_applies(int dtype, const GemvArgs& a);
 
@@ -256,6 +260,7 @@ struct WinDecodeArgs {
     int n_seq = 1, qkv_stride = 0, out_stride = 0, n_heads = 0, n_kv_heads = 0, s_max = 0, n_split = 1;
     int qk_dim = 0, rot_dims = 0, window = 0, sink = 0, gate_off = -1;      // gate_off: column of head 0's gate in the row, -1 = no gates
     float scale = 1.f, eps = 0.f;
+    int leave = 0;                        // one sequence in several splits: the partials stay as they are for the output projection (launch_gemv_heads), `out` is not written
 };
 // grouped: one workgroup per kv head and split (where decode_win_groups says that it can) instead of one per query head and split; wide: of eight waves instead of four
 void launch_decode_win(int dtype, int D, const WinDecodeArgs& a, bool grouped, bool wide, hipStream_t st);

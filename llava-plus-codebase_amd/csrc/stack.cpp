@@ -677,16 +677,22 @@ void Model::stack_decode_step(Seq* s, hipStream_t st, int64_t* id_out) {
         const GemvArgs go{s->d_attn, l.wo, s->d_y, nullptr, nullptr, nullptr, 0.f, H, l.out_k, l.out_k, l.out_k, H, 0, kActNone};
         const bool par = l.parallel() && opt_stack_fuse, join_gu = par && l.dense() && l.c.mixer == LMX_MIXER_DELTA && delta_decode_joins(dt, l.ds, gu);
         const bool join_o = par && l.moe() && act_gated(l.act()) && !group_gemm_applies(dt, l.c.top_experts, l.c.experts) && group_gemv_joins(dt, stack_moe_first(l, s->d_x, s->sw), l.c.top_experts, go);
+        HeadSplitArgs heads{};                               // splits that the output projection adds
         if (l.c.mixer == LMX_MIXER_ATTENTION) {
             LMX_PROF_K("decode.attn");
             WinForm f;
             WinDecodeArgs a = decode_args(S, l, dt, s->d_qkv, s->d_attn, 1, s->len, kv_pitch, f);
             a.one = stack_seq_ref(r, s);
             a.pos = s->len;
+            if (!f.grouped && a.n_split > 1 && !l.parallel() && opt_stack_fuse && a.n_split <= gemv_heads_splits(dt, go, l.c.n_heads, l.D)) {
+                a.leave = 1;
+                heads = HeadSplitArgs{a.one.ws, a.gate_off >= 0 ? static_cast<char*>(s->d_qkv) + (size_t)a.gate_off * es : nullptr, l.c.n_heads, a.n_split, l.D, a.sink};
+            }
             launch_decode_win(dt, l.D, a, f.grouped, f.wide, st);
         } else routed = stack_mix_decode(r, nullptr, stack_seq_ref(r, s), 1, s->len, s->d_x, s->d_qkv, s->d_attn, s->sw, nullptr, st, join_gu ? &gu : nullptr);
         if (l.parallel() && l.dense() && !join_gu) { LMX_PROF_K("decode.gemv.gate_up"); launch_gemv(dt, gu, 1, st); }
-        if (!join_o) { LMX_PROF_K("decode.gemv.o"); launch_gemv(dt, go, 1, st); }
+        if (heads.ws) { LMX_PROF_K("decode.gemv.o"); launch_gemv_heads(dt, go, heads, st); }
+        else if (!join_o) { LMX_PROF_K("decode.gemv.o"); launch_gemv(dt, go, 1, st); }
         y = s->d_y;
         if (l.ff && !l.parallel()) {
             const StackStep sp = stack_step(S, r, 0, final_norm);

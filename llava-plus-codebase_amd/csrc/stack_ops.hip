@@ -409,13 +409,6 @@ void launch_qkv_norm_rope_kv(int dtype, int D, const QkvNormRopeArgs& a, hipStre
     LMX_CHECK_HIP(hipGetLastError());
 }
 
-// softmax end of one (row, head): unnormalised o, sum l and log2-domain maximum M -> output value.  A sink is one more key of score 0 without a value.
-__device__ __forceinline__ float softmax_scale(float l, float M, bool sink) {
-    if (!sink) return l > 0.f ? 1.f / l : 0.f;
-    const float m2 = fmaxf(M, 0.f), f = __builtin_amdgcn_exp2f(M - m2);
-    return f / (l * f + __builtin_amdgcn_exp2f(-m2));
-}
-__device__ __forceinline__ float sigmoid_f32(float g) { return 1.f / (1.f + __expf(-g)); }
 
 // ---------------------------------------------------------------------------------------------------------------
 // attention of prompt rows on the vector ALUs: grid (n_heads, rows).  Scores of the row's visible keys wait in LDS.
@@ -536,7 +529,7 @@ __device__ __forceinline__ void norm_rope_vec(const T* __restrict__ x, const T* 
     }
 }
 
-template <typename T, int D>
+template <typename T, int D, bool LEAVE = false>
 __global__ __launch_bounds__(256) void decode_win_kernel(WinDecodeArgs a) {
     __shared__ __attribute__((aligned(16))) float sc[DF_CHUNK];
     __shared__ __attribute__((aligned(16))) float qs[D], ks[D];
@@ -656,10 +649,15 @@ __global__ __launch_bounds__(256) void decode_win_kernel(WinDecodeArgs a) {
         if (s8 == 0) {
             const int d = db * 32 + drow;
             if (a.n_split == 1) out[d] = from_f32<T>(t * fin);
+            else if constexpr (LEAVE) ws[d] = t;
             else __hip_atomic_store(ws + d, t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
     if (a.n_split == 1) return;
+    if constexpr (LEAVE) {                                   // the next launch adds the splits (gemv2.h)
+        if (tid == 0) { ws[D] = m; ws[D + 1] = l; }
+        return;
+    }
     if (tid == 0) {
         __hip_atomic_store(ws + D, m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __hip_atomic_store(ws + D + 1, l, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1004,6 +1002,7 @@ void launch_decode_win(int dtype, int D, const WinDecodeArgs& a, bool grouped, b
     LMX_REQUIRE(a.n_heads >= 1 && a.n_kv_heads >= 1 && a.n_heads % a.n_kv_heads == 0 && a.qkv && a.out, "decode_win: bad arguments");
     LMX_REQUIRE(a.rot_dims % 2 == 0 && a.rot_dims <= a.qk_dim && a.qk_dim <= D && (a.rot_dims == 0 || a.cos_sin), "decode_win: bad rotation");
     LMX_REQUIRE(a.tab || (a.n_seq == 1 && a.one.K && a.one.VT && a.one.ws && a.one.counters && (a.pos >= 0 || a.one.pos_ptr)), "decode_win: bad sequence");
+    LMX_REQUIRE(!a.leave || (a.n_seq == 1 && !grouped), "decode_win: splits are left to the next launch by one sequence");
     if (grouped && decode_win_groups(dtype, D, a.n_heads, a.n_kv_heads, a.n_seq) && a.qkv_stride % 4 == 0 && reinterpret_cast<uintptr_t>(a.qkv) % 8 == 0) {
         const dim3 grid(a.n_kv_heads, a.n_split, a.n_seq);
         const int group = a.n_heads / a.n_kv_heads;
@@ -1024,7 +1023,7 @@ void launch_decode_win(int dtype, int D, const WinDecodeArgs& a, bool grouped, b
         return;
     }
     const dim3 grid(a.n_heads, a.n_split, a.n_seq);
-#define L(TT, DD) LMX_LAUNCH((decode_win_kernel<TT, DD>), grid, dim3(256), 0, st, a)
+#define L(TT, DD) do { if (a.leave) LMX_LAUNCH((decode_win_kernel<TT, DD, true>), grid, dim3(256), 0, st, a); else LMX_LAUNCH((decode_win_kernel<TT, DD>), grid, dim3(256), 0, st, a); } while (0)
 #define LD(TT) do { if (D == 256) L(TT, 256); else if (D == 128) L(TT, 128); else L(TT, 64); } while (0)
     if (dtype == kBF16) LD(bf16_t); else if (dtype == kF16) LD(f16_t); else LD(float);
 #undef LD

@@ -105,7 +105,7 @@ __device__ __forceinline__ void gemv2_body(const GemvArgs& a, int bid, char* sme
     }
     const ws_v4i rsG = ws_make_rsrc(a.norm_w ? a.norm_w : a.W, 0x7fffffffu);
     ws_u32x4 graw[GEMV2_NX];                                  // RMSNorm weights of the same chunks (same queue position: older than every weight load)
-    if (a.norm_w) {
+    if (SPLITS == 0 && a.norm_w) {                            // (the merged row has no norm: nothing would wait for these registers)
 #pragma unroll
         for (int i = 0; i < GEMV2_NX; ++i) {
             const int c = tid + 64 * NW * i;

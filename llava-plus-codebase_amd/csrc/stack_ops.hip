@@ -409,7 +409,6 @@ void launch_qkv_norm_rope_kv(int dtype, int D, const QkvNormRopeArgs& a, hipStre
     LMX_CHECK_HIP(hipGetLastError());
 }
 
-
 // ---------------------------------------------------------------------------------------------------------------
 // attention of prompt rows on the vector ALUs: grid (n_heads, rows).  Scores of the row's visible keys wait in LDS.
 // ---------------------------------------------------------------------------------------------------------------

@@ -15,6 +15,9 @@
 //   * Between the first issue and the drain the wave must not execute stores or other loads whose completion order matters: vmcnt counts loads and
 //     stores in one queue and only loads retire in order.  (LDS traffic is on lgkmcnt and is free to interleave.)  Loads issued by hipcc BEFORE or
 //     BETWEEN are safe in the other direction: its own counted waits only ever become more conservative.
+//   * A register whose load is on the way must not be moved: a copy reads what stood there before, and the register, free for other use, is overwritten when the load lands (an address held in
+//     it then faults).  hipcc moves them once a kernel needs more than 256 registers beside its accumulators: such forms are not to be built, and the listing shows it (v_accvgpr_write of a
+//     destination in front of its wait).  For the same reason every load has a consumer behind its wait on every path.
 //   * The count must stay exact up to the last round, so rounds past the end of the stream are issued as dummy loads of one hot line (offset 0 of W).
 #pragma once
 #include "common.h"

@@ -298,10 +298,15 @@ __device__ __forceinline__ void flash_body(const FlashArgs& a, const int block, 
             round(next, sa, sb, r);
             round(next, sb, sa, r + 1);
         }
+        // one round without a next tile for odd and even counts: with one of each behind the loop, 128 rows took 256 registers and spilled 23, whose reloads waited for the DMAs (this form: 220, 64
+        // rows 181 instead of 241; the loop is the same, the copy is 32 registers once)
         if (r + 1 < mine) {
             round(next, sa, sb, r);
-            round(last, sb, sa, r + 1);
-        } else if (r < mine) round(last, sa, sb, r);
+#pragma unroll
+            for (int kb = 0; kb < KB; ++kb) sa[kb] = sb[kb];
+            ++r;
+        }
+        if (r < mine) round(last, sa, sb, r);
         if (mine < nrounds) {                  // an odd tile count: group 1 sits out the last round
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             __builtin_amdgcn_s_barrier();

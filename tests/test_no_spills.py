@@ -52,3 +52,11 @@ def test_hot_gemm8p_instantiations_have_no_scratch(tmp_path):
     assert len(hot) == 6, sorted(usage)
     bad = {k: usage[k] for k in hot if usage[k] != 0}
     assert not bad, bad
+
+
+@pytest.mark.skipif(shutil.which("hipcc") is None and not os.path.exists("/opt/rocm/bin/hipcc"), reason="hipcc not available")
+def test_prompt_attention_has_no_scratch(tmp_path):
+    """flash_prefill2_kernel stands at two waves a SIMD; a reload from scratch waits for every tile that is on its way into LDS."""
+    usage = {k: v for k, v in scratch_sizes("attention.hip", tmp_path).items() if "flash_" in k}
+    assert len([k for k in usage if "flash_prefill2" in k]) == 12, sorted(usage)      # {bf16, f16} x {64, 128 / 64 rows, 128 / 128 rows} x {plain, windowed}
+    assert not {k: v for k, v in usage.items() if v}, usage

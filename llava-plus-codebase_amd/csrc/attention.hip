@@ -398,19 +398,19 @@ __global__ __launch_bounds__((FlashShape<D, RW>::THREADS), D == 64 && !WIN ? 4 :
     flash_body<T, D, RW, WIN>(a, blockIdx.x, gridDim.x / a.n_heads, blockIdx.y, smem);
 }
 
-// blockIdx.y: the segment.  Bound: a launch of one short prompt leaves most CUs idle.  32 prompts of 29 .. 64 rows, 32 heads: 8.4 us each, 268 in all -> 19.2 together; three of 1100, 894
+// Bound: a launch of one short prompt leaves most CUs idle.  32 prompts of 29 .. 64 rows, 32 heads: 8.4 us each, 268 in all -> 19.2 together; three of 1100, 894
 // and 688, 16 heads: 54 -> 29
 template <typename T, int D, int RW>
 __global__ __launch_bounds__((FlashShape<D, RW>::THREADS), 2) void flash_segs_kernel(FlashArgs a, RowSegs g) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    const RowSeg& s = g.s[blockIdx.y];
+    int block = blockIdx.x;
+    const RowSeg& s = g.s[row_segs_at(g, block)];
     const int nqb = (s.n + FlashShape<D, RW>::QB - 1) / FlashShape<D, RW>::QB;
-    if ((int)blockIdx.x >= nqb * a.n_heads) return;
     a.Q = reinterpret_cast<const T*>(a.Q) + (size_t)s.row0 * a.q_stride;
     a.O = reinterpret_cast<T*>(a.O) + (size_t)s.row0 * a.o_stride;
     if (a.gate) a.gate = reinterpret_cast<const T*>(a.gate) + (size_t)s.row0 * a.q_stride;
     a.K = s.K; a.VT = s.VT; a.q_len = s.n; a.kv_len = s.pos0 + s.n; a.q_pos0 = s.pos0; a.s_max = s.s_max;
-    flash_body<T, D, RW, true>(a, blockIdx.x, nqb, 0, smem);
+    flash_body<T, D, RW, true>(a, block, nqb, 0, smem);
 }
 
 // the slices' partial rows of one (query row, head), in slice order: four dims a thread
@@ -518,25 +518,32 @@ void launch_flash_prefill(int dtype, int D, const FlashArgs& a, hipStream_t st) 
     }
 }
 
-void launch_flash_segs(int dtype, int D, const FlashArgs& a, const RowSegs& g, hipStream_t st) {
+// the segments with the most keys first, as a segment's own blocks go: a long prompt that the caller names last does not begin last
+FlashSegsPlan flash_segs_plan(int D, int n_heads, RowSegs& g) {
+    const int rows = D == 128 ? 64 : 128;
+    std::stable_sort(g.s, g.s + g.n, [](const RowSeg& x, const RowSeg& y) { return x.pos0 + x.n > y.pos0 + y.n; });
+    return {rows, row_segs_blocks(g, [&](const RowSeg& s) { return cdiv(s.n, rows) * n_heads; })};
+}
+
+void launch_flash_segs(int dtype, int D, const FlashArgs& a, const RowSegs& segs, hipStream_t st) {
+    RowSegs g = segs;
     LMX_REQUIRE(dtype == kBF16 || dtype == kF16, "flash prefill is the 16-bit path");
     LMX_REQUIRE(D == 64 || D == 128, "head_dim must be 64 or 128");
     LMX_REQUIRE(a.win && a.causal && !a.lse && !a.part && a.n_batch == 1, "flash segments: the windowed form");
     LMX_REQUIRE(a.q_stride % 8 == 0 && a.o_stride % 4 == 0, "q/o strides must keep 16-byte alignment");
     LMX_REQUIRE(g.n >= 0 && g.n <= ROW_SEGS, "flash segments: too many");
-    int most = 0;
     for (int i = 0; i < g.n; ++i) {
         const RowSeg& s = g.s[i];
         LMX_REQUIRE(s.K && s.VT && s.n >= 1 && s.row0 >= 0 && s.pos0 >= 0 && s.s_max % 64 == 0 && s.pos0 + s.n <= s.s_max, "flash segments: bad lengths");
-        most = std::max(most, s.n);
     }
     if (g.n == 0) return;
+    const FlashSegsPlan plan = flash_segs_plan(D, a.n_heads, g);
 #define L(TT, DD, RW) do {                                                                                                               \
         using SH = FlashShape<DD, RW>;                                                                                                   \
         auto kern = flash_segs_kernel<TT, DD, RW>;                                                                                       \
         static bool attr_set = false;                                                                                                    \
         if (!attr_set) { LMX_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, SH::LDS)); attr_set = true; } \
-        hipLaunchKernelGGL(kern, dim3(cdiv(most, SH::QB) * a.n_heads, g.n), dim3(SH::THREADS), SH::LDS, st, a, g);                       \
+        hipLaunchKernelGGL(kern, dim3(plan.blocks), dim3(SH::THREADS), SH::LDS, st, a, g);                                                \
     } while (0)
 #define LD(TT) do { if (D == 128) L(TT, 128, 2); else L(TT, 64, 4); } while (0)
     if (dtype == kBF16) LD(bf16_t); else LD(f16_t);

@@ -716,6 +716,23 @@ int lmx_op_window_attn(int32_t dtype, int32_t D, const void* q, int32_t q_stride
     if (rows_form || dtype == kF32 || D > 128) launch_rows_attn(dtype, D, a, S(stream)); else launch_flash_prefill(dtype, D, a, S(stream));
     LMX_API_END
 }
+int lmx_op_flash_segs_plan(int32_t D, int32_t n_heads, int32_t n, const int32_t* lens, const int32_t* pos0, int32_t* form, int32_t* blocks, int32_t cap) {
+    LMX_API_BEGIN
+    LMX_REQUIRE((D == 64 || D == 128) && n_heads >= 1 && n >= 1 && n <= ROW_SEGS && lens && pos0 && form && (blocks || cap <= 0), "flash_segs_plan: bad arguments");
+    RowSegs g{};
+    g.n = n;
+    for (int i = 0; i < n; ++i) {
+        LMX_REQUIRE(lens[i] >= 1 && pos0[i] >= 0, "flash_segs_plan: bad lengths");
+        g.s[i].row0 = i; g.s[i].n = lens[i]; g.s[i].pos0 = pos0[i];
+    }
+    const FlashSegsPlan p = flash_segs_plan(D, n_heads, g);
+    form[0] = p.rows; form[1] = p.blocks;
+    for (int b = 0; b < p.blocks && b < cap; ++b) {
+        int at = b;
+        blocks[2 * b] = g.s[row_segs_at(g, at)].row0; blocks[2 * b + 1] = at;
+    }
+    LMX_API_END
+}
 int lmx_op_decode_win_waves(int32_t dtype, int32_t D, const void* qkv, int32_t qkv_stride, void* out, int32_t out_stride, void* const* kcaches, void* const* vtcaches,
                       const int32_t* const* pos_devs, void* const* ws_devs, int32_t* const* counters_devs, int32_t n_seq, void* tab_dev, const void* q_norm, const void* k_norm,
                       const float* cos_sin_dev, int32_t n_heads, int32_t n_kv_heads, int32_t s_max, int32_t n_split, int32_t qk_dim, int32_t rot_dims, int32_t window, int32_t sink,

@@ -3,6 +3,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <hip/hip_ext.h>
+#include <limits.h>
 #include <stdint.h>
 
 namespace lmx {
@@ -112,7 +113,22 @@ bool gemv2_applies(int dtype, const GemvArgs& a);
 // rows of several sequences in one launch: rows [row0, row0 + n) of a piece are positions pos0 .. of a sequence with these caches of the layer (latents: K alone)
 constexpr int ROW_SEGS = 32;
 struct RowSeg { int row0, n, pos0, s_max, zero_to; void* K; void* VT; };
-struct RowSegs { int n; RowSeg s[ROW_SEGS]; };
+struct RowSegs { int n; RowSeg s[ROW_SEGS]; int end[ROW_SEGS]; };      // end[i]: blocks of a launch up to segment i's last (row_segs_blocks); past the n-th there are none
+// Launches over segments have the workgroups that the segments need, one behind the other (longest x segments would be 32768 of attention for one prompt of 2000 rows beside 31 of 30, of
+// which 2016 have rows): blocks(segment) of each -> their sum
+template <typename F> inline int row_segs_blocks(RowSegs& g, F&& blocks) {
+    int sum = 0;
+    for (int i = 0; i < ROW_SEGS; ++i) g.end[i] = i < g.n ? (sum += blocks(g.s[i])) : INT_MAX;
+    return sum;
+}
+// segment of a block, which becomes the block of that segment.  The sign of each difference (a comparison is twice the scalar instructions)
+__host__ __device__ inline int row_segs_at(const RowSegs& g, int& block) {
+    int i = ROW_SEGS - 1;
+#pragma unroll
+    for (int k = 0; k < ROW_SEGS - 1; ++k) i += (block - g.end[k]) >> 31;
+    block -= i ? g.end[i - 1] : 0;
+    return i;
+}
 struct FlashArgs {
     const void* Q;      // [q_len rows][q_stride] ; head h at column h*D
     void* O;            // [q_len rows][o_stride] ; head h at column h*D
@@ -140,6 +156,8 @@ struct FlashArgs {
 void launch_flash_prefill(int dtype, int D, const FlashArgs& a, hipStream_t st);
 // the windowed form over the rows of several sequences: Q, O and gate are row 0 of the piece; lengths, positions and caches are the segments'
 void launch_flash_segs(int dtype, int D, const FlashArgs& a, const RowSegs& g, hipStream_t st);
+struct FlashSegsPlan { int rows, blocks; };      // query rows of a workgroup, workgroups
+FlashSegsPlan flash_segs_plan(int D, int n_heads, RowSegs& g);      // puts the segments into the launch's order
 
 struct DecodeAttnArgs {
     const void* Q;         // [n_rows][q_stride]; head h at h*D  (already rotated)

@@ -213,9 +213,9 @@ void launch_residual_norm(int dtype, const ResidualNormArgs& a, int rows, hipStr
 // V^T behind the last row is cleared to the end of its 64 keys (or to zero_to).
 // ---------------------------------------------------------------------------------------------------------------
 template <typename T, int D, bool PAIRED>
-__device__ __forceinline__ void qkv_norm_rope_body(const QkvNormRopeArgs& a, char* smem) {
+__device__ __forceinline__ void qkv_norm_rope_body(const QkvNormRopeArgs& a, const int block, char* smem) {
     const int tid = threadIdx.x;
-    const int tok0 = blockIdx.x * 64, slot = blockIdx.y;
+    const int tok0 = block * 64, slot = blockIdx.y;
     const int ntok = (a.T - tok0) < 64 ? (a.T - tok0) : 64;                // <= 0: a block of nothing but rows to clear
     const int nzero = (a.zero_to - tok0) < 64 ? (a.zero_to - tok0) : 64;
     T* qkv = reinterpret_cast<T*>(a.qkv);
@@ -343,34 +343,32 @@ __device__ __forceinline__ void qkv_norm_rope_body(const QkvNormRopeArgs& a, cha
 template <typename T, int D, bool PAIRED>
 __global__ __launch_bounds__(256) void qkv_norm_rope_kv_kernel(QkvNormRopeArgs a) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    qkv_norm_rope_body<T, D, PAIRED>(a, smem);
+    qkv_norm_rope_body<T, D, PAIRED>(a, blockIdx.x, smem);
 }
 
-// blockIdx.z: the segment
 template <typename T, int D>
 __global__ __launch_bounds__(256) void qkv_norm_rope_segs_kernel(QkvNormRopeArgs a, RowSegs g) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    const RowSeg& s = g.s[blockIdx.z];
-    if ((int)blockIdx.x * 64 >= (s.zero_to > s.n ? s.zero_to : s.n)) return;
+    int block = blockIdx.x;
+    const RowSeg& s = g.s[row_segs_at(g, block)];
     a.qkv = reinterpret_cast<T*>(a.qkv) + (size_t)s.row0 * a.qkv_stride;
     a.K = s.K; a.VT = s.VT; a.T = s.n; a.pos0 = s.pos0; a.s_max = s.s_max; a.zero_to = s.zero_to;
-    qkv_norm_rope_body<T, D, true>(a, smem);
+    qkv_norm_rope_body<T, D, true>(a, block, smem);
 }
 
-void launch_qkv_norm_rope_segs(int dtype, int D, const QkvNormRopeArgs& a, const RowSegs& g, hipStream_t st) {
+void launch_qkv_norm_rope_segs(int dtype, int D, const QkvNormRopeArgs& a, const RowSegs& segs, hipStream_t st) {
+    RowSegs g = segs;
     LMX_REQUIRE(D == 64 || D == 128 || D == 256, "qkv_norm_rope_kv: padded head width must be 64, 128 or 256");
     LMX_REQUIRE(a.qkv && a.qkv_stride % 8 == 0 && a.qkv_stride >= (a.n_heads + 2 * a.n_kv_heads) * D, "qkv_norm_rope_kv: bad row pitch");
     LMX_REQUIRE(a.rot_dims % 16 == 0 && a.rot_dims <= a.qk_dim && a.qk_dim <= D && (a.rot_dims == 0 || a.cos_sin), "qkv_norm_rope_kv: bad rotation");
     LMX_REQUIRE(g.n >= 0 && g.n <= ROW_SEGS, "qkv_norm_rope_kv: too many segments");
-    int most = 0;
     for (int i = 0; i < g.n; ++i) {
         const RowSeg& s = g.s[i];
         LMX_REQUIRE(s.K && s.VT && s.n >= 1 && s.row0 >= 0 && s.pos0 >= 0 && s.pos0 + s.n <= s.s_max && s.pos0 + s.zero_to <= s.s_max, "qkv_norm_rope_kv: rows past the cache");
         LMX_REQUIRE(s.zero_to == 0 || a.n_heads == 0, "qkv_norm_rope_kv: clearing is for key / value rows");
-        most = std::max(most, std::max(s.n, s.zero_to));
     }
     if (g.n == 0) return;
-    const dim3 grid(cdiv(most, 64), a.n_heads + 2 * a.n_kv_heads, g.n);
+    const dim3 grid(row_segs_blocks(g, [](const RowSeg& s) { return cdiv(std::max(s.n, s.zero_to), 64); }), a.n_heads + 2 * a.n_kv_heads);
     const size_t smem = (size_t)64 * (D + 2) * dtype_size(dtype);
 #define L(TT, DD) do {                                                                                                                   \
         auto kern = qkv_norm_rope_segs_kernel<TT, DD>;                                                                                   \

@@ -14,7 +14,9 @@
 //   (HBM-bound KV streaming) and as the fp32 verification-mode attention for whole prompts.
 #include <algorithm>
 #include <cstdlib>
+#include <functional>
 #include <type_traits>
+#include <vector>
 #include "common.h"
 #include "kernels.h"
 #include "attention_decode.h"
@@ -399,7 +401,7 @@ __global__ __launch_bounds__((FlashShape<D, RW>::THREADS), D == 64 && !WIN ? 4 :
 }
 
 // Bound: a launch of one short prompt leaves most CUs idle.  32 prompts of 29 .. 64 rows, 32 heads: 8.4 us each, 268 in all -> 19.2 together; three of 1100, 894
-// and 688, 16 heads: 54 -> 29
+// and 688, 16 heads: 54 -> 29 (64-row blocks; the larger ones, flash_segs_wide, were not timed in this launch)
 template <typename T, int D, int RW>
 __global__ __launch_bounds__((FlashShape<D, RW>::THREADS), 2) void flash_segs_kernel(FlashArgs a, RowSegs g) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -518,9 +520,29 @@ void launch_flash_prefill(int dtype, int D, const FlashArgs& a, hipStream_t st) 
     }
 }
 
+// Which query blocks of several prompts' rows, D = 128: 128 rows as flash_wide has it, all blocks taken as heaviest first, and only where their partly empty rows cost less than the smaller
+// blocks do.  With the chip full those take 1.08 times as long for the same tiles (flash_wide's last two figures: 55.8 us for 528 x 32 tiles of 64 x 64 against 52.9 for 544 x 32, 172 against
+// 159 for equally many).  That holds for a few long prompts, 2 x 2048 rows of 32 heads, not for 4 x 900 (142 against 120) nor for 32 of 64.
+static bool flash_segs_wide(int n_heads, int window, const RowSegs& g) {
+    std::vector<int> tiles;                                  // 64-key tiles of every block of 128 rows of a head
+    long all = 0, halves = 0;                                // of these, and of the blocks of 64 rows
+    for (int i = 0; i < g.n; ++i) {
+        const RowSeg& s = g.s[i];
+        auto keys = [&](int r0, int rows) { return cdiv(s.pos0 + std::min(r0 + rows, s.n), FA_KT) - (window > 0 ? std::max(0, s.pos0 + r0 - window + 1) / FA_KT : 0); };
+        for (int r = 0; r < s.n; r += 128) { tiles.push_back(keys(r, 128)); all += tiles.back(); }
+        for (int r = 0; r < s.n; r += 64) halves += keys(r, 64);
+    }
+    const long blocks = (long)tiles.size() * n_heads;
+    if (blocks < 256 || 2.0 * all > 1.08 * halves) return false;
+    if (blocks > 512) return true;
+    std::sort(tiles.begin(), tiles.end(), std::greater<int>());
+    auto nth = [&](long i) { return i < blocks ? tiles[(size_t)(i / n_heads)] : 0; };
+    return (double)all * n_heads >= 0.9 * 256 * std::max(nth(0), nth(255) + nth(256));
+}
+
 // the segments with the most keys first, as a segment's own blocks go: a long prompt that the caller names last does not begin last
-FlashSegsPlan flash_segs_plan(int D, int n_heads, RowSegs& g) {
-    const int rows = D == 128 ? 64 : 128;
+FlashSegsPlan flash_segs_plan(int D, int n_heads, int window, RowSegs& g) {
+    const int rows = D == 64 || flash_segs_wide(n_heads, window, g) ? 128 : 64;
     std::stable_sort(g.s, g.s + g.n, [](const RowSeg& x, const RowSeg& y) { return x.pos0 + x.n > y.pos0 + y.n; });
     return {rows, row_segs_blocks(g, [&](const RowSeg& s) { return cdiv(s.n, rows) * n_heads; })};
 }
@@ -537,7 +559,7 @@ void launch_flash_segs(int dtype, int D, const FlashArgs& a, const RowSegs& segs
         LMX_REQUIRE(s.K && s.VT && s.n >= 1 && s.row0 >= 0 && s.pos0 >= 0 && s.s_max % 64 == 0 && s.pos0 + s.n <= s.s_max, "flash segments: bad lengths");
     }
     if (g.n == 0) return;
-    const FlashSegsPlan plan = flash_segs_plan(D, a.n_heads, g);
+    const FlashSegsPlan plan = flash_segs_plan(D, a.n_heads, a.window, g);
 #define L(TT, DD, RW) do {                                                                                                               \
         using SH = FlashShape<DD, RW>;                                                                                                   \
         auto kern = flash_segs_kernel<TT, DD, RW>;                                                                                       \
@@ -545,7 +567,7 @@ void launch_flash_segs(int dtype, int D, const FlashArgs& a, const RowSegs& segs
         if (!attr_set) { LMX_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, SH::LDS)); attr_set = true; } \
         hipLaunchKernelGGL(kern, dim3(plan.blocks), dim3(SH::THREADS), SH::LDS, st, a, g);                                                \
     } while (0)
-#define LD(TT) do { if (D == 128) L(TT, 128, 2); else L(TT, 64, 4); } while (0)
+#define LD(TT) do { if (D == 64) L(TT, 64, 4); else if (plan.rows == 128) L(TT, 128, 4); else L(TT, 128, 2); } while (0)
     if (dtype == kBF16) LD(bf16_t); else LD(f16_t);
 #undef LD
 #undef L

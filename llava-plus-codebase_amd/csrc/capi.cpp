@@ -716,21 +716,33 @@ int lmx_op_window_attn(int32_t dtype, int32_t D, const void* q, int32_t q_stride
     if (rows_form || dtype == kF32 || D > 128) launch_rows_attn(dtype, D, a, S(stream)); else launch_flash_prefill(dtype, D, a, S(stream));
     LMX_API_END
 }
-int lmx_op_flash_segs_plan(int32_t D, int32_t n_heads, int32_t n, const int32_t* lens, const int32_t* pos0, int32_t* form, int32_t* blocks, int32_t cap) {
+int lmx_op_flash_segs_plan(int32_t D, int32_t n_heads, int32_t window, int32_t n, const int32_t* lens, const int32_t* pos0, int32_t* form, int32_t* blocks, int32_t cap) {
     LMX_API_BEGIN
-    LMX_REQUIRE((D == 64 || D == 128) && n_heads >= 1 && n >= 1 && n <= ROW_SEGS && lens && pos0 && form && (blocks || cap <= 0), "flash_segs_plan: bad arguments");
+    LMX_REQUIRE((D == 64 || D == 128) && n_heads >= 1 && window >= 0 && n >= 1 && n <= ROW_SEGS && lens && pos0 && form && (blocks || cap <= 0), "flash_segs_plan: bad arguments");
     RowSegs g{};
     g.n = n;
     for (int i = 0; i < n; ++i) {
         LMX_REQUIRE(lens[i] >= 1 && pos0[i] >= 0, "flash_segs_plan: bad lengths");
         g.s[i].row0 = i; g.s[i].n = lens[i]; g.s[i].pos0 = pos0[i];
     }
-    const FlashSegsPlan p = flash_segs_plan(D, n_heads, g);
+    const FlashSegsPlan p = flash_segs_plan(D, n_heads, window, g);
     form[0] = p.rows; form[1] = p.blocks;
     for (int b = 0; b < p.blocks && b < cap; ++b) {
         int at = b;
         blocks[2 * b] = g.s[row_segs_at(g, at)].row0; blocks[2 * b + 1] = at;
     }
+    LMX_API_END
+}
+int lmx_op_window_attn_segs(int32_t dtype, int32_t D, const void* q, int32_t q_stride, void* o, int32_t o_stride, int32_t n, const int32_t* lens, const int32_t* pos0, void* const* kcaches,
+                            void* const* vtcaches, int32_t n_heads, int32_t n_kv_heads, int32_t s_max, float scale, int32_t window, int32_t sink, const void* gate, void* stream) {
+    LMX_API_BEGIN
+    LMX_REQUIRE(q && o && n >= 1 && n <= ROW_SEGS && lens && pos0 && kcaches && vtcaches && n_heads >= 1 && n_kv_heads >= 1 && n_heads % n_kv_heads == 0, "window_attn_segs: bad arguments");
+    RowSegs g{};
+    g.n = n;
+    for (int i = 0, row0 = 0; i < n; row0 += lens[i++]) g.s[i] = RowSeg{row0, lens[i], pos0[i], s_max, 0, kcaches[i], vtcaches[i]};
+    FlashArgs a{q, o, nullptr, nullptr, 0, 0, 0, q_stride, o_stride, n_heads, n_kv_heads, s_max, scale, 1};
+    a.win = 1; a.window = window; a.sink = sink; a.gate = gate;
+    launch_flash_segs(dtype, D, a, g, S(stream));
     LMX_API_END
 }
 int lmx_op_decode_win_waves(int32_t dtype, int32_t D, const void* qkv, int32_t qkv_stride, void* out, int32_t out_stride, void* const* kcaches, void* const* vtcaches,

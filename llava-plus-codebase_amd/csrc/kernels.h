@@ -157,7 +157,7 @@ void launch_flash_prefill(int dtype, int D, const FlashArgs& a, hipStream_t st);
 // the windowed form over the rows of several sequences: Q, O and gate are row 0 of the piece; lengths, positions and caches are the segments'
 void launch_flash_segs(int dtype, int D, const FlashArgs& a, const RowSegs& g, hipStream_t st);
 struct FlashSegsPlan { int rows, blocks; };      // query rows of a workgroup, workgroups
-FlashSegsPlan flash_segs_plan(int D, int n_heads, RowSegs& g);      // puts the segments into the launch's order
+FlashSegsPlan flash_segs_plan(int D, int n_heads, int window, RowSegs& g);      // puts the segments into the launch's order
 
 struct DecodeAttnArgs {
     const void* Q;         // [n_rows][q_stride]; head h at h*D  (already rotated)

@@ -266,6 +266,30 @@ def window_attn(qkv, kcache, vtcache, q_pos0, n_heads, n_kv_heads, scale, window
     return out
 
 
+def flash_segs_plan(lens, pos0, n_heads, D, window=0):
+    """(query rows of a workgroup, [(sequence, its workgroup)]) of window_attn_segs.  No GPU needed."""
+    import ctypes
+    n, cap = len(lens), sum(-(-k // 64) for k in lens) * n_heads
+    form, out = (ctypes.c_int32 * 2)(), (ctypes.c_int32 * (2 * cap))()
+    check(lib.lmx_op_flash_segs_plan(D, n_heads, window, n, (ctypes.c_int32 * n)(*lens), (ctypes.c_int32 * n)(*pos0), form, out, cap), "flash_segs_plan")
+    return form[0], [(out[2 * b], out[2 * b + 1]) for b in range(form[1])]
+
+
+def window_attn_segs(qkv, lens, pos0, kcaches, vtcaches, n_heads, n_kv_heads, scale, window=0, sink=True, gate_off=-1):
+    """window_attn of the rows of several sequences, one behind the other in qkv, in one launch."""
+    import ctypes
+    _need_cuda(qkv, *kcaches, *vtcaches)
+    n, D, s_max = len(lens), kcaches[0].shape[2], kcaches[0].shape[1]
+    if sum(lens) != qkv.shape[0] or len(pos0) != n or len(kcaches) != n or len(vtcaches) != n or any(k.shape[1] != s_max for k in kcaches):
+        raise ValueError("window_attn_segs: rows, positions and caches of every sequence")
+    out = torch.empty((qkv.shape[0], n_heads * D), dtype=qkv.dtype, device=qkv.device)
+    gate = None if gate_off < 0 else qkv.data_ptr() + gate_off * qkv.element_size()
+    pp = lambda xs: (ctypes.c_void_p * n)(*[x.data_ptr() for x in xs])  # noqa: E731
+    check(lib.lmx_op_window_attn_segs(torch_dtype_code(qkv.dtype), D, ptr(qkv), qkv.stride(0), ptr(out), out.stride(0), n, (ctypes.c_int32 * n)(*lens), (ctypes.c_int32 * n)(*pos0), pp(kcaches),
+                                      pp(vtcaches), n_heads, n_kv_heads, s_max, scale, window, int(sink), gate, stream_handle()), "window_attn_segs")
+    return out
+
+
 def decode_win(qkv, kcaches, vtcaches, pos_words, cos_sin, n_heads, n_kv_heads, qk_dim, rot_dims, scale, eps, q_norm=None, k_norm=None, window=0, sink=True, gate_off=-1, n_split=1, waves=4):
     """One new token per sequence (row i of qkv, pre-norm, pre-rotation): append to cache i at its position word, windowed attention.  waves: of a workgroup of the grouped kernel, 4 or 8.
     Returns [n_seq, n_heads * D]."""

@@ -80,3 +80,30 @@ def test_log_sum_exp_of_both_forms(cuda):
         i, j = torch.arange(T, device="cuda")[:, None] + ctx, torch.arange(T + ctx, device="cuda")[None]
         want = torch.logsumexp(s.masked_fill(j > i, -math.inf), -1) / math.log(2)
         assert (lse.double() - want).abs().max().item() < 2e-5 * want.abs().max().item()      # fp32: scores of 128 products, sums of up to 428 exponentials
+
+
+@pytest.mark.parametrize("name", DT)
+@pytest.mark.parametrize("lens,pos0,heads,D,window,rows", [
+    ([1, 65, 200, 31], [0, 63, 5, 300], 4, 128, 0, 64), ([40, 129, 64, 97], [10, 0, 190, 1], 8, 128, 33, 64), ([5, 130, 64], [70, 0, 1], 4, 64, 0, 128), ([63, 1], [2, 500], 4, 64, 100, 128),
+    ([128, 128], [700, 640], 256, 128, 0, 128), ([3, 256, 255], [8, 500, 450], 128, 128, 0, 128), ([128, 128], [1300, 1200], 256, 128, 1024, 128),
+])
+def test_rows_of_several_sequences(cuda, name, lens, pos0, heads, D, window, rows):
+    """Both forms, sequences out of order and of unlike length, gates and a sink."""
+    from llava_mi355x import ops
+    dt, kv_heads = DT[name], heads // 4
+    assert ops.flash_segs_plan(lens, pos0, heads, D, window)[0] == rows
+    s_max = max((p + n + 63) // 64 * 64 for p, n in zip(pos0, lens))
+    g = torch.Generator(device="cuda").manual_seed(sum(lens) + heads)
+    rnd = lambda *shape: torch.empty(shape, dtype=dt, device="cuda").normal_(generator=g)  # noqa: E731
+    qkv = rnd(sum(lens), heads * D + (heads + 7) // 8 * 8)
+    ks, vts = [rnd(kv_heads, s_max, D) for _ in lens], [rnd(kv_heads, D, s_max) for _ in lens]
+    for vt, p, n in zip(vts, pos0, lens):
+        vt[:, :, p + n:] = 0
+    got = ops.window_attn_segs(qkv, lens, pos0, ks, vts, heads, kv_heads, D ** -0.5, window=window, sink=True, gate_off=heads * D)
+    at = 0
+    for n, p, k, vt in zip(lens, pos0, ks, vts):
+        r = slice(at, at + n)
+        gate = torch.sigmoid(qkv[r, heads * D:heads * D + heads].double()).repeat_interleave(D, 1)
+        want, absolute = dense(qkv[r, :heads * D].contiguous(), k[:, :p + n], vt[:, :, :p + n], heads, D ** -0.5, p, True, window, True)
+        near(got[r], want * gate, absolute * gate, dt)
+        at += n

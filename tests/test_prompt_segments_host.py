@@ -4,14 +4,9 @@ import ctypes
 import pytest
 
 
-def plan(lens, heads, D=128, pos0=None):
-    """(query rows of a workgroup, [(sequence, its workgroup)])"""
-    from llava_mi355x import _C
-    n, cap = len(lens), sum(-(-k // 64) for k in lens) * heads + 1
-    form, out = (ctypes.c_int32 * 2)(), (ctypes.c_int32 * (2 * cap))()
-    _C.check(_C.lib.lmx_op_flash_segs_plan(D, heads, n, (ctypes.c_int32 * n)(*lens), (ctypes.c_int32 * n)(*(pos0 or [0] * n)), form, out, cap))
-    assert form[1] < cap
-    return form[0], [(out[2 * b], out[2 * b + 1]) for b in range(form[1])]
+def plan(lens, heads, D=128, pos0=None, window=0):
+    from llava_mi355x import ops
+    return ops.flash_segs_plan(lens, pos0 or [0] * len(lens), heads, D, window)
 
 
 @pytest.mark.parametrize("D", [64, 128])
@@ -28,9 +23,22 @@ def test_most_keys_first():
     assert order([30, 200, 64], [900, 0, 136]) == [0, 1, 2]      # 930, 200 and 200 keys: equal ones as they come
 
 
+@pytest.mark.parametrize("lens,pos0,heads,window,rows", [
+    ([2048, 2048], None, 32, 0, 128), ([30] * 31 + [4096], None, 32, 0, 128), ([128, 128], [700, 640], 256, 0, 128), ([2048, 2048], None, 32, 1024, 128),      # the chip full of whole blocks
+    ([900] * 4, None, 32, 0, 64), ([64] * 32, None, 32, 0, 64), ([129, 129], [900, 900], 256, 0, 64),                                                          # full, but of rows that are none
+    ([1100, 894, 688], None, 16, 0, 64), ([128, 128], [700, 100], 140, 0, 64), ([2048, 30], None, 15, 0, 64),                                                   # CUs without work, blocks of unlike length
+])
+def test_larger_blocks_where_they_fill_the_chip(lens, pos0, heads, window, rows):
+    assert plan(lens, heads, 128, pos0, window)[0] == rows
+
+
+def test_the_narrow_heads_have_one_form():
+    assert plan([1], 1, 64)[0] == plan([2048, 2048], 32, 64)[0] == 128
+
+
 @pytest.mark.parametrize("lens,heads,D", [([], 4, 128), ([1] * 33, 4, 128), ([0], 4, 128), ([5], 0, 128), ([5], 4, 256)])
 def test_bad_arguments_raise(lens, heads, D):
     from llava_mi355x import _C
     n = len(lens)
     with pytest.raises(_C.LmxError):
-        _C.check(_C.lib.lmx_op_flash_segs_plan(D, heads, n, (ctypes.c_int32 * 33)(*lens), (ctypes.c_int32 * 33)(), (ctypes.c_int32 * 2)(), None, 0))
+        _C.check(_C.lib.lmx_op_flash_segs_plan(D, heads, 0, n, (ctypes.c_int32 * 33)(*lens), (ctypes.c_int32 * 33)(), (ctypes.c_int32 * 2)(), None, 0))

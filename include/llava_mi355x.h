@@ -390,6 +390,8 @@ int lmx_op_window_attn(int32_t dtype, int32_t D, const void* q, int32_t q_stride
 /* the attention launch over the rows of n (1 .. 32) sequences, lens[i] new rows behind pos0[i] cached ones, on the host alone: form[2] = {query rows of a workgroup, workgroups};
  * blocks[2 b] = {sequence of workgroup b, its workgroup of that sequence} for the first cap of them */
 int lmx_op_flash_segs_plan(int32_t D, int32_t n_heads, int32_t window, int32_t n, const int32_t* lens, const int32_t* pos0, int32_t* form, int32_t* blocks, int32_t cap);
+/* what a latent layer's prompt rows take of a sequence's workspace, on the host alone: `rows` rows of n_seq sequences in one call, the longest context `keys` (0: bad arguments) */
+size_t lmx_op_latent_scratch_bytes(int32_t dtype, int32_t heads_width, int32_t latent_width, int32_t window, int32_t rows, int32_t keys, int32_t n_seq);
 /* that launch: lmx_op_window_attn over the rows of n sequences, one behind the other in q, gate and o (16-bit types; lens, pos0 and the lists of caches are host arrays) */
 int lmx_op_window_attn_segs(int32_t dtype, int32_t D, const void* q, int32_t q_stride, void* o, int32_t o_stride, int32_t n, const int32_t* lens, const int32_t* pos0, void* const* kcaches,
                             void* const* vtcaches, int32_t n_heads, int32_t n_kv_heads, int32_t s_max, float scale, int32_t window, int32_t sink, const void* gate, void* stream);

@@ -733,6 +733,10 @@ int lmx_op_flash_segs_plan(int32_t D, int32_t n_heads, int32_t window, int32_t n
     }
     LMX_API_END
 }
+size_t lmx_op_latent_scratch_bytes(int32_t dtype, int32_t heads_width, int32_t latent_width, int32_t window, int32_t rows, int32_t keys, int32_t n_seq) {
+    if (heads_width < 1 || latent_width < 1 || window < 0 || rows < 1 || keys < 1 || n_seq < 1 || (dtype != kF32 && dtype != kBF16 && dtype != kF16)) return 0;
+    return latent_prefill_scratch(heads_width, latent_width, (int)dtype_size(dtype), window, rows, keys, n_seq);
+}
 int lmx_op_window_attn_segs(int32_t dtype, int32_t D, const void* q, int32_t q_stride, void* o, int32_t o_stride, int32_t n, const int32_t* lens, const int32_t* pos0, void* const* kcaches,
                             void* const* vtcaches, int32_t n_heads, int32_t n_kv_heads, int32_t s_max, float scale, int32_t window, int32_t sink, const void* gate, void* stream) {
     LMX_API_BEGIN

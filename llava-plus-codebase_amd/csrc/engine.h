@@ -103,6 +103,9 @@ struct Batch;
 // memory a row, K rows too: 1/16 at 2048 keys and less above.  Shorter caches pay nothing: at 256 keys it would be half of their size again.
 inline int kv_row_pitch(int dtype, int s_max) { return s_max + (dtype != kF32 && s_max >= 2048 && s_max % 256 == 0 ? 128 : 0); }
 
+// scratch of a latent layer (an: its heads' width, R: the latents') over `rows` rows of n sequences, `keys` the longest context
+size_t latent_prefill_scratch(int an, int R, int es, int window, int rows, int keys, int n);
+
 struct Model {
     lmx_config cfg{};
     int es = 2;                 // element size

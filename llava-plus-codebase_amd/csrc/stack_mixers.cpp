@@ -47,18 +47,25 @@ static bool fresh_together(int dtype, int D, const std::vector<Model::Segment>& 
     return true;
 }
 
+// Rows whose keys and values are there at a time, of whole prompts: 8192 or the longest prompt (`keys` bounds it).  5 x their heads' width stands in scratch: 32 prompts of 2000 rows at 4096
+// would take 2.76 GB all at once, 0.92 so, and a product of 8192 rows fills the chip as well as one of 64000
+static int together_rows(int rows, int keys) { return std::min(rows, std::max(keys, 8192)); }
+
+size_t latent_prefill_scratch(int an, int R, int es, int window, int rows, int keys, int n) {
+    const int nk = window > 0 ? std::min(keys, rows + window + 64) : keys;
+    const size_t q = up256((size_t)rows * an * es), apart = q + up256((size_t)nk * 2 * an * es) + 2 * up256((size_t)round_up(nk, 128) * an * es);
+    if (n < 2) return apart;
+    const int t = together_rows(rows, keys);                 // fresh_together: latents of all rows, of t rows keys and values by row and caches of whole 128 keys each
+    return std::max(apart, q + up256((size_t)rows * R * es) + up256((size_t)t * 2 * an * es) + 2 * up256((size_t)(t + 127 * std::min(n, ROW_SEGS)) * an * es));
+}
+
 // scratch of the widest mixer; keys: longest context of the call, n: sequences
 size_t Model::stack_mix_scratch(int rows, int keys, int n) const {
     size_t most = 0;
     for (const StackLayer& l : stk->layers) {
         size_t b = 0;
-        if (l.c.mixer == LMX_MIXER_LATENT) {
-            const int nk = l.c.window > 0 ? std::min(keys, rows + l.c.window + 64) : keys;
-            b = up256((size_t)rows * l.an * es) + up256((size_t)nk * 2 * l.an * es) + 2 * up256((size_t)round_up(nk, 128) * l.an * es);
-            if (n > 1)                                       // together (fresh_together): latents and their keys and values by row, caches of whole 128 keys each
-                b = std::max(b, up256((size_t)rows * l.an * es) + up256((size_t)rows * l.R * es) + up256((size_t)rows * 2 * l.an * es) +
-                                    2 * up256((size_t)(rows + 127 * std::min(n, ROW_SEGS)) * l.an * es));
-        } else if (l.c.mixer == LMX_MIXER_DELTA) b = up256((size_t)rows * l.ds.H * (l.ds.DK + l.ds.DV) * es) + delta_scratch_bytes(l.ds, rows, es);
+        if (l.c.mixer == LMX_MIXER_LATENT) b = latent_prefill_scratch(l.an, l.R, es, l.c.window, rows, keys, n);
+        else if (l.c.mixer == LMX_MIXER_DELTA) b = up256((size_t)rows * l.ds.H * (l.ds.DK + l.ds.DV) * es) + delta_scratch_bytes(l.ds, rows, es);
         most = std::max(most, b);
     }
     return most;
@@ -102,20 +109,23 @@ void Model::stack_mix_prefill(int r, Seq* const* seqs, const std::vector<Segment
         return;
     }
     if (fresh_together(dt, l.D, seg)) {
-        // every key is a row of this piece: one product makes all keys and values
-        void* q = take((size_t)fill * l.an * es);
-        void* lat = take((size_t)fill * l.R * es);
-        char* kv = take((size_t)fill * 2 * l.an * es);
-        const size_t cache = (size_t)(fill + 127 * std::min((int)seg.size(), ROW_SEGS)) * l.an * es;
+        // every key is a row of this piece: one product makes the keys and values of many prompts
+        int longest = 0;
+        for (const Segment& g : seg) longest = std::max(longest, g.n);
+        const int most = together_rows(fill, longest);
+        char* q = take((size_t)fill * l.an * es);
+        char* lat = take((size_t)fill * l.R * es);
+        char* kv = take((size_t)most * 2 * l.an * es);
+        const size_t cache = (size_t)(most + 127 * std::min((int)seg.size(), ROW_SEGS)) * l.an * es;
         char *kc = take(cache), *vt = take(cache);
-        auto groups = [&](auto&& f) {
-            for (size_t s0 = 0; s0 < seg.size(); s0 += ROW_SEGS) {
+        auto groups = [&](size_t s0, size_t end, auto&& f) {             // as many segments as a launch takes
+            for (; s0 < end; s0 += ROW_SEGS) {
                 RowSegs g{};
-                g.n = (int)std::min(seg.size() - s0, (size_t)ROW_SEGS);
+                g.n = (int)std::min(end - s0, (size_t)ROW_SEGS);
                 f(g, seg.data() + s0);
             }
         };
-        groups([&](RowSegs& g, const Segment* s) {
+        groups(0, seg.size(), [&](RowSegs& g, const Segment* s) {
             LMX_PROF("prefill.latent_norm");
             for (int i = 0; i < g.n; ++i) g.s[i] = RowSeg{s[i].dst0, s[i].n, 0, s_max, 0, seqs[s[i].seq]->kc.as<char>() + run.k_off, nullptr};
             LatentNormArgs n{qkv, l.qkv_n, l.Q, d.q_rank, l.R, d.kv_rank, l.qn_lat, l.kn_lat, nullptr, 0};
@@ -123,23 +133,28 @@ void Model::stack_mix_prefill(int r, Seq* const* seqs, const std::vector<Segment
             launch_latent_norm_segs(dt, n, g, st);
         });
         gemm("prefill.gemm.uq", GemmArgs{qkv, l.wuq, q, nullptr, nullptr, fill, l.an, l.Q, l.qkv_n, l.Q, l.an, 0, kActNone});
-        gemm("prefill.gemm.ukv", GemmArgs{lat, l.wukv, kv, nullptr, nullptr, fill, 2 * l.an, l.R, l.R, l.R, 2 * l.an, 0, kActNone});
-        groups([&](RowSegs& g, const Segment* s) {
-            size_t at = 0;
-            for (int i = 0; i < g.n; ++i) {
-                const int cap = round_up(s[i].n, 128);
-                g.s[i] = RowSeg{s[i].dst0, s[i].n, 0, cap, cap, kc + at, vt + at};      // the attention tiles are whole: what lies behind the last key must not be NaN bits
-                at += (size_t)cap * l.an * es;
-            }
-            {
-                LMX_PROF("prefill.kv_rows");
-                launch_qkv_norm_rope_segs(dt, l.D, QkvNormRopeArgs{kv, nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, 2 * l.an, 0, d.n_heads, 0, l.D, 0, S.c.norm_eps}, g, st);
-            }
-            LMX_PROF("prefill.attn");
-            FlashArgs fa{q, mix, nullptr, nullptr, 0, 0, 0, l.an, l.out_k, d.n_heads, d.n_heads, 0, d.attn_scale, 1};
-            fa.win = 1; fa.window = d.window; fa.sink = d.softmax_sink;
-            launch_flash_segs(dt, l.D, fa, g, st);
-        });
+        for (size_t s0 = 0, s1; s0 < seg.size(); s0 = s1) {
+            const int first = seg[s0].dst0;
+            int rows = 0;
+            for (s1 = s0; s1 < seg.size() && rows + seg[s1].n <= most; ++s1) rows += seg[s1].n;
+            gemm("prefill.gemm.ukv", GemmArgs{lat + (size_t)first * l.R * es, l.wukv, kv, nullptr, nullptr, rows, 2 * l.an, l.R, l.R, l.R, 2 * l.an, 0, kActNone});
+            groups(s0, s1, [&](RowSegs& g, const Segment* s) {
+                size_t at = 0;
+                for (int i = 0; i < g.n; ++i) {
+                    const int cap = round_up(s[i].n, 128);
+                    g.s[i] = RowSeg{s[i].dst0 - first, s[i].n, 0, cap, cap, kc + at, vt + at};      // the attention tiles are whole: what lies behind the last key must not be NaN bits
+                    at += (size_t)cap * l.an * es;
+                }
+                {
+                    LMX_PROF("prefill.kv_rows");
+                    launch_qkv_norm_rope_segs(dt, l.D, QkvNormRopeArgs{kv, nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, 2 * l.an, 0, d.n_heads, 0, l.D, 0, S.c.norm_eps}, g, st);
+                }
+                LMX_PROF("prefill.attn");
+                FlashArgs fa{q + (size_t)first * l.an * es, static_cast<char*>(mix) + (size_t)first * l.out_k * es, nullptr, nullptr, 0, 0, 0, l.an, l.out_k, d.n_heads, d.n_heads, 0, d.attn_scale, 1};
+                fa.win = 1; fa.window = d.window; fa.sink = d.softmax_sink;
+                launch_flash_segs(dt, l.D, fa, g, st);
+            });
+        }
         return;
     }
     // latent attention: latents into the cache, queries, then per segment the keys and values its rows can see

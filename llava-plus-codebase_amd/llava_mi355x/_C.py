@@ -159,6 +159,7 @@ _SIGS = {
     "lmx_op_qkv_norm_rope_kv": (c_int32, [c_int32, c_int32, c_void_p, c_int32] + [c_void_p] * 5 + [c_int32] * 7 + [c_float, c_void_p]),
     "lmx_op_window_attn": (c_int32, [c_int32, c_int32, c_void_p, c_int32, c_void_p, c_int32, c_void_p, c_void_p] + [c_int32] * 5 + [c_float, c_int32, c_int32, c_void_p, c_int32, c_void_p]),
     "lmx_op_flash_segs_plan": (c_int32, [c_int32] * 4 + [POINTER(c_int32)] * 4 + [c_int32]),
+    "lmx_op_latent_scratch_bytes": (c_size_t, [c_int32] * 7),
     "lmx_op_window_attn_segs": (c_int32, [c_int32, c_int32, c_void_p, c_int32, c_void_p, c_int32, c_int32] + [POINTER(c_int32)] * 2 + [POINTER(c_void_p)] * 2 + [c_int32] * 3 + [c_float, c_int32, c_int32, c_void_p, c_void_p]),
     "lmx_op_decode_win": (c_int32, [c_int32, c_int32, c_void_p, c_int32, c_void_p, c_int32] + [POINTER(c_void_p)] * 5 + [c_int32] + [c_void_p] * 4 + [c_int32] * 9 + [c_float, c_float, c_void_p]),
     "lmx_op_decode_win_waves": (c_int32, [c_int32, c_int32, c_void_p, c_int32, c_void_p, c_int32] + [POINTER(c_void_p)] * 5 + [c_int32] + [c_void_p] * 4 + [c_int32] * 9 + [c_float, c_float, c_int32, c_void_p]),

@@ -65,3 +65,17 @@ def test_chosen_rows_of_several_sequences(cuda, dt):
     assert max(siterax.rel(g, o[c]) for g, o, c in zip(got, oracle, chosen)) < siterax.TOL[dt]
     for c in caches:
         c.close()
+
+
+@pytest.mark.parametrize("name", ["plain", "mixed"])
+def test_more_rows_than_the_latents_expand_at_once(cuda, name):
+    """9000 rows of new prompts: the first 20 of them together, the 21st would pass 8192 rows."""
+    from llava_mi355x.engine_lm import LmxKVCache
+    m = vizosun.model(name, "bf16")
+    n = [400] * 20 + [300, 390, 310]
+    ts = [vizosun.tokens(name, k, 700 + i) for i, k in enumerate(n)]
+    caches = [LmxKVCache(m, 1) for _ in ts]
+    rows = read(m, caches, ts)
+    for c in caches:
+        c.close()
+    assert max(vizosun.rel(rows[i], vizosun.oracle(name, ts[i], "bf16")) for i in (0, 19, 20, 21, 22)) < vizosun.TOL["bf16"]

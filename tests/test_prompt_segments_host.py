@@ -1,4 +1,5 @@
-"""Workgroups of the launches over the rows of several sequences (csrc/kernels.h: row_segs_at, csrc/attention.hip: flash_segs_plan), asked of the library on the host."""
+"""Workgroups of the launches over the rows of several sequences (csrc/kernels.h: row_segs_at, csrc/attention.hip: flash_segs_plan) and the scratch of their latent layers
+(csrc/stack_mixers.cpp: latent_prefill_scratch), asked of the library on the host."""
 import ctypes
 
 import pytest
@@ -42,3 +43,18 @@ def test_bad_arguments_raise(lens, heads, D):
     n = len(lens)
     with pytest.raises(_C.LmxError):
         _C.check(_C.lib.lmx_op_flash_segs_plan(D, heads, 0, n, (ctypes.c_int32 * 33)(*lens), (ctypes.c_int32 * 33)(), (ctypes.c_int32 * 2)(), None, 0))
+
+
+@pytest.mark.parametrize("width,latent,window", [(4096, 512, 0), (2048, 256, 1024)])
+def test_latent_scratch_of_many_rows(width, latent, window):
+    """Queries and latents of all rows; keys and values, by row and in caches, of 8192 rows or of the longest prompt."""
+    from llava_mi355x import _C
+    size = lambda rows, keys, n: _C.lib.lmx_op_latent_scratch_bytes(_C.DTYPE_BF16, width, latent, window, rows, keys, n)  # noqa: E731
+    row = lambda w: w * 2  # noqa: E731
+    for prompts, n in ((2000, 32), (300, 200), (64, 32), (20000, 2)):
+        rows, apart = prompts * n, max(8192, prompts)
+        assert size(rows, prompts, n) <= rows * row(width + latent) + (2 * apart + 2 * (apart + 127 * 32)) * row(width) + 5 * 256
+        assert size(rows, prompts, n) >= rows * row(width)
+    assert size(2000, 2000, 1) <= 2000 * row(width) + (2 * 2000 + 2 * 2048) * row(width) + 5 * 256      # a prompt alone
+    assert size(0, 1, 1) == size(1, 0, 1) == size(1, 1, 0) == 0
+

@@ -129,7 +129,9 @@ __device__ __forceinline__ void flash_body(const FlashArgs& a, const int block, 
     const int my_pos = a.q_pos0 + qrow;                   // causal limit of this lane's row
 
     // ---- K / Vᵀ tiles by LDS-DMA into a ring of two rounds (inline asm: see gemm_pipe_kernel for why) -----------------------
-    // per-lane source offsets (bytes) inside a tile; the swizzle lives in the SOURCE address, the LDS image is lane-linear
+    // per-lane source offsets (bytes) inside a tile; the swizzle lives in the SOURCE address, the LDS image is lane-linear.
+    // Vᵀ tile in LDS: [D rows][KT keys], KT / 8 chunks of 16 bytes (8 keys) a row, chunk c of row r at c ^ (r >> 1) (64 keys) or c ^ (r >> 2) (32 keys) in the chunk's bits: a product of
+    // probabilities reads whole chunks, the keys of a 32-key block being fed to QKᵀ in the order fa_key_perm, and the 16 lanes of every ds_read_b128 service group hit 16 distinct slots
     uint32_t ksrc[KPPW], vsrc[VPPW];
 #pragma unroll
     for (int i = 0; i < KPPW; ++i) {
@@ -172,7 +174,7 @@ __device__ __forceinline__ void flash_body(const FlashArgs& a, const int block, 
     auto v_frag = [&](int ring, int f) { return *reinterpret_cast<const uint4*>(smem + ((ring + v_lane) ^ ((f / DB) << 5)) + (f % DB) * 64 * KT); };
     auto scores = [&](f32x16 (&s)[KB], int f, const uint4& kf) { s[f % KB] = Mfma32<T>::run(kf, qf[f / KB], f < KB ? f32x16{} : s[f % KB]); };
 
-    // s[kb][r] = score of key = tile * 64 + kb * 32 + 16 (r >> 3) + 8 hi + (r & 7) and row qrow, before the scale.  What a row does not see becomes -inf (masking only on tiles that
+    // s[kb][r] = score of key = tile * KT + kb * 32 + 16 (r >> 3) + 8 hi + (r & 7) and row qrow, before the scale.  What a row does not see becomes -inf (masking only on tiles that
     // can hold an invisible key for some row of this wave: a wave-uniform test); the running maximum follows.
     auto see = [&](f32x16 (&s)[KB], int t) {
         const int tile_first = (tile0 + t) * KT, tile_last = tile_first + KT - 1;

@@ -16,22 +16,17 @@ template <> struct Mfma32<f16_t> {
     }
 };
 
-constexpr int FA_KT = 64;      // keys per tile
+constexpr int FA_KT = 64;      // keys per tile (flash_body with 64 rows of 128: 32)
 // log2 units: skip the O rescale until a row max grows by more.  The probability that stands at the maximum is 1, which 16 bits hold exactly, others are rounded: a larger threshold leaves
 // the maximum behind in more rows.  1087 causal rows in bf16, relative error against 64 bits at 8 | 4 | 2 | 1 | 0: 2.039e-3 | 2.038e-3 | 2.003e-3 | 1.975e-3 | 1.968e-3, time 22.0 | 22.4 | 22.9 | 23.6 | 23.7 us
 constexpr float FA_DEFER = 2.f;
 
-// K tile in LDS: [64 keys][D] 16-bit; 16-byte chunks XOR-swizzled so a ds_read_b128 lane group (16 distinct rows,
+// K tile in LDS: [keys][D] 16-bit; 16-byte chunks XOR-swizzled so a ds_read_b128 lane group (16 distinct rows,
 // same logical chunk) touches 16 distinct 16-byte slots of the 256-byte bank row.
 template <int D> __device__ __forceinline__ int k_lds_off(int row, int chunk) {
     if constexpr (D == 128) return row * 256 + (((chunk ^ row) & 15) << 4);
     else return row * 128 + (((chunk ^ (row >> 1)) & 7) << 4);
 }
-// Vᵀ tile in LDS: [D rows][64 keys] = 128 bytes per row = 8 chunks of 16 bytes (8 keys), chunk c of row r stored at c ^ ((r >> 1) & 7): whole
-// 16-byte chunks, so the image can be written by LDS-DMA.
-// whole 16-byte chunk (8 keys) of a Vᵀ row: what a P·V fragment reads once the keys of a 32-key block are fed to QKᵀ in the order fa_key_perm — the 16
-// lanes of every ds_read_b128 service group then hit 16 distinct 16-byte slots (row & 1 picks the half of the 64 banks, (chunk ^ row >> 1) & 7 the slot)
-__device__ __forceinline__ int vt_lds_chunk(int row, int chunk) { return row * 128 + (((chunk ^ (row >> 1)) & 7) << 4); }
 // Key order inside a 32-key block.  The 32x32 accumulator of Sᵀ = K Qᵀ holds tile row (r & 3) + 8 (r >> 2) + 4 hi in register r of lane half hi, and the
 // P·V step (kb, s2) takes registers 8 s2 .. + 7 as its 8 k-values: with K fed in natural order those are keys {4 hi .. + 3} and {8 + 4 hi .. + 3} (+ 16 s2),
 // i.e. the Vᵀ operand needs TWO 8-byte LDS reads, 2-way bank-conflicted (1.46 M conflict cycles per launch in the counters).  Feeding K row pi(l31) =

@@ -63,12 +63,12 @@ __global__ __launch_bounds__(256) void latent_norm_segs_kernel(LatentNormArgs a,
 void launch_latent_norm_segs(int dtype, const LatentNormArgs& a, const RowSegs& segs, hipStream_t st) {
     RowSegs g = segs;
     LMX_REQUIRE(a.Q % 64 == 0 && a.R % 64 == 0 && a.q_n >= 1 && a.q_n <= a.Q && a.r_n >= 1 && a.r_n <= a.R && a.ld % 8 == 0 && a.ld >= a.Q + a.R, "latent_norm: bad widths");
-    LMX_REQUIRE(a.proj && a.q_w && a.r_w && g.n >= 0 && g.n <= ROW_SEGS, "latent_norm: bad arguments");
+    LMX_REQUIRE((dtype == kBF16 || dtype == kF16) && a.proj && a.q_w && a.r_w && g.n >= 0 && g.n <= ROW_SEGS, "latent_norm: bad arguments");
     for (int i = 0; i < g.n; ++i) LMX_REQUIRE(g.s[i].K && g.s[i].n >= 1 && g.s[i].row0 >= 0 && g.s[i].pos0 >= 0 && g.s[i].pos0 + g.s[i].n <= g.s[i].s_max, "latent_norm: bad cache rows");
     if (g.n == 0) return;
     const dim3 grid(row_segs_blocks(g, [](const RowSeg& s) { return s.n; }));
 #define L(TT) LMX_LAUNCH(latent_norm_segs_kernel<TT>, grid, dim3(256), 0, st, a, g)
-    if (dtype == kBF16) L(bf16_t); else if (dtype == kF16) L(f16_t); else L(float);
+    if (dtype == kBF16) L(bf16_t); else L(f16_t);
 #undef L
     LMX_CHECK_HIP(hipGetLastError());
 }

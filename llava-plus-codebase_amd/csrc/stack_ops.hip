@@ -358,7 +358,7 @@ __global__ __launch_bounds__(256) void qkv_norm_rope_segs_kernel(QkvNormRopeArgs
 
 void launch_qkv_norm_rope_segs(int dtype, int D, const QkvNormRopeArgs& a, const RowSegs& segs, hipStream_t st) {
     RowSegs g = segs;
-    LMX_REQUIRE(D == 64 || D == 128 || D == 256, "qkv_norm_rope_kv: padded head width must be 64, 128 or 256");
+    LMX_REQUIRE((dtype == kBF16 || dtype == kF16) && (D == 64 || D == 128), "qkv_norm_rope_kv: rows of several sequences are of 16 bits and padded to heads of 64 or 128");
     LMX_REQUIRE(a.qkv && a.qkv_stride % 8 == 0 && a.qkv_stride >= (a.n_heads + 2 * a.n_kv_heads) * D, "qkv_norm_rope_kv: bad row pitch");
     LMX_REQUIRE(a.rot_dims % 16 == 0 && a.rot_dims <= a.qk_dim && a.qk_dim <= D && (a.rot_dims == 0 || a.cos_sin), "qkv_norm_rope_kv: bad rotation");
     LMX_REQUIRE(g.n >= 0 && g.n <= ROW_SEGS, "qkv_norm_rope_kv: too many segments");
@@ -376,8 +376,8 @@ void launch_qkv_norm_rope_segs(int dtype, int D, const QkvNormRopeArgs& a, const
         if (!attr_set) { LMX_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024)); attr_set = true; } \
         hipLaunchKernelGGL(kern, grid, dim3(256), smem, st, a, g);                                                                       \
     } while (0)
-#define LD(TT) do { if (D == 256) L(TT, 256); else if (D == 128) L(TT, 128); else L(TT, 64); } while (0)
-    if (dtype == kBF16) LD(bf16_t); else if (dtype == kF16) LD(f16_t); else LD(float);
+#define LD(TT) do { if (D == 128) L(TT, 128); else L(TT, 64); } while (0)
+    if (dtype == kBF16) LD(bf16_t); else LD(f16_t);
 #undef LD
 #undef L
     LMX_CHECK_HIP(hipGetLastError());
@@ -999,7 +999,7 @@ void launch_decode_win(int dtype, int D, const WinDecodeArgs& a, bool grouped, b
     LMX_REQUIRE(a.n_heads >= 1 && a.n_kv_heads >= 1 && a.n_heads % a.n_kv_heads == 0 && a.qkv && a.out, "decode_win: bad arguments");
     LMX_REQUIRE(a.rot_dims % 2 == 0 && a.rot_dims <= a.qk_dim && a.qk_dim <= D && (a.rot_dims == 0 || a.cos_sin), "decode_win: bad rotation");
     LMX_REQUIRE(a.tab || (a.n_seq == 1 && a.one.K && a.one.VT && a.one.ws && a.one.counters && (a.pos >= 0 || a.one.pos_ptr)), "decode_win: bad sequence");
-    LMX_REQUIRE(!a.leave || (a.n_seq == 1 && !grouped), "decode_win: splits are left to the next launch by one sequence");
+    LMX_REQUIRE(!a.leave || (a.n_seq == 1 && !grouped && dtype != kF32), "decode_win: splits are left to the next launch by one sequence of a 16-bit model");
     if (grouped && decode_win_groups(dtype, D, a.n_heads, a.n_kv_heads, a.n_seq) && a.qkv_stride % 4 == 0 && reinterpret_cast<uintptr_t>(a.qkv) % 8 == 0) {
         const dim3 grid(a.n_kv_heads, a.n_split, a.n_seq);
         const int group = a.n_heads / a.n_kv_heads;
@@ -1020,9 +1020,11 @@ void launch_decode_win(int dtype, int D, const WinDecodeArgs& a, bool grouped, b
         return;
     }
     const dim3 grid(a.n_heads, a.n_split, a.n_seq);
-#define L(TT, DD) do { if (a.leave) LMX_LAUNCH((decode_win_kernel<TT, DD, true>), grid, dim3(256), 0, st, a); else LMX_LAUNCH((decode_win_kernel<TT, DD>), grid, dim3(256), 0, st, a); } while (0)
-#define LD(TT) do { if (D == 256) L(TT, 256); else if (D == 128) L(TT, 128); else L(TT, 64); } while (0)
-    if (dtype == kBF16) LD(bf16_t); else if (dtype == kF16) LD(f16_t); else LD(float);
+#define L(TT, DD, LV) LMX_LAUNCH((decode_win_kernel<TT, DD, LV>), grid, dim3(256), 0, st, a)
+#define LD(TT, LV) do { if (D == 256) L(TT, 256, LV); else if (D == 128) L(TT, 128, LV); else L(TT, 64, LV); } while (0)
+    if (dtype == kF32) LD(float, false);
+    else if (a.leave) { if (dtype == kBF16) LD(bf16_t, true); else LD(f16_t, true); }
+    else if (dtype == kBF16) LD(bf16_t, false); else LD(f16_t, false);
 #undef LD
 #undef L
     LMX_CHECK_HIP(hipGetLastError());

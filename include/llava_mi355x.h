@@ -382,6 +382,11 @@ int lmx_op_residual_norm(int32_t dtype, const float* x_in, const void* y, const 
 int lmx_op_residual_norm_form(int32_t dtype, int32_t rows, int32_t H, int32_t inject, int32_t* ahead);
 int lmx_op_gemv_residual(int32_t dtype, const float* x_in, const void* y, const void* post_w, const void* inject, const void* pre_w, float* x_out, const void* w, const void* bias,
                          void* c, int32_t N, int32_t H, int32_t H_real, float mult, float eps, int32_t act, void* stream);
+/* w [N][n_heads D] behind an attention of one row in n_split parts: partials [n_heads][n_split][D + 4] = {unnormalised output, log2-domain maximum, sum, 2 unused} of each head's parts in fp32 (a
+ * part without keys: 0, -inf, 0), gate: n_heads values whose sigmoid scales the heads, or null; sink: one more key of score 0 without a value.  16-bit types; c [N] */
+int lmx_op_gemv_heads(int32_t dtype, const float* partials, const void* gate, int32_t n_heads, int32_t n_split, int32_t D, int32_t sink, const void* w, void* c, int32_t N, void* stream);
+/* parts that it takes at most, on the host alone (0: a decode step leaves them to the attention's own merge) */
+int lmx_op_gemv_heads_splits(int32_t dtype, int32_t N, int32_t n_heads, int32_t D, int32_t* splits);
 int lmx_op_linear_f32(int32_t dtype, const void* x, const void* w, float* c, int32_t M, int32_t N, int32_t K, float cap, int32_t form, void* stream);
 int lmx_op_qkv_norm_rope_kv(int32_t dtype, int32_t D, void* qkv, int32_t qkv_stride, void* kcache, void* vtcache, const void* q_norm, const void* k_norm, const float* cos_sin_dev,
                             int32_t T, int32_t pos0, int32_t n_heads, int32_t n_kv_heads, int32_t s_max, int32_t qk_dim, int32_t rot_dims, float eps, void* stream);

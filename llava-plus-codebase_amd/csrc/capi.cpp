@@ -687,6 +687,20 @@ int lmx_op_gemv_residual(int32_t dtype, const float* x_in, const void* y, const 
                          S(stream));
     LMX_API_END
 }
+int lmx_op_gemv_heads_splits(int32_t dtype, int32_t N, int32_t n_heads, int32_t D, int32_t* splits) {
+    LMX_API_BEGIN
+    LMX_REQUIRE(splits && N >= 1 && n_heads >= 1 && D >= 8 && D % 8 == 0, "gemv_heads_splits: bad arguments");
+    const int K = n_heads * D;
+    *splits = gemv_heads_splits(dtype, GemvArgs{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0.f, N, K, K, K, N, 0, kActNone}, n_heads, D);
+    LMX_API_END
+}
+int lmx_op_gemv_heads(int32_t dtype, const float* partials, const void* gate, int32_t n_heads, int32_t n_split, int32_t D, int32_t sink, const void* w, void* c, int32_t N, void* stream) {
+    LMX_API_BEGIN
+    LMX_REQUIRE(partials && w && c && N >= 1 && n_heads >= 1 && D >= 8 && D % 8 == 0 && (reinterpret_cast<uintptr_t>(partials) | reinterpret_cast<uintptr_t>(w)) % 16 == 0, "gemv_heads: bad arguments");
+    const int K = n_heads * D;
+    launch_gemv_heads(dtype, GemvArgs{nullptr, w, c, nullptr, nullptr, nullptr, 0.f, N, K, K, K, N, 0, kActNone}, HeadSplitArgs{partials, gate, n_heads, n_split, D, sink}, S(stream));
+    LMX_API_END
+}
 int lmx_op_linear_f32(int32_t dtype, const void* x, const void* w, float* c, int32_t M, int32_t N, int32_t K, float cap, int32_t form, void* stream) {
     LMX_API_BEGIN
     LMX_REQUIRE(x && w && c && form >= 0 && form <= 2, "linear_f32: bad arguments");

@@ -155,6 +155,8 @@ _SIGS = {
     "lmx_op_residual_norm_form": (c_int32, [c_int32] * 4 + [POINTER(c_int32)]),
     "lmx_op_residual_norm": (c_int32, [c_int32] + [c_void_p] * 7 + [c_int32] * 3 + [c_float, c_float, c_void_p]),
     "lmx_op_gemv_residual": (c_int32, [c_int32] + [c_void_p] * 9 + [c_int32] * 3 + [c_float, c_float, c_int32, c_void_p]),
+    "lmx_op_gemv_heads": (c_int32, [c_int32, c_void_p, c_void_p] + [c_int32] * 4 + [c_void_p, c_void_p, c_int32, c_void_p]),
+    "lmx_op_gemv_heads_splits": (c_int32, [c_int32] * 4 + [POINTER(c_int32)]),
     "lmx_op_linear_f32": (c_int32, [c_int32] + [c_void_p] * 3 + [c_int32] * 3 + [c_float, c_int32, c_void_p]),
     "lmx_op_qkv_norm_rope_kv": (c_int32, [c_int32, c_int32, c_void_p, c_int32] + [c_void_p] * 5 + [c_int32] * 7 + [c_float, c_void_p]),
     "lmx_op_window_attn": (c_int32, [c_int32, c_int32, c_void_p, c_int32, c_void_p, c_int32, c_void_p, c_void_p] + [c_int32] * 5 + [c_float, c_int32, c_int32, c_void_p, c_int32, c_void_p]),

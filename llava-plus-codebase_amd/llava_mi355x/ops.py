@@ -239,6 +239,17 @@ def gemv_residual(x_in, y, post_w, inject, pre_w, w, mult, eps, bias=None, width
     return x, c
 
 
+def gemv_heads(partials, w, gate=None, sink=False):
+    """w on the merge of one row's split attention, [1, N]: partials [heads, splits, D + 4] fp32 (unnormalised output, log2-domain maximum, sum, 2 unused)."""
+    _need_cuda(partials, w, gate)
+    heads, n_split, row = partials.shape
+    if partials.dtype != torch.float32 or not partials.is_contiguous() or not w.is_contiguous() or w.shape[1] != heads * (row - 4) or (gate is not None and (gate.numel() != heads or gate.dtype != w.dtype or not gate.is_contiguous())):
+        raise ValueError("gemv_heads: contiguous fp32 partials, weights of all heads, a gate a head")
+    out = torch.empty((1, w.shape[0]), dtype=w.dtype, device=w.device)
+    check(lib.lmx_op_gemv_heads(torch_dtype_code(w.dtype), ptr(partials), ptr(gate), heads, n_split, row - 4, int(sink), ptr(w), ptr(out), w.shape[0], stream_handle()), "gemv_heads")
+    return out
+
+
 def linear_f32(x, w, cap=0.0, form=0):
     """x @ w.T with fp32 output, soft-capped; form 0 GEMM, 1 GEMV, 2 decode-batch kernel."""
     _need_cuda(x, w)

@@ -1,5 +1,6 @@
 """One sequence's decode step whose attention runs in splits: the output projection adds them (csrc/gemv2.h: SPLITS) against the attention's own merge and the oracle.  Two to sixteen splits
-and more, windows on a few of them, gates and sinks, rows of up to the 4096 a workgroup holds and past it, outputs below and above a row a wave."""
+and more, windows on a few of them, gates and sinks, rows of up to the 4096 a workgroup holds and past it, outputs below and above a row a wave; the projection
+itself on given splits against float64."""
 import pytest
 import torch
 
@@ -13,6 +14,7 @@ AT = (127, 128, 300, 511, 700, 897, 1024, 2046, 2100)
 FORMS = {
     "mixed": CONFIGS["mixed"], "wide": CONFIGS["wide"],
     "full": config([layer(32, 4, 128, 128, 0, 64, 64)], 2056, 64, None),       # 4096 inputs, two rows a wave
+    "ten": config([layer(24, 3, 128, 128, 0, 64, 64)], 2056, 64, None),        # 3072 inputs, two rows a wave: ten splits at most
     "past": config([layer(33, 3, 128, 128, 0, 64, 64)], 96, 64, None),         # 4224 inputs: the attention merges
 }
 
@@ -45,3 +47,42 @@ def test_splits_added_by_the_projection(cuda, name, dt):
     m.set_option("stack_fuse", 0)
     b = steps(m, toks)
     assert rel(a, want) < TOL[dt] and rel(a, b.double().cpu()) < TOL[dt] / 2
+
+
+def merged(p, gate, sink):
+    """the row that partials stand for, in float64"""
+    p = p.double()
+    D = p.shape[2] - 4
+    m = p[:, :, D]
+    M = m.max(1, keepdim=True).values.clamp_min(0.0 if sink else -float("inf"))
+    w = torch.exp2(m - M)
+    x = (w[:, :, None] * p[:, :, :D]).sum(1) / ((w * p[:, :, D + 1]).sum(1, keepdim=True) + (torch.exp2(-M) if sink else 0.0))
+    return (x if gate is None else x * torch.sigmoid(gate.double())[:, None]).reshape(-1)
+
+
+def partials(heads, n_split, D, g):
+    """maxima some powers of two apart, sums as of a few dozen keys; what follows a row's sum is nobody's"""
+    p = torch.randn(heads, n_split, D + 4, generator=g)
+    l = 1 + 40 * torch.rand(heads, n_split, generator=g)
+    p[:, :, :D] *= l[:, :, None]
+    p[:, :, D], p[:, :, D + 1], p[:, :, D + 2:] = 6 * torch.randn(heads, n_split, generator=g), l, float("nan")
+    return p
+
+
+@pytest.mark.parametrize("dt", list(DT))
+@pytest.mark.parametrize("heads,D,N,splits", [(8, 128, 200, range(2, 17)), (1, 64, 9, (2, 16)), (3, 256, 2050, (5, 11, 16)), (16, 256, 2056, (2, 7, 8)), (24, 128, 2049, (3, 9, 10)), (32, 128, 97, (4, 8)), (5, 64, 4100, (6, 13))])
+def test_given_splits_against_float64(cuda, dt, heads, D, N, splits):
+    from llava_mi355x import ops
+    g = torch.Generator().manual_seed(heads * D + N)
+    w = (torch.randn(N, heads * D, generator=g) / (heads * D) ** 0.5).to(DT[dt])
+    for n in splits:
+        p, gate, sink = partials(heads, n, D, g), (torch.randn(heads, generator=g) if n % 2 else None), n % 3 == 0
+        if n > 2:                                            # a split whose keys the window has left
+            p[::2, 1, :D], p[::2, 1, D], p[::2, 1, D + 1] = 0, -float("inf"), 0
+        gate = None if gate is None else gate.to(DT[dt])
+        got = ops.gemv_heads(p.to(cuda), w.to(cuda), None if gate is None else gate.to(cuda), sink)[0].double().cpu()
+        x = merged(p, gate, sink)
+        want, absolute = w.double() @ x, w.double().abs() @ x.abs()
+        # the row and the output are rounded once each: at most 2^-9 (bf16) or 2^-12 (f16) off, relative; 1e-5 for the fp32 weights, sums of 17 terms and products
+        half = 2.0 ** -9 if dt == "bf16" else 2.0 ** -12
+        assert bool(((got - want).abs() <= 1.01 * (absolute * (half + 1e-5) + want.abs() * half) + 1e-6).all()), (n, ((got - want).abs() / absolute).max().item())

@@ -1,4 +1,4 @@
-"""How a linear of one row streams its weights (csrc/gemm.hip: gemv2_form, gemv2_res_form), asked of the library on the host.  Cases of one row a wave were timed with two and with four loads of it on the way."""
+"""How a linear of one row streams its weights (csrc/gemm.hip: gemv2_form, gemv2_res_form, gemv_heads_splits), asked of the library on the host.  Cases of one row a wave were timed with two and with four loads of it on the way."""
 import ctypes
 
 import pytest
@@ -30,3 +30,15 @@ def test_a_row_formed_in_front(N, K, act, form):
     f = (ctypes.c_int32 * 3)()
     _C.check(_C.lib.lmx_op_gemv_residual_form(N, K, act, f))
     assert tuple(f) == form
+
+
+def test_splits_that_the_projection_takes():
+    from llava_mi355x import _C
+
+    def most(dt, N, heads, D):
+        s = ctypes.c_int32(-1)
+        _C.check(_C.lib.lmx_op_gemv_heads_splits(dt, N, heads, D, s))
+        return s.value
+    for dt in (_C.DTYPE_BF16, _C.DTYPE_F16):
+        assert [most(dt, 2056, h, 128) for h in (1, 8, 16, 17, 24, 32, 33)] == [16, 16, 16, 15, 10, 8, 0]
+    assert most(_C.DTYPE_F32, 2056, 8, 128) == 0

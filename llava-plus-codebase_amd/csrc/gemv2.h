@@ -199,6 +199,7 @@ __device__ __forceinline__ void gemv2_body(const GemvArgs& a, int bid, char* sme
         for (int s = 0; s < SPLITS; ++s) { m[s] = s < hs->n_split ? __uint_as_float(mraw[s][0]) : -INFINITY; M = fmaxf(M, m[s]); }
 #pragma unroll
         for (int s = 0; s < SPLITS; ++s) {
+            if (s > 0 && s >= hs->n_split) break;            // the last one once more counts nothing, whatever it holds (0 times infinity would)
             const float w = __builtin_amdgcn_exp2f(m[s] - M);
             l += w * __uint_as_float(mraw[s][1]);
 #pragma unroll

@@ -86,3 +86,15 @@ def test_given_splits_against_float64(cuda, dt, heads, D, N, splits):
         # the row and the output are rounded once each: at most 2^-9 (bf16) or 2^-12 (f16) off, relative; 1e-5 for the fp32 weights, sums of 17 terms and products
         half = 2.0 ** -9 if dt == "bf16" else 2.0 ** -12
         assert bool(((got - want).abs() <= 1.01 * (absolute * (half + 1e-5) + want.abs() * half) + 1e-6).all()), (n, ((got - want).abs() / absolute).max().item())
+
+
+@pytest.mark.parametrize("n", [3, 5, 7, 9])
+def test_an_infinite_value_stays_one(cuda, n):
+    """Forms for more splits than there are read the last one more than once: it weighs nothing the second time, whatever it holds."""
+    from llava_mi355x import ops
+    g = torch.Generator().manual_seed(n)
+    p, w = partials(4, n, 64, g), torch.randn(40, 256, generator=g).bfloat16()
+    p[2, n - 1, 5] = float("inf")
+    w[w == 0] = 1
+    got = ops.gemv_heads(p.to(cuda), w.to(cuda))[0].cpu()
+    assert torch.equal(got.float(), torch.where(w[:, 2 * 64 + 5] > 0, float("inf"), -float("inf")))

@@ -33,8 +33,9 @@ namespace lmx {
 //   * D = 128 takes K a round ahead of Vᵀ: a tile's exponentials stand between the next tile's score products, whose results they do not wait for, in one instruction stream (turn), with
 //     the LDS reads some products ahead.  8 waves on 128 rows, 64-key tiles: 2.0 -> 1.85 us;
 //   * where blocks of 128 rows leave CUs idle (flash_wide), 64 rows and 32-key tiles: four waves, two workgroups a CU, in step with nobody but themselves.
-// 1087 causal rows of 32 heads 25.0 -> 22.5 us, 139 rows on 1347 keys (with the merge of their slices) 26.8 -> 20.0, 2048 rows of 16 heads with 4 kv heads 39.6 -> 33.2, D = 64: four images of
-// 577 rows, 16 heads, 18.6 -> 17.7 (the scale in the exponential's own multiply-add).  Behind 9216 keys, 256 heads, 128 rows: 163 -> 153.
+// The launch alone, repeated: 1087 causal rows of 32 heads 25.0 -> 22.5 us (inside a prompt's pass 27 -> 24.1), 139 rows on 1347 keys (with the merge of their slices) 26.8 -> 20.0, 2048
+// rows of 16 heads with 4 kv heads 39.6 -> 33.2 (41 -> 35.0), D = 64: four images of 577 rows, 16 heads, 18.6 -> 17.7 (the scale in the exponential's own multiply-add).  Behind 9216 keys,
+// 256 heads, 128 rows: 163 -> 153.
 // WIN (FlashArgs::win): sliding window, softmax sink and output gate of the windowed decoders.  Only the key tiles a query block can see are walked: the tile
 // range starts at the tile of the first row's oldest visible key, so the work per block is bounded by the window.
 // Without a causal limit every row's position lies behind the last key (launch_flash_prefill): the same code, and fewer registers than a form of its own took.
@@ -302,8 +303,8 @@ __device__ __forceinline__ void flash_body(const FlashArgs& a, const int block, 
             round(next, sa, sb, r);
             round(next, sb, sa, r + 1);
         }
-        // one round without a next tile for odd and even counts: with one of each behind the loop, 128 rows took 256 registers and spilled 23, whose reloads waited for the DMAs (this form: 220, 64
-        // rows 181 instead of 241; the loop is the same, the copy is 32 registers once)
+        // One round without a next tile for odd and even counts.  With one of each behind the loop, 128 rows took 256 registers and spilled 23, whose reloads waited for the DMAs; this form
+        // takes 238 (windowed 244), 64 rows 197 for 241.  The loop is the same, the copy is 32 registers once
         if (r + 1 < mine) {
             round(next, sa, sb, r);
 #pragma unroll
@@ -459,7 +460,8 @@ static int flash_slices(int D, const FlashArgs& a, int workgroups, bool wide) {
 // their own) divide the work twice as finely, and the matrix cores of one workgroup run beside the exponentials of the other.  The larger blocks where they keep the chip busy to the end:
 // their work over 256 CUs against what the busiest CU has, the block with the most tiles or, in a second round (heaviest first), what the last of the first and the first of the second
 // take together.  us, 128 -> 64 rows:  1087 causal rows, 32 heads (0.65 of the time busy) 25.0 -> 22.5;  1100, 16 heads (0.31) 22.6 -> 19.8;  2048, 16 heads (0.53) 36.6 -> 33.2;  2048 in a
-// window of 1024, 32 heads (0.79) 50.5 -> 45.5;  2048, 32 heads (1.0) 52.9 -> 55.8;  128 rows behind 9216, 256 heads (1.0) 159 -> 172.
+// window of 1024, 32 heads (0.79) 50.5 -> 45.5;  2048, 32 heads (1.0) 52.9 -> 55.8;  128 rows behind 9216, 256 heads (1.0) 159 -> 172.  The line lies between 0.79 and 1.0.  Past two rounds,
+// 512 blocks, always 128 rows, as before there were smaller ones: a third round of a few blocks (513 .. 767) was not compared.  The 128-row figures are of a form that spilled 23 registers.
 static bool flash_wide(int D, const FlashArgs& a) {
     if (D != 128) return true;
     const int nqb = cdiv(a.q_len, 128);
